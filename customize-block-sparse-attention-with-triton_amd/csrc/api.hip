@@ -333,4 +333,36 @@ int bsattn_reorder(const void* x, void* out, int BS, int NH, int F, int Hh, int 
   return launch_reorder(x, out, BS, NH, F, Hh, W, (int)row_bytes, orders, inv_orders, (hipStream_t)stream);
 }
 
+int bsattn_reorder_inplace_workspace(int n, int BS, int NH, int F, int Hh, int W, int D, int elem_bytes, size_t* bytes) {
+  if (bytes == nullptr) return BSATTN_ERR_NULL;
+  if (n <= 0 || n > 4 || BS <= 0 || NH <= 0 || F <= 0 || Hh <= 0 || W <= 0 || D <= 0 || elem_bytes <= 0) return BSATTN_ERR_SHAPE;
+  const int64_t row_bytes = (int64_t)D * elem_bytes;
+  if (row_bytes % 16 != 0) return BSATTN_ERR_STRIDE;
+  if ((int64_t)n * BS * NH > 0x7fffffffLL || (int64_t)F * Hh * W > 0x7fffffffLL || row_bytes > 0x7fffffffLL) return BSATTN_ERR_RANGE;
+  *bytes = reorder_workspace_bytes(n, BS, NH, F, Hh, W, (int)row_bytes);
+  return *bytes == 0 ? BSATTN_ERR_RANGE : BSATTN_OK;
+}
+
+int bsattn_reorder_inplace(void* const* x, const int64_t* strides, int n, int BS, int NH, int F, int Hh, int W, int D,
+                           int elem_bytes, const void* numbers, int number_bytes, int inverse, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  if (x == nullptr || strides == nullptr || numbers == nullptr) return BSATTN_ERR_NULL;
+  if (number_bytes != 4 && number_bytes != 8) return BSATTN_ERR_DTYPE;
+  size_t need = 0;
+  const int rc = bsattn_reorder_inplace_workspace(n, BS, NH, F, Hh, W, D, elem_bytes, &need);
+  if (rc != BSATTN_OK) return rc;
+  int64_t bytes[12];
+  for (int i = 0; i < 3 * n; ++i) {
+    bytes[i] = strides[i] * elem_bytes;
+    if (bytes[i] % 16 != 0) return BSATTN_ERR_STRIDE;
+  }
+  for (int i = 0; i < n; ++i) {
+    if (x[i] == nullptr) return BSATTN_ERR_NULL;
+    if (((uintptr_t)x[i] & 15) != 0) return BSATTN_ERR_STRIDE;
+  }
+  if (workspace == nullptr || workspace_bytes < need) return BSATTN_ERR_WORKSPACE;
+  if (((uintptr_t)workspace & 15) != 0) return BSATTN_ERR_STRIDE;
+  return launch_reorder_inplace(x, bytes, n, BS, NH, F, Hh, W, D * elem_bytes, numbers, number_bytes, inverse, workspace, (hipStream_t)stream);
+}
+
 }  // extern "C"

@@ -72,6 +72,9 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
 // reorder.hip
 int launch_reorder(const void* x, void* out, int BS, int NH, int F, int Hh, int W, int row_bytes,
                    const int32_t* orders, const int32_t* inv_orders, hipStream_t st);
+size_t reorder_workspace_bytes(int n, int BS, int NH, int F, int Hh, int W, int row_bytes);
+int launch_reorder_inplace(void* const* x, const int64_t* strides, int n, int BS, int NH, int F, int Hh, int W,
+                           int row_bytes, const void* numbers, int number_bytes, int inverse, void* ws, hipStream_t st);   // strides in bytes
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? BSATTN_OK : BSATTN_ERR_LAUNCH; }
 

@@ -42,6 +42,8 @@ _SIGNATURES = {
     "bsattn_bwd_workspace": ([_i, _i, _i, _i, ctypes.POINTER(ctypes.c_size_t)], _i),
     "bsattn_bwd": ([_p] * 13 + [_i] * 8 + [_f] + [_p] * 8 + [_p, ctypes.c_size_t, _p], _i),
     "bsattn_bwd_elementwise": ([_p] * 15 + [_i] * 8 + [_f] + [_p] * 8 + [_p, ctypes.c_size_t, _p], _i),
+    "bsattn_reorder_inplace_workspace": ([_i] * 8 + [ctypes.POINTER(ctypes.c_size_t)], _i),
+    "bsattn_reorder_inplace": ([_p, _p] + [_i] * 8 + [_p, _i, _i, _p, ctypes.c_size_t, _p], _i),
     "bsattn_reorder": ([_p, _p, _i, _i, _i, _i, _i, _i, _i, _p, _p, _p], _i),
 }
 EXPORTS = tuple(_SIGNATURES)
@@ -104,6 +106,14 @@ def mask_lists_workspace(Bm, Hm, nb):
     n = ctypes.c_size_t()
     check(lib().bsattn_mask_lists_workspace(Bm, Hm, nb, ctypes.byref(n)), "bsattn_mask_lists_workspace")
     return n.value
+
+
+@functools.lru_cache(maxsize=64)
+def reorder_inplace_workspace(n_tensors, BS, NH, F, H, W, D, elem_bytes):
+    """Bytes, or None where the in-place reorder does not take the shape."""
+    n = ctypes.c_size_t()
+    rc = lib().bsattn_reorder_inplace_workspace(n_tensors, BS, NH, F, H, W, D, elem_bytes, ctypes.byref(n))
+    return n.value if rc == 0 else None
 
 
 def _device_index(device):

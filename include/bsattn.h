@@ -54,7 +54,7 @@ extern "C" {
  *   100: first layout.
  *   200: bsattn_bwd and bsattn_bwd_elementwise take dq_strides, dk_strides, dv_strides after
  *        do_strides; the entry points of the forward over quads of row blocks are gone. */
-#define BSATTN_ABI_VERSION 200
+#define BSATTN_ABI_VERSION 201
 int bsattn_version(void);
 /* Process-wide switch (default off), returns the previous setting.  On: the forward's result
  * depends on nothing but its inputs and the device (two runs give the same bits).  Off: the
@@ -301,6 +301,22 @@ int bsattn_bwd_elementwise(const void* q, const void* k, const void* v, const vo
 int bsattn_reorder(const void* x, void* out, int BS, int NH, int F, int Hh, int W, int D,
                    int elem_bytes, const int32_t* orders, const int32_t* inv_orders,
                    void* stream);
+
+/* The same reorder in place on 1 to 4 tensors of one shape (q, k and v of a layer, or the attention result), as
+ * permute_qkv_triton / inv_permute_attn_triton do to the image tokens of theirs (fa2_custom_mask/functional.py:22-84).
+ * x[i]: first image token of tensor i; strides[3 i ..]: its batch, head and token strides in elements (innermost
+ * stride 1; rows, strides and addresses multiples of 16 bytes); the tensors must not overlap.  numbers: device memory,
+ * NH integers of number_bytes (4 or 8), the row of the permutation table (functional.py:23-26) each head takes, negative
+ * ones counted from its end (a head with a number outside the table is left alone); inverse != 0: the orders back (:69-76).
+ * A head may have up to 57344 rows and 7 MB; the workspace query returns BSATTN_ERR_RANGE for larger ones.  The
+ * workspace (16-byte aligned) needs no particular contents on entry.
+ * The workgroups that hold the rows of a head wait for each other, each for a limited time only: where they do not get
+ * to run together (a launch confined to a few compute units) one of them moves the head. */
+int bsattn_reorder_inplace_workspace(int n, int BS, int NH, int F, int Hh, int W, int D, int elem_bytes,
+                                     size_t* bytes);
+int bsattn_reorder_inplace(void* const* x, const int64_t* strides, int n, int BS, int NH, int F, int Hh, int W,
+                           int D, int elem_bytes, const void* numbers, int number_bytes, int inverse,
+                           void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }
