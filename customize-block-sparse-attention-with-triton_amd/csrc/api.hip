@@ -103,14 +103,18 @@ int bsattn_tail_mask_tiles(int Bm, int Hm, int nb, int valid_last, int transpose
                            (unsigned long long*)tile_bits, (hipStream_t)stream);
 }
 
-static int check_attn(int Bm, int Hm, int B, int H, int N, int D, int dtype, int out_dtype) {
-  if (B <= 0 || H <= 0 || N <= 0 || N % BSATTN_TILE != 0) return BSATTN_ERR_SHAPE;
+static int blocks_of(int N) { return (N + BSATTN_TILE - 1) / BSATTN_TILE; }
+
+// any_n: N may be any positive number of tokens (the _tokens entry points)
+static int check_attn(int Bm, int Hm, int B, int H, int N, int D, int dtype, int out_dtype, bool any_n = false) {
+  if (B <= 0 || H <= 0 || N <= 0 || (!any_n && N % BSATTN_TILE != 0)) return BSATTN_ERR_SHAPE;
+  if (N > 0x7fffffff - BSATTN_TILE) return BSATTN_ERR_RANGE;
   if (!((Bm == 1 || Bm == B) && (Hm == 1 || Hm == H))) return BSATTN_ERR_SHAPE;
   if (D != 64 && D != 128 && D != 256) return BSATTN_ERR_HEAD_DIM;
   if (dtype != BSATTN_F16 && dtype != BSATTN_BF16) return BSATTN_ERR_DTYPE;
   if (out_dtype != dtype && out_dtype != BSATTN_F32) return BSATTN_ERR_DTYPE;
   if ((int64_t)B * H > 65535) return BSATTN_ERR_RANGE;
-  const int64_t nb = N / BSATTN_TILE;
+  const int64_t nb = blocks_of(N);
   if ((int64_t)Bm * Hm * nb * nb > 0x7fffffffLL) return BSATTN_ERR_RANGE;
   return BSATTN_OK;
 }
@@ -136,10 +140,10 @@ int bsattn_fwd_workspace(int B, int H, int N, int D, size_t* bytes) {
 static int fwd_check(const void* q, const void* k, const void* v, void* o, const int32_t* row_ptr,
                      const int32_t* col_idx, int Bm, int Hm, int B, int H, int N, int D, int dtype,
                      int out_dtype, const int64_t* q_strides, const int64_t* k_strides,
-                     const int64_t* v_strides, const int64_t* o_strides) {
+                     const int64_t* v_strides, const int64_t* o_strides, bool any_n = false) {
   if (q == nullptr || k == nullptr || v == nullptr || o == nullptr || row_ptr == nullptr || col_idx == nullptr)
     return BSATTN_ERR_NULL;
-  int rc = check_attn(Bm, Hm, B, H, N, D, dtype, out_dtype);
+  int rc = check_attn(Bm, Hm, B, H, N, D, dtype, out_dtype, any_n);
   if (rc != BSATTN_OK) return rc;
   if ((rc = check_strides(q_strides, 2, q)) != BSATTN_OK) return rc;
   if ((rc = check_strides(k_strides, 2, k)) != BSATTN_OK) return rc;
@@ -152,9 +156,9 @@ static int fwd_common(const void* q, const void* k, const void* v, void* o, floa
                       const uint64_t* tile_bits, int Bm, int Hm, int B, int H, int N,
                       int D, int dtype, int out_dtype, float sm_scale, const int64_t* q_strides,
                       const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides,
-                      void* workspace, size_t workspace_bytes, void* stream) {
+                      void* workspace, size_t workspace_bytes, void* stream, bool any_n = false) {
   const int rc = fwd_check(q, k, v, o, row_ptr, col_idx, Bm, Hm, B, H, N, D, dtype, out_dtype, q_strides, k_strides,
-                           v_strides, o_strides);
+                           v_strides, o_strides, any_n);
   if (rc != BSATTN_OK) return rc;
   if (workspace == nullptr || workspace_bytes < coop_workspace_bytes(B, H, N, D)) return BSATTN_ERR_WORKSPACE;
   if (((uintptr_t)workspace & 15) != 0) return BSATTN_ERR_STRIDE;
@@ -189,20 +193,20 @@ int bsattn_fwd_block_mask_workspace(int Bm, int Hm, int B, int H, int N, int D, 
   return BSATTN_OK;
 }
 
-int bsattn_fwd_block_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+static int fwd_block_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
                           const int64_t* mask_strides, int Bm, int Hm, int32_t* row_ptr, int32_t* col_idx,
                           int32_t* counts, int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
                           const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
-                          const int64_t* o_strides, void* workspace, size_t workspace_bytes, void* stream) {
+                          const int64_t* o_strides, void* workspace, size_t workspace_bytes, void* stream, bool any_n) {
   if (block == nullptr || mask_strides == nullptr || counts == nullptr) return BSATTN_ERR_NULL;
   int rc = fwd_check(q, k, v, o, row_ptr, col_idx, Bm, Hm, B, H, N, D, dtype, out_dtype, q_strides, k_strides,
-                     v_strides, o_strides);
+                     v_strides, o_strides, any_n);
   if (rc != BSATTN_OK) return rc;
   size_t need = 0;
-  if ((rc = bsattn_fwd_block_mask_workspace(Bm, Hm, B, H, N, D, &need)) != BSATTN_OK) return rc;
+  if ((rc = bsattn_fwd_block_mask_workspace(Bm, Hm, B, H, blocks_of(N) * BSATTN_TILE, D, &need)) != BSATTN_OK) return rc;
   if (workspace == nullptr || workspace_bytes < need) return BSATTN_ERR_WORKSPACE;
   if (((uintptr_t)workspace & 15) != 0) return BSATTN_ERR_STRIDE;
-  const int nb = N / BSATTN_TILE;
+  const int nb = blocks_of(N);
   rc = launch_block_mask_to_lists(block, Bm, Hm, nb, mask_strides[0], mask_strides[1], mask_strides[2], mask_strides[3],
                                   row_ptr, col_idx, nullptr, counts, (int32_t*)workspace, (hipStream_t)stream);
   if (rc != BSATTN_OK) return rc;
@@ -214,6 +218,35 @@ int bsattn_fwd_block_mask(const void* q, const void* k, const void* v, void* o, 
                     (hipStream_t)stream);
 }
 
+int bsattn_fwd_block_mask(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+                          const int64_t* mask_strides, int Bm, int Hm, int32_t* row_ptr, int32_t* col_idx,
+                          int32_t* counts, int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                          const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                          const int64_t* o_strides, void* workspace, size_t workspace_bytes, void* stream) {
+  return fwd_block_mask(q, k, v, o, lse, block, mask_strides, Bm, Hm, row_ptr, col_idx, counts, B, H, N, D, dtype, out_dtype,
+                        sm_scale, q_strides, k_strides, v_strides, o_strides, workspace, workspace_bytes, stream, false);
+}
+
+int bsattn_fwd_block_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+                                 const int64_t* mask_strides, int Bm, int Hm, int32_t* row_ptr, int32_t* col_idx,
+                                 int32_t* counts, int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                                 const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                                 const int64_t* o_strides, void* workspace, size_t workspace_bytes, void* stream) {
+  return fwd_block_mask(q, k, v, o, lse, block, mask_strides, Bm, Hm, row_ptr, col_idx, counts, B, H, N, D, dtype, out_dtype,
+                        sm_scale, q_strides, k_strides, v_strides, o_strides, workspace, workspace_bytes, stream, true);
+}
+
+int bsattn_fwd_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const int32_t* row_ptr,
+                      const int32_t* col_idx, const uint8_t* tile_partial, const uint64_t* tile_bits, int Bm, int Hm,
+                      int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale, const int64_t* q_strides,
+                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* o_strides, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  if ((tile_partial == nullptr) != (tile_bits == nullptr)) return BSATTN_ERR_NULL;
+  if (((uintptr_t)tile_bits & 7) != 0) return BSATTN_ERR_STRIDE;
+  return fwd_common(q, k, v, o, lse, row_ptr, col_idx, tile_partial, tile_bits, Bm, Hm, B, H, N, D, dtype, out_dtype,
+                    sm_scale, q_strides, k_strides, v_strides, o_strides, workspace, workspace_bytes, stream, true);
+}
+
 int bsattn_fwd_static(const void* q, const void* k, const void* v, void* o, float* lse,
                       const int32_t* row_ptr, const int32_t* col_idx, int Bm, int Hm, int B, int H, int N,
                       int D, int dtype, int out_dtype, float sm_scale, const int64_t* q_strides,
@@ -222,12 +255,13 @@ int bsattn_fwd_static(const void* q, const void* k, const void* v, void* o, floa
   int rc = fwd_check(q, k, v, o, row_ptr, col_idx, Bm, Hm, B, H, N, D, dtype, out_dtype, q_strides, k_strides,
                      v_strides, o_strides);
   if (rc != BSATTN_OK) return rc;
-  const size_t need = coop_workspace_bytes(B, H, N, D);
+  const size_t need = coop_workspace_bytes(B, H, N, D, /*compact=*/true);
   if (need > (size_t)BSATTN_STATIC_SCRATCH_BYTES) return BSATTN_ERR_STATIC_LIMIT;
   void* ws = nullptr;
   if ((rc = static_scratch(&ws)) != BSATTN_OK) return rc;
   AttnShape s;
   s.B = B; s.H = H; s.N = N; s.D = D; s.Bm = Bm; s.Hm = Hm; s.dtype = dtype; s.out_dtype = out_dtype;
+  s.compact = true;
   s.sm_scale = sm_scale;
   for (int i = 0; i < 3; ++i) { s.qs[i] = q_strides[i]; s.ks[i] = k_strides[i]; s.vs[i] = v_strides[i]; s.os[i] = o_strides[i]; s.dos[i] = 0; }
   return launch_fwd(q, k, v, o, lse, row_ptr, col_idx, nullptr, nullptr, s, ws, (hipStream_t)stream);
@@ -262,12 +296,12 @@ static int bwd_common(const void* q, const void* k, const void* v, const void* o
                       const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
                       const int64_t* o_strides, const int64_t* do_strides, const int64_t* dq_strides,
                       const int64_t* dk_strides, const int64_t* dv_strides, void* workspace,
-                      size_t workspace_bytes, void* stream) {
+                      size_t workspace_bytes, void* stream, bool any_n = false) {
   if (q == nullptr || k == nullptr || v == nullptr || o == nullptr || d_o == nullptr || lse == nullptr ||
       dq == nullptr || dk == nullptr || dv == nullptr || row_ptr == nullptr || col_idx == nullptr ||
       col_ptr == nullptr || row_idx == nullptr)
     return BSATTN_ERR_NULL;
-  int rc = check_attn(Bm, Hm, B, H, N, D, dtype, out_dtype);
+  int rc = check_attn(Bm, Hm, B, H, N, D, dtype, out_dtype, any_n);
   if (rc != BSATTN_OK) return rc;
   if ((rc = check_strides(q_strides, 2, q)) != BSATTN_OK) return rc;
   if ((rc = check_strides(k_strides, 2, k)) != BSATTN_OK) return rc;
@@ -321,6 +355,22 @@ int bsattn_bwd_elementwise(const void* q, const void* k, const void* v, const vo
   return bwd_common(q, k, v, o, d_o, lse, dq, dk, dv, row_ptr, col_idx, col_ptr, row_idx, tile_bits_rows,
                     tile_bits_cols, Bm, Hm, B, H, N, D, dtype, out_dtype, sm_scale, q_strides, k_strides, v_strides,
                     o_strides, do_strides, dq_strides, dk_strides, dv_strides, workspace, workspace_bytes, stream);
+}
+
+int bsattn_bwd_tokens(const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                      const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
+                      const int32_t* col_idx, const int32_t* col_ptr, const int32_t* row_idx,
+                      const uint64_t* tile_bits_rows, const uint64_t* tile_bits_cols, int Bm, int Hm,
+                      int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                      const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                      const int64_t* o_strides, const int64_t* do_strides, const int64_t* dq_strides,
+                      const int64_t* dk_strides, const int64_t* dv_strides, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+  if ((tile_bits_rows == nullptr) != (tile_bits_cols == nullptr)) return BSATTN_ERR_NULL;
+  if ((((uintptr_t)tile_bits_rows | (uintptr_t)tile_bits_cols) & 7) != 0) return BSATTN_ERR_STRIDE;
+  return bwd_common(q, k, v, o, d_o, lse, dq, dk, dv, row_ptr, col_idx, col_ptr, row_idx, tile_bits_rows,
+                    tile_bits_cols, Bm, Hm, B, H, N, D, dtype, out_dtype, sm_scale, q_strides, k_strides, v_strides,
+                    o_strides, do_strides, dq_strides, dk_strides, dv_strides, workspace, workspace_bytes, stream, true);
 }
 
 int bsattn_reorder(const void* x, void* out, int BS, int NH, int F, int Hh, int W, int D, int elem_bytes,

@@ -87,6 +87,29 @@ __device__ __forceinline__ void half_tile_load_async(const unsigned short* tile,
   }
 }
 
+// The same for rows first .. first + ROWS - 1 of a tile of which only `valid` rows exist (N is not a multiple of 64):
+// the last one is repeated in place of the others, so that no address lies beyond the tensor.  tile: row 0 of it.
+// (The lane index as a value the compiler cannot trace back: the offsets would otherwise be computed before the
+// walk and held through it.)
+template <int NWV, int D, int ROWS>
+__device__ __forceinline__ void tail_tile_load_async(const unsigned short* tile, int64_t stride, int first, int valid, int wv,
+                                                     int lane, unsigned lds_addr) {
+  constexpr int CPR = D / 8, PER_WAVE = ROWS * CPR / (64 * NWV);
+  asm volatile("" : "+v"(lane));
+#pragma unroll 1
+  for (int j = wv * PER_WAVE; j < (wv + 1) * PER_WAVE; ++j) {
+    const int c = j * 64 + lane, row = c / CPR, ch = c % CPR, src = first + row < valid ? first + row : valid - 1;
+    tile_load_async_one(tile, 2u * (unsigned)(src * (int)stride + ((ch ^ u_swz<D>(row)) * 8)), lds_addr + j * 1024);
+  }
+}
+
+// Mask word of a lane in such a tile, shifted for mask_scores: bit = row or column of the tile, set for the first
+// `valid` < 64.  (From a value the compiler cannot trace back, or its tests are made before the walk and held.)
+__device__ __forceinline__ unsigned long long tail_word(int valid, int g) {
+  asm volatile("" : "+s"(valid));
+  return ((1ull << valid) - 1ull) >> (4 * g);
+}
+
 // asynchronous copy of 64 consecutive floats (one per lane)
 __device__ __forceinline__ void stat_load_async(const float* src, int lane, unsigned lds_addr) {
   const unsigned off = 4u * (unsigned)lane;
@@ -172,7 +195,10 @@ __device__ __forceinline__ void head_and_block(int L, int BH, int nb, int& bh, i
 // KB: 32-key blocks of a tile handled per step.  2: a whole tile per step.  1 (used at D = 128): a
 // tile is walked in two steps of 32 keys; the staged halves are 8 KB, four workgroups fit a compute
 // unit and the wavefront stays within 256 registers: two wavefronts per SIMD.
-template <int D, bool BF16, bool EW, bool PB, int KB>
+// TAIL: N is not a multiple of 64.  The last row block has queries that do not exist (its loads repeat the last query,
+// nothing is written for them), the last tile of a list keys that do not exist (the copy repeats the last one, the scores
+// are -inf).
+template <int D, bool BF16, bool EW, bool PB, int KB, bool TAIL>
 __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdParams prm) {
   using C = BwdCfg<D, EW, 32 * KB>;
   constexpr int KS = D / 16, DB = D / 32, STEPS = 2 / KB;
@@ -194,9 +220,12 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   // The rows this workgroup owns for its whole walk (Q, dO, O, lse of its queries) depend on the block index only:
   // they are asked for first, and travel while the list is looked up and the first tiles are requested.
   const int64_t qrow = (int64_t)m * 64 + 32 * wv + ln;
-  const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + qrow * prm.qs[2];
-  const unsigned short* gp = (const unsigned short*)prm.d_o + b * prm.dos[0] + h * prm.dos[1] + qrow * prm.dos[2];
-  const unsigned short* op = (const unsigned short*)prm.o + b * prm.os[0] + h * prm.os[1] + qrow * prm.os[2];
+  const bool exists = !TAIL || qrow < prm.N;
+  const int64_t qsrc = exists ? qrow : prm.N - 1;
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64;
+  const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + qsrc * prm.qs[2];
+  const unsigned short* gp = (const unsigned short*)prm.d_o + b * prm.dos[0] + h * prm.dos[1] + qsrc * prm.dos[2];
+  const unsigned short* op = (const unsigned short*)prm.o + b * prm.os[0] + h * prm.os[1] + qsrc * prm.os[2];
   uintx4 qfr[KS], dofr[KS], ofr[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -205,7 +234,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   }
 #pragma unroll
   for (int s = 0; s < KS; ++s) ofr[s] = *reinterpret_cast<const uintx4*>(op + 16 * s + 8 * g);
-  const float lse_q = prm.lse[(int64_t)bh * prm.N + qrow];
+  const float lse_q = prm.lse[(int64_t)bh * prm.N + qsrc];
   int u0, u1;                                                  // steps: tile u / STEPS, part u % STEPS
   {
     const int t0 = rp[m], len = rp[m + 1] - t0;                // this workgroup's share of the row's list
@@ -216,12 +245,19 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
 
   const unsigned short* kg = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1];
   const unsigned short* vg = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1];
+  int blk_issued = 0;        // (TAIL) column block of the step issued last
   auto issue = [&](int u, int stage) {
-    const int t = u / STEPS;
-    const int64_t key0 = (int64_t)cols[t] * 64 + (u % STEPS) * 32 * KB;
-    half_tile_load_async<D, 32 * KB>(kg + key0 * prm.ks[2], prm.ks[2], wv, lane, lds_addr + stage * C::STAGE_BYTES);
-    half_tile_load_async<D, 32 * KB>(vg + key0 * prm.vs[2], prm.vs[2], wv, lane,
-                                     lds_addr + stage * C::STAGE_BYTES + C::TILE_BYTES);
+    const int t = u / STEPS, cb = cols[t];
+    const unsigned sa = lds_addr + stage * C::STAGE_BYTES;
+    blk_issued = cb;
+    if (TAIL && cb == nb - 1) {
+      tail_tile_load_async<2, D, 32 * KB>(kg + (int64_t)cb * 64 * prm.ks[2], prm.ks[2], (u % STEPS) * 32 * KB, valid, wv, lane, sa);
+      tail_tile_load_async<2, D, 32 * KB>(vg + (int64_t)cb * 64 * prm.vs[2], prm.vs[2], (u % STEPS) * 32 * KB, valid, wv, lane, sa + C::TILE_BYTES);
+    } else {
+      const int64_t key0 = (int64_t)cb * 64 + (u % STEPS) * 32 * KB;
+      half_tile_load_async<D, 32 * KB>(kg + key0 * prm.ks[2], prm.ks[2], wv, lane, sa);
+      half_tile_load_async<D, 32 * KB>(vg + key0 * prm.vs[2], prm.vs[2], wv, lane, sa + C::TILE_BYTES);
+    }
     if constexpr (EW)   // the tile's 64 mask words, 256 bytes per wavefront
       stat_load_async(reinterpret_cast<const float*>(prm.bits_rows + (int64_t)t * 64) + wv * 64, lane,
                       lds_addr + stage * C::STAGE_BYTES + 2 * C::TILE_BYTES + C::STAT_BYTES + wv * 256);
@@ -238,7 +274,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
 #pragma unroll
     for (int s = 0; s < KS; ++s) acc = dot8<BF16>(ofr[s], dofr[s], acc);
     dlt = acc + __shfl_xor(acc, 32);
-    if (chunk == 0 && g == 0) prm.delta[(int64_t)bh * prm.N + qrow] = dlt;
+    if (chunk == 0 && g == 0 && exists) prm.delta[(int64_t)bh * prm.N + qrow] = dlt;
   }
 #pragma unroll
   for (int s = 0; s < KS; ++s) { settle(qfr[s]); settle(dofr[s]); }
@@ -253,6 +289,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
     const int stage = (u - u0) & 1;
     wait_vm<0>();
     __syncthreads();   // step u complete in `stage`; everyone is done with the other stage
+    const bool tail_step = TAIL && !EW && blk_issued == nb - 1;
     if (u + 1 < u1) issue(u + 1, stage ^ 1);
     const unsigned char* kt = lds + stage * C::STAGE_BYTES;
     const unsigned char* vt = kt + C::TILE_BYTES;
@@ -290,6 +327,11 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
       if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw);
       else mask_scores(sacc[0], (unsigned)mw);
     }
+    if (tail_step) {
+      const unsigned long long mw = tail_word(valid, g);
+      if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw);
+      else mask_scores(sacc[0], (unsigned)(mw >> (32 * (u % STEPS))));
+    }
     // K^T fragments of the second product, read under the exponentials below
     uintx4 fkt[2 * KB][DB];
 #pragma unroll
@@ -316,6 +358,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   }
 
   if (prm.split > 1) {   // unscaled fp32 part; sum_parts_kernel adds the parts up
+    if (!exists) return;
     float* part = prm.part_dq + ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -330,24 +373,22 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   __syncthreads();           // the other wavefront has left its last step
   const float sc = prm.sm_scale;
   rows_out<BF16, D>(lds + wv * C::STAGE_BYTES, prm.dq, b * prm.dqs[0] + h * prm.dqs[1] + ((int64_t)m * 64 + 32 * wv) * prm.dqs[2],
-                    prm.dqs[2], prm.out_f32, lane, [&](int db, int i) { return dqacc[db][i] * sc; });
+                    prm.dqs[2], prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * wv) : 32, [&](int db, int i) { return dqacc[db][i] * sc; });
 }
 
 // ---------------------------------------------------------------------------------------
 // dK, dV: workgroup = column block n, wavefront wv owns keys 64n + 32wv + ln
 // ---------------------------------------------------------------------------------------
-// QB: 32-query blocks of a tile handled per step (2: a whole tile; 1: a tile in two halves, which
-// halves the fragments in flight).
+// A tile is walked in two steps of 32 queries, which halves the fragments in flight.
 // DH: -1, or at D = 256 the half (0 / 1) of the head dimension whose dK and dV columns this launch
 // accumulates and writes (the first products always contract over the whole head dimension): with
 // 128 columns at a time the accumulators and K, V of 32 keys are 256 registers instead of 384.
-template <int D, bool BF16, bool EW, bool PB, int QB, int DH>
-__global__ __launch_bounds__(128, (QB == 1 && D == 64) ? 2 : 1) void dkdv_kernel(const BwdParams prm) {
-  using C = BwdCfg<D, EW, 32 * QB>;
-  constexpr int KS = D / 16, STEPS = 2 / QB;
+template <int D, bool BF16, bool EW, bool PB, int DH, bool TAIL>
+__global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdParams prm) {
+  using C = BwdCfg<D, EW, 32>;
+  constexpr int KS = D / 16, STEPS = 2;
   constexpr int DB = DH < 0 ? D / 32 : D / 64, DB0 = DH < 0 ? 0 : DH * DB;   // 32-column blocks of this launch, the first one
   constexpr int PORTIONS = D == 256 ? 2 : 1, KSP = KS / PORTIONS;            // fragments of the first products in portions
-  static_assert(QB == 1 || PORTIONS == 1, "whole tiles per step only without portions");
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
@@ -373,14 +414,24 @@ __global__ __launch_bounds__(128, (QB == 1 && D == 64) ? 2 : 1) void dkdv_kernel
   const unsigned short* gg = (const unsigned short*)prm.d_o + b * prm.dos[0] + h * prm.dos[1];
   const float* lse_h = prm.lse + (int64_t)bh * prm.N;
   const float* dlt_h = prm.delta + (int64_t)bh * prm.N;
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64;
+  int blk_issued = 0;        // (TAIL) row block of the step issued last
   auto issue = [&](int u, int stage) {
     const int t = u / STEPS;
     const int rb = rows[t];
-    const int64_t row0 = (int64_t)rb * 64 + (u % STEPS) * 32 * QB;
     const unsigned sa = lds_addr + stage * C::STAGE_BYTES;
-    half_tile_load_async<D, 32 * QB>(qg + row0 * prm.qs[2], prm.qs[2], wv, lane, sa);
-    half_tile_load_async<D, 32 * QB>(gg + row0 * prm.dos[2], prm.dos[2], wv, lane, sa + C::TILE_BYTES);
-    stat_load_async((wv == 0 ? lse_h : dlt_h) + rb * 64, lane, sa + 2 * C::TILE_BYTES + wv * 256);   // all 64 rows of the tile
+    blk_issued = rb;
+    int stat_lane = lane;
+    if (TAIL && rb == nb - 1) {
+      tail_tile_load_async<2, D, 32>(qg + (int64_t)rb * 64 * prm.qs[2], prm.qs[2], (u % STEPS) * 32, valid, wv, lane, sa);
+      tail_tile_load_async<2, D, 32>(gg + (int64_t)rb * 64 * prm.dos[2], prm.dos[2], (u % STEPS) * 32, valid, wv, lane, sa + C::TILE_BYTES);
+      stat_lane = lane < valid ? lane : valid - 1;
+    } else {
+      const int64_t row0 = (int64_t)rb * 64 + (u % STEPS) * 32;
+      half_tile_load_async<D, 32>(qg + row0 * prm.qs[2], prm.qs[2], wv, lane, sa);
+      half_tile_load_async<D, 32>(gg + row0 * prm.dos[2], prm.dos[2], wv, lane, sa + C::TILE_BYTES);
+    }
+    stat_load_async((wv == 0 ? lse_h : dlt_h) + rb * 64, stat_lane, sa + 2 * C::TILE_BYTES + wv * 256);   // all 64 rows of the tile
     if constexpr (EW)   // the tile's 64 mask words (one per key, bit = query), 256 bytes per wavefront
       stat_load_async(reinterpret_cast<const float*>(prm.bits_cols + (int64_t)t * 64) + wv * 64, lane,
                       sa + 2 * C::TILE_BYTES + C::STAT_BYTES + wv * 256);
@@ -388,8 +439,10 @@ __global__ __launch_bounds__(128, (QB == 1 && D == 64) ? 2 : 1) void dkdv_kernel
   if (u0 < u1) issue(u0, 0);
 
   const int64_t krow = (int64_t)n * 64 + 32 * wv + ln;
-  const unsigned short* kp = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1] + krow * prm.ks[2];
-  const unsigned short* vp = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1] + krow * prm.vs[2];
+  const bool exists = !TAIL || krow < prm.N;
+  const int64_t ksrc = exists ? krow : prm.N - 1;
+  const unsigned short* kp = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1] + ksrc * prm.ks[2];
+  const unsigned short* vp = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1] + ksrc * prm.vs[2];
   uintx4 kfr[KS], vfr[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -408,180 +461,78 @@ __global__ __launch_bounds__(128, (QB == 1 && D == 64) ? 2 : 1) void dkdv_kernel
     const int stage = (u - u0) & 1;
     wait_vm<0>();
     __syncthreads();
+    const bool tail_step = TAIL && !EW && blk_issued == nb - 1;
     if (u + 1 < u1) issue(u + 1, stage ^ 1);
     const unsigned char* qt = lds + stage * C::STAGE_BYTES;
     const unsigned char* gt = qt + C::TILE_BYTES;
-    const int qoff = QB == 1 ? 32 * (u % STEPS) : 0;            // first query of this step within the tile
+    const int qoff = 32 * (u % STEPS);            // first query of this step within the tile
     const float* st_lse = reinterpret_cast<const float*>(gt + C::TILE_BYTES) + qoff;
     const float* st_dlt = st_lse + 64;
 
-    if constexpr (QB == 2) {
-      // Whole tile per step, one query block after the other, so that the vector work on one query
-      // block (P and dS) sits beside matrix work on the other: scores of block 0; scores of block 1
-      // beside P, dS of block 0; second products of block 0 beside P, dS of block 1; second
-      // products of block 1.
-      floatx16 sacc[2], dpacc[2];
-      uintx4 pf[4], dsf[4];
-      uintx4 fq[KS], fg[KS];
-      auto read_rows = [&](int qb) {
+    // operand fragments are read from LDS ahead of the block of MFMAs that consumes them
+    floatx16 sacc = zero16(), dpacc = zero16();
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          fq[s] = frag_rows<D>(qt, 32 * qb, s, ln, g);
-          fg[s] = frag_rows<D>(gt, 32 * qb, s, ln, g);
-        }
-      };
-      auto first = [&](int qb) {
-        sacc[qb] = zero16(); dpacc[qb] = zero16();
+    for (int pt = 0; pt < PORTIONS; ++pt) {
+      uintx4 fq[KSP], fg[KSP];
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-          sacc[qb] = mfma_qk<BF16>(fq[s], kfr[s], sacc[qb]);      // S = Q K^T
-          dpacc[qb] = mfma_qk<BF16>(fg[s], vfr[s], dpacc[qb]);    // dP = dO V^T
-        }
-      };
-      unsigned long long mw = 0ull;
-      if constexpr (EW)
-        mw = *reinterpret_cast<const unsigned long long*>(gt + C::TILE_BYTES + C::STAT_BYTES + (32 * wv + ln) * 8) >> (4 * g);
-      auto p_and_ds = [&](int qb) {          // rows of the results are queries: register i <-> query 32qb + 8(i/4) + 4g + i%4
-        if constexpr (EW) mask_scores(sacc[qb], (unsigned)(mw >> (32 * qb)));
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-          for (int jh = 0; jh < 2; ++jh) {
-            const int ts = 2 * qb + t2, i0 = 8 * t2 + 4 * jh;
-            const int q0 = 32 * qb + 8 * (i0 >> 2) + 4 * g;
-            const floatx4 l4 = *reinterpret_cast<const floatx4*>(st_lse + q0);
-            const floatx4 d4 = *reinterpret_cast<const floatx4*>(st_dlt + q0);
-            float p[4], ds[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float nl = EW && l4[e] == -INFINITY ? -INFINITY : -l4[e] * kLog2e;
-              p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[qb][i0 + e], qk_scale, nl));
-              ds[e] = p[e] * (dpacc[qb][i0 + e] - d4[e]);
-            }
-            pf[ts][2 * jh] = pack2<PB>(p[0], p[1]);   pf[ts][2 * jh + 1] = pack2<PB>(p[2], p[3]);
-            dsf[ts][2 * jh] = pack2<PB>(ds[0], ds[1]); dsf[ts][2 * jh + 1] = pack2<PB>(ds[2], ds[3]);
-          }
-      };
-      uintx4 fgt[2][DB], fqt[2][DB];
-      auto read_cols = [&](int qb) {
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            fgt[t2][db] = frag_cols<D, BF16 && !PB>(gt, DB0 + db, 2 * qb + t2, lane);
-            fqt[t2][db] = frag_cols<D, BF16 && !PB>(qt, DB0 + db, 2 * qb + t2, lane);
-          }
-      };
-      auto second = [&](int qb) {
-#pragma unroll
-        for (int t2 = 0; t2 < 2; ++t2)
-#pragma unroll
-          for (int db = 0; db < DB; ++db) {
-            dvacc[db] = mfma_qk<PB>(fgt[t2][db], pf[2 * qb + t2], dvacc[db]);    // dV^T += dO^T P
-            dkacc[db] = mfma_qk<PB>(fqt[t2][db], dsf[2 * qb + t2], dkacc[db]);   // dK^T += Q^T dS
-          }
-      };
-      read_rows(0);
-      __builtin_amdgcn_sched_barrier(0);
-      first(0);
-      __builtin_amdgcn_sched_barrier(0);
-      read_rows(1);
-      read_cols(0);
-      __builtin_amdgcn_sched_barrier(0);
-      first(1);
-      p_and_ds(0);
-#pragma unroll
-      for (int it = 0; it < 2 * KS; ++it) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+      for (int s = 0; s < KSP; ++s) {
+        fq[s] = frag_rows<D>(qt, 0, pt * KSP + s, ln, g);
+        fg[s] = frag_rows<D>(gt, 0, pt * KSP + s, ln, g);
       }
       __builtin_amdgcn_sched_barrier(0);
-      second(0);
-      p_and_ds(1);
 #pragma unroll
-      for (int it = 0; it < 4 * DB; ++it) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 7, 0);
+      for (int s = 0; s < KSP; ++s) {
+        sacc = mfma_qk<BF16>(fq[s], kfr[pt * KSP + s], sacc);      // S = Q K^T
+        dpacc = mfma_qk<BF16>(fg[s], vfr[pt * KSP + s], dpacc);    // dP = dO V^T
       }
       __builtin_amdgcn_sched_barrier(0);
-      read_cols(1);
-      __builtin_amdgcn_sched_barrier(0);
-      second(1);
-    } else {
-      // operand fragments are read from LDS ahead of the block of MFMAs that consumes them
-      floatx16 sacc[QB], dpacc[QB];
-  #pragma unroll
-      for (int qb = 0; qb < QB; ++qb) { sacc[qb] = zero16(); dpacc[qb] = zero16(); }
-  #pragma unroll
-      for (int pt = 0; pt < PORTIONS; ++pt) {
-        uintx4 fq[QB][KSP], fg[QB][KSP];
-  #pragma unroll
-        for (int s = 0; s < KSP; ++s)
-  #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            fq[qb][s] = frag_rows<D>(qt, 32 * qb, pt * KSP + s, ln, g);
-            fg[qb][s] = frag_rows<D>(gt, 32 * qb, pt * KSP + s, ln, g);
-          }
-        __builtin_amdgcn_sched_barrier(0);
-  #pragma unroll
-        for (int s = 0; s < KSP; ++s)
-  #pragma unroll
-          for (int qb = 0; qb < QB; ++qb) {
-            sacc[qb] = mfma_qk<BF16>(fq[qb][s], kfr[pt * KSP + s], sacc[qb]);      // S = Q K^T
-            dpacc[qb] = mfma_qk<BF16>(fg[qb][s], vfr[pt * KSP + s], dpacc[qb]);    // dP = dO V^T
-          }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if constexpr (EW) {
-        unsigned long long mw = *reinterpret_cast<const unsigned long long*>(
-            gt + C::TILE_BYTES + C::STAT_BYTES + (32 * wv + ln) * 8);
-        if constexpr (QB == 1) mw >>= qoff;
-        mw >>= 4 * g;
-        if constexpr (QB == 2) mask_scores(sacc[0], sacc[1], mw);
-        else mask_scores(sacc[0], (unsigned)mw);
-      }
-      // dO^T and Q^T fragments of the second products, read under the exponentials below
-      uintx4 fgt[2 * QB][DB], fqt[2 * QB][DB];
-  #pragma unroll
-      for (int ts = 0; ts < 2 * QB; ++ts)
-  #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-          fgt[ts][db] = frag_cols<D, BF16 && !PB>(gt, DB0 + db, ts, lane);
-          fqt[ts][db] = frag_cols<D, BF16 && !PB>(qt, DB0 + db, ts, lane);
-        }
-      __builtin_amdgcn_sched_barrier(0);
-      // rows of the results are queries: register i of block qb <-> query 32qb + 8(i/4) + 4g + i%4
-      uintx4 pf[2 * QB], dsf[2 * QB];
-  #pragma unroll
-      for (int ts = 0; ts < 2 * QB; ++ts)
-  #pragma unroll
-        for (int jh = 0; jh < 2; ++jh) {
-          const int qb = ts >> 1, i0 = 8 * (ts & 1) + 4 * jh;
-          const int q0 = 32 * qb + 8 * (i0 >> 2) + 4 * g;
-          const floatx4 l4 = *reinterpret_cast<const floatx4*>(st_lse + q0);
-          const floatx4 d4 = *reinterpret_cast<const floatx4*>(st_dlt + q0);
-          float p[4], ds[4];
-  #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            // (a query without any unmasked key has lse = -inf: its P must come out as 0)
-            const float nl = EW && l4[e] == -INFINITY ? -INFINITY : -l4[e] * kLog2e;
-            p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[qb][i0 + e], qk_scale, nl));
-            ds[e] = p[e] * (dpacc[qb][i0 + e] - d4[e]);
-          }
-          pf[ts][2 * jh] = pack2<PB>(p[0], p[1]);   pf[ts][2 * jh + 1] = pack2<PB>(p[2], p[3]);
-          dsf[ts][2 * jh] = pack2<PB>(ds[0], ds[1]); dsf[ts][2 * jh + 1] = pack2<PB>(ds[2], ds[3]);
-        }
-  #pragma unroll
-      for (int ts = 0; ts < 2 * QB; ++ts)
-  #pragma unroll
-        for (int db = 0; db < DB; ++db) {
-          dvacc[db] = mfma_qk<PB>(fgt[ts][db], pf[ts], dvacc[db]);    // dV^T += dO^T P
-          dkacc[db] = mfma_qk<PB>(fqt[ts][db], dsf[ts], dkacc[db]);   // dK^T += Q^T dS
-        }
-  
     }
+    if constexpr (EW) {
+      unsigned long long mw = *reinterpret_cast<const unsigned long long*>(
+          gt + C::TILE_BYTES + C::STAT_BYTES + (32 * wv + ln) * 8);
+      mask_scores(sacc, (unsigned)(mw >> (qoff + 4 * g)));
+    }
+    if (tail_step) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> qoff));
+    // dO^T and Q^T fragments of the second products, read under the exponentials below
+    uintx4 fgt[2][DB], fqt[2][DB];
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        fgt[ts][db] = frag_cols<D, BF16 && !PB>(gt, DB0 + db, ts, lane);
+        fqt[ts][db] = frag_cols<D, BF16 && !PB>(qt, DB0 + db, ts, lane);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+    // rows of the results are queries: register i <-> query 8(i/4) + 4g + i%4
+    uintx4 pf[2], dsf[2];
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+      for (int jh = 0; jh < 2; ++jh) {
+        const int i0 = 8 * ts + 4 * jh, q0 = 8 * (i0 >> 2) + 4 * g;
+        const floatx4 l4 = *reinterpret_cast<const floatx4*>(st_lse + q0);
+        const floatx4 d4 = *reinterpret_cast<const floatx4*>(st_dlt + q0);
+        float p[4], ds[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          // (a query without any unmasked key has lse = -inf: its P must come out as 0)
+          const float nl = EW && l4[e] == -INFINITY ? -INFINITY : -l4[e] * kLog2e;
+          p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[i0 + e], qk_scale, nl));
+          ds[e] = p[e] * (dpacc[i0 + e] - d4[e]);
+        }
+        pf[ts][2 * jh] = pack2<PB>(p[0], p[1]);   pf[ts][2 * jh + 1] = pack2<PB>(p[2], p[3]);
+        dsf[ts][2 * jh] = pack2<PB>(ds[0], ds[1]); dsf[ts][2 * jh + 1] = pack2<PB>(ds[2], ds[3]);
+      }
+#pragma unroll
+    for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        dvacc[db] = mfma_qk<PB>(fgt[ts][db], pf[ts], dvacc[db]);    // dV^T += dO^T P
+        dkacc[db] = mfma_qk<PB>(fqt[ts][db], dsf[ts], dkacc[db]);   // dK^T += Q^T dS
+      }
   }
 
+  if (!exists) return;
   if (prm.split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
     const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
@@ -676,7 +627,7 @@ __device__ __forceinline__ uintx4 three_pieces(float x, bool holder) {
 }
 
 constexpr int DKDV4_LDS_BYTES = 4 * 64 * 2 * 128 + 4 * 4096;   // two stages of a Q and a dO tile, 4 KB of exchange per wavefront
-template <int D, bool BF16, bool PB, bool EW>
+template <int D, bool BF16, bool PB, bool EW, bool TAIL>
 __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   static_assert(D == 128, "two 32-column blocks of dK and dV per wavefront");
   constexpr int KS = D / 16, DBW = D / 64;           // 32-column blocks per wavefront
@@ -698,8 +649,11 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   // The K and V rows this wavefront owns for the whole walk depend on the block index only: asked for first, they
   // travel while the list is looked up and the first tiles are requested.
   const int64_t krow = (int64_t)n * 64 + 32 * kh + ln;
-  const unsigned short* kp = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1] + krow * prm.ks[2];
-  const unsigned short* vp = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1] + krow * prm.vs[2];
+  const bool exists = !TAIL || krow < prm.N;
+  const int64_t ksrc = exists ? krow : prm.N - 1;
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64;
+  const unsigned short* kp = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1] + ksrc * prm.ks[2];
+  const unsigned short* vp = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1] + ksrc * prm.vs[2];
   uintx4 kfr[KS], vfr[KS];
 #pragma unroll
   for (int s = 0; s < KS; ++s) {
@@ -718,10 +672,17 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   const float* lse_h = prm.lse + (int64_t)bh * prm.N;
   const float* dlt_h = prm.delta + (int64_t)bh * prm.N;
   const float inv_scale = 1.0f / prm.sm_scale;
+  int blk_issued = 0;        // (TAIL) row block of the step issued last
   // tile copies of step u into `stage`
   auto issue = [&](int u, int stage) {
     const int rb = rows[u];
     const unsigned sa = lds_addr + stage * STAGE_BYTES;
+    blk_issued = rb;
+    if (TAIL && rb == nb - 1) {
+      tail_tile_load_async<4, D, 64>(qg + (int64_t)rb * 64 * prm.qs[2], prm.qs[2], 0, valid, wv, lane, sa);
+      tail_tile_load_async<4, D, 64>(gg + (int64_t)rb * 64 * prm.dos[2], prm.dos[2], 0, valid, wv, lane, sa + TILE_BYTES);
+      return;
+    }
     part_tile_load_async<4, D, 64>(qg + (int64_t)rb * 64 * prm.qs[2], prm.qs[2], wv, lane, sa);
     part_tile_load_async<4, D, 64>(gg + (int64_t)rb * 64 * prm.dos[2], prm.dos[2], wv, lane, sa + TILE_BYTES);
   };
@@ -733,7 +694,8 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   float st_lse = 0.f, st_dlt = 0.f;
   unsigned long long st_bits = 0ull;
   auto ask_stats = [&](int u) {
-    const int q = rows[u] * 64 + 32 * dh + ln;
+    int q = rows[u] * 64 + 32 * dh + ln;
+    if (TAIL && q >= prm.N) q = prm.N - 1;
     st_lse = lse_h[q];
     st_dlt = dlt_h[q];
     if constexpr (EW) st_bits = prm.bits_cols[(int64_t)u * 64 + 32 * kh + ln];
@@ -786,6 +748,7 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
     // 8(i/4) + i%4 belongs to register i
     const unsigned mw = EW ? (unsigned)(st_bits >> (32 * dh)) >> (4 * g) : 0u;
     __builtin_amdgcn_sched_barrier(0);
+    const bool tail_step = TAIL && !EW && blk_issued == nb - 1;
     if (u + 1 < u1) { ask_stats(u + 1); issue(u + 1, stage ^ 1); }
     const unsigned char* qt = lds + stage * STAGE_BYTES;
     const unsigned char* gt = qt + TILE_BYTES;
@@ -814,6 +777,7 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
       dpacc = mfma_qk<BF16>(dlt_slice, ones_frag, dpacc);
     }
     if constexpr (EW) mask_scores(sacc, mw);
+    if (tail_step) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> (32 * dh)));
     // (the fragments of the own block's second products are on their way while the vector ALU works)
     uintx4 fgt_own[2][DBW], fqt_own[2][DBW];
     read_cols(qt, gt, dh, fgt_own, fqt_own);
@@ -852,6 +816,7 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   }
 
   if (prm.split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
+    if (!exists) return;
     const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
     for (int db = 0; db < DBW; ++db)
@@ -876,10 +841,11 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   unsigned char* mine = lds + wv * 2 * OUT_BYTES;
   const int64_t r0 = (int64_t)n * 64 + 32 * kh;
   const float sc = prm.sm_scale;
+  const int rows_here = TAIL ? prm.N - (int)r0 : 32;
   rows_out<BF16, 32 * DBW>(mine, prm.dk, b * prm.dks[0] + h * prm.dks[1] + r0 * prm.dks[2] + 32 * DBW * dh, prm.dks[2],
-                           prm.out_f32, lane_out, [&](int db, int i) { return dkacc[db][i] * sc; });
+                           prm.out_f32, lane_out, rows_here, [&](int db, int i) { return dkacc[db][i] * sc; });
   rows_out<BF16, 32 * DBW>(mine + OUT_BYTES, prm.dv, b * prm.dvs[0] + h * prm.dvs[1] + r0 * prm.dvs[2] + 32 * DBW * dh, prm.dvs[2],
-                           prm.out_f32, lane_out, [&](int db, int i) { return dvacc[db][i]; });
+                           prm.out_f32, lane_out, rows_here, [&](int db, int i) { return dvacc[db][i]; });
 }
 
 // ---------------------------------------------------------------------------------------
@@ -911,7 +877,7 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 // Workgroups per row / column list.  One is enough when the launch has at least four workgroups
 // per compute unit; a single long head would otherwise walk its lists on a fraction of the GPU.
 static int bwd_split(int B, int H, int N) {
-  const int64_t lists = (int64_t)B * H * (N / 64), want = 4 * (int64_t)compute_units();
+  const int64_t lists = (int64_t)B * H * ((N + 63) / 64), want = 4 * (int64_t)compute_units();
   if (lists >= want) return 1;
   int64_t s = (want + lists - 1) / lists;
   const int cap = N / 64 / 8 > 1 ? N / 64 / 8 : 1;        // a share should have a few tiles even in a dense list
@@ -919,13 +885,16 @@ static int bwd_split(int B, int H, int N) {
   return (int)(s > 8 ? 8 : s);
 }
 
+// floats in front of the parts (the parts are accessed 16 bytes at a time)
+static size_t delta_floats(int B, int H, int N) { return ((size_t)B * H * N + 63) & ~(size_t)63; }
+
 size_t bwd_workspace_bytes(int B, int H, int N, int D) {
-  const size_t delta = (size_t)B * H * N * sizeof(float);
+  const size_t delta = delta_floats(B, H, N) * sizeof(float);
   const int split = bwd_split(B, H, N);
   return delta + (split > 1 ? (size_t)3 * split * B * H * N * D * sizeof(float) : 0);   // + parts of dQ, dK, dV
 }
 
-template <int D, bool BF16, bool EW, bool PB>
+template <int D, bool BF16, bool EW, bool PB, bool TAIL>
 static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
   using C = BwdCfg<D, EW>;
   constexpr int KB = D >= 128 ? 1 : 2;          // dq_kernel walks D >= 128 tiles in two halves (no gain at D = 64: two wavefronts per SIMD anyway)
@@ -933,35 +902,34 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
   // dkdv_kernel (D = 64 and 256; D = 128 runs dkdv4_kernel): halves at D = 64 (191 instead of 318 registers: two
   // wavefronts per SIMD; B*H = 32 N = 8192 dense block-causal backward 1417 -> 1167 us); at D = 256 halves too, and
   // the head dimension of dK, dV in two launches.
-  constexpr int QB = 1;
-  using CK = BwdCfg<D, EW, 32 * QB>;
+  using CK = BwdCfg<D, EW, 32>;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dq_kernel<D, BF16, EW, PB, KB>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dq_kernel<D, BF16, EW, PB, KB, TAIL>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, CQ::LDS_BYTES);
     if constexpr (D == 256) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, QB, 0>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, 0, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, QB, 1>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, 1, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
     } else if constexpr (D == 128) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, DKDV4_LDS_BYTES);
     } else {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, QB, -1>),
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, -1, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
     }
   });
   const int BH = prm.B * prm.H;
   const int grid = ((BH + 7) / 8) * 8 * prm.nb * prm.split;   // heads in groups of 8, the last group padded
-  hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
+  hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
   if constexpr (D == 256) {   // the two halves of the head dimension of dK, dV in two launches
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, QB, 0>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, QB, 1>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
+    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, 0, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
+    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, 1, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   } else if constexpr (D == 128) {   // D = 128: four wavefronts per column block, two per SIMD
-    hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW>), dim3(grid), dim3(256), DKDV4_LDS_BYTES, st, prm);
+    hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), DKDV4_LDS_BYTES, st, prm);
   } else {
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, QB, -1>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
+    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, -1, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   }
   if (prm.split > 1) {
     const int64_t quads = (int64_t)BH * prm.N * D / 4;
@@ -979,12 +947,12 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   prm.dq = dq; prm.dk = dk; prm.dv = dv;
   prm.row_ptr = row_ptr; prm.col_idx = col_idx; prm.col_ptr = col_ptr; prm.row_idx = row_idx;
   prm.bits_rows = (const unsigned long long*)bits_rows; prm.bits_cols = (const unsigned long long*)bits_cols;
-  prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = s.N / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
+  prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   prm.out_f32 = s.out_dtype == BSATTN_F32;
   prm.split = bwd_split(s.B, s.H, s.N);
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
-    prm.part_dq = (float*)ws + (size_t)s.B * s.H * s.N;
+    prm.part_dq = (float*)ws + delta_floats(s.B, s.H, s.N);
     prm.part_dk = prm.part_dq + one;
     prm.part_dv = prm.part_dk + one;
   }
@@ -1000,21 +968,26 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   // bf16 inputs keep P and dS in fp16.
   const bool pb = bf && !prm.out_f32;
   const bool ew = bits_rows != nullptr;
-  auto pick = [&](auto dc) {
+  auto pick = [&](auto dc, auto tail) {
     constexpr int DD = decltype(dc)::value;
+    constexpr bool TL = decltype(tail)::value;
     if (!ew) {
-      if (!bf) launch_bwd_t<DD, false, false, false>(prm, st);
-      else if (pb) launch_bwd_t<DD, true, false, true>(prm, st);
-      else launch_bwd_t<DD, true, false, false>(prm, st);
+      if (!bf) launch_bwd_t<DD, false, false, false, TL>(prm, st);
+      else if (pb) launch_bwd_t<DD, true, false, true, TL>(prm, st);
+      else launch_bwd_t<DD, true, false, false, TL>(prm, st);
     } else {   // elementwise mask
-      if (!bf) launch_bwd_t<DD, false, true, false>(prm, st);
-      else if (pb) launch_bwd_t<DD, true, true, true>(prm, st);
-      else launch_bwd_t<DD, true, true, false>(prm, st);
+      if (!bf) launch_bwd_t<DD, false, true, false, TL>(prm, st);
+      else if (pb) launch_bwd_t<DD, true, true, true, TL>(prm, st);
+      else launch_bwd_t<DD, true, true, false, TL>(prm, st);
     }
   };
-  if (s.D == 64) pick(std::integral_constant<int, 64>{});
-  else if (s.D == 128) pick(std::integral_constant<int, 128>{});
-  else pick(std::integral_constant<int, 256>{});
+  auto pick_tail = [&](auto dc) {
+    if (s.N % 64 == 0) pick(dc, std::false_type{});
+    else pick(dc, std::true_type{});
+  };
+  if (s.D == 64) pick_tail(std::integral_constant<int, 64>{});
+  else if (s.D == 128) pick_tail(std::integral_constant<int, 128>{});
+  else pick_tail(std::integral_constant<int, 256>{});
   return launch_status();
 }
 

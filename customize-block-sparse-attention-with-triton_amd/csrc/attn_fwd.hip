@@ -49,6 +49,10 @@ template <int D> struct FwdCfg {
   static constexpr int COLS_CAP = 2048;                     // column indices of the range kept in LDS
   static constexpr int BITS_OFF = NW * WAVE_LDS + ML_BYTES + COLS_CAP * 4;   // mask words of the current tile, 512 bytes per wavefront
   static constexpr int LDS_BYTES = BITS_OFF + NW * 512;
+  // one wavefront per workgroup (ROWS): eight workgroups share the 160 KB of a compute unit
+  static constexpr int ROWS_COLS_CAP = 896;
+  static constexpr int ROWS_BITS_OFF = WAVE_LDS + ROWS_COLS_CAP * 4;
+  static constexpr int ROWS_LDS_BYTES = ROWS_BITS_OFF + 512;
   static constexpr int R = WAVE_LDS / 256;                  // accumulator registers exchanged per round (K and V buffer)
   static constexpr int ROUNDS = D / R;
   static constexpr int QPW = (R / 4) / NW;                  // output quads per wavefront and round
@@ -57,13 +61,26 @@ template <int D> struct FwdCfg {
 };
 
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
-// CONTIG: the rows of K and of V follow each other without gaps (row stride = D).
-template <int D, int DT, bool ROWS, bool EW, bool CONTIG>
-__global__ __launch_bounds__(FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
+// MODE.  COOP: the ranges of four-wavefront workgroups described above (launches with few row blocks).  ROWS: a workgroup
+// is one wavefront and takes one row block (many row blocks: nothing to merge, the dispatcher balances the load).
+// WAVE: a workgroup is one wavefront and takes one range of its head's list (in between: about as many row blocks as
+// wavefronts fit the GPU, which whole row blocks would leave half idle in a second round).
+// LAYOUT: GENERAL any strides, any number of tokens; CONTIG_WHOLE the rows of K and of V follow each other without gaps
+// (row stride = D) and N is a multiple of 64; CONTIG_TAIL without gaps, any N; STRIDED_WHOLE any strides, N a multiple of 64
+// (D = 128, where the code for the rest costs registers that are not there).
+// Where N is not a multiple of 64 the last tile of a row list holds `valid` < 64 keys: its copy repeats the last
+// key (no address lies beyond the tensor) and its scores beyond `valid` are set to -inf; the query rows of the last
+// row block beyond N repeat the last query and are not written.
+enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2, STRIDED_WHOLE = 3 };
+enum { COOP = 0, ROWS_MODE = 1, WAVE = 2 };
+template <int D, int DT, int MODE, bool EW, int LAYOUT>
+__global__ __launch_bounds__(MODE != COOP ? 64 : FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
 void fwd_kernel(const FwdParams prm) {
   constexpr bool BF16 = DT != 0, PB = DT == 2;
+  constexpr bool CONTIG = LAYOUT == CONTIG_WHOLE || LAYOUT == CONTIG_TAIL, TAIL = LAYOUT == GENERAL || LAYOUT == CONTIG_TAIL;
   using C = FwdCfg<D>;
-  constexpr int NW = C::NW;
+  constexpr bool ROWS = MODE == ROWS_MODE, ONE = MODE != COOP;     // ONE: one wavefront per workgroup
+  constexpr int NW = ONE ? 1 : C::NW;
   constexpr bool FOLD = !BF16;     // fp16: scale folded into Q, reference exponent via an extra MFMA slice
   constexpr int KS = D / 16;       // k-slices of the first product
   constexpr int DB = D / 32;       // 32-wide blocks of the head dimension
@@ -76,79 +93,94 @@ void fwd_kernel(const FwdParams prm) {
   const int ln = lane & 31, g = lane >> 5;
   // linear id -> (head, range): heads interleaved, so that every head gets its share of the
   // workgroups that are first on their compute unit
-  const int BH = prm.B * prm.H;
-  const int bh = blockIdx.x % BH;
-  int wg = blockIdx.x / BH;
+  const int BH = prm.B * prm.H, nb = prm.nb;
+  int bh, wg;
+  if constexpr (ROWS) {
+    // (head, row block): heads in groups of 8, one per XCD (workgroups go to the XCDs round-robin), so that the row
+    // blocks at work on an XCD share the K and V of one head in its L2; the last row blocks, the long ones of
+    // block-causal masks, first
+    const int L = blockIdx.x, grp = L / (8 * nb), l = L - grp * 8 * nb, hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;
+    bh = 8 * grp + l % hg;
+    wg = nb - 1 - l / hg;
+    if (wg < 0) return;                // padding of an incomplete last group
+  } else {
+    bh = blockIdx.x % BH;
+    wg = blockIdx.x / BH;
+  }
   const int b = bh / prm.H, h = bh % prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
-  const int nb = prm.nb;
+  // keys of the last tile column; its column block (-1: every tile is whole)
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64;
+  const int tail_cb = TAIL && valid < 64 ? nb - 1 : -1;
   // the lists are read-only for the whole launch: constant address space => scalar loads
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
-  HeadSplit hs = head_split(rp, nb, prm.W, /*min_tiles=*/NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
-  // Long ranges (the regime of the weighted shares) are cut on the axis with gaps and boundaries move to a row
-  // block's end only from very close; short ranges are cut on the plain tile axis and their boundaries move to
-  // the nearer end of a row block from up to half a range (and at least SNAP tiles) away: a row block is shared
-  // only where a boundary falls into its middle, row blocks of up to a range's length or 2 SNAP tiles never (N = 17536,
-  // one head, against 8 tiles for every head: keep 0.15 36.0 -> 31.4 us, keep 0.2 40.0 -> 34.6, keep 0.25 43.2 -> 39.8,
-  // keep 0.05 21.8 -> 20.2, keep 0.1 25.8 -> 25.1; keep 0.35 and above, other sizes: +-1 %).
-  constexpr int LONG_GAP = 12, LONG_SNAP = 2;
-  const bool long_ranges = !ROWS && ((int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff || hs.Peff >= 3 * nb);   // (or row blocks much longer than the ranges)
-  // (D = 128, one workgroup per compute unit and tiles twice as long: sharing a row block is cheaper against the
-  // imbalance it avoids; 8 tiles for every head.  Half a range there: keep 0.1 87 -> 98 us, keep 0.15 107 -> 129 us.)
-  const int half_range = hs.T / (2 * (hs.Peff > 0 ? hs.Peff : 1)) + 1;
-  // (long ranges over short row blocks, up to 32 tiles on average: a boundary moves to the nearer end of its row block
-  // from up to half such a row block away, so that next to no row block is shared; against 2 tiles: 8 heads of
-  // N = 17536 at keep 0.05 67.9 -> 62 us, 4 heads at keep 0.1 57.9 -> 54.6 us; with longer row blocks the imbalance
-  // costs more than the sharing: keep 0.35, one head, 48.0 -> 50.4 us with 12 tiles)
-  const int avg_row = hs.T / (nb > 0 ? nb : 1);
-  const int long_snap = avg_row <= 32 ? avg_row / 2 + 1 : LONG_SNAP;
-  const int snap = long_ranges ? long_snap : (C::WG_PER_CU > 1 && half_range > C::SNAP ? half_range : C::SNAP);
-  // (ranges that are long only against the row blocks they lie in, several to a row block: 24 positions; N = 6400
-  // dense 31.2 -> 29.0 us, where 12 are best for N = 17536 dense, 102.1 against 104.0 us)
-  const int long_gap = (int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff ? LONG_GAP : 2 * LONG_GAP;
-  if (long_ranges) { hs.gap = long_gap; hs.X = (int64_t)hs.T + (int64_t)long_gap * nb; }
-  // Which range this workgroup takes (launches with few heads and long ranges): the ranges of a head start at
-  // all phases of a row, and workgroups that share an XCD, hence an L2, get ranges of like phase, so that they
-  // walk the same column blocks at the same time (dense N = 17536, one head: 42 instead of 196 MB fetched from
-  // HBM per launch, 104.5 instead of 106.6 us).  The phases are those of rows of equal length: heads that keep less
-  // than three quarters of their tiles are left alone (keep 0.5 measured 2 % slower with the permutation), except
-  // the dense block-causal mask, which has a table of its own (N = 32000: 185 instead of 193 us).
-  if (prm.perm_n > 0 && prm.perm_n == hs.Peff && prm.perm_fast == hs.fast) {
-    if (hs.T >= prm.perm_min_tiles) wg = prm.perm[wg];
-    // the dense block-causal mask (by its number of kept tiles and the length of one row in the middle; a mask
-    // taken for it by mistake merely gets its ranges in another order): ranges sorted by their first column block
-    else if ((int64_t)hs.T * 2 == (int64_t)nb * (nb + 1) && rp[nb / 2 + 1] - rp[nb / 2] == nb / 2 + 1) wg = prm.perm_causal[wg];
-  }
-  // Heads cut into equal shares: the two workgroups of a compute unit (linear ids L and L + first_ids: the
-  // dispatcher places them in the same order in both rounds) take neighbouring ranges 2k and 2k + 1.  A boundary that
-  // moves to a row block's end moves tiles from one range to its neighbour; between the two workgroups of a compute
-  // unit that changes nothing in what the compute unit has to do, and only every other boundary unbalances the
-  // compute units (keep 0.1, N = 17536: 26.2 -> 24.8 us; keep 0.25: 42.2 -> 41.6 us).  (All boundaries move by the
-  // same rule: one that may move further than its neighbours can overtake them.)
-  {
-    const int Fh = prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0;
-    if (!ROWS && hs.fast == 0 && hs.Peff == prm.W && prm.W == 2 * Fh) wg = wg < Fh ? 2 * wg : 2 * (wg - Fh) + 1;
-  }
-  // Row blocks without kept tiles belong to no range: they are dealt round-robin over all workgroups
-  // of the head, which write O = 0, lse = -inf for their share.  (With whole row blocks per
-  // wavefront the ranges are row-aligned and cover them, unless the head keeps nothing at all.)
-  if (!ROWS || hs.T == 0) {
-    for (int r0 = wg; r0 < nb; r0 += prm.W) {
-      if (rp[r0 + 1] > rp[r0]) continue;
-      void* ob = out_base(prm, b, h);
-      for (int i = threadIdx.x; i < 64 * (D / 4); i += NW * 64) {
-        const int64_t qrow = (int64_t)r0 * 64 + i / (D / 4);
-        store_out4<BF16>(ob, qrow * prm.os[2] + 4 * (i % (D / 4)), prm.out_f32, 0.f, 0.f, 0.f, 0.f);
-      }
-      if (prm.lse != nullptr && threadIdx.x < 64) prm.lse[(int64_t)bh * prm.N + (int64_t)r0 * 64 + threadIdx.x] = -INFINITY;
-    }
-  }
-  if (hs.T == 0 || wg >= hs.Peff) return;
-  // where the range begins and ends on the cutting axis (ROWS: the plain tile axis, as absolute tile offsets)
-  const int64_t x0 = split_pos(hs, wg), x1 = split_pos(hs, wg + 1);
-  int g0 = hs.lo + (int)x0, g1 = hs.lo + (int)x1;     // (ROWS; the other mode finds its tiles below)
+  HeadSplit hs;
+  int snap = 0;
+  int64_t x0 = 0, x1 = 0;
   if constexpr (!ROWS) {
+    hs = head_split(rp, nb, prm.W, /*min_tiles=*/ONE ? 4 : NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
+    // Long ranges (the regime of the weighted shares) are cut on the axis with gaps and boundaries move to a row
+    // block's end only from very close; short ranges are cut on the plain tile axis and their boundaries move to
+    // the nearer end of a row block from up to half a range (and at least SNAP tiles) away: a row block is shared
+    // only where a boundary falls into its middle, row blocks of up to a range's length or 2 SNAP tiles never (N = 17536,
+    // one head, against 8 tiles for every head: keep 0.15 36.0 -> 31.4 us, keep 0.2 40.0 -> 34.6, keep 0.25 43.2 -> 39.8,
+    // keep 0.05 21.8 -> 20.2, keep 0.1 25.8 -> 25.1; keep 0.35 and above, other sizes: +-1 %).
+    constexpr int LONG_GAP = MODE == WAVE ? 2 : 12, LONG_SNAP = 2;
+    const bool long_ranges = MODE == WAVE || ((int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff || hs.Peff >= 3 * nb);   // (or row blocks much longer than the ranges)
+    // (D = 128, one workgroup per compute unit and tiles twice as long: sharing a row block is cheaper against the
+    // imbalance it avoids; 8 tiles for every head.  Half a range there: keep 0.1 87 -> 98 us, keep 0.15 107 -> 129 us.)
+    const int half_range = hs.T / (2 * (hs.Peff > 0 ? hs.Peff : 1)) + 1;
+    // (long ranges over short row blocks, up to 32 tiles on average: a boundary moves to the nearer end of its row block
+    // from up to half such a row block away, so that next to no row block is shared; against 2 tiles: 8 heads of
+    // N = 17536 at keep 0.05 67.9 -> 62 us, 4 heads at keep 0.1 57.9 -> 54.6 us; with longer row blocks the imbalance
+    // costs more than the sharing: keep 0.35, one head, 48.0 -> 50.4 us with 12 tiles)
+    const int avg_row = hs.T / (nb > 0 ? nb : 1);
+    const int long_snap = MODE != WAVE && avg_row <= 32 ? avg_row / 2 + 1 : LONG_SNAP;
+    snap = long_ranges ? long_snap : (C::WG_PER_CU > 1 && half_range > C::SNAP ? half_range : C::SNAP);
+    // (ranges that are long only against the row blocks they lie in, several to a row block: 24 positions; N = 6400
+    // dense 31.2 -> 29.0 us, where 12 are best for N = 17536 dense, 102.1 against 104.0 us)
+    const int long_gap = MODE == WAVE || (int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff ? LONG_GAP : 2 * LONG_GAP;
+    if (long_ranges) { hs.gap = long_gap; hs.X = (int64_t)hs.T + (int64_t)long_gap * nb; }
+    // Which range this workgroup takes (launches with few heads and long ranges): the ranges of a head start at
+    // all phases of a row, and workgroups that share an XCD, hence an L2, get ranges of like phase, so that they
+    // walk the same column blocks at the same time (dense N = 17536, one head: 42 instead of 196 MB fetched from
+    // HBM per launch, 104.5 instead of 106.6 us).  The phases are those of rows of equal length: heads that keep less
+    // than three quarters of their tiles are left alone (keep 0.5 measured 2 % slower with the permutation), except
+    // the dense block-causal mask, which has a table of its own (N = 32000: 185 instead of 193 us).
+    if (MODE == COOP && prm.perm_n > 0 && prm.perm_n == hs.Peff && prm.perm_fast == hs.fast) {
+      if (hs.T >= prm.perm_min_tiles) wg = prm.perm[wg];
+      // the dense block-causal mask (by its number of kept tiles and the length of one row in the middle; a mask
+      // taken for it by mistake merely gets its ranges in another order): ranges sorted by their first column block
+      else if ((int64_t)hs.T * 2 == (int64_t)nb * (nb + 1) && rp[nb / 2 + 1] - rp[nb / 2] == nb / 2 + 1) wg = prm.perm_causal[wg];
+    }
+    // Heads cut into equal shares: the two workgroups of a compute unit (linear ids L and L + first_ids: the
+    // dispatcher places them in the same order in both rounds) take neighbouring ranges 2k and 2k + 1.  A boundary that
+    // moves to a row block's end moves tiles from one range to its neighbour; between the two workgroups of a compute
+    // unit that changes nothing in what the compute unit has to do, and only every other boundary unbalances the
+    // compute units (keep 0.1, N = 17536: 26.2 -> 24.8 us; keep 0.25: 42.2 -> 41.6 us).  (All boundaries move by the
+    // same rule: one that may move further than its neighbours can overtake them.)
+    {
+      const int Fh = prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0;
+      if (MODE == COOP && hs.fast == 0 && hs.Peff == prm.W && prm.W == 2 * Fh) wg = wg < Fh ? 2 * wg : 2 * (wg - Fh) + 1;
+    }
+    // Row blocks without kept tiles belong to no range: they are dealt round-robin over all workgroups
+    // of the head, which write O = 0, lse = -inf for their share.
+    {
+      for (int r0 = wg; r0 < nb; r0 += prm.W) {
+        if (rp[r0 + 1] > rp[r0]) continue;
+        void* ob = out_base(prm, b, h);
+        for (int i = threadIdx.x; i < 64 * (D / 4); i += NW * 64) {
+          const int64_t qrow = (int64_t)r0 * 64 + i / (D / 4);
+          if (TAIL && qrow >= prm.N) break;
+          store_out4<BF16>(ob, qrow * prm.os[2] + 4 * (i % (D / 4)), prm.out_f32, 0.f, 0.f, 0.f, 0.f);
+        }
+        if (prm.lse != nullptr && threadIdx.x < 64 && (!TAIL || r0 * 64 + (int)threadIdx.x < prm.N)) prm.lse[(int64_t)bh * prm.N + (int64_t)r0 * 64 + threadIdx.x] = -INFINITY;
+      }
+    }
+    if (hs.T == 0 || wg >= hs.Peff) return;
+    // where the range begins and ends on the cutting axis
+    x0 = split_pos(hs, wg); x1 = split_pos(hs, wg + 1);
     if (x0 >= x1) return;
   }
 
@@ -184,8 +216,9 @@ void fwd_kernel(const FwdParams prm) {
   auto v_copy = [&](const unsigned short* tile, int j) {
     tile_load_async_one(tile + (int64_t)j * RPI * prm.vs[2], voff[0], lds_v_addr + j * 1024);
   };
-  const unsigned lds_bits_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds + C::BITS_OFF + w * 512;
-  const unsigned long long* lds_bits = reinterpret_cast<const unsigned long long*>(lds + C::BITS_OFF + w * 512);
+  constexpr int BITS_OFF = ONE ? C::ROWS_BITS_OFF : C::BITS_OFF, COLS_CAP = ONE ? C::ROWS_COLS_CAP : C::COLS_CAP;
+  const unsigned lds_bits_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds + BITS_OFF + w * 512;
+  const unsigned long long* lds_bits = reinterpret_cast<const unsigned long long*>(lds + BITS_OFF + w * 512);
   constexpr int KOPS = CPR + (EW ? 2 : 0);      // instructions of one K copy
   // copy of the K tile `tile` = entry t of the kept-tile list (EW: with its 512 bytes of mask words)
   // CONTIG (rows that follow each other without gaps, the usual case): copy instruction j reads at
@@ -194,8 +227,23 @@ void fwd_kernel(const FwdParams prm) {
   // instructions per tile copy at D = 64).
   constexpr bool k_contig = CONTIG, v_contig = CONTIG;
   const int64_t k_rs = CONTIG ? (int64_t)D : prm.ks[2], v_rs = CONTIG ? (int64_t)D : prm.vs[2];   // row strides (a constant: a tile's address is a shift)
-  auto k_copy_all = [&](const unsigned short* tile, int t) {
-    if constexpr (k_contig) {
+  // copy of a tile whose last rows do not exist (`valid` of them do): every instruction's rows are bounded
+  // (the lane index as a value the compiler cannot trace back: the offsets would otherwise be computed before the
+  // tile loop and occupy registers throughout it)
+  auto tail_copy = [&](const unsigned short* tile, int64_t rs, unsigned lds_addr, auto&& swz) {
+    int lane_t = lane;
+    asm volatile("" : "+v"(lane_t));
+#pragma unroll 1
+    for (int j = 0; j < CPR; ++j) {
+      const int row = j * RPI + lane_t / CPR, src = row < valid ? row : valid - 1;
+      tile_load_async_one(tile, 2u * (unsigned)(src * (int)rs + (((lane_t % CPR) ^ swz(row)) * 8)), lds_addr + j * 1024);
+    }
+  };
+  auto k_copy_all = [&](int cb, int t) {
+    const unsigned short* tile = kg + (int64_t)cb * 64 * k_rs;
+    if (TAIL && cb == tail_cb) {
+      tail_copy(tile, k_rs, lds_k_addr, [](int row) { return k_swz<D>(row); });
+    } else if constexpr (k_contig) {
 #pragma unroll
       for (int jb = 0; jb < CPR; jb += 4)
         tile_load_async_four(tile + jb * RPI * D, koff[jb % KPER], koff[(jb + 1) % KPER], koff[(jb + 2) % KPER], koff[(jb + 3) % KPER],
@@ -212,8 +260,11 @@ void fwd_kernel(const FwdParams prm) {
                      :: "s"(lds_bits_addr + j * 256), "v"(4u * (unsigned)lane + 256u * j), "s"(src) : "memory", "m0");
     }
   };
-  auto v_copy_all = [&](const unsigned short* tile) {
-    if constexpr (v_contig) {
+  auto v_copy_all = [&](int cb) {
+    const unsigned short* tile = vg + (int64_t)cb * 64 * v_rs;
+    if (TAIL && cb == tail_cb) {
+      tail_copy(tile, v_rs, lds_v_addr, [](int row) { return v_swz<D>(row); });
+    } else if constexpr (v_contig) {
 #pragma unroll
       for (int jb = 0; jb < CPR; jb += 4)
         tile_load_async_four(tile + jb * RPI * D, voff[0], voff[0], voff[0], voff[0], lds_v_addr + jb * 1024);
@@ -262,10 +313,19 @@ void fwd_kernel(const FwdParams prm) {
     fresh = true;
     any_m = 0;
   };
+  // WAVE: per-lane addresses that do not change from row block to row block are not to be held through the tile loops:
+  // the lane index as a value the compiler cannot trace back
+  auto fresh_lane = [&](int x) {
+    if constexpr (MODE == WAVE) asm volatile("" : "+v"(x));
+    return x;
+  };
   auto load_q = [&](int r) {
+    const int lane_q = fresh_lane(lane), ln = lane_q & 31, g = lane_q >> 5;
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const unsigned short* qrow = qg + (int64_t)(r * 64 + qb * 32 + ln) * prm.qs[2];
+      int row = r * 64 + qb * 32 + ln;
+      if (TAIL && row >= prm.N) row = prm.N - 1;
+      const unsigned short* qrow = qg + (int64_t)row * prm.qs[2];
 #pragma unroll
       for (int s = 0; s < KS; ++s) qf[qb][s] = *reinterpret_cast<const uintx4*>(qrow + 16 * s + 8 * g);
     }
@@ -373,14 +433,21 @@ void fwd_kernel(const FwdParams prm) {
 #pragma unroll
       for (int s = 0; s < KS; ++s) kfr[kb][s] = *reinterpret_cast<const uintx4*>(lds_k + kaddr[kb][s]);
     // EW: the 64 mask bits of this lane's two queries, shifted so that bit 8(i/4) + i%4 (+ 32 for
-    // the second key block) is the key of score register i
+    // the second key block) is the key of score register i; without EW only a tile with missing keys is `partial`
     unsigned long long mw0 = 0ull, mw1 = 0ull;
     if constexpr (EW) {
       if (partial) { mw0 = lds_bits[ln] >> (4 * g); mw1 = lds_bits[32 + ln] >> (4 * g); }
     }
+    // (the count as a value the compiler cannot trace back, or the 32 tests of the word are made before the tile loop
+    // and held; made where it is used, so that it occupies no registers in between)
+    auto tail_word = [&]() {
+      int v = valid;                                              // < 64 here
+      asm volatile("" : "+s"(v));
+      return ((1ull << v) - 1ull) >> (4 * g);
+    };
     lds_wait();      // the K fragments have arrived: the K buffer is free
     mid();
-    if (has1) k_copy_all(kg + (int64_t)cbn * 64 * k_rs, tn);
+    if (has1) k_copy_all(cbn, tn);
     auto mask_scores = [&](floatx16& s0, floatx16& s1, unsigned long long mw) {
       const unsigned lo = (unsigned)mw, hi = (unsigned)(mw >> 32);
 #pragma unroll
@@ -393,7 +460,7 @@ void fwd_kernel(const FwdParams prm) {
     // [1]
     scores(0, sa0, sa1);
     mslice(0, sa0, sa1);
-    if constexpr (EW) { if (partial) mask_scores(sa0, sa1, mw0); }
+    if constexpr (EW || TAIL) { if (partial) mask_scores(sa0, sa1, EW ? mw0 : tail_word()); }
     __builtin_amdgcn_sched_barrier(0);
     // [2]
     scores(1, sb0, sb1);
@@ -410,14 +477,14 @@ void fwd_kernel(const FwdParams prm) {
     }
     __builtin_amdgcn_sched_barrier(0);
     mslice(1, sb0, sb1);
-    if constexpr (EW) { if (partial) mask_scores(sb0, sb1, mw1); }
+    if constexpr (EW || TAIL) { if (partial) mask_scores(sb0, sb1, EW ? mw1 : tail_word()); }
     settle(0, sa0, sa1, lnew0);
     if constexpr (!EARLY_V) {
       if (has1) wait_vm<KOPS>(); else wait_vm<0>();  // V(cur) has landed (K(nxt) may be in flight)
       read_v();
     }
     lds_wait();      // the V fragments have arrived: the V buffer is free
-    if (copy_v) v_copy_all(vg + (int64_t)cbn * 64 * v_rs);
+    if (copy_v) v_copy_all(cbn);
     // [3]
     second(0);
     float lnew1 = softmax_tile<FOLD, PB>(sb0, sb1, qk_scale, m_i[1], l_i[1], pf, 1);
@@ -474,7 +541,7 @@ void fwd_kernel(const FwdParams prm) {
   };
 
   int* ctr = reinterpret_cast<int*>(ml + NW * 2 * 64);
-  int* lcols = ctr + 16;
+  int* lcols = ONE ? reinterpret_cast<int*>(lds + C::WAVE_LDS) : ctr + 16;
   // The column indices of the range are staged in LDS: a scalar load per tile would put its whole
   // latency in front of the tile's first LDS wait (scalar loads return out of order, so any wait
   // on the shared counter becomes a wait for all of them).
@@ -486,17 +553,57 @@ void fwd_kernel(const FwdParams prm) {
     return c;
   };
   constexpr int COL_MASK = 0x3fffffff;
+  auto is_partial = [&](int c) { return EW ? (c >> 30) != 0 : TAIL && c == tail_cb; };
   auto stage_cols = [&](int t_lo, int t_hi) {
-    for (int i = threadIdx.x; i < t_hi - t_lo && i < C::COLS_CAP; i += NW * 64) {
+    for (int i = threadIdx.x; i < t_hi - t_lo && i < COLS_CAP; i += NW * 64) {
       int c = prm.col_idx[t_lo + i];
       if constexpr (EW) c |= (int)prm.tile_partial[t_lo + i] << 30;     // EW: "partly set" rides in bit 30
       lcols[i] = c;
     }
   };
 
+  void* obase = out_base(prm, b, h);
+  auto exists = [&](int64_t qrow) { return !TAIL || qrow < prm.N; };
+  // normalise and write a row block that this wavefront has run alone
+  auto write_row = [&](int row) {
+    const int lane_o = fresh_lane(lane), ln = lane_o & 31, g = lane_o >> 5;
+    float lsum[2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const float inv = lsum[qb] > 0.f ? 1.0f / lsum[qb] : 0.f;      // no unmasked key at all: O = 0
+      const int64_t qrow = (int64_t)(row * 64 + qb * 32 + ln);
+      if (!exists(qrow)) continue;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32,
+                           oacc[db][qb][4 * i4] * inv, oacc[db][qb][4 * i4 + 1] * inv,
+                           oacc[db][qb][4 * i4 + 2] * inv, oacc[db][qb][4 * i4 + 3] * inv);
+      if (prm.lse != nullptr && g == 0)
+        prm.lse[((int64_t)bh * prm.N) + qrow] =
+            lsum[qb] > 0.f ? (m_i[qb] + __builtin_amdgcn_logf(lsum[qb])) * 0.6931471805599453f : -INFINITY;
+    }
+  };
+  // row block without kept tiles: O = 0, lse = -inf
+  auto write_empty_row = [&](int row) {
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const int64_t qrow = (int64_t)(row * 64 + qb * 32 + ln);
+      if (!exists(qrow)) continue;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4)
+          store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, 0.f, 0.f, 0.f, 0.f);
+      if (prm.lse != nullptr && g == 0) prm.lse[((int64_t)bh * prm.N) + qrow] = -INFINITY;
+    }
+  };
+
   // Whole row blocks [r_lo, r_hi), one wavefront each: handed out through the LDS counter *rctr
   // (set to r_lo + 2 NW beforehand), written directly, nothing to merge.
-  void* obase = out_base(prm, b, h);
   auto run_rows = [&](int r_lo, int r_hi, int* rctr, auto&& col_of) {
     // Tickets r_lo, r_lo + 1, ... stand for the row blocks r_hi - 1, r_hi - 2, ...: with block-causal
     // masks the late row blocks are the long ones, and the long ones should not come last.
@@ -513,8 +620,8 @@ void fwd_kernel(const FwdParams prm) {
       if (ta < tb) {
         int cx = __builtin_amdgcn_readfirstlane(col_of(ta));      // current tile: column block | flag
         if (kdone != ta) {
-          k_copy_all(kg + (int64_t)(cx & COL_MASK) * 64 * k_rs, ta);
-          v_copy_all(vg + (int64_t)(cx & COL_MASK) * 64 * v_rs);
+          k_copy_all(cx & COL_MASK, ta);
+          v_copy_all(cx & COL_MASK);
         }
         reset_acc();
         load_q(row);
@@ -522,41 +629,13 @@ void fwd_kernel(const FwdParams prm) {
           const bool last = j + 1 == tb;
           const bool has1 = !last || next_has;
           const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(last ? tn : j + 1)) : 0;
-          tile(has1, cxn & COL_MASK, last ? tn : j + 1, has1, (cx >> 30) != 0, [] {});
+          tile(has1, cxn & COL_MASK, last ? tn : j + 1, has1, is_partial(cx), [] {});
           cx = cxn;
         }
         kdone = next_has ? tn : -1;
-        // normalise and write the row block
-        float lsum[2];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          const float inv = lsum[qb] > 0.f ? 1.0f / lsum[qb] : 0.f;      // no unmasked key at all: O = 0
-          const int64_t qrow = (int64_t)(row * 64 + qb * 32 + ln);
-#pragma unroll
-          for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4)
-              store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32,
-                               oacc[db][qb][4 * i4] * inv, oacc[db][qb][4 * i4 + 1] * inv,
-                               oacc[db][qb][4 * i4 + 2] * inv, oacc[db][qb][4 * i4 + 3] * inv);
-          if (prm.lse != nullptr && g == 0)
-            prm.lse[((int64_t)bh * prm.N) + qrow] =
-                lsum[qb] > 0.f ? (m_i[qb] + __builtin_amdgcn_logf(lsum[qb])) * 0.6931471805599453f : -INFINITY;
-        }
+        write_row(row);
       } else {
-        // row block without kept tiles: O = 0, lse = -inf
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          const int64_t qrow = (int64_t)(row * 64 + qb * 32 + ln);
-#pragma unroll
-          for (int db = 0; db < DB; ++db)
-#pragma unroll
-            for (int i4 = 0; i4 < 4; ++i4)
-              store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, 0.f, 0.f, 0.f, 0.f);
-          if (prm.lse != nullptr && g == 0) prm.lse[((int64_t)bh * prm.N) + qrow] = -INFINITY;
-        }
+        write_empty_row(row);
       }
       tick = tick_next;
       tick_next = __builtin_amdgcn_readfirstlane(drawn);
@@ -564,26 +643,152 @@ void fwd_kernel(const FwdParams prm) {
   };
 
   if constexpr (ROWS) {
-    // ================= one wavefront per row block =================
-    // The workgroup owns the row blocks whose first kept tile lies in its range [g0, g1); they are
-    // handed out to the wavefronts through the LDS counter, and a wavefront runs a whole row block
-    // alone and writes its result directly: no merge, no partials.
-    int r_lo, r_hi;
-    {
-      // smallest r with rp[r] >= g = number of r with rp[r] <= g - 1 (capped at nb)
-      int u0, u1, u2, u3;
-      count_le2(g0 - 1, g1 - 1, 0, r_lo, r_hi, u0, u1, u2, u3);
-      r_lo = r_lo < nb ? r_lo : nb;
-      r_hi = r_hi < nb ? r_hi : nb;
-      if (wg >= hs.Peff - 1) r_hi = nb;    // trailing row blocks without kept tiles
-      if (wg == 0) r_lo = 0;               // leading ones
+    // ================= one wavefront, one row block =================
+    const int ta = rp[wg], tb = rp[wg + 1];
+    if (ta == tb) { write_empty_row(wg); return; }
+    int cx = flagged_col(ta);                                  // current tile: column block | flag
+    k_copy_all(cx & COL_MASK, ta);
+    v_copy_all(cx & COL_MASK);
+    stage_cols(ta, tb);
+    auto col_of = [&](int t) { return t - ta < COLS_CAP ? lcols[t - ta] : flagged_col(t); };
+    reset_acc();
+    load_q(wg);
+    for (int j = ta; j < tb; ++j) {
+      const bool has1 = j + 1 < tb;
+      const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(j + 1)) : 0;
+      tile(has1, cxn & COL_MASK, j + 1, has1, is_partial(cx), [] {});
+      cx = cxn;
     }
-    const int t_lo = rp[r_lo];
-    stage_cols(t_lo, rp[r_hi]);
-    if (threadIdx.x == 0) *ctr = r_lo + 2 * NW;
-    __syncthreads();
-    auto col_of = [&](int t) { return t - t_lo < C::COLS_CAP ? lcols[t - t_lo] : flagged_col(t); };
-    run_rows(r_lo, r_hi, ctr, col_of);
+    write_row(wg);
+  } else if constexpr (MODE == WAVE) {
+    // ================= one wavefront, one range =================
+    // first row block of the range: largest r with rp[r] <= g0 < rp[r+1]
+    // A range boundary within `snap` tiles of an end of the row block it falls in moves to that end
+    // (the nearer one): sharing a row block costs a merge, a published part and a pull, several
+    // tiles' worth each, and row blocks of up to 2 `snap` tiles are never shared.  Every workgroup
+    // applies the same rule with the same distance to both of its boundaries, so the ranges still tile the list.
+    int r, g0, g1;
+    {
+      // the row blocks in which the two ends of the range lie (positions behind a row block's tiles count as
+      // its end), then the tiles themselves
+      int c0, c1, s0, e0, s1, e1;
+      count_le2(x0 + hs.lo, x1 + hs.lo, hs.gap, c0, c1, s0, e0, s1, e1);
+      r = c0 - 1;
+      g0 = tile_of_pos(hs, x0, r, s0, e0);
+      const int n0 = snap_boundary(snap, g0, s0, e0);
+      if (n0 >= e0) ++r;
+      g0 = n0;
+      if (x1 < hs.X) {
+        g1 = tile_of_pos(hs, x1, c1 - 1, s1, e1);
+        g1 = snap_boundary(snap, g1, s1, e1);
+      } else {
+        g1 = hs.lo + hs.T;
+      }
+      if (g0 >= g1) return;
+    }
+    int cx = flagged_col(g0);                                  // current tile: column block | flag
+    k_copy_all(cx & COL_MASK, g0);
+    v_copy_all(cx & COL_MASK);
+    stage_cols(g0, g1);
+    auto col_of = [&](int t) { return t - g0 < COLS_CAP ? lcols[t - g0] : flagged_col(t); };
+    int t = g0;
+    while (t < g1) {
+      const int row_s = rp[r], row_e = rp[r + 1];
+      if (row_e <= t) { ++r; continue; }          // row block without kept tiles in the range
+      const int seg_b = row_e < g1 ? row_e : g1;
+      reset_acc();
+      load_q(r);
+      for (int j = t; j < seg_b; ++j) {           // (the next tile is prefetched across the end of the row block)
+        const bool has1 = j + 1 < g1;
+        const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(j + 1)) : 0;
+        tile(has1, cxn & COL_MASK, j + 1, has1, is_partial(cx), [] {});
+        cx = cxn;
+      }
+      if (t == row_s && seg_b == row_e) {
+        write_row(r);
+      } else {
+        // a part of a row block that ranges share: published and counted in as in the other mode below; the last one
+        // in reads all parts (its own as well) and sums them in the order of the ranges
+        float lsum[2], M[2];
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+          lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
+          if (!(lsum[qb] > 0.f)) lsum[qb] = 0.f;
+          M[qb] = lsum[qb] > 0.f ? m_i[qb] : -INFINITY;
+        }
+        const int lane_p = fresh_lane(lane), ln = lane_p & 31, g = lane_p >> 5;
+        auto slot_of = [&](int p, bool head) { return prm.ws + (((int64_t)bh * prm.W + p) * 2 + (head ? 1 : 0)) * partial_floats(D); };
+        float* slot = slot_of(wg, t == row_s);
+        unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + r;
+        unsigned long long seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int quad = 0; quad < D / 4; ++quad) {
+          const int idx = 4 * quad;
+          const floatx16& o = oacc[idx / 32][(idx / 16) & 1];
+          coherent_store4(slot + idx * 64 + lane_p * 4, o[idx & 15], o[(idx & 15) + 1], o[(idx & 15) + 2], o[(idx & 15) + 3]);
+        }
+        if (g == 0) {
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb) {
+            coherent_store(slot + 64 * D + qb * 32 + ln, M[qb]);
+            coherent_store(slot + 64 * D + 64 + qb * 32 + ln, lsum[qb]);
+          }
+        }
+        const int64_t xrow = row_pos(hs, r, row_s);
+        int pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)), pf_ = split_of_pos(hs, xrow);
+        while (pl_ > pf_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pl_), r, row_s, row_e), row_s, row_e) >= row_e) --pl_;
+        while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
+        const int nparts = pl_ - pf_ + 1;
+        wait_vm<0>();                             // every store of the part has been acknowledged
+        int counted_v = 0;
+        if (lane == 0) {
+          unsigned long long old = seen;
+          for (;;) {     // (ends: the counter only changes when another part is counted, at most nparts times)
+            const unsigned long long want = (old >> 16) == prm.epoch ? old + 1 : ((prm.epoch << 16) | 1ull);
+            if (__hip_atomic_compare_exchange_strong(arrivals, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                     __HIP_MEMORY_SCOPE_AGENT)) {
+              counted_v = (int)(want & 0xffffull);
+              break;
+            }
+          }
+        }
+        if (__builtin_amdgcn_readfirstlane(counted_v) == nparts) {
+          float Ms[2] = {-INFINITY, -INFINITY}, Ls[2] = {0.f, 0.f};
+          reset_acc();
+          for (int p = pf_; p <= pl_; ++p) {
+            const float* sp = slot_of(p, p == pf_);
+            float sc_own[2], sc_p[2];
+#pragma unroll
+            for (int qb = 0; qb < 2; ++qb) {
+              const float mp = coherent_load(sp + 64 * D + qb * 32 + ln), lp = coherent_load(sp + 64 * D + 64 + qb * 32 + ln);
+              const float mn = fmaxf(Ms[qb], mp);     // a side without mass has maximum -inf and weight 0
+              sc_own[qb] = Ms[qb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Ms[qb] - mn);
+              sc_p[qb] = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mn);
+              Ls[qb] = Ls[qb] * sc_own[qb] + lp * sc_p[qb];
+              Ms[qb] = mn;
+            }
+#pragma unroll
+            for (int q4 = 0; q4 < D / 4; q4 += 4) {    // (four quads, 4 KB, per wait)
+              floatx4 ld[4];
+              coherent_load4x4(sp + q4 * 256 + lane_p * 4, ld[0], ld[1], ld[2], ld[3]);
+#pragma unroll
+              for (int e = 0; e < 16; ++e) {
+                const int idx = 4 * q4 + e, qb = (idx / 16) & 1;
+                oacc[idx / 32][qb][idx & 15] = oacc[idx / 32][qb][idx & 15] * sc_own[qb] + sc_p[qb] * ld[e / 4][e & 3];
+              }
+            }
+          }
+          // (write_row sums the two halves of a query)
+#pragma unroll
+          for (int qb = 0; qb < 2; ++qb) { m_i[qb] = Ms[qb]; l_i[qb] = g == 0 ? Ls[qb] : 0.f; }
+          write_row(r);
+          // back to zero, so that a replay of this launch (same mark) starts from a clean counter
+          if (lane == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+      }
+      t = seg_b;
+      ++r;
+    }
   } else {
     // ================= all wavefronts on one row block at a time =================
     // Tiles of the range are handed out to the wavefronts dynamically (the LDS counter), because
@@ -598,7 +803,7 @@ void fwd_kernel(const FwdParams prm) {
     // (the nearer one): sharing a row block costs a merge, a published part and a pull, several
     // tiles' worth each, and row blocks of up to 2 `snap` tiles are never shared.  Every workgroup
     // applies the same rule with the same distance to both of its boundaries, so the ranges still tile the list.
-    int r;
+    int r, g0, g1;
     {
       // the row blocks in which the two ends of the range lie (positions behind a row block's tiles count as
       // its end), then the tiles themselves
@@ -622,14 +827,14 @@ void fwd_kernel(const FwdParams prm) {
     // scalar load), so that they travel while the column list is staged and Q is read.
     if (g0 + w < g1) {
       const int c0 = flagged_col(g0 + w) & COL_MASK;
-      k_copy_all(kg + (int64_t)c0 * 64 * k_rs, g0 + w);
-      v_copy_all(vg + (int64_t)c0 * 64 * v_rs);
+      k_copy_all(c0, g0 + w);
+      v_copy_all(c0);
       kdone = vdone = g0 + w;
     }
     stage_cols(g0, g1);
     if (threadIdx.x == 0) { ctr[0] = g0 + 2 * NW; ctr[3] = 0; }
     __syncthreads();
-    auto col_of = [&](int t) { return t - g0 < C::COLS_CAP ? lcols[t - g0] : flagged_col(t); };
+    auto col_of = [&](int t) { return t - g0 < COLS_CAP ? lcols[t - g0] : flagged_col(t); };
     int cur = g0 + w, nxt = g0 + NW + w;      // the first two rounds are fixed
     int cb_nxt = nxt < g1 ? __builtin_amdgcn_readfirstlane(col_of(nxt)) : 0;   // column block of tile nxt
     int t = g0;
@@ -674,8 +879,8 @@ void fwd_kernel(const FwdParams prm) {
       reset_acc();
       if (mine) {
         int cx = __builtin_amdgcn_readfirstlane(col_of(cur));     // current tile: column block | flag
-        if (kdone != cur) { k_copy_all(kg + (int64_t)(cx & COL_MASK) * 64 * k_rs, cur); kdone = cur; }
-        if (vdone != cur) { v_copy_all(vg + (int64_t)(cx & COL_MASK) * 64 * v_rs); vdone = cur; }
+        if (kdone != cur) { k_copy_all(cx & COL_MASK, cur); kdone = cur; }
+        if (vdone != cur) { v_copy_all(cx & COL_MASK); vdone = cur; }
         load_q(r);
         while (cur < seg_b) {
           // draw the tile after next; the value is picked up inside the tile
@@ -684,7 +889,7 @@ void fwd_kernel(const FwdParams prm) {
           // the next tile is only prefetched inside the row block: the merge at its end borrows both buffers
           const bool has1 = nxt < seg_b, copy_v = has1;
           int nn = 0, cb_nn_v = 0;
-          tile(has1, cb_nxt & COL_MASK, nxt, copy_v, (cx >> 30) != 0, [&] {
+          tile(has1, cb_nxt & COL_MASK, nxt, copy_v, is_partial(cx), [&] {
             // (deterministic: every wavefront takes every NW-th tile, whatever its pace)
             nn = prm.deterministic ? nxt + NW : __builtin_amdgcn_readfirstlane(drawn);
             cb_nn_v = nn < g1 ? col_of(nn) : 0;     // looked up now, needed at the end of the tile
@@ -791,7 +996,8 @@ void fwd_kernel(const FwdParams prm) {
             if (full) {
               const float inv = L[qb] > 0.f ? 1.0f / L[qb] : 0.f;
               const int64_t qrow = (int64_t)(r * 64 + qb * 32 + ln);
-              store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, x[0] * inv, x[1] * inv,
+              if (exists(qrow))
+                store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, x[0] * inv, x[1] * inv,
                                x[2] * inv, x[3] * inv);
             } else {
               // (WIDE_PARTS: 16 bytes per lane and access, the part laid out [quad][lane][4])
@@ -811,7 +1017,7 @@ void fwd_kernel(const FwdParams prm) {
           if (w == 0 && g == 0 && prm.lse != nullptr) {
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
-              prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
+              if (exists((int64_t)(r * 64 + qb * 32 + ln))) prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
                   L[qb] > 0.f ? (M[qb] + __builtin_amdgcn_logf(L[qb])) * 0.6931471805599453f : -INFINITY;
           }
         } else {
@@ -929,13 +1135,13 @@ void fwd_kernel(const FwdParams prm) {
                 const int db = idx0 / 32, qb = (idx0 / 16) & 1, i4 = (idx0 & 15) / 4;
                 const float inv = Ls[qb] > 0.f ? 1.0f / Ls[qb] : 0.f;
                 const int64_t qrow = (int64_t)(r * 64 + qb * 32 + ln);
-                store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32,
+                if (exists(qrow)) store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32,
                                  acc[rd][tq][0] * inv, acc[rd][tq][1] * inv, acc[rd][tq][2] * inv, acc[rd][tq][3] * inv);
               }
             if (w == 0 && g == 0 && prm.lse != nullptr) {
 #pragma unroll
               for (int qb = 0; qb < 2; ++qb)
-                prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
+                if (exists((int64_t)(r * 64 + qb * 32 + ln))) prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
                     Ls[qb] > 0.f ? (Ms[qb] + __builtin_amdgcn_logf(Ls[qb])) * 0.6931471805599453f : -INFINITY;
             }
             // back to zero, so that a replay of this launch (same mark) starts from a clean counter
@@ -975,9 +1181,21 @@ int compute_units() {
   return cus;
 }
 
-static int groups_per_head(int B, int H, int nb, int D) {
+// How a launch is split at D = 64, by its row blocks against the wavefronts that are resident at once (8 per compute unit).
+// From half as many more on a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us; 24 heads of
+// N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there); with about as many a
+// wavefront takes a range of the list (32 heads of N = 4096 dense 174 -> 149 us; 8 heads of N = 17536 dense 702 -> 680,
+// keep 0.07 82 -> 74); with fewer the ranges of whole workgroups are the faster ones (6 heads of N = 17776 at keep 0.3: 236
+// against 250 us).
+static int fwd_mode(int B, int H, int nb, int D, bool compact) {
+  if (D != 64) return COOP;
+  const int64_t rows = (int64_t)B * H * nb, slots = FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * (int64_t)compute_units();
+  return 2 * rows >= 3 * slots ? ROWS_MODE : (rows >= slots && !compact ? WAVE : COOP);     // (compact: WAVE has four times as many ranges, hence parts)
+}
+
+static int groups_per_head(int B, int H, int nb, int D, int mode) {
   const int cus = compute_units();
-  const int per_cu = D == 64 ? FwdCfg<64>::WG_PER_CU : FwdCfg<128>::WG_PER_CU;
+  const int per_cu = D != 64 ? FwdCfg<128>::WG_PER_CU : (mode == COOP ? 1 : FwdCfg<64>::NW) * FwdCfg<64>::WG_PER_CU;
   int64_t W = (int64_t)cus * per_cu / ((int64_t)B * H);   // as many workgroups as are resident at once
   const int64_t cap = (int64_t)nb * nb;
   if (W > cap) W = cap;
@@ -1006,10 +1224,12 @@ static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
   return split > 1 ? (size_t)split * B * H * N * (D + 2) * sizeof(float) : 0;
 }
 
-size_t coop_workspace_bytes(int B, int H, int N, int D) {
-  if (D == 256) return 256 + pair_parts_bytes(B, H, N, D, pair_split(B, H, N / 64, D));   // the pair kernel only
-  const int nb = N / 64;
-  const int W = groups_per_head(B, H, nb, D);
+size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
+  if (D == 256) return 256 + pair_parts_bytes(B, H, N, D, pair_split(B, H, (N + 63) / 64, D));   // the pair kernel only
+  const int nb = (N + 63) / 64;
+  const int mode = fwd_mode(B, H, nb, D, compact);
+  if (mode == ROWS_MODE) return 256;      // nothing is shared
+  const int W = groups_per_head(B, H, nb, D, mode);
   return slots_bytes(B, H, W, D) + (size_t)B * H * nb * sizeof(unsigned long long);
 }
 
@@ -1027,35 +1247,46 @@ static bool use_pair_kernel(int64_t row_blocks, int nb) {
   return row_blocks >= 2 * cus || (row_blocks >= cus && nb <= 32);
 }
 
-// With few row blocks per workgroup all wavefronts of a workgroup share one row block at a time
-// (K and V tiles are spread over them and the results merged); with many (>= 8 per workgroup) each
-// wavefront takes whole row blocks, which needs no merge and no second kernel.
-static bool rows_mode(const FwdParams& prm) { return prm.nb >= 8 * prm.W; }
-
-template <int D, int DT, bool EW, bool CONTIG>
-static void launch_fwd_c(const FwdParams& prm, int BH, hipStream_t st) {
+// D = 64.  With few row blocks the wavefronts of a workgroup share one row block at a time (K and V tiles are spread
+// over them and the results merged); with many a wavefront takes a whole row block, which needs no merge.
+template <int D, int DT, int MODE, bool EW, int LAYOUT>
+static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
+  constexpr int LDS = MODE != COOP ? C::ROWS_LDS_BYTES : C::LDS_BYTES;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<D, DT, false, EW, CONTIG>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<D, DT, true, EW, CONTIG>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS_BYTES);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<D, DT, MODE, EW, LAYOUT>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   });
-  if (rows_mode(prm)) {
-    hipLaunchKernelGGL((fwd_kernel<D, DT, true, EW, CONTIG>), dim3(prm.W * BH), dim3(C::NW * 64), C::LDS_BYTES, st, prm);
-  } else {
-    hipLaunchKernelGGL((fwd_kernel<D, DT, false, EW, CONTIG>), dim3(prm.W * BH), dim3(C::NW * 64), C::LDS_BYTES, st, prm);
-  }
+  hipLaunchKernelGGL((fwd_kernel<D, DT, MODE, EW, LAYOUT>), dim3(grid), dim3(MODE != COOP ? 64 : C::NW * 64), LDS, st, prm);
 }
 
 // The copies with immediate offsets are compiled where they were measured faster: D = 64 (2-4 %) and
 // D = 128 with bf16 inputs (4-8 %; with fp16 inputs 1-3 % slower).
-template <int D, int DT, bool EW>
-static void launch_fwd_t(const FwdParams& prm, int BH, hipStream_t st) {
+template <int D, int DT, int MODE, bool EW>
+static void launch_fwd_t(const FwdParams& prm, int grid, hipStream_t st) {
+  const bool contig = prm.ks[2] == D && prm.vs[2] == D, whole = prm.N % 64 == 0;
   constexpr bool HAS_CONTIG = D == 64 || DT != 0;
-  if (HAS_CONTIG && prm.ks[2] == D && prm.vs[2] == D) launch_fwd_c<D, DT, EW, HAS_CONTIG>(prm, BH, st);
-  else launch_fwd_c<D, DT, EW, false>(prm, BH, st);
+  if (HAS_CONTIG && contig && whole) launch_fwd_c<D, DT, MODE, EW, HAS_CONTIG ? CONTIG_WHOLE : GENERAL>(prm, grid, st);
+  else if (D == 64 && contig) launch_fwd_c<D, DT, MODE, EW, D == 64 ? CONTIG_TAIL : GENERAL>(prm, grid, st);
+  else if (D == 128 && whole) launch_fwd_c<D, DT, MODE, EW, D == 128 ? STRIDED_WHOLE : GENERAL>(prm, grid, st);
+  else launch_fwd_c<D, DT, MODE, EW, GENERAL>(prm, grid, st);
+}
+
+template <int D, int MODE, bool EW>
+static void launch_fwd_m(const FwdParams& prm, int dt, int grid, hipStream_t st) {
+  if (dt == 0) launch_fwd_t<D, 0, MODE, EW>(prm, grid, st);
+  else if (dt == 1) launch_fwd_t<D, 1, MODE, EW>(prm, grid, st);
+  else launch_fwd_t<D, 2, MODE, EW>(prm, grid, st);
+}
+
+template <bool EW>
+static void launch_fwd_d(const FwdParams& prm, int D, int mode, int dt, hipStream_t st) {
+  const int BH = prm.B * prm.H, grid = prm.W * BH;
+  if (D == 128) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
+  else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, ((BH + 7) / 8) * 8 * prm.nb, st);
+  else if (mode == WAVE) launch_fwd_m<64, WAVE, EW>(prm, dt, grid, st);
+  else launch_fwd_m<64, COOP, EW>(prm, dt, grid, st);
 }
 
 // ---- forward without any allocation by anybody: the scratch memory is part of the library ----
@@ -1103,17 +1334,20 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.q = q; prm.k = k; prm.v = v; prm.o = o; prm.lse = lse;
   prm.row_ptr = row_ptr; prm.col_idx = col_idx; prm.ws = (float*)ws;
   prm.tile_partial = tile_partial; prm.tile_bits = (const unsigned long long*)tile_bits;
-  prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = s.N / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
-  prm.W = groups_per_head(s.B, s.H, prm.nb, s.D);
+  prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
+  const int mode = fwd_mode(s.B, s.H, prm.nb, s.D, s.compact);
+  prm.W = groups_per_head(s.B, s.H, prm.nb, s.D, mode);
   // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are
-  prm.first_ids = (s.D == 64 ? FwdCfg<64>::WG_PER_CU : FwdCfg<128>::WG_PER_CU) > 1 ? compute_units() : 0;
+  // (WAVE: wavefronts instead of workgroups; where a range is a whole number of row blocks the shares stay equal: 16 heads of
+  // N = 8192 dense 304 against 287 us)
+  prm.first_ids = s.D == 64 ? compute_units() * (mode == COOP ? 1 : prm.nb % prm.W == 0 ? 0 : FwdCfg<64>::NW) : 0;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();
   {
     const int BHl = s.B * s.H;
     const int F = prm.first_ids > 0 && prm.first_ids % BHl == 0 ? (prm.first_ids / BHl < prm.W ? prm.first_ids / BHl : prm.W) : 0;
-    const bool ok = (prm.first_ids == 0 || prm.first_ids % BHl == 0) && range_permutation(prm.nb, prm.W, F, BHl, prm.perm, prm.perm_causal);
+    const bool ok = mode == COOP && (prm.first_ids == 0 || prm.first_ids % BHl == 0) && range_permutation(prm.nb, prm.W, F, BHl, prm.perm, prm.perm_causal);
     prm.perm_n = ok ? prm.W : 0;
     prm.perm_fast = F;
     prm.perm_min_tiles = (int)((int64_t)prm.nb * prm.nb * 3 / 4);
@@ -1137,13 +1371,8 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // bf16 with a bf16-typed result: P is rounded to bf16 as well (the reference rounds P to the type of
   // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
   const int dt = !bf ? 0 : (prm.out_f32 ? 1 : 2);
-  if (tile_bits == nullptr) {
-    if (s.D == 64) { if (dt == 0) launch_fwd_t<64, 0, false>(prm, BH, st); else if (dt == 1) launch_fwd_t<64, 1, false>(prm, BH, st); else launch_fwd_t<64, 2, false>(prm, BH, st); }
-    else { if (dt == 0) launch_fwd_t<128, 0, false>(prm, BH, st); else if (dt == 1) launch_fwd_t<128, 1, false>(prm, BH, st); else launch_fwd_t<128, 2, false>(prm, BH, st); }
-  } else {   // elementwise mask
-    if (s.D == 64) { if (dt == 0) launch_fwd_t<64, 0, true>(prm, BH, st); else if (dt == 1) launch_fwd_t<64, 1, true>(prm, BH, st); else launch_fwd_t<64, 2, true>(prm, BH, st); }
-    else { if (dt == 0) launch_fwd_t<128, 0, true>(prm, BH, st); else if (dt == 1) launch_fwd_t<128, 1, true>(prm, BH, st); else launch_fwd_t<128, 2, true>(prm, BH, st); }
-  }
+  if (tile_bits == nullptr) launch_fwd_d<false>(prm, s.D, mode, dt, st);
+  else launch_fwd_d<true>(prm, s.D, mode, dt, st);
   return launch_status();
 }
 

@@ -25,7 +25,9 @@ constexpr int PAIR_COLS_CAP = 1024;                               // column indi
 template <int D> constexpr int pair_lds_bytes() { return 2 * 64 * 2 * D + 512 + PAIR_COLS_CAP * 4; }   // K tile, V tile, mask words, columns
 
 // CONTIG: the rows of K and of V follow each other without gaps (row stride = D).
-template <int D, int DT, bool EW, bool CONTIG>
+// TAIL: N is not a multiple of 64 (as in attn_fwd.hip: the copy of the last tile repeats its last key, the scores beyond
+// it are -inf, the queries beyond N are not written).
+template <int D, int DT, bool EW, bool CONTIG, bool TAIL>
 __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const FwdParams prm) {
   constexpr int KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, TILE_BYTES = 64 * ROWB;
   constexpr int PORTIONS = D / 128;              // K and V fragments are read in this many portions
@@ -58,9 +60,11 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   // Q of this lane's query (second operand of S^T = K Q^T) depends on the block index only: asked for first, it
   // travels while the list is looked up and the first tiles are requested.
   const int64_t qrow = (int64_t)m * 64 + 32 * w + ln;          // this lane's query
+  const bool exists = !TAIL || qrow < prm.N;
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64, tail_cb = TAIL ? nb - 1 : -1;
   uintx4 qf[1][KS];
   {
-    const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + qrow * prm.qs[2];
+    const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + (exists ? qrow : prm.N - 1) * prm.qs[2];
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[0][s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
   }
@@ -73,6 +77,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   }
   void* obase = out_base(prm, b, h);
   if (t0 == t1) {                                // no kept tile: O = 0, lse = -inf
+    if (!exists) return;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -120,9 +125,21 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
       voff[par] = 2u * (unsigned)(row0 * (int)prm.vs[2] + ((ch ^ v_swz<D>(par * RPI + row0)) * 8));
   }
   const int64_t k_rs = CONTIG ? (int64_t)D : prm.ks[2], v_rs = CONTIG ? (int64_t)D : prm.vs[2];   // row strides
+  // (the lane index as a value the compiler cannot trace back, or the offsets are computed before the loop and held)
+  auto tail_copy = [&](const unsigned short* tile, int64_t rs, unsigned lds_addr, auto&& swz) {
+    int lane_t = lane;
+    asm volatile("" : "+v"(lane_t));
+#pragma unroll 1
+    for (int j = w * HALF; j < (w + 1) * HALF; ++j) {
+      const int row = j * RPI + lane_t / CPR, src = row < valid ? row : valid - 1;
+      tile_load_async_one(tile, 2u * (unsigned)(src * (int)rs + (((lane_t % CPR) ^ swz(row)) * 8)), lds_addr + j * 1024);
+    }
+  };
   auto k_copy = [&](int cb, int t) {
     const unsigned short* tile = kg + (int64_t)cb * 64 * k_rs;
-    if constexpr (CONTIG) {     // (instruction j reads at byte 1024 j of the tile and writes at byte 1024 j of the buffer)
+    if (TAIL && cb == tail_cb) {
+      tail_copy(tile, k_rs, lds_k_addr, [](int row) { return k_swz<D>(row); });
+    } else if constexpr (CONTIG) {     // (instruction j reads at byte 1024 j of the tile and writes at byte 1024 j of the buffer)
 #pragma unroll
       for (int jb = 0; jb < HALF; jb += 4)
         tile_load_async_four(tile + (w * HALF + jb) * RPI * D, koff[jb % KPER], koff[(jb + 1) % KPER], koff[(jb + 2) % KPER],
@@ -142,7 +159,9 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   };
   auto v_copy = [&](int cb) {
     const unsigned short* tile = vg + (int64_t)cb * 64 * v_rs;
-    if constexpr (CONTIG) {
+    if (TAIL && cb == tail_cb) {
+      tail_copy(tile, v_rs, lds_v_addr, [](int row) { return v_swz<D>(row); });
+    } else if constexpr (CONTIG) {
 #pragma unroll
       for (int jb = 0; jb < HALF; jb += 4)
         tile_load_async_four(tile + (w * HALF + jb) * RPI * D, voff[jb % VPER], voff[(jb + 1) % VPER], voff[(jb + 2) % VPER],
@@ -203,7 +222,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   for (int t = t0; t < t1; ++t) {
     const bool has1 = t + 1 < t1;
     const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(t + 1)) : 0;
-    const bool partial = EW && (cx >> 30) != 0;
+    const bool partial = EW ? (cx >> 30) != 0 : TAIL && cx == tail_cb;
     // ---- S^T = K Q^T (- m when FOLD); the K fragments (and the mask word of this lane's query) ----
     floatx16 s0, s1;
 #pragma unroll
@@ -218,6 +237,9 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
         for (int s = 0; s < KSP; ++s) kfr[kb][s] = *reinterpret_cast<const uintx4*>(lds_k + kaddr[kb][pt * KSP + s]);
       if (pt == PORTIONS - 1) {
         if constexpr (EW) { if (partial) mw = lds_bits[32 * w + ln] >> (4 * g); }
+        else if constexpr (TAIL) {
+          if (partial) { mw = ((1ull << valid) - 1ull) >> (4 * g); asm volatile("" : "+v"(mw)); }
+        }
         lds_wait();
         __syncthreads();                            // both wavefronts hold their K fragments: the K buffer is free
         if (has1) k_copy(cxn & COL_MASK, t + 1);
@@ -234,7 +256,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
         s1 = mfma_qk<BF16>(ones_frag, mfrag, s1);
       }
     }
-    if constexpr (EW) {
+    if constexpr (EW || TAIL) {
       if (partial) {
         const unsigned lo = (unsigned)mw, hi = (unsigned)(mw >> 32);
 #pragma unroll
@@ -327,6 +349,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   // ---- normalise and write ----
   const float lsum = l_i + __shfl_xor(l_i, 32);
   if (prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
+    if (!exists) return;
     float* part = prm.part_o + ((int64_t)chunk * BH + bh) * prm.N * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -345,8 +368,8 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   static_assert(2 * rows_out_bytes(D, true) <= pair_lds_bytes<D>(), "room for the result rows of both wavefronts");
   __syncthreads();           // the other wavefront has left its last tile
   rows_out<BF16, D>(lds + w * rows_out_bytes(D, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2], prm.os[2], prm.out_f32,
-                    lane, [&](int db, int i) { return oacc[db][0][i] * inv; });
-  if (prm.lse != nullptr && g == 0)
+                    lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return oacc[db][0][i] * inv; });
+  if (prm.lse != nullptr && g == 0 && exists)
     prm.lse[(int64_t)bh * prm.N + qrow] =
         lsum > 0.f ? (m_i + __builtin_amdgcn_logf(lsum)) * 0.6931471805599453f : -INFINITY;
 }
@@ -389,14 +412,14 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
     prm.lse[(int64_t)bh * prm.N + row] = L > 0.f ? (M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f : -INFINITY;
 }
 
-template <int D, int DT, bool EW, bool CONTIG>
+template <int D, int DT, bool EW, bool CONTIG, bool TAIL>
 static void launch_pair_c(const FwdParams& prm, int grid, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_pair_kernel<D, DT, EW, CONTIG>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_pair_kernel<D, DT, EW, CONTIG, TAIL>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds_bytes<D>());
   });
-  hipLaunchKernelGGL((fwd_pair_kernel<D, DT, EW, CONTIG>), dim3(grid), dim3(128), pair_lds_bytes<D>(), st, prm);
+  hipLaunchKernelGGL((fwd_pair_kernel<D, DT, EW, CONTIG, TAIL>), dim3(grid), dim3(128), pair_lds_bytes<D>(), st, prm);
 }
 
 template <int D, int DT, bool EW>
@@ -404,8 +427,9 @@ static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   const int BH = prm.B * prm.H;
   const int grid = ((BH + 7) / 8) * 8 * prm.nb * prm.split;
   // (the variant with immediate copy offsets: 5 % faster at D = 256, 3 % slower on dense masks at D = 128)
-  if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256>(prm, grid, st);
-  else launch_pair_c<D, DT, EW, false>(prm, grid, st);
+  if (prm.N % 64 != 0) launch_pair_c<D, DT, EW, false, true>(prm, grid, st);
+  else if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256, false>(prm, grid, st);
+  else launch_pair_c<D, DT, EW, false, false>(prm, grid, st);
   if (prm.split > 1) {
     const int64_t quads = (int64_t)BH * prm.N * D / 4;
     hipLaunchKernelGGL((pair_sum_parts_kernel<DT != 0>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, st, prm, D, quads);

@@ -30,6 +30,7 @@ int launch_pack_tiles(const uint8_t* dense, int Bm, int Hm, int nb, int64_t sb, 
 struct AttnShape {
   int B, H, N, D, Bm, Hm;
   int dtype, out_dtype;
+  bool compact = false;   // forward: the split with the smaller workspace (bsattn_fwd_static)
   float sm_scale;
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];  // batch, head, row strides (elements)
   int64_t dqs[3], dks[3], dvs[3];              // ... of the backward's results
@@ -57,7 +58,7 @@ int get_deterministic();
 int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                const int32_t* row_ptr, const int32_t* col_idx, const uint8_t* tile_partial,
                const uint64_t* tile_bits, const AttnShape& s, void* ws, hipStream_t st);
-size_t coop_workspace_bytes(int B, int H, int N, int D);   // what launch_fwd itself needs
+size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact = false);   // what launch_fwd itself needs
 // Address, on the current device, of the library's own scratch array (BSATTN_STATIC_SCRATCH_BYTES).
 int static_scratch(void** ptr);
 

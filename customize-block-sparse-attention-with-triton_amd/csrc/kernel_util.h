@@ -162,11 +162,12 @@ __device__ __forceinline__ void store_out4(void* obase, int64_t elem_off, bool o
 // layout in which a 32x32 MFMA result holds its rows), db < NCOL / 32.
 // stage: ROWS_OUT_BYTES(NCOL, out_f32) bytes of LDS that only this wavefront touches (its LDS accesses are executed
 // in order, so the reads below see the writes above them without a barrier).
-// out + elem_off: row 0, first of the NCOL columns; row_stride in elements; rows 16-byte aligned.
+// out + elem_off: row 0, first of the NCOL columns; row_stride in elements; rows 16-byte aligned; only the first `rows`
+// rows are written.
 __host__ __device__ constexpr int rows_out_bytes(int ncol, bool out_f32) { return 32 * (ncol * (out_f32 ? 4 : 2) + 16); }
 template <bool BF16, int NCOL, typename F>
 __device__ __forceinline__ void rows_out(unsigned char* stage, void* out, int64_t elem_off, int64_t row_stride,
-                                         bool out_f32, int lane, F&& value) {
+                                         bool out_f32, int lane, int rows, F&& value) {
   const int ln = lane & 31, g = lane >> 5;
   if (out_f32) {
     constexpr int PITCH = NCOL * 4 + 16, LPR = NCOL / 4, RPI = 64 / LPR;   // lanes per row, rows per instruction
@@ -183,7 +184,7 @@ __device__ __forceinline__ void rows_out(unsigned char* stage, void* out, int64_
     for (int it = 0; it < 32 / RPI; ++it) {
       const int r = it * RPI + lane / LPR, c = lane % LPR;
       const floatx4 w = *reinterpret_cast<const floatx4*>(stage + r * PITCH + 16 * c);
-      *reinterpret_cast<floatx4*>(o + r * row_stride + 4 * c) = w;
+      if (r < rows) *reinterpret_cast<floatx4*>(o + r * row_stride + 4 * c) = w;
     }
   } else {
     constexpr int PITCH = NCOL * 2 + 16, LPR = NCOL / 8, RPI = 64 / LPR;
@@ -200,7 +201,7 @@ __device__ __forceinline__ void rows_out(unsigned char* stage, void* out, int64_
     for (int it = 0; it < 32 / RPI; ++it) {
       const int r = it * RPI + lane / LPR, c = lane % LPR;
       const uintx4 w = *reinterpret_cast<const uintx4*>(stage + r * PITCH + 16 * c);
-      *reinterpret_cast<uintx4*>(o + r * row_stride + 8 * c) = w;
+      if (r < rows) *reinterpret_cast<uintx4*>(o + r * row_stride + 8 * c) = w;
     }
   }
 }

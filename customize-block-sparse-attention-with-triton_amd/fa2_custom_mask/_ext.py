@@ -33,6 +33,11 @@ _SIGNATURES = {
     "bsattn_fwd": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f,
                     _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_block_mask_workspace": ([_i, _i, _i, _i, _i, _i, ctypes.POINTER(ctypes.c_size_t)], _i),
+    "bsattn_fwd_tokens": ([_p, _p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f,
+                           _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
+    "bsattn_bwd_tokens": ([_p] * 15 + [_i] * 8 + [_f] + [_p] * 8 + [_p, ctypes.c_size_t, _p], _i),
+    "bsattn_fwd_block_mask_tokens": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f,
+                                      _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_block_mask": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f,
                                _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_static": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f,
@@ -149,13 +154,17 @@ def _fused_workspace_on(Bm, Hm, B, H, N, D, index):
     return n.value
 
 
+def _whole(N):
+    return (N + 63) // 64 * 64
+
+
 def fwd_block_mask_workspace(Bm, Hm, B, H, N, D, device=None):
-    return _fused_workspace_on(Bm, Hm, B, H, N, D, _device_index(device))
+    return _fused_workspace_on(Bm, Hm, B, H, _whole(N), D, _device_index(device))
 
 
 def fwd_workspace(B, H, N, D, device=None):
-    return _workspace_on("bsattn_fwd_workspace", B, H, N, D, _device_index(device))
+    return _workspace_on("bsattn_fwd_workspace", B, H, _whole(N), D, _device_index(device))
 
 
 def bwd_workspace(B, H, N, D, device=None):
-    return _workspace_on("bsattn_bwd_workspace", B, H, N, D, _device_index(device))
+    return _workspace_on("bsattn_bwd_workspace", B, H, _whole(N), D, _device_index(device))

@@ -104,15 +104,13 @@ def _check_qkv(q, k, v, mask):
     return B, H, N, D
 
 
-def _padded(x, N, D):
-    """The kernels work on whole 64-token tiles and on head dimensions 64 and 128: other shapes
-    are embedded in zeros.  Zero columns change neither q k^T nor the real columns of the
-    output; the keys of zero rows are masked (utils.mask_to_lists), their query rows are dropped."""
-    Np, Dp = num_tiles(N) * TILE, (64 if D < 64 else D)
-    if (Np, Dp) == (x.shape[2], x.shape[3]):
+def _padded(x):
+    """The kernels work on head dimensions 64, 128 and 256: smaller ones are embedded in zeros.  Zero columns change neither
+    q k^T nor the real columns of the output."""
+    if x.shape[3] >= 64:
         return x
-    xp = x.new_zeros((x.shape[0], x.shape[1], Np, Dp))
-    xp[:, :, :x.shape[2], :x.shape[3]] = x
+    xp = x.new_zeros((x.shape[0], x.shape[1], x.shape[2], 64))
+    xp[:, :, :, :x.shape[3]] = x
     return xp
 
 
@@ -165,10 +163,8 @@ def _forward(q, k, v, lists, sm_scale, out_dtype, want_lse):
               *strides, ws.data_ptr(), wsb, stream)
     ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if want_lse else None,
             lists.row_ptr_ptr, lists.col_idx_ptr)
-    if lists.bits is None:
-        rc = _ext.lib().bsattn_fwd(*ptrs, *common)
-    else:                                      # elementwise mask: exact inside partly set tiles
-        rc = _ext.lib().bsattn_fwd_elementwise(*ptrs, lists.partial.data_ptr(), lists.bits.data_ptr(), *common)
+    words = (None, None) if lists.bits is None else (lists.partial.data_ptr(), lists.bits.data_ptr())   # elementwise mask: exact inside partly set tiles
+    rc = _ext.lib().bsattn_fwd_tokens(*ptrs, *words, *common)
     _ext.check(rc, "bsattn_fwd")
     return o, lse
 
@@ -220,10 +216,8 @@ def _backward(q, k, v, o, do, lse, lists, lists_t, sm_scale, out_dtype):
               _ext.strides4(q), _ext.strides4(k), _ext.strides4(v), _ext.strides4(o), _ext.strides4(do),
               _ext.strides4(dq), _ext.strides4(dk), _ext.strides4(dv),
               ws.data_ptr(), wsb, stream)
-    if lists.bits is None:
-        rc = _ext.lib().bsattn_bwd(*tensors, *common)
-    else:                                      # elementwise mask
-        rc = _ext.lib().bsattn_bwd_elementwise(*tensors, lists.bits.data_ptr(), lists_t.bits.data_ptr(), *common)
+    words = (None, None) if lists.bits is None else (lists.bits.data_ptr(), lists_t.bits.data_ptr())   # elementwise mask
+    rc = _ext.lib().bsattn_bwd_tokens(*tensors, *words, *common)
     _ext.check(rc, "bsattn_bwd")
     return dq, dk, dv
 
@@ -270,7 +264,7 @@ def _forward_from_block_mask(q, k, v, mask, sm_scale, out_dtype, want_lse):
     lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device) if want_lse else None
     wsb = _ext.fwd_block_mask_workspace(Bm, Hm, B, H, N, D, q.device)
     ws, stream = _workspace(wsb, q.device)
-    rc = _ext.lib().bsattn_fwd_block_mask(
+    rc = _ext.lib().bsattn_fwd_block_mask_tokens(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if want_lse else None,
         mask.data_ptr(), _ext.strides4(mask), Bm, Hm, lists.row_ptr_ptr, lists.col_idx_ptr, lists.counts_ptr,
         B, H, N, D, _ext.dtype_code(q.dtype), _ext.dtype_code(out_dtype), float(sm_scale),
@@ -285,22 +279,19 @@ def _forward_only(q, k, v, mask, sm_scale, out_fp32, return_lse):
     if mask is None:
         mask = _dense_mask(q.device, num_tiles(N))
     out_dtype = torch.float32 if out_fp32 else q.dtype
-    whole = N % TILE == 0 and D >= 64
     lists = lists_cache.get(mask, N, False)
-    if lists is None and whole and mask.shape[2] * TILE == N:
+    if D < 64:
+        q, k, v = _padded(q), _padded(k), _padded(v)
+    if lists is None and is_block_form(mask, N):
         # a block mask seen for the first time (or one that changes with every call): lists and forward in one call
         o, lse, lists = _forward_from_block_mask(q, k, v, mask, sm_scale, out_dtype, return_lse)
         lists_cache.put(mask, N, False, lists)
-        return (o, lse) if return_lse else o
-    if lists is None:
-        lists = mask_to_lists(mask, N)
-    if whole:
+    else:
+        if lists is None:
+            lists = mask_to_lists(mask, N)
         o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, return_lse)
-        return (o, lse) if return_lse else o
-    q, k, v = _padded(q, N, D), _padded(k, N, D), _padded(v, N, D)
-    o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, return_lse)
-    if o.shape[2:] != (N, D):
-        o, lse = o[:, :, :N, :D], (lse[:, :, :N] if lse is not None else None)
+    if D < 64:
+        o = o[:, :, :, :D]
     return (o, lse) if return_lse else o
 
 
@@ -316,7 +307,7 @@ class _attention(torch.autograd.Function):
         # (a backward will ask for the column lists too when a gradient is wanted)
         lists = mask_to_lists(mask, N, both=any(ctx.needs_input_grad[:3]))   # :48
         out_dtype = torch.float32 if out_fp32 else q.dtype
-        q, k, v = _padded(q, N, D), _padded(k, N, D), _padded(v, N, D)
+        q, k, v = _padded(q), _padded(k), _padded(v)
         o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, True)
         ctx.save_for_backward(q, k, v, o, lse, mask)                         # :89
         ctx.lists = lists
@@ -324,8 +315,8 @@ class _attention(torch.autograd.Function):
         ctx.out_dtype = out_dtype
         ctx.return_lse = return_lse
         ctx.shape = (N, D)
-        if o.shape[2:] != (N, D):
-            o, lse = o[:, :, :N, :D], lse[:, :, :N]
+        if D < 64:
+            o = o[:, :, :, :D]
         if return_lse:
             ctx.mark_non_differentiable(lse)
             return o, lse
@@ -337,11 +328,11 @@ class _attention(torch.autograd.Function):
         N, D = ctx.shape
         lists_t = mask_to_lists(mask, N, transpose=True)
         o_in = o if o.dtype == q.dtype else o.to(q.dtype)
-        do_in = _padded(do if do.dtype == q.dtype else do.to(q.dtype), N, D)
+        do_in = _padded(do if do.dtype == q.dtype else do.to(q.dtype))
         # autograd hands gradients back in the dtype of q, k, v
         dq, dk, dv = _backward(q, k, v, o_in, do_in, lse, ctx.lists, lists_t, ctx.sm_scale, q.dtype)
-        if dq.shape[2:] != (N, D):
-            dq, dk, dv = dq[:, :, :N, :D], dk[:, :, :N, :D], dv[:, :, :N, :D]
+        if D < 64:
+            dq, dk, dv = dq[:, :, :, :D], dk[:, :, :, :D], dv[:, :, :, :D]
         return dq, dk, dv, None, None, None, None                            # :155
 
 
@@ -350,8 +341,8 @@ def flash_attention_custom_mask(q, k, v, mask=None, sm_scale=1.3):
     (fa2_custom_mask.py:157): q,k,v [B,H,N,D] fp16/bf16 on the GPU, mask bool
     [B|1,H|1,nb,nb] with nb = ceil(N/64) (or elementwise [B|1,H|1,N,N]; None = dense attention),
     returns o like q.  D is 16, 32, 64, 128 or 256; N need not be a multiple of 64 (the last block of a
-    block mask then covers the remaining tokens).  Shapes other than D in {64,128,256}, N % 64 == 0
-    cost one zero-padded copy of q, k, v per call.  The kept-tile lists of a mask tensor are cached
+    block mask then covers the remaining tokens).  D = 16 and 32 cost one zero-padded copy of
+    q, k, v per call.  The kept-tile lists of a mask tensor are cached
     until the tensor is modified.  When no gradient can be asked for (gradients disabled, or none of q, k, v
     requires one) the call does not go through torch.autograd.Function, which costs about as much host time
     as everything else in a small call."""
@@ -378,11 +369,10 @@ def attention_forward_backward(q, k, v, mask, sm_scale, do, out_fp32=False):
     lists = mask_to_lists(mask, N, both=True)
     lists_t = mask_to_lists(mask, N, transpose=True)
     out_dtype = torch.float32 if out_fp32 else q.dtype
-    q, k, v = _padded(q, N, D), _padded(k, N, D), _padded(v, N, D)
+    q, k, v = _padded(q), _padded(k), _padded(v)
     o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, True)
     o_in = o if o.dtype == q.dtype else o.to(q.dtype)
-    dq, dk, dv = _backward(q, k, v, o_in, _padded(do.to(q.dtype), N, D), lse, lists, lists_t, sm_scale, out_dtype)
-    if o.shape[2:] != (N, D):
-        o, lse = o[:, :, :N, :D], lse[:, :, :N]
-        dq, dk, dv = dq[:, :, :N, :D], dk[:, :, :N, :D], dv[:, :, :N, :D]
+    dq, dk, dv = _backward(q, k, v, o_in, _padded(do.to(q.dtype)), lse, lists, lists_t, sm_scale, out_dtype)
+    if D < 64:
+        o, dq, dk, dv = o[:, :, :, :D], dq[:, :, :, :D], dk[:, :, :, :D], dv[:, :, :, :D]
     return o, lse, dq, dk, dv

@@ -327,11 +327,9 @@ def mask_to_lists(mask, N, transpose=False, both=False):
     lists = lists_cache.get(mask, N, transpose)
     if lists is None:
         _check_mask(mask)
-        pad = num_tiles(N) * TILE - N          # > 0: q, k, v get `pad` zero rows, whose keys are masked here
+        pad = num_tiles(N) * TILE - N          # keys of the last tile that do not exist: their bits stay clear
         if is_block_form(mask, N):
             lists = block_mask_to_lists(mask, transpose=transpose)
-            if pad:
-                lists.partial, lists.bits = tail_mask_tiles(lists, TILE - pad, transpose=transpose)
         else:                                  # elementwise form: exact inside tiles
             grid = grid_cache.get(mask, N)
             if grid is None and not (both or transpose):

@@ -291,6 +291,38 @@ int bsattn_bwd_elementwise(const void* q, const void* k, const void* v, const vo
                            size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------
+ * Any number of tokens.  The entry points above take whole 64-token tiles (N a multiple of 64), as the reference's
+ * block pointers do (fa2_custom_mask/fa2_fwd.py:137-172); these take any N >= 1 with nb = ceil(N / 64) blocks, the
+ * last of which holds the remaining tokens: the lists are those of a [Bm,Hm,nb,nb] mask, the tensors have N rows (no
+ * memory beyond them is touched), lse is [B,H,N].  tile_partial / tile_bits (and tile_bits_rows / tile_bits_cols) as for
+ * the elementwise entry points, with the bits of missing keys and queries clear, or all NULL for a block mask.  A
+ * workspace as large as the query returns for the next multiple of 64 is enough.  Otherwise as bsattn_fwd,
+ * bsattn_fwd_elementwise, bsattn_fwd_block_mask, bsattn_bwd, bsattn_bwd_elementwise.
+ * ---------------------------------------------------------------------------------- */
+int bsattn_fwd_tokens(const void* q, const void* k, const void* v, void* o, float* lse,
+                      const int32_t* row_ptr, const int32_t* col_idx, const uint8_t* tile_partial,
+                      const uint64_t* tile_bits, int Bm, int Hm, int B, int H, int N, int D, int dtype,
+                      int out_dtype, float sm_scale, const int64_t* q_strides, const int64_t* k_strides,
+                      const int64_t* v_strides, const int64_t* o_strides, void* workspace,
+                      size_t workspace_bytes, void* stream);
+int bsattn_fwd_block_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse,
+                                 const uint8_t* block, const int64_t* mask_strides, int Bm, int Hm,
+                                 int32_t* row_ptr, int32_t* col_idx, int32_t* counts,
+                                 int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                                 const int64_t* q_strides, const int64_t* k_strides,
+                                 const int64_t* v_strides, const int64_t* o_strides, void* workspace,
+                                 size_t workspace_bytes, void* stream);
+int bsattn_bwd_tokens(const void* q, const void* k, const void* v, const void* o, const void* d_o,
+                      const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
+                      const int32_t* col_idx, const int32_t* col_ptr, const int32_t* row_idx,
+                      const uint64_t* tile_bits_rows, const uint64_t* tile_bits_cols,
+                      int Bm, int Hm, int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                      const int64_t* q_strides, const int64_t* k_strides, const int64_t* v_strides,
+                      const int64_t* o_strides, const int64_t* do_strides,
+                      const int64_t* dq_strides, const int64_t* dk_strides, const int64_t* dv_strides,
+                      void* workspace, size_t workspace_bytes, void* stream);
+
+/* ------------------------------------------------------------------------------------
  * Head-wise token reorder.  Replaces reorder_kernel / inv_reorder_kernel
  * (fa2_custom_mask/permute.py:5-58, 60-126) as launched from apply_head_wise_reorder /
  * apply_inv_reorder (fa2_custom_mask/functional.py:5-20, 46-62).

@@ -1,0 +1,78 @@
+"""The ways the forward at D = 64 splits a launch (ranges of workgroups, ranges of wavefronts, whole row blocks), and
+sequence lengths that are not a multiple of 64, whose last tile must touch nothing beyond the tensors.  Against the CPU
+oracle on sampled heads."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import bsattn_oracle as orc
+from helpers import make_qkv, uniform_block_mask, errors, f32
+
+pytestmark = pytest.mark.gpu
+
+MAXABS = {torch.float16: 2e-2, torch.bfloat16: 3e-2}
+RELL2 = {torch.float16: 1e-3, torch.bfloat16: 3e-3}          # bf16-typed results: rounding an exact one costs 1.7e-3
+
+
+def block_mask(nb, keep, seed):
+    m = uniform_block_mask(1, 1, nb, keep, seed)
+    m[0, 0, nb // 3, :] = False                              # a row block without kept tiles
+    m[0, 0, nb // 2, :] = True                               # a full one: ranges end inside it
+    m[0, 0, :, nb - 1] |= torch.arange(nb) % 2 == 0          # the last, partly filled column
+    return m
+
+
+# wavefronts of the GPU: 2048.  2048 row blocks: ranges of wavefronts, each a whole number of row blocks on average;
+# 2080 and 2400: ranges that cut row blocks; 3200: whole row blocks; 8 ragged row blocks of 4 heads: ranges of workgroups
+@pytest.mark.parametrize("B,H,N", [(2, 16, 4096), (1, 40, 3300), (1, 24, 6337), (4, 40, 1250), (1, 4, 449)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("elementwise", [False, True])
+def test_modes(dev, B, H, N, dtype, elementwise):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v = make_qkv(B, H, N, 64, dtype, 500 + N)
+    block = block_mask(nb, 0.3, 501 + N)
+    dense = torch.from_numpy(orc.expand_block_mask(block.numpy())[..., :N, :N].copy())
+    if elementwise:
+        i = torch.arange(N)
+        dense = dense & ((i[:, None] - i[None, :]) % 7 != 0)
+        dense[0, 0, 5, :] = False                            # a query without keys
+    mask = dense if elementwise else block
+    o, lse = fm.flash_attention_custom_mask_lse(q.to(dev), k.to(dev), v.to(dev), mask.to(dev), 0.125)
+    torch.cuda.synchronize()
+    assert o.shape == (B, H, N, 64) and lse.shape == (B, H, N) and bool(torch.isfinite(o.float()).all())
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        sl = (slice(b, b + 1), slice(h, h + 1))
+        o_ref, lse_ref = orc.naive_attention(f32(q[sl]), f32(k[sl]), f32(v[sl]), dense.numpy(), 0.125, return_lse=True)
+        ma, rl = errors(o[sl], o_ref)
+        assert ma <= MAXABS[dtype] and rl <= RELL2[dtype], (b, h, ma, rl)
+        fin = np.isfinite(lse_ref)
+        got = lse[sl].cpu().numpy()
+        assert np.array_equal(np.isfinite(got), fin) and np.abs(got[fin] - lse_ref[fin]).max() <= 2e-3
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("N", [1, 63, 130, 191])
+@pytest.mark.parametrize("contiguous_rows", [True, False])
+def test_nothing_beyond_the_last_token_is_touched(dev, D, N, contiguous_rows):
+    """q, k, v, dO are the first N rows of larger tensors that hold NaN behind them: a value read from there would
+    reach a result (even with weight zero)."""
+    import fa2_custom_mask as fm
+    B, H = 1, 3
+    pad = 64 - N % 64
+    row = D if contiguous_rows else D + 8
+    g = torch.Generator().manual_seed(600 + N)
+    big = torch.full((4, B, H, N + pad, row), float("nan"))
+    big[:, :, :, :N, :D] = torch.randn(4, B, H, N, D, generator=g)
+    q, k, v, do = big.half().to(dev)[:, :, :, :N, :D].unbind(0)
+    nb = -(-N // 64)
+    block = uniform_block_mask(1, 1, nb, 0.7, 601 + N)
+    dense = orc.expand_block_mask(block.numpy())[..., :N, :N]
+    sc = D ** -0.5
+    res = fm.attention_forward_backward(q, k, v, block.to(dev), sc, do, out_fp32=True)
+    torch.cuda.synchronize()
+    o_ref, lse_ref = orc.naive_attention(f32(q), f32(k), f32(v), dense, sc, return_lse=True)
+    dq, dk, dv = orc.attention_backward(f32(q), f32(k), f32(v), dense, sc, f32(do))[:3]
+    for name, got, ref in zip(("o", "lse", "dq", "dk", "dv"), res, (o_ref, lse_ref, dq, dk, dv)):
+        ma, rl = errors(got, ref)
+        assert ma <= 2e-2 and (rl <= 1e-3 or ma <= 1e-5), (name, ma, rl)     # (a zero gradient has no relative error)
