@@ -1,0 +1,382 @@
+// The host path of the operator: what happens between a call in Python and the C ABI (include/bsattn.h), natively.
+// A small call is bound by it: argument checks, result and list allocation, workspace look-up, marshalling and the
+// autograd bookkeeping took 12 us per forward and over 100 us per training step in Python and ctypes.
+// The library itself is reached through its C ABI only, by the path Python gives to bind().
+//
+// Mirrors fa2_custom_mask/fa2_custom_mask.py:15-155 of the reference (build_groups_from_block_mask's lists, _attention).
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <dlfcn.h>
+#include <list>
+#include <mutex>
+#include "bsattn.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+
+namespace {
+
+// ---- the library ----
+struct Library {
+  decltype(&::bsattn_strerror) strerror_ = nullptr;
+  decltype(&::bsattn_mask_lists_workspace) lists_workspace = nullptr;
+  decltype(&::bsattn_block_mask_to_lists) lists = nullptr;
+  decltype(&::bsattn_fwd_workspace) fwd_workspace = nullptr;
+  decltype(&::bsattn_fwd_tokens) fwd = nullptr;
+  decltype(&::bsattn_fwd_block_mask_workspace) fwd_block_mask_workspace = nullptr;
+  decltype(&::bsattn_fwd_block_mask_tokens) fwd_block_mask = nullptr;
+  decltype(&::bsattn_bwd_workspace) bwd_workspace = nullptr;
+  decltype(&::bsattn_bwd_tokens) bwd = nullptr;
+} lib;
+
+void bind(const std::string& path) {
+  void* h = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+  TORCH_CHECK(h != nullptr, "cannot load ", path, ": ", dlerror());
+  auto get = [&](auto& f, const char* name) {
+    f = reinterpret_cast<std::decay_t<decltype(f)>>(dlsym(h, name));
+    TORCH_CHECK(f != nullptr, path, " has no ", name);
+  };
+  get(lib.strerror_, "bsattn_strerror");
+  get(lib.lists_workspace, "bsattn_mask_lists_workspace");
+  get(lib.lists, "bsattn_block_mask_to_lists");
+  get(lib.fwd_workspace, "bsattn_fwd_workspace");
+  get(lib.fwd, "bsattn_fwd_tokens");
+  get(lib.fwd_block_mask_workspace, "bsattn_fwd_block_mask_workspace");
+  get(lib.fwd_block_mask, "bsattn_fwd_block_mask_tokens");
+  get(lib.bwd_workspace, "bsattn_bwd_workspace");
+  get(lib.bwd, "bsattn_bwd_tokens");
+}
+
+void check(int rc, const char* what) {
+  if (rc != 0) throw std::runtime_error(std::string(what) + " failed: " + lib.strerror_(rc) + " (code " + std::to_string(rc) + ")");
+}
+
+int dtype_code(at::ScalarType t) {
+  if (t == at::kHalf) return BSATTN_F16;
+  if (t == at::kBFloat16) return BSATTN_BF16;
+  if (t == at::kFloat) return BSATTN_F32;
+  throw py::type_error(std::string("unsupported dtype ") + toString(t));
+}
+
+constexpr int64_t TILE = BSATTN_TILE;
+int64_t whole(int64_t n) { return (n + TILE - 1) / TILE * TILE; }
+
+hipStream_t stream_of(const Tensor& x) { return c10::hip::getCurrentHIPStream(x.device().index()).stream(); }
+
+// ---- workspaces ----
+// Scratch memory for one call, kept per (device, stream) and reused by the next call on that stream: the kernels need no
+// particular contents on entry, and what is enqueued on one stream runs in order.  The lock is held while a call is
+// enqueued, so that the launches of two threads on one stream, which share a workspace, do not interleave.  Bounded:
+// the least recently used stream's workspace goes first, one above WORKSPACE_CACHE_BYTES is not kept.  Nothing is kept
+// or taken from the cache while the stream is being captured: memory first allocated under capture belongs to the
+// graph's pool.
+constexpr size_t WORKSPACE_CACHE_STREAMS = 8, WORKSPACE_CACHE_BYTES = (size_t)256 << 20;
+struct Kept { int device; hipStream_t stream; Tensor memory; };
+std::mutex workspace_mutex;
+std::list<Kept>& workspaces() {       // most recently used last (never destroyed: tensors must not outlive the runtime)
+  static auto* list = new std::list<Kept>;
+  return *list;
+}
+
+Tensor workspace_locked(size_t bytes, at::Device device, hipStream_t stream) {
+  const auto fresh = [&] {
+    return at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(device));
+  };
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return fresh();
+  auto& kept = workspaces();
+  for (auto it = kept.begin(); it != kept.end(); ++it) {
+    if (it->device != device.index() || it->stream != stream) continue;
+    if ((size_t)it->memory.numel() < bytes) { kept.erase(it); break; }
+    if (std::next(it) != kept.end()) kept.splice(kept.end(), kept, it);
+    return kept.back().memory;
+  }
+  Tensor t = fresh();
+  if (bytes <= WORKSPACE_CACHE_BYTES) {
+    kept.push_back({device.index(), stream, t});
+    while (kept.size() > WORKSPACE_CACHE_STREAMS) kept.pop_front();
+  }
+  return t;
+}
+
+void clear_workspaces() {
+  std::lock_guard<std::mutex> lock(workspace_mutex);
+  workspaces().clear();
+}
+
+// ---- kept-tile lists ----
+// Of a block mask [Bm, Hm, nb, nb] (fixed shapes, no host synchronisation): row_ptr int32 [Bm*Hm*nb+1], col_idx int32
+// [Bm*Hm*nb*nb] (first T entries valid), counts int32 [2] = (G, T), groups int32 [Bm*Hm*nb, 5] (first G rows valid) or
+// none, all in one int32 buffer (workspace | row_ptr | counts | col_idx | groups).  Elementwise masks: per kept tile the
+// "partly set" flag and its packed 64 x 64 bits.
+struct TileLists : torch::CustomClassHolder {
+  int64_t Bm, Hm, nb, ws_bytes, off_ptr, off_counts, off_cols, off_groups;
+  bool has_groups;
+  Tensor buf, partial, bits;
+
+  TileLists(int64_t Bm_, int64_t Hm_, int64_t nb_, at::Device device, bool want_groups)
+      : Bm(Bm_), Hm(Hm_), nb(nb_), has_groups(want_groups) {
+    size_t bytes = 0;
+    check(lib.lists_workspace((int)Bm, (int)Hm, (int)nb, &bytes), "bsattn_mask_lists_workspace");
+    const int64_t rows = Bm * Hm * nb;
+    ws_bytes = (int64_t)bytes;
+    off_ptr = (ws_bytes + 3) / 4;
+    off_counts = off_ptr + rows + 1;
+    off_cols = off_counts + 2;
+    off_groups = off_cols + rows * nb;
+    buf = at::empty({off_groups + (want_groups ? rows * 5 : 0)}, at::TensorOptions().dtype(at::kInt).device(device));
+  }
+  int32_t* at_(int64_t off) const { return buf.data_ptr<int32_t>() + off; }
+  int32_t* row_ptr() const { return at_(off_ptr); }
+  int32_t* counts() const { return at_(off_counts); }
+  int32_t* col_idx() const { return at_(off_cols); }
+  int32_t* groups() const { return has_groups ? at_(off_groups) : nullptr; }
+  Tensor view(int64_t from, int64_t to) const { return buf.narrow(0, from, to - from); }
+};
+using ListsPtr = c10::intrusive_ptr<TileLists>;
+
+ListsPtr block_mask_to_lists(const Tensor& block, bool transpose, bool want_groups) {
+  c10::DeviceGuard guard(block.device());
+  auto lists = c10::make_intrusive<TileLists>(block.size(0), block.size(1), block.size(2), block.device(), want_groups);
+  const int64_t sm = block.stride(transpose ? 3 : 2), sn = block.stride(transpose ? 2 : 3);
+  check(lib.lists((const uint8_t*)block.const_data_ptr(), (int)lists->Bm, (int)lists->Hm, (int)lists->nb, block.stride(0),
+                  block.stride(1), sm, sn, lists->row_ptr(), lists->col_idx(), lists->groups(), lists->counts(),
+                  lists->at_(0), (size_t)lists->ws_bytes, stream_of(block)), "bsattn_block_mask_to_lists");
+  return lists;
+}
+
+// ---- q, k, v ----
+void check_qkv(const Tensor& q, const Tensor& k, const Tensor& v) {
+  if (!(q.is_cuda() && k.is_cuda() && v.is_cuda())) throw std::runtime_error("q, k, v must be GPU tensors (there is no CPU path)");
+  if (q.dim() != 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes())
+    throw py::value_error("q, k, v must share one shape [B, H, N, D]");            // :53-57
+  const auto t = q.scalar_type();
+  if ((t != at::kHalf && t != at::kBFloat16) || k.scalar_type() != t || v.scalar_type() != t)
+    throw py::type_error("q, k, v must all be float16 or all bfloat16");
+  const int64_t D = q.size(3);
+  if (D != 16 && D != 32 && D != 64 && D != 128 && D != 256)                       // :58
+    throw py::value_error("head dimension must be 16, 32, 64, 128 or 256");
+  if (q.size(2) < 1) throw py::value_error("empty sequence");
+}
+
+void check_mask_heads(int64_t Bm, int64_t Hm, const Tensor& q) {
+  if ((Bm != 1 && Bm != q.size(0)) || (Hm != 1 && Hm != q.size(1))) throw py::value_error("mask batch/head sizes must be 1 or match q");
+}
+
+// The kernels work on head dimensions 64, 128 and 256: smaller ones are embedded in zeros.  Zero columns change neither
+// q k^T nor the real columns of the output.
+Tensor padded(const Tensor& x) {
+  if (x.size(3) >= 64) return x;
+  Tensor p = at::zeros({x.size(0), x.size(1), x.size(2), 64}, x.options());
+  p.narrow(3, 0, x.size(3)).copy_(x);
+  return p;
+}
+Tensor unpadded(const Tensor& x, int64_t D) { return x.size(3) == D ? x : x.narrow(3, 0, D); }
+
+// Unit stride along the head dimension, 16-byte aligned rows.
+bool rows_aligned(const Tensor& x) {
+  const int64_t e = x.element_size();
+  return x.stride(3) == 1 && (((x.stride(0) | x.stride(1) | x.stride(2)) * e) & 15) == 0 && ((uintptr_t)x.const_data_ptr() & 15) == 0;
+}
+Tensor prepared(const Tensor& x) { return rows_aligned(x) ? x : x.clone(at::MemoryFormat::Contiguous); }
+
+// A result laid out as the reference's torch.empty_like(x) lays it out (:59, 101-103): the dimension order of x by
+// stride, without gaps.  For q, k, v sliced out of one packed [B, N, 3, H, D] tensor that is [B, N, H, D] order behind a
+// [B, H, N, D] shape.
+Tensor like(const Tensor& x, at::ScalarType dtype) {
+  Tensor t = at::empty_like(x, x.options().dtype(dtype));
+  return rows_aligned(t) ? t : at::empty(x.sizes(), x.options().dtype(dtype));
+}
+
+std::tuple<Tensor, Tensor> forward_core(const Tensor& q_, const Tensor& k_, const Tensor& v_, const TileLists& l, double sm_scale,
+                                        at::ScalarType out_dtype, bool want_lse) {
+  c10::DeviceGuard guard(q_.device());
+  const Tensor q = prepared(q_), k = prepared(k_), v = prepared(v_), o = like(q, out_dtype);
+  const int B = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3);
+  Tensor lse;
+  if (want_lse) lse = at::empty({B, H, N}, q.options().dtype(at::kFloat));
+  size_t bytes = 0;
+  check(lib.fwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_fwd_workspace");
+  const hipStream_t stream = stream_of(q);
+  std::lock_guard<std::mutex> lock(workspace_mutex);
+  const Tensor ws = workspace_locked(bytes, q.device(), stream);
+  const bool words = l.bits.defined();          // elementwise mask: exact inside partly set tiles
+  check(lib.fwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(), want_lse ? lse.data_ptr<float>() : nullptr,
+                l.row_ptr(), l.col_idx(), words ? (const uint8_t*)l.partial.const_data_ptr() : nullptr,
+                words ? (const uint64_t*)l.bits.const_data_ptr() : nullptr, (int)l.Bm, (int)l.Hm, B, H, N, D,
+                dtype_code(q.scalar_type()), dtype_code(out_dtype), (float)sm_scale, q.strides().data(), k.strides().data(),
+                v.strides().data(), o.strides().data(), ws.data_ptr(), bytes, stream), "bsattn_fwd");
+  return {o, lse};
+}
+
+std::tuple<Tensor, Tensor, Tensor> backward_core(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& o_,
+                                                 const Tensor& do_, const Tensor& lse, const TileLists& l, const TileLists& lt,
+                                                 double sm_scale, at::ScalarType out_dtype) {
+  c10::DeviceGuard guard(q_.device());
+  const Tensor q = prepared(q_), k = prepared(k_), v = prepared(v_), o = prepared(o_), g = prepared(do_);
+  const Tensor dq = like(q, out_dtype), dk = like(k, out_dtype), dv = like(v, out_dtype);       // :101-103
+  const int B = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3);
+  size_t bytes = 0;
+  check(lib.bwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_bwd_workspace");
+  const hipStream_t stream = stream_of(q);
+  std::lock_guard<std::mutex> lock(workspace_mutex);
+  const Tensor ws = workspace_locked(bytes, q.device(), stream);
+  const bool words = l.bits.defined();
+  check(lib.bwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.const_data_ptr(), g.const_data_ptr(),
+                lse.const_data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), l.row_ptr(), l.col_idx(), lt.row_ptr(),
+                lt.col_idx(), words ? (const uint64_t*)l.bits.const_data_ptr() : nullptr,
+                words ? (const uint64_t*)lt.bits.const_data_ptr() : nullptr, (int)l.Bm, (int)l.Hm, B, H, N, D,
+                dtype_code(q.scalar_type()), dtype_code(out_dtype), (float)sm_scale, q.strides().data(), k.strides().data(),
+                v.strides().data(), o.strides().data(), g.strides().data(), dq.strides().data(), dk.strides().data(),
+                dv.strides().data(), ws.data_ptr(), bytes, stream), "bsattn_bwd");
+  return {dq, dk, dv};
+}
+
+at::ScalarType result_type(const Tensor& q, bool out_fp32) { return out_fp32 ? at::kFloat : q.scalar_type(); }
+
+py::object results(const Tensor& o, const Tensor& lse, int64_t D, bool return_lse) {
+  if (return_lse) return py::make_tuple(unpadded(o, D), lse);
+  return py::cast(unpadded(o, D));
+}
+
+// Forward without anything kept for a backward.
+py::object forward(const Tensor& q, const Tensor& k, const Tensor& v, const ListsPtr& lists, double sm_scale, bool out_fp32,
+                   bool return_lse) {
+  check_qkv(q, k, v);
+  check_mask_heads(lists->Bm, lists->Hm, q);
+  at::NoGradGuard no_grad;
+  auto [o, lse] = forward_core(padded(q), padded(k), padded(v), *lists, sm_scale, result_type(q, out_fp32), return_lse);
+  return results(o, lse, q.size(3), return_lse);
+}
+
+// Lists and forward from one call into the library, for a block mask whose lists are not at hand: (results, lists).
+py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale, bool out_fp32,
+                             bool return_lse) {
+  check_qkv(q_, k_, v_);
+  check_mask_heads(mask.size(0), mask.size(1), q_);
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(q_.device());
+  const Tensor q = prepared(padded(q_)), k = prepared(padded(k_)), v = prepared(padded(v_));
+  const at::ScalarType out_dtype = result_type(q, out_fp32);
+  const Tensor o = like(q, out_dtype);
+  const int B = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3), Bm = (int)mask.size(0), Hm = (int)mask.size(1);
+  auto lists = c10::make_intrusive<TileLists>(Bm, Hm, mask.size(2), q.device(), false);
+  Tensor lse;
+  if (return_lse) lse = at::empty({B, H, N}, q.options().dtype(at::kFloat));
+  size_t bytes = 0;
+  check(lib.fwd_block_mask_workspace(Bm, Hm, B, H, (int)whole(N), D, &bytes), "bsattn_fwd_block_mask_workspace");
+  const hipStream_t stream = stream_of(q);
+  {
+    std::lock_guard<std::mutex> lock(workspace_mutex);
+    const Tensor ws = workspace_locked(bytes, q.device(), stream);
+    check(lib.fwd_block_mask(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(),
+                             return_lse ? lse.data_ptr<float>() : nullptr, (const uint8_t*)mask.const_data_ptr(),
+                             mask.strides().data(), Bm, Hm, lists->row_ptr(), lists->col_idx(), lists->counts(), B, H, N, D,
+                             dtype_code(q.scalar_type()), dtype_code(out_dtype), (float)sm_scale, q.strides().data(),
+                             k.strides().data(), v.strides().data(), o.strides().data(), ws.data_ptr(), bytes, stream),
+          "bsattn_fwd_block_mask");
+  }
+  return py::make_tuple(results(o, lse, q_.size(3), return_lse), lists);
+}
+
+// ---- autograd ----
+// forward(q, k, v, mask, sm_scale) and backward of the reference's _attention (:43-155) for a mask given by its lists;
+// two further arguments select an fp32 output and the LSE as second result.  Autograd hands gradients back in the type
+// of q, k, v.
+struct Attention : torch::autograd::Function<Attention> {
+  static variable_list forward(AutogradContext* ctx, const Variable& q_, const Variable& k_, const Variable& v_, const ListsPtr& lists,
+                               const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
+    const Tensor q = padded(q_), k = padded(k_), v = padded(v_);
+    auto [o, lse] = forward_core(q, k, v, *lists, sm_scale, result_type(q, out_fp32), true);
+    const Tensor out = unpadded(o, q_.size(3));
+    ctx->save_for_backward({q, k, v, out, lse});                         // :89
+    ctx->saved_data["lists"] = c10::IValue::make_capsule(lists);
+    ctx->saved_data["lists_t"] = c10::IValue::make_capsule(lists_t);
+    ctx->saved_data["sm_scale"] = sm_scale;
+    if (!return_lse) return {out};                                       // :94
+    ctx->mark_non_differentiable({lse});
+    return {out, lse};
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &out = saved[3], &lse = saved[4];
+    at::NoGradGuard no_grad;
+    const int64_t D = out.size(3);
+    const auto t = q.scalar_type();
+    const Tensor o = padded(out.scalar_type() == t ? out : out.to(t));
+    const Tensor g = grads[0].defined() ? padded(grads[0].scalar_type() == t ? grads[0] : grads[0].to(t)) : at::zeros_like(o);
+    const auto lists = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists"].toCapsule());
+    const auto lists_t = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists_t"].toCapsule());
+    auto [dq, dk, dv] = backward_core(q, k, v, o, g, lse, *lists, *lists_t, ctx->saved_data["sm_scale"].toDouble(), t);
+    return {unpadded(dq, D), unpadded(dk, D), unpadded(dv, D), Variable(), Variable(), Variable(), Variable(), Variable()};   // :155
+  }
+};
+
+py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const ListsPtr& lists, const ListsPtr& lists_t, double sm_scale,
+                     bool out_fp32, bool return_lse) {
+  check_qkv(q, k, v);
+  check_mask_heads(lists->Bm, lists->Hm, q);
+  variable_list r = Attention::apply(q, k, v, lists, lists_t, sm_scale, out_fp32, return_lse);
+  if (return_lse) return py::make_tuple(r[0], r[1]);
+  return py::cast(r[0]);
+}
+
+// (o, lse, dq, dk, dv) in one call, in the result type
+py::tuple forward_backward(const Tensor& q_, const Tensor& k_, const Tensor& v_, const ListsPtr& lists, const ListsPtr& lists_t,
+                           double sm_scale, const Tensor& do_, bool out_fp32) {
+  check_qkv(q_, k_, v_);
+  check_mask_heads(lists->Bm, lists->Hm, q_);
+  at::NoGradGuard no_grad;
+  const auto t = q_.scalar_type(), out_dtype = result_type(q_, out_fp32);
+  const int64_t D = q_.size(3);
+  const Tensor q = padded(q_), k = padded(k_), v = padded(v_);
+  auto [o, lse] = forward_core(q, k, v, *lists, sm_scale, out_dtype, true);
+  const Tensor g = padded(do_.scalar_type() == t ? do_ : do_.to(t));
+  auto [dq, dk, dv] = backward_core(q, k, v, o.scalar_type() == t ? o : o.to(t), g, lse, *lists, *lists_t, sm_scale, out_dtype);
+  return py::make_tuple(unpadded(o, D), lse, unpadded(dq, D), unpadded(dk, D), unpadded(dv, D));
+}
+
+std::optional<Tensor> defined_or_none(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+  m.def("bind", &bind);
+  m.def("check_qkv", [](const Tensor& q, const Tensor& k, const Tensor& v) { check_qkv(q, k, v); return q.size(2); });
+  m.def("clear_workspaces", &clear_workspaces);
+  m.def("workspace", [](size_t bytes, const Tensor& like) {
+    std::lock_guard<std::mutex> lock(workspace_mutex);
+    return workspace_locked(bytes, like.device(), stream_of(like));
+  });
+  m.def("block_mask_to_lists", &block_mask_to_lists);
+  m.def("forward", &forward);
+  m.def("forward_block_mask", &forward_block_mask);
+  m.def("attention", &attention);
+  m.def("forward_backward", &forward_backward);
+  py::class_<TileLists, ListsPtr>(m, "TileLists")
+      .def(py::init([](int64_t Bm, int64_t Hm, int64_t nb, py::object device, bool want_groups) {
+             return c10::make_intrusive<TileLists>(Bm, Hm, nb, at::Device(py::cast<std::string>(py::str(device))), want_groups);
+           }), py::arg("Bm"), py::arg("Hm"), py::arg("nb"), py::arg("device"), py::arg("want_groups") = false)
+      .def_readonly("Bm", &TileLists::Bm)
+      .def_readonly("Hm", &TileLists::Hm)
+      .def_readonly("nb", &TileLists::nb)
+      .def_readonly("buf", &TileLists::buf)
+      .def_readonly("has_groups", &TileLists::has_groups)
+      .def_property("partial", [](const TileLists& l) { return defined_or_none(l.partial); },
+                    [](TileLists& l, const std::optional<Tensor>& t) { l.partial = t ? *t : Tensor(); })
+      .def_property("bits", [](const TileLists& l) { return defined_or_none(l.bits); },
+                    [](TileLists& l, const std::optional<Tensor>& t) { l.bits = t ? *t : Tensor(); })
+      .def_property_readonly("row_ptr", [](const TileLists& l) { return l.view(l.off_ptr, l.off_counts); })
+      .def_property_readonly("counts", [](const TileLists& l) { return l.view(l.off_counts, l.off_cols); })
+      .def_property_readonly("col_idx", [](const TileLists& l) { return l.view(l.off_cols, l.off_groups); })
+      .def_property_readonly("groups", [](const TileLists& l) {
+        return l.has_groups ? std::optional<Tensor>(l.view(l.off_groups, l.buf.size(0)).view({-1, 5})) : std::nullopt;
+      })
+      .def_property_readonly("row_ptr_ptr", [](const TileLists& l) { return (uintptr_t)l.row_ptr(); })
+      .def_property_readonly("col_idx_ptr", [](const TileLists& l) { return (uintptr_t)l.col_idx(); });
+}

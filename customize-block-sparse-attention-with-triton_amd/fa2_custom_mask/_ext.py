@@ -1,4 +1,5 @@
-"""ctypes binding of libbsattn.so, the C-ABI library holding the gfx950 kernels.
+"""Loads libbsattn.so, the C-ABI library holding the gfx950 kernels (bound with ctypes here), and _host.so, the native
+host path between Python and that library.
 
 There is deliberately no fallback: if the library is missing, or a call returns an error
 code, a RuntimeError is raised.
@@ -74,6 +75,18 @@ def lib():
     return _lib
 
 
+def host():
+    """The module _host, bound to the library."""
+    try:
+        from . import _host
+    except ImportError as e:
+        raise RuntimeError("_host.so cannot be loaded (%s): build it with "
+                           "`python customize-block-sparse-attention-with-triton_amd/build.py`" % e) from e
+    lib()
+    _host.bind(LIB_PATH)
+    return _host
+
+
 def check(rc, what):
     if rc != 0:
         raise RuntimeError("%s failed: %s (code %d)" % (what, lib().bsattn_strerror(rc).decode(), rc))
@@ -106,13 +119,6 @@ def current_stream(device):
     return ctypes.c_void_p(raw_stream(device))
 
 
-@functools.lru_cache(maxsize=256)
-def mask_lists_workspace(Bm, Hm, nb):
-    n = ctypes.c_size_t()
-    check(lib().bsattn_mask_lists_workspace(Bm, Hm, nb, ctypes.byref(n)), "bsattn_mask_lists_workspace")
-    return n.value
-
-
 @functools.lru_cache(maxsize=64)
 def reorder_inplace_workspace(n_tensors, BS, NH, F, H, W, D, elem_bytes):
     """Bytes, or None where the in-place reorder does not take the shape."""
@@ -142,24 +148,8 @@ def _workspace_on(which, B, H, N, D, index):
     return n.value
 
 
-@functools.lru_cache(maxsize=256)
-def _fused_workspace_on(Bm, Hm, B, H, N, D, index):
-    n = ctypes.c_size_t()
-    if index >= 0 and index != torch.cuda.current_device():
-        with torch.cuda.device(index):
-            rc = lib().bsattn_fwd_block_mask_workspace(Bm, Hm, B, H, N, D, ctypes.byref(n))
-    else:
-        rc = lib().bsattn_fwd_block_mask_workspace(Bm, Hm, B, H, N, D, ctypes.byref(n))
-    check(rc, "bsattn_fwd_block_mask_workspace")
-    return n.value
-
-
 def _whole(N):
     return (N + 63) // 64 * 64
-
-
-def fwd_block_mask_workspace(Bm, Hm, B, H, N, D, device=None):
-    return _fused_workspace_on(Bm, Hm, B, H, _whole(N), D, _device_index(device))
 
 
 def fwd_workspace(B, H, N, D, device=None):

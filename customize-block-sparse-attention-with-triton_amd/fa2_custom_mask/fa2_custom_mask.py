@@ -4,14 +4,12 @@ Mirrors fa2_custom_mask/fa2_custom_mask.py of the reference: `build_groups_from_
 (:15-38) and the autograd function behind `flash_attention_custom_mask` (:40-157), with the
 device work done by hand-written gfx950 kernels reached through the C ABI in include/bsattn.h.
 """
-import collections
 import ctypes
 
 import torch
 
 from . import _ext
-from .utils import (TILE, TileLists, block_mask_to_lists, lists_cache, mask_to_lists, num_tiles, is_block_form,
-                    _check_mask)
+from .utils import TILE, _host, block_mask_to_lists, lists_cache, mask_to_lists, num_tiles, is_block_form, _check_mask
 
 
 def build_groups_from_block_mask(mask):
@@ -37,38 +35,9 @@ def _prep(x):
     return x
 
 
-_workspaces = collections.OrderedDict()
-WORKSPACE_CACHE_STREAMS = 8          # (device, stream) pairs whose workspace is kept
-WORKSPACE_CACHE_BYTES = 256 << 20    # a larger workspace serves its call and is then given back
-
-
 def clear_workspaces():
-    """Gives back the workspaces kept for reuse."""
-    _workspaces.clear()
-
-
-def _workspace(nbytes, device):
-    """Scratch memory for one call, kept per (device, stream) and reused by the next call on that stream:
-    the kernels need no particular contents on entry, and calls on one stream run one after the
-    other.  The cache is bounded (the least recently used stream's workspace goes first, a workspace above
-    WORKSPACE_CACHE_BYTES is not kept), and nothing is kept or taken from it while a graph is being captured:
-    memory first allocated under capture belongs to the graph's pool.  (Plans own their workspaces: they may be
-    replayed from graphs on any stream.)"""
-    raw = _ext.raw_stream(device)
-    handle = ctypes.c_void_p(raw)
-    if torch.cuda.is_current_stream_capturing():
-        return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device), handle
-    key = (device.index, raw)
-    ws = _workspaces.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-        if nbytes <= WORKSPACE_CACHE_BYTES:
-            _workspaces[key] = ws
-            while len(_workspaces) > WORKSPACE_CACHE_STREAMS:
-                _workspaces.popitem(last=False)
-    if key in _workspaces:
-        _workspaces.move_to_end(key)
-    return ws, handle
+    """Gives back the workspaces kept for reuse (one per device and stream, at most 8 and 256 MB each)."""
+    _host.clear_workspaces()
 
 
 def _like(x, dtype):
@@ -81,37 +50,6 @@ def _like(x, dtype):
     if t.stride(3) != 1 or any((s * t.element_size()) % 16 for s in t.stride()[:3]):
         t = torch.empty(x.shape, dtype=dtype, device=x.device)
     return t
-
-
-def _check_qkv(q, k, v, mask):
-    if not (q.is_cuda and k.is_cuda and v.is_cuda):
-        raise RuntimeError("q, k, v must be GPU tensors (there is no CPU path)")
-    if q.dim() != 4 or k.shape != q.shape or v.shape != q.shape:
-        raise ValueError("q, k, v must share one shape [B, H, N, D]")   # :53-57
-    if q.dtype not in (torch.float16, torch.bfloat16) or k.dtype != q.dtype or v.dtype != q.dtype:
-        raise TypeError("q, k, v must all be float16 or all bfloat16")
-    B, H, N, D = q.shape
-    if D not in (16, 32, 64, 128, 256):                                # :58
-        raise ValueError("head dimension must be 16, 32, 64, 128 or 256")
-    if N < 1:
-        raise ValueError("empty sequence")
-    if mask is None:
-        return B, H, N, D
-    _check_mask(mask)
-    if mask.shape[0] not in (1, B) or mask.shape[1] not in (1, H):
-        raise ValueError("mask batch/head sizes must be 1 or match q")
-    is_block_form(mask, N)                                              # raises on any other shape
-    return B, H, N, D
-
-
-def _padded(x):
-    """The kernels work on head dimensions 64, 128 and 256: smaller ones are embedded in zeros.  Zero columns change neither
-    q k^T nor the real columns of the output."""
-    if x.shape[3] >= 64:
-        return x
-    xp = x.new_zeros((x.shape[0], x.shape[1], x.shape[2], 64))
-    xp[:, :, :, :x.shape[3]] = x
-    return xp
 
 
 _all_true = {}
@@ -135,38 +73,10 @@ def set_deterministic(on):
     return bool(_ext.lib().bsattn_set_deterministic(1 if on else 0))
 
 
-def _plain(q, k, v):
-    """q, k, v of one shape without gaps and 16-byte aligned: one stride array serves all three and a result
-    laid out like them (the usual case, decided without looking at strides)."""
-    return (q.is_contiguous() and k.is_contiguous() and v.is_contiguous() and q.shape[3] % 8 == 0
-            and (q.data_ptr() | k.data_ptr() | v.data_ptr()) % 16 == 0)
-
-
-def _operands(q, k, v, out_dtype):
-    """(q, k, v, o, their four stride arrays) as the library takes them."""
-    if _plain(q, k, v):
-        o = torch.empty_like(q, dtype=out_dtype)                                # :59
-        sq = _ext.strides4(q)
-        return q, k, v, o, (sq, sq, sq, sq)
-    q, k, v = _prep(q), _prep(k), _prep(v)
-    o = _like(q, out_dtype)                                                     # :59
-    return q, k, v, o, (_ext.strides4(q), _ext.strides4(k), _ext.strides4(v), _ext.strides4(o))
-
-
 def _forward(q, k, v, lists, sm_scale, out_dtype, want_lse):
-    B, H, N, D = q.shape
-    q, k, v, o, strides = _operands(q, k, v, out_dtype)
-    lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device) if want_lse else None  # :70
-    wsb = _ext.fwd_workspace(B, H, N, D, q.device)
-    ws, stream = _workspace(wsb, q.device)
-    common = (lists.Bm, lists.Hm, B, H, N, D, _ext.dtype_code(q.dtype), _ext.dtype_code(out_dtype), float(sm_scale),
-              *strides, ws.data_ptr(), wsb, stream)
-    ptrs = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if want_lse else None,
-            lists.row_ptr_ptr, lists.col_idx_ptr)
-    words = (None, None) if lists.bits is None else (lists.partial.data_ptr(), lists.bits.data_ptr())   # elementwise mask: exact inside partly set tiles
-    rc = _ext.lib().bsattn_fwd_tokens(*ptrs, *words, *common)
-    _ext.check(rc, "bsattn_fwd")
-    return o, lse
+    """(o, lse or None) for lists that are at hand."""
+    r = _host.forward(q, k, v, lists, sm_scale, out_dtype == torch.float32, want_lse)
+    return r if want_lse else (r, None)
 
 
 class ForwardPlan:
@@ -201,27 +111,6 @@ class ForwardPlan:
         return self.o, self.lse
 
 
-def _backward(q, k, v, o, do, lse, lists, lists_t, sm_scale, out_dtype):
-    B, H, N, D = q.shape
-    q, k, v, o, do = _prep(q), _prep(k), _prep(v), _prep(o), _prep(do)
-    dq, dk, dv = _like(q, out_dtype), _like(k, out_dtype), _like(v, out_dtype)   # :101-103
-    wsb = _ext.bwd_workspace(B, H, N, D, q.device)
-    ws, stream = _workspace(wsb, q.device)
-    tensors = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), do.data_ptr(), lse.data_ptr(),
-               dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-               lists.row_ptr_ptr, lists.col_idx_ptr, lists_t.row_ptr_ptr,
-               lists_t.col_idx_ptr)
-    common = (lists.Bm, lists.Hm, B, H, N, D,
-              _ext.dtype_code(q.dtype), _ext.dtype_code(out_dtype), float(sm_scale),
-              _ext.strides4(q), _ext.strides4(k), _ext.strides4(v), _ext.strides4(o), _ext.strides4(do),
-              _ext.strides4(dq), _ext.strides4(dk), _ext.strides4(dv),
-              ws.data_ptr(), wsb, stream)
-    words = (None, None) if lists.bits is None else (lists.bits.data_ptr(), lists_t.bits.data_ptr())   # elementwise mask
-    rc = _ext.lib().bsattn_bwd_tokens(*tensors, *words, *common)
-    _ext.check(rc, "bsattn_bwd")
-    return dq, dk, dv
-
-
 class BackwardPlan:
     """The backward counterpart of ForwardPlan: dq, dk, dv and the workspace allocated once, the C
     arguments marshalled once; run() only enqueues the kernels.  o and lse are the forward's
@@ -254,86 +143,41 @@ class BackwardPlan:
         return self.dq, self.dk, self.dv
 
 
-def _forward_from_block_mask(q, k, v, mask, sm_scale, out_dtype, want_lse):
-    """Lists and forward from one call into the library (bsattn_fwd_block_mask), for a block mask whose lists
-    are not in the cache: one buffer for the lists, one for the result, and the stream's workspace."""
-    B, H, N, D = q.shape
-    Bm, Hm, nb = mask.shape[0], mask.shape[1], mask.shape[2]
-    q, k, v, o, strides = _operands(q, k, v, out_dtype)
-    lists = TileLists(Bm, Hm, nb, q.device)
-    lse = torch.empty((B, H, N), dtype=torch.float32, device=q.device) if want_lse else None
-    wsb = _ext.fwd_block_mask_workspace(Bm, Hm, B, H, N, D, q.device)
-    ws, stream = _workspace(wsb, q.device)
-    rc = _ext.lib().bsattn_fwd_block_mask_tokens(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr() if want_lse else None,
-        mask.data_ptr(), _ext.strides4(mask), Bm, Hm, lists.row_ptr_ptr, lists.col_idx_ptr, lists.counts_ptr,
-        B, H, N, D, _ext.dtype_code(q.dtype), _ext.dtype_code(out_dtype), float(sm_scale),
-        *strides, ws.data_ptr(), wsb, stream)
-    _ext.check(rc, "bsattn_fwd_block_mask")
-    return o, lse, lists
-
-
-def _forward_only(q, k, v, mask, sm_scale, out_fp32, return_lse):
-    """The forward of _attention without anything kept for a backward."""
-    B, H, N, D = _check_qkv(q, k, v, mask)
+def _mask_of(q, k, v, mask):
+    """(mask, N); mask=None is the dense mask."""
+    N = _host.check_qkv(q, k, v)
     if mask is None:
         mask = _dense_mask(q.device, num_tiles(N))
-    out_dtype = torch.float32 if out_fp32 else q.dtype
+    return mask, N
+
+
+def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
+    mask, N = _mask_of(q, k, v, mask)
     lists = lists_cache.get(mask, N, False)
-    if D < 64:
-        q, k, v = _padded(q), _padded(k), _padded(v)
-    if lists is None and is_block_form(mask, N):
-        # a block mask seen for the first time (or one that changes with every call): lists and forward in one call
-        o, lse, lists = _forward_from_block_mask(q, k, v, mask, sm_scale, out_dtype, return_lse)
-        lists_cache.put(mask, N, False, lists)
-    else:
+    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+        # (the backward walks the column lists: both orientations are made here)
         if lists is None:
-            lists = mask_to_lists(mask, N)
-        o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, return_lse)
-    if D < 64:
-        o = o[:, :, :, :D]
-    return (o, lse) if return_lse else o
+            lists = mask_to_lists(mask, N, both=True)                        # :48
+        return _host.attention(q, k, v, lists, mask_to_lists(mask, N, transpose=True), sm_scale, out_fp32, return_lse)
+    if lists is None:
+        _check_mask(mask)
+        if is_block_form(mask, N):
+            # a block mask seen for the first time (or one that changes with every call): lists and forward in one call
+            result, lists = _host.forward_block_mask(q, k, v, mask, sm_scale, out_fp32, return_lse)
+            lists_cache.put(mask, N, False, lists)
+            return result
+        lists = mask_to_lists(mask, N)
+    return _host.forward(q, k, v, lists, sm_scale, out_fp32, return_lse)
 
 
-class _attention(torch.autograd.Function):
-    """forward(q, k, v, mask, sm_scale) as the reference (fa2_custom_mask.py:43-94); two extra
-    trailing arguments select an fp32 output and the LSE as second result."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, mask=None, sm_scale=1.3, out_fp32=False, return_lse=False):
-        B, H, N, D = _check_qkv(q, k, v, mask)
-        if mask is None:
-            mask = _dense_mask(q.device, num_tiles(N))
-        # (a backward will ask for the column lists too when a gradient is wanted)
-        lists = mask_to_lists(mask, N, both=any(ctx.needs_input_grad[:3]))   # :48
-        out_dtype = torch.float32 if out_fp32 else q.dtype
-        q, k, v = _padded(q), _padded(k), _padded(v)
-        o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, True)
-        ctx.save_for_backward(q, k, v, o, lse, mask)                         # :89
-        ctx.lists = lists
-        ctx.sm_scale = sm_scale
-        ctx.out_dtype = out_dtype
-        ctx.return_lse = return_lse
-        ctx.shape = (N, D)
-        if D < 64:
-            o = o[:, :, :, :D]
-        if return_lse:
-            ctx.mark_non_differentiable(lse)
-            return o, lse
-        return o                                                              # :94
+class _attention:
+    """What the reference's autograd function offers (fa2_custom_mask.py:40-155): apply(q, k, v, mask, sm_scale); two extra
+    trailing arguments select an fp32 output and the LSE as second result.  The function itself is Attention in
+    csrc/host.cpp."""
 
     @staticmethod
-    def backward(ctx, do, *unused):
-        q, k, v, o, lse, mask = ctx.saved_tensors
-        N, D = ctx.shape
-        lists_t = mask_to_lists(mask, N, transpose=True)
-        o_in = o if o.dtype == q.dtype else o.to(q.dtype)
-        do_in = _padded(do if do.dtype == q.dtype else do.to(q.dtype))
-        # autograd hands gradients back in the dtype of q, k, v
-        dq, dk, dv = _backward(q, k, v, o_in, do_in, lse, ctx.lists, lists_t, ctx.sm_scale, q.dtype)
-        if D < 64:
-            dq, dk, dv = dq[:, :, :, :D], dk[:, :, :, :D], dv[:, :, :, :D]
-        return dq, dk, dv, None, None, None, None                            # :155
+    def apply(q, k, v, mask=None, sm_scale=1.3, out_fp32=False, return_lse=False):
+        return _attend(q, k, v, mask, sm_scale, out_fp32, return_lse)
 
 
 def flash_attention_custom_mask(q, k, v, mask=None, sm_scale=1.3):
@@ -344,35 +188,20 @@ def flash_attention_custom_mask(q, k, v, mask=None, sm_scale=1.3):
     block mask then covers the remaining tokens).  D = 16 and 32 cost one zero-padded copy of
     q, k, v per call.  The kept-tile lists of a mask tensor are cached
     until the tensor is modified.  When no gradient can be asked for (gradients disabled, or none of q, k, v
-    requires one) the call does not go through torch.autograd.Function, which costs about as much host time
-    as everything else in a small call."""
-    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)):
-        return _forward_only(q, k, v, mask, sm_scale, False, False)
-    return _attention.apply(q, k, v, mask, sm_scale)
+    requires one) nothing is kept for a backward."""
+    return _attend(q, k, v, mask, sm_scale, False, False)
 
 
 def flash_attention_custom_mask_lse(q, k, v, mask, sm_scale, out_fp32=False):
     """Same operator, also returning the natural-log logsumexp [B,H,N] fp32 of the kept scaled
     scores; out_fp32=True returns O in fp32.  (Not in the reference, whose second output M is
     only the running maximum: fa2_fwd.py:194-196.)"""
-    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)):
-        return _forward_only(q, k, v, mask, sm_scale, out_fp32, True)
-    return _attention.apply(q, k, v, mask, sm_scale, out_fp32, True)
+    return _attend(q, k, v, mask, sm_scale, out_fp32, True)
 
 
 def attention_forward_backward(q, k, v, mask, sm_scale, do, out_fp32=False):
     """Non-autograd entry: (o, lse, dq, dk, dv) in one call; with out_fp32 all five results
     are fp32 (autograd itself can only hand back gradients in the dtype of q)."""
-    B, H, N, D = _check_qkv(q, k, v, mask)
-    if mask is None:
-        mask = _dense_mask(q.device, num_tiles(N))
+    mask, N = _mask_of(q, k, v, mask)
     lists = mask_to_lists(mask, N, both=True)
-    lists_t = mask_to_lists(mask, N, transpose=True)
-    out_dtype = torch.float32 if out_fp32 else q.dtype
-    q, k, v = _padded(q), _padded(k), _padded(v)
-    o, lse = _forward(q, k, v, lists, sm_scale, out_dtype, True)
-    o_in = o if o.dtype == q.dtype else o.to(q.dtype)
-    dq, dk, dv = _backward(q, k, v, o_in, _padded(do.to(q.dtype)), lse, lists, lists_t, sm_scale, out_dtype)
-    if D < 64:
-        o, dq, dk, dv = o[:, :, :, :D], dq[:, :, :, :D], dk[:, :, :, :D], dv[:, :, :, :D]
-    return o, lse, dq, dk, dv
+    return _host.forward_backward(q, k, v, lists, mask_to_lists(mask, N, transpose=True), sm_scale, do, out_fp32)

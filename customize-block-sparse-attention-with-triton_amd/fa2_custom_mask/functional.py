@@ -6,7 +6,7 @@ import ctypes
 import torch
 
 from . import _ext
-from .fa2_custom_mask import _workspace
+from .utils import _host
 
 _PERMUTATIONS = [[0, 1, 2], [0, 2, 1], [1, 2, 0], [1, 0, 2], [2, 1, 0], [2, 0, 1]]       # functional.py:23-26
 _PERMUTATIONS_INV = [[0, 1, 2], [0, 2, 1], [2, 0, 1], [1, 0, 2], [2, 1, 0], [1, 2, 0]]   # functional.py:69-76
@@ -68,12 +68,12 @@ def _reorder_image_tokens(tensors, idx, inverse, F, H, W, n_text_tokens):
             numbers = _table(x.device)[2][idx]
         if numbers.shape == (NH,):
             n = len(image)
-            ws, stream = _workspace(wsb, x.device)
+            ws = _host.workspace(wsb, x)
             strides = (ctypes.c_int64 * (3 * n))(*[s for v in image for s in v.stride()[:3]])
             ptrs = (ctypes.c_void_p * n)(*[v.data_ptr() for v in image])
             rc = _ext.lib().bsattn_reorder_inplace(
                 ptrs, strides, n, BS, NH, F, H, W, D, x.element_size(), numbers.data_ptr(), numbers.element_size(),
-                1 if inverse else 0, ws.data_ptr(), wsb, stream)
+                1 if inverse else 0, ws.data_ptr(), wsb, _ext.current_stream(x.device))
             _ext.check(rc, "bsattn_reorder_inplace")
             for t in tensors:
                 if not t.is_inference():

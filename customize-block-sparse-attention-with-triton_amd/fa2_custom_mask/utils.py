@@ -2,12 +2,14 @@
 
 `is_hip` / `keep` keep the names exported by the reference (fa2_custom_mask/utils.py:3-14).
 """
-import ctypes
+import collections
 import weakref
 
 import torch
 
 from . import _ext
+
+_host = _ext.host()
 
 TILE = 64
 
@@ -23,59 +25,8 @@ def keep(conf):
     return True
 
 
-class TileLists:
-    """Device-resident kept-tile lists of a block mask [Bm, Hm, nb, nb] (fixed shapes, no
-    host synchronisation): row_ptr int32 [Bm*Hm*nb+1], col_idx int32 [Bm*Hm*nb*nb] (first T
-    entries valid), counts int32 [2] = (G, T), groups int32 [Bm*Hm*nb, 5] (first G rows
-    valid) or None.  All of them live in one int32 buffer (workspace | row_ptr | counts | col_idx | groups);
-    the tensor views are made when first asked for, the calls into the library only need the addresses."""
-
-    __slots__ = ("buf", "Bm", "Hm", "nb", "has_groups", "partial", "bits", "_views",
-                 "ws_ptr", "ws_bytes", "row_ptr_ptr", "counts_ptr", "col_idx_ptr", "groups_ptr", "_off")
-
-    def __init__(self, Bm, Hm, nb, device, want_groups=False):
-        rows = Bm * Hm * nb
-        wsb = _ext.mask_lists_workspace(Bm, Hm, nb)
-        o_ptr = (wsb + 3) // 4
-        o_counts = o_ptr + rows + 1
-        o_cols = o_counts + 2
-        o_groups = o_cols + rows * nb
-        self.buf = torch.empty(o_groups + (rows * 5 if want_groups else 0), dtype=torch.int32, device=device)
-        self.Bm, self.Hm, self.nb, self.has_groups = Bm, Hm, nb, want_groups
-        self._off = (o_ptr, o_counts, o_cols, o_groups)
-        base = self.buf.data_ptr()
-        self.ws_ptr, self.ws_bytes = base, wsb
-        self.row_ptr_ptr, self.counts_ptr = base + 4 * o_ptr, base + 4 * o_counts
-        self.col_idx_ptr = base + 4 * o_cols
-        self.groups_ptr = base + 4 * o_groups if want_groups else None
-        # elementwise masks only: per kept tile "partly set" flag and packed 64 x 64 bits
-        self.partial, self.bits = None, None
-        self._views = None
-
-    def _make_views(self):
-        if self._views is None:
-            o_ptr, o_counts, o_cols, o_groups = self._off
-            b = self.buf
-            rows = self.Bm * self.Hm * self.nb
-            self._views = (b[o_ptr:o_counts], b[o_counts:o_cols], b[o_cols:o_groups],
-                           b[o_groups:].view(rows, 5) if self.has_groups else None)
-        return self._views
-
-    @property
-    def row_ptr(self):
-        return self._make_views()[0]
-
-    @property
-    def counts(self):
-        return self._make_views()[1]
-
-    @property
-    def col_idx(self):
-        return self._make_views()[2]
-
-    @property
-    def groups(self):
-        return self._make_views()[3]
+# Device-resident kept-tile lists of a block mask (csrc/host.cpp)
+TileLists = _host.TileLists
 
 
 def _check_mask(mask):
@@ -112,15 +63,7 @@ def block_mask_to_lists(block, transpose=False, want_groups=False):
     Bm, Hm, nb, nb2 = block.shape
     if nb != nb2:
         raise ValueError("block mask must be square")
-    lists = TileLists(Bm, Hm, nb, block.device, want_groups)
-    sb, sh, sm, sn = block.stride()
-    if transpose:
-        sm, sn = sn, sm
-    rc = _ext.lib().bsattn_block_mask_to_lists(
-        block.data_ptr(), Bm, Hm, nb, sb, sh, sm, sn, lists.row_ptr_ptr, lists.col_idx_ptr,
-        lists.groups_ptr, lists.counts_ptr, lists.ws_ptr, lists.ws_bytes, _ext.current_stream(block.device))
-    _ext.check(rc, "bsattn_block_mask_to_lists")
-    return lists
+    return _host.block_mask_to_lists(block, transpose, want_groups)
 
 
 def pack_mask_tiles(mask, lists, transpose=False):
@@ -232,8 +175,8 @@ class _ListsCache:
 
     def __init__(self, capacity=8):
         self.capacity = capacity
-        # (weakref to mask, version, N, transpose, lists, stream the lists were built on), most recent last
-        self._entries = []
+        # (id of mask, N, transpose) -> (weakref to mask, version, lists, stream the lists were built on), most recent last
+        self._entries = collections.OrderedDict()
 
     @staticmethod
     def _version(mask):
@@ -245,32 +188,37 @@ class _ListsCache:
             return None
 
     def get(self, mask, N, transpose):
-        version = self._version(mask)
-        if version is None:
+        key = (id(mask), N, transpose)
+        entry = self._entries.get(key)
+        if entry is None:
             return None
-        for i, (ref, ver, n, tr, lists, stream) in enumerate(self._entries):
-            if ref() is mask and ver == version and n == N and tr == transpose:
-                if i != len(self._entries) - 1:
-                    self._entries.append(self._entries.pop(i))
-                # the lists were filled by kernels on `stream` (a raw handle): work on another stream waits for
-                # what that stream has been given so far (no event is recorded when the lists are made: a mask
-                # that changes with every call would pay for it every time)
-                if _ext.raw_stream(mask.device) != stream:
-                    torch.cuda.current_stream(mask.device).wait_stream(
-                        torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
-                return lists
-        return None
+        ref, version, lists, stream = entry
+        if ref() is not mask or self._version(mask) != version:
+            return None
+        self._entries.move_to_end(key)
+        # the lists were filled by kernels on `stream` (a raw handle): work on another stream waits for
+        # what that stream has been given so far (no event is recorded when the lists are made: a mask
+        # that changes with every call would pay for it every time)
+        if _ext.raw_stream(mask.device) != stream:
+            torch.cuda.current_stream(mask.device).wait_stream(
+                torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
+        return lists
 
     def put(self, mask, N, transpose, lists):
         version = self._version(mask)
         if version is None:
             return
+        key = (id(mask), N, transpose)
+        self._entries.pop(key, None)
         if len(self._entries) >= self.capacity:
-            self._entries = [e for e in self._entries if e[0]() is not None][-(self.capacity - 1):]
-        self._entries.append((weakref.ref(mask), version, N, transpose, lists, _ext.raw_stream(mask.device)))
+            for dead in [k for k, e in self._entries.items() if e[0]() is None]:
+                del self._entries[dead]
+            while len(self._entries) >= self.capacity:
+                self._entries.popitem(last=False)
+        self._entries[key] = (weakref.ref(mask), version, lists, _ext.raw_stream(mask.device))
 
     def clear(self):
-        self._entries = []
+        self._entries.clear()
         if "grid_cache" in globals():
             grid_cache.clear()
 
