@@ -70,19 +70,34 @@ hipStream_t stream_of(const Tensor& x) { return c10::hip::getCurrentHIPStream(x.
 // ---- workspaces ----
 // Scratch memory for one call, kept per (device, stream) and reused by the next call on that stream: the kernels need no
 // particular contents on entry, and what is enqueued on one stream runs in order.  The lock is held while a call is
-// enqueued, so that the launches of two threads on one stream, which share a workspace, do not interleave.  Bounded:
-// the least recently used stream's workspace goes first, one above WORKSPACE_CACHE_BYTES is not kept.  Nothing is kept
-// or taken from the cache while the stream is being captured: memory first allocated under capture belongs to the
-// graph's pool.
+// enqueued, so that the launches of two threads on one stream, which share a workspace, do not interleave.  The token
+// reorder, whose one launch is not made under the lock, has a workspace of its own: it may land between the launches of
+// an attention call.  Bounded: the least recently used workspace goes first, one above WORKSPACE_CACHE_BYTES is not
+// kept.  Nothing is kept or taken from the cache while the stream is being captured: memory first allocated under
+// capture belongs to the graph's pool.
 constexpr size_t WORKSPACE_CACHE_STREAMS = 8, WORKSPACE_CACHE_BYTES = (size_t)256 << 20;
-struct Kept { int device; hipStream_t stream; Tensor memory; };
+enum class Use { attention, reorder };
+struct Kept { int device; hipStream_t stream; Use use; Tensor memory; };
 std::mutex workspace_mutex;
+// The lock, waited for without the GIL: its holder may need the GIL (backward runs on threads that do not have it).
+struct WorkspaceLock {
+  std::unique_lock<std::mutex> lock{workspace_mutex, std::try_to_lock};
+  WorkspaceLock() {
+    if (lock.owns_lock()) return;
+    if (PyGILState_Check()) {
+      py::gil_scoped_release release;
+      lock.lock();
+    } else {
+      lock.lock();
+    }
+  }
+};
 std::list<Kept>& workspaces() {       // most recently used last (never destroyed: tensors must not outlive the runtime)
   static auto* list = new std::list<Kept>;
   return *list;
 }
 
-Tensor workspace_locked(size_t bytes, at::Device device, hipStream_t stream) {
+Tensor workspace_locked(size_t bytes, at::Device device, hipStream_t stream, Use use = Use::attention) {
   const auto fresh = [&] {
     return at::empty({(int64_t)std::max<size_t>(bytes, 1)}, at::TensorOptions().dtype(at::kByte).device(device));
   };
@@ -90,21 +105,21 @@ Tensor workspace_locked(size_t bytes, at::Device device, hipStream_t stream) {
   if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return fresh();
   auto& kept = workspaces();
   for (auto it = kept.begin(); it != kept.end(); ++it) {
-    if (it->device != device.index() || it->stream != stream) continue;
+    if (it->device != device.index() || it->stream != stream || it->use != use) continue;
     if ((size_t)it->memory.numel() < bytes) { kept.erase(it); break; }
     if (std::next(it) != kept.end()) kept.splice(kept.end(), kept, it);
     return kept.back().memory;
   }
   Tensor t = fresh();
   if (bytes <= WORKSPACE_CACHE_BYTES) {
-    kept.push_back({device.index(), stream, t});
+    kept.push_back({device.index(), stream, use, t});
     while (kept.size() > WORKSPACE_CACHE_STREAMS) kept.pop_front();
   }
   return t;
 }
 
 void clear_workspaces() {
-  std::lock_guard<std::mutex> lock(workspace_mutex);
+  const WorkspaceLock lock;
   workspaces().clear();
 }
 
@@ -202,7 +217,7 @@ std::tuple<Tensor, Tensor> forward_core(const Tensor& q_, const Tensor& k_, cons
   size_t bytes = 0;
   check(lib.fwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_fwd_workspace");
   const hipStream_t stream = stream_of(q);
-  std::lock_guard<std::mutex> lock(workspace_mutex);
+  const WorkspaceLock lock;
   const Tensor ws = workspace_locked(bytes, q.device(), stream);
   const bool words = l.bits.defined();          // elementwise mask: exact inside partly set tiles
   check(lib.fwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(), want_lse ? lse.data_ptr<float>() : nullptr,
@@ -223,7 +238,7 @@ std::tuple<Tensor, Tensor, Tensor> backward_core(const Tensor& q_, const Tensor&
   size_t bytes = 0;
   check(lib.bwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_bwd_workspace");
   const hipStream_t stream = stream_of(q);
-  std::lock_guard<std::mutex> lock(workspace_mutex);
+  const WorkspaceLock lock;
   const Tensor ws = workspace_locked(bytes, q.device(), stream);
   const bool words = l.bits.defined();
   check(lib.bwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.const_data_ptr(), g.const_data_ptr(),
@@ -271,7 +286,7 @@ py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v
   check(lib.fwd_block_mask_workspace(Bm, Hm, B, H, (int)whole(N), D, &bytes), "bsattn_fwd_block_mask_workspace");
   const hipStream_t stream = stream_of(q);
   {
-    std::lock_guard<std::mutex> lock(workspace_mutex);
+    const WorkspaceLock lock;
     const Tensor ws = workspace_locked(bytes, q.device(), stream);
     check(lib.fwd_block_mask(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(),
                              return_lse ? lse.data_ptr<float>() : nullptr, (const uint8_t*)mask.const_data_ptr(),
@@ -288,12 +303,12 @@ py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v
 // two further arguments select an fp32 output and the LSE as second result.  Autograd hands gradients back in the type
 // of q, k, v.
 struct Attention : torch::autograd::Function<Attention> {
-  static variable_list forward(AutogradContext* ctx, const Variable& q_, const Variable& k_, const Variable& v_, const ListsPtr& lists,
-                               const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
+  static variable_list forward(AutogradContext* ctx, const Variable& q_, const Variable& k_, const Variable& v_, const Variable& mask,
+                               const ListsPtr& lists, const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
     const Tensor q = padded(q_), k = padded(k_), v = padded(v_);
     auto [o, lse] = forward_core(q, k, v, *lists, sm_scale, result_type(q, out_fp32), true);
     const Tensor out = unpadded(o, q_.size(3));
-    ctx->save_for_backward({q, k, v, out, lse});                         // :89
+    ctx->save_for_backward({q, k, v, out, lse, mask});                   // :89 (a mask written to before the backward is refused)
     ctx->saved_data["lists"] = c10::IValue::make_capsule(lists);
     ctx->saved_data["lists_t"] = c10::IValue::make_capsule(lists_t);
     ctx->saved_data["sm_scale"] = sm_scale;
@@ -313,15 +328,15 @@ struct Attention : torch::autograd::Function<Attention> {
     const auto lists = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists"].toCapsule());
     const auto lists_t = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists_t"].toCapsule());
     auto [dq, dk, dv] = backward_core(q, k, v, o, g, lse, *lists, *lists_t, ctx->saved_data["sm_scale"].toDouble(), t);
-    return {unpadded(dq, D), unpadded(dk, D), unpadded(dv, D), Variable(), Variable(), Variable(), Variable(), Variable()};   // :155
+    return {unpadded(dq, D), unpadded(dk, D), unpadded(dv, D), Variable(), Variable(), Variable(), Variable(), Variable(), Variable()};   // :155
   }
 };
 
-py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const ListsPtr& lists, const ListsPtr& lists_t, double sm_scale,
-                     bool out_fp32, bool return_lse) {
+py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, const ListsPtr& lists,
+                     const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
   check_qkv(q, k, v);
   check_mask_heads(lists->Bm, lists->Hm, q);
-  variable_list r = Attention::apply(q, k, v, lists, lists_t, sm_scale, out_fp32, return_lse);
+  variable_list r = Attention::apply(q, k, v, mask, lists, lists_t, sm_scale, out_fp32, return_lse);
   if (return_lse) return py::make_tuple(r[0], r[1]);
   return py::cast(r[0]);
 }
@@ -349,9 +364,10 @@ PYBIND11_MODULE(_host, m) {
   m.def("bind", &bind);
   m.def("check_qkv", [](const Tensor& q, const Tensor& k, const Tensor& v) { check_qkv(q, k, v); return q.size(2); });
   m.def("clear_workspaces", &clear_workspaces);
-  m.def("workspace", [](size_t bytes, const Tensor& like) {
-    std::lock_guard<std::mutex> lock(workspace_mutex);
-    return workspace_locked(bytes, like.device(), stream_of(like));
+  m.def("reorder_workspace", [](size_t bytes, const Tensor& like) {
+    const WorkspaceLock lock;
+    // (a view: the kept tensor itself never has a Python object, so it can be dropped without the GIL)
+    return workspace_locked(bytes, like.device(), stream_of(like), Use::reorder).view({-1});
   });
   m.def("block_mask_to_lists", &block_mask_to_lists);
   m.def("forward", &forward);

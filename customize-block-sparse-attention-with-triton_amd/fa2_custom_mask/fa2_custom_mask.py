@@ -158,7 +158,7 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
         # (the backward walks the column lists: both orientations are made here)
         if lists is None:
             lists = mask_to_lists(mask, N, both=True)                        # :48
-        return _host.attention(q, k, v, lists, mask_to_lists(mask, N, transpose=True), sm_scale, out_fp32, return_lse)
+        return _host.attention(q, k, v, mask, lists, mask_to_lists(mask, N, transpose=True), sm_scale, out_fp32, return_lse)
     if lists is None:
         _check_mask(mask)
         if is_block_form(mask, N):

@@ -68,7 +68,7 @@ def _reorder_image_tokens(tensors, idx, inverse, F, H, W, n_text_tokens):
             numbers = _table(x.device)[2][idx]
         if numbers.shape == (NH,):
             n = len(image)
-            ws = _host.workspace(wsb, x)
+            ws = _host.reorder_workspace(wsb, x)
             strides = (ctypes.c_int64 * (3 * n))(*[s for v in image for s in v.stride()[:3]])
             ptrs = (ctypes.c_void_p * n)(*[v.data_ptr() for v in image])
             rc = _ext.lib().bsattn_reorder_inplace(

@@ -66,3 +66,62 @@ def test_gradients_in_odd_layouts(dev, deterministic, D):
     q1, k1, v1 = q.detach(), k.detach().requires_grad_(True), v.detach()
     only_k = torch.autograd.grad(fm.flash_attention_custom_mask(q1, k1, v1, mask, 0.2), k1, torch.ones_like(q))[0]
     assert torch.equal(only_k, ref[1])
+
+
+def test_reorder_beside_training_on_one_stream(dev, deterministic):
+    """One thread reorders tokens (sizes that grow, so its workspace is replaced) while two train on the same stream: the
+    gradients equal those of the step made alone."""
+    import fa2_custom_mask as fm
+    q, k, v, do = [x.to(dev) for x in make_qkv(1, 4, 900, 64, torch.float16, 730, n=4)]
+    mask = uniform_block_mask(1, 1, 15, 0.5, 731).to(dev)
+    for x in (q, k, v):
+        x.requires_grad_(True)
+
+    def step():
+        o = fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+        return torch.autograd.grad(o, (q, k, v), do)
+
+    alone = step()
+    torch.cuda.synchronize()
+    runs, moved = [], []
+
+    def reorder():
+        for heads in range(1, 41):
+            x = torch.randn(1, heads, 2 * 3 * 64, 64, device=dev, dtype=torch.float16)
+            plan = {"permute": [torch.full((heads,), 4, device=dev)]}
+            y = fm.inv_permute_attn_triton(fm.permute_qkv_triton(x.clone(), x.clone(), x.clone(), plan, 0, 2, 3, 64, 0)[0], plan, 0, 2, 3, 64, 0)
+            moved.append(torch.equal(x, y))
+
+    threads = [threading.Thread(target=reorder)]
+    threads += [threading.Thread(target=lambda: runs.extend(step() for _ in range(40))) for _ in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert len(runs) == 80 and len(moved) == 40 and all(moved)
+    for run in runs:
+        assert all(torch.equal(a, b) for a, b in zip(run, alone))
+
+
+def test_mask_written_before_the_backward_is_refused(dev):
+    import fa2_custom_mask as fm
+    q, k, v = [x.to(dev).requires_grad_(True) for x in make_qkv(1, 1, 128, 64, torch.float16, 740)]
+    mask = uniform_block_mask(1, 1, 2, 1.0, 741).to(dev)
+    o = fm.flash_attention_custom_mask(q, k, v, mask, 0.2)
+    mask[0, 0, 0, 1] = False
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        o.backward(torch.ones_like(o))
+
+
+def test_transforms_are_refused(dev):
+    """vmap and forward-mode differentiation of the autograd function have no rule and raise."""
+    import fa2_custom_mask as fm
+    import torch.autograd.forward_ad as fwad
+    q, k, v = [x.to(dev).requires_grad_(True) for x in make_qkv(1, 1, 128, 64, torch.float16, 750)]
+    mask = uniform_block_mask(1, 1, 2, 1.0, 751).to(dev)
+    with pytest.raises(RuntimeError):
+        torch.vmap(lambda x: fm.flash_attention_custom_mask(x, k, v, mask, 0.2))(torch.stack([q, q]))
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        with fwad.dual_level():
+            fm.flash_attention_custom_mask(fwad.make_dual(q, torch.ones_like(q)), k, v, mask, 0.2)
