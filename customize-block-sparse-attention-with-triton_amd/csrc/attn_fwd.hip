@@ -1208,6 +1208,18 @@ static size_t slots_bytes(int B, int H, int W, int D) {
   return (size_t)B * H * W * 2 * partial_floats(D) * sizeof(float);
 }
 
+// D = 128 with enough row blocks in the launch to fill the chip goes to the kernel that gives each
+// row block to one wavefront pair (two wavefronts per SIMD, no merges between workgroups).  With
+// fewer row blocks its critical path is the longest row, which the host cannot see (the lists
+// stay on the device): from two row blocks per compute unit on it won in every measured case,
+// from one on only when rows are short (at most 32 tiles).  (Elementwise masks and numbers of tokens
+// that are not whole tiles always go there, see pair_split_128: fwd_kernel with their extra state has 200 bytes of
+// spills per lane.)
+static bool use_pair_kernel(int64_t row_blocks, int nb) {
+  const int64_t cus = compute_units();
+  return row_blocks >= 2 * cus || (row_blocks >= cus && nb <= 32);
+}
+
 // Pair kernel: workgroups per row block.  One when the launch has enough row blocks to fill the GPU twice
 // over; otherwise the row lists are shared (up to 8 ways, a share of a dense list keeping at least 8 tiles).
 static int pair_split(int B, int H, int nb, int D) {
@@ -1220,6 +1232,26 @@ static int pair_split(int B, int H, int nb, int D) {
   return (int)(s > 8 ? 8 : s);
 }
 
+// The same at D = 128 for the launches only the pair kernel takes (elementwise masks, N not a multiple of 64): about four
+// workgroups per compute unit over the launch; at most 4 shares of a row unless it is long (a share of a dense row then
+// has 16 tiles), at least two tiles in one.  us, N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares, and fwd_kernel before:
+//   8 heads N = 4000, token window of 1000   46 /  47 /  55 /  61 /  72 /  89    84
+//   8 heads N = 4000, token-causal          147 /  99 /  82 /  90 /  95 / 103   131
+//   4 heads N = 4096, token window of 1228   32 /  32 /  36 /  36 /  46 /  50    58
+//   1 head N = 8192, token-causal           160 /  93 /  73 /  67 /  57 /  57    73
+//   1 head N = 17000, keep 0.5              233 / 152 / 119 / 138 / 126 / 131   260
+//   2 heads N = 1000, token-causal           40 /  27 /  27 /  24 /  24 /  27    34
+// Whole tiles with a block mask and at least use_pair_kernel's row blocks were not shared before and are not without whole
+// tiles either (8 heads N = 4000, fp16: keep 0.25 44 / 49, dense 95 / 97).
+static int pair_split_128(int64_t row_blocks, int nb, bool elementwise) {
+  const int64_t cus = compute_units();
+  if (!elementwise && use_pair_kernel(row_blocks, nb)) return 1;
+  int64_t s = 4 * cus / row_blocks;
+  const int few = nb / 2 < 4 ? nb / 2 : 4, cap = nb / 16 > few ? nb / 16 : few;
+  if (s > cap) s = cap;
+  return (int)(s > 8 ? 8 : s < 1 ? 1 : s);
+}
+
 static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
   return split > 1 ? (size_t)split * B * H * N * (D + 2) * sizeof(float) : 0;
 }
@@ -1230,23 +1262,16 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
   const int mode = fwd_mode(B, H, nb, D, compact);
   if (mode == ROWS_MODE) return 256;      // nothing is shared
   const int W = groups_per_head(B, H, nb, D, mode);
-  return slots_bytes(B, H, W, D) + (size_t)B * H * nb * sizeof(unsigned long long);
+  const size_t bytes = slots_bytes(B, H, W, D) + (size_t)B * H * nb * sizeof(unsigned long long);
+  if (D != 128 || compact) return bytes;      // (compact launches: whole tiles and block masks only)
+  const size_t parts = 256 + pair_parts_bytes(B, H, N, D, pair_split_128((int64_t)B * H * nb, nb, true));
+  return parts > bytes ? parts : bytes;
 }
 
 // one size for bsattn_fwd and bsattn_fwd_elementwise
 size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_bytes(B, H, N, D); }
 
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
-// D = 128 with enough row blocks in the launch to fill the chip goes to the kernel that gives each
-// row block to one wavefront pair (two wavefronts per SIMD, no merges between workgroups).  With
-// fewer row blocks its critical path is the longest row, which the host cannot see (the lists
-// stay on the device): from two row blocks per compute unit on it won in every measured case,
-// from one on only when rows are short (at most 32 tiles).
-static bool use_pair_kernel(int64_t row_blocks, int nb) {
-  const int64_t cus = compute_units();
-  return row_blocks >= 2 * cus || (row_blocks >= cus && nb <= 32);
-}
-
 // D = 64.  With few row blocks the wavefronts of a workgroup share one row block at a time (K and V tiles are spread
 // over them and the results merged); with many a wavefront takes a whole row block, which needs no merge.
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
@@ -1266,11 +1291,14 @@ static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
 template <int D, int DT, int MODE, bool EW>
 static void launch_fwd_t(const FwdParams& prm, int grid, hipStream_t st) {
   const bool contig = prm.ks[2] == D && prm.vs[2] == D, whole = prm.N % 64 == 0;
-  constexpr bool HAS_CONTIG = D == 64 || DT != 0;
-  if (HAS_CONTIG && contig && whole) launch_fwd_c<D, DT, MODE, EW, HAS_CONTIG ? CONTIG_WHOLE : GENERAL>(prm, grid, st);
-  else if (D == 64 && contig) launch_fwd_c<D, DT, MODE, EW, D == 64 ? CONTIG_TAIL : GENERAL>(prm, grid, st);
-  else if (D == 128 && whole) launch_fwd_c<D, DT, MODE, EW, D == 128 ? STRIDED_WHOLE : GENERAL>(prm, grid, st);
-  else launch_fwd_c<D, DT, MODE, EW, GENERAL>(prm, grid, st);
+  if constexpr (D == 128) {      // (whole tiles only)
+    if (DT != 0 && contig) launch_fwd_c<D, DT, MODE, EW, DT != 0 ? CONTIG_WHOLE : STRIDED_WHOLE>(prm, grid, st);
+    else launch_fwd_c<D, DT, MODE, EW, STRIDED_WHOLE>(prm, grid, st);
+  } else {
+    if (contig && whole) launch_fwd_c<D, DT, MODE, EW, CONTIG_WHOLE>(prm, grid, st);
+    else if (contig) launch_fwd_c<D, DT, MODE, EW, CONTIG_TAIL>(prm, grid, st);
+    else launch_fwd_c<D, DT, MODE, EW, GENERAL>(prm, grid, st);
+  }
 }
 
 template <int D, int MODE, bool EW>
@@ -1283,8 +1311,9 @@ static void launch_fwd_m(const FwdParams& prm, int dt, int grid, hipStream_t st)
 template <bool EW>
 static void launch_fwd_d(const FwdParams& prm, int D, int mode, int dt, hipStream_t st) {
   const int BH = prm.B * prm.H, grid = prm.W * BH;
-  if (D == 128) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
-  else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, ((BH + 7) / 8) * 8 * prm.nb, st);
+  if (D == 128) {
+    if constexpr (!EW) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
+  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, ((BH + 7) / 8) * 8 * prm.nb, st);
   else if (mode == WAVE) launch_fwd_m<64, WAVE, EW>(prm, dt, grid, st);
   else launch_fwd_m<64, COOP, EW>(prm, dt, grid, st);
 }
@@ -1358,11 +1387,14 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   const bool bf = s.dtype == BSATTN_BF16;
   const int BH = s.B * s.H;
   prm.split = 1;
-  if (s.D == 256 || (s.D == 128 && use_pair_kernel((int64_t)BH * prm.nb, prm.nb))) {   // (D = 256 has no other kernel)
-    // D = 256 launches with few row blocks share the row lists between workgroups; at D = 128 the
-    // cooperative kernel below takes those launches (sharing was measured: faster on dense masks with 2-3
+  const int64_t row_blocks = (int64_t)BH * prm.nb;
+  const bool only_pair = s.D == 256 || (s.D == 128 && (tile_bits != nullptr || s.N % 64 != 0));   // no other kernel
+  if (only_pair || (s.D == 128 && use_pair_kernel(row_blocks, prm.nb))) {
+    // launches with few row blocks share the row lists between workgroups; at D = 128 with whole tiles and a block mask
+    // the cooperative kernel below takes those launches (sharing was measured: faster on dense masks with 2-3
     // heads, 25-30 % slower on sparse ones)
     if (s.D == 256) prm.split = pair_split(s.B, s.H, prm.nb, s.D);
+    else if (only_pair) prm.split = pair_split_128(row_blocks, prm.nb, tile_bits != nullptr);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * BH * s.N * s.D;
     launch_fwd_pair(prm, s.D, !bf ? 0 : (prm.out_f32 ? 1 : 2), tile_bits != nullptr, st);

@@ -35,6 +35,9 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   constexpr bool BF16 = DT != 0;
   constexpr bool PB = DT == 2;                   // P rounded to bf16, second product in bf16 (V as it is)
   constexpr bool FOLD = !BF16;
+  // V read before the softmax (see the loop): not where the compiler would then spill V's 64 registers in every tile (bf16
+  // elementwise; 8 heads of N = 4000, token window of 1000: 84.7 us with the spills)
+  constexpr bool EARLY_V = PORTIONS <= PAIR_EARLY_V && !(EW && BF16 && (TAIL || !PB));
   constexpr int HALF = CPR / 2;                  // copy instructions per wavefront and tile
   constexpr int KOPS = HALF + (EW ? 1 : 0), VOPS = HALF;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
       l_i = lnew;
       fresh = false;
     };
-    if constexpr (PORTIONS <= PAIR_EARLY_V) {
+    if constexpr (EARLY_V) {
       // The V fragments are read before the softmax (they take the registers of the K fragments), so
       // that the next V tile is requested that much earlier: its latency was exposed otherwise.
       uintx4 vfr[PORTIONS][4][DBP];

@@ -76,3 +76,41 @@ def test_nothing_beyond_the_last_token_is_touched(dev, D, N, contiguous_rows):
     for name, got, ref in zip(("o", "lse", "dq", "dk", "dv"), res, (o_ref, lse_ref, dq, dk, dv)):
         ma, rl = errors(got, ref)
         assert ma <= 2e-2 and (rl <= 1e-3 or ma <= 1e-5), (name, ma, rl)     # (a zero gradient has no relative error)
+
+
+# D = 128, elementwise masks and ragged lengths: row lists shared by 2 (504 row blocks), 4 (short rows), 1 (two tiles a
+# row) and 5 (81 long rows) workgroups, shares without tiles among them; 512 row blocks: by 2 with an elementwise mask
+# only.  Backward: lists of 13 and 16 tiles shared at D = 64 and 256.
+@pytest.mark.parametrize("H,N,D", [(8, 4000, 128), (8, 4090, 128), (2, 1000, 128), (3, 100, 128), (1, 5184, 128), (8, 777, 64),
+                                   (2, 1000, 64), (8, 777, 256), (2, 1000, 256), (12, 1400, 256)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("elementwise", [False, True])
+@pytest.mark.parametrize("out_fp32", [False, True])
+def test_shared_lists(dev, H, N, D, dtype, elementwise, out_fp32):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v, do = make_qkv(1, H, N, D, dtype, 800 + N, n=4)
+    block = block_mask(nb, 0.3, 801 + N)
+    dense = torch.from_numpy(orc.expand_block_mask(block.numpy())[..., :N, :N].copy())
+    if elementwise:
+        i = torch.arange(N)
+        dense = dense & (i[:, None] - i[None, :] < N // 3) & ((i[:, None] - i[None, :]) % 7 != 0)
+        dense[0, 0, 5, :] = False
+    mask = dense if elementwise else block
+    sc = D ** -0.5
+    res = fm.attention_forward_backward(q.to(dev), k.to(dev), v.to(dev), mask.to(dev), sc, do.to(dev), out_fp32=out_fp32)
+    torch.cuda.synchronize()
+    sl = (slice(None), slice(H - 1, H))
+    o_ref, lse_ref = orc.naive_attention(f32(q[sl]), f32(k[sl]), f32(v[sl]), dense.numpy(), sc, return_lse=True)
+    # fp32 results: P and dS have 16 bits; 16-bit ones are rounded once more (bf16: 2^-9 for O, the gradients' P and dS too)
+    rel = 1e-3 if out_fp32 or dtype == torch.float16 else 3e-3
+    ma, rl = errors(res[0][sl], o_ref)
+    assert ma <= MAXABS[dtype] and rl <= rel, (ma, rl)
+    fin = np.isfinite(lse_ref)
+    lse = res[1][sl].cpu().numpy()
+    assert np.array_equal(np.isfinite(lse), fin) and np.abs(lse[fin] - lse_ref[fin]).max() <= 2e-3
+    if N <= 1400:
+        grads = orc.attention_backward(f32(q[sl]), f32(k[sl]), f32(v[sl]), dense.numpy(), sc, f32(do[sl]))[:3]
+        for name, got, ref in zip(("dq", "dk", "dv"), res[2:], grads):
+            ma, rl = errors(got[sl], ref)
+            assert rl <= (2e-3 if rel == 1e-3 else 1e-2), (name, ma, rl)
