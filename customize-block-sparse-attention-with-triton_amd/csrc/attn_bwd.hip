@@ -874,15 +874,35 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 // ---------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------
-// Workgroups per row / column list.  One is enough when the launch has at least four workgroups
-// per compute unit; a single long head would otherwise walk its lists on a fraction of the GPU.
-static int bwd_split(int B, int H, int N) {
-  const int64_t lists = (int64_t)B * H * ((N + 63) / 64), want = 4 * (int64_t)compute_units();
-  if (lists >= want) return 1;
-  int64_t s = (want + lists - 1) / lists;
-  const int cap = N / 64 / 8 > 1 ? N / 64 / 8 : 1;        // a share should have a few tiles even in a dense list
+// Workgroups per row / column list.  A single long head would otherwise walk its lists on a fraction of the GPU; every
+// further share costs a write and a read of fp32 parts of dQ, dK and dV and, once, the launch that adds them up.
+// us of a backward, N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares (256 compute units):
+//   D = 64    8 heads N = 4096, keep 0.3    88 /  78 /  87 /  90 / 101 / 115     block-causal  149 / 123 / 109 / 115 / 122 / 135
+//             8 heads N = 777,  keep 0.6    35 /  31 /  33 /  32 /  34 /  38
+//             2 heads N = 1000, causal 0.8  38 /  28 /  29 /  26 /  26 /  28
+//   D = 128   8 heads N = 4096, keep 0.3   119 / 131 / 148 / 160 / 217 / 264     block-causal  197 / 184 / 189 / 199 / 249 / 297
+//            16 heads N = 1500, keep 0.3    58 /  77 /  90 / 101 / 131 / 179
+//             2 heads N = 4096, keep 0.25   79 /  65 /  59 /  60 /  68 /  71     block-causal  178 / 116 /  99 /  93 /  92 /  90
+//             4 heads N = 8192, keep 0.2   150 / 169 / 173 / 188 / 240 / 288     block-causal  386 / 334 / 333 / 333 / 366 / 410
+//   D = 256   8 heads N = 4000, window     230 / 306 / 361 / 415 / 530 / 638     token-causal  682 / 464 / 599 / 577 / 682 / 779
+//            12 heads N = 4096, causal 0.5 423 / 519 / 570 / 631 / 774 / 919
+//             2 heads N = 4096, keep 0.25  239 / 157 / 132 / 121 / 155 / 162     block-causal  571 / 323 / 243 / 197 / 230 / 233
+//             8 heads N = 777,  keep 0.6   129 / 103 /  98 /  91 / 114 / 127
+// D = 64 fills four workgroups per compute unit.  D = 128 has two in dkdv4_kernel and parts twice as large: two per
+// compute unit, rounded to the nearest, but four where rows are long (the imbalance of a causal mask then weighs more
+// than the parts).  D = 256 has one or two per compute unit: two, yet always two shares below 2.5.  A share keeps at least
+// 8 tiles of a dense list; 5 in a launch of few short lists (at D = 128 that was slower), where the walk's latency is all.
+static int bwd_split(int B, int H, int N, int D) {
+  const int64_t lists = (int64_t)B * H * ((N + 63) / 64), cus = compute_units();
+  const int nb = (N + 63) / 64;
+  int64_t s;
+  if (D == 64 || (D == 128 && nb >= 96)) s = (4 * cus + lists - 1) / lists;
+  else s = (2 * cus + lists / 2) / lists;
+  if (D == 256 && s < 2 && 2 * lists < 5 * cus) s = 2;
+  const bool few_short = D != 128 && nb <= 32 && 2 * lists <= cus;
+  const int cap = few_short ? nb / 5 : nb / 8;
   if (s > cap) s = cap;
-  return (int)(s > 8 ? 8 : s);
+  return (int)(s > 8 ? 8 : s < 1 ? 1 : s);
 }
 
 // floats in front of the parts (the parts are accessed 16 bytes at a time)
@@ -890,7 +910,7 @@ static size_t delta_floats(int B, int H, int N) { return ((size_t)B * H * N + 63
 
 size_t bwd_workspace_bytes(int B, int H, int N, int D) {
   const size_t delta = delta_floats(B, H, N) * sizeof(float);
-  const int split = bwd_split(B, H, N);
+  const int split = bwd_split(B, H, N, D);
   return delta + (split > 1 ? (size_t)3 * split * B * H * N * D * sizeof(float) : 0);   // + parts of dQ, dK, dV
 }
 
@@ -949,7 +969,7 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   prm.bits_rows = (const unsigned long long*)bits_rows; prm.bits_cols = (const unsigned long long*)bits_cols;
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   prm.out_f32 = s.out_dtype == BSATTN_F32;
-  prm.split = bwd_split(s.B, s.H, s.N);
+  prm.split = bwd_split(s.B, s.H, s.N, s.D);
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
     prm.part_dq = (float*)ws + delta_floats(s.B, s.H, s.N);
