@@ -380,15 +380,12 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
 // dK, dV: workgroup = column block n, wavefront wv owns keys 64n + 32wv + ln
 // ---------------------------------------------------------------------------------------
 // A tile is walked in two steps of 32 queries, which halves the fragments in flight.
-// DH: -1, or at D = 256 the half (0 / 1) of the head dimension whose dK and dV columns this launch
-// accumulates and writes (the first products always contract over the whole head dimension): with
-// 128 columns at a time the accumulators and K, V of 32 keys are 256 registers instead of 384.
-template <int D, bool BF16, bool EW, bool PB, int DH, bool TAIL>
-__global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdParams prm) {
+// (D = 64; larger head dimensions run dkdv4_kernel.)
+template <int D, bool BF16, bool EW, bool PB, bool TAIL>
+__global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
   using C = BwdCfg<D, EW, 32>;
   constexpr int KS = D / 16, STEPS = 2;
-  constexpr int DB = DH < 0 ? D / 32 : D / 64, DB0 = DH < 0 ? 0 : DH * DB;   // 32-column blocks of this launch, the first one
-  constexpr int PORTIONS = D == 256 ? 2 : 1, KSP = KS / PORTIONS;            // fragments of the first products in portions
+  constexpr int DB = D / 32;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
@@ -471,19 +468,18 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
 
     // operand fragments are read from LDS ahead of the block of MFMAs that consumes them
     floatx16 sacc = zero16(), dpacc = zero16();
+    {
+      uintx4 fq[KS], fg[KS];
 #pragma unroll
-    for (int pt = 0; pt < PORTIONS; ++pt) {
-      uintx4 fq[KSP], fg[KSP];
-#pragma unroll
-      for (int s = 0; s < KSP; ++s) {
-        fq[s] = frag_rows<D>(qt, 0, pt * KSP + s, ln, g);
-        fg[s] = frag_rows<D>(gt, 0, pt * KSP + s, ln, g);
+      for (int s = 0; s < KS; ++s) {
+        fq[s] = frag_rows<D>(qt, 0, s, ln, g);
+        fg[s] = frag_rows<D>(gt, 0, s, ln, g);
       }
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < KSP; ++s) {
-        sacc = mfma_qk<BF16>(fq[s], kfr[pt * KSP + s], sacc);      // S = Q K^T
-        dpacc = mfma_qk<BF16>(fg[s], vfr[pt * KSP + s], dpacc);    // dP = dO V^T
+      for (int s = 0; s < KS; ++s) {
+        sacc = mfma_qk<BF16>(fq[s], kfr[s], sacc);      // S = Q K^T
+        dpacc = mfma_qk<BF16>(fg[s], vfr[s], dpacc);    // dP = dO V^T
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -499,8 +495,8 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
     for (int ts = 0; ts < 2; ++ts)
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
-        fgt[ts][db] = frag_cols<D, BF16 && !PB>(gt, DB0 + db, ts, lane);
-        fqt[ts][db] = frag_cols<D, BF16 && !PB>(qt, DB0 + db, ts, lane);
+        fgt[ts][db] = frag_cols<D, BF16 && !PB>(gt, db, ts, lane);
+        fqt[ts][db] = frag_cols<D, BF16 && !PB>(qt, db, ts, lane);
       }
     __builtin_amdgcn_sched_barrier(0);
     // rows of the results are queries: register i <-> query 8(i/4) + 4g + i%4
@@ -539,7 +535,7 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4) {
-        const int64_t off = krow * D + 32 * (DB0 + db) + 8 * i4 + 4 * g;
+        const int64_t off = krow * D + 32 * db + 8 * i4 + 4 * g;
         store_out4<BF16>(prm.part_dk + poff, off, true, dkacc[db][4 * i4], dkacc[db][4 * i4 + 1], dkacc[db][4 * i4 + 2],
                          dkacc[db][4 * i4 + 3]);
         store_out4<BF16>(prm.part_dv + poff, off, true, dvacc[db][4 * i4], dvacc[db][4 * i4 + 1], dvacc[db][4 * i4 + 2],
@@ -554,7 +550,7 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i4 = 0; i4 < 4; ++i4) {
-      const int col = 32 * (DB0 + db) + 8 * i4 + 4 * g;
+      const int col = 32 * db + 8 * i4 + 4 * g;
       const int64_t off = krow * prm.dks[2] + col;
       store_out4<BF16>(kbase, off, prm.out_f32, dkacc[db][4 * i4] * prm.sm_scale, dkacc[db][4 * i4 + 1] * prm.sm_scale,
                        dkacc[db][4 * i4 + 2] * prm.sm_scale, dkacc[db][4 * i4 + 3] * prm.sm_scale);
@@ -564,7 +560,7 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
 }
 
 // ---------------------------------------------------------------------------------------
-// dK, dV at D = 128: workgroup = column block n, four wavefronts (one per SIMD).
+// dK, dV at D = 128 and 256: workgroup = column block n, four wavefronts (one per SIMD).
 // Wavefront (kh, dh) owns keys 64n + 32kh + ln and the columns 64dh .. 64dh + 63 of their dK and dV rows: half
 // the accumulators of dkdv_kernel's wavefront, which, with K, V, dK and dV of its keys in 192 of 512
 // registers, runs alone on its SIMD and leaves the matrix cores idle two thirds of the time.  Here a wavefront
@@ -579,6 +575,11 @@ __global__ __launch_bounds__(128, D == 64 ? 2 : 1) void dkdv_kernel(const BwdPar
 // instruction per element, and the row statistics need no place in LDS: a lane reads the two values of its
 // query from memory a step ahead.  (Two stages of a Q and a dO tile, 64 KB, + 16 KB of exchange are exactly half
 // the 160 KB of a compute unit: two workgroups per compute unit, two wavefronts per SIMD.)
+// D = 256: the same split with 128 columns, 500 registers and 145 KB of LDS per wavefront and workgroup, one wavefront per
+// SIMD; lse and delta are staged in LDS and stay fp32 (the pieces have a limited range).  Before, dkdv_kernel ran twice,
+// 128 columns of dK and dV each time: S and dP twice (6 products for 4) and every tile copied twice.  Backward, bf16:
+// 12 heads N = 4096 causal 0.5 519 -> 333 us, 16 heads N = 8192 keep 0.3 1780 -> 1540, 2 heads N = 1000 96 -> 61 (two
+// shares each).  Bound by its lone wavefront's chain: first products, exponentials, exchange, second products.
 // ---------------------------------------------------------------------------------------
 template <int NWV, int D, int ROWS>
 __device__ __forceinline__ void part_tile_load_async(const unsigned short* tile, int64_t stride, int wv, int lane,
@@ -626,12 +627,15 @@ __device__ __forceinline__ uintx4 three_pieces(float x, bool holder) {
   return r;
 }
 
-constexpr int DKDV4_LDS_BYTES = 4 * 64 * 2 * 128 + 4 * 4096;   // two stages of a Q and a dO tile, 4 KB of exchange per wavefront
+// two stages of a Q and a dO tile, 4 KB of exchange per wavefront, at D = 256 two stages of lse and delta
+template <int D> constexpr int dkdv4_lds_bytes() { return 4 * 64 * 2 * D + 4 * 4096 + (D == 256 ? 2 * 512 : 0); }
 template <int D, bool BF16, bool PB, bool EW, bool TAIL>
-__global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
-  static_assert(D == 128, "two 32-column blocks of dK and dV per wavefront");
+__global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdParams prm) {
+  static_assert(D == 128 || D == 256, "two or four 32-column blocks of dK and dV per wavefront");
   constexpr int KS = D / 16, DBW = D / 64;           // 32-column blocks per wavefront
-  constexpr int TILE_BYTES = 64 * 2 * D, STAGE_BYTES = 2 * TILE_BYTES, EXCH_OFF = 2 * STAGE_BYTES;
+  constexpr int TILE_BYTES = 64 * 2 * D, STAGE_BYTES = 2 * TILE_BYTES, EXCH_OFF = 2 * STAGE_BYTES, STAT_OFF = EXCH_OFF + 4 * 4096;
+  constexpr bool PIECES = D == 128;                  // lse and delta by way of the matrix cores
+  constexpr int PORTIONS = KS / 4, KSP = KS / PORTIONS;   // fragments of the first products in portions
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int kh = wv & 1, dh = wv >> 1;
@@ -678,6 +682,9 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
     const int rb = rows[u];
     const unsigned sa = lds_addr + stage * STAGE_BYTES;
     blk_issued = rb;
+    if constexpr (!PIECES)
+      if (wv < 2) stat_load_async((wv == 0 ? lse_h : dlt_h) + (int64_t)rb * 64, TAIL && rb == nb - 1 && lane >= valid ? valid - 1 : lane,
+                                  lds_addr + STAT_OFF + stage * 512 + wv * 256);
     if (TAIL && rb == nb - 1) {
       tail_tile_load_async<4, D, 64>(qg + (int64_t)rb * 64 * prm.qs[2], prm.qs[2], 0, valid, wv, lane, sa);
       tail_tile_load_async<4, D, 64>(gg + (int64_t)rb * 64 * prm.dos[2], prm.dos[2], 0, valid, wv, lane, sa + TILE_BYTES);
@@ -696,8 +703,10 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   auto ask_stats = [&](int u) {
     int q = rows[u] * 64 + 32 * dh + ln;
     if (TAIL && q >= prm.N) q = prm.N - 1;
-    st_lse = lse_h[q];
-    st_dlt = dlt_h[q];
+    if constexpr (PIECES) {
+      st_lse = lse_h[q];
+      st_dlt = dlt_h[q];
+    }
     if constexpr (EW) st_bits = prm.bits_cols[(int64_t)u * 64 + 32 * kh + ln];
   };
   if (u0 < u1) { ask_stats(u0); issue(u0, 0); }
@@ -742,8 +751,11 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
     __syncthreads();                 // the step's tiles are complete; everybody has left the previous step
     // the extra slices of this step from the statistics asked for a step ago; then the next step's
     // (a query without any unmasked key has lse = -inf; all its scores are masked below, whatever the slice holds)
-    const uintx4 lse_slice = three_pieces<BF16>(EW && st_lse == -INFINITY ? 0.f : -st_lse * inv_scale, g == 0);
-    const uintx4 dlt_slice = three_pieces<BF16>(-st_dlt, g == 0);
+    uintx4 lse_slice, dlt_slice;
+    if constexpr (PIECES) {
+      lse_slice = three_pieces<BF16>(EW && st_lse == -INFINITY ? 0.f : -st_lse * inv_scale, g == 0);
+      dlt_slice = three_pieces<BF16>(-st_dlt, g == 0);
+    }
     // the mask bits of this lane's key for the queries of this wavefront's block, shifted so that bit
     // 8(i/4) + i%4 belongs to register i
     const unsigned mw = EW ? (unsigned)(st_bits >> (32 * dh)) >> (4 * g) : 0u;
@@ -756,25 +768,27 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
     // ---- first products of this wavefront's query block: S' = Q K^T - lse / sm_scale, dP' = dO V^T - delta ----
     floatx16 sacc = zero16(), dpacc = zero16();
     {
-      // (the fragments in two portions: all sixteen at once do not fit beside K, V and the accumulators)
+      // (the fragments in portions of four slices: all at once they do not fit beside K, V and the accumulators)
 #pragma unroll
-      for (int pt = 0; pt < 2; ++pt) {
-        uintx4 fq[KS / 2], fg[KS / 2];
+      for (int pt = 0; pt < PORTIONS; ++pt) {
+        uintx4 fq[KSP], fg[KSP];
 #pragma unroll
-        for (int s = 0; s < KS / 2; ++s) {
-          fq[s] = frag_rows<D>(qt, 32 * dh, pt * (KS / 2) + s, ln, g);
-          fg[s] = frag_rows<D>(gt, 32 * dh, pt * (KS / 2) + s, ln, g);
+        for (int s = 0; s < KSP; ++s) {
+          fq[s] = frag_rows<D>(qt, 32 * dh, pt * KSP + s, ln, g);
+          fg[s] = frag_rows<D>(gt, 32 * dh, pt * KSP + s, ln, g);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < KS / 2; ++s) {
-          sacc = mfma_qk<BF16>(fq[s], kfr[pt * (KS / 2) + s], sacc);
-          dpacc = mfma_qk<BF16>(fg[s], vfr[pt * (KS / 2) + s], dpacc);
+        for (int s = 0; s < KSP; ++s) {
+          sacc = mfma_qk<BF16>(fq[s], kfr[pt * KSP + s], sacc);
+          dpacc = mfma_qk<BF16>(fg[s], vfr[pt * KSP + s], dpacc);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      sacc = mfma_qk<BF16>(lse_slice, ones_frag, sacc);
-      dpacc = mfma_qk<BF16>(dlt_slice, ones_frag, dpacc);
+      if constexpr (PIECES) {
+        sacc = mfma_qk<BF16>(lse_slice, ones_frag, sacc);
+        dpacc = mfma_qk<BF16>(dlt_slice, ones_frag, dpacc);
+      }
     }
     if constexpr (EW) mask_scores(sacc, mw);
     if (tail_step) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> (32 * dh)));
@@ -791,10 +805,22 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
       for (int jh = 0; jh < 2; ++jh) {
         const int i0 = 8 * t2 + 4 * jh;
         float p[4], ds[4];
+        floatx4 l4, d4;
+        if constexpr (!PIECES) {
+          const float* st = reinterpret_cast<const float*>(lds + STAT_OFF + stage * 512) + 32 * dh + 8 * (i0 >> 2) + 4 * g;
+          l4 = *reinterpret_cast<const floatx4*>(st);
+          d4 = *reinterpret_cast<const floatx4*>(st + 64);
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          p[e] = __builtin_amdgcn_exp2f(sacc[i0 + e] * qk_scale);
-          ds[e] = p[e] * dpacc[i0 + e];
+          if constexpr (PIECES) {
+            p[e] = __builtin_amdgcn_exp2f(sacc[i0 + e] * qk_scale);
+            ds[e] = p[e] * dpacc[i0 + e];
+          } else {   // (a query without any unmasked key has lse = -inf: its P must come out as 0)
+            const float nl = EW && l4[e] == -INFINITY ? -INFINITY : -l4[e] * kLog2e;
+            p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[i0 + e], qk_scale, nl));
+            ds[e] = p[e] * (dpacc[i0 + e] - d4[e]);
+          }
         }
         pm[t2][2 * jh] = pack2<PB>(p[0], p[1]);   pm[t2][2 * jh + 1] = pack2<PB>(p[2], p[3]);
         dm[t2][2 * jh] = pack2<PB>(ds[0], ds[1]); dm[t2][2 * jh + 1] = pack2<PB>(ds[2], ds[3]);
@@ -832,7 +858,7 @@ __global__ __launch_bounds__(256, 2) void dkdv4_kernel(const BwdParams prm) {
   }
   // the wavefront's 32 x 64 blocks of dK and dV leave through a stretch of the (now idle) tile stages and exchange area
   constexpr int OUT_BYTES = rows_out_bytes(32 * DBW, true);
-  static_assert(4 * 2 * OUT_BYTES <= DKDV4_LDS_BYTES, "room for dK and dV of four wavefronts");
+  static_assert(4 * 2 * OUT_BYTES <= dkdv4_lds_bytes<D>(), "room for dK and dV of four wavefronts");
   __syncthreads();           // everybody has left the last step
   // (the lane index as a value the compiler cannot trace back: the per-lane addresses of the stores below would
   // otherwise be computed before the walk and held, or spilled, through it)
@@ -884,21 +910,20 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 //            16 heads N = 1500, keep 0.3    58 /  77 /  90 / 101 / 131 / 179
 //             2 heads N = 4096, keep 0.25   79 /  65 /  59 /  60 /  68 /  71     block-causal  178 / 116 /  99 /  93 /  92 /  90
 //             4 heads N = 8192, keep 0.2   150 / 169 / 173 / 188 / 240 / 288     block-causal  386 / 334 / 333 / 333 / 366 / 410
-//   D = 256   8 heads N = 4000, window     230 / 306 / 361 / 415 / 530 / 638     token-causal  682 / 464 / 599 / 577 / 682 / 779
-//            12 heads N = 4096, causal 0.5 423 / 519 / 570 / 631 / 774 / 919
-//             2 heads N = 4096, keep 0.25  239 / 157 / 132 / 121 / 155 / 162     block-causal  571 / 323 / 243 / 197 / 230 / 233
-//             8 heads N = 777,  keep 0.6   129 / 103 /  98 /  91 / 114 / 127
-// D = 64 fills four workgroups per compute unit.  D = 128 has two in dkdv4_kernel and parts twice as large: two per
-// compute unit, rounded to the nearest, but four where rows are long (the imbalance of a causal mask then weighs more
-// than the parts).  D = 256 has one or two per compute unit: two, yet always two shares below 2.5.  A share keeps at least
-// 8 tiles of a dense list; 5 in a launch of few short lists (at D = 128 that was slower), where the walk's latency is all.
+//   D = 256   8 heads N = 4000, window     174 / 251 / 305 / 363 / 472 / 578     token-causal  402 / 404 / 480 / 514 / 618 / 715
+//            16 heads N = 1500, keep 0.3   113 / 151 / 189 / 233 / 325 / 399
+//             2 heads N = 4096, keep 0.25  140 / 101 / 107 / 103 / 127 / 146     block-causal  322 / 191 / 170 / 161 / 181 / 195
+//             8 heads N = 777,  keep 0.6    76 /  69 /  77 /  74 /  93 / 110
+// D = 64 fills four workgroups per compute unit.  The larger head dimensions have one or two in dkdv4_kernel and parts two
+// and four times as large: two per compute unit, rounded to the nearest, but at D = 128 four where rows are long (the
+// imbalance of a causal mask then weighs more than the parts).  A share keeps at least 8 tiles of a dense list; 5 in a
+// launch of few short lists (at D = 128 that was slower), where the walk's latency is all.
 static int bwd_split(int B, int H, int N, int D) {
   const int64_t lists = (int64_t)B * H * ((N + 63) / 64), cus = compute_units();
   const int nb = (N + 63) / 64;
   int64_t s;
   if (D == 64 || (D == 128 && nb >= 96)) s = (4 * cus + lists - 1) / lists;
   else s = (2 * cus + lists / 2) / lists;
-  if (D == 256 && s < 2 && 2 * lists < 5 * cus) s = 2;
   const bool few_short = D != 128 && nb <= 32 && 2 * lists <= cus;
   const int cap = few_short ? nb / 5 : nb / 8;
   if (s > cap) s = cap;
@@ -919,38 +944,26 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
   using C = BwdCfg<D, EW>;
   constexpr int KB = D >= 128 ? 1 : 2;          // dq_kernel walks D >= 128 tiles in two halves (no gain at D = 64: two wavefronts per SIMD anyway)
   using CQ = BwdCfg<D, EW, 32 * KB>;
-  // dkdv_kernel (D = 64 and 256; D = 128 runs dkdv4_kernel): halves at D = 64 (191 instead of 318 registers: two
-  // wavefronts per SIMD; B*H = 32 N = 8192 dense block-causal backward 1417 -> 1167 us); at D = 256 halves too, and
-  // the head dimension of dK, dV in two launches.
+  // dkdv_kernel walks halves (191 instead of 318 registers: two wavefronts per SIMD; B*H = 32 N = 8192 dense block-causal
+  // backward 1417 -> 1167 us)
   using CK = BwdCfg<D, EW, 32>;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dq_kernel<D, BF16, EW, PB, KB, TAIL>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, CQ::LDS_BYTES);
-    if constexpr (D == 256) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, 0, TAIL>),
+    if constexpr (D == 64) {
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, 1, TAIL>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
-    } else if constexpr (D == 128) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW, TAIL>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, DKDV4_LDS_BYTES);
     } else {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv_kernel<D, BF16, EW, PB, -1, TAIL>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, CK::LDS_BYTES);
+      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW, TAIL>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, dkdv4_lds_bytes<D>());
     }
   });
   const int BH = prm.B * prm.H;
   const int grid = ((BH + 7) / 8) * 8 * prm.nb * prm.split;   // heads in groups of 8, the last group padded
   hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
-  if constexpr (D == 256) {   // the two halves of the head dimension of dK, dV in two launches
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, 0, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, 1, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
-  } else if constexpr (D == 128) {   // D = 128: four wavefronts per column block, two per SIMD
-    hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), DKDV4_LDS_BYTES, st, prm);
-  } else {
-    hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, -1, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
-  }
+  if constexpr (D == 64) hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
+  else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);
   if (prm.split > 1) {
     const int64_t quads = (int64_t)BH * prm.N * D / 4;
     hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3((unsigned)((quads + 255) / 256), 3), dim3(256), 0, st, prm, quads, D);
