@@ -155,3 +155,21 @@ def test_one_pass_words_bit_exact(dev, transpose):
             assert np.array_equal(bits[:T].cpu().numpy().view(np.uint64), w_ref)
             p2, b2 = utils.pack_mask_tiles(md, lists, transpose=transpose)
             assert torch.equal(p2[:T], partial[:T]) and torch.equal(b2[:T], bits[:T])
+
+
+# the launch that scans and fills: rows that are and are not whole workgroups of 16, rows longer than what it asks for ahead
+# (384 tiles), either side of its limit of 16384 rows; column lists (strided rows)
+@pytest.mark.parametrize("shape,keep", [((1, 8, 274, 274), 0.1), ((2, 3, 401, 401), 0.3), ((1, 4, 385, 385), 0.9),
+                                        ((4, 256, 16, 16), 0.1), ((1, 16385, 1, 1), 0.5), ((1, 17, 65, 65), 0.02)])
+def test_scan_and_fill(dev, shape, keep):
+    import fa2_custom_mask as fm
+    g = torch.Generator().manual_seed(8)
+    mask = torch.rand(*shape, generator=g) < keep
+    mask[:, :, 0] = False
+    _check_lists(mask, dev)
+    nb = shape[2]
+    lists = fm.block_mask_to_lists(mask.to(dev), transpose=True)
+    by_column = mask.transpose(2, 3).reshape(-1, nb)
+    assert np.array_equal(lists.row_ptr.cpu().numpy(), np.concatenate([[0], np.cumsum(by_column.sum(1).numpy())]))
+    assert np.array_equal(lists.col_idx.cpu().numpy()[:int(by_column.sum())], by_column.nonzero()[:, 1].numpy())
+    assert lists.counts.tolist() == [int(by_column.any(1).sum()), int(by_column.sum())]
