@@ -1366,10 +1366,11 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.D, s.compact);
   prm.W = groups_per_head(s.B, s.H, prm.nb, s.D, mode);
-  // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are
-  // (WAVE: wavefronts instead of workgroups; where a range is a whole number of row blocks the shares stay equal: 16 heads of
-  // N = 8192 dense 304 against 287 us)
-  prm.first_ids = s.D == 64 ? compute_units() * (mode == COOP ? 1 : prm.nb % prm.W == 0 ? 0 : FwdCfg<64>::NW) : 0;
+  // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are.  (Not WAVE: single
+  // wavefronts that arrive while another kernel ends do not fill the SIMDs in order, and two with the larger share on one
+  // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
+  // after a pause 677 against 707.)
+  prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : 0;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();
