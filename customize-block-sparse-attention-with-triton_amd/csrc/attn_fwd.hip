@@ -1184,8 +1184,8 @@ int compute_units() {
 // How a launch is split at D = 64, by its row blocks against the wavefronts that are resident at once (8 per compute unit).
 // From half as many more on a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us; 24 heads of
 // N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there); with about as many a
-// wavefront takes a range of the list (32 heads of N = 4096 dense 174 -> 149 us; 8 heads of N = 17536 dense 702 -> 680,
-// keep 0.07 82 -> 74); with fewer the ranges of whole workgroups are the faster ones (6 heads of N = 17776 at keep 0.3: 236
+// wavefront takes a range of the list (32 heads of N = 4096 dense 174 -> 149 us; 8 heads of N = 17536 dense 710
+// either way, keep 0.1 with a new mask per call 115 -> 106); with fewer the ranges of whole workgroups are the faster ones (6 heads of N = 17776 at keep 0.3: 236
 // against 250 us).
 static int fwd_mode(int B, int H, int nb, int D, bool compact) {
   if (D != 64) return COOP;
