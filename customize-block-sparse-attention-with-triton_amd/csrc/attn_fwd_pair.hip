@@ -372,14 +372,13 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   __syncthreads();           // the other wavefront has left its last tile
   rows_out<BF16, D>(lds + w * rows_out_bytes(D, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2], prm.os[2], prm.out_f32,
                     lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return oacc[db][0][i] * inv; });
-  if (prm.lse != nullptr && g == 0 && exists)
-    prm.lse[(int64_t)bh * prm.N + qrow] =
-        lsum > 0.f ? (m_i + __builtin_amdgcn_logf(lsum)) * 0.6931471805599453f : -INFINITY;
+  if (prm.lse != nullptr && g == 0 && exists) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(m_i, lsum);
 }
 
 // split > 1: O = sum_c 2^(m_c - M) O_c / sum_c 2^(m_c - M) l_c over the non-empty shares c of a row block
-// (M = max m_c over shares with mass), lse = (M + log2 of the denominator) ln 2.  One thread per 4
-// consecutive output values.  Bound by latency: the (m, l) and the values of all S shares are asked for together, an empty share
+// (M = max m_c over shares with mass), lse = (M + log2 of the denominator) ln 2.  A share without mass is one whose
+// sum is zero: a sum that is not a number (a score that is not finite) goes into the result like any other.  One thread
+// per 4 consecutive output values.  Bound by latency: the (m, l) and the values of all S shares are asked for together, an empty share
 // (nothing was written) reads the last one's, which is never empty, in its place.  Before, one share's loads
 // waited for another's and rows were found by 64-bit divisions: 2 heads of N = 4096, D = 256, 8 shares 21.8 -> 14.9 us (71 MB:
 // 4.8 TB/s); 8 heads of N = 4000, D = 128, 2 shares, the whole training step 136.9 -> 132.3.
@@ -411,10 +410,10 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
     }
 #pragma unroll
     for (int c = 0; c < S; ++c)
-      if (l[c] > 0.f) M = fmaxf(M, m[c]);
+      if (l[c] != 0.f) M = fmaxf(M, m[c]);
 #pragma unroll
     for (int c = 0; c < S; ++c) {
-      if (!(l[c] > 0.f)) continue;
+      if (l[c] == 0.f) continue;
       const float wgt = __builtin_amdgcn_exp2f(m[c] - M);
       L += wgt * l[c];
       acc += wgt * part[c];
@@ -423,8 +422,7 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
   const float inv = L > 0.f ? 1.0f / L : 0.f;
   store_out4<BF16>(out_base(prm, b, h), (int64_t)row * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv,
                    acc[3] * inv);
-  if (col == 0 && prm.lse != nullptr)
-    prm.lse[(int64_t)bh * prm.N + row] = L > 0.f ? (M + __builtin_amdgcn_logf(L)) * 0.6931471805599453f : -INFINITY;
+  if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + row] = row_lse(M, L);
 }
 
 // (shared lists: at most four workgroups per compute unit, so the values fit 32 bits)

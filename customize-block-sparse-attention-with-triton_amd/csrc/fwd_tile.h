@@ -58,6 +58,12 @@ __device__ __forceinline__ void* out_base(const FwdParams& prm, int b, int h) {
   return prm.out_f32 ? (void*)((float*)prm.o + off) : (void*)((unsigned short*)prm.o + off);
 }
 
+// Natural logarithm of the sum of exponentials of a row with reference exponent m and sum l of its numerators: -inf
+// for a row without mass (l = 0) or with no score above -inf (m = -inf), NaN where a score is not a number.
+__device__ __forceinline__ float row_lse(float m, float l) {
+  return l == 0.f || m == -INFINITY ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+}
+
 // Rare path of the softmax: re-centre the reference exponent of one query block on the row
 // maximum of the current tile and redo the tile's numerators.
 // With elementwise masks (EW) a query may have had nothing but masked keys so far (l == 0, or the
