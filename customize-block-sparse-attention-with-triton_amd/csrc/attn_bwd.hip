@@ -32,6 +32,7 @@ struct BwdParams {
   int B, H, N, nb, Bm, Hm;
   int out_f32;
   int split;                  // workgroups per row / column list (1: results written directly)
+  int whole;                  // split > 1: lists of up to this many tiles are one workgroup's all the same (-1: none)
   float* part_dq; float* part_dk; float* part_dv;   // split > 1: fp32 partial results [split][B*H][N][D]
   float sm_scale, qk_scale;   // qk_scale = sm_scale * log2(e)
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];
@@ -187,6 +188,23 @@ __device__ __forceinline__ void head_and_block(int L, int BH, int nb, int& bh, i
   blk = l / hg;          // >= nb for the padding of an incomplete last group
 }
 
+// Is the list at lp, lp + 1 so short that the first share's workgroup walks all of it?  (The pointer as a value the
+// compiler cannot trace back, or it makes these loads, and waits for them, in the workgroups of the first share too.)
+__device__ __forceinline__ bool walked_by_first(cint_ptr_t lp, int whole) {
+  asm volatile("" : "+s"(lp));
+  return lp[1] - lp[0] <= whole;
+}
+
+// Entries [u0, u1) of a list [t0, t0 + len) are share `chunk` of it.  Returns the number of its shares (1: chunk is 0).
+__device__ __forceinline__ int share_of_list(const BwdParams& prm, int t0, int len, int chunk, int& u0, int& u1) {
+  u0 = t0;
+  u1 = t0 + len;
+  if (len <= prm.whole || prm.split == 1) return 1;
+  u0 = t0 + (int)((int64_t)len * chunk / prm.split);
+  u1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
+  return prm.split;
+}
+
 // ---------------------------------------------------------------------------------------
 // dQ: workgroup = row block m, wavefront wv owns queries 64m + 32wv + ln
 // ---------------------------------------------------------------------------------------
@@ -217,6 +235,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
+  if (chunk > 0 && walked_by_first(rp + m, prm.whole)) return;
   // The rows this workgroup owns for its whole walk (Q, dO, O, lse of its queries) depend on the block index only:
   // they are asked for first, and travel while the list is looked up and the first tiles are requested.
   const int64_t qrow = (int64_t)m * 64 + 32 * wv + ln;
@@ -235,11 +254,12 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
 #pragma unroll
   for (int s = 0; s < KS; ++s) ofr[s] = *reinterpret_cast<const uintx4*>(op + 16 * s + 8 * g);
   const float lse_q = prm.lse[(int64_t)bh * prm.N + qsrc];
-  int u0, u1;                                                  // steps: tile u / STEPS, part u % STEPS
+  int u0, u1, split;                                           // steps: tile u / STEPS, part u % STEPS
   {
     const int t0 = rp[m], len = rp[m + 1] - t0;                // this workgroup's share of the row's list
-    u0 = (t0 + (int)((int64_t)len * chunk / prm.split)) * STEPS;
-    u1 = (t0 + (int)((int64_t)len * (chunk + 1) / prm.split)) * STEPS;
+    split = share_of_list(prm, t0, len, chunk, u0, u1);
+    u0 *= STEPS;
+    u1 *= STEPS;
   }
   const unsigned lds_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
 
@@ -357,7 +377,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
         dqacc[db] = mfma_qk<PB>(fkt[ts][db], dsf[ts], dqacc[db]);       // dQ^T += K^T dS^T
   }
 
-  if (prm.split > 1) {   // unscaled fp32 part; sum_parts_kernel adds the parts up
+  if (split > 1) {   // unscaled fp32 part; sum_parts_kernel adds the parts up
     if (!exists) return;
     float* part = prm.part_dq + ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
@@ -399,11 +419,13 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
-  int u0, u1;                                                  // steps: tile u / STEPS, part u % STEPS
+  if (chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
+  int u0, u1, split;                                           // steps: tile u / STEPS, part u % STEPS
   {
     const int t0 = cp[n], len = cp[n + 1] - t0;                // this workgroup's share of the column's list
-    u0 = (t0 + (int)((int64_t)len * chunk / prm.split)) * STEPS;
-    u1 = (t0 + (int)((int64_t)len * (chunk + 1) / prm.split)) * STEPS;
+    split = share_of_list(prm, t0, len, chunk, u0, u1);
+    u0 *= STEPS;
+    u1 *= STEPS;
   }
   const unsigned lds_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
 
@@ -529,7 +551,7 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
   }
 
   if (!exists) return;
-  if (prm.split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
+  if (split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
     const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -650,6 +672,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
+  if (chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
   // The K and V rows this wavefront owns for the whole walk depend on the block index only: asked for first, they
   // travel while the list is looked up and the first tiles are requested.
   const int64_t krow = (int64_t)n * 64 + 32 * kh + ln;
@@ -664,11 +687,10 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
     kfr[s] = *reinterpret_cast<const uintx4*>(kp + 16 * s + 8 * g);
     vfr[s] = *reinterpret_cast<const uintx4*>(vp + 16 * s + 8 * g);
   }
-  int u0, u1;
+  int u0, u1, split;
   {
     const int t0 = cp[n], len = cp[n + 1] - t0;                // this workgroup's share of the column's list
-    u0 = t0 + (int)((int64_t)len * chunk / prm.split);
-    u1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
+    split = share_of_list(prm, t0, len, chunk, u0, u1);
   }
   const unsigned lds_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
   const unsigned short* qg = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1];
@@ -841,7 +863,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
     second(fgt_oth, fqt_oth, pp, dp);
   }
 
-  if (prm.split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
+  if (split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
     if (!exists) return;
     const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
 #pragma unroll
@@ -875,26 +897,41 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
 }
 
 // ---------------------------------------------------------------------------------------
-// split > 1: out = scale * sum of the fp32 parts, rounded to the result type.  blockIdx.y: 0 dQ, 1 dK, 2 dV.
+// split > 1: out = scale * sum of the fp32 parts, rounded to the result type.  blockIdx.y: 0 dQ, 1 dK, 2 dV.  A workgroup
+// takes 256 quads (4 consecutive values); where lists that are not shared are written already (whole >= 0) a quarter of a
+// list's rows, most of which it leaves at once (D = 128, 16 heads N = 2176, keep 0.3, the whole backward: 256 quads 93 us,
+// a quarter 88, a list 87; 8 heads N = 4096 dense 276 / 276 / 285).
 // ---------------------------------------------------------------------------------------
+constexpr int SUM_ROWS = 16;
 template <bool BF16>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int64_t quads, int D) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;     // one thread per 4 consecutive values
-  if (i >= quads) return;
+  const int qpr = D / 4;                                   // quads per row
+  int64_t first = (int64_t)blockIdx.x * 256, last = quads < first + 256 ? quads : first + 256;
+  if (prm.whole >= 0) {
+    const int list = blockIdx.x / (64 / SUM_ROWS), unit = list / prm.nb, blk = list - unit * prm.nb;
+    const int b = unit / prm.H, h = unit - b * prm.H, mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
+    const cint_ptr_t lp = (cint_ptr_t)(uintptr_t)((blockIdx.y == 0 ? prm.row_ptr : prm.col_ptr) + (int64_t)mh * prm.nb);
+    if (lp[blk + 1] - lp[blk] <= prm.whole) return;
+    const int row0 = 64 * blk + SUM_ROWS * (blockIdx.x % (64 / SUM_ROWS)), rows = prm.N - row0 < SUM_ROWS ? prm.N - row0 : SUM_ROWS;
+    first = ((int64_t)unit * prm.N + row0) * qpr;
+    last = first + rows * qpr;
+  }
   const float* part = blockIdx.y == 0 ? prm.part_dq : (blockIdx.y == 1 ? prm.part_dk : prm.part_dv);
   void* out = blockIdx.y == 0 ? prm.dq : (blockIdx.y == 1 ? prm.dk : prm.dv);
   const int64_t* st = blockIdx.y == 0 ? prm.dqs : (blockIdx.y == 1 ? prm.dks : prm.dvs);
   const float scale = blockIdx.y == 2 ? 1.0f : prm.sm_scale;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int c = 0; c < prm.split; ++c) acc += reinterpret_cast<const floatx4*>(part)[c * quads + i];
-  // the parts are [B*H][N][D] without gaps; the result has its own strides
-  const int qpr = D / 4;                                   // quads per row
-  const int64_t row_all = i / qpr;
-  const int col = (int)(i - row_all * qpr) * 4;
-  const int bh = (int)(row_all / prm.N), row = (int)(row_all - (int64_t)bh * prm.N);
-  const int b = bh / prm.H, h = bh - b * prm.H;
-  store_out4<BF16>(out, b * st[0] + h * st[1] + row * st[2] + col, prm.out_f32, acc[0] * scale, acc[1] * scale,
-                   acc[2] * scale, acc[3] * scale);
+#pragma unroll 2
+  for (int64_t i = first + threadIdx.x; i < last; i += 256) {
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < prm.split; ++c) acc += reinterpret_cast<const floatx4*>(part)[c * quads + i];
+    // the parts are [B*H][N][D] without gaps; the result has its own strides
+    const int64_t row_all = i / qpr;
+    const int col = (int)(i - row_all * qpr) * 4;
+    const int bh = (int)(row_all / prm.N), row = (int)(row_all - (int64_t)bh * prm.N);
+    const int b = bh / prm.H, h = bh - b * prm.H;
+    store_out4<BF16>(out, b * st[0] + h * st[1] + row * st[2] + col, prm.out_f32, acc[0] * scale, acc[1] * scale,
+                     acc[2] * scale, acc[3] * scale);
+  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -917,17 +954,35 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 // D = 64 fills four workgroups per compute unit.  The larger head dimensions have one or two in dkdv4_kernel and parts two
 // and four times as large: two per compute unit, rounded to the nearest, but at D = 128 four where rows are long (the
 // imbalance of a causal mask then weighs more than the parts).  A share keeps at least 8 tiles of a dense list; 5 in a
-// launch of few short lists (at D = 128 that was slower), where the walk's latency is all.
-static int bwd_split(int B, int H, int N, int D) {
+// launch of few short lists (at D = 128 that was slower), where the walk's latency is all, except that lists of 16 or 17
+// tiles keep two shares (8 heads N = 1024: 35 with two, 39 with three) and shorter ones one from 112 lists on (12 heads
+// N = 640, keep 0.3: 24 with one, 28 with two).
+// At D = 128, block masks with about one to two lists per compute unit: the longest lists of a causal mask are what a launch
+// takes, and the shares of a sparse mask's cost more than they give.  So only lists longer than a share of a dense list are
+// shared there (`whole`).  One share for all / as many as here for all / this:
+//             4 heads N = 4096, keep 0.3    86 /  92 /  86     block-causal  183 / 132 / 122     dense  185 / 164 / 164
+//             6 heads N = 4096             108 / 120 / 111                   192 / 167 / 160            260 / 225 / 226
+//             8 heads N = 4096             113 / 136 / 119                   199 / 195 / 187            280 / 274 / 276
+//            16 heads N = 2176              86 / 109 /  88                   144 / 138 / 125            195 / 208 / 206
+//            12 heads N = 2048              70 /  84 /  73                   135 / 117 / 105            138 / 134 / 134
+//            14 heads N = 1792              60 /  -  /  68                   105 /  -  /  92            121 /  -  / 135   (one share there)
+// (Elementwise masks, 8 heads N = 4000, a training step: window of 1000 135 / 156 / 140, of 2000 212 / 218 / 226,
+// token-causal 316 / 291 / 287: one share from 1.33 lists per compute unit on.)
+struct BwdShares { int split, whole; };
+static BwdShares bwd_shares(int B, int H, int N, int D, bool elementwise) {
   const int64_t lists = (int64_t)B * H * ((N + 63) / 64), cus = compute_units();
   const int nb = (N + 63) / 64;
+  if (D == 128 && !elementwise && nb < 96 && 3 * lists >= 2 * cus && 4 * lists <= 9 * cus) {
+    const int split = 4 * lists <= 5 * cus ? 3 : 2;
+    if (nb > (split == 2 ? 28 : 24)) return {split, nb / split};
+  }
   int64_t s;
   if (D == 64 || (D == 128 && nb >= 96)) s = (4 * cus + lists - 1) / lists;
   else s = (2 * cus + lists / 2) / lists;
-  const bool few_short = D != 128 && nb <= 32 && 2 * lists <= cus;
-  const int cap = few_short ? nb / 5 : nb / 8;
+  int cap = nb / 8;
+  if (D != 128 && nb <= 32 && 2 * lists <= cus && (nb >= 18 || (nb < 16 && 16 * lists <= 7 * cus))) cap = nb / 5;
   if (s > cap) s = cap;
-  return (int)(s > 8 ? 8 : s < 1 ? 1 : s);
+  return {(int)(s > 8 ? 8 : s < 1 ? 1 : s), -1};
 }
 
 // floats in front of the parts (the parts are accessed 16 bytes at a time)
@@ -935,7 +990,8 @@ static size_t delta_floats(int B, int H, int N) { return ((size_t)B * H * N + 63
 
 size_t bwd_workspace_bytes(int B, int H, int N, int D) {
   const size_t delta = delta_floats(B, H, N) * sizeof(float);
-  const int split = bwd_split(B, H, N, D);
+  const int block = bwd_shares(B, H, N, D, false).split, words = bwd_shares(B, H, N, D, true).split;
+  const int split = block > words ? block : words;           // one size for both kinds of masks
   return delta + (split > 1 ? (size_t)3 * split * B * H * N * D * sizeof(float) : 0);   // + parts of dQ, dK, dV
 }
 
@@ -966,7 +1022,8 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
   else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);
   if (prm.split > 1) {
     const int64_t quads = (int64_t)BH * prm.N * D / 4;
-    hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3((unsigned)((quads + 255) / 256), 3), dim3(256), 0, st, prm, quads, D);
+    const unsigned blocks = prm.whole >= 0 ? (unsigned)(BH * prm.nb * (64 / SUM_ROWS)) : (unsigned)((quads + 255) / 256);
+    hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3(blocks, 3), dim3(256), 0, st, prm, quads, D);
   }
 }
 
@@ -982,7 +1039,9 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   prm.bits_rows = (const unsigned long long*)bits_rows; prm.bits_cols = (const unsigned long long*)bits_cols;
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   prm.out_f32 = s.out_dtype == BSATTN_F32;
-  prm.split = bwd_split(s.B, s.H, s.N, s.D);
+  const BwdShares shares = bwd_shares(s.B, s.H, s.N, s.D, bits_rows != nullptr);
+  prm.split = shares.split;
+  prm.whole = shares.whole;
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
     prm.part_dq = (float*)ws + delta_floats(s.B, s.H, s.N);

@@ -84,3 +84,22 @@ def test_python_wrapper_rejects_bad_input_without_gpu():
     with pytest.raises(RuntimeError):
         fm.build_groups_from_block_mask(m)                                       # CPU mask: no CPU path
 
+
+def test_backward_workspace_holds_the_shares_of_lists():
+    """D = 128, one to two lists per compute unit (256 of them): three and two workgroups share the long lists, or a
+    dense causal mask waits for its longest one; short lists and launches with more of them are not shared."""
+    from fa2_custom_mask import _ext
+    n = ctypes.c_size_t()
+
+    def shares(H, N, D):
+        assert _ext.lib().bsattn_bwd_workspace(1, H, N, D, ctypes.byref(n)) == 0
+        delta = H * N * 4
+        assert n.value >= delta
+        parts, rest = divmod(n.value - (delta + 255) // 256 * 256, 3 * H * N * D * 4)
+        assert rest == 0
+        return max(parts, 1)
+
+    assert [shares(H, 4096, 128) for H in (3, 4, 5, 6, 7, 8, 9, 10)] == [3, 3, 3, 2, 2, 2, 2, 1]
+    assert shares(12, 2048, 128) == 2 and shares(14, 1792, 128) == 1 and shares(7, 1600, 128) == 3
+    # D = 64: two shares of short lists only where the launch is small
+    assert [shares(8, N, 64) for N in (832, 1024)] == [2, 2] and shares(12, 640, 64) == 1 and shares(4, 1280, 64) == 4

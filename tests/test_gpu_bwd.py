@@ -273,3 +273,40 @@ def test_large_magnitudes_backward_d128_fp16(dev):
         # (the softmax is nearly one-hot and the exponents carry the rounding of the 16-bit scaled Q: a looser
         # bar than for N(0,1) data; an overflowing piece gives NaN or errors of the size of the result)
         assert rl <= 5e-3, name
+
+
+# (heads, N): 3 shares of lists longer than 8 tiles, 2 shares of lists longer than 15, N not whole tiles
+@pytest.mark.parametrize("H,N", [(7, 1600), (16, 1860)])
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+def test_only_long_lists_are_shared(dev, H, N, dtype, out_fp32):
+    """D = 128 with one to two lists per compute unit: rows and columns with no tile, with as many as one workgroup
+    walks, with one more, and full ones, side by side."""
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    whole = 8 if H == 7 else 15
+    m = torch.zeros(nb, nb, dtype=torch.bool)
+    m[0] = True                                              # full
+    m[2, :whole] = True                                      # the longest that is not shared, and one more
+    m[3, :whole + 1] = True
+    m[4:4 + whole - 2, nb - 1] = True                        # (with row 0 and the diagonal: columns of the same lengths)
+    m[4:4 + whole - 1, nb - 3] = True
+    m[:, nb - 2] = True
+    m |= torch.eye(nb, dtype=torch.bool) & (torch.arange(nb) > 4)[:, None]
+    m[1] = False                                             # no tile
+    m[:, 6] = False
+    assert m.sum(1)[[0, 1, 2, 3]].tolist() == [nb - 1, 0, whole, whole + 1]
+    assert m.sum(0)[[6, nb - 1, nb - 3]].tolist() == [0, whole, whole + 1]
+    mask = m[None, None]
+    q, k, v, do = make_qkv(1, H, N, 128, dtype, 71, n=4)
+    sc = 128 ** -0.5
+    o, lse, dq, dk, dv = fm.attention_forward_backward(q.to(dev), k.to(dev), v.to(dev), mask.to(dev), sc, do.to(dev), out_fp32=out_fp32)
+    torch.cuda.synchronize()
+    dense = np.ascontiguousarray(orc.expand_block_mask(mask.numpy())[..., :N, :N])
+    for h in (0, H - 1):
+        sl = (slice(None), slice(h, h + 1))
+        refs = orc.attention_backward(f32(q[sl]), f32(k[sl]), f32(v[sl]), dense, sc, f32(do[sl]))
+        for got, ref in zip((dq[sl], dk[sl], dv[sl]), refs):
+            ma, rl = errors(got, ref)
+            assert ma <= MAXABS[dtype] and rl <= (1e-3 if (dtype == torch.float16 or out_fp32) else 3e-3), (h, ma, rl)
+    assert float(dq[:, :, 64:128].abs().max()) == 0.0
+    assert float(dk[:, :, 384:448].abs().max()) == 0.0 and float(dv[:, :, 384:448].abs().max()) == 0.0
