@@ -34,6 +34,7 @@
 #include "fwd_tile.h"
 #include "kernel_util.h"
 #include "range_perm.h"
+#include "row_parts.h"
 
 namespace bsattn {
 
@@ -73,6 +74,8 @@ template <int D> struct FwdCfg {
 // row block beyond N repeat the last query and are not written.
 enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2, STRIDED_WHOLE = 3 };
 enum { COOP = 0, ROWS_MODE = 1, WAVE = 2 };
+// ROWS: workgroups for long row blocks in a launch; a multiple of 8, so that those behind them keep their XCD
+__host__ __device__ constexpr int rows_extras(int BH, int W) { return (BH * W + 7) & ~7; }
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
 __global__ __launch_bounds__(MODE != COOP ? 64 : FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
 void fwd_kernel(const FwdParams prm) {
@@ -98,11 +101,15 @@ void fwd_kernel(const FwdParams prm) {
   if constexpr (ROWS) {
     // (head, row block): heads in groups of 8, one per XCD (workgroups go to the XCDs round-robin), so that the row
     // blocks at work on an XCD share the K and V of one head in its L2; the last row blocks, the long ones of
-    // block-causal masks, first
-    const int L = blockIdx.x, grp = L / (8 * nb), l = L - grp * 8 * nb, hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;
+    // block-causal masks, first.  Behind the first `first_ids` of them, which fill the GPU, W workgroups per head for the
+    // long row blocks (wg >= nb; see below).
+    const int extras = rows_extras(BH, prm.W), id = blockIdx.x;
+    const bool extra = id >= prm.first_ids && id < prm.first_ids + extras;
+    const int L = id < prm.first_ids ? id : extra ? id - prm.first_ids : id - extras, per = extra ? prm.W : nb;
+    if (extra && L >= BH * prm.W) return;
+    const int grp = L / (8 * per), l = L - grp * 8 * per, hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;
     bh = 8 * grp + l % hg;
-    wg = nb - 1 - l / hg;
-    if (wg < 0) return;                // padding of an incomplete last group
+    wg = per - 1 - l / hg + (extra ? nb : 0);
   } else {
     bh = blockIdx.x % BH;
     wg = blockIdx.x / BH;
@@ -313,10 +320,10 @@ void fwd_kernel(const FwdParams prm) {
     fresh = true;
     any_m = 0;
   };
-  // WAVE: per-lane addresses that do not change from row block to row block are not to be held through the tile loops:
-  // the lane index as a value the compiler cannot trace back
+  // One wavefront: per-lane addresses that do not change from row block to row block are not to be held through the tile
+  // loops: the lane index as a value the compiler cannot trace back
   auto fresh_lane = [&](int x) {
-    if constexpr (MODE == WAVE) asm volatile("" : "+v"(x));
+    if constexpr (ONE) asm volatile("" : "+v"(x));
     return x;
   };
   auto load_q = [&](int r) {
@@ -642,24 +649,170 @@ void fwd_kernel(const FwdParams prm) {
     }
   };
 
+  // One wavefront: a part of a row block that several workgroups share is published and counted in as in the other mode
+  // below; the last one in reads all parts (its own as well) and sums them in their order.  own: this part's slot;
+  // parts(first, count): the number of parts and where they begin; slot_of(i, first): part i.
+  auto share_row = [&](int row, float* own, auto&& parts, auto&& slot_of) {
+    float lsum[2], M[2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
+      if (!(lsum[qb] > 0.f)) lsum[qb] = 0.f;
+      M[qb] = lsum[qb] > 0.f ? m_i[qb] : -INFINITY;
+    }
+    const int lane_p = fresh_lane(lane), ln = lane_p & 31, g = lane_p >> 5;
+    unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + row;
+    unsigned long long seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int quad = 0; quad < D / 4; ++quad) {
+      const int idx = 4 * quad;
+      const floatx16& o = oacc[idx / 32][(idx / 16) & 1];
+      coherent_store4(own + idx * 64 + lane_p * 4, o[idx & 15], o[(idx & 15) + 1], o[(idx & 15) + 2], o[(idx & 15) + 3]);
+    }
+    if (g == 0) {
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        coherent_store(own + 64 * D + qb * 32 + ln, M[qb]);
+        coherent_store(own + 64 * D + 64 + qb * 32 + ln, lsum[qb]);
+      }
+    }
+    int first = 0, nparts = 0;
+    parts(first, nparts);
+    wait_vm<0>();                             // every store of the part has been acknowledged
+    int counted_v = 0;
+    if (lane == 0) {
+      unsigned long long old = seen;
+      for (;;) {     // (ends: the counter only changes when another part is counted, at most nparts times)
+        const unsigned long long want = (old >> 16) == prm.epoch ? old + 1 : ((prm.epoch << 16) | 1ull);
+        if (__hip_atomic_compare_exchange_strong(arrivals, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT)) {
+          counted_v = (int)(want & 0xffffull);
+          break;
+        }
+      }
+    }
+    if (__builtin_amdgcn_readfirstlane(counted_v) != nparts) return;
+    float Ms[2] = {-INFINITY, -INFINITY}, Ls[2] = {0.f, 0.f};
+    reset_acc();
+    for (int p = 0; p < nparts; ++p) {
+      const float* sp = slot_of(p, first);
+      float sc_own[2], sc_p[2];
+#pragma unroll
+      for (int qb = 0; qb < 2; ++qb) {
+        const float mp = coherent_load(sp + 64 * D + qb * 32 + ln), lp = coherent_load(sp + 64 * D + 64 + qb * 32 + ln);
+        const float mn = fmaxf(Ms[qb], mp);     // a side without mass has maximum -inf and weight 0
+        sc_own[qb] = Ms[qb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Ms[qb] - mn);
+        sc_p[qb] = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mn);
+        Ls[qb] = Ls[qb] * sc_own[qb] + lp * sc_p[qb];
+        Ms[qb] = mn;
+      }
+#pragma unroll
+      for (int q4 = 0; q4 < D / 4; q4 += 4) {    // (four quads, 4 KB, per wait)
+        floatx4 ld[4];
+        coherent_load4x4(sp + q4 * 256 + lane_p * 4, ld[0], ld[1], ld[2], ld[3]);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int idx = 4 * q4 + e, qb = (idx / 16) & 1;
+          oacc[idx / 32][qb][idx & 15] = oacc[idx / 32][qb][idx & 15] * sc_own[qb] + sc_p[qb] * ld[e / 4][e & 3];
+        }
+      }
+    }
+    // (write_row sums the two halves of a query)
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) { m_i[qb] = Ms[qb]; l_i[qb] = g == 0 ? Ls[qb] : 0.f; }
+    write_row(row);
+    // back to zero, so that a replay of this launch (same mark) starts from a clean counter
+    if (lane == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+
   if constexpr (ROWS) {
     // ================= one wavefront, one row block =================
-    const int ta = rp[wg], tb = rp[wg + 1];
-    if (ta == tb) { write_empty_row(wg); return; }
-    int cx = flagged_col(ta);                                  // current tile: column block | flag
-    k_copy_all(cx & COL_MASK, ta);
-    v_copy_all(cx & COL_MASK);
-    stage_cols(ta, tb);
-    auto col_of = [&](int t) { return t - ta < COLS_CAP ? lcols[t - ta] : flagged_col(t); };
-    reset_acc();
-    load_q(wg);
-    for (int j = ta; j < tb; ++j) {
-      const bool has1 = j + 1 < tb;
-      const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(j + 1)) : 0;
-      tile(has1, cxn & COL_MASK, j + 1, has1, is_partial(cx), [] {});
-      cx = cxn;
+    // Row blocks much longer than the others (the rows of text tokens in front of a video, kept whole) would still be
+    // walked when all others are done: those above 2.5 times the head's mean length are left to W workgroups per head
+    // (wg = nb + p), which cut them into parts (row_parts.h).  Such a workgroup takes the parts p, p + W, ...; the parts of a
+    // row block that is cut meet as those of ranges do, in one of W slots each.
+    // The W workgroups come when the first row blocks have filled the GPU: in front of them they made a causal launch slower (48
+    // heads N = 4096 152 -> 168 us: row blocks then go where a workgroup without work has just ended, long ones side by
+    // side), behind all others the parts of a small launch are a tail (24 heads, below: 114 us).
+    // bf16, us before / after, and the ranges of workgroups (MODE 0) that this mode replaced:
+    //   48 heads N = 17792, keep 0.05, row blocks 0-3 and columns 0-3 kept whole   735 / 415   643     keep 0.2  1238 / 1008   1639
+    //   24 heads N = 8192,  keep 0.1,  the same rows and columns                   251 / 101   116     12 heads N = 17792  525 / 172   193
+    //   without long row blocks: 48 heads keep 0.05 295 / 285, keep 0.2 913 / 913; 24 heads keep 0.1 75 / 75, causal 299 / 293
+    const int T = rp[nb] - rp[0];
+    auto is_long = [&](int len) { return is_long_row(len, T, nb); };
+    int row = wg, ta, tb, parts = 1, slot0 = 0, slot_own = 0, item = wg - nb, part_len = 0;
+    auto find = [&]() {       // the row block, tiles and slots of `item`; false if there is no such item
+      const int32_t* rpg = prm.row_ptr + (int64_t)mh * nb;
+      int items = 0, slots = 0;
+      for (int r0 = 0; r0 < nb; r0 += 64) {
+        const int r = r0 + lane, len = r < nb ? rpg[r + 1] - rpg[r] : 0;
+        const int n = is_long(len) ? parts_of_row(len, part_len) : 0;
+        int upto = n, slots_upto = n > 1 ? n : 0;                  // ... of this row block and those before it
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int a = __shfl_up(upto, off), b = __shfl_up(slots_upto, off);
+          if (lane >= off) { upto += a; slots_upto += b; }
+        }
+        const unsigned long long behind = __ballot(items + upto > item);
+        if (behind != 0ull) {
+          const int at = __builtin_ctzll(behind);
+          parts = __builtin_amdgcn_readfirstlane(__shfl(n, at));
+          const int part = item - (items + __builtin_amdgcn_readfirstlane(__shfl(upto, at)) - parts);
+          slot0 = slots + __builtin_amdgcn_readfirstlane(__shfl(slots_upto, at)) - parts;      // (parts > 1)
+          row = r0 + at;
+          const int row_s = rp[row], row_len = rp[row + 1] - row_s;
+          ta = row_s + part_begin(row_len, parts, part);
+          tb = row_s + part_begin(row_len, parts, part + 1);
+          slot_own = slot0 + part;
+          return true;
+        }
+        items += __builtin_amdgcn_readfirstlane(__shfl(upto, 63));
+        slots += __builtin_amdgcn_readfirstlane(__shfl(slots_upto, 63));
+      }
+      return false;
+    };
+    if (wg < nb) {
+      ta = rp[wg]; tb = rp[wg + 1];
+      if (ta == tb) { write_empty_row(wg); return; }
+      if (prm.W > 0 && is_long(tb - ta)) return;
+    } else {
+      const int32_t* rpg = prm.row_ptr + (int64_t)mh * nb;
+      int sum = 0, count = 0;
+      for (int r = lane; r < nb; r += 64) {
+        const int len = rpg[r + 1] - rpg[r];
+        if (is_long(len)) { sum += len; ++count; }
+      }
+      if (!__any(count > 0)) return;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) { sum += __shfl_xor(sum, off); count += __shfl_xor(count, off); }
+      part_len = long_part_tiles(__builtin_amdgcn_readfirstlane(sum), __builtin_amdgcn_readfirstlane(count), prm.W, T / nb);
+      if (!find()) return;
     }
-    write_row(wg);
+    for (;;) {
+      int cx = flagged_col(ta);                                // current tile: column block | flag
+      k_copy_all(cx & COL_MASK, ta);
+      v_copy_all(cx & COL_MASK);
+      stage_cols(ta, tb);
+      auto col_of = [&](int t) { return t - ta < COLS_CAP ? lcols[t - ta] : flagged_col(t); };
+      reset_acc();
+      load_q(row);
+      for (int j = ta; j < tb; ++j) {
+        const bool has1 = j + 1 < tb;
+        const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(j + 1)) : 0;
+        tile(has1, cxn & COL_MASK, j + 1, has1, is_partial(cx), [] {});
+        cx = cxn;
+      }
+      if (parts == 1) {
+        write_row(row);
+      } else {
+        auto slot_at = [&](int i) { return prm.ws + ((int64_t)bh * prm.W + i) * partial_floats(D); };
+        share_row(row, slot_at(slot_own), [&](int& first, int& count) { first = slot0; count = parts; },
+                  [&](int i, int first) { return slot_at(first + i); });
+      }
+      if (wg < nb) return;
+      item += prm.W;
+      if (!find()) return;
+    }
   } else if constexpr (MODE == WAVE) {
     // ================= one wavefront, one range =================
     // first row block of the range: largest r with rp[r] <= g0 < rp[r+1]
@@ -686,6 +839,9 @@ void fwd_kernel(const FwdParams prm) {
       }
       if (g0 >= g1) return;
     }
+    // two slots per workgroup: a range can end inside one row block (that part goes to slot 1: it holds the row
+    // block's first tiles) after having begun inside another (slot 0)
+    auto wg_slot = [&](int p, bool head) { return prm.ws + (((int64_t)bh * prm.W + p) * 2 + (head ? 1 : 0)) * partial_floats(D); };
     int cx = flagged_col(g0);                                  // current tile: column block | flag
     k_copy_all(cx & COL_MASK, g0);
     v_copy_all(cx & COL_MASK);
@@ -707,84 +863,14 @@ void fwd_kernel(const FwdParams prm) {
       if (t == row_s && seg_b == row_e) {
         write_row(r);
       } else {
-        // a part of a row block that ranges share: published and counted in as in the other mode below; the last one
-        // in reads all parts (its own as well) and sums them in the order of the ranges
-        float lsum[2], M[2];
-#pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
-          lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
-          if (!(lsum[qb] > 0.f)) lsum[qb] = 0.f;
-          M[qb] = lsum[qb] > 0.f ? m_i[qb] : -INFINITY;
-        }
-        const int lane_p = fresh_lane(lane), ln = lane_p & 31, g = lane_p >> 5;
-        auto slot_of = [&](int p, bool head) { return prm.ws + (((int64_t)bh * prm.W + p) * 2 + (head ? 1 : 0)) * partial_floats(D); };
-        float* slot = slot_of(wg, t == row_s);
-        unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + r;
-        unsigned long long seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int quad = 0; quad < D / 4; ++quad) {
-          const int idx = 4 * quad;
-          const floatx16& o = oacc[idx / 32][(idx / 16) & 1];
-          coherent_store4(slot + idx * 64 + lane_p * 4, o[idx & 15], o[(idx & 15) + 1], o[(idx & 15) + 2], o[(idx & 15) + 3]);
-        }
-        if (g == 0) {
-#pragma unroll
-          for (int qb = 0; qb < 2; ++qb) {
-            coherent_store(slot + 64 * D + qb * 32 + ln, M[qb]);
-            coherent_store(slot + 64 * D + 64 + qb * 32 + ln, lsum[qb]);
-          }
-        }
-        const int64_t xrow = row_pos(hs, r, row_s);
-        int pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)), pf_ = split_of_pos(hs, xrow);
-        while (pl_ > pf_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pl_), r, row_s, row_e), row_s, row_e) >= row_e) --pl_;
-        while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
-        const int nparts = pl_ - pf_ + 1;
-        wait_vm<0>();                             // every store of the part has been acknowledged
-        int counted_v = 0;
-        if (lane == 0) {
-          unsigned long long old = seen;
-          for (;;) {     // (ends: the counter only changes when another part is counted, at most nparts times)
-            const unsigned long long want = (old >> 16) == prm.epoch ? old + 1 : ((prm.epoch << 16) | 1ull);
-            if (__hip_atomic_compare_exchange_strong(arrivals, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                                     __HIP_MEMORY_SCOPE_AGENT)) {
-              counted_v = (int)(want & 0xffffull);
-              break;
-            }
-          }
-        }
-        if (__builtin_amdgcn_readfirstlane(counted_v) == nparts) {
-          float Ms[2] = {-INFINITY, -INFINITY}, Ls[2] = {0.f, 0.f};
-          reset_acc();
-          for (int p = pf_; p <= pl_; ++p) {
-            const float* sp = slot_of(p, p == pf_);
-            float sc_own[2], sc_p[2];
-#pragma unroll
-            for (int qb = 0; qb < 2; ++qb) {
-              const float mp = coherent_load(sp + 64 * D + qb * 32 + ln), lp = coherent_load(sp + 64 * D + 64 + qb * 32 + ln);
-              const float mn = fmaxf(Ms[qb], mp);     // a side without mass has maximum -inf and weight 0
-              sc_own[qb] = Ms[qb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Ms[qb] - mn);
-              sc_p[qb] = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mn);
-              Ls[qb] = Ls[qb] * sc_own[qb] + lp * sc_p[qb];
-              Ms[qb] = mn;
-            }
-#pragma unroll
-            for (int q4 = 0; q4 < D / 4; q4 += 4) {    // (four quads, 4 KB, per wait)
-              floatx4 ld[4];
-              coherent_load4x4(sp + q4 * 256 + lane_p * 4, ld[0], ld[1], ld[2], ld[3]);
-#pragma unroll
-              for (int e = 0; e < 16; ++e) {
-                const int idx = 4 * q4 + e, qb = (idx / 16) & 1;
-                oacc[idx / 32][qb][idx & 15] = oacc[idx / 32][qb][idx & 15] * sc_own[qb] + sc_p[qb] * ld[e / 4][e & 3];
-              }
-            }
-          }
-          // (write_row sums the two halves of a query)
-#pragma unroll
-          for (int qb = 0; qb < 2; ++qb) { m_i[qb] = Ms[qb]; l_i[qb] = g == 0 ? Ls[qb] : 0.f; }
-          write_row(r);
-          // back to zero, so that a replay of this launch (same mark) starts from a clean counter
-          if (lane == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        share_row(r, wg_slot(wg, t == row_s), [&](int& first, int& count) {
+          const int64_t xrow = row_pos(hs, r, row_s);
+          int pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)), pf_ = split_of_pos(hs, xrow);
+          while (pl_ > pf_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pl_), r, row_s, row_e), row_s, row_e) >= row_e) --pl_;
+          while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
+          first = pf_;
+          count = pl_ - pf_ + 1;
+        }, [&](int i, int first) { return wg_slot(first + i, i == 0); });
       }
       t = seg_b;
       ++r;
@@ -1187,13 +1273,20 @@ int compute_units() {
 // wavefront takes a range of the list (32 heads of N = 4096 dense 174 -> 149 us; 8 heads of N = 17536 dense 710
 // either way, keep 0.1 with a new mask per call 115 -> 106); with fewer the ranges of whole workgroups are the faster ones (6 heads of N = 17776 at keep 0.3: 236
 // against 250 us).
+static int wave_slots() { return FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * compute_units(); }    // wavefronts resident at once, D = 64
 static int fwd_mode(int B, int H, int nb, int D, bool compact) {
   if (D != 64) return COOP;
-  const int64_t rows = (int64_t)B * H * nb, slots = FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * (int64_t)compute_units();
+  const int64_t rows = (int64_t)B * H * nb, slots = wave_slots();
   return 2 * rows >= 3 * slots ? ROWS_MODE : (rows >= slots && !compact ? WAVE : COOP);     // (compact: WAVE has four times as many ranges, hence parts)
 }
 
-static int groups_per_head(int B, int H, int nb, int D, int mode) {
+// ROWS_MODE: the workgroups per head for long row blocks, and the slots for their parts: as many as are resident at once,
+// half of them where the scratch memory is the library's.  None with so many heads that a wavefront has the tiles of an
+// eighth of a head to do, or where the library's scratch memory does not hold the counters.
+static int long_row_groups(int B, int H, int nb, bool compact);
+
+static int groups_per_head(int B, int H, int nb, int D, int mode, bool compact) {
+  if (mode == ROWS_MODE) return long_row_groups(B, H, nb, compact);
   const int cus = compute_units();
   const int per_cu = D != 64 ? FwdCfg<128>::WG_PER_CU : (mode == COOP ? 1 : FwdCfg<64>::NW) * FwdCfg<64>::WG_PER_CU;
   int64_t W = (int64_t)cus * per_cu / ((int64_t)B * H);   // as many workgroups as are resident at once
@@ -1203,9 +1296,19 @@ static int groups_per_head(int B, int H, int nb, int D, int mode) {
   return (int)W;
 }
 
-// workspace: partial slots [B*H][W][2][partial_floats] (fp32), then the arrival counters [B*H][nb] (64 bit)
-static size_t slots_bytes(int B, int H, int W, int D) {
-  return (size_t)B * H * W * 2 * partial_floats(D) * sizeof(float);
+// workspace: partial slots [B*H][W][2][partial_floats] (fp32; ROWS_MODE: one per workgroup for long row blocks), then the
+// arrival counters [B*H][nb] (64 bit)
+static size_t slots_bytes(int B, int H, int W, int D, int mode) {
+  return (size_t)B * H * W * (mode == ROWS_MODE ? 1 : 2) * partial_floats(D) * sizeof(float);
+}
+static size_t parts_bytes(int B, int H, int nb, int W, int D, int mode) {
+  return slots_bytes(B, H, W, D, mode) + (size_t)B * H * nb * sizeof(unsigned long long);
+}
+
+static int long_row_groups(int B, int H, int nb, bool compact) {
+  const int64_t W = wave_slots() / (compact ? 2 : 1) / ((int64_t)B * H);
+  if (W < 8) return 0;
+  return compact && parts_bytes(B, H, nb, (int)W, 64, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
 // D = 128 with enough row blocks in the launch to fill the chip goes to the kernel that gives each
@@ -1260,9 +1363,9 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
   if (D == 256) return 256 + pair_parts_bytes(B, H, N, D, pair_split(B, H, (N + 63) / 64, D));   // the pair kernel only
   const int nb = (N + 63) / 64;
   const int mode = fwd_mode(B, H, nb, D, compact);
-  if (mode == ROWS_MODE) return 256;      // nothing is shared
-  const int W = groups_per_head(B, H, nb, D, mode);
-  const size_t bytes = slots_bytes(B, H, W, D) + (size_t)B * H * nb * sizeof(unsigned long long);
+  const int W = groups_per_head(B, H, nb, D, mode, compact);
+  if (W == 0) return 256;                 // nothing is shared
+  const size_t bytes = parts_bytes(B, H, nb, W, D, mode);
   if (D != 128 || compact) return bytes;      // (compact launches: whole tiles and block masks only)
   const size_t parts = 256 + pair_parts_bytes(B, H, N, D, pair_split_128((int64_t)B * H * nb, nb, true));
   return parts > bytes ? parts : bytes;
@@ -1313,7 +1416,7 @@ static void launch_fwd_d(const FwdParams& prm, int D, int mode, int dt, hipStrea
   const int BH = prm.B * prm.H, grid = prm.W * BH;
   if (D == 128) {
     if constexpr (!EW) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
-  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, ((BH + 7) / 8) * 8 * prm.nb, st);
+  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, BH * prm.nb + rows_extras(BH, prm.W), st);
   else if (mode == WAVE) launch_fwd_m<64, WAVE, EW>(prm, dt, grid, st);
   else launch_fwd_m<64, COOP, EW>(prm, dt, grid, st);
 }
@@ -1365,13 +1468,13 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.tile_partial = tile_partial; prm.tile_bits = (const unsigned long long*)tile_bits;
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.D, s.compact);
-  prm.W = groups_per_head(s.B, s.H, prm.nb, s.D, mode);
+  prm.W = groups_per_head(s.B, s.H, prm.nb, s.D, mode, s.compact);
   // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are.  (Not WAVE: single
   // wavefronts that arrive while another kernel ends do not fill the SIMDs in order, and two with the larger share on one
   // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
   // after a pause 677 against 707.)
-  prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : 0;
-  prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D));
+  prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
+  prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();
   {

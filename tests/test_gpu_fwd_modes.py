@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import make_qkv, uniform_block_mask, errors, f32
+from helpers import make_qkv, uniform_block_mask, errors, f32, same_up_to_rounding
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +114,72 @@ def test_shared_lists(dev, H, N, D, dtype, elementwise, out_fp32):
         for name, got, ref in zip(("dq", "dk", "dv"), res[2:], grads):
             ma, rl = errors(got[sl], ref)
             assert rl <= (2e-3 if rel == 1e-3 else 1e-2), (name, ma, rl)
+
+
+def long_row_masks(nb, H):
+    """Block masks [1, H, nb, nb] with row blocks that are much longer than the others (ROWS_MODE cuts them)."""
+    g = torch.Generator().manual_seed(77)
+    m = torch.rand(1, H, nb, nb, generator=g) < 0.06
+    m[:, :, :, 1] = True
+    m[0, 0, :4] = True                                       # the rows of leading text tokens
+    m[0, 1] = False
+    m[0, 1, nb // 2] = True                                  # one full row block, nothing else
+    m[0, 2] = False
+    m[0, 2, torch.arange(nb) % 4 == 1] = True                # a quarter of the row blocks full, the others empty
+    m[0, 3, nb - 1] = True                                   # the last, partly filled row block
+    m[0, 3, 0, :25] = True                                   # (25 tiles: the shortest that is cut)
+    m[0, 4] = True                                           # no row block longer than the others
+    return m
+
+
+# 3240 and 3264 row blocks: one wavefront takes one; the long ones are cut
+@pytest.mark.parametrize("H,N,elementwise", [(60, 3450, False), (60, 3450, True), (24, 8704, False)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_long_row_blocks(dev, H, N, dtype, elementwise):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 64, dtype, 600 + N)]
+    block = long_row_masks(nb, H)
+    mask = block.to(dev)
+    if elementwise:
+        i = torch.arange(N, device=dev)
+        mask = mask.repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N] & ((i[:, None] - i[None, :]) % 7 != 0)
+    call = lambda: fm.flash_attention_custom_mask_lse(q, k, v, mask, 0.125)
+    o, lse = call()
+    for _ in range(3):                                       # parts are summed in their order: the same bits every time
+        o2, lse2 = call()
+        assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream(dev).wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        o3, lse3 = call()
+    for _ in range(3):                                       # (a replay counts its parts in again)
+        o3.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, o3) and torch.equal(lse, lse3)
+        call()
+    if N % 64 == 0:                                          # the library's own scratch memory: half as many parts
+        from fa2_custom_mask import _ext
+        lists = fm.block_mask_to_lists(mask)
+        o4, lse4 = torch.empty_like(o), torch.empty_like(lse)
+        code, st = _ext.dtype_code(dtype), _ext.strides4(q)
+        rc = _ext.lib().bsattn_fwd_static(q.data_ptr(), k.data_ptr(), v.data_ptr(), o4.data_ptr(), lse4.data_ptr(), lists.row_ptr_ptr,
+                                          lists.col_idx_ptr, 1, H, 1, H, N, 64, code, code, 0.125, st, st, st, st, _ext.current_stream(dev))
+        torch.cuda.synchronize()
+        assert rc == 0 and same_up_to_rounding(o4, o, rel=2.0 ** -6, abs_=2e-3)
+        fin = torch.isfinite(lse)
+        assert torch.equal(torch.isfinite(lse4), fin) and float((lse4 - lse)[fin].abs().max()) <= 2e-3
+    for h in range(6 if N < 4000 else 3):
+        keep = (mask[0, h] if elementwise else mask[0, h].repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N])
+        s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~keep, float("-inf"))
+        ref_lse = torch.logsumexp(s, -1)
+        ref = torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float()
+        ma, rl = errors(o[0, h], ref)
+        assert ma <= MAXABS[dtype] and rl <= RELL2[dtype], (h, ma, rl)
+        fin = torch.isfinite(ref_lse)
+        assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref_lse)[fin].abs().max()) <= 2e-3
