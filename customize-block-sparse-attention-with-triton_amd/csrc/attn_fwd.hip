@@ -99,16 +99,16 @@ void fwd_kernel(const FwdParams prm) {
   const int BH = prm.B * prm.H, nb = prm.nb;
   int bh, wg;
   if constexpr (ROWS) {
-    // (head, row block): heads in groups of 8, one per XCD (workgroups go to the XCDs round-robin), so that the row
-    // blocks at work on an XCD share the K and V of one head in its L2; the last row blocks, the long ones of
-    // block-causal masks, first.  Behind the first `first_ids` of them, which fill the GPU, W workgroups per head for the
-    // long row blocks (wg >= nb; see below).
+    // (head, row block): heads in groups of `group`, a multiple of 8, spread over the XCDs (workgroups go to them
+    // round-robin), so that the row blocks at work on an XCD share the K and V of few heads in its L2 (rows_group); in a
+    // group the last row blocks of all heads, the long ones of block-causal masks, first.  Behind the first `first_ids`
+    // of them, which fill the GPU, W workgroups per head for the long row blocks (wg >= nb; see below).
     const int extras = rows_extras(BH, prm.W), id = blockIdx.x;
     const bool extra = id >= prm.first_ids && id < prm.first_ids + extras;
     const int L = id < prm.first_ids ? id : extra ? id - prm.first_ids : id - extras, per = extra ? prm.W : nb;
     if (extra && L >= BH * prm.W) return;
-    const int grp = L / (8 * per), l = L - grp * 8 * per, hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;
-    bh = 8 * grp + l % hg;
+    const int gs = prm.group, grp = L / (gs * per), l = L - grp * gs * per, hg = BH - gs * grp < gs ? BH - gs * grp : gs;
+    bh = gs * grp + l % hg;
     wg = per - 1 - l / hg + (extra ? nb : 0);
   } else {
     bh = blockIdx.x % BH;
@@ -738,44 +738,47 @@ void fwd_kernel(const FwdParams prm) {
     //   48 heads N = 17792, keep 0.05, row blocks 0-3 and columns 0-3 kept whole   735 / 415   643     keep 0.2  1238 / 1008   1639
     //   24 heads N = 8192,  keep 0.1,  the same rows and columns                   251 / 101   116     12 heads N = 17792  525 / 172   193
     //   without long row blocks: 48 heads keep 0.05 295 / 285, keep 0.2 913 / 913; 24 heads keep 0.1 75 / 75, causal 299 / 293
-    const int T = rp[nb] - rp[0];
+    int row = wg, ta, tb, parts = 1, slot0 = 0, slot_own = 0, item = wg - nb, part_len = 0, T = 0;
     auto is_long = [&](int len) { return is_long_row(len, T, nb); };
-    int row = wg, ta, tb, parts = 1, slot0 = 0, slot_own = 0, item = wg - nb, part_len = 0;
+    // (the head's tiles; the pointer as a value the compiler cannot trace back: looked up only where needed)
+    auto total = [&]() {
+      cint_ptr_t p = rp;
+      asm volatile("" : "+s"(p));
+      return p[nb] - p[0];
+    };
     auto find = [&]() {       // the row block, tiles and slots of `item`; false if there is no such item
       const int32_t* rpg = prm.row_ptr + (int64_t)mh * nb;
       int items = 0, slots = 0;
       for (int r0 = 0; r0 < nb; r0 += 64) {
-        const int r = r0 + lane, len = r < nb ? rpg[r + 1] - rpg[r] : 0;
-        const int n = is_long(len) ? parts_of_row(len, part_len) : 0;
-        int upto = n, slots_upto = n > 1 ? n : 0;                  // ... of this row block and those before it
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const int a = __shfl_up(upto, off), b = __shfl_up(slots_upto, off);
-          if (lane >= off) { upto += a; slots_upto += b; }
+        const int r = r0 + fresh_lane(lane), len = r < nb ? rpg[r + 1] - rpg[r] : 0;
+        for (unsigned long long left = __ballot(is_long(len)); left != 0ull; left &= left - 1ull) {
+          const int at = __builtin_ctzll(left), row_len = __builtin_amdgcn_readlane(len, at);
+          const int n = parts_of_row(row_len, part_len);
+          if (item < items + n) {
+            const int part = item - items;
+            row = r0 + at;
+            ta = rp[row] + part_begin(row_len, n, part);
+            tb = rp[row] + part_begin(row_len, n, part + 1);
+            parts = n;
+            slot0 = slots;
+            slot_own = slots + part;
+            return true;
+          }
+          items += n;
+          if (n > 1) slots += n;
         }
-        const unsigned long long behind = __ballot(items + upto > item);
-        if (behind != 0ull) {
-          const int at = __builtin_ctzll(behind);
-          parts = __builtin_amdgcn_readfirstlane(__shfl(n, at));
-          const int part = item - (items + __builtin_amdgcn_readfirstlane(__shfl(upto, at)) - parts);
-          slot0 = slots + __builtin_amdgcn_readfirstlane(__shfl(slots_upto, at)) - parts;      // (parts > 1)
-          row = r0 + at;
-          const int row_s = rp[row], row_len = rp[row + 1] - row_s;
-          ta = row_s + part_begin(row_len, parts, part);
-          tb = row_s + part_begin(row_len, parts, part + 1);
-          slot_own = slot0 + part;
-          return true;
-        }
-        items += __builtin_amdgcn_readfirstlane(__shfl(upto, 63));
-        slots += __builtin_amdgcn_readfirstlane(__shfl(slots_upto, 63));
       }
       return false;
     };
     if (wg < nb) {
       ta = rp[wg]; tb = rp[wg + 1];
       if (ta == tb) { write_empty_row(wg); return; }
-      if (prm.W > 0 && is_long(tb - ta)) return;
+      if (prm.W > 0 && tb - ta > LONG_ROW_MIN) {
+        T = total();
+        if (is_long(tb - ta)) return;
+      }
     } else {
+      T = total();
       const int32_t* rpg = prm.row_ptr + (int64_t)mh * nb;
       int sum = 0, count = 0;
       for (int r = lane; r < nb; r += 64) {
@@ -1305,6 +1308,22 @@ static size_t parts_bytes(int B, int H, int nb, int W, int D, int mode) {
   return slots_bytes(B, H, W, D, mode) + (size_t)B * H * nb * sizeof(unsigned long long);
 }
 
+// ROWS_MODE: heads whose row blocks go out together, the longest first.  One per XCD keeps one head's K and V in an L2, but a
+// group's long row blocks then start when the short ones of the group before end, the last group's last of all; as many as
+// are at work at once anyway (their row blocks fill the wavefronts of an XCD) cost little locality, above 8 more (300 heads
+// N = 1024, keep 0.5, with 1 / 8 / 13: 72 / 73 / 78 us).  Groups of like size.
+// Block-causal, bf16, us with 1 / 2 / 3 / 4 / 6 / 8 / 16 heads per XCD and group, and the ranges of workgroups that this mode
+// replaced:       128 heads N = 2048 (8 at once)  118 / 115 / 116 /  98 / 105 /  94 /  94    99     256 heads  200 / 195 / 195 / 189 / 193 / 182 / 172   201
+//                  64 heads N = 4096 (4)          214 / 189 / 198 / 174 / 221 / 173 / 173   198      96 heads  286 / 276 / 259 / 265 / 251 / 272 / 246   294
+//                  48 heads N = 8192 (2)          537 / 509 / 491 / 526 / 463 / 462 / 461   573      24 heads  291 / 271 / 252 / 252 / 252 / 253 / 255   269
+//   keep 0.2:      48 heads N = 8192              221 / 222 / 227 / 226 / 256 / 256 / 257   279     keep 0.5, 256 heads N = 2048  184 / 183 / 186 / 184 / 187 / 186 / 205
+//   keep 0.05:     48 heads N = 17792 (1)         307 / 315 / 354 / 356 / 408 / 410 / 409   430
+static int rows_group(int B, int H, int nb) {
+  const int per_xcd = (B * H + 7) / 8, at_work = (wave_slots() / 8 + nb / 2) / nb;
+  const int most = at_work < 1 ? 1 : (at_work > 8 ? 8 : at_work), groups = (per_xcd + most - 1) / most;
+  return 8 * ((per_xcd + groups - 1) / groups);
+}
+
 static int long_row_groups(int B, int H, int nb, bool compact) {
   const int64_t W = wave_slots() / (compact ? 2 : 1) / ((int64_t)B * H);
   if (W < 8) return 0;
@@ -1474,6 +1493,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
   // after a pause 677 against 707.)
   prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
+  prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();
