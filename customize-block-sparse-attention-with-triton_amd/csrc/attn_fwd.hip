@@ -590,8 +590,7 @@ void fwd_kernel(const FwdParams prm) {
                            oacc[db][qb][4 * i4] * inv, oacc[db][qb][4 * i4 + 1] * inv,
                            oacc[db][qb][4 * i4 + 2] * inv, oacc[db][qb][4 * i4 + 3] * inv);
       if (prm.lse != nullptr && g == 0)
-        prm.lse[((int64_t)bh * prm.N) + qrow] =
-            lsum[qb] > 0.f ? (m_i[qb] + __builtin_amdgcn_logf(lsum[qb])) * 0.6931471805599453f : -INFINITY;
+        prm.lse[((int64_t)bh * prm.N) + qrow] = row_lse(m_i[qb], lsum[qb]);
     }
   };
   // row block without kept tiles: O = 0, lse = -inf
@@ -657,8 +656,7 @@ void fwd_kernel(const FwdParams prm) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
-      if (!(lsum[qb] > 0.f)) lsum[qb] = 0.f;
-      M[qb] = lsum[qb] > 0.f ? m_i[qb] : -INFINITY;
+      M[qb] = lsum[qb] == 0.f ? -INFINITY : m_i[qb];      // (a sum that is not a number stays in)
     }
     const int lane_p = fresh_lane(lane), ln = lane_p & 31, g = lane_p >> 5;
     unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + row;
@@ -1006,7 +1004,7 @@ void fwd_kernel(const FwdParams prm) {
         if (g == 0) {
 #pragma unroll
           for (int qb = 0; qb < 2; ++qb) {
-            const bool mass = mine && lsum[qb] > 0.f;
+            const bool mass = mine && lsum[qb] != 0.f;      // (a sum that is not a number stays in)
             ml[(w * 2 + 0) * 64 + qb * 32 + ln] = mass ? m_i[qb] : -INFINITY;
             ml[(w * 2 + 1) * 64 + qb * 32 + ln] = mass ? lsum[qb] : 0.f;
           }
@@ -1107,7 +1105,7 @@ void fwd_kernel(const FwdParams prm) {
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb)
               if (exists((int64_t)(r * 64 + qb * 32 + ln))) prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
-                  L[qb] > 0.f ? (M[qb] + __builtin_amdgcn_logf(L[qb])) * 0.6931471805599453f : -INFINITY;
+                  row_lse(M[qb], L[qb]);
           }
         } else {
           if (w == 0 && g == 0) {
@@ -1231,7 +1229,7 @@ void fwd_kernel(const FwdParams prm) {
 #pragma unroll
               for (int qb = 0; qb < 2; ++qb)
                 if (exists((int64_t)(r * 64 + qb * 32 + ln))) prm.lse[((int64_t)bh * prm.N) + (int64_t)(r * 64 + qb * 32 + ln)] =
-                    Ls[qb] > 0.f ? (Ms[qb] + __builtin_amdgcn_logf(Ls[qb])) * 0.6931471805599453f : -INFINITY;
+                    row_lse(Ms[qb], Ls[qb]);
             }
             // back to zero, so that a replay of this launch (same mark) starts from a clean counter
             if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -55,3 +55,13 @@ def check(dev, H, N, D, dtype, elementwise, what):
                                                (256, 2, 1024, False), (256, 2, 1000, True), (256, 100, 704, False)])
 def test_row_blocks_of_wavefront_pairs(dev, D, H, N, elementwise, dtype, what):
     check(dev, H, N, D, dtype, elementwise, what)
+
+
+# D = 64: ranges of workgroups (row blocks inside a range, and shared by several), ranges of wavefronts, a wavefront per
+# row block, long row blocks cut; D = 128: ranges of workgroups
+@pytest.mark.parametrize("what", ["key", "query", "inf"])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D,H,N,elementwise", [(64, 2, 704, False), (64, 1, 4096, False), (64, 2, 1000, True), (64, 66, 2000, False),
+                                               (64, 160, 1300, False), (128, 2, 1024, False), (128, 1, 2048, False)])
+def test_ranges_and_row_blocks(dev, D, H, N, elementwise, dtype, what):
+    check(dev, H, N, D, dtype, elementwise, what)
