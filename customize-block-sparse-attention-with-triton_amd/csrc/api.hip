@@ -23,6 +23,7 @@ const char* bsattn_strerror(int code) {
     case BSATTN_ERR_LAUNCH: return "HIP launch failed";
     case BSATTN_ERR_RANGE: return "size exceeds 32-bit index range";
     case BSATTN_ERR_STATIC_LIMIT: return "shape needs more scratch memory than the library's static buffer holds";
+    case BSATTN_ERR_ORDER: return "an earlier in-place reorder was given a permutation number outside the table (-6 .. 5): those heads were not moved";
     default: return "unknown error code";
   }
 }

@@ -12,6 +12,7 @@
 // head, and the last one to leave moves the head alone, a column of 4 bytes at a time.  The members of a group have
 // neighbouring places in the dispatch order of one XCD, so this happens only where the launch is confined to a few
 // compute units.  Heads whose order is the identity are left alone.
+#include <mutex>
 #include "common.h"
 
 namespace bsattn {
@@ -38,6 +39,7 @@ struct ReorderParams {
   int units, BS, NH, F, H, W, row_bytes;
   const int32_t* orders; const int32_t* inv_orders;      // out of place: [NH][3]
   const void* numbers; int number_bytes, inverse;         // in place: permutation number of every head (int32 or int64)
+  unsigned* bad_number;               // ... host memory: set to 1 for a number outside the table
   int vshift;                         // log2(pieces per row), -1 if that is not a power of two
   unsigned blocks_per_unit, rows_per_block;         // out of place
   unsigned parts, pieces_per_part;                  // in place
@@ -122,7 +124,11 @@ __global__ __launch_bounds__(GROUP_THREADS, 4) void reorder_group_kernel(const R
   const int per = prm.BS * prm.NH, ten = unit / per, bh = unit - ten * per, h = bh % prm.NH;
   long long number = prm.number_bytes == 8 ? ((const long long*)prm.numbers)[h] : ((const int*)prm.numbers)[h];
   if (number < 0) number += 6;
-  if (number <= 0 || number > 5) return;            // the identity (and numbers that stand for no order)
+  if (number < 0 || number > 5) {                   // no order: the head stays as it is, and the next call says so
+    if (part == 0 && threadIdx.x == 0) __hip_atomic_store(prm.bad_number, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    return;
+  }
+  if (number == 0) return;                          // the identity
   const Order order(prm, ORDERS[number], ORDERS_BACK[number], prm.inverse != 0);
   char* rows = prm.x[ten] + (bh / prm.NH) * prm.sb[ten] + h * prm.sh[ten];
   const int64_t xs = prm.st[ten];
@@ -247,6 +253,30 @@ size_t reorder_workspace_bytes(int n, int BS, int NH, int F, int Hh, int W, int 
   return (size_t)units * COUNTER_STRIDE * sizeof(unsigned long long);
 }
 
+// Where a device's kernels report a permutation number outside the table: a word of host memory per device, allocated by
+// the first call on it and kept (a call that is being captured may make that allocation too).
+struct BadNumber { unsigned* host; unsigned* device; };
+static int bad_number_word(BadNumber& w) {
+  static std::mutex mu;
+  static BadNumber words[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return BSATTN_ERR_LAUNCH;
+  std::lock_guard<std::mutex> lock(mu);
+  if (words[dev].host == nullptr) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return BSATTN_ERR_LAUNCH;
+    void *host = nullptr, *device = nullptr;
+    const bool ok = hipHostMalloc(&host, sizeof(unsigned), hipHostMallocMapped) == hipSuccess &&
+                    hipHostGetDevicePointer(&device, host, 0) == hipSuccess;
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (!ok) return BSATTN_ERR_LAUNCH;
+    *(unsigned*)host = 0;
+    words[dev] = {(unsigned*)host, (unsigned*)device};
+  }
+  w = words[dev];
+  return BSATTN_OK;
+}
+
 int launch_reorder_inplace(void* const* x, const int64_t* strides, int n, int BS, int NH, int F, int Hh, int W,
                            int row_bytes, const void* numbers, int number_bytes, int inverse, void* ws, hipStream_t st) {
   ReorderParams prm = {};
@@ -257,6 +287,10 @@ int launch_reorder_inplace(void* const* x, const int64_t* strides, int n, int BS
   prm.units = n * BS * NH;
   prm.BS = BS; prm.NH = NH; prm.F = F; prm.H = Hh; prm.W = W; prm.row_bytes = row_bytes;
   prm.numbers = numbers; prm.number_bytes = number_bytes; prm.inverse = inverse;
+  BadNumber bad;
+  if (const int rc = bad_number_word(bad); rc != BSATTN_OK) return rc;
+  if (__atomic_load_n(bad.host, __ATOMIC_RELAXED) != 0 && __atomic_exchange_n(bad.host, 0u, __ATOMIC_RELAXED) != 0) return BSATTN_ERR_ORDER;
+  prm.bad_number = bad.device;
   prm.counters = (unsigned long long*)ws;
   do { prm.mark = next_epoch() & 0xffffffffffull; } while (prm.mark == 0);
   pieces_of_row(prm, 16);

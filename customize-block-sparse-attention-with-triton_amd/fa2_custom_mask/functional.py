@@ -3,6 +3,7 @@ reference (same names, arguments, defaults and in-place write-back); the rows ar
 bsattn_reorder and bsattn_reorder_inplace."""
 import ctypes
 
+import numpy as np
 import torch
 
 from . import _ext
@@ -53,9 +54,21 @@ def _table(device):
     return _tables[device]
 
 
+def _check_numbers(idx):
+    """Permutation numbers that the host can read are checked before anything is moved.  Those in GPU memory are checked by
+    the kernel, and the next reorder on the device raises (reading them here would wait for the GPU in every call)."""
+    if isinstance(idx, torch.Tensor) and idx.is_cuda or not isinstance(idx, (torch.Tensor, np.ndarray, list, tuple)):
+        return
+    numbers = torch.as_tensor(idx)
+    if numbers.dtype in (torch.int64, torch.int32, torch.int16, torch.int8) and numbers.numel() and (
+            int(numbers.min()) < -len(_PERMUTATIONS) or int(numbers.max()) >= len(_PERMUTATIONS)):
+        raise IndexError("permutation numbers %s: the table has %d rows" % (numbers.tolist(), len(_PERMUTATIONS)))
+
+
 def _reorder_image_tokens(tensors, idx, inverse, F, H, W, n_text_tokens):
     """Reorders (inverse: brings back) the image tokens of every tensor where they are, head by head, by the
     permutation numbers idx [heads]."""
+    _check_numbers(idx)
     x = tensors[0]
     image = [t[:, :, n_text_tokens:, :] for t in tensors]                     # functional.py:31-33, 81
     BS, NH, T, D = image[0].shape

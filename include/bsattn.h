@@ -42,6 +42,8 @@ extern "C" {
 #define BSATTN_ERR_RANGE (-8)      /* a size exceeds what 32-bit indices can address */
 #define BSATTN_ERR_STATIC_LIMIT (-9) /* bsattn_fwd_static: the shape needs more scratch memory than
                                         BSATTN_STATIC_SCRATCH_BYTES */
+#define BSATTN_ERR_ORDER (-10)     /* an earlier bsattn_reorder_inplace on this device was given a
+                                      permutation number outside the table */
 
 /* dtype codes */
 #define BSATTN_F16 0
@@ -54,7 +56,7 @@ extern "C" {
  *   100: first layout.
  *   200: bsattn_bwd and bsattn_bwd_elementwise take dq_strides, dk_strides, dv_strides after
  *        do_strides; the entry points of the forward over quads of row blocks are gone. */
-#define BSATTN_ABI_VERSION 201
+#define BSATTN_ABI_VERSION 202
 int bsattn_version(void);
 /* Process-wide switch (default off), returns the previous setting.  On: the forward's result
  * depends on nothing but its inputs and the device (two runs give the same bits).  Off: the
@@ -339,7 +341,9 @@ int bsattn_reorder(const void* x, void* out, int BS, int NH, int F, int Hh, int 
  * x[i]: first image token of tensor i; strides[3 i ..]: its batch, head and token strides in elements (innermost
  * stride 1; rows, strides and addresses multiples of 16 bytes); the tensors must not overlap.  numbers: device memory,
  * NH integers of number_bytes (4 or 8), the row of the permutation table (functional.py:23-26) each head takes, negative
- * ones counted from its end (a head with a number outside the table is left alone); inverse != 0: the orders back (:69-76).
+ * ones counted from its end; inverse != 0: the orders back (:69-76).  The numbers are not read by the host: a head with a
+ * number outside the table (-6 .. 5) is left as it is, and the next call on the device once that kernel has run returns
+ * BSATTN_ERR_ORDER, enqueues nothing, and clears the condition.
  * A head may have up to 57344 rows and 7 MB; the workspace query returns BSATTN_ERR_RANGE for larger ones.  The
  * workspace (16-byte aligned) needs no particular contents on entry.
  * The workgroups that hold the rows of a head wait for each other, each for a limited time only: where they do not get

@@ -96,3 +96,33 @@ def test_group_that_cannot_run_together(dev):
         hip.hipStreamDestroy(handle)
     assert torch.equal(xd.cpu(), x)
     assert np.array_equal(back.cpu().view(torch.int16).numpy(), reference(x, numbers, F, H, W, text, inverse=True))
+
+
+@pytest.mark.parametrize("number_type", [torch.int64, torch.int32])
+@pytest.mark.parametrize("bad", [6, 100, -7])
+def test_number_outside_the_table(dev, bad, number_type):
+    """Numbers the host can read are refused before anything is moved; numbers in GPU memory are checked by the kernel:
+    the head stays as it is and the next reorder raises, once."""
+    import fa2_custom_mask as fm
+    F, H, W, D, text = 5, 12, 17, 64, 3
+    numbers = [3, bad, 1]
+    size = dict(F=F, H=H, W=W, n_text_tokens=text)
+    g = torch.Generator().manual_seed(13)
+    x = torch.randn(1, 3, text + F * H * W, D, generator=g).half()
+    for host_numbers in (numbers, torch.tensor(numbers, dtype=number_type), np.array(numbers)):
+        xd = x.to(dev)
+        with pytest.raises(IndexError):
+            fm.inv_permute_attn_triton(xd, {"permute": [host_numbers]}, 0, **size)
+        assert torch.equal(xd.cpu(), x)
+    plan = {"permute": [torch.tensor(numbers, dtype=number_type, device=dev)]}
+    good = {"permute": [torch.tensor([3, 0, 1], dtype=number_type, device=dev)]}
+    moved = x.to(dev)
+    fm.permute_qkv_triton(moved, moved.clone(), moved.clone(), plan, 0, **size)
+    torch.cuda.synchronize()
+    assert np.array_equal(moved.cpu().view(torch.int16).numpy(), reference(x, [3, 0, 1], F, H, W, text))
+    xd = x.to(dev)
+    with pytest.raises(RuntimeError, match="permutation number"):
+        fm.permute_qkv_triton(xd, xd.clone(), xd.clone(), good, 0, **size)
+    assert torch.equal(xd.cpu(), x)                          # nothing was enqueued
+    fm.permute_qkv_triton(xd, xd.clone(), xd.clone(), good, 0, **size)
+    assert torch.equal(xd.cpu(), moved.cpu())
