@@ -5,6 +5,7 @@
 //
 // Mirrors fa2_custom_mask/fa2_custom_mask.py:15-155 of the reference (build_groups_from_block_mask's lists, _attention).
 #include <torch/extension.h>
+#include <torch/csrc/Exceptions.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <dlfcn.h>
@@ -25,6 +26,7 @@ struct Library {
   decltype(&::bsattn_strerror) strerror_ = nullptr;
   decltype(&::bsattn_mask_lists_workspace) lists_workspace = nullptr;
   decltype(&::bsattn_block_mask_to_lists) lists = nullptr;
+  decltype(&::bsattn_gather_mask_tiles) gather = nullptr;
   decltype(&::bsattn_fwd_workspace) fwd_workspace = nullptr;
   decltype(&::bsattn_fwd_tokens) fwd = nullptr;
   decltype(&::bsattn_fwd_block_mask_workspace) fwd_block_mask_workspace = nullptr;
@@ -43,6 +45,7 @@ void bind(const std::string& path) {
   get(lib.strerror_, "bsattn_strerror");
   get(lib.lists_workspace, "bsattn_mask_lists_workspace");
   get(lib.lists, "bsattn_block_mask_to_lists");
+  get(lib.gather, "bsattn_gather_mask_tiles");
   get(lib.fwd_workspace, "bsattn_fwd_workspace");
   get(lib.fwd, "bsattn_fwd_tokens");
   get(lib.fwd_block_mask_workspace, "bsattn_fwd_block_mask_workspace");
@@ -299,18 +302,67 @@ py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v
 }
 
 // ---- autograd ----
-// forward(q, k, v, mask, sm_scale) and backward of the reference's _attention (:43-155) for a mask given by its lists;
+// The column lists of an elementwise mask, which only a backward walks and which hold as many words as the row lists, are
+// made by the first backward that needs them: a forward may have none.  While the words by grid position are in Python's
+// cache (held weakly here) without the GIL and before the cache of lists is told, so that the GPU does not wait for it
+// (a training step with a new mask, 8 heads N = 4000: 300 us, through Python 375, made in the forward 284).
+struct Grid : torch::CustomClassHolder {       // of an elementwise mask: block mask, "partly set" flags, words
+  using Weak = c10::weak_intrusive_ptr<c10::TensorImpl, c10::UndefinedTensorImpl>;
+  Weak block, partial, bits;
+  Grid(const Tensor& a, const Tensor& b, const Tensor& c) : block(a.getIntrusivePtr()), partial(b.getIntrusivePtr()), bits(c.getIntrusivePtr()) {}
+};
+
+struct PythonLists { py::object make, keep; };                     // mask_to_lists of the column lists, their cache
+PythonLists* python_lists = nullptr;                               // (set once, never destroyed)
+
+template <typename F>
+auto in_python(F&& f) {
+  py::gil_scoped_acquire gil;
+  TORCH_CHECK(python_lists != nullptr, "the host path has not been given Python's list functions");
+  try {
+    return f();
+  } catch (py::error_already_set& e) {       // as autograd hands Python errors on
+    e.restore();
+    python_error err;
+    err.persist();
+    throw std::move(err);
+  }
+}
+
+// fresh: Python's cache does not know them yet
+ListsPtr column_lists(const Tensor& mask, int64_t N, const c10::intrusive_ptr<Grid>& grid, bool& fresh) {
+  if (grid) {
+    const auto block = grid->block.lock(), partial = grid->partial.lock(), bits = grid->bits.lock();
+    if (block.defined() && partial.defined() && bits.defined()) {
+      const Tensor grid_block{block}, grid_partial{partial}, grid_bits{bits};
+      ListsPtr lists = block_mask_to_lists(grid_block, true, false);
+      lists->partial = at::empty_like(grid_partial);
+      lists->bits = at::empty_like(grid_bits);
+      check(lib.gather((const uint8_t*)grid_partial.const_data_ptr(), (const uint64_t*)grid_bits.const_data_ptr(), (int)lists->Bm, (int)lists->Hm,
+                       (int)lists->nb, 1, lists->row_ptr(), lists->col_idx(), (uint8_t*)lists->partial.data_ptr(),
+                       (uint64_t*)lists->bits.data_ptr(), stream_of(mask)), "bsattn_gather_mask_tiles");
+      fresh = true;
+      return lists;
+    }
+  }
+  return in_python([&] { return py::cast<ListsPtr>(python_lists->make(mask, N)); });
+}
+
+// forward(q, k, v, mask, sm_scale) and backward of the reference's _attention (:43-155) for a mask given by its row lists
+// (and its column lists, where they are at hand);
 // two further arguments select an fp32 output and the LSE as second result.  Autograd hands gradients back in the type
 // of q, k, v.
 struct Attention : torch::autograd::Function<Attention> {
   static variable_list forward(AutogradContext* ctx, const Variable& q_, const Variable& k_, const Variable& v_, const Variable& mask,
-                               const ListsPtr& lists, const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
+                               const ListsPtr& lists, const ListsPtr& lists_t, const c10::intrusive_ptr<Grid>& grid, double sm_scale,
+                               bool out_fp32, bool return_lse) {
     const Tensor q = padded(q_), k = padded(k_), v = padded(v_);
     auto [o, lse] = forward_core(q, k, v, *lists, sm_scale, result_type(q, out_fp32), true);
     const Tensor out = unpadded(o, q_.size(3));
     ctx->save_for_backward({q, k, v, out, lse, mask});                   // :89 (a mask written to before the backward is refused)
     ctx->saved_data["lists"] = c10::IValue::make_capsule(lists);
-    ctx->saved_data["lists_t"] = c10::IValue::make_capsule(lists_t);
+    if (lists_t) ctx->saved_data["lists_t"] = c10::IValue::make_capsule(lists_t);
+    else if (grid) ctx->saved_data["grid"] = c10::IValue::make_capsule(grid);
     ctx->saved_data["sm_scale"] = sm_scale;
     if (!return_lse) return {out};                                       // :94
     ctx->mark_non_differentiable({lse});
@@ -326,17 +378,29 @@ struct Attention : torch::autograd::Function<Attention> {
     const Tensor o = padded(out.scalar_type() == t ? out : out.to(t));
     const Tensor g = grads[0].defined() ? padded(grads[0].scalar_type() == t ? grads[0] : grads[0].to(t)) : at::zeros_like(o);
     const auto lists = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists"].toCapsule());
-    const auto lists_t = c10::static_intrusive_pointer_cast<TileLists>(ctx->saved_data["lists_t"].toCapsule());
+    const Tensor& mask = saved[5];
+    ListsPtr lists_t;
+    bool fresh = false;
+    if (const auto at_hand = ctx->saved_data.find("lists_t"); at_hand != ctx->saved_data.end()) {
+      lists_t = c10::static_intrusive_pointer_cast<TileLists>(at_hand->second.toCapsule());
+    } else {
+      const auto grid = ctx->saved_data.find("grid");
+      lists_t = column_lists(mask, q.size(2), grid == ctx->saved_data.end() ? nullptr : c10::static_intrusive_pointer_cast<Grid>(grid->second.toCapsule()), fresh);
+    }
     auto [dq, dk, dv] = backward_core(q, k, v, o, g, lse, *lists, *lists_t, ctx->saved_data["sm_scale"].toDouble(), t);
-    return {unpadded(dq, D), unpadded(dk, D), unpadded(dv, D), Variable(), Variable(), Variable(), Variable(), Variable(), Variable()};   // :155
+    if (fresh) in_python([&] { python_lists->keep(mask, q.size(2), true, lists_t); });
+    return {unpadded(dq, D), unpadded(dk, D), unpadded(dv, D), Variable(), Variable(), Variable(), Variable(), Variable(), Variable(), Variable()};   // :155
   }
 };
 
 py::object attention(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& mask, const ListsPtr& lists,
-                     const ListsPtr& lists_t, double sm_scale, bool out_fp32, bool return_lse) {
+                     const ListsPtr& lists_t, const std::optional<std::tuple<Tensor, Tensor, Tensor>>& grid, double sm_scale, bool out_fp32,
+                     bool return_lse) {
   check_qkv(q, k, v);
   check_mask_heads(lists->Bm, lists->Hm, q);
-  variable_list r = Attention::apply(q, k, v, mask, lists, lists_t, sm_scale, out_fp32, return_lse);
+  c10::intrusive_ptr<Grid> weak;
+  if (grid) weak = c10::make_intrusive<Grid>(std::get<0>(*grid), std::get<1>(*grid), std::get<2>(*grid));
+  variable_list r = Attention::apply(q, k, v, mask, lists, lists_t, weak, sm_scale, out_fp32, return_lse);
   if (return_lse) return py::make_tuple(r[0], r[1]);
   return py::cast(r[0]);
 }
@@ -372,7 +436,9 @@ PYBIND11_MODULE(_host, m) {
   m.def("block_mask_to_lists", &block_mask_to_lists);
   m.def("forward", &forward);
   m.def("forward_block_mask", &forward_block_mask);
-  m.def("attention", &attention);
+  m.def("attention", &attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("lists"),
+        py::arg("lists_t").none(true), py::arg("grid"), py::arg("sm_scale"), py::arg("out_fp32"), py::arg("return_lse"));
+  m.def("set_python_lists", [](py::object make, py::object keep) { python_lists = new PythonLists{std::move(make), std::move(keep)}; });
   m.def("forward_backward", &forward_backward);
   py::class_<TileLists, ListsPtr>(m, "TileLists")
       .def(py::init([](int64_t Bm, int64_t Hm, int64_t nb, py::object device, bool want_groups) {

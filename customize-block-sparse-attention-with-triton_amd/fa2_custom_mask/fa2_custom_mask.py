@@ -9,7 +9,7 @@ import ctypes
 import torch
 
 from . import _ext
-from .utils import TILE, _host, block_mask_to_lists, lists_cache, mask_to_lists, num_tiles, is_block_form, _check_mask
+from .utils import TILE, _host, block_mask_to_lists, lists_cache, grid_cache, mask_to_lists, num_tiles, is_block_form, _check_mask
 
 
 def build_groups_from_block_mask(mask):
@@ -155,10 +155,18 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
     mask, N = _mask_of(q, k, v, mask)
     lists = lists_cache.get(mask, N, False)
     if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
-        # (the backward walks the column lists: both orientations are made here)
         if lists is None:
             lists = mask_to_lists(mask, N, both=True)                        # :48
-        return _host.attention(q, k, v, mask, lists, mask_to_lists(mask, N, transpose=True), sm_scale, out_fp32, return_lse)
+        # The backward walks the column lists.  A block mask's are made here, where the GPU does not wait for them; those of
+        # an elementwise mask, with a second set of its words, by the backward, which may never come.
+        grid = None
+        if lists.bits is None:
+            lists_t = mask_to_lists(mask, N, transpose=True)
+        else:
+            lists_t = lists_cache.get(mask, N, True)
+            if lists_t is None:
+                grid = grid_cache.get(mask, N)
+        return _host.attention(q, k, v, mask, lists, lists_t, grid, sm_scale, out_fp32, return_lse)
     if lists is None:
         _check_mask(mask)
         if is_block_form(mask, N):
@@ -168,6 +176,9 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
             return result
         lists = mask_to_lists(mask, N)
     return _host.forward(q, k, v, lists, sm_scale, out_fp32, return_lse)
+
+
+_host.set_python_lists(lambda mask, N: mask_to_lists(mask, N, transpose=True), lists_cache.put)
 
 
 class _attention:

@@ -104,6 +104,43 @@ def test_reorder_beside_training_on_one_stream(dev, deterministic):
         assert all(torch.equal(a, b) for a, b in zip(run, alone))
 
 
+@pytest.mark.parametrize("elementwise", [False, True])
+def test_column_lists(dev, deterministic, elementwise):
+    """A forward with an elementwise mask that is never followed by a backward makes row lists only; the first backward
+    makes the column lists, on whatever thread and stream it runs, and the next forward with the mask finds them."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask.utils import lists_cache
+    q, k, v, do = [x.to(dev) for x in make_qkv(1, 2, 200, 64, torch.float16, 760, n=4)]
+    for x in (q, k, v):
+        x.requires_grad_(True)
+    mask = uniform_block_mask(1, 1, 4, 0.6, 761).to(dev)
+    if elementwise:
+        mask = mask.repeat_interleave(64, 2).repeat_interleave(64, 3)[:, :, :200, :200].tril().contiguous()
+    o = fm.flash_attention_custom_mask(q, k, v, mask, 0.2)
+    assert lists_cache.get(mask, 200, False) is not None and (lists_cache.get(mask, 200, True) is None) == elementwise
+    got = []
+    thread = threading.Thread(target=lambda: got.extend(torch.autograd.grad(o, (q, k, v), do, retain_graph=True)))
+    thread.start()
+    thread.join()
+    assert lists_cache.get(mask, 200, True) is not None
+    side = torch.cuda.Stream(dev)
+    side.wait_stream(torch.cuda.current_stream(dev))
+    fresh = mask.clone()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        o2 = fm.flash_attention_custom_mask(q, k, v, fresh, 0.2)
+    again = torch.autograd.grad(o2, (q, k, v), do)                        # lists made on the side stream
+    at_hand = torch.autograd.grad(fm.flash_attention_custom_mask(q, k, v, mask, 0.2), (q, k, v), do)
+    torch.cuda.synchronize()
+    lists_cache.clear()
+    rebuilt = torch.autograd.grad(o, (q, k, v), do)
+    torch.cuda.synchronize()
+    o_ref, _, *ref = fm.attention_forward_backward(q.detach(), k.detach(), v.detach(), mask, 0.2, do)
+    assert torch.equal(o.detach(), o_ref)
+    for grads in (got, again, at_hand, rebuilt):
+        assert all(torch.equal(a, b) for a, b in zip(grads, ref))
+
+
 def test_mask_written_before_the_backward_is_refused(dev):
     import fa2_custom_mask as fm
     q, k, v = [x.to(dev).requires_grad_(True) for x in make_qkv(1, 1, 128, 64, torch.float16, 740)]
