@@ -205,8 +205,9 @@ class _ListsCache:
         return lists
 
     def put(self, mask, N, transpose, lists):
+        # (lists made while a graph is being captured are filled by its replays only, in memory that is the graph's)
         version = self._version(mask)
-        if version is None:
+        if version is None or torch.cuda.is_current_stream_capturing():
             return
         key = (id(mask), N, transpose)
         self._entries.pop(key, None)
@@ -250,7 +251,7 @@ class _GridCache:
 
     def put(self, mask, N, grid):
         version = _ListsCache._version(mask)
-        if version is None:
+        if version is None or torch.cuda.is_current_stream_capturing():
             return
         stream = torch.cuda.current_stream(mask.device)
         ready = torch.cuda.Event()

@@ -100,3 +100,32 @@ def test_replay_mask_to_lists(dev):
         assert G == len(g_ref) and T == len(n_ref)
         assert np.array_equal(lists.groups[:G].cpu().numpy(), g_ref)
         assert np.array_equal(lists.col_idx[:T].cpu().numpy(), n_ref)
+
+
+@pytest.mark.parametrize("elementwise", [False, True])
+def test_lists_made_under_capture_are_the_graphs(dev, elementwise):
+    """A mask that is first seen while a graph is being captured: its lists are made by the replays, also of what is written
+    to the mask between them, and no eager call takes them for its own."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask.utils import lists_cache, grid_cache
+    N = 640
+    q, k, v = [x.to(dev) for x in make_qkv(1, 2, N, 64, torch.float16, 81)]
+    masks = [uniform_block_mask(1, 1, 10, 0.4, 82 + i).to(dev) for i in range(4)]
+    if elementwise:
+        masks = [m.repeat_interleave(64, 2).repeat_interleave(64, 3).tril().contiguous() for m in masks]
+    call = lambda mask: fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+    eager = [call(m.clone()) for m in masks]
+    mask = masks[0].clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = call(mask)
+    assert lists_cache.get(mask, N, False) is None and grid_cache.get(mask, N) is None
+    assert same_up_to_rounding(call(mask), eager[0])                 # no replay has filled the graph's lists yet
+    for i in (0, 1, 2, 3, 1):
+        mask.copy_(masks[i])
+        captured.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same_up_to_rounding(captured, eager[i]), i
+        assert same_up_to_rounding(call(mask), eager[i]), i
