@@ -692,7 +692,7 @@ void fwd_kernel(const FwdParams prm) {
     if (__builtin_amdgcn_readfirstlane(counted_v) != nparts) return;
     float Ms[2] = {-INFINITY, -INFINITY}, Ls[2] = {0.f, 0.f};
     reset_acc();
-    for (int p = 0; p < nparts; ++p) {
+    for (int p = first; p < first + nparts; ++p) {
       const float* sp = slot_of(p, first);
       float sc_own[2], sc_p[2];
 #pragma unroll
@@ -808,7 +808,7 @@ void fwd_kernel(const FwdParams prm) {
       } else {
         auto slot_at = [&](int i) { return prm.ws + ((int64_t)bh * prm.W + i) * partial_floats(D); };
         share_row(row, slot_at(slot_own), [&](int& first, int& count) { first = slot0; count = parts; },
-                  [&](int i, int first) { return slot_at(first + i); });
+                  [&](int p, int) { return slot_at(p); });
       }
       if (wg < nb) return;
       item += prm.W;
@@ -871,7 +871,7 @@ void fwd_kernel(const FwdParams prm) {
           while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
           first = pf_;
           count = pl_ - pf_ + 1;
-        }, [&](int i, int first) { return wg_slot(first + i, i == 0); });
+        }, [&](int p, int first) { return wg_slot(p, p == first); });
       }
       t = seg_b;
       ++r;
