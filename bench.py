@@ -211,8 +211,8 @@ def elementwise_case(torch, dev, fm, q, k, v, sm_scale):
     mask = torch.ones(N, N, dtype=torch.bool, device=dev).tril_().reshape(1, 1, N, N)
     lists = utils.mask_to_lists(mask, N)
     tiles = int(lists.counts[1])
-    o, _ = fm.fa2_custom_mask._forward(q, k, v, lists, sm_scale, torch.float16, True)
-    tf = event_times(lambda: fm.fa2_custom_mask._forward(q, k, v, lists, sm_scale, torch.float16, False), 20, 3, torch)
+    o = fm.flash_attention_custom_mask(q, k, v, mask, sm_scale)          # (the lists are cached)
+    tf = event_times(lambda: fm.flash_attention_custom_mask(q, k, v, mask, sm_scale), 20, 3, torch)
 
     def prep():
         utils.lists_cache.clear()
@@ -453,7 +453,7 @@ def main():
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_F16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_F16_TFLOPS, 4), "traffic": measured_traffic(),
                      "ms_per_launch": round(dense_avg_ms, 5), "ms_single_launch_between_events": sweep["1.0"]["ms_avg"],
-                     "kernel": "fwd_kernel<64, 0, false, false, true> (fp16, contiguous rows, one bsattn_fwd call)",
+                     "kernel": "fwd_kernel<64, 0, 0, false, 1> (fp16, ranges of workgroups, block mask, contiguous rows; one bsattn_fwd call)",
                      "algorithmic_flops_per_launch": tile_flops(kept[1.0])},
     }
     if not args.no_cpu:

@@ -11,8 +11,8 @@
 // range is normalised and written straight to O.  A row block cut by range boundaries is
 // finished by the workgroup that holds its first tiles: the others publish unnormalised parts
 // in the workspace (device-scope stores, then a flag), and it pulls them when it gets there.
-// With many row blocks per workgroup (many heads) each wavefront takes whole row blocks
-// instead, and nothing is merged.
+// That is the way of launches with few row blocks (COOP).  At D = 64, with about as many as wavefronts fit the GPU, a range
+// belongs to a single wavefront (WAVE); with more a wavefront takes a whole row block, or a part of a long one (ROWS).
 //
 // Per tile a wavefront computes S^T = K Q^T (keys along MFMA rows, queries along lanes), so
 // that one lane owns one query: softmax statistics are in-lane reductions plus a single
@@ -63,7 +63,8 @@ template <int D> struct FwdCfg {
 
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
 // MODE.  COOP: the ranges of four-wavefront workgroups described above (launches with few row blocks).  ROWS: a workgroup
-// is one wavefront and takes one row block (many row blocks: nothing to merge, the dispatcher balances the load).
+// is one wavefront and takes one row block, or parts of long ones (many row blocks: next to nothing to merge, the
+// dispatcher balances the load).
 // WAVE: a workgroup is one wavefront and takes one range of its head's list (in between: about as many row blocks as
 // wavefronts fit the GPU, which whole row blocks would leave half idle in a second round).
 // LAYOUT: GENERAL any strides, any number of tokens; CONTIG_WHOLE the rows of K and of V follow each other without gaps
@@ -1392,8 +1393,6 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
 size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_bytes(B, H, N, D); }
 
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
-// D = 64.  With few row blocks the wavefronts of a workgroup share one row block at a time (K and V tiles are spread
-// over them and the results merged); with many a wavefront takes a whole row block, which needs no merge.
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
 static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;

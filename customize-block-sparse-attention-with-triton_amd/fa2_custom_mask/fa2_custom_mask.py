@@ -73,12 +73,6 @@ def set_deterministic(on):
     return bool(_ext.lib().bsattn_set_deterministic(1 if on else 0))
 
 
-def _forward(q, k, v, lists, sm_scale, out_dtype, want_lse):
-    """(o, lse or None) for lists that are at hand."""
-    r = _host.forward(q, k, v, lists, sm_scale, out_dtype == torch.float32, want_lse)
-    return r if want_lse else (r, None)
-
-
 class ForwardPlan:
     """A forward call with every buffer allocated and every C argument marshalled once; run()
     only enqueues the kernels.  For loops that repeat the same shapes (serving, benchmarks)."""
