@@ -196,14 +196,20 @@ __device__ __forceinline__ bool walked_by_first(cint_ptr_t lp, int whole) {
 }
 
 // Entries [u0, u1) of a list [t0, t0 + len) are share `chunk` of it.  Returns the number of its shares (1: chunk is 0).
+// BY_LENGTH: short lists may be one workgroup's (only in the kernels that are launched so, bwd_shares: the look at the
+// length costs 0.3 us of a launch).
+template <bool BY_LENGTH>
 __device__ __forceinline__ int share_of_list(const BwdParams& prm, int t0, int len, int chunk, int& u0, int& u1) {
-  u0 = t0;
-  u1 = t0 + len;
-  if (len <= prm.whole || prm.split == 1) return 1;
+  if constexpr (BY_LENGTH) {
+    u0 = t0;
+    u1 = t0 + len;
+    if (len <= prm.whole || prm.split == 1) return 1;
+  }
   u0 = t0 + (int)((int64_t)len * chunk / prm.split);
   u1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
   return prm.split;
 }
+template <int D, bool EW> constexpr bool by_length = D == 128 && !EW;
 
 // ---------------------------------------------------------------------------------------
 // dQ: workgroup = row block m, wavefront wv owns queries 64m + 32wv + ln
@@ -235,7 +241,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
-  if (chunk > 0 && walked_by_first(rp + m, prm.whole)) return;
+  if (by_length<D, EW> && chunk > 0 && walked_by_first(rp + m, prm.whole)) return;
   // The rows this workgroup owns for its whole walk (Q, dO, O, lse of its queries) depend on the block index only:
   // they are asked for first, and travel while the list is looked up and the first tiles are requested.
   const int64_t qrow = (int64_t)m * 64 + 32 * wv + ln;
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   int u0, u1, split;                                           // steps: tile u / STEPS, part u % STEPS
   {
     const int t0 = rp[m], len = rp[m + 1] - t0;                // this workgroup's share of the row's list
-    split = share_of_list(prm, t0, len, chunk, u0, u1);
+    split = share_of_list<by_length<D, EW>>(prm, t0, len, chunk, u0, u1);
     u0 *= STEPS;
     u1 *= STEPS;
   }
@@ -419,11 +425,11 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
-  if (chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
+  if (by_length<D, EW> && chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
   int u0, u1, split;                                           // steps: tile u / STEPS, part u % STEPS
   {
     const int t0 = cp[n], len = cp[n + 1] - t0;                // this workgroup's share of the column's list
-    split = share_of_list(prm, t0, len, chunk, u0, u1);
+    split = share_of_list<by_length<D, EW>>(prm, t0, len, chunk, u0, u1);
     u0 *= STEPS;
     u1 *= STEPS;
   }
@@ -672,7 +678,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
-  if (chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
+  if (by_length<D, EW> && chunk > 0 && walked_by_first(cp + n, prm.whole)) return;
   // The K and V rows this wavefront owns for the whole walk depend on the block index only: asked for first, they
   // travel while the list is looked up and the first tiles are requested.
   const int64_t krow = (int64_t)n * 64 + 32 * kh + ln;
@@ -690,7 +696,7 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
   int u0, u1, split;
   {
     const int t0 = cp[n], len = cp[n + 1] - t0;                // this workgroup's share of the column's list
-    split = share_of_list(prm, t0, len, chunk, u0, u1);
+    split = share_of_list<by_length<D, EW>>(prm, t0, len, chunk, u0, u1);
   }
   const unsigned lds_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
   const unsigned short* qg = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1];
