@@ -18,6 +18,7 @@
 // double buffer (one barrier per tile).
 #include "common.h"
 #include "kernel_util.h"
+#include "place.h"
 #include <type_traits>
 
 namespace bsattn {
@@ -177,15 +178,13 @@ __device__ __forceinline__ floatx16 zero16() {
 __device__ __forceinline__ void settle(uintx4& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void settle(float& x) { asm volatile("" : "+v"(x)); }
 
-// Workgroup -> (head, block) for the walking kernels.  Workgroups go to the 8 XCDs round-robin by
-// linear id, and each XCD has its own L2: heads are taken in groups of 8, head i of a group on
-// XCD i, so that the tiles a head's workgroups walk over (K and V, or Q and dO, of that head) are
-// shared in one L2 instead of being fetched into all of them.
+// Workgroup -> (head, block) for the walking kernels: heads in groups of 8, one head per XCD (place.h), so that the tiles a
+// head's workgroups walk over (K and V, or Q and dO, of that head) are shared in one L2 instead of being fetched into
+// all of them.
 __device__ __forceinline__ void head_and_block(int L, int BH, int nb, int& bh, int& blk) {
-  const int grp = L / (8 * nb), l = L - grp * 8 * nb;
-  const int hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;     // heads in this group
-  bh = 8 * grp + l % hg;
-  blk = l / hg;          // >= nb for the padding of an incomplete last group
+  const Place p = place(L, BH, XCDS, nb);
+  bh = p.head;
+  blk = p.item;          // >= nb for the padding of an incomplete last group
 }
 
 // Is the list at lp, lp + 1 so short that the first share's workgroup walks all of it?  (The pointer as a value the
@@ -1022,7 +1021,7 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
     }
   });
   const int BH = prm.B * prm.H;
-  const int grid = ((BH + 7) / 8) * 8 * prm.nb * prm.split;   // heads in groups of 8, the last group padded
+  const int grid = placed(BH, XCDS, prm.nb) * prm.split;   // heads in groups of 8, the last group padded
   hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
   if constexpr (D == 64) hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);

@@ -23,6 +23,7 @@
 // statistics, P rounded to 16 bits for the second product), with two changes that keep the
 // vector ALU out of the way of the matrix cores: the softmax scale is folded into Q, and the
 // running maximum is replaced by a reference exponent that is only moved when needed.
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <map>
@@ -33,6 +34,7 @@
 #include "fwd_split.h"
 #include "fwd_tile.h"
 #include "kernel_util.h"
+#include "place.h"
 #include "range_perm.h"
 #include "row_parts.h"
 
@@ -75,8 +77,6 @@ template <int D> struct FwdCfg {
 // row block beyond N repeat the last query and are not written.
 enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2, STRIDED_WHOLE = 3 };
 enum { COOP = 0, ROWS_MODE = 1, WAVE = 2 };
-// ROWS: workgroups for long row blocks in a launch; a multiple of 8, so that those behind them keep their XCD
-__host__ __device__ constexpr int rows_extras(int BH, int W) { return (BH * W + 7) & ~7; }
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
 __global__ __launch_bounds__(MODE != COOP ? 64 : FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
 void fwd_kernel(const FwdParams prm) {
@@ -95,25 +95,30 @@ void fwd_kernel(const FwdParams prm) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
-  // linear id -> (head, range): heads interleaved, so that every head gets its share of the
-  // workgroups that are first on their compute unit
+  // linear id -> (head, range): every head gets its share of the workgroups that are first on their compute unit, and an
+  // XCD as few heads as possible (place_range; 1, 2, 4 or 8 heads are interleaved, which is the same and what the range
+  // permutations below are made for)
   const int BH = prm.B * prm.H, nb = prm.nb;
   int bh, wg;
   if constexpr (ROWS) {
-    // (head, row block): heads in groups of `group`, a multiple of 8, spread over the XCDs (workgroups go to them
-    // round-robin), so that the row blocks at work on an XCD share the K and V of few heads in its L2 (rows_group); in a
-    // group the last row blocks of all heads, the long ones of block-causal masks, first.  Behind the first `first_ids`
-    // of them, which fill the GPU, W workgroups per head for the long row blocks (wg >= nb; see below).
-    const int extras = rows_extras(BH, prm.W), id = blockIdx.x;
+    // (head, row block): heads in groups of `group` (place.h), so that the row blocks at work on an XCD share the K and V of
+    // few heads in its L2 (rows_group); in a group the last row blocks of all heads, the long ones of block-causal masks,
+    // first.  Behind the first `first_ids` of them, which fill the GPU, W workgroups per head for the long row blocks
+    // (wg >= nb; see below).
+    const int extras = placed(BH, prm.group, prm.W), id = blockIdx.x;
     const bool extra = id >= prm.first_ids && id < prm.first_ids + extras;
     const int L = id < prm.first_ids ? id : extra ? id - prm.first_ids : id - extras, per = extra ? prm.W : nb;
-    if (extra && L >= BH * prm.W) return;
-    const int gs = prm.group, grp = L / (gs * per), l = L - grp * gs * per, hg = BH - gs * grp < gs ? BH - gs * grp : gs;
-    bh = gs * grp + l % hg;
-    wg = per - 1 - l / hg + (extra ? nb : 0);
-  } else {
+    const Place p = place(L, BH, prm.group, per);
+    if (p.item >= per) return;                   // padding of the last group
+    bh = p.head;
+    wg = per - 1 - p.item + (extra ? nb : 0);
+  } else if (prm.place_fast < 0) {
     bh = blockIdx.x % BH;
     wg = blockIdx.x / BH;
+  } else {
+    const Place p = place_range(blockIdx.x, BH, prm.W, prm.place_fast, prm.place_quot, prm.place_rest);
+    bh = p.head;
+    wg = p.item;
   }
   const int b = bh / prm.H, h = bh % prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
@@ -1271,15 +1276,21 @@ int compute_units() {
 
 // How a launch is split at D = 64, by its row blocks against the wavefronts that are resident at once (8 per compute unit).
 // From half as many more on a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us; 24 heads of
-// N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there); with about as many a
-// wavefront takes a range of the list (32 heads of N = 4096 dense 174 -> 149 us; 8 heads of N = 17536 dense 710
-// either way, keep 0.1 with a new mask per call 115 -> 106); with fewer the ranges of whole workgroups are the faster ones (6 heads of N = 17776 at keep 0.3: 236
-// against 250 us).
+// N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there).  From three
+// quarters as many on a wavefront takes a range of the list, with fewer the ranges of whole workgroups are the faster
+// ones: they share a row block's merge.  bf16, us, ranges of workgroups / of wavefronts, keep 0.1, 0.3, 1 and block-causal:
+//   12 heads N = 8192 (0.75)   53 /  47    92 /  90   247 / 250   137 / 138      8 heads N = 8192 (0.5)   36 / 41   65 / 72   167 / 162    98 / 105
+//    9 heads N = 12000 (0.83)  71 /  65   139 / 138   398 / 404   211 / 208      6 heads N = 12000 (0.55) 53 / 52   96 / 98   265 / 270   153 / 153
+//   24 heads N = 4096 (0.75)   33 /  31    61 /  55   137 / 135    86 /  77     17 heads N = 4096 (0.53)  30 / 28   47 / 45    99 / 101    66 /  67
+//   48 heads N = 2048 (0.75)   26 /  24    40 /  38    85 /  79    54 /  58     56 heads N = 2048 (0.88)  28 / 25   41 / 42    94 /  86    61 /  60
+//    5 heads N = 24064 (0.92) 115 / 116   273 / 288   889 / 902   435 / 445    (above 300 row blocks per head: from one per wavefront on)
 static int wave_slots() { return FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * compute_units(); }    // wavefronts resident at once, D = 64
 static int fwd_mode(int B, int H, int nb, int D, bool compact) {
   if (D != 64) return COOP;
   const int64_t rows = (int64_t)B * H * nb, slots = wave_slots();
-  return 2 * rows >= 3 * slots ? ROWS_MODE : (rows >= slots && !compact ? WAVE : COOP);     // (compact: WAVE has four times as many ranges, hence parts)
+  if (2 * rows >= 3 * slots) return ROWS_MODE;
+  if (compact) return COOP;                                             // (WAVE has four times as many ranges, hence parts)
+  return rows >= slots || (nb >= 32 && nb <= 300 && 20 * rows >= (nb >= 48 ? 15 : 16) * slots) ? WAVE : COOP;
 }
 
 // ROWS_MODE: the workgroups per head for long row blocks, and the slots for their parts: as many as are resident at once,
@@ -1317,8 +1328,19 @@ static size_t parts_bytes(int B, int H, int nb, int W, int D, int mode) {
 //                  48 heads N = 8192 (2)          537 / 509 / 491 / 526 / 463 / 462 / 461   573      24 heads  291 / 271 / 252 / 252 / 252 / 253 / 255   269
 //   keep 0.2:      48 heads N = 8192              221 / 222 / 227 / 226 / 256 / 256 / 257   279     keep 0.5, 256 heads N = 2048  184 / 183 / 186 / 184 / 187 / 186 / 205
 //   keep 0.05:     48 heads N = 17792 (1)         307 / 315 / 354 / 356 / 408 / 410 / 409   430
+// With little more than one row block per wavefront the last group's long row blocks are all that is left to do in the end,
+// on wavefronts each alone with its row of up to nb tiles: all heads go out together there, longest row blocks first (what a
+// smaller L2 share costs the sparse uniform masks is less).  8 heads per group / all, block-causal, causal keep 0.2, keep 0.1, 0.5:
+//    9 heads N = 24064 (1.65 row blocks per wavefront)  1001 /  794   238 / 185   201 / 194   848 / 849
+//   11 heads N = 24064 (2.02)                           1103 /  909   261 / 215   223 / 228  1028 / 1033
+//   17 heads N = 12000 (1.56)                            541 /  384   130 / 102   110 / 106   430 / 426
+//   20 heads N = 12000 (1.84)                            549 /  456   130 / 112   117 / 117   456 / 464
+//   25 heads N = 8192 (1.56)                             295 /  272    90 /  75    78 /  79   293 / 294
+//   25 heads N = 12000 (2.29)                            660 /  536   158 / 135   145 / 157   574 / 582    (not there: 8 % on a sparse mask)
+//    9 heads N = 32000 (2.20)                              -          384 / 305   311 / 329      -         (nor there)
 static int rows_group(int B, int H, int nb) {
-  const int per_xcd = (B * H + 7) / 8, at_work = (wave_slots() / 8 + nb / 2) / nb;
+  const int heads = B * H, per_xcd = (heads + 7) / 8, at_work = (wave_slots() / 8 + nb / 2) / nb;
+  if (nb >= 128 && nb <= 400 && 8 * (int64_t)heads * nb <= 17 * (int64_t)wave_slots()) return 8 * per_xcd;
   const int most = at_work < 1 ? 1 : (at_work > 8 ? 8 : at_work), groups = (per_xcd + most - 1) / most;
   return 8 * ((per_xcd + groups - 1) / groups);
 }
@@ -1432,7 +1454,7 @@ static void launch_fwd_d(const FwdParams& prm, int D, int mode, int dt, hipStrea
   const int BH = prm.B * prm.H, grid = prm.W * BH;
   if (D == 128) {
     if constexpr (!EW) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
-  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, BH * prm.nb + rows_extras(BH, prm.W), st);
+  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, placed(BH, prm.group, prm.nb) + placed(BH, prm.group, prm.W), st);
   else if (mode == WAVE) launch_fwd_m<64, WAVE, EW>(prm, dt, grid, st);
   else launch_fwd_m<64, COOP, EW>(prm, dt, grid, st);
 }
@@ -1490,6 +1512,13 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
   // after a pause 677 against 707.)
   prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
+  {
+    const int heads = s.B * s.H;
+    prm.place_fast = s.D == 64 && mode == COOP ? std::min(compute_units(), prm.W * heads) : 0;
+    prm.place_quot = prm.place_fast / heads;
+    prm.place_rest = prm.place_fast % heads;
+    if (XCDS % heads == 0) prm.place_fast = -1;
+  }
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D, mode));
   prm.epoch = next_epoch();

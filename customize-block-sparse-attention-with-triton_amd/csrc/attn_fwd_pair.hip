@@ -17,6 +17,7 @@
 #include "common.h"
 #include "fwd_tile.h"
 #include "kernel_util.h"
+#include "place.h"
 
 namespace bsattn {
 
@@ -45,16 +46,14 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb, BH = prm.B * prm.H;
-  // linear id -> (head, row block): groups of 8 heads, one head per XCD, long row blocks first
+  // linear id -> (head, row block): groups of 8 heads, one head per XCD (place.h), long row blocks first
   int bh, m;
   const int per_chunk = gridDim.x / prm.split;    // chunk = slowest index: head i of a group stays on XCD i
   const int chunk = blockIdx.x / per_chunk;
   {
-    const int L = blockIdx.x - chunk * per_chunk;
-    const int grp = L / (8 * nb), l = L - grp * 8 * nb;
-    const int hg = BH - 8 * grp < 8 ? BH - 8 * grp : 8;
-    bh = 8 * grp + l % hg;
-    m = nb - 1 - l / hg;
+    const Place p = place(blockIdx.x - chunk * per_chunk, BH, XCDS, nb);
+    bh = p.head;
+    m = nb - 1 - p.item;
     if (m < 0) return;                           // padding of an incomplete last group
   }
   const int b = bh / prm.H, h = bh % prm.H;
@@ -448,7 +447,7 @@ static void launch_pair_c(const FwdParams& prm, int grid, hipStream_t st) {
 template <int D, int DT, bool EW>
 static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   const int BH = prm.B * prm.H;
-  const int grid = ((BH + 7) / 8) * 8 * prm.nb * prm.split;
+  const int grid = placed(BH, XCDS, prm.nb) * prm.split;
   // (the variant with immediate copy offsets: 5 % faster at D = 256, 3 % slower on dense masks at D = 128)
   if (prm.N % 64 != 0) launch_pair_c<D, DT, EW, false, true>(prm, grid, st);
   else if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256, false>(prm, grid, st);

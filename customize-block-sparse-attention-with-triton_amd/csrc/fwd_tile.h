@@ -19,6 +19,7 @@ struct FwdParams {
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
+  int place_fast, place_quot, place_rest;   // COOP, WAVE: place_range's arguments (place_fast < 0: heads interleaved)
   int group;                    // ROWS: heads whose row blocks go out together
   int out_f32;
   float qk_scale;  // sm_scale * log2(e)

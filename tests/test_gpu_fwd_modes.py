@@ -183,3 +183,30 @@ def test_long_row_blocks(dev, H, N, dtype, elementwise):
         assert ma <= MAXABS[dtype] and rl <= RELL2[dtype], (h, ma, rl)
         fin = torch.isfinite(ref_lse)
         assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref_lse)[fin].abs().max()) <= 2e-3
+
+
+# Heads that are not a multiple of 8 share the XCDs unevenly (place.h); every head has a mask of its own, so that one taken
+# for another shows.  D = 64: 24 row blocks (ranges of workgroups), 1690 (ranges of wavefronts), 3375 (row blocks, heads in
+# groups), 3250 (row blocks, all heads at once).
+@pytest.mark.parametrize("H,N,D", [(3, 449, 64), (13, 8300, 64), (27, 8000, 64), (25, 8320, 64), (3, 1000, 128), (11, 3200, 128), (5, 700, 256)])
+def test_uneven_heads(dev, H, N, D):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v, do = [x.to(dev) for x in make_qkv(1, H, N, D, torch.float16, 900 + N, n=4)]
+    block = uniform_block_mask(1, H, nb, 0.2, 901 + N).to(dev)
+    sc = D ** -0.5
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, block, sc)
+    for h in range(H):
+        keep = block[0, h].repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N]
+        s = (q[0, h].float() @ k[0, h].float().T * sc).masked_fill(~keep, float("-inf"))
+        ma, rl = errors(o[0, h], torch.softmax(s, -1) @ v[0, h].float())
+        assert ma <= MAXABS[torch.float16] and rl <= RELL2[torch.float16], (h, ma, rl)
+        assert float((lse[0, h] - torch.logsumexp(s, -1)).abs().max()) <= 2e-3
+    if N > 4000:
+        return
+    grads = fm.attention_forward_backward(q, k, v, block, sc, do)[2:]
+    for h in range(H):
+        sl = (slice(None), slice(h, h + 1))
+        alone = fm.attention_forward_backward(q[sl], k[sl], v[sl], block[sl], sc, do[sl])[2:]
+        for got, ref in zip(grads, alone):        # (another number of shares: another order of summation)
+            assert errors(got[sl], ref)[1] <= 1e-3, h
