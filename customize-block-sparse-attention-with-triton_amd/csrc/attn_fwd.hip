@@ -1,4 +1,5 @@
-// Block-sparse FlashAttention-2 forward for gfx950.
+// Block-sparse FlashAttention-2 forward for gfx950, head dimension 64 (attn_fwd_pair.hip has the larger ones), and what
+// the host decides about a forward launch.
 //
 // Work decomposition.  The kept tiles of one head form a list in row-major order; it is cut
 // into W contiguous ranges, one per workgroup, regardless of row boundaries (W depends on
@@ -11,7 +12,7 @@
 // range is normalised and written straight to O.  A row block cut by range boundaries is
 // finished by the workgroup that holds its first tiles: the others publish unnormalised parts
 // in the workspace (device-scope stores, then a flag), and it pulls them when it gets there.
-// That is the way of launches with few row blocks (COOP).  At D = 64, with about as many as wavefronts fit the GPU, a range
+// That is the way of launches with few row blocks (COOP).  With about as many as wavefronts fit the GPU, a range
 // belongs to a single wavefront (WAVE); with more a wavefront takes a whole row block, or a part of a long one (ROWS).
 //
 // Per tile a wavefront computes S^T = K Q^T (keys along MFMA rows, queries along lanes), so
@@ -40,12 +41,13 @@
 
 namespace bsattn {
 
-// A workgroup is four wavefronts, one per SIMD.  At D=64 a wavefront needs 256 registers and two
-// workgroups share a compute unit (while one merges or waits for its first tiles the other computes);
-// at D=128 a wavefront needs all 512 registers of its SIMD.
+// A workgroup is four wavefronts, one per SIMD.  A wavefront needs 256 registers and two workgroups share a compute unit
+// (while one merges or waits for its first tiles the other computes).
+// (At D = 128 a wavefront that owns 64 queries needs all 512 registers of its SIMD and spills beside them: every launch was
+// slower here than with the pairs of attn_fwd_pair.hip, see pair_split_128.)
 template <int D> struct FwdCfg {
   static constexpr int NW = 4;
-  static constexpr int WG_PER_CU = D == 64 ? 2 : 1;
+  static constexpr int WG_PER_CU = 2;
   static constexpr int TILE_BYTES = 64 * 2 * D;             // one K or V tile in LDS
   static constexpr int WAVE_LDS = 2 * TILE_BYTES;           // K buffer + V buffer
   static constexpr int ML_BYTES = NW * 2 * 64 * 4 + 64;     // exchange of (m, l) per query + the tile counter
@@ -60,7 +62,7 @@ template <int D> struct FwdCfg {
   static constexpr int ROUNDS = D / R;
   static constexpr int QPW = (R / 4) / NW;                  // output quads per wavefront and round
   static constexpr int SHORT_ROW = 6 * NW;                  // row blocks up to this many tiles may go to one wavefront
-  static constexpr int SNAP = WG_PER_CU > 1 ? 16 : 8;       // short ranges: a boundary at least this close to an end of its row block moves there
+  static constexpr int SNAP = 16;                           // short ranges: a boundary at least this close to an end of its row block moves there
 };
 
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
@@ -70,12 +72,11 @@ template <int D> struct FwdCfg {
 // WAVE: a workgroup is one wavefront and takes one range of its head's list (in between: about as many row blocks as
 // wavefronts fit the GPU, which whole row blocks would leave half idle in a second round).
 // LAYOUT: GENERAL any strides, any number of tokens; CONTIG_WHOLE the rows of K and of V follow each other without gaps
-// (row stride = D) and N is a multiple of 64; CONTIG_TAIL without gaps, any N; STRIDED_WHOLE any strides, N a multiple of 64
-// (D = 128, where the code for the rest costs registers that are not there).
+// (row stride = D) and N is a multiple of 64; CONTIG_TAIL without gaps, any N.
 // Where N is not a multiple of 64 the last tile of a row list holds `valid` < 64 keys: its copy repeats the last
 // key (no address lies beyond the tensor) and its scores beyond `valid` are set to -inf; the query rows of the last
 // row block beyond N repeat the last query and are not written.
-enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2, STRIDED_WHOLE = 3 };
+enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2 };
 enum { COOP = 0, ROWS_MODE = 1, WAVE = 2 };
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
 __global__ __launch_bounds__(MODE != COOP ? 64 : FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
@@ -141,8 +142,6 @@ void fwd_kernel(const FwdParams prm) {
     // keep 0.05 21.8 -> 20.2, keep 0.1 25.8 -> 25.1; keep 0.35 and above, other sizes: +-1 %).
     constexpr int LONG_GAP = MODE == WAVE ? 2 : 12, LONG_SNAP = 2;
     const bool long_ranges = MODE == WAVE || ((int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff || hs.Peff >= 3 * nb);   // (or row blocks much longer than the ranges)
-    // (D = 128, one workgroup per compute unit and tiles twice as long: sharing a row block is cheaper against the
-    // imbalance it avoids; 8 tiles for every head.  Half a range there: keep 0.1 87 -> 98 us, keep 0.15 107 -> 129 us.)
     const int half_range = hs.T / (2 * (hs.Peff > 0 ? hs.Peff : 1)) + 1;
     // (long ranges over short row blocks, up to 32 tiles on average: a boundary moves to the nearer end of its row block
     // from up to half such a row block away, so that next to no row block is shared; against 2 tiles: 8 heads of
@@ -150,7 +149,7 @@ void fwd_kernel(const FwdParams prm) {
     // costs more than the sharing: keep 0.35, one head, 48.0 -> 50.4 us with 12 tiles)
     const int avg_row = hs.T / (nb > 0 ? nb : 1);
     const int long_snap = MODE != WAVE && avg_row <= 32 ? avg_row / 2 + 1 : LONG_SNAP;
-    snap = long_ranges ? long_snap : (C::WG_PER_CU > 1 && half_range > C::SNAP ? half_range : C::SNAP);
+    snap = long_ranges ? long_snap : (half_range > C::SNAP ? half_range : C::SNAP);
     // (ranges that are long only against the row blocks they lie in, several to a row block: 24 positions; N = 6400
     // dense 31.2 -> 29.0 us, where 12 are best for N = 17536 dense, 102.1 against 104.0 us)
     const int long_gap = MODE == WAVE || (int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff ? LONG_GAP : 2 * LONG_GAP;
@@ -213,7 +212,7 @@ void fwd_kernel(const FwdParams prm) {
   // added to the (scalar) tile pointer, the per-lane part only depends on j through the chunk
   // swizzle, whose pattern repeats with period KPER in j (K) or not at all (V).
   constexpr int RPI = 64 / CPR;                 // tile rows per copy instruction
-  constexpr int KPER = D == 64 ? 2 : 4;         // period of the K swizzle in copy instructions
+  constexpr int KPER = 2;                       // period of the K swizzle in copy instructions
   unsigned koff[KPER], voff[1];
   {
     const int row0 = lane / CPR, ch = lane % CPR;
@@ -222,7 +221,7 @@ void fwd_kernel(const FwdParams prm) {
       koff[par] = 2u * (unsigned)(row0 * (int)prm.ks[2] + ((ch ^ k_swz<D>(par * RPI + row0)) * 8));
     voff[0] = 2u * (unsigned)(row0 * (int)prm.vs[2] + ((ch ^ v_swz<D>(row0)) * 8));
   }
-  static_assert(D == 64 || D == 128, "swizzle periods below are derived for 64 and 128");
+  static_assert(D == 64, "swizzle period");
   auto k_copy = [&](const unsigned short* tile, int j) {
     tile_load_async_one(tile + (int64_t)j * RPI * prm.ks[2], koff[j % KPER], lds_k_addr + j * 1024);
   };
@@ -373,10 +372,6 @@ void fwd_kernel(const FwdParams prm) {
   // once, all at once (the read latency is a multiple of an MFMA's issue interval), and serve
   // both query blocks.
   auto tile = [&](bool has1, int cbn, int tn, bool copy_v, bool partial, auto&& mid) {
-    // D = 128, fp16: the V fragments are read before the first softmax, so that the next V tile is requested
-    // earlier (B*H = 1 N = 17536 dense block-causal 206 -> 184 us; with bf16 inputs the same order is 5-10 %
-    // slower, and at D = 64 the registers are not there)
-    constexpr bool EARLY_V = D == 128 && DT == 0;
     uintx4 kfr[2][KS], vfr[4][DB];
     uintx4 pf[4][2];  // P^T operand fragments: [16-key slice][qb]
     auto scores = [&](int qb, floatx16& s0, floatx16& s1) {   // S^T[.][qb] = K Q[qb]^T (- m_i when FOLD)
@@ -477,10 +472,6 @@ void fwd_kernel(const FwdParams prm) {
     __builtin_amdgcn_sched_barrier(0);
     // [2]
     scores(1, sb0, sb1);
-    if constexpr (EARLY_V) {
-      if (has1) wait_vm<KOPS>(); else wait_vm<0>();  // V(cur) has landed (K(nxt) may be in flight)
-      read_v();
-    }
     float lnew0 = softmax_tile<FOLD, PB>(sa0, sa1, qk_scale, m_i[0], l_i[0], pf, 0);
     constexpr int NSC = 2 * KS;
 #pragma unroll
@@ -492,10 +483,8 @@ void fwd_kernel(const FwdParams prm) {
     mslice(1, sb0, sb1);
     if constexpr (EW || TAIL) { if (partial) mask_scores(sb0, sb1, EW ? mw1 : tail_word()); }
     settle(0, sa0, sa1, lnew0);
-    if constexpr (!EARLY_V) {
-      if (has1) wait_vm<KOPS>(); else wait_vm<0>();  // V(cur) has landed (K(nxt) may be in flight)
-      read_v();
-    }
+    if (has1) wait_vm<KOPS>(); else wait_vm<0>();  // V(cur) has landed (K(nxt) may be in flight)
+    read_v();
     lds_wait();      // the V fragments have arrived: the V buffer is free
     if (copy_v) v_copy_all(cbn);
     // [3]
@@ -1024,10 +1013,8 @@ void fwd_kernel(const FwdParams prm) {
         float wgt[NW][2];   // weight of wavefront p's partial for this lane's query of block qb
         float M[2], L[2];
         float keep[C::ROUNDS][C::QPW][4];   // this wavefront's share of the workgroup's part
-        // parts travel 16 bytes per lane and access at D = 64 (N = 17536, one head: dense 101.6 -> 101.0 us, keep 0.25
-        // 41.8 -> 41.1, keep 0.05 20.6 -> 20.0); at D = 128 that is faster for long ranges (keep 0.5 241 -> 233 us) and
-        // slower for short ones (keep 0.07 79 -> 82 us), and choosing by regime at run time gains nothing: 4 bytes there
-        constexpr bool WIDE_PARTS = D == 64;
+        // (parts travel 16 bytes per lane and access: N = 17536, one head, against 4 bytes: dense 101.6 -> 101.0 us, keep 0.25
+        // 41.8 -> 41.1, keep 0.05 20.6 -> 20.0)
         // A zero the compiler cannot see through (ctr[3] stays 0): the per-lane addresses into the
         // workspace do not change from row block to row block and would otherwise be computed
         // once, up front, and occupy registers throughout the tile loops.
@@ -1093,13 +1080,7 @@ void fwd_kernel(const FwdParams prm) {
                 store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, x[0] * inv, x[1] * inv,
                                x[2] * inv, x[3] * inv);
             } else {
-              // (WIDE_PARTS: 16 bytes per lane and access, the part laid out [quad][lane][4])
-              if constexpr (WIDE_PARTS) {
-                coherent_store4(slot + idx0 * 64 + lane * 4, x[0], x[1], x[2], x[3]);
-              } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) coherent_store(slot + (idx0 + e) * 64 + lane, x[e]);
-              }
+              coherent_store4(slot + idx0 * 64 + lane * 4, x[0], x[1], x[2], x[3]);   // (a part is laid out [quad][lane][4])
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) keep[rd][tq][e] = x[e];
@@ -1181,26 +1162,15 @@ void fwd_kernel(const FwdParams prm) {
                   mp[qb] = coherent_load(sp + 64 * D + qb * 32 + ln);
                   lp[qb] = coherent_load(sp + 64 * D + 64 + qb * 32 + ln);
                 }
-                if constexpr (WIDE_PARTS) {
-                  static_assert(!WIDE_PARTS || (C::ROUNDS == 1 && C::QPW == 4), "four 16-byte loads per lane and part");
-                  floatx4 ld[4];
-                  coherent_load4x4(sp + 4 * (w * C::QPW) * 64 + lane * 4, ld[0], ld[1], ld[2], ld[3]);   // ([quad][lane][4]: a quad is 1 KB)
+                static_assert(C::ROUNDS == 1 && C::QPW == 4, "four 16-byte loads per lane and part");
+                floatx4 ld[4];
+                coherent_load4x4(sp + 4 * (w * C::QPW) * 64 + lane * 4, ld[0], ld[1], ld[2], ld[3]);   // ([quad][lane][4]: a quad is 1 KB)
 #pragma unroll
-                  for (int rd = 0; rd < C::ROUNDS; ++rd)
+                for (int rd = 0; rd < C::ROUNDS; ++rd)
 #pragma unroll
-                    for (int tq = 0; tq < C::QPW; ++tq)
+                  for (int tq = 0; tq < C::QPW; ++tq)
 #pragma unroll
-                      for (int e = 0; e < 4; ++e) dat[rd][tq][e] = ld[rd * C::QPW + tq][e];
-                } else {
-#pragma unroll
-                  for (int rd = 0; rd < C::ROUNDS; ++rd)
-#pragma unroll
-                    for (int tq = 0; tq < C::QPW; ++tq)
-#pragma unroll
-                      for (int e = 0; e < 4; ++e)
-                        dat[rd][tq][e] = coherent_load(sp + (rd * C::R + 4 * (w * C::QPW + tq) + e) * 64 + lane);
-                  __builtin_amdgcn_sched_barrier(0);
-                }
+                    for (int e = 0; e < 4; ++e) dat[rd][tq][e] = ld[rd * C::QPW + tq][e];
               }
               float sc_own[2], sc_p[2];
 #pragma unroll
@@ -1285,8 +1255,7 @@ int compute_units() {
 //   48 heads N = 2048 (0.75)   26 /  24    40 /  38    85 /  79    54 /  58     56 heads N = 2048 (0.88)  28 / 25   41 / 42    94 /  86    61 /  60
 //    5 heads N = 24064 (0.92) 115 / 116   273 / 288   889 / 902   435 / 445    (above 300 row blocks per head: from one per wavefront on)
 static int wave_slots() { return FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * compute_units(); }    // wavefronts resident at once, D = 64
-static int fwd_mode(int B, int H, int nb, int D, bool compact) {
-  if (D != 64) return COOP;
+static int fwd_mode(int B, int H, int nb, bool compact) {
   const int64_t rows = (int64_t)B * H * nb, slots = wave_slots();
   if (2 * rows >= 3 * slots) return ROWS_MODE;
   if (compact) return COOP;                                             // (WAVE has four times as many ranges, hence parts)
@@ -1298,10 +1267,10 @@ static int fwd_mode(int B, int H, int nb, int D, bool compact) {
 // eighth of a head to do, or where the library's scratch memory does not hold the counters.
 static int long_row_groups(int B, int H, int nb, bool compact);
 
-static int groups_per_head(int B, int H, int nb, int D, int mode, bool compact) {
+static int groups_per_head(int B, int H, int nb, int mode, bool compact) {
   if (mode == ROWS_MODE) return long_row_groups(B, H, nb, compact);
   const int cus = compute_units();
-  const int per_cu = D != 64 ? FwdCfg<128>::WG_PER_CU : (mode == COOP ? 1 : FwdCfg<64>::NW) * FwdCfg<64>::WG_PER_CU;
+  const int per_cu = (mode == COOP ? 1 : FwdCfg<64>::NW) * FwdCfg<64>::WG_PER_CU;
   int64_t W = (int64_t)cus * per_cu / ((int64_t)B * H);   // as many workgroups as are resident at once
   const int64_t cap = (int64_t)nb * nb;
   if (W > cap) W = cap;
@@ -1311,11 +1280,11 @@ static int groups_per_head(int B, int H, int nb, int D, int mode, bool compact) 
 
 // workspace: partial slots [B*H][W][2][partial_floats] (fp32; ROWS_MODE: one per workgroup for long row blocks), then the
 // arrival counters [B*H][nb] (64 bit)
-static size_t slots_bytes(int B, int H, int W, int D, int mode) {
-  return (size_t)B * H * W * (mode == ROWS_MODE ? 1 : 2) * partial_floats(D) * sizeof(float);
+static size_t slots_bytes(int B, int H, int W, int mode) {
+  return (size_t)B * H * W * (mode == ROWS_MODE ? 1 : 2) * partial_floats(64) * sizeof(float);
 }
-static size_t parts_bytes(int B, int H, int nb, int W, int D, int mode) {
-  return slots_bytes(B, H, W, D, mode) + (size_t)B * H * nb * sizeof(unsigned long long);
+static size_t parts_bytes(int B, int H, int nb, int W, int mode) {
+  return slots_bytes(B, H, W, mode) + (size_t)B * H * nb * sizeof(unsigned long long);
 }
 
 // ROWS_MODE: heads whose row blocks go out together, the longest first.  One per XCD keeps one head's K and V in an L2, but a
@@ -1348,26 +1317,13 @@ static int rows_group(int B, int H, int nb) {
 static int long_row_groups(int B, int H, int nb, bool compact) {
   const int64_t W = wave_slots() / (compact ? 2 : 1) / ((int64_t)B * H);
   if (W < 8) return 0;
-  return compact && parts_bytes(B, H, nb, (int)W, 64, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
+  return compact && parts_bytes(B, H, nb, (int)W, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
-// D = 128 with enough row blocks in the launch to fill the chip goes to the kernel that gives each
-// row block to one wavefront pair (two wavefronts per SIMD, no merges between workgroups).  With
-// fewer row blocks its critical path is the longest row, which the host cannot see (the lists
-// stay on the device): from two row blocks per compute unit on it won in every measured case,
-// from one on only when rows are short (at most 32 tiles).  (Elementwise masks and numbers of tokens
-// that are not whole tiles always go there, see pair_split_128: fwd_kernel with their extra state has 200 bytes of
-// spills per lane.)
-static bool use_pair_kernel(int64_t row_blocks, int nb) {
-  const int64_t cus = compute_units();
-  return row_blocks >= 2 * cus || (row_blocks >= cus && nb <= 32);
-}
-
-// Pair kernel: workgroups per row block.  One when the launch has enough row blocks to fill the GPU twice
+// Pair kernel, D = 256: workgroups per row block.  One when the launch has enough row blocks to fill the GPU twice
 // over; otherwise the row lists are shared (up to 8 ways, a share of a dense list keeping at least 8 tiles).
-static int pair_split(int B, int H, int nb, int D) {
-  const int64_t row_blocks = (int64_t)B * H * nb;
-  const int64_t want = (int64_t)compute_units() * (D == 128 ? 4 : 2) * 2;
+static int pair_split_256(int64_t row_blocks, int nb) {
+  const int64_t want = (int64_t)compute_units() * 4;
   if (row_blocks >= want) return 1;
   int64_t s = (want + row_blocks - 1) / row_blocks;
   const int cap = nb / 8 > 1 ? nb / 8 : 1;
@@ -1375,40 +1331,68 @@ static int pair_split(int B, int H, int nb, int D) {
   return (int)(s > 8 ? 8 : s);
 }
 
-// The same at D = 128 for the launches only the pair kernel takes (elementwise masks, N not a multiple of 64): about four
-// workgroups per compute unit over the launch; at most 4 shares of a row unless it is long (a share of a dense row then
-// has 16 tiles), at least two tiles in one.  us, N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares, and fwd_kernel before:
-//   8 heads N = 4000, token window of 1000   46 /  47 /  55 /  61 /  72 /  89    84
-//   8 heads N = 4000, token-causal          147 /  99 /  82 /  90 /  95 / 103   131
-//   4 heads N = 4096, token window of 1228   32 /  32 /  36 /  36 /  46 /  50    58
-//   1 head N = 8192, token-causal           160 /  93 /  73 /  67 /  57 /  57    73
-//   1 head N = 17000, keep 0.5              233 / 152 / 119 / 138 / 126 / 131   260
-//   2 heads N = 1000, token-causal           40 /  27 /  27 /  24 /  24 /  27    34
-// Whole tiles with a block mask and at least use_pair_kernel's row blocks were not shared before and are not without whole
-// tiles either (8 heads N = 4000, fp16: keep 0.25 44 / 49, dense 95 / 97).
-static int pair_split_128(int64_t row_blocks, int nb, bool elementwise) {
-  const int64_t cus = compute_units();
-  if (!elementwise && use_pair_kernel(row_blocks, nb)) return 1;
-  int64_t s = 4 * cus / row_blocks;
+// The same at D = 128 with block masks.  A share costs the launch that sums the parts (3 us) and their traffic, so short
+// lists are shared only where few of them are in the launch.  us, N(0,1), 1 / 2 / 3 / 4 / 6 shares, and fwd_kernel (ranges of
+// the lists, 512 registers a wavefront), which had these launches up to 512 row blocks before, with bf16 and with fp16:
+//   1 head  N = 832    keep 0.3  12 /  12 /  11 /  10 /  10    20   28     dense  20 /  16 /  14 /  13 /  12    21   30
+//   5 heads N = 832              13 /  14 /  14 /  16 /  16    21   29            20 /  18 /  17 /  19 /  20    22   31
+//  11 heads N = 1344             17 /  23 /  24 /  26 /  30    25   34            30 /  31 /  31 /  31 /  37    40   60
+//   1 head  N = 2048             23 /  17 /  15 /  14 /  16    22   31            42 /  27 /  22 /  19 /  18    32   47
+//   4 heads N = 2048             24 /  22 /  23 /  24 /  25    23   32            43 /  32 /  31 /  31 /  32    29   40
+//   2 heads N = 4096             36 /  27 /  27 /  26 /  26    27   41            81 /  51 /  44 /  39 /  37    37   59
+//   4 heads N = 4096             37 /  33 /  32 /  33 /  40    43   67            82 /  58 /  54 /  55 /  67    52   91
+//   6 heads N = 4096             46 /  41 /  44 /  45 /  52    50   80            88 /  74 /  91 /  85 /  90    89  165
+//   1 head  N = 8192             67 /  42 /  35 /  32 /  32    41   67           157 /  88 /  69 /  58 /  54    58   98
+//   3 heads N = 8192             75 /  58 /  68 /  63 /  70    71  124           168 / 128 / 159 / 143 / 146   143  257
+//   2 heads N = 12032            92 /  71 /  83 /  78 /  83    84  154           240 / 176 / 223 / 195 / 197   192  338
+//   8 heads N = 3072             31 /  34 /  39                                   67 /  64 /  73                  (1, 2, 3 shares)
+//   9 heads N = 2048             24 /  27 /  27                                   47 /  44 /  41    keep 0.1  15 / 25 / 24
+//   7 heads N = 4096             47 /  43 /  48                                   95 /  87 / 100    keep 0.1  24 / 32 / 34
+// From 480 row blocks on one: 8 heads N = 4000, keep 0.25, 44 / 49.
+static int pair_split_128(int64_t row_blocks, int nb) {
+  const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
+  if (nb < 56 && rows > 6 * nb) return 1;
+  const int s = rows >= 480 ? 1 : rows >= 320 ? 2 : rows >= 208 ? 3 : 4;
+  // a share of a dense list keeps 8 tiles, 4 in a launch of few lists, 12 in one of many short ones
+  const int cap = rows <= 64 && nb >= 12 ? nb / 4 : rows > 96 && nb < 48 ? nb / 12 : nb / 8;
+  return s < cap ? s : cap > 1 ? cap : 1;
+}
+
+// The same at D = 128 with elementwise masks: about four workgroups per compute unit over the launch; at most 4 shares of a
+// row unless it is long (a share of a dense row then has 16 tiles), at least two tiles in one.  us, N(0,1) bf16, 1 / 2 / 3 /
+// 4 / 6 / 8 shares:
+//   8 heads N = 4000, token window of 1000   46 /  47 /  55 /  61 /  72 /  89
+//   8 heads N = 4000, token-causal          147 /  99 /  82 /  90 /  95 / 103
+//   4 heads N = 4096, token window of 1228   32 /  32 /  36 /  36 /  46 /  50
+//   1 head N = 8192, token-causal           160 /  93 /  73 /  67 /  57 /  57
+//   1 head N = 17000, keep 0.5              233 / 152 / 119 / 138 / 126 / 131
+//   2 heads N = 1000, token-causal           40 /  27 /  27 /  24 /  24 /  27
+static int pair_split_words(int64_t row_blocks, int nb) {
+  int64_t s = 4 * (int64_t)compute_units() / row_blocks;
   const int few = nb / 2 < 4 ? nb / 2 : 4, cap = nb / 16 > few ? nb / 16 : few;
   if (s > cap) s = cap;
   return (int)(s > 8 ? 8 : s < 1 ? 1 : s);
 }
 
 static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
-  return split > 1 ? (size_t)split * B * H * N * (D + 2) * sizeof(float) : 0;
+  return 256 + (split > 1 ? (size_t)split * B * H * N * (D + 2) * sizeof(float) : 0);
+}
+
+static int pair_split(int B, int H, int N, int D, bool words) {
+  const int nb = (N + 63) / 64;
+  const int64_t row_blocks = (int64_t)B * H * nb;
+  return D == 256 ? pair_split_256(row_blocks, nb) : words ? pair_split_words(row_blocks, nb) : pair_split_128(row_blocks, nb);
 }
 
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
-  if (D == 256) return 256 + pair_parts_bytes(B, H, N, D, pair_split(B, H, (N + 63) / 64, D));   // the pair kernel only
+  if (D != 64) {     // (compact launches: block masks only; their parts at D = 128 are 32 MB at most)
+    const int block = pair_split(B, H, N, D, false);
+    return pair_parts_bytes(B, H, N, D, compact ? block : std::max(block, pair_split(B, H, N, D, true)));
+  }
   const int nb = (N + 63) / 64;
-  const int mode = fwd_mode(B, H, nb, D, compact);
-  const int W = groups_per_head(B, H, nb, D, mode, compact);
-  if (W == 0) return 256;                 // nothing is shared
-  const size_t bytes = parts_bytes(B, H, nb, W, D, mode);
-  if (D != 128 || compact) return bytes;      // (compact launches: whole tiles and block masks only)
-  const size_t parts = 256 + pair_parts_bytes(B, H, N, D, pair_split_128((int64_t)B * H * nb, nb, true));
-  return parts > bytes ? parts : bytes;
+  const int mode = fwd_mode(B, H, nb, compact);
+  const int W = groups_per_head(B, H, nb, mode, compact);
+  return W == 0 ? 256 : parts_bytes(B, H, nb, W, mode);      // (0: nothing is shared)
 }
 
 // one size for bsattn_fwd and bsattn_fwd_elementwise
@@ -1427,36 +1411,28 @@ static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
   hipLaunchKernelGGL((fwd_kernel<D, DT, MODE, EW, LAYOUT>), dim3(grid), dim3(MODE != COOP ? 64 : C::NW * 64), LDS, st, prm);
 }
 
-// The copies with immediate offsets are compiled where they were measured faster: D = 64 (2-4 %) and
-// D = 128 with bf16 inputs (4-8 %; with fp16 inputs 1-3 % slower).
-template <int D, int DT, int MODE, bool EW>
+// (The copies with immediate offsets are 2-4 % faster.)
+template <int DT, int MODE, bool EW>
 static void launch_fwd_t(const FwdParams& prm, int grid, hipStream_t st) {
-  const bool contig = prm.ks[2] == D && prm.vs[2] == D, whole = prm.N % 64 == 0;
-  if constexpr (D == 128) {      // (whole tiles only)
-    if (DT != 0 && contig) launch_fwd_c<D, DT, MODE, EW, DT != 0 ? CONTIG_WHOLE : STRIDED_WHOLE>(prm, grid, st);
-    else launch_fwd_c<D, DT, MODE, EW, STRIDED_WHOLE>(prm, grid, st);
-  } else {
-    if (contig && whole) launch_fwd_c<D, DT, MODE, EW, CONTIG_WHOLE>(prm, grid, st);
-    else if (contig) launch_fwd_c<D, DT, MODE, EW, CONTIG_TAIL>(prm, grid, st);
-    else launch_fwd_c<D, DT, MODE, EW, GENERAL>(prm, grid, st);
-  }
+  const bool contig = prm.ks[2] == 64 && prm.vs[2] == 64, whole = prm.N % 64 == 0;
+  if (contig && whole) launch_fwd_c<64, DT, MODE, EW, CONTIG_WHOLE>(prm, grid, st);
+  else if (contig) launch_fwd_c<64, DT, MODE, EW, CONTIG_TAIL>(prm, grid, st);
+  else launch_fwd_c<64, DT, MODE, EW, GENERAL>(prm, grid, st);
 }
 
-template <int D, int MODE, bool EW>
+template <int MODE, bool EW>
 static void launch_fwd_m(const FwdParams& prm, int dt, int grid, hipStream_t st) {
-  if (dt == 0) launch_fwd_t<D, 0, MODE, EW>(prm, grid, st);
-  else if (dt == 1) launch_fwd_t<D, 1, MODE, EW>(prm, grid, st);
-  else launch_fwd_t<D, 2, MODE, EW>(prm, grid, st);
+  if (dt == 0) launch_fwd_t<0, MODE, EW>(prm, grid, st);
+  else if (dt == 1) launch_fwd_t<1, MODE, EW>(prm, grid, st);
+  else launch_fwd_t<2, MODE, EW>(prm, grid, st);
 }
 
 template <bool EW>
-static void launch_fwd_d(const FwdParams& prm, int D, int mode, int dt, hipStream_t st) {
+static void launch_fwd_d(const FwdParams& prm, int mode, int dt, hipStream_t st) {
   const int BH = prm.B * prm.H, grid = prm.W * BH;
-  if (D == 128) {
-    if constexpr (!EW) launch_fwd_m<128, COOP, EW>(prm, dt, grid, st);
-  } else if (mode == ROWS_MODE) launch_fwd_m<64, ROWS_MODE, EW>(prm, dt, placed(BH, prm.group, prm.nb) + placed(BH, prm.group, prm.W), st);
-  else if (mode == WAVE) launch_fwd_m<64, WAVE, EW>(prm, dt, grid, st);
-  else launch_fwd_m<64, COOP, EW>(prm, dt, grid, st);
+  if (mode == ROWS_MODE) launch_fwd_m<ROWS_MODE, EW>(prm, dt, placed(BH, prm.group, prm.nb) + placed(BH, prm.group, prm.W), st);
+  else if (mode == WAVE) launch_fwd_m<WAVE, EW>(prm, dt, grid, st);
+  else launch_fwd_m<COOP, EW>(prm, dt, grid, st);
 }
 
 // ---- forward without any allocation by anybody: the scratch memory is part of the library ----
@@ -1505,56 +1481,43 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.row_ptr = row_ptr; prm.col_idx = col_idx; prm.ws = (float*)ws;
   prm.tile_partial = tile_partial; prm.tile_bits = (const unsigned long long*)tile_bits;
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
-  const int mode = fwd_mode(s.B, s.H, prm.nb, s.D, s.compact);
-  prm.W = groups_per_head(s.B, s.H, prm.nb, s.D, mode, s.compact);
+  prm.out_f32 = s.out_dtype == BSATTN_F32;
+  prm.qk_scale = s.sm_scale * 1.4426950408889634f;
+  for (int i = 0; i < 3; ++i) { prm.qs[i] = s.qs[i]; prm.ks[i] = s.ks[i]; prm.vs[i] = s.vs[i]; prm.os[i] = s.os[i]; }
+  // bf16 with a bf16-typed result: P is rounded to bf16 as well (the reference rounds P to the type of
+  // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
+  const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
+  if (s.D != 64) {
+    prm.split = pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr);
+    prm.part_o = (float*)ws + 64;
+    prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
+    launch_fwd_pair(prm, s.D, dt, tile_bits != nullptr, st);
+    return launch_status();
+  }
+  const int mode = fwd_mode(s.B, s.H, prm.nb, s.compact);
+  prm.W = groups_per_head(s.B, s.H, prm.nb, mode, s.compact);
   // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are.  (Not WAVE: single
   // wavefronts that arrive while another kernel ends do not fill the SIMDs in order, and two with the larger share on one
   // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
   // after a pause 677 against 707.)
-  prm.first_ids = s.D == 64 && mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
-  {
-    const int heads = s.B * s.H;
-    prm.place_fast = s.D == 64 && mode == COOP ? std::min(compute_units(), prm.W * heads) : 0;
-    prm.place_quot = prm.place_fast / heads;
-    prm.place_rest = prm.place_fast % heads;
-    if (XCDS % heads == 0) prm.place_fast = -1;
-  }
+  prm.first_ids = mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
+  prm.place_fast = mode == COOP ? std::min(compute_units(), prm.W * heads) : 0;
+  prm.place_quot = prm.place_fast / heads;
+  prm.place_rest = prm.place_fast % heads;
+  if (XCDS % heads == 0) prm.place_fast = -1;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
-  prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, s.D, mode));
+  prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();
   {
-    const int BHl = s.B * s.H;
-    const int F = prm.first_ids > 0 && prm.first_ids % BHl == 0 ? (prm.first_ids / BHl < prm.W ? prm.first_ids / BHl : prm.W) : 0;
-    const bool ok = mode == COOP && (prm.first_ids == 0 || prm.first_ids % BHl == 0) && range_permutation(prm.nb, prm.W, F, BHl, prm.perm, prm.perm_causal);
+    const int F = prm.first_ids > 0 && prm.first_ids % heads == 0 ? (prm.first_ids / heads < prm.W ? prm.first_ids / heads : prm.W) : 0;
+    const bool ok = mode == COOP && (prm.first_ids == 0 || prm.first_ids % heads == 0) && range_permutation(prm.nb, prm.W, F, heads, prm.perm, prm.perm_causal);
     prm.perm_n = ok ? prm.W : 0;
     prm.perm_fast = F;
     prm.perm_min_tiles = (int)((int64_t)prm.nb * prm.nb * 3 / 4);
   }
-  prm.out_f32 = s.out_dtype == BSATTN_F32;
-  prm.qk_scale = s.sm_scale * 1.4426950408889634f;
-  for (int i = 0; i < 3; ++i) { prm.qs[i] = s.qs[i]; prm.ks[i] = s.ks[i]; prm.vs[i] = s.vs[i]; prm.os[i] = s.os[i]; }
-  const bool bf = s.dtype == BSATTN_BF16;
-  const int BH = s.B * s.H;
-  prm.split = 1;
-  const int64_t row_blocks = (int64_t)BH * prm.nb;
-  const bool only_pair = s.D == 256 || (s.D == 128 && (tile_bits != nullptr || s.N % 64 != 0));   // no other kernel
-  if (only_pair || (s.D == 128 && use_pair_kernel(row_blocks, prm.nb))) {
-    // launches with few row blocks share the row lists between workgroups; at D = 128 with whole tiles and a block mask
-    // the cooperative kernel below takes those launches (sharing was measured: faster on dense masks with 2-3
-    // heads, 25-30 % slower on sparse ones)
-    if (s.D == 256) prm.split = pair_split(s.B, s.H, prm.nb, s.D);
-    else if (only_pair) prm.split = pair_split_128(row_blocks, prm.nb, tile_bits != nullptr);
-    prm.part_o = (float*)ws + 64;
-    prm.part_ml = prm.part_o + (size_t)prm.split * BH * s.N * s.D;
-    launch_fwd_pair(prm, s.D, !bf ? 0 : (prm.out_f32 ? 1 : 2), tile_bits != nullptr, st);
-    return launch_status();
-  }
-  // bf16 with a bf16-typed result: P is rounded to bf16 as well (the reference rounds P to the type of
-  // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
-  const int dt = !bf ? 0 : (prm.out_f32 ? 1 : 2);
-  if (tile_bits == nullptr) launch_fwd_d<false>(prm, s.D, mode, dt, st);
-  else launch_fwd_d<true>(prm, s.D, mode, dt, st);
+  if (tile_bits == nullptr) launch_fwd_d<false>(prm, mode, dt, st);
+  else launch_fwd_d<true>(prm, mode, dt, st);
   return launch_status();
 }
 

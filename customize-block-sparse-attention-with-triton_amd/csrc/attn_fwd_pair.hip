@@ -1,14 +1,13 @@
-// Block-sparse FlashAttention-2 forward, head dimension 128 for launches with many row blocks, and
-// head dimension 256 (the only forward kernel for it; one wavefront per SIMD there, K and V fragments
+// Block-sparse FlashAttention-2 forward, head dimensions 128 and 256 (one wavefront per SIMD there, K and V fragments
 // taken from LDS in two portions).
 //
-// At D = 128 a wavefront that owns 64 queries needs all 512 registers of its SIMD, so the
-// general kernel (attn_fwd.hip) runs one wavefront per SIMD and is bound by instruction issue.
+// At D = 128 a wavefront that owns 64 queries would need all 512 registers of its SIMD and be bound by instruction issue.
 // Here a row block belongs to a pair of wavefronts, 32 queries each (256 registers: two
 // wavefronts per SIMD), which share one K and one V tile buffer: a workgroup is one pair, four
 // workgroups fit a compute unit, and the grid has one workgroup per (head, row block) - the
-// hardware's dispatcher balances the load, no merge is ever needed.  Heads are taken in groups
-// of 8, head i of a group on XCD i (workgroups go to XCDs round-robin by linear id), so that the
+// hardware's dispatcher balances the load - or, where that leaves the GPU idle, several that share a row block's list and
+// whose parts a second launch sums (pair_split).  Heads are taken in groups
+// of 8, head i of a group on XCD i (place.h), so that the
 // row blocks resident on an XCD share one head's K and V in its L2; long row blocks of
 // block-causal masks come first.
 //

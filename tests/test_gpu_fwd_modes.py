@@ -210,3 +210,25 @@ def test_uneven_heads(dev, H, N, D):
         alone = fm.attention_forward_backward(q[sl], k[sl], v[sl], block[sl], sc, do[sl])[2:]
         for got, ref in zip(grads, alone):        # (another number of shares: another order of summation)
             assert errors(got[sl], ref)[1] <= 1e-3, h
+
+
+# D = 128, block masks: 3 shares of 13 tiles, 2 of 24 (with a ragged length too), 4 and 3 of long lists, 1 with more row blocks
+@pytest.mark.parametrize("H,N", [(1, 832), (6, 1536), (6, 1500), (2, 4096), (4, 4096), (5, 4096), (7, 2048)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_shares_of_block_mask_lists(dev, H, N, dtype):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 128, dtype, 950 + N)]
+    block = torch.cat([block_mask(nb, 0.3, 951 + N + h) for h in range(H)], 1)
+    block[0, 0, 1] = False
+    block[0, 0, 1, :2] = True                                # fewer tiles than shares
+    sc = 128 ** -0.5
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, block.to(dev), sc)
+    for h in range(H):
+        keep = block[0, h].to(dev).repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N]
+        s = (q[0, h].float() @ k[0, h].float().T * sc).masked_fill(~keep, float("-inf"))
+        ma, rl = errors(o[0, h], torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float())
+        assert ma <= MAXABS[dtype] and rl <= RELL2[dtype], (h, ma, rl)
+        ref = torch.logsumexp(s, -1)
+        fin = torch.isfinite(ref)
+        assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3
