@@ -1320,15 +1320,29 @@ static int long_row_groups(int B, int H, int nb, bool compact) {
   return compact && parts_bytes(B, H, nb, (int)W, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
-// Pair kernel, D = 256: workgroups per row block.  One when the launch has enough row blocks to fill the GPU twice
-// over; otherwise the row lists are shared (up to 8 ways, a share of a dense list keeping at least 8 tiles).
+// Pair kernel, D = 256: workgroups per row block.  A share costs the launch that sums the parts and their traffic (64 KB of
+// fp32 per row block and share, as much as a tile's operands), so only launches that leave the GPU's 512 pairs short share,
+// and short lists where few of them are in the launch.  us, N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares:
+//    1 head  N = 512    keep 0.3   16 /  15 /  13 /  14 /  11 /  12    dense   23 /  18 /  16 /  14 /  15 /  13
+//    5 heads N = 832               21 /  22 /  21 /  22 /  24 /  26            35 /  29 /  27 /  29 /  29 /  32
+//   12 heads N = 832               29 /  30 /  29 /  36 /  35 /  37            36 /  37 /  34 /  45 /  45 /  53
+//   24 heads N = 1344              40 /  59 /  72 /  82 / 109 / 133            60 /  88 / 102 / 114 / 141 / 173
+//    4 heads N = 2048              41 /  34 /  32 /  30 /  42 /  44            78 /  54 /  47 /  42 /  57 /  57
+//    7 heads N = 2048              40 /  38 /  46 /  47 /  58 /  68            78 /  58 /  75 /  70 /  83 /  94
+//   14 heads N = 2048              46 /  64 /  73 /  84 / 105 / 130            82 / 108 / 118 / 132 / 154 / 173
+//    2 heads N = 4096              66 /  45 /  40 /  38 /  50 /  53           149 /  88 /  72 /  62 /  78 /  77
+//    4 heads N = 4096              80 /  60 /  66 /  65 /  74 /  88           149 /  97 / 131 / 110 / 120 / 138
+//   10 heads N = 4096             119 / 120 / 125 / 137 / 171 / 216           303 / 266 / 258 / 265 / 308 / 352
+//    3 heads N = 6016              89 /  95 /  81 /  90 /  98 / 107           217 / 242 / 176 / 196 / 195 / 195
+//    1 head  N = 8192             123 /  73 /  59 /  53 /  67 /  67           291 / 160 / 120 /  99 / 131 / 114
+//    5 heads N = 8192             211 / 191 / 188 / 201 / 231 / 271           595 / 489 / 456 / 452 / 505 / 533
+//    1 head  N = 12032            159 /  99 / 119 / 102 / 109 / 105           425 / 236 / 310 / 247 / 254 / 209
 static int pair_split_256(int64_t row_blocks, int nb) {
-  const int64_t want = (int64_t)compute_units() * 4;
-  if (row_blocks >= want) return 1;
-  int64_t s = (want + row_blocks - 1) / row_blocks;
-  const int cap = nb / 8 > 1 ? nb / 8 : 1;
-  if (s > cap) s = cap;
-  return (int)(s > 8 ? 8 : s);
+  const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
+  if (rows > 8 * nb || rows >= 1024) return 1;
+  const int s = rows >= 320 ? 2 : rows >= 208 ? (nb >= 80 ? 3 : 2) : rows > 128 && nb < 80 ? 3 : 4;
+  const int cap = rows <= 64 ? nb / 4 : nb / 6;
+  return s < cap ? s : cap > 1 ? cap : 1;
 }
 
 // The same at D = 128 with block masks.  A share costs the launch that sums the parts (3 us) and their traffic, so short
