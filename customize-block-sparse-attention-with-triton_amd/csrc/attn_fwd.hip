@@ -1,5 +1,5 @@
-// Block-sparse FlashAttention-2 forward for gfx950, head dimension 64 (attn_fwd_pair.hip has the larger ones), and what
-// the host decides about a forward launch.
+// Block-sparse FlashAttention-2 forward for gfx950, head dimension 64 (attn_fwd_short.hip has its launches with few row blocks,
+// attn_fwd_pair.hip the larger head dimensions), and what the host decides about a forward launch.
 //
 // Work decomposition.  The kept tiles of one head form a list in row-major order; it is cut
 // into W contiguous ranges, one per workgroup, regardless of row boundaries (W depends on
@@ -336,7 +336,10 @@ void fwd_kernel(const FwdParams prm) {
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
       int row = r * 64 + qb * 32 + ln;
-      if (TAIL && row >= prm.N) row = prm.N - 1;
+      if (TAIL && row >= prm.N) {
+        row = prm.N - 1;
+        if constexpr (EW) l_i[qb] = 1e-30f;      // (a query that has no mass yet is recentred in every tile; this one never will)
+      }
       const unsigned short* qrow = qg + (int64_t)row * prm.qs[2];
 #pragma unroll
       for (int s = 0; s < KS; ++s) qf[qb][s] = *reinterpret_cast<const uintx4*>(qrow + 16 * s + 8 * g);
@@ -1398,12 +1401,39 @@ static int pair_split(int B, int H, int N, int D, bool words) {
   return D == 256 ? pair_split_256(row_blocks, nb) : words ? pair_split_words(row_blocks, nb) : pair_split_128(row_blocks, nb);
 }
 
+// Which launches fwd_short_kernel (D = 64) takes: pairs of wavefronts per workgroup (0: none) and shares of a row block's list.
+// With 4 pairs a row block has a compute unit to itself, with 2 two share it.  us, ranges of workgroups or of wavefronts /
+// 2 pairs / 4 pairs / 4 pairs and 2 shares; keep 0.1, 0.3, 1, block-causal (fp16 the first five, bf16 the others):
+//    5 heads N = 512 (40 row blocks)   11 /  8 /  8 / 10     11 /  8 /  8 / 10     12 /  8 /  8 / 10     11 /  8 /  8 / 10
+//    8 heads N = 2048 (256)            13 /  9 /  9 / 19     16 / 12 / 11 / 21     20 / 19 / 17 / 27     19 / 18 / 16 / 22
+//    1 head  N = 4096 (64; 4 shares 12, 12, 15, 15)  13 / 10 / 10 / 12   16 / 15 / 13 / 13   22 / 30 / 25 / 19   23 / 29 / 24 / 18
+//    1 head  N = 6400 (100)            17 / 12 / 11 / 13     21 / 20 / 18 / 17     27 / 43 / 36 / 26     24 / 43 / 35 / 24
+//    2 heads N = 8192 (256)            17 / 15 / 14 / 21     27 / 26 / 23 / 30     53 / 55 / 44 / 57     38 / 54 / 44 / 35
+//   16 heads N = 3072 (768)            22 / 18 / 21          32 / 28 / 32          59 / 56 / 60          42 / 34 / 40
+//   32 heads N = 3072 (1536)           30 / 27 / 40          52 / 47 / 61         101 /103 /126          65 / 62 / 81
+//   44 heads N = 3072 (2112)           39 / 37 / 57          57 / 63 / 84         137 /149 /176          81 / 91 /109   (not there)
+//   14 heads N = 4096 (896)            29 / 21 / 29          42 / 37 / 47          84 / 87 / 99          53 / 51 / 57
+//   24 heads N = 4096 (1536)           31 / 32 / 45          55 / 57 / 70         132 /133 /153          78 / 89 / 93   (nor there)
+//    3 heads N = 6400 (300)            20 / 15 / 17          29 / 29 / 30          50 / 65 / 73          37 / 48 / 37   (nor there)
+//    5 heads N = 6400 (500)            26 / 16 / 20          41 / 30 / 34          73 / 71 / 75          46 / 51 / 45
+//    1 head  N = 10048 (157)           19 / 16 / 13 / 20     26 / 30 / 25 / 30     44 / 72 / 55 / 64     32 / 71 / 53 / 35   (nor there)
+struct ShortPlan { int pairs, split; };
+static ShortPlan short_plan(int64_t row_blocks, int nb) {
+  const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
+  if (nb > SHORT_MAX_BLOCKS) return {0, 1};
+  // long lists: as many shares as fill the GPU
+  if (rows <= 256) return {4, nb < 56 || rows > 128 ? 1 : rows > 64 ? 2 : 4};
+  const bool takes = nb <= 48 ? rows <= 1792 : nb <= 64 ? rows <= 1024 : rows >= 400 && rows <= 512;
+  return {takes ? 2 : 0, 1};
+}
+
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
   if (D != 64) {     // (compact launches: block masks only; their parts at D = 128 are 32 MB at most)
     const int block = pair_split(B, H, N, D, false);
     return pair_parts_bytes(B, H, N, D, compact ? block : std::max(block, pair_split(B, H, N, D, true)));
   }
   const int nb = (N + 63) / 64;
+  if (const ShortPlan plan = short_plan((int64_t)B * H * nb, nb); plan.pairs > 0) return pair_parts_bytes(B, H, N, D, plan.split);
   const int mode = fwd_mode(B, H, nb, compact);
   const int W = groups_per_head(B, H, nb, mode, compact);
   return W == 0 ? 256 : parts_bytes(B, H, nb, W, mode);      // (0: nothing is shared)
@@ -1413,6 +1443,7 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
 size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_bytes(B, H, N, D); }
 
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
+void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st);   // attn_fwd_short.hip
 template <int D, int DT, int MODE, bool EW, int LAYOUT>
 static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
@@ -1501,11 +1532,13 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // bf16 with a bf16-typed result: P is rounded to bf16 as well (the reference rounds P to the type of
   // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
   const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
-  if (s.D != 64) {
-    prm.split = pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr);
+  const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
+  if (s.D != 64 || plan.pairs > 0) {
+    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
-    launch_fwd_pair(prm, s.D, dt, tile_bits != nullptr, st);
+    if (s.D == 64) launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
+    else launch_fwd_pair(prm, s.D, dt, tile_bits != nullptr, st);
     return launch_status();
   }
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.compact);

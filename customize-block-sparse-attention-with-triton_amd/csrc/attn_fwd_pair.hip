@@ -214,7 +214,8 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) { oacc[db][0][i] = 0.f; oacc[db][1][i] = 0.f; }
-  float m_i = 0.f, l_i = 0.f;
+  // (EW: a query that has no mass yet is recentred in every tile; one that does not exist never will have any)
+  float m_i = 0.f, l_i = EW && TAIL && !exists ? 1e-30f : 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
@@ -384,7 +385,7 @@ template <bool BF16, int S>
 __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm, int D, unsigned quads) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i >= quads) return;
-  const int qshift = D == 256 ? 6 : 5;                       // log2 of the threads per query row
+  const int qshift = D == 256 ? 6 : D == 128 ? 5 : 4;        // log2 of the threads per query row
   const unsigned rowg = i >> qshift;                         // row over all heads
   const int col = (int)(i & ((1u << qshift) - 1)) * 4;
   const int bh = (int)(rowg / (unsigned)prm.N), row = (int)(rowg - (unsigned)bh * prm.N);
@@ -425,12 +426,17 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
 
 // (shared lists: at most four workgroups per compute unit, so the values fit 32 bits)
 template <bool BF16, int S = 2>
-static void launch_sum_parts(const FwdParams& prm, int D, hipStream_t st) {
+static void launch_sum_parts_t(const FwdParams& prm, int D, hipStream_t st) {
   if constexpr (S < 8) {
-    if (prm.split != S) { launch_sum_parts<BF16, S + 1>(prm, D, st); return; }
+    if (prm.split != S) { launch_sum_parts_t<BF16, S + 1>(prm, D, st); return; }
   }
   const unsigned quads = (unsigned)((int64_t)prm.B * prm.H * prm.N * D / 4);
   hipLaunchKernelGGL((pair_sum_parts_kernel<BF16, S>), dim3((quads + 255) / 256), dim3(256), 0, st, prm, D, quads);
+}
+
+void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st) {
+  if (bf16) launch_sum_parts_t<true>(prm, D, st);
+  else launch_sum_parts_t<false>(prm, D, st);
 }
 
 template <int D, int DT, bool EW, bool CONTIG, bool TAIL>
@@ -451,7 +457,7 @@ static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   if (prm.N % 64 != 0) launch_pair_c<D, DT, EW, false, true>(prm, grid, st);
   else if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256, false>(prm, grid, st);
   else launch_pair_c<D, DT, EW, false, false>(prm, grid, st);
-  if (prm.split > 1) launch_sum_parts<DT != 0>(prm, D, st);
+  if (prm.split > 1) launch_sum_parts(prm, D, DT != 0, st);
 }
 
 template <int D>

@@ -6,6 +6,8 @@
 
 namespace bsattn {
 
+constexpr int SHORT_MAX_BLOCKS = 128;   // row blocks of a head up to which fwd_short_kernel takes a launch
+
 struct FwdParams {
   const void* q; const void* k; const void* v; void* o; float* lse;
   const int32_t* row_ptr; const int32_t* col_idx;

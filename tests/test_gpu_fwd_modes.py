@@ -232,3 +232,31 @@ def test_shares_of_block_mask_lists(dev, H, N, dtype):
         ref = torch.logsumexp(s, -1)
         fin = torch.isfinite(ref)
         assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3
+
+
+# D = 64, few row blocks: 4 pairs of wavefronts per row block (1, 2 and 4 shares of its list), 2 pairs, the longest lists
+# (128 tiles), the first length beyond; lists shorter than the pairs are many, empty ones, ragged lengths, queries without keys
+@pytest.mark.parametrize("H,N", [(1, 64), (3, 130), (5, 512), (8, 2048), (9, 2048), (1, 3584), (1, 4090), (1, 5000), (2, 8192), (5, 6400), (1, 8193)])
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("elementwise", [False, True])
+def test_short_lists(dev, H, N, dtype, out_fp32, elementwise):
+    import fa2_custom_mask as fm
+    nb = -(-N // 64)
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 64, dtype, 970 + N)]
+    block = torch.cat([block_mask(nb, 0.3, 971 + N + h) for h in range(H)], 1) if nb > 2 else torch.ones(1, H, nb, nb, dtype=torch.bool)
+    block[0, -1, nb - 1] = True                              # the last row block: all tiles
+    mask = block.to(dev)
+    if elementwise:
+        i = torch.arange(N, device=dev)
+        mask = mask.repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N] & ((i[:, None] - i[None, :]) % 7 != 0)
+        mask[:, :, N // 2] = False                           # a query without keys
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, 0.125, out_fp32=out_fp32)
+    rel = 1e-3 if out_fp32 or dtype == torch.float16 else RELL2[dtype]
+    for h in range(H):
+        keep = mask[0, h] if elementwise else mask[0, h].repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N]
+        s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~keep, float("-inf"))
+        ma, rl = errors(o[0, h], torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float())
+        assert ma <= MAXABS[dtype] and rl <= rel, (h, ma, rl)
+        ref = torch.logsumexp(s, -1)
+        fin = torch.isfinite(ref)
+        assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3

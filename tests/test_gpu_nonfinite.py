@@ -65,3 +65,10 @@ def test_row_blocks_of_wavefront_pairs(dev, D, H, N, elementwise, dtype, what):
                                                (64, 160, 1300, False), (128, 2, 1024, False), (128, 1, 2048, False)])
 def test_ranges_and_row_blocks(dev, D, H, N, elementwise, dtype, what):
     check(dev, H, N, D, dtype, elementwise, what)
+
+
+# D = 64: ranges of workgroups (more row blocks than the kernel for short lists takes)
+@pytest.mark.parametrize("what", ["key", "query", "inf"])
+@pytest.mark.parametrize("N,elementwise", [(8256, False), (8300, True)])
+def test_ranges_of_long_heads(dev, N, elementwise, what):
+    check(dev, 1, N, 64, torch.float16, elementwise, what)
