@@ -237,6 +237,32 @@ int bsattn_fwd_block_mask_tokens(const void* q, const void* k, const void* v, vo
                         sm_scale, q_strides, k_strides, v_strides, o_strides, workspace, workspace_bytes, stream, true);
 }
 
+int bsattn_fwd_takes_mask(int B, int H, int N, int D) {
+  return check_attn(1, 1, B, H, N, D, BSATTN_F16, BSATTN_F16, true) == BSATTN_OK && launch_fwd_takes_mask(B, H, N, D) ? 1 : 0;
+}
+
+int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+                           const int64_t* mask_strides, int Bm, int Hm, int B, int H, int N, int D, int dtype,
+                           int out_dtype, float sm_scale, const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* o_strides, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+  if (block == nullptr || mask_strides == nullptr) return BSATTN_ERR_NULL;
+  static const int32_t no_list = 0;
+  const int rc = fwd_check(q, k, v, o, &no_list, &no_list, Bm, Hm, B, H, N, D, dtype, out_dtype, q_strides, k_strides,
+                           v_strides, o_strides, true);
+  if (rc != BSATTN_OK) return rc;
+  if (!launch_fwd_takes_mask(B, H, N, D)) return BSATTN_ERR_RANGE;
+  if (workspace == nullptr || workspace_bytes < coop_workspace_bytes(B, H, N, D)) return BSATTN_ERR_WORKSPACE;
+  if (((uintptr_t)workspace & 15) != 0) return BSATTN_ERR_STRIDE;
+  AttnShape s;
+  s.B = B; s.H = H; s.N = N; s.D = D; s.Bm = Bm; s.Hm = Hm; s.dtype = dtype; s.out_dtype = out_dtype;
+  s.sm_scale = sm_scale;
+  for (int i = 0; i < 3; ++i) { s.qs[i] = q_strides[i]; s.ks[i] = k_strides[i]; s.vs[i] = v_strides[i]; s.os[i] = o_strides[i]; s.dos[i] = 0; }
+  s.mask = block;
+  for (int i = 0; i < 4; ++i) s.ms[i] = mask_strides[i];
+  return launch_fwd(q, k, v, o, lse, nullptr, nullptr, nullptr, nullptr, s, workspace, (hipStream_t)stream);
+}
+
 int bsattn_fwd_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const int32_t* row_ptr,
                       const int32_t* col_idx, const uint8_t* tile_partial, const uint64_t* tile_bits, int Bm, int Hm,
                       int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale, const int64_t* q_strides,

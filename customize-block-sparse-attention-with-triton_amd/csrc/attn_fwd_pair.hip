@@ -69,9 +69,14 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[0][s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
   }
-  int t0 = rp[m], t1 = rp[m + 1];
+  int* lcols = reinterpret_cast<int*>(lds + 2 * TILE_BYTES + 512);
+  const bool listed = EW || prm.mask == nullptr;
+  int t0, t1;
+  if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
+  else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols); }
   if (prm.split > 1) {                           // this workgroup's share of the row block's list
     const int len = t1 - t0;
+    if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
     t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
     t0 = t0 + (int)((int64_t)len * chunk / prm.split);
     if (t0 == t1) return;                        // (pair_sum_parts_kernel knows which shares are empty)
@@ -91,7 +96,6 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   unsigned char* lds_k = lds;
   unsigned char* lds_v = lds + TILE_BYTES;
   const unsigned long long* lds_bits = reinterpret_cast<const unsigned long long*>(lds + 2 * TILE_BYTES);
-  int* lcols = reinterpret_cast<int*>(lds + 2 * TILE_BYTES + 512);
   const unsigned lds_k_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
   const unsigned lds_v_addr = lds_k_addr + TILE_BYTES;
   const unsigned lds_bits_addr = lds_k_addr + 2 * TILE_BYTES;
@@ -109,7 +113,9 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
     return c;
   };
   constexpr int COL_MASK = 0x3fffffff;
-  auto col_of = [&](int t) { return t - t0 < PAIR_COLS_CAP ? lcols[t - t0] : flagged_col(t); };
+  static_assert(MASK_MAX_BLOCKS <= PAIR_COLS_CAP, "all columns from the mask are in LDS");
+  const int first_t = listed ? t0 : 0;           // entry t of the list is lcols[t - first_t] once it is staged
+  auto col_of = [&](int t) { return t - first_t < PAIR_COLS_CAP ? lcols[t - first_t] : flagged_col(t); };
 
   // asynchronous tile copies: copy instruction j covers tile rows [4j, 4j+4); this wavefront issues
   // the instructions [HALF w, HALF (w+1)) of every tile (and 256 of the 512 bytes of mask words)
@@ -191,13 +197,15 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   const uintx4 ones_frag = {g == 0 ? 0x3c003c00u : 0u, 0u, 0u, 0u};
 
   // first tile's copies (its column from one scalar load), then the column list into LDS
-  int cx = flagged_col(t0);
+  int cx = listed ? flagged_col(t0) : __builtin_amdgcn_readfirstlane(lcols[t0]);
   k_copy(cx & COL_MASK, t0);
   v_copy(cx & COL_MASK);
-  for (int i = threadIdx.x; i < t1 - t0 && i < PAIR_COLS_CAP; i += 128) {
-    int c = prm.col_idx[t0 + i];
-    if constexpr (EW) c |= (int)prm.tile_partial[t0 + i] << 30;
-    lcols[i] = c;
+  if (listed) {
+    for (int i = threadIdx.x; i < t1 - t0 && i < PAIR_COLS_CAP; i += 128) {
+      int c = prm.col_idx[t0 + i];
+      if constexpr (EW) c |= (int)prm.tile_partial[t0 + i] << 30;
+      lcols[i] = c;
+    }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0), visible to the compiler: Q and the first tiles
   if constexpr (FOLD) {
@@ -390,9 +398,7 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
   const int col = (int)(i & ((1u << qshift) - 1)) * 4;
   const int bh = (int)(rowg / (unsigned)prm.N), row = (int)(rowg - (unsigned)bh * prm.N);
   const int b = bh / prm.H, h = bh % prm.H, BH = prm.B * prm.H;
-  const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
-  const int32_t* rp = prm.row_ptr + (int64_t)mh * prm.nb;
-  const int t0 = rp[row / 64], len = rp[row / 64 + 1] - t0;
+  const int len = prm.part_len[bh * prm.nb + row / 64];
   floatx4 acc = {0.f, 0.f, 0.f, 0.f};
   float M = -INFINITY, L = 0.f;
   if (len > 0) {

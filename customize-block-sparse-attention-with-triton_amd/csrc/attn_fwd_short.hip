@@ -62,9 +62,14 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[0][s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
   }
-  int t0 = rp[m], t1 = rp[m + 1];
+  int* lcols = reinterpret_cast<int*>(lds + C::COLS_OFF);
+  const bool listed = EW || prm.mask == nullptr;
+  int t0, t1;
+  if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
+  else { t0 = 0; t1 = columns_of_row<SHORT_MAX_BLOCKS>(prm, b, h, m, lane, lcols); }
   if (prm.split > 1) {                            // this workgroup's share of the row block's list
     const int len = t1 - t0;
+    if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
     t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
     t0 = t0 + (int)((int64_t)len * chunk / prm.split);
     if (t0 == t1) return;                         // (pair_sum_parts_kernel knows which shares are empty)
@@ -75,7 +80,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   const float qk_scale = prm.qk_scale;
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
   constexpr int COL_MASK = 0x3fffffff;            // (EW: bit 30 of a staged column says "partly set")
-  int* lcols = reinterpret_cast<int*>(lds + C::COLS_OFF);
+  const int first_t = listed ? t0 : 0;            // entry t of the list is lcols[t - first_t] once it is staged
   unsigned char* mine = lds + c * C::PAIR_BYTES;
   const unsigned mine_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds + c * C::PAIR_BYTES;
 
@@ -130,13 +135,15 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   // the first step's copies (their column from one scalar load), then the column list into LDS
   int t = t0 + c, cx = 0;
   if (t < t1) {
-    cx = cols[t];
+    cx = listed ? cols[t] : __builtin_amdgcn_readfirstlane(lcols[t]);
     issue(cx, t, 0);
   }
-  for (int i = threadIdx.x; i < t1 - t0 && i < C::COLS_CAP; i += 128 * S) {
-    int x = prm.col_idx[t0 + i];
-    if constexpr (EW) x |= (int)prm.tile_partial[t0 + i] << 30;
-    lcols[i] = x;
+  if (listed) {
+    for (int i = threadIdx.x; i < t1 - t0 && i < C::COLS_CAP; i += 128 * S) {
+      int x = prm.col_idx[t0 + i];
+      if constexpr (EW) x |= (int)prm.tile_partial[t0 + i] << 30;
+      lcols[i] = x;
+    }
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0), visible to the compiler: Q and the first tiles
   if constexpr (FOLD) {
@@ -167,7 +174,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
     const int tn = t + S;
     int cxn = 0;
     if (tn < t1) {
-      cxn = __builtin_amdgcn_readfirstlane(lcols[tn - t0]);
+      cxn = __builtin_amdgcn_readfirstlane(lcols[tn - first_t]);
       issue(cxn & COL_MASK, tn, (it + 1) & 1);
     }
     if (t < t1) {

@@ -30,6 +30,8 @@ int launch_pack_tiles(const uint8_t* dense, int Bm, int Hm, int nb, int64_t sb, 
 struct AttnShape {
   int B, H, N, D, Bm, Hm;
   int dtype, out_dtype;
+  const uint8_t* mask = nullptr;   // forward: the block mask in place of the lists (launch_fwd_takes_mask), with its strides
+  int64_t ms[4];
   bool compact = false;   // forward: the split with the smaller workspace (bsattn_fwd_static)
   float sm_scale;
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];  // batch, head, row strides (elements)
@@ -58,6 +60,7 @@ int get_deterministic();
 int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                const int32_t* row_ptr, const int32_t* col_idx, const uint8_t* tile_partial,
                const uint64_t* tile_bits, const AttnShape& s, void* ws, hipStream_t st);
+bool launch_fwd_takes_mask(int B, int H, int N, int D);   // can launch_fwd do without lists?
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact = false);   // what launch_fwd itself needs
 // Address, on the current device, of the library's own scratch array (BSATTN_STATIC_SCRATCH_BYTES).
 int static_scratch(void** ptr);

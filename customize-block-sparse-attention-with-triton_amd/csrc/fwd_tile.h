@@ -6,11 +6,14 @@
 
 namespace bsattn {
 
+constexpr int MASK_MAX_BLOCKS = 512;    // ... up to which a kernel takes the columns of a row block from the block mask
 constexpr int SHORT_MAX_BLOCKS = 128;   // row blocks of a head up to which fwd_short_kernel takes a launch
 
 struct FwdParams {
   const void* q; const void* k; const void* v; void* o; float* lse;
   const int32_t* row_ptr; const int32_t* col_idx;
+  const unsigned char* mask;       // the block mask itself in place of the lists (kernels whose workgroups have a row block each), or null
+  int64_t ms[4];                   // its strides
   const unsigned char* tile_partial;        // elementwise masks: per kept tile, 1 = only partly set
   const unsigned long long* tile_bits;      // ... and its 64 row words (bit c = column c)
   float* ws;                       // partial slots of row blocks shared between workgroups (two per workgroup)
@@ -19,6 +22,7 @@ struct FwdParams {
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair kernel: workgroups per row block (1: results written directly)
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
+  int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
   int place_fast, place_quot, place_rest;   // COOP, WAVE: place_range's arguments (place_fast < 0: heads interleaved)
@@ -55,6 +59,32 @@ __device__ __forceinline__ float softmax_tile(const floatx16& s0, const floatx16
     }
   }
   return l;
+}
+
+// The kept columns of row block m, ascending, from the block mask into cols (LDS), by every wavefront of the workgroup by
+// itself (all write the same): no list kernels in front of the launch, and one dependent access instead of two (row
+// pointer, then column).  Returns their number, at most nb <= MAX.
+template <int MAX>
+__device__ __forceinline__ int columns_of_row(const FwdParams& prm, int b, int h, int m, int lane, int* cols) {
+  const unsigned char* row = prm.mask + (prm.Bm > 1 ? b : 0) * prm.ms[0] + (prm.Hm > 1 ? h : 0) * prm.ms[1] + m * prm.ms[2];
+  constexpr int AHEAD = MAX < 256 ? MAX / 64 : 4;      // accesses on their way at once
+  int n = 0;
+  for (int c0 = 0; c0 < prm.nb; c0 += 64 * AHEAD) {
+    bool keep[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const int c = c0 + 64 * i + lane;
+      keep[i] = c < prm.nb && row[(int64_t)c * prm.ms[3]] != 0;
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+      const unsigned long long bal = __ballot(keep[i]);
+      if (keep[i]) cols[n + __popcll(bal & ((1ull << lane) - 1ull))] = c0 + 64 * i + lane;
+      n += __popcll(bal);
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+  return n;
 }
 
 __device__ __forceinline__ void* out_base(const FwdParams& prm, int b, int h) {

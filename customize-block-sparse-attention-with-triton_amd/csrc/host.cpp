@@ -31,6 +31,8 @@ struct Library {
   decltype(&::bsattn_fwd_tokens) fwd = nullptr;
   decltype(&::bsattn_fwd_block_mask_workspace) fwd_block_mask_workspace = nullptr;
   decltype(&::bsattn_fwd_block_mask_tokens) fwd_block_mask = nullptr;
+  decltype(&::bsattn_fwd_takes_mask) fwd_takes_mask = nullptr;
+  decltype(&::bsattn_fwd_mask_tokens) fwd_mask = nullptr;
   decltype(&::bsattn_bwd_workspace) bwd_workspace = nullptr;
   decltype(&::bsattn_bwd_tokens) bwd = nullptr;
 } lib;
@@ -50,6 +52,8 @@ void bind(const std::string& path) {
   get(lib.fwd, "bsattn_fwd_tokens");
   get(lib.fwd_block_mask_workspace, "bsattn_fwd_block_mask_workspace");
   get(lib.fwd_block_mask, "bsattn_fwd_block_mask_tokens");
+  get(lib.fwd_takes_mask, "bsattn_fwd_takes_mask");
+  get(lib.fwd_mask, "bsattn_fwd_mask_tokens");
   get(lib.bwd_workspace, "bsattn_bwd_workspace");
   get(lib.bwd, "bsattn_bwd_tokens");
 }
@@ -301,6 +305,34 @@ py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v
   return py::make_tuple(results(o, lse, q_.size(3), return_lse), lists);
 }
 
+// Forward straight from a block mask; None where the launch needs its lists (or the mask is on another device).
+py::object forward_mask(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale, bool out_fp32,
+                        bool return_lse) {
+  check_mask_heads(mask.size(0), mask.size(1), q_);
+  const int64_t D_ = q_.size(3) < 64 ? 64 : q_.size(3);
+  at::NoGradGuard no_grad;
+  c10::DeviceGuard guard(q_.device());
+  if (mask.device() != q_.device() || lib.fwd_takes_mask((int)q_.size(0), (int)q_.size(1), (int)q_.size(2), (int)D_) == 0) return py::none();
+  const Tensor q = prepared(padded(q_)), k = prepared(padded(k_)), v = prepared(padded(v_));
+  const at::ScalarType out_dtype = result_type(q, out_fp32);
+  const Tensor o = like(q, out_dtype);
+  const int B = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3);
+  Tensor lse;
+  if (return_lse) lse = at::empty({B, H, N}, q.options().dtype(at::kFloat));
+  size_t bytes = 0;
+  check(lib.fwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_fwd_workspace");
+  const hipStream_t stream = stream_of(q);
+  {
+    const WorkspaceLock lock;
+    const Tensor ws = workspace_locked(bytes, q.device(), stream);
+    check(lib.fwd_mask(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(), return_lse ? lse.data_ptr<float>() : nullptr,
+                       (const uint8_t*)mask.const_data_ptr(), mask.strides().data(), (int)mask.size(0), (int)mask.size(1), B, H, N, D,
+                       dtype_code(q.scalar_type()), dtype_code(out_dtype), (float)sm_scale, q.strides().data(), k.strides().data(),
+                       v.strides().data(), o.strides().data(), ws.data_ptr(), bytes, stream), "bsattn_fwd_mask");
+  }
+  return results(o, lse, q_.size(3), return_lse);
+}
+
 // ---- autograd ----
 // The column lists of an elementwise mask, which only a backward walks and which hold as many words as the row lists, are
 // made by the first backward that needs them: a forward may have none.  While the words by grid position are in Python's
@@ -436,6 +468,7 @@ PYBIND11_MODULE(_host, m) {
   m.def("block_mask_to_lists", &block_mask_to_lists);
   m.def("forward", &forward);
   m.def("forward_block_mask", &forward_block_mask);
+  m.def("forward_mask", &forward_mask);
   m.def("attention", &attention, py::arg("q"), py::arg("k"), py::arg("v"), py::arg("mask"), py::arg("lists"),
         py::arg("lists_t").none(true), py::arg("grid"), py::arg("sm_scale"), py::arg("out_fp32"), py::arg("return_lse"));
   m.def("set_python_lists", [](py::object make, py::object keep) { python_lists = new PythonLists{std::move(make), std::move(keep)}; });

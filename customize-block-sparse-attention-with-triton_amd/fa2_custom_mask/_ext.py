@@ -39,6 +39,9 @@ _SIGNATURES = {
     "bsattn_bwd_tokens": ([_p] * 15 + [_i] * 8 + [_f] + [_p] * 8 + [_p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_block_mask_tokens": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f,
                                       _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
+    "bsattn_fwd_takes_mask": ([_i, _i, _i, _i], _i),
+    "bsattn_fwd_mask_tokens": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _p, _p, _p, _p,
+                                ctypes.c_size_t, _p], _i),
     "bsattn_fwd_block_mask": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f,
                                _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_static": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f,

@@ -9,7 +9,7 @@ import ctypes
 import torch
 
 from . import _ext
-from .utils import TILE, _host, block_mask_to_lists, lists_cache, grid_cache, mask_to_lists, num_tiles, is_block_form, _check_mask
+from .utils import TILE, UNMADE, _host, block_mask_to_lists, lists_cache, grid_cache, mask_to_lists, num_tiles, is_block_form, _check_mask
 
 
 def build_groups_from_block_mask(mask):
@@ -147,8 +147,20 @@ def _mask_of(q, k, v, mask):
 
 def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
     mask, N = _mask_of(q, k, v, mask)
+    seen = lists_cache.seen(mask, N)
+    grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    if not grad and (seen is None or seen is UNMADE):
+        # launches whose workgroups have a row block each take its columns from a block mask, new or not
+        if seen is None:
+            _check_mask(mask)
+        if seen is UNMADE or is_block_form(mask, N):
+            result = _host.forward_mask(q, k, v, mask, sm_scale, out_fp32, return_lse)
+            if result is not None:
+                if seen is None:
+                    lists_cache.put(mask, N, False, UNMADE)
+                return result
     lists = lists_cache.get(mask, N, False)
-    if torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad):
+    if grad:
         if lists is None:
             lists = mask_to_lists(mask, N, both=True)                        # :48
         # The backward walks the column lists.  A block mask's are made here, where the GPU does not wait for them; those of
@@ -162,7 +174,6 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
                 grid = grid_cache.get(mask, N)
         return _host.attention(q, k, v, mask, lists, lists_t, grid, sm_scale, out_fp32, return_lse)
     if lists is None:
-        _check_mask(mask)
         if is_block_form(mask, N):
             # a block mask seen for the first time (or one that changes with every call): lists and forward in one call
             result, lists = _host.forward_block_mask(q, k, v, mask, sm_scale, out_fp32, return_lse)

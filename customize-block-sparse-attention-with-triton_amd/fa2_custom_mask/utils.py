@@ -167,6 +167,11 @@ def to_block_mask(mask, N):
     return mask if is_block_form(mask, N) else reduce_dense_mask(mask)
 
 
+# In place of the lists of a block mask that forwards so far have done without (they took its rows from the mask itself): they are made
+# when they are asked for.
+UNMADE = object()
+
+
 class _ListsCache:
     """Kept-tile lists of the most recently used masks.  A static mask (the usual case: one mask
     for every layer and step) is indexed once instead of once per call.  An entry is only used
@@ -187,6 +192,13 @@ class _ListsCache:
         except RuntimeError:
             return None
 
+    def seen(self, mask, N):
+        """Is there an entry for the row lists of the mask as it is: its lists, UNMADE, or None."""
+        entry = self._entries.get((id(mask), N, False))
+        if entry is None or entry[0]() is not mask or self._version(mask) != entry[1]:
+            return None
+        return entry[2]
+
     def get(self, mask, N, transpose):
         key = (id(mask), N, transpose)
         entry = self._entries.get(key)
@@ -195,6 +207,10 @@ class _ListsCache:
         ref, version, lists, stream = entry
         if ref() is not mask or self._version(mask) != version:
             return None
+        if lists is UNMADE:
+            lists = block_mask_to_lists(mask, transpose=transpose)
+            self.put(mask, N, transpose, lists)
+            return lists
         self._entries.move_to_end(key)
         # the lists were filled by kernels on `stream` (a raw handle): work on another stream waits for
         # what that stream has been given so far (no event is recorded when the lists are made: a mask

@@ -56,7 +56,7 @@ extern "C" {
  *   100: first layout.
  *   200: bsattn_bwd and bsattn_bwd_elementwise take dq_strides, dk_strides, dv_strides after
  *        do_strides; the entry points of the forward over quads of row blocks are gone. */
-#define BSATTN_ABI_VERSION 202
+#define BSATTN_ABI_VERSION 203
 int bsattn_version(void);
 /* Process-wide switch (default off), returns the previous setting.  On: the forward's result
  * depends on nothing but its inputs and the device (two runs give the same bits).  Off: the
@@ -314,6 +314,16 @@ int bsattn_fwd_block_mask_tokens(const void* q, const void* k, const void* v, vo
                                  const int64_t* q_strides, const int64_t* k_strides,
                                  const int64_t* v_strides, const int64_t* o_strides, void* workspace,
                                  size_t workspace_bytes, void* stream);
+/* The forward straight from a block mask (strides in elements of its 4 dimensions, bytes != 0 kept), without lists, where
+ * bsattn_fwd_takes_mask(B, H, N, D) returns 1: launches whose workgroups have a row block each.  Other shapes are refused
+ * with BSATTN_ERR_RANGE.  The workspace of bsattn_fwd_workspace. */
+int bsattn_fwd_takes_mask(int B, int H, int N, int D);
+int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse,
+                           const uint8_t* block, const int64_t* mask_strides, int Bm, int Hm,
+                           int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                           const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* o_strides, void* workspace,
+                           size_t workspace_bytes, void* stream);
 int bsattn_bwd_tokens(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                       const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
                       const int32_t* col_idx, const int32_t* col_ptr, const int32_t* row_idx,

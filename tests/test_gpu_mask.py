@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import uniform_block_mask, causal_block_mask
+from helpers import make_qkv, uniform_block_mask, causal_block_mask
 
 pytestmark = pytest.mark.gpu
 
@@ -173,3 +173,44 @@ def test_scan_and_fill(dev, shape, keep):
     assert np.array_equal(lists.row_ptr.cpu().numpy(), np.concatenate([[0], np.cumsum(by_column.sum(1).numpy())]))
     assert np.array_equal(lists.col_idx.cpu().numpy()[:int(by_column.sum())], by_column.nonzero()[:, 1].numpy())
     assert lists.counts.tolist() == [int(by_column.any(1).sum()), int(by_column.sum())]
+
+
+# D = 64: 4 pairs of wavefronts and 1, 2 and 4 shares, 2 pairs; D = 128: no shares, 3 and 4; 130 and 512 row blocks; D = 256
+@pytest.mark.parametrize("B,H,N,D", [(1, 2, 1000, 64), (1, 1, 5000, 64), (1, 1, 4096, 64), (2, 9, 1100, 64), (2, 40, 300, 128),
+                                     (1, 4, 4096, 128), (1, 1, 8300, 128), (1, 1, 32768, 128), (1, 3, 700, 256)])
+@pytest.mark.parametrize("form", ["one", "per head", "transposed", "every other"])
+def test_forward_from_the_mask_itself(dev, B, H, N, D, form):
+    """A forward that takes the columns of its row blocks from the block mask gives the bits of one that walks the mask's
+    lists, whatever the mask's strides; the lists are made when they are asked for."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask import utils
+    q, k, v = [x.to(dev) for x in make_qkv(B, H, N, D, torch.float16, 30 + N)]
+    nb = -(-N // 64)
+    g = torch.Generator().manual_seed(31 + N)
+    bm, hm = (B, H) if form == "per head" else (1, 1)
+    m = torch.rand(bm, hm, 2 * nb, 2 * nb, generator=g) < (0.3 if nb < 200 else 0.05)
+    m[:, :, nb // 2] = False                                    # (a row block without tiles)
+    m = m.to(dev)
+    mask = m[:, :, ::2, ::2] if form == "every other" else m[:, :, :nb, :nb].transpose(2, 3) if form == "transposed" else m[:, :, :nb, :nb].contiguous()
+    utils.lists_cache.clear()
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, D ** -0.5)
+    assert utils.lists_cache.seen(mask, N) is utils.UNMADE
+    lists = utils.lists_cache.get(mask, N, False)
+    assert utils.lists_cache.seen(mask, N) is lists
+    ref = utils.block_mask_to_lists(mask.contiguous())
+    T = int(ref.counts[1])
+    assert torch.equal(lists.row_ptr, ref.row_ptr) and torch.equal(lists.col_idx[:T], ref.col_idx[:T])
+    o2, lse2 = fm.flash_attention_custom_mask_lse(q, k, v, mask, D ** -0.5)
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+def test_forward_from_the_mask_is_refused_where_lists_are_needed(dev):
+    import ctypes
+    from fa2_custom_mask import _ext
+    l = _ext.lib()
+    assert l.bsattn_fwd_takes_mask(1, 1, 1024, 64) == 1 and l.bsattn_fwd_takes_mask(1, 1, 17536, 64) == 0
+    assert l.bsattn_fwd_takes_mask(1, 1, 32768, 128) == 1 and l.bsattn_fwd_takes_mask(1, 1, 32769, 128) == 0
+    assert l.bsattn_fwd_takes_mask(1, 1, 1024, 96) == 0
+    P, s = ctypes.c_void_p(4096), (ctypes.c_int64 * 4)(17536 * 64, 17536 * 64, 64, 1)      # (never dereferenced)
+    call = lambda block, N, ws: l.bsattn_fwd_mask_tokens(P, P, P, P, None, block, s, 1, 1, 1, 1, N, 64, 0, 0, 0.1, s, s, s, s, P, ws, None)
+    assert call(P, 17536, 1 << 40) == -8 and call(None, 1024, 1 << 40) == -1 and call(P, 1024, 16) == -6 and call(P, 0, 1 << 40) == -2
