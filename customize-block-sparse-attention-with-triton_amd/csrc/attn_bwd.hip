@@ -38,6 +38,8 @@ struct BwdParams {
   float sm_scale, qk_scale;   // qk_scale = sm_scale * log2(e)
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];
   int64_t dqs[3], dks[3], dvs[3];   // batch, head, row strides of the results (elements)
+  PlaceOfEight place;         // workgroup -> (head, list, share)
+  Divisor per_batch;          // H
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -178,15 +180,6 @@ __device__ __forceinline__ floatx16 zero16() {
 __device__ __forceinline__ void settle(uintx4& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void settle(float& x) { asm volatile("" : "+v"(x)); }
 
-// Workgroup -> (head, block) for the walking kernels: heads in groups of 8, one head per XCD (place.h), so that the tiles a
-// head's workgroups walk over (K and V, or Q and dO, of that head) are shared in one L2 instead of being fetched into
-// all of them.
-__device__ __forceinline__ void head_and_block(int L, int BH, int nb, int& bh, int& blk) {
-  const Place p = place(L, BH, XCDS, nb);
-  bh = p.head;
-  blk = p.item;          // >= nb for the padding of an incomplete last group
-}
-
 // Is the list at lp, lp + 1 so short that the first share's workgroup walks all of it?  (The pointer as a value the
 // compiler cannot trace back, or it makes these loads, and waits for them, in the workgroups of the first share too.)
 __device__ __forceinline__ bool walked_by_first(cint_ptr_t lp, int whole) {
@@ -230,13 +223,11 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb;
-  int bh, blk;
-  const int per_chunk = gridDim.x / prm.split;               // chunk = slowest index: head i of a group stays on XCD i
-  const int chunk = blockIdx.x / per_chunk;
-  head_and_block(blockIdx.x - chunk * per_chunk, prm.B * prm.H, nb, bh, blk);
-  if (blk >= nb) return;
-  const int m = nb - 1 - blk;                 // long rows of block-causal masks first
-  const int b = bh / prm.H, h = bh % prm.H;
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);   // heads in groups of 8, one per XCD: the tiles its workgroups walk are shared in one L2
+  if (p.item >= nb) return;
+  const int bh = p.head, m = nb - 1 - p.item;        // long rows of block-causal masks first
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
@@ -415,12 +406,11 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb;
-  int bh, n;                                  // early columns of block-causal masks are the long ones
-  const int per_chunk = gridDim.x / prm.split;
-  const int chunk = blockIdx.x / per_chunk;
-  head_and_block(blockIdx.x - chunk * per_chunk, prm.B * prm.H, nb, bh, n);
-  if (n >= nb) return;
-  const int b = bh / prm.H, h = bh % prm.H;
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);   // (as in dq_kernel; early columns of block-causal masks are the long ones)
+  if (p.item >= nb) return;
+  const int bh = p.head, n = p.item;
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
@@ -668,12 +658,11 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
   const int kh = wv & 1, dh = wv >> 1;
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb;
-  int bh, n;
-  const int per_chunk = gridDim.x / prm.split;
-  const int chunk = blockIdx.x / per_chunk;
-  head_and_block(blockIdx.x - chunk * per_chunk, prm.B * prm.H, nb, bh, n);
-  if (n >= nb) return;
-  const int b = bh / prm.H, h = bh % prm.H;
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);   // (as in dq_kernel; early columns of block-causal masks are the long ones)
+  if (p.item >= nb) return;
+  const int bh = p.head, n = p.item;
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t cp = (cint_ptr_t)(uintptr_t)(prm.col_ptr + (int64_t)mh * nb);
   const cint_ptr_t rows = (cint_ptr_t)(uintptr_t)prm.row_idx;
@@ -1021,7 +1010,7 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
     }
   });
   const int BH = prm.B * prm.H;
-  const int grid = placed(BH, XCDS, prm.nb) * prm.split;   // heads in groups of 8, the last group padded
+  const int grid = prm.place.per_share * prm.split;
   hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
   if constexpr (D == 64) hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);
@@ -1047,6 +1036,8 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   const BwdShares shares = bwd_shares(s.B, s.H, s.N, s.D, bits_rows != nullptr);
   prm.split = shares.split;
   prm.whole = shares.whole;
+  prm.place = place_of_eight(s.B * s.H, prm.nb, prm.split);
+  prm.per_batch = divisor((unsigned)s.H, (uint64_t)s.B * s.H);
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
     prm.part_dq = (float*)ws + delta_floats(s.B, s.H, s.N);

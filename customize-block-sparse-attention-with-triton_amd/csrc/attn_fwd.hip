@@ -35,7 +35,6 @@
 #include "fwd_split.h"
 #include "fwd_tile.h"
 #include "kernel_util.h"
-#include "place.h"
 #include "range_perm.h"
 #include "row_parts.h"
 
@@ -78,9 +77,11 @@ template <int D> struct FwdCfg {
 // row block beyond N repeat the last query and are not written.
 enum { GENERAL = 0, CONTIG_WHOLE = 1, CONTIG_TAIL = 2 };
 enum { COOP = 0, ROWS_MODE = 1, WAVE = 2 };
-template <int D, int DT, int MODE, bool EW, int LAYOUT>
+// SPREAD: COOP and WAVE with a number of heads that does not divide 8 (place_range).  A variant of its own: the code of the other
+// way in the prologue, even where it is jumped over, costs a launch of one head 0.3 us and eight heads 0.7 %.
+template <int D, int DT, int MODE, bool EW, int LAYOUT, bool SPREAD>
 __global__ __launch_bounds__(MODE != COOP ? 64 : FwdCfg<D>::NW * 64, FwdCfg<D>::WG_PER_CU)
-void fwd_kernel(const FwdParams prm) {
+void fwd_kernel(const FwdRangeParams prm) {
   constexpr bool BF16 = DT != 0, PB = DT == 2;
   constexpr bool CONTIG = LAYOUT == CONTIG_WHOLE || LAYOUT == CONTIG_TAIL, TAIL = LAYOUT == GENERAL || LAYOUT == CONTIG_TAIL;
   using C = FwdCfg<D>;
@@ -113,15 +114,15 @@ void fwd_kernel(const FwdParams prm) {
     if (p.item >= per) return;                   // padding of the last group
     bh = p.head;
     wg = per - 1 - p.item + (extra ? nb : 0);
-  } else if (prm.place_fast < 0) {
-    bh = blockIdx.x % BH;
-    wg = blockIdx.x / BH;
-  } else {
+  } else if constexpr (SPREAD) {
     const Place p = place_range(blockIdx.x, BH, prm.W, prm.place_fast, prm.place_quot, prm.place_rest);
     bh = p.head;
     wg = p.item;
+  } else {      // (1, 2, 4 or 8 heads)
+    bh = blockIdx.x & (BH - 1);
+    wg = blockIdx.x >> __builtin_ctz(BH);
   }
-  const int b = bh / prm.H, h = bh % prm.H;
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   // keys of the last tile column; its column block (-1: every tile is whole)
   const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64;
@@ -1451,21 +1452,29 @@ size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_b
 
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
 void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st);   // attn_fwd_short.hip
-template <int D, int DT, int MODE, bool EW, int LAYOUT>
-static void launch_fwd_c(const FwdParams& prm, int grid, hipStream_t st) {
+template <int D, int DT, int MODE, bool EW, int LAYOUT, bool SPREAD>
+static void launch_fwd_s(const FwdRangeParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
   constexpr int LDS = MODE != COOP ? C::ROWS_LDS_BYTES : C::LDS_BYTES;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<D, DT, MODE, EW, LAYOUT>),
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<D, DT, MODE, EW, LAYOUT, SPREAD>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   });
-  hipLaunchKernelGGL((fwd_kernel<D, DT, MODE, EW, LAYOUT>), dim3(grid), dim3(MODE != COOP ? 64 : C::NW * 64), LDS, st, prm);
+  hipLaunchKernelGGL((fwd_kernel<D, DT, MODE, EW, LAYOUT, SPREAD>), dim3(grid), dim3(MODE != COOP ? 64 : C::NW * 64), LDS, st, prm);
+}
+
+template <int D, int DT, int MODE, bool EW, int LAYOUT>
+static void launch_fwd_c(const FwdRangeParams& prm, int grid, hipStream_t st) {
+  if constexpr (MODE != ROWS_MODE) {
+    if (XCDS % (prm.B * prm.H) != 0) { launch_fwd_s<D, DT, MODE, EW, LAYOUT, true>(prm, grid, st); return; }
+  }
+  launch_fwd_s<D, DT, MODE, EW, LAYOUT, false>(prm, grid, st);
 }
 
 // (The copies with immediate offsets are 2-4 % faster.)
 template <int DT, int MODE, bool EW>
-static void launch_fwd_t(const FwdParams& prm, int grid, hipStream_t st) {
+static void launch_fwd_t(const FwdRangeParams& prm, int grid, hipStream_t st) {
   const bool contig = prm.ks[2] == 64 && prm.vs[2] == 64, whole = prm.N % 64 == 0;
   if (contig && whole) launch_fwd_c<64, DT, MODE, EW, CONTIG_WHOLE>(prm, grid, st);
   else if (contig) launch_fwd_c<64, DT, MODE, EW, CONTIG_TAIL>(prm, grid, st);
@@ -1473,14 +1482,14 @@ static void launch_fwd_t(const FwdParams& prm, int grid, hipStream_t st) {
 }
 
 template <int MODE, bool EW>
-static void launch_fwd_m(const FwdParams& prm, int dt, int grid, hipStream_t st) {
+static void launch_fwd_m(const FwdRangeParams& prm, int dt, int grid, hipStream_t st) {
   if (dt == 0) launch_fwd_t<0, MODE, EW>(prm, grid, st);
   else if (dt == 1) launch_fwd_t<1, MODE, EW>(prm, grid, st);
   else launch_fwd_t<2, MODE, EW>(prm, grid, st);
 }
 
 template <bool EW>
-static void launch_fwd_d(const FwdParams& prm, int mode, int dt, hipStream_t st) {
+static void launch_fwd_d(const FwdRangeParams& prm, int mode, int dt, hipStream_t st) {
   const int BH = prm.B * prm.H, grid = prm.W * BH;
   if (mode == ROWS_MODE) launch_fwd_m<ROWS_MODE, EW>(prm, dt, placed(BH, prm.group, prm.nb) + placed(BH, prm.group, prm.W), st);
   else if (mode == WAVE) launch_fwd_m<WAVE, EW>(prm, dt, grid, st);
@@ -1528,13 +1537,14 @@ static bool range_permutation(int nb, int W, int F, int BH, unsigned short* out,
 int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                const int32_t* row_ptr, const int32_t* col_idx, const uint8_t* tile_partial,
                const uint64_t* tile_bits, const AttnShape& s, void* ws, hipStream_t st) {
-  FwdParams prm;
+  FwdRangeParams prm;
   prm.q = q; prm.k = k; prm.v = v; prm.o = o; prm.lse = lse;
   prm.mask = s.mask;
   for (int i = 0; i < 4; ++i) prm.ms[i] = s.mask != nullptr ? s.ms[i] : 0;
   prm.row_ptr = row_ptr; prm.col_idx = col_idx; prm.ws = (float*)ws;
   prm.tile_partial = tile_partial; prm.tile_bits = (const unsigned long long*)tile_bits;
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
+  prm.per_batch = divisor((unsigned)s.H, (uint64_t)s.B * s.H);
   prm.out_f32 = s.out_dtype == BSATTN_F32;
   prm.qk_scale = s.sm_scale * 1.4426950408889634f;
   for (int i = 0; i < 3; ++i) { prm.qs[i] = s.qs[i]; prm.ks[i] = s.ks[i]; prm.vs[i] = s.vs[i]; prm.os[i] = s.os[i]; }
@@ -1544,6 +1554,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
   if (s.D != 64 || plan.pairs > 0) {
     prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr);
+    prm.place = place_of_eight(heads, prm.nb, prm.split);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
     prm.part_len = (int*)(prm.part_ml + (size_t)prm.split * heads * s.N * 2);
@@ -1561,7 +1572,6 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.place_fast = mode == COOP ? std::min(compute_units(), prm.W * heads) : 0;
   prm.place_quot = prm.place_fast / heads;
   prm.place_rest = prm.place_fast % heads;
-  if (XCDS % heads == 0) prm.place_fast = -1;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();

@@ -16,7 +16,6 @@
 #include "common.h"
 #include "fwd_tile.h"
 #include "kernel_util.h"
-#include "place.h"
 
 namespace bsattn {
 
@@ -46,16 +45,11 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb, BH = prm.B * prm.H;
   // linear id -> (head, row block): groups of 8 heads, one head per XCD (place.h), long row blocks first
-  int bh, m;
-  const int per_chunk = gridDim.x / prm.split;    // chunk = slowest index: head i of a group stays on XCD i
-  const int chunk = blockIdx.x / per_chunk;
-  {
-    const Place p = place(blockIdx.x - chunk * per_chunk, BH, XCDS, nb);
-    bh = p.head;
-    m = nb - 1 - p.item;
-    if (m < 0) return;                           // padding of an incomplete last group
-  }
-  const int b = bh / prm.H, h = bh % prm.H;
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);
+  const int bh = p.head, m = nb - 1 - p.item;
+  if (m < 0) return;                             // padding of an incomplete last group
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   // Q of this lane's query (second operand of S^T = K Q^T) depends on the block index only: asked for first, it
@@ -457,8 +451,7 @@ static void launch_pair_c(const FwdParams& prm, int grid, hipStream_t st) {
 
 template <int D, int DT, bool EW>
 static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
-  const int BH = prm.B * prm.H;
-  const int grid = placed(BH, XCDS, prm.nb) * prm.split;
+  const int grid = prm.place.per_share * prm.split;
   // (the variant with immediate copy offsets: 5 % faster at D = 256, 3 % slower on dense masks at D = 128)
   if (prm.N % 64 != 0) launch_pair_c<D, DT, EW, false, true>(prm, grid, st);
   else if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256, false>(prm, grid, st);

@@ -16,7 +16,6 @@
 #include "common.h"
 #include "fwd_tile.h"
 #include "kernel_util.h"
-#include "place.h"
 
 namespace bsattn {
 
@@ -46,12 +45,11 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = wave >> 1, w = wave & 1;
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb, BH = prm.B * prm.H;
-  const int per_chunk = gridDim.x / prm.split;    // chunk = slowest index: a head stays on its XCD
-  const int chunk = prm.split > 1 ? blockIdx.x / per_chunk : 0;
-  const Place p = place(blockIdx.x - chunk * per_chunk, BH, XCDS, nb);
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);
   const int bh = p.head, m = nb - 1 - p.item;
   if (m < 0) return;                              // padding of an incomplete last group
-  const int b = bh / prm.H, h = bh - b * prm.H;
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   // Q of this lane's query depends on the block index only: asked for first, it travels while the list is looked up
@@ -316,7 +314,7 @@ static void launch_short_t(const FwdParams& prm, hipStream_t st) {
   once_per_device(configured, [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_short_kernel<S, DT, EW, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   });
-  const int grid = placed(prm.B * prm.H, XCDS, prm.nb) * prm.split;
+  const int grid = prm.place.per_share * prm.split;
   hipLaunchKernelGGL((fwd_short_kernel<S, DT, EW, TAIL>), dim3(grid), dim3(128 * S), LDS, st, prm);
 }
 

@@ -3,6 +3,7 @@
 #pragma once
 #include "common.h"
 #include "kernel_util.h"
+#include "place.h"
 
 namespace bsattn {
 
@@ -25,11 +26,17 @@ struct FwdParams {
   int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
-  int place_fast, place_quot, place_rest;   // COOP, WAVE: place_range's arguments (place_fast < 0: heads interleaved)
+  int place_fast, place_quot, place_rest;   // SPREAD: place_range's arguments
   int group;                    // ROWS: heads whose row blocks go out together
   int out_f32;
   float qk_scale;  // sm_scale * log2(e)
   int64_t qs[3], ks[3], vs[3], os[3];
+  PlaceOfEight place;              // kernels whose workgroups have a row block each
+  Divisor per_batch;               // H
+};
+
+// fwd_kernel's
+struct FwdRangeParams : FwdParams {
   // fwd_kernel: which range of its head workgroup wg takes, for heads with at least perm_min_tiles kept tiles that
   // are cut into exactly perm_n ranges, the first perm_fast of them with the larger weight (perm_n = 0: none; see
   // range_permutation)

@@ -15,6 +15,14 @@ int main() {
         std::vector<std::vector<int>> of_xcd(XCDS, std::vector<int>(heads));
         for (int L = 0; L < placed(heads, group, items); ++L) {
           const Place p = place(L, heads, group, items);
+          if (group == XCDS) {
+            const PlaceOfEight e = place_of_eight(heads, items, 3);
+            for (int share = 0; share < 3; ++share) {
+              int got = -1;
+              const Place same = e.of(L + share * e.per_share, got);
+              if (got != share || same.head != p.head || same.item != p.item) return bad("eight", heads, items, L);
+            }
+          }
           if (p.item >= items) continue;
           if (p.head < 0 || p.head >= heads || p.item < 0 || seen[p.head * items + p.item]++) return bad("group", heads, group, items);
           of_xcd[L % XCDS][p.head] = 1;
@@ -27,6 +35,13 @@ int main() {
           if (n > heads / XCDS + 2) return bad("heads of an XCD", heads, group, items);
         }
       }
+  for (unsigned d : {1u, 2u, 3u, 5u, 6u, 7u, 8u, 24u, 513u, 2192u, 65535u, 1u << 20})
+    for (uint64_t most : {10ull, 1000ull, 65535ull, 1ull << 20, 1ull << 31}) {
+      const Divisor v = divisor(d, most);
+      const uint64_t at[] = {0, 1, d - 1, d, d + 1, most / 2, most - 1, most, most / d * d, most / d * d - 1};
+      for (uint64_t n : at) if (n <= most && v.of((unsigned)n) != (unsigned)n / d) return bad("division", (int)d, (int)n, (int)most);
+      for (uint64_t n = 0; n <= most && n < 100000; ++n) if (v.of((unsigned)n) != (unsigned)n / d) return bad("division", (int)d, (int)n, (int)most);
+    }
   for (int heads = 1; heads <= 600; ++heads)
     for (int slots : {256, 512, 2048, 250})
       for (int cap : {1, 3, 100, 100000})
