@@ -16,169 +16,12 @@
 // dq_kernel, P and dS leave the first products already in the operand layout of the second
 // ones, and the tiles that change per step are staged in LDS by asynchronous copies into a
 // double buffer (one barrier per tile).
-#include "common.h"
-#include "kernel_util.h"
-#include "place.h"
+// (D = 64 with few lists: attn_bwd_short.hip.)
+#include <algorithm>
+#include "bwd_tile.h"
 #include <type_traits>
 
 namespace bsattn {
-
-struct BwdParams {
-  const void* q; const void* k; const void* v; const void* o; const void* d_o;
-  const float* lse; float* delta;
-  void* dq; void* dk; void* dv;
-  const int32_t* row_ptr; const int32_t* col_idx; const int32_t* col_ptr; const int32_t* row_idx;
-  // elementwise masks: 64 words per entry of the row lists (bit = key) / of the column lists (bit = query)
-  const unsigned long long* bits_rows; const unsigned long long* bits_cols;
-  int B, H, N, nb, Bm, Hm;
-  int out_f32;
-  int split;                  // workgroups per row / column list (1: results written directly)
-  int whole;                  // split > 1: lists of up to this many tiles are one workgroup's all the same (-1: none)
-  float* part_dq; float* part_dk; float* part_dv;   // split > 1: fp32 partial results [split][B*H][N][D]
-  float sm_scale, qk_scale;   // qk_scale = sm_scale * log2(e)
-  int64_t qs[3], ks[3], vs[3], os[3], dos[3];
-  int64_t dqs[3], dks[3], dvs[3];   // batch, head, row strides of the results (elements)
-  PlaceOfEight place;         // workgroup -> (head, list, share)
-  Divisor per_batch;          // H
-};
-
-constexpr float kLog2e = 1.4426950408889634f;
-
-// sum of the products of the eight 16-bit elements of a and b
-template <bool BF16>
-__device__ __forceinline__ float dot8(const uintx4& a, const uintx4& b, float acc) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float a0, a1, b0, b1;
-    const unsigned int au = a[i], bu = b[i];   // by value: bit_cast of a vector element lvalue miscompiles
-    if constexpr (BF16) {
-      a0 = __builtin_bit_cast(float, au << 16); a1 = __builtin_bit_cast(float, au & 0xffff0000u);
-      b0 = __builtin_bit_cast(float, bu << 16); b1 = __builtin_bit_cast(float, bu & 0xffff0000u);
-    } else {
-      const half2v ah = __builtin_bit_cast(half2v, au), bhh = __builtin_bit_cast(half2v, bu);
-      a0 = (float)ah[0]; a1 = (float)ah[1]; b0 = (float)bhh[0]; b1 = (float)bhh[1];
-    }
-    acc += a0 * b0 + a1 * b1;
-  }
-  return acc;
-}
-
-// ---------------------------------------------------------------------------------------
-// helpers of the two walking kernels
-// ---------------------------------------------------------------------------------------
-// ROWS: rows of a tile staged per step (64, or 32 when a tile is walked in two halves)
-template <int D, bool EW, int ROWS = 64> struct BwdCfg {
-  static constexpr int TILE_BYTES = ROWS * 2 * D;
-  static constexpr int STAT_BYTES = 2 * 64 * 4;                    // lse2[64] + delta[64] of a row block
-  static constexpr int BITS_BYTES = EW ? 64 * 8 : 0;               // mask words of the tile (elementwise masks)
-  static constexpr int STAGE_BYTES = 2 * TILE_BYTES + STAT_BYTES + BITS_BYTES;  // two tiles, row statistics, mask words
-  static constexpr int LDS_BYTES = 2 * STAGE_BYTES;                // double buffer
-};
-
-// This wavefront's half of the asynchronous copy of a ROWS x D tile (rows `stride` elements apart)
-// into LDS with the u_swz chunk swizzle: wavefront wv issues half of the ROWS*D/512 instructions.
-template <int D, int ROWS = 64>
-__device__ __forceinline__ void half_tile_load_async(const unsigned short* tile, int64_t stride, int wv, int lane,
-                                                     unsigned lds_addr) {
-  constexpr int CPR = D / 8, PER_WAVE = ROWS * CPR / 128;
-#pragma unroll
-  for (int jj = 0; jj < PER_WAVE; ++jj) {
-    const int j = wv * PER_WAVE + jj;
-    const int c = j * 64 + lane, row = c / CPR, ch = c % CPR;
-    const unsigned off = 2u * (unsigned)(row * (int)stride + ((ch ^ u_swz<D>(row)) * 8));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(lds_addr + j * 1024), "v"(off), "s"(tile) : "memory", "m0");
-  }
-}
-
-// The same for rows first .. first + ROWS - 1 of a tile of which only `valid` rows exist (N is not a multiple of 64):
-// the last one is repeated in place of the others, so that no address lies beyond the tensor.  tile: row 0 of it.
-// (The lane index as a value the compiler cannot trace back: the offsets would otherwise be computed before the
-// walk and held through it.)
-template <int NWV, int D, int ROWS>
-__device__ __forceinline__ void tail_tile_load_async(const unsigned short* tile, int64_t stride, int first, int valid, int wv,
-                                                     int lane, unsigned lds_addr) {
-  constexpr int CPR = D / 8, PER_WAVE = ROWS * CPR / (64 * NWV);
-  asm volatile("" : "+v"(lane));
-#pragma unroll 1
-  for (int j = wv * PER_WAVE; j < (wv + 1) * PER_WAVE; ++j) {
-    const int c = j * 64 + lane, row = c / CPR, ch = c % CPR, src = first + row < valid ? first + row : valid - 1;
-    tile_load_async_one(tile, 2u * (unsigned)(src * (int)stride + ((ch ^ u_swz<D>(row)) * 8)), lds_addr + j * 1024);
-  }
-}
-
-// Mask word of a lane in such a tile, shifted for mask_scores: bit = row or column of the tile, set for the first
-// `valid` < 64.  (From a value the compiler cannot trace back, or its tests are made before the walk and held.)
-__device__ __forceinline__ unsigned long long tail_word(int valid, int g) {
-  asm volatile("" : "+s"(valid));
-  return ((1ull << valid) - 1ull) >> (4 * g);
-}
-
-// asynchronous copy of 64 consecutive floats (one per lane)
-__device__ __forceinline__ void stat_load_async(const float* src, int lane, unsigned lds_addr) {
-  const unsigned off = 4u * (unsigned)lane;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds_addr), "v"(off), "s"(src) : "memory", "m0");
-}
-
-// operand fragment (32 rows x 16 columns slice s) of a swizzled LDS tile: row r0 + ln, chunk 2s + g
-template <int D>
-__device__ __forceinline__ uintx4 frag_rows(const unsigned char* tile, int r0, int s, int ln, int g) {
-  const int row = r0 + ln;
-  return *reinterpret_cast<const uintx4*>(tile + row * 2 * D + (((2 * s + g) ^ u_swz<D>(row)) * 16));
-}
-
-// transposed operand fragment: columns 32db + ln of the tile along the lanes, contraction slots j
-// of slice ts <-> tile rows 16ts + 8(j/4) + 4g + (j%4) (the order in which a 32x32 MFMA result
-// holds its rows), by two LDS transpose reads
-template <int D, bool BF16>
-__device__ __forceinline__ uintx4 frag_cols(const unsigned char* tile, int db, int ts, int lane) {
-  const int blk = lane >> 4, s16 = lane & 15;
-  uintx4 a;
-#pragma unroll
-  for (int jh = 0; jh < 2; ++jh) {
-    const int row = 16 * ts + 8 * jh + 4 * (blk >> 1) + (s16 >> 2);
-    const int col = 32 * db + 16 * (blk & 1) + 4 * (s16 & 3);
-    const int addr = row * 2 * D + (((col >> 3) ^ u_swz<D>(row)) * 16) + (col & 7) * 2;
-    const short4v rr = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4v __attribute__((address_space(3)))*)(tile + addr));
-    const uintx2 r2 = __builtin_bit_cast(uintx2, rr);
-    a[2 * jh] = r2[0]; a[2 * jh + 1] = r2[1];
-  }
-  if constexpr (BF16) a = bf16x8_to_f16x8(a);
-  return a;
-}
-
-// scores of unset mask elements become -inf; mw: the 64 mask bits of this lane's row, already
-// shifted right by 4 g, so that bit 8(i/4) + i%4 (+ 32 for the second block) belongs to register i
-__device__ __forceinline__ void mask_scores(floatx16& s0, floatx16& s1, unsigned long long mw) {
-  const unsigned lo = (unsigned)mw, hi = (unsigned)(mw >> 32);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const unsigned bit = 1u << (8 * (i / 4) + (i % 4));
-    s0[i] = (lo & bit) ? s0[i] : -INFINITY;
-    s1[i] = (hi & bit) ? s1[i] : -INFINITY;
-  }
-}
-
-// the same for one block of 32 keys (bits 0..31 of the shifted word)
-__device__ __forceinline__ void mask_scores(floatx16& s0, unsigned lo) {
-#pragma unroll
-  for (int i = 0; i < 16; ++i) s0[i] = (lo & (1u << (8 * (i / 4) + (i % 4)))) ? s0[i] : -INFINITY;
-}
-
-__device__ __forceinline__ floatx16 zero16() {
-  floatx16 z;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) z[i] = 0.f;
-  return z;
-}
-
-
-// Values that live in registers through a walking loop (fragments of the stationary operand, row statistics) are
-// passed through here once they have been asked for: the compiler waits for their loads at this point.  Left to
-// itself it moves the loads next to the loop and plants its waits at their first uses inside it, where, being
-// counted waits, they also wait for the tile copies of the next step that have just been issued, in every step.
-__device__ __forceinline__ void settle(uintx4& x) { asm volatile("" : "+v"(x)); }
-__device__ __forceinline__ void settle(float& x) { asm volatile("" : "+v"(x)); }
 
 // Is the list at lp, lp + 1 so short that the first share's workgroup walks all of it?  (The pointer as a value the
 // compiler cannot trace back, or it makes these loads, and waits for them, in the workgroups of the first share too.)
@@ -962,6 +805,7 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 //            14 heads N = 1792              60 /  -  /  68                   105 /  -  /  92            121 /  -  / 135   (one share there)
 // (Elementwise masks, 8 heads N = 4000, a training step: window of 1000 135 / 156 / 140, of 2000 212 / 218 / 226,
 // token-causal 316 / 291 / 287: one share from 1.33 lists per compute unit on.)
+// (D = 64: what bwd_short_kernel does not take; the workspace has room for these shares all the same.)
 struct BwdShares { int split, whole; };
 static BwdShares bwd_shares(int B, int H, int N, int D, bool elementwise) {
   const int64_t lists = (int64_t)B * H * ((N + 63) / 64), cus = compute_units();
@@ -979,14 +823,48 @@ static BwdShares bwd_shares(int B, int H, int N, int D, bool elementwise) {
   return {(int)(s > 8 ? 8 : s < 1 ? 1 : s), -1};
 }
 
+// Which launches bwd_short_kernel (D = 64) takes: pairs of wavefronts per workgroup (0: none) and shares of a list.  us of a backward,
+// the two kernels with their shares and sums / 2 pairs / 4 pairs / 2 pairs, 2 shares / 4 pairs, 2 shares; fp16, keep 0.1, 0.3, 1, causal:
+//    4 heads N = 512 (32 lists)     15 /  9 / 10 / 11 / 14     18 /  9 / 10 / 12 / 13     26 / 13 / 12 / 13 / 14     25 / 13 / 12 / 13 / 13
+//    1 head  N = 3072 (48)          23 / 15 / 14 /  - / 14     28 / 24 / 21 /  - / 18     44 / 46 / 38 /  - / 28     36 / 46 / 37 /  - / 26
+//    8 heads N = 1024 (128)         23 / 11 / 11 / 20 / 24     29 / 15 / 14 / 22 / 26     36 / 22 / 19 / 26 / 30     35 / 21 / 18 / 25 / 28
+//    1 head  N = 8192 (128)         40 / 30 / 25 / 28 / 31     56 / 52 / 43 / 41 / 46     95 /128 /100 / 89 / 92     82 /118 / 91 / 78 / 72
+//    8 heads N = 2048 (256)         38 / 16 / 21 / 29 / 39     43 / 21 / 25 / 34 / 44     65 / 46 / 51 / 58 / 68     57 / 40 / 35 / 42 / 51
+//    2 heads N = 8192 (256)         50 / 35 / 36 / 41 / 53     76 / 63 / 67 / 72 / 82    162 /158 /160 /163 /174    134 /135 / 99 /106 /109
+//    1 head  N = 17536 (274)        76 / 56 / 62 / 60 /  -    159 /137 /140 /130 /  -    427 /403 /425 /373 /  -    253 /276 /227 /212 /  -    (bf16)
+//    4 heads N = 8192 (512)         68 / 53 / 65 / 71         121 /111 /123 /126         295 /302 /314 /316         237 /159 /175 /190
+//   14 heads N = 4096 (896)         79 / 55 / 76              133 /103 /129              283 /269 /298              188 /153 /174
+//   16 heads N = 4096 (1024)        55 / 60 / 85              121 /119 /146              279 /303 /334              197 /171 /191    (bf16; not there)
+//    8 heads N = 12032 (1504)      167 /156 /204              437 /407 /449             1303/1274/1343              641 /644 /699    (bf16)
+//    2 heads N = 32000 (1000)      266 /258 /286              680 /711 /750             2070/2239/2320             1073/1116/1168    (bf16; not there)
+struct BwdShort { int pairs, split; };
+static BwdShort bwd_short(int64_t lists_, int nb) {
+  const int64_t lists = lists_ * 256 / compute_units();        // (as if there were 256 compute units)
+  if (nb > BWD_SHORT_MAX_BLOCKS) return {0, 1};
+  if (lists <= 128) return {4, nb >= 90 || (lists <= 64 && nb >= 48) ? 2 : 1};
+  if (lists <= 288 && nb >= 150) return {2, 2};
+  if (lists <= 256 && nb >= 64) return {4, 1};
+  const int64_t most = nb > 300 ? 640 : nb > 128 ? 1536 : 1023;
+  return {lists <= most ? 2 : 0, 1};
+}
+
 // floats in front of the parts (the parts are accessed 16 bytes at a time)
 static size_t delta_floats(int B, int H, int N) { return ((size_t)B * H * N + 63) & ~(size_t)63; }
 
 size_t bwd_workspace_bytes(int B, int H, int N, int D) {
   const size_t delta = delta_floats(B, H, N) * sizeof(float);
   const int block = bwd_shares(B, H, N, D, false).split, words = bwd_shares(B, H, N, D, true).split;
-  const int split = block > words ? block : words;           // one size for both kinds of masks
+  int split = block > words ? block : words;                 // one size for both kinds of masks
+  if (const int nb = (N + 63) / 64; D == 64) split = std::max(split, bwd_short((int64_t)B * H * nb, nb).split);
   return delta + (split > 1 ? (size_t)3 * split * B * H * N * D * sizeof(float) : 0);   // + parts of dQ, dK, dV
+}
+
+template <bool BF16>
+static void launch_sum_parts(const BwdParams& prm, int D, hipStream_t st) {
+  const int BH = prm.B * prm.H;
+  const int64_t quads = (int64_t)BH * prm.N * D / 4;
+  const unsigned blocks = prm.whole >= 0 ? (unsigned)(BH * prm.nb * (64 / SUM_ROWS)) : (unsigned)((quads + 255) / 256);
+  hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3(blocks, 3), dim3(256), 0, st, prm, quads, D);
 }
 
 template <int D, bool BF16, bool EW, bool PB, bool TAIL>
@@ -1009,17 +887,14 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
                                 hipFuncAttributeMaxDynamicSharedMemorySize, dkdv4_lds_bytes<D>());
     }
   });
-  const int BH = prm.B * prm.H;
   const int grid = prm.place.per_share * prm.split;
   hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
   if constexpr (D == 64) hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);
-  if (prm.split > 1) {
-    const int64_t quads = (int64_t)BH * prm.N * D / 4;
-    const unsigned blocks = prm.whole >= 0 ? (unsigned)(BH * prm.nb * (64 / SUM_ROWS)) : (unsigned)((quads + 255) / 256);
-    hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3(blocks, 3), dim3(256), 0, st, prm, quads, D);
-  }
+  if (prm.split > 1) launch_sum_parts<BF16>(prm, D, st);
 }
+
+void launch_bwd_short(const BwdParams& prm, int pairs, bool bf16, bool pb, hipStream_t st);   // attn_bwd_short.hip
 
 int launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
@@ -1034,9 +909,10 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   prm.B = s.B; prm.H = s.H; prm.N = s.N; prm.nb = (s.N + 63) / 64; prm.Bm = s.Bm; prm.Hm = s.Hm;
   prm.out_f32 = s.out_dtype == BSATTN_F32;
   const BwdShares shares = bwd_shares(s.B, s.H, s.N, s.D, bits_rows != nullptr);
-  prm.split = shares.split;
-  prm.whole = shares.whole;
-  prm.place = place_of_eight(s.B * s.H, prm.nb, prm.split);
+  const BwdShort plan = s.D == 64 ? bwd_short((int64_t)s.B * s.H * prm.nb, prm.nb) : BwdShort{0, 1};
+  prm.split = plan.pairs > 0 ? plan.split : shares.split;
+  prm.whole = plan.pairs > 0 ? -1 : shares.whole;
+  prm.place = place_of_eight(s.B * s.H, prm.nb, plan.pairs > 0 ? 2 * prm.split : prm.split);
   prm.per_batch = divisor((unsigned)s.H, (uint64_t)s.B * s.H);
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
@@ -1056,6 +932,11 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   // bf16 inputs keep P and dS in fp16.
   const bool pb = bf && !prm.out_f32;
   const bool ew = bits_rows != nullptr;
+  if (plan.pairs > 0) {
+    launch_bwd_short(prm, plan.pairs, bf, pb, st);
+    if (prm.split > 1) { if (bf) launch_sum_parts<true>(prm, s.D, st); else launch_sum_parts<false>(prm, s.D, st); }
+    return launch_status();
+  }
   auto pick = [&](auto dc, auto tail) {
     constexpr int DD = decltype(dc)::value;
     constexpr bool TL = decltype(tail)::value;
