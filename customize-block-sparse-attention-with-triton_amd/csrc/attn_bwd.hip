@@ -440,6 +440,9 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
 // 128 columns of dK and dV each time: S and dP twice (6 products for 4) and every tile copied twice.  Backward, bf16:
 // 12 heads N = 4096 causal 0.5 519 -> 333 us, 16 heads N = 8192 keep 0.3 1780 -> 1540, 2 heads N = 1000 96 -> 61 (two
 // shares each).  Bound by its lone wavefront's chain: first products, exponentials, exchange, second products.
+// G = 2 (D = 128): two such groups of four wavefronts in a workgroup have half of the column's list each, and their sums are added
+// through LDS, dK by the first group and dV by the second.  (The loop is each group's own; the shorter half's group then meets the
+// two barriers of the other's last step.  With that case inside the loop the compiler held K and V in scratch.)
 // ---------------------------------------------------------------------------------------
 template <int NWV, int D, int ROWS>
 __device__ __forceinline__ void part_tile_load_async(const unsigned short* tile, int64_t stride, int wv, int lane,
@@ -489,15 +492,17 @@ __device__ __forceinline__ uintx4 three_pieces(float x, bool holder) {
 
 // two stages of a Q and a dO tile, 4 KB of exchange per wavefront, at D = 256 two stages of lse and delta
 template <int D> constexpr int dkdv4_lds_bytes() { return 4 * 64 * 2 * D + 4 * 4096 + (D == 256 ? 2 * 512 : 0); }
-template <int D, bool BF16, bool PB, bool EW, bool TAIL>
-__global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdParams prm) {
+template <int D, bool BF16, bool PB, bool EW, bool TAIL, int G = 1>
+__global__ __launch_bounds__(256 * G, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdParams prm) {
   static_assert(D == 128 || D == 256, "two or four 32-column blocks of dK and dV per wavefront");
   constexpr int KS = D / 16, DBW = D / 64;           // 32-column blocks per wavefront
   constexpr int TILE_BYTES = 64 * 2 * D, STAGE_BYTES = 2 * TILE_BYTES, EXCH_OFF = 2 * STAGE_BYTES, STAT_OFF = EXCH_OFF + 4 * 4096;
   constexpr bool PIECES = D == 128;                  // lse and delta by way of the matrix cores
   constexpr int PORTIONS = KS / 4, KSP = KS / PORTIONS;   // fragments of the first products in portions
-  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds_all[];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  unsigned char* lds = lds_all + grp * dkdv4_lds_bytes<D>();
   const int kh = wv & 1, dh = wv >> 1;
   const int ln = lane & 31, g = lane >> 5;
   const int nb = prm.nb;
@@ -528,6 +533,13 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
   {
     const int t0 = cp[n], len = cp[n + 1] - t0;                // this workgroup's share of the column's list
     split = share_of_list<by_length<D, EW>>(prm, t0, len, chunk, u0, u1);
+  }
+  int rounds = 0;            // G = 2: steps of the group with the longer half of the list, one more than the other's at most
+  if constexpr (G == 2) {
+    const int half = (u1 - u0 + 1) / 2;
+    if (grp == 0) u1 = u0 + half;
+    else u0 = u0 + half;
+    rounds = half;
   }
   const unsigned lds_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
   const unsigned short* qg = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1];
@@ -700,6 +712,48 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
     second(fgt_oth, fqt_oth, pp, dp);
   }
 
+  if (G == 2 && u1 - u0 < rounds) {  // the first group has one more step: its two barriers
+    __syncthreads();
+    __syncthreads();
+  }
+  if constexpr (G == 2) {            // the two groups' sums: the first adds up dK, the second dV
+    static_assert(D == 128, "fits");
+    __syncthreads();                 // everybody has left the last step
+    // (the lane index as a value the compiler cannot trace back, as below)
+    int lane_out = lane;
+    asm volatile("" : "+v"(lane_out));
+    floatx4* give = reinterpret_cast<floatx4*>(lds + wv * DBW * 4096);
+    const floatx4* take = reinterpret_cast<const floatx4*>(lds_all + (1 - grp) * dkdv4_lds_bytes<D>() + wv * DBW * 4096);
+    auto quads = [&](floatx16 (&mine_acc)[DBW], const floatx16 (&given)[DBW]) {
+#pragma unroll
+      for (int db = 0; db < DBW; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const floatx4 x = {given[db][4 * i4], given[db][4 * i4 + 1], given[db][4 * i4 + 2], given[db][4 * i4 + 3]};
+          give[(4 * db + i4) * 64 + lane_out] = x;
+        }
+      __syncthreads();
+#pragma unroll
+      for (int db = 0; db < DBW; ++db)
+#pragma unroll
+        for (int i4 = 0; i4 < 4; ++i4) {
+          const floatx4 x = take[(4 * db + i4) * 64 + lane_out];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) mine_acc[db][4 * i4 + e] += x[e];
+        }
+    };
+    const int64_t r0 = (int64_t)n * 64 + 32 * kh;
+    constexpr int OUT_BYTES = rows_out_bytes(32 * DBW, true);
+    static_assert(4 * (DBW * 4096 + OUT_BYTES) <= dkdv4_lds_bytes<D>(), "room for the sums and for the results of four wavefronts");
+    unsigned char* mine = lds + 4 * DBW * 4096 + wv * OUT_BYTES;
+    auto put = [&](const floatx16 (&acc)[DBW], void* out, const int64_t* st, float sc) {
+      rows_out<BF16, 32 * DBW>(mine, out, b * st[0] + h * st[1] + r0 * st[2] + 32 * DBW * dh, st[2], prm.out_f32, lane_out,
+                               TAIL ? prm.N - (int)r0 : 32, [&](int db, int i) { return acc[db][i] * sc; });
+    };
+    if (grp == 0) { quads(dkacc, dvacc); put(dkacc, prm.dk, prm.dks, prm.sm_scale); }
+    else { quads(dvacc, dkacc); put(dvacc, prm.dv, prm.dvs, 1.0f); }
+    return;
+  }
   if (split > 1) {   // unscaled fp32 parts; sum_parts_kernel adds them up
     if (!exists) return;
     const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
@@ -742,21 +796,22 @@ __global__ __launch_bounds__(256, D == 128 ? 2 : 1) void dkdv4_kernel(const BwdP
 constexpr int SUM_ROWS = 16;
 template <bool BF16>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int64_t quads, int D) {
+  const int what = blockIdx.y + prm.first_sum;
   const int qpr = D / 4;                                   // quads per row
   int64_t first = (int64_t)blockIdx.x * 256, last = quads < first + 256 ? quads : first + 256;
   if (prm.whole >= 0) {
     const int list = blockIdx.x / (64 / SUM_ROWS), unit = list / prm.nb, blk = list - unit * prm.nb;
     const int b = unit / prm.H, h = unit - b * prm.H, mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
-    const cint_ptr_t lp = (cint_ptr_t)(uintptr_t)((blockIdx.y == 0 ? prm.row_ptr : prm.col_ptr) + (int64_t)mh * prm.nb);
+    const cint_ptr_t lp = (cint_ptr_t)(uintptr_t)((what == 0 ? prm.row_ptr : prm.col_ptr) + (int64_t)mh * prm.nb);
     if (lp[blk + 1] - lp[blk] <= prm.whole) return;
     const int row0 = 64 * blk + SUM_ROWS * (blockIdx.x % (64 / SUM_ROWS)), rows = prm.N - row0 < SUM_ROWS ? prm.N - row0 : SUM_ROWS;
     first = ((int64_t)unit * prm.N + row0) * qpr;
     last = first + rows * qpr;
   }
-  const float* part = blockIdx.y == 0 ? prm.part_dq : (blockIdx.y == 1 ? prm.part_dk : prm.part_dv);
-  void* out = blockIdx.y == 0 ? prm.dq : (blockIdx.y == 1 ? prm.dk : prm.dv);
-  const int64_t* st = blockIdx.y == 0 ? prm.dqs : (blockIdx.y == 1 ? prm.dks : prm.dvs);
-  const float scale = blockIdx.y == 2 ? 1.0f : prm.sm_scale;
+  const float* part = what == 0 ? prm.part_dq : (what == 1 ? prm.part_dk : prm.part_dv);
+  void* out = what == 0 ? prm.dq : (what == 1 ? prm.dk : prm.dv);
+  const int64_t* st = what == 0 ? prm.dqs : (what == 1 ? prm.dks : prm.dvs);
+  const float scale = what == 2 ? 1.0f : prm.sm_scale;
 #pragma unroll 2
   for (int64_t i = first + threadIdx.x; i < last; i += 256) {
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -848,6 +903,42 @@ static BwdShort bwd_short(int64_t lists_, int nb) {
   return {lists <= most ? 2 : 0, 1};
 }
 
+// D = 128, few lists: dq_pairs_kernel with `dq_pairs` pairs of wavefronts per row block (0: dq_kernel), dkdv4_kernel with `groups`
+// groups of wavefronts per column block.  Two groups have the compute unit that two shares of a list would have, but add up in LDS: no
+// parts, no launch that adds them up.  `split`: the shares there would be (1: nothing to merge, one group).
+// us of a backward, bf16, as before / 2 pairs for dQ / 2 pairs, 2 groups / 4 pairs, 2 groups; keep 0.1, 0.3, 1, causal:
+//   12 heads N = 768  (144 lists)     22 / 22 / 23 / 24     30 / 28 / 29 / 30      43 / 38 / 37 / 37      43 / 38 / 37 / 37
+//    4 heads N = 1024 (64)            26 / 27 / 23 / 25     33 / 35 / 31 / 33      42 / 44 / 43 / 42      39 / 41 / 42 / 41
+//   16 heads N = 1024 (256)           43 / 38 / 25 / 26     52 / 47 / 33 / 34      67 / 61 / 47 / 47      64 / 57 / 44 / 44
+//    3 heads N = 2048 (96)            37 / 37 / 28 / 29     42 / 44 / 37 / 37      62 / 69 / 70 / 66      55 / 64 / 69 / 65     (not there)
+//    8 heads N = 2048 (256)           35 / 32 / 30 / 32     54 / 51 / 40 / 40     102 / 97 / 77 / 75      82 / 78 / 71 / 68
+//   10 heads N = 2048 (320)           44 / 41 / 44 / 52     76 / 71 / 65 / 72     122 /124 /126 /138      96 /102 / 93 / 87     (not there)
+//   14 heads N = 2048 (448)           48 / 46 / 47 / 54     79 / 69 / 70 / 76     154 /146 /130 /137     113 /112 / 97 / 93
+//    2 heads N = 4096 (128)           46 / 46 / 39 / 39     61 / 68 / 66 / 62      98 /114 /125 /115      94 /109 /123 /113     (not there)
+//    4 heads N = 4096 (256)           52 / 45 / 40 / 41     84 / 81 / 69 / 66     163 /157 /137 /131     125 /125 /125 /115
+//    5 heads N = 4096 (320)           64 / 57 / 57 / 64    108 /100 /109 /116     199 /208 /230 /246     137 /142 /132 /121     (not there)
+//    8 heads N = 4096 (512)           64 / 58 / 62 / 70    139 /125 /117 /125     277 /270 /251 /258     188 /175 /152 /145
+//   10 heads N = 4096 (640)           68 / 72 / 77 / 88    145 /144 /142 /152     372 /370 /369 /375     240 /215 /234 /235     (dQ only)
+//    2 heads N = 6144 (192)           77 / 72 / 51 / 50    104 /107 / 88 / 82     202 /203 /183 /169     140 /168 /178 /162     (not there)
+//    4 heads N = 8192 (512)          112 /104 / 90 / 95    200 /192 /176 /186     508 /501 /482 /488     335 /303 /278 /260
+//    6 heads N = 8192 (768)          152 /145 /125 /134    300 /294 /271 /274     815 /770 /747 /754     448 /419 /404 /420
+//    1 head  N = 16384 (256)         107 /105 / 88 / 85    209 /216 /200 /189     525 /542 /521 /497     366 /413 /472 /428     (not there)
+//    2 heads N = 16384 (512)         168 /161 /145 /155    361 /355 /348 /357    1002 /993 /977 /987     639 /584 /563 /520
+//    8 heads N = 8192 (1024)         140 /147 /162 /177    336 /337 /343 /362     943 /944 /952 /970     558 /520 /509 /515     (not there)
+// So: enough lists that nobody needs more than two streams of a long one, and not a bit more than one list per compute unit, which
+// would be a second round of workgroups that fill it.  Token masks, 8 heads N = 4000: window of 1000 84 / 80 / 86 / 94, causal 301 / 263 / 242 / 236.
+struct BwdPairs { int dq_pairs, groups; };
+static BwdPairs bwd_pairs_128(int64_t lists_, int nb, int split) {
+  const int64_t lists = lists_ * 256 / compute_units();        // (as if there were 256 compute units)
+  if (nb < 12 || nb > BWD_SHORT_MAX_BLOCKS) return {0, 1};
+  if (split > 1) {
+    const int64_t least = nb <= 64 ? std::min(4 * nb, 192) : nb <= 128 ? 256 : 2 * nb, most = nb >= 96 && nb <= 128 ? 768 : 512;
+    if (lists >= least && lists <= most && (nb < 32 || lists <= 256 || lists >= 384)) return {lists <= 256 && nb >= 32 ? 4 : 2, 2};
+    if (lists <= most) return {0, 1};
+  }
+  return {lists <= 800 ? 2 : 0, 1};
+}
+
 // floats in front of the parts (the parts are accessed 16 bytes at a time)
 static size_t delta_floats(int B, int H, int N) { return ((size_t)B * H * N + 63) & ~(size_t)63; }
 
@@ -864,11 +955,11 @@ static void launch_sum_parts(const BwdParams& prm, int D, hipStream_t st) {
   const int BH = prm.B * prm.H;
   const int64_t quads = (int64_t)BH * prm.N * D / 4;
   const unsigned blocks = prm.whole >= 0 ? (unsigned)(BH * prm.nb * (64 / SUM_ROWS)) : (unsigned)((quads + 255) / 256);
-  hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3(blocks, 3), dim3(256), 0, st, prm, quads, D);
+  hipLaunchKernelGGL((sum_parts_kernel<BF16>), dim3(blocks, 3 - prm.first_sum), dim3(256), 0, st, prm, quads, D);
 }
 
 template <int D, bool BF16, bool EW, bool PB, bool TAIL>
-static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
+static void launch_bwd_t(const BwdParams& prm, int groups, hipStream_t st) {
   using C = BwdCfg<D, EW>;
   constexpr int KB = D >= 128 ? 1 : 2;          // dq_kernel walks D >= 128 tiles in two halves (no gain at D = 64: two wavefronts per SIMD anyway)
   using CQ = BwdCfg<D, EW, 32 * KB>;
@@ -885,16 +976,26 @@ static void launch_bwd_t(const BwdParams& prm, hipStream_t st) {
     } else {
       (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW, TAIL>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, dkdv4_lds_bytes<D>());
+      if constexpr (D == 128)
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dkdv4_kernel<D, BF16, PB, EW, TAIL, 2>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, 2 * dkdv4_lds_bytes<D>());
     }
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
+  if (prm.first_sum == 0) hipLaunchKernelGGL((dq_kernel<D, BF16, EW, PB, KB, TAIL>), dim3(grid), dim3(128), CQ::LDS_BYTES, st, prm);
+  if constexpr (D == 128) {
+    if (groups == 2) {
+      hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL, 2>), dim3(grid), dim3(512), 2 * dkdv4_lds_bytes<D>(), st, prm);
+      return;                                   // (one share of a list)
+    }
+  }
   if constexpr (D == 64) hipLaunchKernelGGL((dkdv_kernel<D, BF16, EW, PB, TAIL>), dim3(grid), dim3(128), CK::LDS_BYTES, st, prm);
   else hipLaunchKernelGGL((dkdv4_kernel<D, BF16, PB, EW, TAIL>), dim3(grid), dim3(256), dkdv4_lds_bytes<D>(), st, prm);
   if (prm.split > 1) launch_sum_parts<BF16>(prm, D, st);
 }
 
 void launch_bwd_short(const BwdParams& prm, int pairs, bool bf16, bool pb, hipStream_t st);   // attn_bwd_short.hip
+void launch_dq_pairs(const BwdParams& prm, int pairs, bool bf16, bool pb, hipStream_t st);
 
 int launch_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
@@ -910,9 +1011,12 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   prm.out_f32 = s.out_dtype == BSATTN_F32;
   const BwdShares shares = bwd_shares(s.B, s.H, s.N, s.D, bits_rows != nullptr);
   const BwdShort plan = s.D == 64 ? bwd_short((int64_t)s.B * s.H * prm.nb, prm.nb) : BwdShort{0, 1};
-  prm.split = plan.pairs > 0 ? plan.split : shares.split;
-  prm.whole = plan.pairs > 0 ? -1 : shares.whole;
+  const BwdPairs pairs = s.D == 128 ? bwd_pairs_128((int64_t)s.B * s.H * prm.nb, prm.nb, shares.split) : BwdPairs{0, 1};
+  prm.split = plan.pairs > 0 ? plan.split : pairs.groups > 1 ? 1 : shares.split;
+  prm.whole = plan.pairs > 0 || pairs.groups > 1 ? -1 : shares.whole;
   prm.place = place_of_eight(s.B * s.H, prm.nb, plan.pairs > 0 ? 2 * prm.split : prm.split);
+  prm.place_dq = place_of_eight(s.B * s.H, prm.nb, 1);
+  prm.first_sum = pairs.dq_pairs > 0 ? 1 : 0;
   prm.per_batch = divisor((unsigned)s.H, (uint64_t)s.B * s.H);
   {
     const size_t one = (size_t)prm.split * s.B * s.H * s.N * s.D;
@@ -937,17 +1041,18 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
     if (prm.split > 1) { if (bf) launch_sum_parts<true>(prm, s.D, st); else launch_sum_parts<false>(prm, s.D, st); }
     return launch_status();
   }
+  if (pairs.dq_pairs > 0) launch_dq_pairs(prm, pairs.dq_pairs, bf, pb, st);
   auto pick = [&](auto dc, auto tail) {
     constexpr int DD = decltype(dc)::value;
     constexpr bool TL = decltype(tail)::value;
     if (!ew) {
-      if (!bf) launch_bwd_t<DD, false, false, false, TL>(prm, st);
-      else if (pb) launch_bwd_t<DD, true, false, true, TL>(prm, st);
-      else launch_bwd_t<DD, true, false, false, TL>(prm, st);
+      if (!bf) launch_bwd_t<DD, false, false, false, TL>(prm, pairs.groups, st);
+      else if (pb) launch_bwd_t<DD, true, false, true, TL>(prm, pairs.groups, st);
+      else launch_bwd_t<DD, true, false, false, TL>(prm, pairs.groups, st);
     } else {   // elementwise mask
-      if (!bf) launch_bwd_t<DD, false, true, false, TL>(prm, st);
-      else if (pb) launch_bwd_t<DD, true, true, true, TL>(prm, st);
-      else launch_bwd_t<DD, true, true, false, TL>(prm, st);
+      if (!bf) launch_bwd_t<DD, false, true, false, TL>(prm, pairs.groups, st);
+      else if (pb) launch_bwd_t<DD, true, true, true, TL>(prm, pairs.groups, st);
+      else launch_bwd_t<DD, true, true, false, TL>(prm, pairs.groups, st);
     }
   };
   auto pick_tail = [&](auto dc) {

@@ -18,7 +18,7 @@ namespace bsattn {
 
 // S: pairs of wavefronts per workgroup.  Lists of at most BWD_SHORT_MAX_BLOCKS tiles.
 template <int S, bool EW> struct BwdShortCfg {
-  static constexpr int D = 64, PITCH = D + 4;                        // PITCH: floats per row of a pair's sums in LDS
+  static constexpr int D = 64, PITCH = D + 4;                        // PITCH: floats per row of a pair's sums in LDS (add_pairs)
   static constexpr int KV_BYTES = 64 * 2 * D, HALF_BYTES = KV_BYTES / 2, BITS_BYTES = EW ? 512 : 0;
   static constexpr int DQ_STAGE = 2 * KV_BYTES + BITS_BYTES;         // K tile, V tile, mask words
   static constexpr int DKV_STAGE = 3 * HALF_BYTES + 256 + BITS_BYTES;   // 32 rows of Q, dO and O, lse of the 64, mask words
@@ -43,18 +43,17 @@ __device__ __forceinline__ float dot8_packed(const uintx4& a, const uintx4& b, f
   return acc;
 }
 
-// This workgroup's share of list `list` (entries list[0], list[1] of its pointers), and the list in LDS.
-// Four consecutive values of the sum over the pairs per thread, `rows` rows of 64: result or fp32 part.
-template <int S, bool BF16, typename F>
-__device__ __forceinline__ void add_pairs(const unsigned char* lds, int pair_bytes, int pitch, int rows, F&& put) {
-#pragma unroll
-  for (int i = threadIdx.x; i < 64 * 16; i += 128 * S) {
-    const int r = i >> 4, col = (i & 15) * 4;
+// The sums over the pairs, four consecutive values of one of the first `rows` rows per thread.  A pair's rows are D + 4 floats apart.
+template <int D, int S, typename F>
+__device__ __forceinline__ void add_pairs(const unsigned char* lds, int pair_bytes, int rows, F&& put) {
+#pragma unroll 4
+  for (int i = threadIdx.x; i < 64 * (D / 4); i += 128 * S) {
+    const int r = i / (D / 4), col = i % (D / 4) * 4;
     if (r >= rows) break;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < S; ++c) {
-      const floatx4 x = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(lds + c * pair_bytes) + r * pitch + col);
+      const floatx4 x = *reinterpret_cast<const floatx4*>(reinterpret_cast<const float*>(lds + c * pair_bytes) + r * (D + 4) + col);
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] += x[e];
     }
@@ -62,10 +61,13 @@ __device__ __forceinline__ void add_pairs(const unsigned char* lds, int pair_byt
   }
 }
 
-template <int S, bool BF16, bool EW, bool PB, bool TAIL>
-__device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* lds, int bh, int b, int h, int mh, int m, int chunk) {
-  using C = BwdShortCfg<S, EW>;
-  constexpr int D = 64, KS = D / 16, DB = D / 32;
+// dQ of row block m.  D = 64 walks whole tiles, D = 128 halves of 32 keys (attn_bwd.hip's dq_kernel).  C: where what is in LDS.
+// delta: where delta of the queries goes for a dK/dV kernel that comes later, or null.
+template <int D, int S, typename C, bool BF16, bool EW, bool PB, bool TAIL>
+__device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* lds, int bh, int b, int h, int mh, int m, int chunk, int split,
+                                         float* delta) {
+  constexpr int KS = D / 16, DB = D / 32, KB = D == 64 ? 2 : 1, ROWS = 32 * KB, STEPS = 2 / KB;
+  constexpr int TILE_BYTES = ROWS * 2 * D, BITS_OFF = 2 * TILE_BYTES;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = wave >> 1, w = wave & 1;
   const int ln = lane & 31, g = lane >> 5, nb = prm.nb;
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
@@ -80,36 +82,36 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
   for (int s = 0; s < KS; ++s) {
     qfr[s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
     dofr[s] = *reinterpret_cast<const uintx4*>(gp + 16 * s + 8 * g);
-    ofr[s] = *reinterpret_cast<const uintx4*>(op + 16 * s + 8 * g);
   }
+#pragma unroll
+  for (int s = 0; s < KS; ++s) ofr[s] = *reinterpret_cast<const uintx4*>(op + 16 * s + 8 * g);
   const float lse_q = prm.lse[(int64_t)bh * prm.N + qsrc];
   int t0, t1;
   {
     const int first = rp[m], len = rp[m + 1] - first;
-    t0 = first + (int)((int64_t)len * chunk / prm.split);
-    t1 = first + (int)((int64_t)len * (chunk + 1) / prm.split);
+    t0 = first + (int)((int64_t)len * chunk / split);
+    t1 = first + (int)((int64_t)len * (chunk + 1) / split);
   }
   int* lcols = reinterpret_cast<int*>(lds + C::COLS_OFF);
   unsigned char* mine = lds + c * C::PAIR_BYTES;
   const unsigned mine_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds + c * C::PAIR_BYTES;
   const unsigned short* kg = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1];
   const unsigned short* vg = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1];
-  auto issue = [&](int cb, int t, int stage) {
+  auto issue = [&](int cb, int t, int part, int stage) {       // rows ROWS part .. of the tile
     const unsigned sa = mine_addr + stage * C::DQ_STAGE;
-    const unsigned short* kt = kg + (int64_t)cb * 64 * prm.ks[2];
-    const unsigned short* vt = vg + (int64_t)cb * 64 * prm.vs[2];
     if (TAIL && cb == nb - 1) {
-      tail_tile_load_async<2, D, 64>(kt, prm.ks[2], 0, valid, w, lane, sa);
-      tail_tile_load_async<2, D, 64>(vt, prm.vs[2], 0, valid, w, lane, sa + C::KV_BYTES);
+      tail_tile_load_async<2, D, ROWS>(kg + (int64_t)cb * 64 * prm.ks[2], prm.ks[2], part * ROWS, valid, w, lane, sa);
+      tail_tile_load_async<2, D, ROWS>(vg + (int64_t)cb * 64 * prm.vs[2], prm.vs[2], part * ROWS, valid, w, lane, sa + TILE_BYTES);
     } else {
-      half_tile_load_async<D, 64>(kt, prm.ks[2], w, lane, sa);
-      half_tile_load_async<D, 64>(vt, prm.vs[2], w, lane, sa + C::KV_BYTES);
+      const int64_t key0 = (int64_t)cb * 64 + part * ROWS;
+      half_tile_load_async<D, ROWS>(kg + key0 * prm.ks[2], prm.ks[2], w, lane, sa);
+      half_tile_load_async<D, ROWS>(vg + key0 * prm.vs[2], prm.vs[2], w, lane, sa + TILE_BYTES);
     }
     if constexpr (EW)   // the tile's 64 mask words, 256 bytes per wavefront
-      stat_load_async(reinterpret_cast<const float*>(prm.bits_rows + (int64_t)t * 64) + w * 64, lane, sa + 2 * C::KV_BYTES + w * 256);
+      stat_load_async(reinterpret_cast<const float*>(prm.bits_rows + (int64_t)t * 64) + w * 64, lane, sa + BITS_OFF + w * 256);
   };
   int t = t0 + c, cb = 0;
-  if (t < t1) { cb = cols[t]; issue(cb, t, 0); }
+  if (t < t1) { cb = cols[t]; issue(cb, t, 0, 0); }
   for (int i = threadIdx.x; i < t1 - t0 && i < BWD_SHORT_MAX_BLOCKS; i += 128 * S) lcols[i] = prm.col_idx[t0 + i];
   // a query without any unmasked key has lse = -inf: every P of its row must come out as 0
   float lse2 = EW && lse_q == -INFINITY ? INFINITY : lse_q * kLog2e, dlt;
@@ -118,6 +120,7 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
 #pragma unroll
     for (int s = 0; s < KS; ++s) acc = dot8<BF16>(ofr[s], dofr[s], acc);
     dlt = acc + __shfl_xor(acc, 32);
+    if (delta != nullptr && chunk == 0 && c == 0 && g == 0 && (!TAIL || qrow < prm.N)) delta[(int64_t)bh * prm.N + qrow] = dlt;
   }
 #pragma unroll
   for (int s = 0; s < KS; ++s) { settle(qfr[s]); settle(dofr[s]); }
@@ -127,26 +130,28 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
 #pragma unroll
   for (int db = 0; db < DB; ++db) dqacc[db] = zero16();
 
-  const int steps = (t1 - t0 + S - 1) / S;
+  const int steps = STEPS * ((t1 - t0 + S - 1) / S);
   for (int it = 0; it < steps; ++it) {
     wait_vm<0>();
     __syncthreads();                              // the step's tiles are complete; everybody has left the step before
-    const int tn = t + S;
-    int cbn = 0;
+    const int part = it % STEPS, tn = part == STEPS - 1 ? t + S : t;
+    int cbn = cb;
     if (tn < t1) {
-      cbn = __builtin_amdgcn_readfirstlane(lcols[tn - t0]);
-      issue(cbn, tn, (it + 1) & 1);
+      if (part == STEPS - 1) cbn = __builtin_amdgcn_readfirstlane(lcols[tn - t0]);
+      issue(cbn, tn, (it + 1) % STEPS, (it + 1) & 1);
     }
     if (t < t1) {
       const unsigned char* kt = mine + (it & 1) * C::DQ_STAGE;
-      const unsigned char* vt = kt + C::KV_BYTES;
-      floatx16 sacc[2] = {zero16(), zero16()}, dpacc[2] = {zero16(), zero16()};
+      const unsigned char* vt = kt + TILE_BYTES;
+      floatx16 sacc[KB], dpacc[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) { sacc[kb] = zero16(); dpacc[kb] = zero16(); }
       {
-        uintx4 fk[2][KS], fv[2][KS];
+        uintx4 fk[KB][KS], fv[KB][KS];
 #pragma unroll
         for (int s = 0; s < KS; ++s)
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
+          for (int kb = 0; kb < KB; ++kb) {
             fk[kb][s] = frag_rows<D>(kt, 32 * kb, s, ln, g);
             fv[kb][s] = frag_rows<D>(vt, 32 * kb, s, ln, g);
           }
@@ -154,23 +159,30 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
 #pragma unroll
         for (int s = 0; s < KS; ++s)
 #pragma unroll
-          for (int kb = 0; kb < 2; ++kb) {
+          for (int kb = 0; kb < KB; ++kb) {
             sacc[kb] = mfma_qk<BF16>(fk[kb][s], qfr[s], sacc[kb]);      // S^T = K Q^T
             dpacc[kb] = mfma_qk<BF16>(fv[kb][s], dofr[s], dpacc[kb]);   // dP^T = V dO^T
           }
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (EW) mask_scores(sacc[0], sacc[1], *reinterpret_cast<const unsigned long long*>(vt + C::KV_BYTES + (32 * w + ln) * 8) >> (4 * g));
-      else if (TAIL && cb == nb - 1) mask_scores(sacc[0], sacc[1], tail_word(valid, g));
-      uintx4 fkt[4][DB];
+      if constexpr (EW) {
+        const unsigned long long mw = *reinterpret_cast<const unsigned long long*>(kt + BITS_OFF + (32 * w + ln) * 8);
+        if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw >> (4 * g));
+        else mask_scores(sacc[0], (unsigned)(mw >> (32 * part + 4 * g)));
+      } else if (TAIL && cb == nb - 1) {
+        const unsigned long long mw = tail_word(valid, g);
+        if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw);
+        else mask_scores(sacc[0], (unsigned)(mw >> (32 * part)));
+      }
+      uintx4 fkt[2 * KB][DB];
 #pragma unroll
-      for (int ts = 0; ts < 4; ++ts)
+      for (int ts = 0; ts < 2 * KB; ++ts)
 #pragma unroll
         for (int db = 0; db < DB; ++db) fkt[ts][db] = frag_cols<D, BF16 && !PB>(kt, db, ts, lane);
       __builtin_amdgcn_sched_barrier(0);
-      uintx4 dsf[4];       // dS^T = P^T * (dP^T - delta), packed as operand slices of 16 keys
+      uintx4 dsf[2 * KB];       // dS^T = P^T * (dP^T - delta), packed as operand slices of 16 keys
 #pragma unroll
-      for (int ts = 0; ts < 4; ++ts)
+      for (int ts = 0; ts < 2 * KB; ++ts)
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) {
           const int kb = ts >> 1, i = 8 * (ts & 1) + 2 * jj;
@@ -179,7 +191,7 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
           dsf[ts][jj] = pack2<PB>(p0 * (dpacc[kb][i] - dlt), p1 * (dpacc[kb][i + 1] - dlt));
         }
 #pragma unroll
-      for (int ts = 0; ts < 4; ++ts)
+      for (int ts = 0; ts < 2 * KB; ++ts)
 #pragma unroll
         for (int db = 0; db < DB; ++db) dqacc[db] = mfma_qk<PB>(fkt[ts][db], dsf[ts], dqacc[db]);       // dQ^T += K^T dS^T
     }
@@ -189,7 +201,7 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
 
   __syncthreads();           // everybody has left the last step
   {
-    float* own = reinterpret_cast<float*>(mine) + (32 * w + ln) * C::PITCH + 4 * g;
+    float* own = reinterpret_cast<float*>(mine) + (32 * w + ln) * (D + 4) + 4 * g;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -203,8 +215,8 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
   void* base = prm.out_f32 ? (void*)((float*)prm.dq + off) : (void*)((unsigned short*)prm.dq + off);
   float* part = prm.part_dq + ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
   const float sc = prm.sm_scale;
-  add_pairs<S, BF16>(lds, C::PAIR_BYTES, C::PITCH, TAIL && r0 + 64 > prm.N ? prm.N - (int)r0 : 64, [&](int r, int col, const floatx4& x) {
-    if (prm.split > 1) *reinterpret_cast<floatx4*>(part + (r0 + r) * D + col) = x;
+  add_pairs<D, S>(lds, C::PAIR_BYTES, TAIL && r0 + 64 > prm.N ? prm.N - (int)r0 : 64, [&](int r, int col, const floatx4& x) {
+    if (split > 1) *reinterpret_cast<floatx4*>(part + (r0 + r) * D + col) = x;
     else store_out4<BF16>(base, (r0 + r) * prm.dqs[2] + col, prm.out_f32, x[0] * sc, x[1] * sc, x[2] * sc, x[3] * sc);
   });
 }
@@ -373,11 +385,11 @@ __device__ __forceinline__ void short_dkdv(const BwdParams& prm, unsigned char* 
   const int64_t poff = ((int64_t)chunk * prm.B * prm.H + bh) * prm.N * D;
   const int here = TAIL && r0 + 64 > prm.N ? prm.N - (int)r0 : 64;
   const float sc = prm.sm_scale;
-  add_pairs<S, BF16>(lds, C::PAIR_BYTES, C::PITCH, here, [&](int r, int col, const floatx4& x) {
+  add_pairs<D, S>(lds, C::PAIR_BYTES, here, [&](int r, int col, const floatx4& x) {
     if (prm.split > 1) *reinterpret_cast<floatx4*>(prm.part_dk + poff + (r0 + r) * D + col) = x;
     else store_out4<BF16>(kbase, (r0 + r) * prm.dks[2] + col, prm.out_f32, x[0] * sc, x[1] * sc, x[2] * sc, x[3] * sc);
   });
-  add_pairs<S, BF16>(lds + C::SUM_BYTES, C::PAIR_BYTES, C::PITCH, here, [&](int r, int col, const floatx4& x) {
+  add_pairs<D, S>(lds + C::SUM_BYTES, C::PAIR_BYTES, here, [&](int r, int col, const floatx4& x) {
     if (prm.split > 1) *reinterpret_cast<floatx4*>(prm.part_dv + poff + (r0 + r) * D + col) = x;
     else store_out4<BF16>(vbase, (r0 + r) * prm.dvs[2] + col, prm.out_f32, x[0], x[1], x[2], x[3]);
   });
@@ -393,7 +405,57 @@ __global__ __launch_bounds__(128 * S, 2) void bwd_short_kernel(const BwdParams p
   const int bh = p.head, b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
   const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
   if (share < prm.split) short_dkdv<S, BF16, EW, PB, TAIL>(prm, lds, bh, b, h, mh, p.item, share);
-  else short_dq<S, BF16, EW, PB, TAIL>(prm, lds, bh, b, h, mh, prm.nb - 1 - p.item, share - prm.split);   // (long rows of causal masks first)
+  else short_dq<64, S, BwdShortCfg<S, EW>, BF16, EW, PB, TAIL>(prm, lds, bh, b, h, mh, prm.nb - 1 - p.item, share - prm.split, prm.split, nullptr);   // (long rows of causal masks first)
+}
+
+// dQ alone at D = 128, for launches with few lists (attn_bwd.hip, bwd_pairs_128): S pairs of wavefronts per row block where dq_kernel
+// has one or several workgroups of one.  Bound by the chain of a step, S and dP, exponentials, dQ: at two wavefronts per SIMD one's
+// products hide half of the other's chain.  One share per list: no parts, no sums.  (D = 256 with two pairs, a lone wavefront per SIMD
+// like dq_kernel's, took longer than dq_kernel's shares at every size: 2 heads N = 4096 dense, backward 183 -> 281 us.)
+template <int D, int S, bool EW> struct DqPairsCfg {
+  static constexpr int DQ_STAGE = 2 * 32 * 2 * D + (EW ? 512 : 0), SUM_BYTES = 64 * (D + 4) * 4;
+  static constexpr int PAIR_BYTES = (2 * DQ_STAGE > SUM_BYTES ? 2 * DQ_STAGE : SUM_BYTES) + 255 & ~255;
+  static constexpr int COLS_OFF = S * PAIR_BYTES, LDS_BYTES = COLS_OFF + BWD_SHORT_MAX_BLOCKS * 4;
+  static_assert(LDS_BYTES <= 160 * 1024, "fits a compute unit");
+};
+
+template <int D, int S, bool BF16, bool EW, bool PB, bool TAIL>
+__global__ __launch_bounds__(128 * S, 2) void dq_pairs_kernel(const BwdParams prm) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  int share;
+  const Place p = prm.place_dq.of(blockIdx.x, share);
+  if (p.item >= prm.nb) return;                   // padding of an incomplete last group
+  const int bh = p.head, b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
+  const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
+  short_dq<D, S, DqPairsCfg<D, S, EW>, BF16, EW, PB, TAIL>(prm, lds, bh, b, h, mh, prm.nb - 1 - p.item, 0, 1, prm.delta);
+}
+
+template <int D, int S, bool BF16, bool EW, bool PB, bool TAIL>
+static void launch_dq_t(const BwdParams& prm, hipStream_t st) {
+  constexpr int LDS = DqPairsCfg<D, S, EW>::LDS_BYTES;
+  static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
+  once_per_device(configured, [] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&dq_pairs_kernel<D, S, BF16, EW, PB, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+  });
+  hipLaunchKernelGGL((dq_pairs_kernel<D, S, BF16, EW, PB, TAIL>), dim3(prm.place_dq.per_share), dim3(128 * S), LDS, st, prm);
+}
+
+// pairs: 2 or 4 per workgroup
+void launch_dq_pairs(const BwdParams& prm, int pairs, bool bf16, bool pb, hipStream_t st) {
+  const bool ew = prm.bits_rows != nullptr, tail = prm.N % 64 != 0;
+  auto pick = [&](auto ss, auto e, auto t) {
+    constexpr int SS = decltype(ss)::value;
+    constexpr bool E = decltype(e)::value, T = decltype(t)::value;
+    if (!bf16) launch_dq_t<128, SS, false, E, false, T>(prm, st);
+    else if (pb) launch_dq_t<128, SS, true, E, true, T>(prm, st);
+    else launch_dq_t<128, SS, true, E, false, T>(prm, st);
+  };
+  auto pick_mask = [&](auto ss) {
+    if (ew) { if (tail) pick(ss, std::true_type{}, std::true_type{}); else pick(ss, std::true_type{}, std::false_type{}); }
+    else { if (tail) pick(ss, std::false_type{}, std::true_type{}); else pick(ss, std::false_type{}, std::false_type{}); }
+  };
+  if (pairs == 2) pick_mask(std::integral_constant<int, 2>{});
+  else pick_mask(std::integral_constant<int, 4>{});
 }
 
 template <int S, bool BF16, bool EW, bool PB, bool TAIL>

@@ -25,6 +25,8 @@ struct BwdParams {
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];
   int64_t dqs[3], dks[3], dvs[3];   // batch, head, row strides of the results (elements)
   PlaceOfEight place;         // workgroup -> (head, list, share)
+  PlaceOfEight place_dq;      // dq_pairs_kernel's (one share)
+  int first_sum;              // parts are added up of: 0 dQ, dK and dV, 1 dK and dV (dQ is dq_pairs_kernel's)
   Divisor per_batch;          // H
 };
 

@@ -313,15 +313,19 @@ def test_only_long_lists_are_shared(dev, H, N, dtype, out_fp32):
 
 
 # D = 64, few lists (dQ, dK, dV in one launch): 4 pairs of wavefronts with and without shares, 2 pairs, 2 pairs with shares, long
-# lists of many heads; lists shorter than the pairs are many, empty ones, ragged lengths, queries without keys
-@pytest.mark.parametrize("H,N", [(1, 64), (3, 130), (5, 512), (8, 1000), (1, 3100), (1, 6000), (9, 1000), (2, 4100), (1, 9700), (20, 2000)])
+# lists of many heads; lists shorter than the pairs are many, empty ones, ragged lengths, queries without keys.
+# D = 128: dQ by 2 pairs of wavefronts beside dK and dV whole, by 2 and by 4 beside two groups of wavefronts that add up dK and dV,
+# at the ends of each range; the last one beside shares whose parts are added up without dQ's
+@pytest.mark.parametrize("D,H,N", [(64, 1, 64), (64, 3, 130), (64, 5, 512), (64, 8, 1000), (64, 1, 3100), (64, 1, 6000), (64, 9, 1000), (64, 2, 4100),
+                                   (64, 1, 9700), (64, 20, 2000), (128, 1, 768), (128, 3, 800), (128, 4, 1000), (128, 4, 2048), (128, 8, 2000),
+                                   (128, 7, 4100), (128, 2, 8192), (128, 9, 5000), (128, 4, 9000)])
 @pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 @pytest.mark.parametrize("elementwise", [False, True])
-def test_few_lists(dev, H, N, dtype, out_fp32, elementwise):
+def test_few_lists(dev, D, H, N, dtype, out_fp32, elementwise):
     import fa2_custom_mask as fm
     from helpers import make_qkv, uniform_block_mask, errors
     nb = -(-N // 64)
-    q, k, v, do = [x.to(dev) for x in make_qkv(1, H, N, 64, dtype, 1000 + N, n=4)]
+    q, k, v, do = [x.to(dev) for x in make_qkv(1, H, N, D, dtype, 1000 + N, n=4)]
     mask = uniform_block_mask(1, H, nb, 0.3, 1001 + N).to(dev)
     if nb > 3:
         mask[0, 0, 1] = False                                # a row block and a column block without tiles
@@ -330,15 +334,15 @@ def test_few_lists(dev, H, N, dtype, out_fp32, elementwise):
         i = torch.arange(N, device=dev)
         mask = mask.repeat_interleave(64, 2)[:, :, :N].repeat_interleave(64, 3)[..., :N] & ((i[:, None] - i[None, :]) % 7 != 0)
     mask_h = lambda h: mask[0, h] if elementwise else mask[0, h].repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N]
-    grads = fm.attention_forward_backward(q, k, v, mask, 0.125, do, out_fp32=out_fp32)[2:]
-    again = fm.attention_forward_backward(q, k, v, mask, 0.125, do, out_fp32=out_fp32)[2:]
+    grads = fm.attention_forward_backward(q, k, v, mask, D ** -0.5, do, out_fp32=out_fp32)[2:]
+    again = fm.attention_forward_backward(q, k, v, mask, D ** -0.5, do, out_fp32=out_fp32)[2:]
     assert all(torch.equal(a, b) for a, b in zip(grads, again)) or N > 8192      # (beyond, the forward's last bits vary)
     # P and dS have 16 bits, results too unless out_fp32 (bf16: 2^-9 each)
     rel = 2e-3 if out_fp32 or dtype == torch.float16 else 1e-2
     for h in (range(H) if N < 4000 else (0, H - 1)):
         qf, kf, vf = [x[0, h].float().requires_grad_(True) for x in (q, k, v)]
         keep = mask_h(h)
-        p = torch.softmax((qf @ kf.T * 0.125).masked_fill(~keep, -1e30), -1) * keep.any(-1, keepdim=True)
+        p = torch.softmax((qf @ kf.T * D ** -0.5).masked_fill(~keep, -1e30), -1) * keep.any(-1, keepdim=True)
         ref = torch.autograd.grad(p @ vf, (qf, kf, vf), do[0, h].float())
         for name, got, r in zip(("dq", "dk", "dv"), grads, ref):
             ma, rl = errors(got[0, h], r)
