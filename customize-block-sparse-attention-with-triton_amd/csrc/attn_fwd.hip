@@ -1324,9 +1324,9 @@ static int long_row_groups(int B, int H, int nb, bool compact) {
   return compact && parts_bytes(B, H, nb, (int)W, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
-// Pair kernel, D = 256: workgroups per row block.  A share costs the launch that sums the parts and their traffic (64 KB of
+// D = 256: workgroups per row block, of fwd_pair_kernel and of fwd_wide_kernel alike (both have two on a compute unit).  A share costs the launch that sums the parts and their traffic (64 KB of
 // fp32 per row block and share, as much as a tile's operands), so only launches that leave the GPU's 512 pairs short share,
-// and short lists where few of them are in the launch.  us, N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares:
+// and short lists where few of them are in the launch.  us, N(0,1) bf16, fwd_pair_kernel, 1 / 2 / 3 / 4 / 6 / 8 shares:
 //    1 head  N = 512    keep 0.3   16 /  15 /  13 /  14 /  11 /  12    dense   23 /  18 /  16 /  14 /  15 /  13
 //    5 heads N = 832               21 /  22 /  21 /  22 /  24 /  26            35 /  29 /  27 /  29 /  29 /  32
 //   12 heads N = 832               29 /  30 /  29 /  36 /  35 /  37            36 /  37 /  34 /  45 /  45 /  53

@@ -1,5 +1,5 @@
-// Block-sparse FlashAttention-2 forward, head dimensions 128 and 256 (one wavefront per SIMD there, K and V fragments
-// taken from LDS in two portions).
+// Block-sparse FlashAttention-2 forward, head dimension 128, and 256 with elementwise masks or a ragged length (one wavefront per
+// SIMD there, K and V fragments taken from LDS in two portions).
 //
 // At D = 128 a wavefront that owns 64 queries would need all 512 registers of its SIMD and be bound by instruction issue.
 // Here a row block belongs to a pair of wavefronts, 32 queries each (256 registers: two
@@ -472,9 +472,12 @@ static void launch_pair_d(const FwdParams& prm, int dt, bool elementwise, hipStr
   }
 }
 
-// D: 128 or 256.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st);   // attn_fwd_wide.hip
+
+// D: 128 or 256 (whole tiles of block masks: attn_fwd_wide.hip, whose registers hold no more).  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st) {
   if (D == 128) launch_pair_d<128>(prm, dt, elementwise, st);
+  else if (!elementwise && prm.N % 64 == 0) launch_fwd_wide(prm, dt, st);
   else launch_pair_d<256>(prm, dt, elementwise, st);
 }
 

@@ -1,0 +1,330 @@
+// Block-sparse FlashAttention-2 forward, head dimension 256.
+//
+// A workgroup of four wavefronts has one row block, or one of `split` contiguous shares of its list: wavefront (kh, w) takes keys
+// 32 kh .. of every tile for queries 32 w .. .  O of 32 queries is 128 registers and Q 64; with the scores of 32 keys in place of
+// 64 the rest fits a quarter of a SIMD's registers, so two wavefronts share a SIMD and one's products run beside the other's
+// softmax.  A K and a V tile (64 KB) are shared by the four, two workgroups per compute unit; the next K tile is asked for as soon
+// as all hold their K fragments, the next V tile as soon as all hold their V fragments (four barriers per tile).  The two key halves
+// keep a reference exponent and a sum each and meet in LDS at the end, half of the columns each way.
+//
+// Before, fwd_pair_kernel: a wavefront with the scores of all 64 keys, up to 512 registers, alone on its SIMD, so that scores, softmax
+// and second product came one after the other.  us: 16 heads N = 4096 block-causal keep 0.5 bf16 108 -> 96, results in fp32
+// 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  The 256 registers
+// leave no room for mask words or the bounds of a ragged length (20 to 140 spilled): those launches stay on
+// fwd_pair_kernel.
+//
+// Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196 of the reference).
+#include "common.h"
+#include "fwd_tile.h"
+#include "kernel_util.h"
+
+namespace bsattn {
+
+constexpr int WIDE_D = 256, WIDE_COLS_CAP = 1024;                               // column indices of the row block kept in LDS
+constexpr int WIDE_TILE_BYTES = 64 * 2 * WIDE_D;
+constexpr int WIDE_COLS_OFF = 2 * WIDE_TILE_BYTES;
+constexpr int WIDE_LDS_BYTES = WIDE_COLS_OFF + WIDE_COLS_CAP * 4;               // K tile, V tile, columns
+static_assert(MASK_MAX_BLOCKS <= WIDE_COLS_CAP, "all columns from the mask are in LDS");
+static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the result rows of all wavefronts");
+
+// DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
+// CONTIG: the rows of K and of V follow each other without gaps (row stride = 256).
+template <int DT, bool CONTIG>
+__global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
+  constexpr int D = WIDE_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
+  constexpr int COPIES = CPR / 4;                // copy instructions per wavefront and tile
+  constexpr bool BF16 = DT != 0, PB = DT == 2, FOLD = !BF16;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kh = wave >> 1, w = wave & 1;
+  const int ln = lane & 31, g = lane >> 5;
+  const int nb = prm.nb, BH = prm.B * prm.H;
+  int chunk;
+  const Place p = prm.place.of(blockIdx.x, chunk);
+  const int bh = p.head, m = nb - 1 - p.item;
+  if (m < 0) return;                             // padding of an incomplete last group
+  const int b = (int)prm.per_batch.of((unsigned)bh), h = bh - b * prm.H;
+  const int mh = (prm.Bm > 1 ? b : 0) * prm.Hm + (prm.Hm > 1 ? h : 0);
+  const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
+  // Q of this lane's query depends on the block index only: asked for first, it travels while the list is looked up
+  const int64_t qrow = (int64_t)m * 64 + 32 * w + ln;
+  uintx4 qf[KS];
+  {
+    const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + qrow * prm.qs[2];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
+  }
+  int* lcols = reinterpret_cast<int*>(lds + WIDE_COLS_OFF);
+  const bool listed = prm.mask == nullptr;
+  int t0, t1;
+  if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
+  else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols); }
+  if (prm.split > 1) {                           // this workgroup's share of the row block's list
+    const int len = t1 - t0;
+    if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
+    t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
+    t0 = t0 + (int)((int64_t)len * chunk / prm.split);
+    if (t0 == t1) return;                        // (pair_sum_parts_kernel knows which shares are empty)
+  }
+  void* obase = out_base(prm, b, h);
+  if (t0 == t1) {                                // no kept tile: O = 0, lse = -inf
+#pragma unroll
+    for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        store_out4<BF16>(obase, qrow * prm.os[2] + 128 * kh + 32 * db + 8 * i4 + 4 * g, prm.out_f32, 0.f, 0.f, 0.f, 0.f);
+    if (prm.lse != nullptr && wave == w && g == 0) prm.lse[(int64_t)bh * prm.N + qrow] = -INFINITY;
+    return;
+  }
+
+  unsigned char* lds_v = lds + WIDE_TILE_BYTES;
+  const unsigned lds_k_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds;
+  const unsigned lds_v_addr = lds_k_addr + WIDE_TILE_BYTES;
+  const unsigned short* kg = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1];
+  const unsigned short* vg = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1];
+  const float qk_scale = prm.qk_scale;
+
+  const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
+  const int first_t = listed ? t0 : 0;           // entry t of the list is lcols[t - first_t] once it is staged
+  auto col_of = [&](int t) { return t - first_t < WIDE_COLS_CAP ? lcols[t - first_t] : cols[t]; };
+
+  // asynchronous tile copies: instruction j covers tile rows 2j, 2j + 1; this wavefront issues [8 wave, 8 wave + 8) of a tile.
+  // The swizzles repeat every 16 rows for K (8 instructions) and every 4 rows for V (2): instruction j reads chunk
+  // (lane % 32) ^ (2 j + row0) % 16 of K's row 2j + row0, ... ^ 4 ((2 j + row0) % 4) of V's.
+  constexpr int KPER = 16 / RPI, VPER = 4 / RPI;
+  static_assert(COPIES % KPER == 0 && COPIES % VPER == 0, "the swizzle patterns of a wavefront's instructions start at phase 0");
+  const int row0 = lane / CPR;
+  unsigned kx = 16u * (unsigned)((lane % CPR) ^ row0), vx = 16u * (unsigned)((lane % CPR) ^ (4 * row0));
+  const unsigned krow = 2u * (unsigned)(row0 * (int)prm.ks[2]), vrow = 2u * (unsigned)(row0 * (int)prm.vs[2]);
+  if constexpr (CONTIG) { kx += row0 * ROWB; vx += row0 * ROWB; }
+  auto tile_copy = [&](const unsigned short* tile, int64_t rs, unsigned lds_addr, auto&& off) {
+    if constexpr (CONTIG) {            // (instruction j reads at byte 1024 j of the tile and writes at byte 1024 j of the buffer)
+#pragma unroll
+      for (int jb = 0; jb < COPIES; jb += 4)
+        tile_load_async_four(tile + (wave * COPIES + jb) * RPI * D, off(jb), off(jb + 1), off(jb + 2), off(jb + 3),
+                             lds_addr + (wave * COPIES + jb) * 1024);
+    } else {
+#pragma unroll
+      for (int jj = 0; jj < COPIES; ++jj) {
+        const int j = wave * COPIES + jj;
+        tile_load_async_one(tile + (int64_t)j * RPI * rs, off(jj), lds_addr + j * 1024);
+      }
+    }
+  };
+  auto k_copy = [&](int cb) {
+    tile_copy(kg + (int64_t)cb * 64 * (CONTIG ? (int64_t)D : prm.ks[2]), prm.ks[2], lds_k_addr,
+              [&](int j) { return (kx ^ (32u * (j % KPER))) + (CONTIG ? 0u : krow); });
+  };
+  auto v_copy = [&](int cb) {
+    tile_copy(vg + (int64_t)cb * 64 * (CONTIG ? (int64_t)D : prm.vs[2]), prm.vs[2], lds_v_addr,
+              [&](int j) { return (vx ^ (128u * (j % VPER))) + (CONTIG ? 0u : vrow); });
+  };
+
+  // Fragment addresses.  K: chunk (2s + g) ^ (row & 15) of row 32 kh + ln, i.e. kbase with bits 5-7 turned by s % 8, and 256 s / 8
+  // further on.  V: chunk (4 db + ..) ^ 4 (key & 3), i.e. vbase with bits 6-7 turned by db % 4, and 256 (db / 4) further on.
+  int kbase = (32 * kh + ln) * ROWB + ((g ^ k_swz<D>(ln)) * 16);
+  int vbase;
+  {
+    const int blk = lane >> 4, vs = lane & 15, key0 = 4 * (blk >> 1) + (vs >> 2), col0 = 16 * (blk & 1) + 4 * (vs & 3);
+    vbase = (32 * kh + key0) * ROWB + (((col0 >> 3) ^ v_swz<D>(key0)) * 16) + (col0 & 7) * 2;
+  }
+  const uintx4 ones_frag = {g == 0 ? 0x3c003c00u : 0u, 0u, 0u, 0u};
+
+  // first tile's copies (its column from one scalar load), then the column list into LDS
+  const int cb0 = listed ? cols[t0] : __builtin_amdgcn_readfirstlane(lcols[t0]);
+  k_copy(cb0);
+  v_copy(cb0);
+  if (listed)
+    for (int i = threadIdx.x; i < t1 - t0 && i < WIDE_COLS_CAP; i += 256) lcols[i] = prm.col_idx[t0 + i];
+  __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0), visible to the compiler: Q and the first tiles
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const uintx4 raw = qf[s];
+      const uintx4 scaled = {scale_half2(raw[0], qk_scale), scale_half2(raw[1], qk_scale),
+                             scale_half2(raw[2], qk_scale), scale_half2(raw[3], qk_scale)};
+      qf[s] = scaled;
+    }
+  }
+  floatx16 oacc[DB][1];
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) oacc[db][0][i] = 0.f;
+  float m_i = 0.f, l_i = 0.f;
+  uintx4 mfrag = {0u, 0u, 0u, 0u};
+  bool fresh = true;
+  int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
+  __syncthreads();                                  // all of K(t0), V(t0) and the column list are in LDS
+
+  for (int t = t0; t < t1; ++t) {
+    const bool has1 = t + 1 < t1;
+    const int cbn = has1 ? __builtin_amdgcn_readfirstlane(col_of(t + 1)) : 0;
+    asm volatile("" : "+v"(kbase), "+v"(vbase), "+v"(kx), "+v"(vx));    // (or the turned addresses are computed before the loop and held)
+    // ---- S^T = K Q^T (- m when FOLD), K fragments in portions of four ----
+    floatx16 sc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+    uintx4 kfr[2][4];
+    auto read_k = [&](int pt) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int s = 4 * pt + i;
+        kfr[pt & 1][i] = *reinterpret_cast<const uintx4*>(lds + (kbase ^ (32 * (s & 7))) + 256 * (s >> 3));
+      }
+    };
+    read_k(0);
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt) {
+      if (pt < 3) read_k(pt + 1);
+      if (pt == 3) {
+        lds_wait();
+        __syncthreads();                            // all wavefronts hold their K fragments: the K buffer is free
+        if (has1) k_copy(cbn);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sc = mfma_qk<BF16>(kfr[pt & 1][i], qf[4 * pt + i], sc);
+    }
+    if constexpr (FOLD) {
+      if (any_m) sc = mfma_qk<BF16>(ones_frag, mfrag, sc);
+    }
+    uintx4 pf[2];
+    float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+    // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
+    const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
+    if (__any(first || !(lnew - l_i < 16384.0f))) {
+      recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
+      any_m = 1;
+      lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+    }
+    l_i = lnew;
+    fresh = false;
+    if (has1) wait_vm<COPIES>(); else wait_vm<0>();   // this wavefront's part of V(t) has landed (K(t+1) may be in flight)
+    if (t > t0) __syncthreads();                    // ... and the others' (the first tile was waited for above)
+    // ---- O^T += V^T P^T, V^T fragments in portions of two column blocks ----
+    uintx4 vfr[2][2][2];
+    auto read_v = [&](int pt) {
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int ts = 0; ts < 2; ++ts) {
+          const int db = 2 * pt + d;
+          uintx4 a;
+#pragma unroll
+          for (int jh = 0; jh < 2; ++jh) {
+            const short4v rr = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (short4v __attribute__((address_space(3)))*)(lds_v + (vbase ^ (64 * (db & 3))) + 256 * (db >> 2) + (16 * ts + 8 * jh) * ROWB));
+            const uintx2 r2 = __builtin_bit_cast(uintx2, rr);
+            a[2 * jh] = r2[0]; a[2 * jh + 1] = r2[1];
+          }
+          vfr[pt & 1][d][ts] = a;
+        }
+    };
+    read_v(0);
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt) {
+      if (pt < 3) read_v(pt + 1);
+      if (pt == 3) {
+        lds_wait();
+        __syncthreads();                            // all wavefronts hold their V fragments: the V buffer is free
+        if (has1) v_copy(cbn);
+      }
+#pragma unroll
+      for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          uintx4 a = vfr[pt & 1][d][ts];
+          if constexpr (BF16 && !PB) a = bf16x8_to_f16x8(a);
+          oacc[2 * pt + d][0] = mfma_qk<PB>(a, pf[ts], oacc[2 * pt + d][0]);
+        }
+    }
+    if (has1) {
+      wait_vm<COPIES>();                              // this wavefront's part of K(t+1) has landed (V(t+1) may be in flight)
+      __syncthreads();                              // ... and the others'
+    }
+  }
+
+  // ---- the key halves meet: each hands over the columns the other finishes ----
+  // (after the last tile's barriers nobody reads a tile or a column any more: all of the LDS is free)
+  const float lsum = l_i + __shfl_xor(l_i, 32);
+  const float m_own = lsum != 0.f ? m_i : -INFINITY;       // (a sum that is not a number stays in)
+  float* ml = reinterpret_cast<float*>(lds + WIDE_COLS_OFF);    // (m, l) per half and query
+  if (g == 0) { ml[(64 * kh + 32 * w + ln) * 2] = m_own; ml[(64 * kh + 32 * w + ln) * 2 + 1] = lsum; }
+  floatx4* give = reinterpret_cast<floatx4*>(lds) + (2 * (1 - kh) + w) * (DB / 2) * 4 * 64 + lane;
+  const floatx4* take = reinterpret_cast<const floatx4*>(lds) + (2 * kh + w) * (DB / 2) * 4 * 64 + lane;
+  floatx16 res[DB / 2];
+#pragma unroll
+  for (int db = 0; db < DB / 2; ++db) {
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      floatx4 x;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[e] = kh == 0 ? oacc[DB / 2 + db][0][4 * i4 + e] : oacc[db][0][4 * i4 + e];
+      give[(4 * db + i4) * 64] = x;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) res[db][i] = kh == 0 ? oacc[db][0][i] : oacc[DB / 2 + db][0][i];
+  }
+  __syncthreads();
+  const int other = (64 * (1 - kh) + 32 * w + ln) * 2;
+  const float m_oth = ml[other], l_oth = ml[other + 1], M = fmaxf(m_own, m_oth);
+  const float wo = m_own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_own - M);
+  const float wt = m_oth == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_oth - M);
+  const float L = wo * lsum + wt * l_oth;
+#pragma unroll
+  for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const floatx4 x = take[(4 * db + i4) * 64];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) res[db][4 * i4 + e] = wo * res[db][4 * i4 + e] + wt * x[e];
+    }
+  if (prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
+    float* part = prm.part_o + ((int64_t)chunk * BH + bh) * prm.N * D;
+#pragma unroll
+    for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+      for (int i4 = 0; i4 < 4; ++i4)
+        store_out4<BF16>(part, qrow * D + 128 * kh + 32 * db + 8 * i4 + 4 * g, true, res[db][4 * i4], res[db][4 * i4 + 1],
+                         res[db][4 * i4 + 2], res[db][4 * i4 + 3]);
+    if (g == 0 && kh == 0) {
+      float* pml = prm.part_ml + (((int64_t)chunk * BH + bh) * prm.N + qrow) * 2;
+      pml[0] = M; pml[1] = L;
+    }
+    return;
+  }
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
+  rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
+                        prm.out_f32, lane, 32, [&](int db, int i) { return res[db][i] * inv; });
+  if (prm.lse != nullptr && kh == 0 && g == 0) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(L == L ? M : L, L);
+}
+
+template <int DT, bool CONTIG>
+static void launch_wide_c(const FwdParams& prm, hipStream_t st) {
+  static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
+  once_per_device(configured, [] {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              WIDE_LDS_BYTES);
+  });
+  const int grid = prm.place.per_share * prm.split;
+  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
+}
+
+template <int DT>
+static void launch_wide_t(const FwdParams& prm, hipStream_t st) {
+  if (prm.ks[2] == WIDE_D && prm.vs[2] == WIDE_D) launch_wide_c<DT, true>(prm, st);
+  else launch_wide_c<DT, false>(prm, st);
+}
+
+void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st);   // attn_fwd_pair.hip
+
+// Block masks, N a multiple of 64.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st) {
+  if (dt == 0) launch_wide_t<0>(prm, st);
+  else if (dt == 1) launch_wide_t<1>(prm, st);
+  else launch_wide_t<2>(prm, st);
+  if (prm.split > 1) launch_sum_parts(prm, WIDE_D, dt != 0, st);
+}
+
+}  // namespace bsattn

@@ -68,6 +68,24 @@ __device__ __forceinline__ float softmax_tile(const floatx16& s0, const floatx16
   return l;
 }
 
+// The same for one block of 32 keys.
+template <bool FOLD, bool PB>
+__device__ __forceinline__ float softmax_block(const floatx16& s, float qk_scale, float m, float l, uintx4 (&pf)[2]) {
+#pragma unroll
+  for (int ts = 0; ts < 2; ++ts) {
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int i = 8 * ts + 2 * jj;
+      const float p0 = __builtin_amdgcn_exp2f(FOLD ? s[i] : __builtin_fmaf(s[i], qk_scale, -m));
+      const float p1 = __builtin_amdgcn_exp2f(FOLD ? s[i + 1] : __builtin_fmaf(s[i + 1], qk_scale, -m));
+      const unsigned int hp = pack2<PB>(p0, p1);
+      l = add_packed2<PB>(hp, l);
+      pf[ts][jj] = hp;
+    }
+  }
+  return l;
+}
+
 // The kept columns of row block m, ascending, from the block mask into cols (LDS), by every wavefront of the workgroup by
 // itself (all write the same): no list kernels in front of the launch, and one dependent access instead of two (row
 // pointer, then column).  Returns their number, at most nb <= MAX.
@@ -109,16 +127,11 @@ __device__ __forceinline__ float row_lse(float m, float l) {
 // maximum of the current tile and redo the tile's numerators.
 // With elementwise masks (EW) a query may have had nothing but masked keys so far (l == 0, or the
 // whole tile masked: maximum -inf): such a lane takes the tile's maximum as its first reference.
-template <int DB, bool FOLD, bool EW>
-__device__ __forceinline__ void recentre(floatx16& s0, floatx16& s1, floatx16 (&oacc)[DB][2], int qb, float qk_scale,
-                                      float& m, float& l, uintx4& mfrag, bool fresh, int g) {
-  float mx = max3f(s0[0], s0[1], s0[2]);
-#pragma unroll
-  for (int i = 3; i < 15; i += 2) mx = max3f(mx, s0[i], s0[i + 1]);
-  mx = max3f(mx, s0[15], s1[0]);
-#pragma unroll
-  for (int i = 1; i < 15; i += 2) mx = max3f(mx, s1[i], s1[i + 1]);
-  mx = xhalf_max(fmaxf(mx, s1[15]));
+// recentre_on: the reference, l and the accumulators, from the lane's maximum; returns what the scores are to be lowered by (FOLD).
+template <int DB, int NQ, bool FOLD, bool EW>
+__device__ __forceinline__ float recentre_on(float mx, floatx16 (&oacc)[DB][NQ], int qb, float qk_scale, float& m, float& l,
+                                             uintx4& mfrag, bool fresh, int g) {
+  mx = xhalf_max(mx);
   // exponent of the largest entry relative to the current reference
   const float smax = FOLD ? mx : __builtin_fmaf(mx, qk_scale, -m);
   float delta = fresh ? smax : fmaxf(smax, 0.f);
@@ -140,12 +153,41 @@ __device__ __forceinline__ void recentre(floatx16& s0, floatx16& s1, floatx16 (&
       for (int i = 0; i < 16; ++i) oacc[db][qb][i] *= alpha;
   }
   if constexpr (FOLD) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) { s0[i] -= delta; s1[i] -= delta; }
     const _Float16 hi = (_Float16)(-m);
     const _Float16 lo = (_Float16)(-m - (float)hi);
     const half2v hl = {hi, lo};
     mfrag[0] = g == 0 ? __builtin_bit_cast(unsigned int, hl) : 0u;
+  }
+  return delta;
+}
+
+template <int DB, bool FOLD, bool EW>
+__device__ __forceinline__ void recentre(floatx16& s0, floatx16& s1, floatx16 (&oacc)[DB][2], int qb, float qk_scale,
+                                      float& m, float& l, uintx4& mfrag, bool fresh, int g) {
+  float mx = max3f(s0[0], s0[1], s0[2]);
+#pragma unroll
+  for (int i = 3; i < 15; i += 2) mx = max3f(mx, s0[i], s0[i + 1]);
+  mx = max3f(mx, s0[15], s1[0]);
+#pragma unroll
+  for (int i = 1; i < 15; i += 2) mx = max3f(mx, s1[i], s1[i + 1]);
+  const float delta = recentre_on<DB, 2, FOLD, EW>(fmaxf(mx, s1[15]), oacc, qb, qk_scale, m, l, mfrag, fresh, g);
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) { s0[i] -= delta; s1[i] -= delta; }
+  }
+}
+
+// The same for one block of 32 keys.
+template <int DB, bool FOLD>
+__device__ __forceinline__ void recentre_block(floatx16& s, floatx16 (&oacc)[DB][1], float qk_scale, float& m, float& l,
+                                               uintx4& mfrag, bool fresh, int g) {
+  float mx = max3f(s[0], s[1], s[2]);
+#pragma unroll
+  for (int i = 3; i < 15; i += 2) mx = max3f(mx, s[i], s[i + 1]);
+  const float delta = recentre_on<DB, 1, FOLD, false>(fmaxf(mx, s[15]), oacc, 0, qk_scale, m, l, mfrag, fresh, g);
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] -= delta;
   }
 }
 

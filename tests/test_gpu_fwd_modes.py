@@ -260,3 +260,36 @@ def test_short_lists(dev, H, N, dtype, out_fp32, elementwise):
         ref = torch.logsumexp(s, -1)
         fin = torch.isfinite(ref)
         assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3
+
+# D = 256, whole tiles: a wavefront has half of a tile's keys, and the halves meet with references of their own (`skew`: scores
+# of one half far above the other's, of the second or by turns).  One tile; shares (fewer tiles than shares); none; strided rows.
+@pytest.mark.parametrize("H,N,skew,strided", [(1, 64, 0, False), (2, 1024, 1, False), (4, 2048, 2, True), (24, 1344, 1, True), (9, 2048, 0, False)])
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+def test_halves_of_keys(dev, H, N, skew, strided, dtype, out_fp32):
+    import fa2_custom_mask as fm
+    nb = N // 64
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 256, dtype, 970 + N)]
+    key = torch.arange(N, device=dev)
+    if skew:
+        k[:, :, (key % 64 >= 32) if skew == 1 else ((key // 32 + key // 64) % 2 == 1)] *= 5
+    if strided:
+        q, k, v = torch.stack([q, k, v], 3).unbind(3)
+    block = torch.cat([uniform_block_mask(1, 1, nb, 0.3, 971 + N + h) for h in range(H)], 1)
+    if nb > 1:
+        block[0, 0, 1] = False
+        block[0, 0, 0] = torch.arange(nb) == 1
+    sc = 256 ** -0.5
+    # fp16: the scale is folded into Q, whose rounding (rms 0.41 of 2^-11 per element) moves a score of rms 5 by 1.0e-3 rms; a
+    # numerator moves by as much of itself, lse by at most 6 of these over all queries.  bf16 results: numerators are rounded to
+    # bf16 and summed so, which moves the sum of a query with one dominant key by up to 2^-8.
+    fold = 0.41 * 2.0 ** -11 * 5 if skew and dtype == torch.float16 else 0.0
+    lse_max = 2.0 ** -8 if dtype == torch.bfloat16 and not out_fp32 else 2e-3 + 6 * fold
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, block.to(dev), sc, out_fp32=out_fp32)
+    for h in sorted({0, 1 % H, H // 2, H - 1}):
+        keep = block[0, h].to(dev).repeat_interleave(64, 0).repeat_interleave(64, 1)
+        s = (q[0, h].float() @ k[0, h].float().T * sc).masked_fill(~keep, float("-inf"))
+        ma, rl = errors(o[0, h], torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float())
+        assert ma <= MAXABS[dtype] and rl <= RELL2[torch.float16 if out_fp32 else dtype] + fold, (h, ma, rl)
+        ref = torch.logsumexp(s, -1)
+        fin = torch.isfinite(ref)
+        assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= lse_max
