@@ -1,5 +1,4 @@
-// Block-sparse FlashAttention-2 forward, head dimension 128, and 256 with elementwise masks or a ragged length (one wavefront per
-// SIMD there, K and V fragments taken from LDS in two portions).
+// Block-sparse FlashAttention-2 forward, head dimension 128, and 256 with elementwise masks (one wavefront per SIMD there, K and V fragments taken from LDS in two portions).
 //
 // At D = 128 a wavefront that owns 64 queries would need all 512 registers of its SIMD and be bound by instruction issue.
 // Here a row block belongs to a pair of wavefronts, 32 queries each (256 registers: two
@@ -461,11 +460,14 @@ static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
 
 template <int D>
 static void launch_pair_d(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
-  if (!elementwise) {
-    if (dt == 0) launch_pair_t<D, 0, false>(prm, st);
-    else if (dt == 1) launch_pair_t<D, 1, false>(prm, st);
-    else launch_pair_t<D, 2, false>(prm, st);
-  } else {
+  if constexpr (D == 128) {
+    if (!elementwise) {
+      if (dt == 0) launch_pair_t<D, 0, false>(prm, st);
+      else if (dt == 1) launch_pair_t<D, 1, false>(prm, st);
+      else launch_pair_t<D, 2, false>(prm, st);
+    }
+  }
+  if (elementwise) {
     if (dt == 0) launch_pair_t<D, 0, true>(prm, st);
     else if (dt == 1) launch_pair_t<D, 1, true>(prm, st);
     else launch_pair_t<D, 2, true>(prm, st);
@@ -474,10 +476,10 @@ static void launch_pair_d(const FwdParams& prm, int dt, bool elementwise, hipStr
 
 void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st);   // attn_fwd_wide.hip
 
-// D: 128 or 256 (whole tiles of block masks: attn_fwd_wide.hip, whose registers hold no more).  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+// D: 128 or 256 (block masks: attn_fwd_wide.hip, whose registers do not hold mask words beside the rest).  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st) {
   if (D == 128) launch_pair_d<128>(prm, dt, elementwise, st);
-  else if (!elementwise && prm.N % 64 == 0) launch_fwd_wide(prm, dt, st);
+  else if (!elementwise) launch_fwd_wide(prm, dt, st);
   else launch_pair_d<256>(prm, dt, elementwise, st);
 }
 

@@ -9,9 +9,10 @@
 //
 // Before, fwd_pair_kernel: a wavefront with the scores of all 64 keys, up to 512 registers, alone on its SIMD, so that scores, softmax
 // and second product came one after the other.  us: 16 heads N = 4096 block-causal keep 0.5 bf16 108 -> 96, results in fp32
-// 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  The 256 registers
-// leave no room for mask words or the bounds of a ragged length (20 to 140 spilled): those launches stay on
-// fwd_pair_kernel.
+// 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  Ragged: 16 heads
+// N = 4000 causal keep 0.5 bf16 168 -> 95 (fwd_pair_kernel spilled), 10 heads N = 4090 keep 0.3 142 -> 93, fp16 N = 4065 dense
+// block-causal 214 -> 170.  The 256 registers
+// leave no room for mask words (20 to 140 spilled): elementwise masks stay on fwd_pair_kernel.
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196 of the reference).
 #include "common.h"
@@ -29,7 +30,9 @@ static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the res
 
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
 // CONTIG: the rows of K and of V follow each other without gaps (row stride = 256).
-template <int DT, bool CONTIG>
+// TAIL: N is not a multiple of 64: the copy of the last tile repeats its last key, the scores beyond it are -inf (a half without
+// any key leaves the tile out), the queries beyond N are not written.
+template <int DT, bool CONTIG, bool TAIL>
 __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   constexpr int D = WIDE_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
   constexpr int COPIES = CPR / 4;                // copy instructions per wavefront and tile
@@ -48,9 +51,10 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   const cint_ptr_t rp = (cint_ptr_t)(uintptr_t)(prm.row_ptr + (int64_t)mh * nb);
   // Q of this lane's query depends on the block index only: asked for first, it travels while the list is looked up
   const int64_t qrow = (int64_t)m * 64 + 32 * w + ln;
+  const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64, tail_cb = TAIL ? nb - 1 : -1;
   uintx4 qf[KS];
   {
-    const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + qrow * prm.qs[2];
+    const unsigned short* qp = (const unsigned short*)prm.q + b * prm.qs[0] + h * prm.qs[1] + (!TAIL || qrow < prm.N ? qrow : prm.N - 1) * prm.qs[2];
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
   }
@@ -68,6 +72,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   }
   void* obase = out_base(prm, b, h);
   if (t0 == t1) {                                // no kept tile: O = 0, lse = -inf
+    if (TAIL && qrow >= prm.N) return;
 #pragma unroll
     for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
@@ -111,11 +116,29 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       }
     }
   };
+  // (the lane index as a value the compiler cannot trace back, or the offsets are computed before the loop and held)
+  auto tail_copy = [&](const unsigned short* tile, int64_t rs, unsigned lds_addr, auto&& swz) {
+    int lane_t = lane;
+    asm volatile("" : "+v"(lane_t));
+#pragma unroll 1
+    for (int j = wave * COPIES; j < (wave + 1) * COPIES; ++j) {
+      const int row = j * RPI + lane_t / CPR, src = row < valid ? row : valid - 1;
+      tile_load_async_one(tile, 2u * (unsigned)(src * (int)rs + (((lane_t % CPR) ^ swz(row)) * 8)), lds_addr + j * 1024);
+    }
+  };
   auto k_copy = [&](int cb) {
+    if (TAIL && cb == tail_cb) {
+      tail_copy(kg + (int64_t)cb * 64 * prm.ks[2], prm.ks[2], lds_k_addr, [](int row) { return k_swz<D>(row); });
+      return;
+    }
     tile_copy(kg + (int64_t)cb * 64 * (CONTIG ? (int64_t)D : prm.ks[2]), prm.ks[2], lds_k_addr,
               [&](int j) { return (kx ^ (32u * (j % KPER))) + (CONTIG ? 0u : krow); });
   };
   auto v_copy = [&](int cb) {
+    if (TAIL && cb == tail_cb) {
+      tail_copy(vg + (int64_t)cb * 64 * prm.vs[2], prm.vs[2], lds_v_addr, [](int row) { return v_swz<D>(row); });
+      return;
+    }
     tile_copy(vg + (int64_t)cb * 64 * (CONTIG ? (int64_t)D : prm.vs[2]), prm.vs[2], lds_v_addr,
               [&](int j) { return (vx ^ (128u * (j % VPER))) + (CONTIG ? 0u : vrow); });
   };
@@ -131,9 +154,9 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   const uintx4 ones_frag = {g == 0 ? 0x3c003c00u : 0u, 0u, 0u, 0u};
 
   // first tile's copies (its column from one scalar load), then the column list into LDS
-  const int cb0 = listed ? cols[t0] : __builtin_amdgcn_readfirstlane(lcols[t0]);
-  k_copy(cb0);
-  v_copy(cb0);
+  int cb = listed ? cols[t0] : __builtin_amdgcn_readfirstlane(lcols[t0]);
+  k_copy(cb);
+  v_copy(cb);
   if (listed)
     for (int i = threadIdx.x; i < t1 - t0 && i < WIDE_COLS_CAP; i += 256) lcols[i] = prm.col_idx[t0 + i];
   __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0), visible to the compiler: Q and the first tiles
@@ -189,16 +212,27 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       if (any_m) sc = mfma_qk<BF16>(ones_frag, mfrag, sc);
     }
     uintx4 pf[2];
-    float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-    // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-    const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
-    if (__any(first || !(lnew - l_i < 16384.0f))) {
-      recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
-      any_m = 1;
-      lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+    const int keys = TAIL && cb == tail_cb ? valid - 32 * kh : 32;      // of this half
+    if (TAIL && keys < 32) {
+      int first_key = 4 * g;
+      asm volatile("" : "+v"(first_key));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sc[i] = 8 * (i / 4) + (i % 4) + first_key < keys ? sc[i] : -INFINITY;
     }
-    l_i = lnew;
-    fresh = false;
+    if (TAIL && keys <= 0) {
+      pf[0] = pf[1] = uintx4{0u, 0u, 0u, 0u};
+    } else {
+      float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+      // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
+      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
+      if (__any(first || !(lnew - l_i < 16384.0f))) {
+        recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
+        any_m = 1;
+        lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+      }
+      l_i = lnew;
+      fresh = false;
+    }
     if (has1) wait_vm<COPIES>(); else wait_vm<0>();   // this wavefront's part of V(t) has landed (K(t+1) may be in flight)
     if (t > t0) __syncthreads();                    // ... and the others' (the first tile was waited for above)
     // ---- O^T += V^T P^T, V^T fragments in portions of two column blocks ----
@@ -242,6 +276,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       wait_vm<COPIES>();                              // this wavefront's part of K(t+1) has landed (V(t+1) may be in flight)
       __syncthreads();                              // ... and the others'
     }
+    if constexpr (TAIL) cb = cbn;
   }
 
   // ---- the key halves meet: each hands over the columns the other finishes ----
@@ -280,6 +315,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       for (int e = 0; e < 4; ++e) res[db][4 * i4 + e] = wo * res[db][4 * i4 + e] + wt * x[e];
     }
   if (prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
+    if (TAIL && qrow >= prm.N) return;
     float* part = prm.part_o + ((int64_t)chunk * BH + bh) * prm.N * D;
 #pragma unroll
     for (int db = 0; db < DB / 2; ++db)
@@ -296,30 +332,31 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   const float inv = L > 0.f ? 1.0f / L : 0.f;
   __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
   rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
-                        prm.out_f32, lane, 32, [&](int db, int i) { return res[db][i] * inv; });
-  if (prm.lse != nullptr && kh == 0 && g == 0) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(L == L ? M : L, L);
+                        prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });
+  if (prm.lse != nullptr && kh == 0 && g == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(L == L ? M : L, L);
 }
 
-template <int DT, bool CONTIG>
+template <int DT, bool CONTIG, bool TAIL>
 static void launch_wide_c(const FwdParams& prm, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize,
                               WIDE_LDS_BYTES);
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
+  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG, TAIL>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
 }
 
 template <int DT>
 static void launch_wide_t(const FwdParams& prm, hipStream_t st) {
-  if (prm.ks[2] == WIDE_D && prm.vs[2] == WIDE_D) launch_wide_c<DT, true>(prm, st);
-  else launch_wide_c<DT, false>(prm, st);
+  const bool contig = prm.ks[2] == WIDE_D && prm.vs[2] == WIDE_D;
+  if (prm.N % 64 != 0) { if (contig) launch_wide_c<DT, true, true>(prm, st); else launch_wide_c<DT, false, true>(prm, st); }
+  else { if (contig) launch_wide_c<DT, true, false>(prm, st); else launch_wide_c<DT, false, false>(prm, st); }
 }
 
 void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st);   // attn_fwd_pair.hip
 
-// Block masks, N a multiple of 64.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+// Block masks.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
 void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st) {
   if (dt == 0) launch_wide_t<0>(prm, st);
   else if (dt == 1) launch_wide_t<1>(prm, st);

@@ -261,13 +261,15 @@ def test_short_lists(dev, H, N, dtype, out_fp32, elementwise):
         fin = torch.isfinite(ref)
         assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3
 
-# D = 256, whole tiles: a wavefront has half of a tile's keys, and the halves meet with references of their own (`skew`: scores
-# of one half far above the other's, of the second or by turns).  One tile; shares (fewer tiles than shares); none; strided rows.
-@pytest.mark.parametrize("H,N,skew,strided", [(1, 64, 0, False), (2, 1024, 1, False), (4, 2048, 2, True), (24, 1344, 1, True), (9, 2048, 0, False)])
+# D = 256, block masks: a wavefront has half of a tile's keys, and the halves meet with references of their own (`skew`: scores
+# of one half far above the other's, of the second or by turns).  One tile; shares (fewer tiles than shares); none; strided rows;
+# ragged lengths with a key or none in the second half of the last tile.
+@pytest.mark.parametrize("H,N,skew,strided", [(1, 64, 0, False), (2, 1024, 1, False), (4, 2048, 2, True), (24, 1344, 1, True), (9, 2048, 0, False),
+                                                (2, 20, 0, False), (2, 33, 0, False), (4, 2000, 1, True), (24, 1313, 2, False)])
 @pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_halves_of_keys(dev, H, N, skew, strided, dtype, out_fp32):
     import fa2_custom_mask as fm
-    nb = N // 64
+    nb = -(-N // 64)
     q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 256, dtype, 970 + N)]
     key = torch.arange(N, device=dev)
     if skew:
@@ -286,7 +288,7 @@ def test_halves_of_keys(dev, H, N, skew, strided, dtype, out_fp32):
     lse_max = 2.0 ** -8 if dtype == torch.bfloat16 and not out_fp32 else 2e-3 + 6 * fold
     o, lse = fm.flash_attention_custom_mask_lse(q, k, v, block.to(dev), sc, out_fp32=out_fp32)
     for h in sorted({0, 1 % H, H // 2, H - 1}):
-        keep = block[0, h].to(dev).repeat_interleave(64, 0).repeat_interleave(64, 1)
+        keep = block[0, h].to(dev).repeat_interleave(64, 0)[:N].repeat_interleave(64, 1)[:, :N]
         s = (q[0, h].float() @ k[0, h].float().T * sc).masked_fill(~keep, float("-inf"))
         ma, rl = errors(o[0, h], torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float())
         assert ma <= MAXABS[dtype] and rl <= RELL2[torch.float16 if out_fp32 else dtype] + fold, (h, ma, rl)
