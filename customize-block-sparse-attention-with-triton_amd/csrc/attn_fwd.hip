@@ -312,6 +312,7 @@ void fwd_kernel(const FwdRangeParams prm) {
   // FOLD: "-m_i" enters the scores through one extra contraction slice, ones x (-m_hi, -m_lo)
   uintx4 mfrag[2];
   bool fresh = true;
+  float limit[2] = {SUM_LIMIT, SUM_LIMIT};
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
 
   auto reset_acc = [&]() {
@@ -322,7 +323,7 @@ void fwd_kernel(const FwdRangeParams prm) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) oacc[db][qb][i] = 0.f;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) { m_i[qb] = 0.f; l_i[qb] = 0.f; mfrag[qb] = uintx4{0u, 0u, 0u, 0u}; }
+    for (int qb = 0; qb < 2; ++qb) { m_i[qb] = 0.f; l_i[qb] = 0.f; mfrag[qb] = uintx4{0u, 0u, 0u, 0u}; limit[qb] = FOLD || EW ? SUM_LIMIT : 0.f; }
     fresh = true;
     any_m = 0;
   };
@@ -429,11 +430,12 @@ void fwd_kernel(const FwdRangeParams prm) {
     // and the numerators are redone from the scores, which are still live.
     auto settle = [&](int qb, floatx16& s0, floatx16& s1, float lnew) {
       // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
-      if (__any(first || (EW && l_i[qb] == 0.f) || !(lnew - l_i[qb] < 16384.0f))) {
+      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : EW && fresh;
+      if (__any(first || (EW && l_i[qb] == 0.f) || !(lnew - l_i[qb] < limit[qb]))) {
         recentre<DB, FOLD, EW>(s0, s1, oacc, qb, qk_scale, m_i[qb], l_i[qb], mfrag[qb], fresh, g);
         any_m = 1;
         lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i[qb], l_i[qb], pf, qb);
+        limit[qb] = sum_limit<EW>(lnew);
       }
       l_i[qb] = lnew;
     };
@@ -578,7 +580,7 @@ void fwd_kernel(const FwdRangeParams prm) {
     for (int qb = 0; qb < 2; ++qb) lsum[qb] = l_i[qb] + __shfl_xor(l_i[qb], 32);
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
-      const float inv = lsum[qb] > 0.f ? 1.0f / lsum[qb] : 0.f;      // no unmasked key at all: O = 0
+      const float inv = row_inverse<EW>(lsum[qb]);
       const int64_t qrow = (int64_t)(row * 64 + qb * 32 + ln);
       if (!exists(qrow)) continue;
 #pragma unroll
@@ -1078,7 +1080,7 @@ void fwd_kernel(const FwdRangeParams prm) {
               for (int e = 0; e < 4; ++e) x[e] += wgt[pw][qb] * src[(4 * quad + e) * 64 + lane];
             }
             if (full) {
-              const float inv = L[qb] > 0.f ? 1.0f / L[qb] : 0.f;
+              const float inv = row_inverse<EW>(L[qb]);
               const int64_t qrow = (int64_t)(r * 64 + qb * 32 + ln);
               if (exists(qrow))
                 store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32, x[0] * inv, x[1] * inv,
@@ -1200,7 +1202,7 @@ void fwd_kernel(const FwdRangeParams prm) {
               for (int tq = 0; tq < C::QPW; ++tq) {
                 const int idx0 = rd * C::R + 4 * (w * C::QPW + tq);
                 const int db = idx0 / 32, qb = (idx0 / 16) & 1, i4 = (idx0 & 15) / 4;
-                const float inv = Ls[qb] > 0.f ? 1.0f / Ls[qb] : 0.f;
+                const float inv = row_inverse<EW>(Ls[qb]);
                 const int64_t qrow = (int64_t)(r * 64 + qb * 32 + ln);
                 if (exists(qrow)) store_out4<BF16>(obase, qrow * prm.os[2] + 32 * db + 8 * i4 + 4 * g, prm.out_f32,
                                  acc[rd][tq][0] * inv, acc[rd][tq][1] * inv, acc[rd][tq][2] * inv, acc[rd][tq][3] * inv);

@@ -219,6 +219,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   float m_i = 0.f, l_i = EW && TAIL && !exists ? 1e-30f : 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
+  float limit = FOLD || EW ? SUM_LIMIT : 0.f;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
   __syncthreads();                                  // both halves of K(t0) and V(t0) and the column list are in LDS
 
@@ -310,11 +311,12 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
     auto numerators = [&]() {
       float lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
       // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
-      if (__any(first || (EW && l_i == 0.f) || !(lnew - l_i < 16384.0f))) {
+      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : EW && fresh;
+      if (__any(first || (EW && l_i == 0.f) || !(lnew - l_i < limit))) {
         recentre<DB, FOLD, EW>(s0, s1, oacc, 0, qk_scale, m_i, l_i, mfrag, fresh, g);
         any_m = 1;
         lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
+        limit = sum_limit<EW>(lnew);
       }
       l_i = lnew;
       fresh = false;
@@ -366,7 +368,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
     }
     return;
   }
-  const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+  const float inv = row_inverse<EW>(lsum);
   // the wavefront's 32 rows of O leave through its half of the (now idle) LDS
   static_assert(2 * rows_out_bytes(D, true) <= pair_lds_bytes<D>(), "room for the result rows of both wavefronts");
   __syncthreads();           // the other wavefront has left its last tile
@@ -417,7 +419,7 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
       acc += wgt * part[c];
     }
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const float inv = len > 0 && prm.tile_bits == nullptr ? row_inverse<false>(L) : row_inverse<true>(L);
   store_out4<BF16>(out_base(prm, b, h), (int64_t)row * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv,
                    acc[3] * inv);
   if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + row] = row_lse(M, L);

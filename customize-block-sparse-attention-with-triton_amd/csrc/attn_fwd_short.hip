@@ -162,6 +162,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   float m_i = 0.f, l_i = EW && TAIL && qrow >= prm.N ? 1e-30f : 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
+  float limit = FOLD || EW ? SUM_LIMIT : 0.f;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
 
   const int steps = (t1 - t0 + S - 1) / S;
@@ -235,11 +236,12 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
       uintx4 pf[4][2];
       float lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
       // (FOLD: the first tile keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
-      if (__any(first || (EW && l_i == 0.f) || !(lnew - l_i < 16384.0f))) {
+      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : EW && fresh;
+      if (__any(first || (EW && l_i == 0.f) || !(lnew - l_i < limit))) {
         recentre<DB, FOLD, EW>(s0, s1, oacc, 0, qk_scale, m_i, l_i, mfrag, fresh, g);
         any_m = 1;
         lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
+        limit = sum_limit<EW>(lnew);
       }
       l_i = lnew;
       fresh = false;
@@ -300,7 +302,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
       *reinterpret_cast<floatx4*>(prm.part_o + at * D + col) = acc;
       if (col == 0) { prm.part_ml[at * 2] = M; prm.part_ml[at * 2 + 1] = L; }
     } else {
-      const float inv = L > 0.f ? 1.0f / L : 0.f;     // (no kept tile or no key: O = 0)
+      const float inv = EW || steps == 0 ? row_inverse<true>(L) : row_inverse<false>(L);     // (no kept tile or no key: O = 0)
       store_out4<BF16>(obase, q * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
       if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + q] = row_lse(L == L ? M : L, L);
     }

@@ -177,6 +177,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   float m_i = 0.f, l_i = 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
+  float limit = FOLD ? SUM_LIMIT : 0.f;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
   __syncthreads();                                  // all of K(t0), V(t0) and the column list are in LDS
 
@@ -224,11 +225,12 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
     } else {
       float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
       // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : fresh;
-      if (__any(first || !(lnew - l_i < 16384.0f))) {
+      const bool first = FOLD && fresh && !(lnew >= 0.25f);
+      if (__any(first || !(lnew - l_i < limit))) {
         recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
         any_m = 1;
         lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+        limit = sum_limit<false>(lnew);
       }
       l_i = lnew;
       fresh = false;
@@ -329,7 +331,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
     }
     return;
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const float inv = row_inverse<false>(L);
   __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
   rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
                         prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });

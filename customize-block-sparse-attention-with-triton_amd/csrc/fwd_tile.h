@@ -123,10 +123,31 @@ __device__ __forceinline__ float row_lse(float m, float l) {
   return l == 0.f || m == -INFINITY ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
 
+// 1 / l for a row with at least one kept tile.  Elementwise masks (EW) may leave a query without a key, whose row of O is 0; with a
+// block mask a sum of 0 says that all scores are -inf, and 0 times infinity gives what softmax gives there: not a number.
+template <bool EW>
+__device__ __forceinline__ float row_inverse(float l) { return EW && !(l > 0.f) ? 0.f : 1.0f / l; }
+
+// Which queries of the wavefront have no mass yet: bit q (and q + 32, its other lane) is set if both lanes' sums are 0.
+__device__ __forceinline__ unsigned long long no_mass(float l) {
+  const unsigned long long zero = __ballot(l == 0.f);
+  return zero & (zero >> 32 | zero << 32);
+}
+
+// A lane whose sum grows by this in a tile calls for a new reference exponent: some P left the safe fp16 range.
+constexpr float SUM_LIMIT = 16384.0f;
+// The limit after a tile that got one: 0, which every tile reaches, while some query has no mass.  (EW: the lanes look at their sums.)
+template <bool EW>
+__device__ __forceinline__ float sum_limit(float l) {
+  if constexpr (EW) return SUM_LIMIT;
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(no_mass(l) != 0ull ? 0 : __builtin_bit_cast(int, SUM_LIMIT)));
+}
+
 // Rare path of the softmax: re-centre the reference exponent of one query block on the row
 // maximum of the current tile and redo the tile's numerators.
-// With elementwise masks (EW) a query may have had nothing but masked keys so far (l == 0, or the
-// whole tile masked: maximum -inf): such a lane takes the tile's maximum as its first reference.
+// A query may have had nothing but masked keys (EW) or scores of -inf so far (l == 0, or the whole tile: maximum -inf, which is no
+// reference: -inf less -inf is not a number).  Such a lane takes the first finite maximum as its reference; until every query has
+// one, block masks' kernels come here in each tile (sum_limit), as with EW they do for every lane whose own sum is 0.
 // recentre_on: the reference, l and the accumulators, from the lane's maximum; returns what the scores are to be lowered by (FOLD).
 template <int DB, int NQ, bool FOLD, bool EW>
 __device__ __forceinline__ float recentre_on(float mx, floatx16 (&oacc)[DB][NQ], int qb, float qk_scale, float& m, float& l,
@@ -134,17 +155,13 @@ __device__ __forceinline__ float recentre_on(float mx, floatx16 (&oacc)[DB][NQ],
   mx = xhalf_max(mx);
   // exponent of the largest entry relative to the current reference
   const float smax = FOLD ? mx : __builtin_fmaf(mx, qk_scale, -m);
-  float delta = fresh ? smax : fmaxf(smax, 0.f);
-  bool nomass = false;
-  if constexpr (EW) {
-    // (a query's keys are split over two lanes, which must keep one common reference: the mass is
-    // the sum of both halves, or a lane whose own keys were all masked would drift away)
-    nomass = !fresh && l + __shfl_xor(l, 32) == 0.f;
-    if (nomass) delta = smax;
-    if (smax == -INFINITY) delta = 0.f;
-  }
+  // (a query's keys are split over two lanes, which must keep one common reference: the mass is
+  // the sum of both halves, or a lane whose own keys were all masked would drift away)
+  const bool nomass = (EW && fresh) || __builtin_amdgcn_inverse_ballot_w64(no_mass(l));
+  float delta = nomass ? smax : fmaxf(smax, 0.f);
+  if (smax == -INFINITY) delta = 0.f;
   m += delta;
-  if (!fresh) {
+  if (EW ? !fresh : __any(!nomass)) {
     const float alpha = nomass ? 1.0f : __builtin_amdgcn_exp2f(-delta);
     l *= alpha;
 #pragma unroll

@@ -72,3 +72,38 @@ def test_ranges_and_row_blocks(dev, D, H, N, elementwise, dtype, what):
 @pytest.mark.parametrize("N,elementwise", [(8256, False), (8300, True)])
 def test_ranges_of_long_heads(dev, N, elementwise, what):
     check(dev, 1, N, 64, torch.float16, elementwise, what)
+
+
+# Keys whose scores are -inf for every query (a bias column of K that Q picks up): half of every tile, the first tiles of every
+# row, all keys but one of a row block.  A wavefront's first tile, half tile or share may then hold nothing else: the result is
+# the softmax over the other keys, and not a number (lse -inf) where there are none, however the launch splits its lists.
+#   D = 64: pairs of wavefronts (4, with 4 shares, 2), ranges of workgroups, of wavefronts, row blocks; D = 128 and 256: shared
+#   lists, whole ones, ragged lengths
+@pytest.mark.parametrize("hidden", ["first halves", "second halves", "first tiles", "all but one"])
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("D,H,N", [(64, 3, 1000), (64, 1, 4096), (64, 16, 3072), (64, 1, 8300), (64, 12, 8192), (64, 160, 1300),
+                                   (128, 2, 1024), (128, 100, 700), (256, 2, 1024), (256, 2, 1000), (256, 100, 704)])
+def test_scores_of_minus_infinity(dev, D, H, N, dtype, out_fp32, hidden):
+    import fa2_custom_mask as fm
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, D, dtype, 950 + N + D)]
+    key = torch.arange(N, device=dev)
+    if hidden == "all but one":
+        gone = key != N - 5
+    else:
+        gone = {"first halves": key % 64 < 32, "second halves": key % 64 >= 32, "first tiles": key < 192}[hidden]
+    q[..., 0] = 1.0
+    k[..., 0] = 0.0
+    k[:, :, gone, 0] = float("-inf")
+    nb = -(-N // 64)
+    tiles = torch.ones(nb, nb, dtype=torch.bool, device=dev).tril()
+    keep = tiles.repeat_interleave(64, 0).repeat_interleave(64, 1)[:N, :N]
+    sc = D ** -0.5
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, tiles[None, None], sc, out_fp32=out_fp32)
+    for h in sorted({0, H - 1}):
+        s = (q[0, h].double() @ k[0, h].double().T * sc).masked_fill(~keep, float("-inf"))
+        ref, ref_lse = torch.softmax(s, -1) @ v[0, h].double(), torch.logsumexp(s, -1)
+        none = torch.isnan(ref).all(-1)
+        assert torch.equal(torch.isnan(o[0, h]), none[:, None].expand(N, D))
+        assert torch.equal(lse[0, h] == float("-inf"), none) and not bool(torch.isnan(lse[0, h]).any())
+        assert float((o[0, h] - ref)[~none].abs().max()) <= MAXABS[dtype]
+        assert float((lse[0, h] - ref_lse)[~none].abs().max()) <= (2e-3 if out_fp32 or dtype == torch.float16 else 2.0 ** -8)
