@@ -304,7 +304,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
     } else {
       const float inv = EW || steps == 0 ? row_inverse<true>(L) : row_inverse<false>(L);     // (no kept tile or no key: O = 0)
       store_out4<BF16>(obase, q * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-      if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + q] = row_lse(L == L ? M : L, L);
+      if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + q] = row_lse(M, L);
     }
   }
 }

@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
   rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
                         prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });
-  if (prm.lse != nullptr && kh == 0 && g == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(L == L ? M : L, L);
+  if (prm.lse != nullptr && kh == 0 && g == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(M, L);
 }
 
 template <int DT, bool CONTIG, bool TAIL>

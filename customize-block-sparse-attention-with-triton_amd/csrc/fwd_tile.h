@@ -118,9 +118,10 @@ __device__ __forceinline__ void* out_base(const FwdParams& prm, int b, int h) {
 }
 
 // Natural logarithm of the sum of exponentials of a row with reference exponent m and sum l of its numerators: -inf
-// for a row without mass (l = 0) or with no score above -inf (m = -inf), NaN where a score is not a number.
+// for a row without mass (l = 0: no key, or no score above -inf), NaN where a score is not a number.  (The largest of the references of
+// several parts leaves out those that are not numbers, and may be -inf then: the sum says what the row is.)
 __device__ __forceinline__ float row_lse(float m, float l) {
-  return l == 0.f || m == -INFINITY ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
+  return l == 0.f ? -INFINITY : (m + __builtin_amdgcn_logf(l)) * 0.6931471805599453f;
 }
 
 // 1 / l for a row with at least one kept tile.  Elementwise masks (EW) may leave a query without a key, whose row of O is 0; with a

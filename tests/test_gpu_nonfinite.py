@@ -43,6 +43,7 @@ def check(dev, H, N, D, dtype, elementwise, what):
     assert 0 < int(bad.sum()) < N
     assert torch.equal(torch.isnan(o[0, 0]), bad[:, None].expand(N, D))
     assert torch.equal(torch.isfinite(lse[0, 0]), ~bad)
+    assert bool(torch.isnan(lse[0, 0])[torch.isnan(ref_lse)].all())          # (-inf would say that there is no key)
     assert float((o[0, 0] - ref)[~bad].abs().max()) <= MAXABS[dtype]
     assert float((lse[0, 0] - ref_lse)[~bad].abs().max()) <= 2e-3
     assert bool(torch.isfinite(o[:, 1:]).all()) and bool(torch.isfinite(lse[:, 1:]).all())
@@ -69,9 +70,9 @@ def test_ranges_and_row_blocks(dev, D, H, N, elementwise, dtype, what):
 
 # D = 64: ranges of workgroups (more row blocks than the kernel for short lists takes)
 @pytest.mark.parametrize("what", ["key", "query", "inf"])
-@pytest.mark.parametrize("N,elementwise", [(8256, False), (8300, True)])
-def test_ranges_of_long_heads(dev, N, elementwise, what):
-    check(dev, 1, N, 64, torch.float16, elementwise, what)
+@pytest.mark.parametrize("H,N,elementwise,dtype", [(1, 8256, False, torch.float16), (1, 8300, True, torch.float16), (3, 8300, False, torch.bfloat16)])
+def test_ranges_of_long_heads(dev, H, N, elementwise, dtype, what):
+    check(dev, H, N, 64, dtype, elementwise, what)
 
 
 # Keys whose scores are -inf for every query (a bias column of K that Q picks up): half of every tile, the first tiles of every
