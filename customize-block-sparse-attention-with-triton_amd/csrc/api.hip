@@ -241,11 +241,11 @@ int bsattn_fwd_takes_mask(int B, int H, int N, int D) {
   return check_attn(1, 1, B, H, N, D, BSATTN_F16, BSATTN_F16, true) == BSATTN_OK && launch_fwd_takes_mask(B, H, N, D) ? 1 : 0;
 }
 
-int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
-                           const int64_t* mask_strides, int Bm, int Hm, int B, int H, int N, int D, int dtype,
-                           int out_dtype, float sm_scale, const int64_t* q_strides, const int64_t* k_strides,
-                           const int64_t* v_strides, const int64_t* o_strides, void* workspace, size_t workspace_bytes,
-                           void* stream) {
+int bsattn_fwd_mask_copy_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+                                const int64_t* mask_strides, uint8_t* block_copy, int Bm, int Hm, int B, int H, int N, int D,
+                                int dtype, int out_dtype, float sm_scale, const int64_t* q_strides, const int64_t* k_strides,
+                                const int64_t* v_strides, const int64_t* o_strides, void* workspace, size_t workspace_bytes,
+                                void* stream) {
   if (block == nullptr || mask_strides == nullptr) return BSATTN_ERR_NULL;
   static const int32_t no_list = 0;
   const int rc = fwd_check(q, k, v, o, &no_list, &no_list, Bm, Hm, B, H, N, D, dtype, out_dtype, q_strides, k_strides,
@@ -260,7 +260,17 @@ int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o,
   for (int i = 0; i < 3; ++i) { s.qs[i] = q_strides[i]; s.ks[i] = k_strides[i]; s.vs[i] = v_strides[i]; s.os[i] = o_strides[i]; s.dos[i] = 0; }
   s.mask = block;
   for (int i = 0; i < 4; ++i) s.ms[i] = mask_strides[i];
+  s.mask_copy = block_copy;
   return launch_fwd(q, k, v, o, lse, nullptr, nullptr, nullptr, nullptr, s, workspace, (hipStream_t)stream);
+}
+
+int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const uint8_t* block,
+                           const int64_t* mask_strides, int Bm, int Hm, int B, int H, int N, int D, int dtype,
+                           int out_dtype, float sm_scale, const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* o_strides, void* workspace, size_t workspace_bytes,
+                           void* stream) {
+  return bsattn_fwd_mask_copy_tokens(q, k, v, o, lse, block, mask_strides, nullptr, Bm, Hm, B, H, N, D, dtype, out_dtype, sm_scale,
+                                     q_strides, k_strides, v_strides, o_strides, workspace, workspace_bytes, stream);
 }
 
 int bsattn_fwd_tokens(const void* q, const void* k, const void* v, void* o, float* lse, const int32_t* row_ptr,

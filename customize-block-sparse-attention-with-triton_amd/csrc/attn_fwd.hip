@@ -1542,6 +1542,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   FwdRangeParams prm;
   prm.q = q; prm.k = k; prm.v = v; prm.o = o; prm.lse = lse;
   prm.mask = s.mask;
+  prm.mask_copy = s.mask_copy;
   for (int i = 0; i < 4; ++i) prm.ms[i] = s.mask != nullptr ? s.ms[i] : 0;
   prm.row_ptr = row_ptr; prm.col_idx = col_idx; prm.ws = (float*)ws;
   prm.tile_partial = tile_partial; prm.tile_bits = (const unsigned long long*)tile_bits;

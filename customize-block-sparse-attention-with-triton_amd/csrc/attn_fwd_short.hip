@@ -64,7 +64,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   const bool listed = EW || prm.mask == nullptr;
   int t0, t1;
   if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
-  else { t0 = 0; t1 = columns_of_row<SHORT_MAX_BLOCKS>(prm, b, h, m, lane, lcols); }
+  else { t0 = 0; t1 = columns_of_row<SHORT_MAX_BLOCKS>(prm, b, h, m, lane, lcols, chunk == 0 && wave == 0); }
   if (prm.split > 1) {                            // this workgroup's share of the row block's list
     const int len = t1 - t0;
     if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   const bool listed = prm.mask == nullptr;
   int t0, t1;
   if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
-  else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols); }
+  else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols, chunk == 0 && wave == 0); }
   if (prm.split > 1) {                           // this workgroup's share of the row block's list
     const int len = t1 - t0;
     if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;

@@ -32,6 +32,7 @@ struct AttnShape {
   int dtype, out_dtype;
   const uint8_t* mask = nullptr;   // forward: the block mask in place of the lists (launch_fwd_takes_mask), with its strides
   int64_t ms[4];
+  uint8_t* mask_copy = nullptr;    // ... and where the launch leaves what it saw of it, or null
   bool compact = false;   // forward: the split with the smaller workspace (bsattn_fwd_static)
   float sm_scale;
   int64_t qs[3], ks[3], vs[3], os[3], dos[3];  // batch, head, row strides (elements)

@@ -15,6 +15,7 @@ struct FwdParams {
   const int32_t* row_ptr; const int32_t* col_idx;
   const unsigned char* mask;       // the block mask itself in place of the lists (kernels whose workgroups have a row block each), or null
   int64_t ms[4];                   // its strides
+  unsigned char* mask_copy;        // the mask as this launch saw it, [Bm][Hm][nb][nb] of 0 and 1, or null (columns_of_row)
   const unsigned char* tile_partial;        // elementwise masks: per kept tile, 1 = only partly set
   const unsigned long long* tile_bits;      // ... and its 64 row words (bit c = column c)
   float* ws;                       // partial slots of row blocks shared between workgroups (two per workgroup)
@@ -89,8 +90,12 @@ __device__ __forceinline__ float softmax_block(const floatx16& s, float qk_scale
 // The kept columns of row block m, ascending, from the block mask into cols (LDS), by every wavefront of the workgroup by
 // itself (all write the same): no list kernels in front of the launch, and one dependent access instead of two (row
 // pointer, then column).  Returns their number, at most nb <= MAX.
+// writer: the one wavefront of the head's workgroups for this row block that also writes mask_copy, if the heads that share the
+// row have it written by the first of them (a store per 64 columns, against 5 us for a launch that copies the mask).
 template <int MAX>
-__device__ __forceinline__ int columns_of_row(const FwdParams& prm, int b, int h, int m, int lane, int* cols) {
+__device__ __forceinline__ int columns_of_row(const FwdParams& prm, int b, int h, int m, int lane, int* cols, bool writer) {
+  const int mb = prm.Bm > 1 ? b : 0, mhd = prm.Hm > 1 ? h : 0;
+  unsigned char* copy = writer && prm.mask_copy != nullptr && mb == b && mhd == h ? prm.mask_copy + ((int64_t)(mb * prm.Hm + mhd) * prm.nb + m) * prm.nb : nullptr;
   const unsigned char* row = prm.mask + (prm.Bm > 1 ? b : 0) * prm.ms[0] + (prm.Hm > 1 ? h : 0) * prm.ms[1] + m * prm.ms[2];
   constexpr int AHEAD = MAX < 256 ? MAX / 64 : 4;      // accesses on their way at once
   int n = 0;
@@ -105,6 +110,7 @@ __device__ __forceinline__ int columns_of_row(const FwdParams& prm, int b, int h
     for (int i = 0; i < AHEAD; ++i) {
       const unsigned long long bal = __ballot(keep[i]);
       if (keep[i]) cols[n + __popcll(bal & ((1ull << lane) - 1ull))] = c0 + 64 * i + lane;
+      if (copy != nullptr && c0 + 64 * i + lane < prm.nb) copy[c0 + 64 * i + lane] = keep[i];
       n += __popcll(bal);
     }
   }

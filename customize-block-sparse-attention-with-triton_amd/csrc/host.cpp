@@ -32,7 +32,7 @@ struct Library {
   decltype(&::bsattn_fwd_block_mask_workspace) fwd_block_mask_workspace = nullptr;
   decltype(&::bsattn_fwd_block_mask_tokens) fwd_block_mask = nullptr;
   decltype(&::bsattn_fwd_takes_mask) fwd_takes_mask = nullptr;
-  decltype(&::bsattn_fwd_mask_tokens) fwd_mask = nullptr;
+  decltype(&::bsattn_fwd_mask_copy_tokens) fwd_mask = nullptr;
   decltype(&::bsattn_bwd_workspace) bwd_workspace = nullptr;
   decltype(&::bsattn_bwd_tokens) bwd = nullptr;
 } lib;
@@ -53,7 +53,7 @@ void bind(const std::string& path) {
   get(lib.fwd_block_mask_workspace, "bsattn_fwd_block_mask_workspace");
   get(lib.fwd_block_mask, "bsattn_fwd_block_mask_tokens");
   get(lib.fwd_takes_mask, "bsattn_fwd_takes_mask");
-  get(lib.fwd_mask, "bsattn_fwd_mask_tokens");
+  get(lib.fwd_mask, "bsattn_fwd_mask_copy_tokens");
   get(lib.bwd_workspace, "bsattn_bwd_workspace");
   get(lib.bwd, "bsattn_bwd_tokens");
 }
@@ -305,9 +305,10 @@ py::tuple forward_block_mask(const Tensor& q_, const Tensor& k_, const Tensor& v
   return py::make_tuple(results(o, lse, q_.size(3), return_lse), lists);
 }
 
-// Forward straight from a block mask; None where the launch needs its lists (or the mask is on another device).
+// Forward straight from a block mask: (results, the mask as the forward saw it if `keep`, else None).  None where the launch needs
+// the mask's lists (or the mask is on another device).
 py::object forward_mask(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& mask, double sm_scale, bool out_fp32,
-                        bool return_lse) {
+                        bool return_lse, bool keep) {
   check_mask_heads(mask.size(0), mask.size(1), q_);
   const int64_t D_ = q_.size(3) < 64 ? 64 : q_.size(3);
   at::NoGradGuard no_grad;
@@ -317,8 +318,9 @@ py::object forward_mask(const Tensor& q_, const Tensor& k_, const Tensor& v_, co
   const at::ScalarType out_dtype = result_type(q, out_fp32);
   const Tensor o = like(q, out_dtype);
   const int B = (int)q.size(0), H = (int)q.size(1), N = (int)q.size(2), D = (int)q.size(3);
-  Tensor lse;
+  Tensor lse, copy;
   if (return_lse) lse = at::empty({B, H, N}, q.options().dtype(at::kFloat));
+  if (keep) copy = at::empty(mask.sizes(), mask.options());
   size_t bytes = 0;
   check(lib.fwd_workspace(B, H, (int)whole(N), D, &bytes), "bsattn_fwd_workspace");
   const hipStream_t stream = stream_of(q);
@@ -326,11 +328,12 @@ py::object forward_mask(const Tensor& q_, const Tensor& k_, const Tensor& v_, co
     const WorkspaceLock lock;
     const Tensor ws = workspace_locked(bytes, q.device(), stream);
     check(lib.fwd_mask(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(), return_lse ? lse.data_ptr<float>() : nullptr,
-                       (const uint8_t*)mask.const_data_ptr(), mask.strides().data(), (int)mask.size(0), (int)mask.size(1), B, H, N, D,
-                       dtype_code(q.scalar_type()), dtype_code(out_dtype), (float)sm_scale, q.strides().data(), k.strides().data(),
-                       v.strides().data(), o.strides().data(), ws.data_ptr(), bytes, stream), "bsattn_fwd_mask");
+                       (const uint8_t*)mask.const_data_ptr(), mask.strides().data(), keep ? (uint8_t*)copy.data_ptr() : nullptr,
+                       (int)mask.size(0), (int)mask.size(1), B, H, N, D, dtype_code(q.scalar_type()), dtype_code(out_dtype),
+                       (float)sm_scale, q.strides().data(), k.strides().data(), v.strides().data(), o.strides().data(), ws.data_ptr(),
+                       bytes, stream), "bsattn_fwd_mask");
   }
-  return results(o, lse, q_.size(3), return_lse);
+  return py::make_tuple(results(o, lse, q_.size(3), return_lse), keep ? py::cast(copy) : py::none());
 }
 
 // ---- autograd ----

@@ -42,6 +42,8 @@ _SIGNATURES = {
     "bsattn_fwd_takes_mask": ([_i, _i, _i, _i], _i),
     "bsattn_fwd_mask_tokens": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _p, _p, _p, _p,
                                 ctypes.c_size_t, _p], _i),
+    "bsattn_fwd_mask_copy_tokens": ([_p, _p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f, _p, _p, _p, _p, _p,
+                                     ctypes.c_size_t, _p], _i),
     "bsattn_fwd_block_mask": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _p, _p, _p, _i, _i, _i, _i, _i, _i, _f,
                                _p, _p, _p, _p, _p, ctypes.c_size_t, _p], _i),
     "bsattn_fwd_static": ([_p, _p, _p, _p, _p, _p, _p, _i, _i, _i, _i, _i, _i, _i, _i, _f,

@@ -151,14 +151,19 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
     grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     if not grad and (seen is None or seen is UNMADE):
         # launches whose workgroups have a row block each take its columns from a block mask, new or not
-        if seen is None:
+        block = None if seen is None else lists_cache.copy_of(mask, N)
+        if block is not None:
+            made = _host.forward_mask(q, k, v, block, sm_scale, out_fp32, return_lse, False)
+            if made is not None:
+                return made[0]
+        else:
             _check_mask(mask)
-        if seen is UNMADE or is_block_form(mask, N):
-            result = _host.forward_mask(q, k, v, mask, sm_scale, out_fp32, return_lse)
-            if result is not None:
-                if seen is None:
-                    lists_cache.put(mask, N, False, UNMADE)
-                return result
+            if is_block_form(mask, N):
+                made = _host.forward_mask(q, k, v, mask, sm_scale, out_fp32, return_lse, lists_cache.keeps(mask))
+                if made is not None:
+                    if made[1] is not None:
+                        lists_cache.put(mask, N, False, UNMADE, made[1])
+                    return made[0]
     lists = lists_cache.get(mask, N, False)
     if grad:
         if lists is None:

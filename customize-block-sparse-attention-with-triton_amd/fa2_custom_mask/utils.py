@@ -168,7 +168,7 @@ def to_block_mask(mask, N):
 
 
 # In place of the lists of a block mask that forwards so far have done without (they took its rows from the mask itself): they are made
-# when they are asked for.
+# when they are asked for, from the copy of the mask that the first of these forwards has left.
 UNMADE = object()
 
 
@@ -180,7 +180,8 @@ class _ListsCache:
 
     def __init__(self, capacity=8):
         self.capacity = capacity
-        # (id of mask, N, transpose) -> (weakref to mask, version, lists, stream the lists were built on), most recent last
+        # (id of mask, N, transpose) -> (weakref to mask, version, lists, stream the lists were built on, copy of the mask if the
+        # lists are UNMADE), most recent last
         self._entries = collections.OrderedDict()
 
     @staticmethod
@@ -199,32 +200,57 @@ class _ListsCache:
             return None
         return entry[2]
 
+    @staticmethod
+    def _wait(mask, stream):
+        # an entry's lists (or copy of the mask) were filled by kernels on `stream` (a raw handle): work on another stream waits
+        # for what that stream has been given so far (no event is recorded when the lists are made: a mask
+        # that changes with every call would pay for it every time)
+        if _ext.raw_stream(mask.device) == stream:
+            return False
+        torch.cuda.current_stream(mask.device).wait_stream(
+            torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
+        return True
+
     def get(self, mask, N, transpose):
         key = (id(mask), N, transpose)
         entry = self._entries.get(key)
         if entry is None:
             return None
-        ref, version, lists, stream = entry
+        ref, version, lists, stream, block = entry
         if ref() is not mask or self._version(mask) != version:
             return None
         if lists is UNMADE:
-            lists = block_mask_to_lists(mask, transpose=transpose)
+            lists = block_mask_to_lists(self._copy(mask, stream, block), transpose=transpose)
             self.put(mask, N, transpose, lists)
             return lists
-        self._entries.move_to_end(key)
-        # the lists were filled by kernels on `stream` (a raw handle): work on another stream waits for
-        # what that stream has been given so far (no event is recorded when the lists are made: a mask
-        # that changes with every call would pay for it every time)
-        if _ext.raw_stream(mask.device) != stream:
-            torch.cuda.current_stream(mask.device).wait_stream(
-                torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
+        self._entries[key] = self._entries.pop(key, entry)
+        self._wait(mask, stream)
         return lists
 
-    def put(self, mask, N, transpose, lists):
-        # (lists made while a graph is being captured are filled by its replays only, in memory that is the graph's)
-        version = self._version(mask)
-        if version is None or torch.cuda.is_current_stream_capturing():
+    def _copy(self, mask, stream, block):
+        if self._wait(mask, stream) and not torch.cuda.is_current_stream_capturing():
+            block.record_stream(torch.cuda.current_stream(mask.device))
+        return block
+
+    def copy_of(self, mask, N):
+        """Of a mask whose row lists are UNMADE: the copy of it that they will be made from, else None.  Forwards that need no lists
+        take the copy, not the mask: a graph that captures one keeps seeing the mask as it was, as it would with lists."""
+        key = (id(mask), N, False)
+        entry = self._entries.get(key)
+        if entry is None or entry[2] is not UNMADE or entry[0]() is not mask or self._version(mask) != entry[1]:
+            return None
+        self._entries[key] = self._entries.pop(key, entry)
+        return self._copy(mask, entry[3], entry[4])
+
+    def keeps(self, mask):
+        """Would `put` keep anything for this mask?  (Lists made while a graph is being captured are filled by its replays only, in
+        memory that is the graph's.)"""
+        return self._version(mask) is not None and not torch.cuda.is_current_stream_capturing()
+
+    def put(self, mask, N, transpose, lists, copy=None):
+        if not self.keeps(mask):
             return
+        version = self._version(mask)
         key = (id(mask), N, transpose)
         self._entries.pop(key, None)
         if len(self._entries) >= self.capacity:
@@ -232,7 +258,7 @@ class _ListsCache:
                 del self._entries[dead]
             while len(self._entries) >= self.capacity:
                 self._entries.popitem(last=False)
-        self._entries[key] = (weakref.ref(mask), version, lists, _ext.raw_stream(mask.device))
+        self._entries[key] = (weakref.ref(mask), version, lists, _ext.raw_stream(mask.device), copy)
 
     def clear(self):
         self._entries.clear()

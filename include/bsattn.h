@@ -56,7 +56,7 @@ extern "C" {
  *   100: first layout.
  *   200: bsattn_bwd and bsattn_bwd_elementwise take dq_strides, dk_strides, dv_strides after
  *        do_strides; the entry points of the forward over quads of row blocks are gone. */
-#define BSATTN_ABI_VERSION 203
+#define BSATTN_ABI_VERSION 204
 int bsattn_version(void);
 /* Process-wide switch (default off), returns the previous setting.  On: the forward's result
  * depends on nothing but its inputs and the device (two runs give the same bits).  Off: the
@@ -324,6 +324,14 @@ int bsattn_fwd_mask_tokens(const void* q, const void* k, const void* v, void* o,
                            const int64_t* q_strides, const int64_t* k_strides,
                            const int64_t* v_strides, const int64_t* o_strides, void* workspace,
                            size_t workspace_bytes, void* stream);
+/* The same; block_copy, [Bm, Hm, nb, nb] bytes without gaps (nb = ceil(N / 64)) apart from `block`, or NULL, receives the mask as
+ * the forward saw it (0 and 1), for callers that want later calls to see it so whatever is written to `block` in between. */
+int bsattn_fwd_mask_copy_tokens(const void* q, const void* k, const void* v, void* o, float* lse,
+                                const uint8_t* block, const int64_t* mask_strides, uint8_t* block_copy, int Bm, int Hm,
+                                int B, int H, int N, int D, int dtype, int out_dtype, float sm_scale,
+                                const int64_t* q_strides, const int64_t* k_strides,
+                                const int64_t* v_strides, const int64_t* o_strides, void* workspace,
+                                size_t workspace_bytes, void* stream);
 int bsattn_bwd_tokens(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                       const float* lse, void* dq, void* dk, void* dv, const int32_t* row_ptr,
                       const int32_t* col_idx, const int32_t* col_ptr, const int32_t* row_idx,

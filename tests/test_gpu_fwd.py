@@ -304,6 +304,31 @@ def test_cached_lists_on_another_stream(dev):
     assert errors(o1, o_ref)[1] <= RELL2 and errors(o2, o_ref)[1] <= RELL2
 
 
+@pytest.mark.parametrize("N,D,takes_mask", [(4096, 64, 1), (8256, 64, 0), (1000, 128, 1), (1024, 256, 1)])
+def test_call_on_another_stream_sees_the_mask_of_the_first(dev, N, D, takes_mask):
+    """A mask is written and used on a stream that is still busy; a second call on another stream sees it as the first did: it
+    waits for the work that made the lists, or for that of a forward that needed none."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask import _ext
+    assert _ext.lib().bsattn_fwd_takes_mask(1, 1, N, D) == takes_mask
+    q, k, v = [x.to(dev) for x in make_qkv(1, 1, N, D, torch.float16, 33)]
+    nb = -(-N // 64)
+    want = uniform_block_mask(1, 1, nb, 0.3, 9).to(dev)
+    o_ref = fm.flash_attention_custom_mask(q, k, v, want, 0.125)
+    mask = torch.ones_like(want)
+    side = torch.cuda.Stream(dev)
+    fm.flash_attention_custom_mask(q, k, v, torch.ones_like(want), 0.125)
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)                                        # (about 0.1 s)
+    mask.copy_(want)
+    o1 = fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+    with torch.cuda.stream(side):
+        o2 = fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+    side.synchronize()
+    torch.cuda.synchronize()
+    assert same_up_to_rounding(o1, o_ref) and same_up_to_rounding(o2, o_ref)
+
+
 @pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_large_magnitudes(dev, dtype, out_fp32):
     """Inputs far from N(0,1): scores with a standard deviation of 23 (a nearly one-hot softmax whose reference

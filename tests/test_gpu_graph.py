@@ -129,3 +129,33 @@ def test_lists_made_under_capture_are_the_graphs(dev, elementwise):
         torch.cuda.synchronize()
         assert same_up_to_rounding(captured, eager[i]), i
         assert same_up_to_rounding(call(mask), eager[i]), i
+
+
+# D = 64 with a row block per workgroup (columns from the mask), 2 shares, ranges (lists); D = 128, 256
+@pytest.mark.parametrize("H,N,D,takes_mask", [(2, 640, 64, 1), (1, 6400, 64, 1), (1, 8256, 64, 0), (2, 700, 128, 1), (1, 1024, 256, 1)])
+@pytest.mark.parametrize("per_head", [False, True])
+def test_mask_seen_before_the_capture_stays_as_it_was(dev, H, N, D, takes_mask, per_head):
+    """A mask that one eager call has seen: a graph captured after it keeps seeing the mask as it was, whatever is written to the
+    mask later, and eager calls see what is written."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask import _ext, utils
+    assert _ext.lib().bsattn_fwd_takes_mask(1, H, N, D) == takes_mask
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, D, torch.float16, 91)]
+    nb = -(-N // 64)
+    masks = [uniform_block_mask(1, H if per_head else 1, nb, 0.3, 92 + i).to(dev) for i in range(3)]
+    call = lambda mask: fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+    eager = [call(m.clone()) for m in masks]
+    utils.lists_cache.clear()
+    mask = masks[0].clone()
+    assert same_up_to_rounding(call(mask), eager[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = call(mask)
+    for i in (0, 1, 2):
+        mask.copy_(masks[i])
+        captured.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same_up_to_rounding(captured, eager[0]), i
+    assert same_up_to_rounding(call(mask), eager[2])

@@ -195,6 +195,7 @@ def test_forward_from_the_mask_itself(dev, B, H, N, D, form):
     utils.lists_cache.clear()
     o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, D ** -0.5)
     assert utils.lists_cache.seen(mask, N) is utils.UNMADE
+    assert torch.equal(utils.lists_cache.copy_of(mask, N), mask)
     lists = utils.lists_cache.get(mask, N, False)
     assert utils.lists_cache.seen(mask, N) is lists
     ref = utils.block_mask_to_lists(mask.contiguous())
