@@ -172,6 +172,30 @@ def to_block_mask(mask, N):
 UNMADE = object()
 
 
+class _Captured:
+    """What captured graphs read of the caches' entries (lists, copies of masks, words by grid position), kept as long as the mask
+    tensor: an entry goes when its mask is written to or many others are used, and a graph's replays would read freed memory."""
+
+    def __init__(self):
+        self._held = {}        # id of mask -> (weakref to mask, [objects])
+
+    def hold(self, mask, *objects):
+        if not torch.cuda.is_current_stream_capturing():
+            return
+        key = id(mask)
+        entry = self._held.get(key)
+        if entry is None or entry[0]() is not mask:
+            held = self._held
+            def drop(ref):
+                if key in held and held[key][0] is ref:
+                    del held[key]
+            entry = self._held[key] = (weakref.ref(mask, drop), [])
+        entry[1].extend(x for x in objects if all(x is not y for y in entry[1]))
+
+
+captured = _Captured()
+
+
 class _ListsCache:
     """Kept-tile lists of the most recently used masks.  A static mask (the usual case: one mask
     for every layer and step) is indexed once instead of once per call.  An entry is only used
@@ -219,6 +243,7 @@ class _ListsCache:
         ref, version, lists, stream, block = entry
         if ref() is not mask or self._version(mask) != version:
             return None
+        captured.hold(mask, block if lists is UNMADE else lists)
         if lists is UNMADE:
             lists = block_mask_to_lists(self._copy(mask, stream, block), transpose=transpose)
             self.put(mask, N, transpose, lists)
@@ -240,6 +265,7 @@ class _ListsCache:
         if entry is None or entry[2] is not UNMADE or entry[0]() is not mask or self._version(mask) != entry[1]:
             return None
         self._entries[key] = self._entries.pop(key, entry)
+        captured.hold(mask, entry[4])
         return self._copy(mask, entry[3], entry[4])
 
     def keeps(self, mask):
@@ -288,6 +314,7 @@ class _GridCache:
                 current = torch.cuda.current_stream(mask.device)
                 if current != stream:
                     current.wait_event(ready)
+                captured.hold(mask, *grid)
                 return grid
         return None
 

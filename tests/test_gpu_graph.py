@@ -159,3 +159,38 @@ def test_mask_seen_before_the_capture_stays_as_it_was(dev, H, N, D, takes_mask, 
         torch.cuda.synchronize()
         assert same_up_to_rounding(captured, eager[0]), i
     assert same_up_to_rounding(call(mask), eager[2])
+
+
+@pytest.mark.parametrize("H,N,D", [(2, 640, 64), (1, 8256, 64), (2, 700, 128)])
+@pytest.mark.parametrize("elementwise", [False, True])
+def test_captured_lists_outlive_their_entries(dev, H, N, D, elementwise):
+    """What a graph has captured of the caches is kept while the mask lives: its replays are right after eager calls with the mask
+    written to, which replace the entries, and with many other masks, which push them out."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask import utils
+    nb = -(-N // 64)
+    if elementwise and N > 1000:
+        N, nb = 1000, 16
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, D, torch.float16, 95)]
+    masks = [uniform_block_mask(1, 1, nb, 0.3, 96 + i).to(dev) for i in range(12)]
+    if elementwise:
+        masks = [m.repeat_interleave(64, 2).repeat_interleave(64, 3)[:, :, :N, :N].tril().contiguous() for m in masks]
+    call = lambda mask: fm.flash_attention_custom_mask(q, k, v, mask, 0.125)
+    mask = masks[0].clone()
+    eager = call(mask)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = call(mask)
+    assert utils.captured._held[id(mask)][0]() is mask
+    for i, other in enumerate(masks):
+        if i % 2:
+            mask.copy_(other)
+        call(mask if i % 2 else other)
+        captured.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same_up_to_rounding(captured, eager), i
+    held = id(mask)
+    del mask
+    assert held not in utils.captured._held
