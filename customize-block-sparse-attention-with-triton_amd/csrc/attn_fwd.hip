@@ -1398,10 +1398,15 @@ static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
   return 256 + (split > 1 ? (size_t)B * H * (split * (size_t)N * (D + 2) + (N + 63) / 64) * sizeof(float) : 0);
 }
 
-static int pair_split(int B, int H, int N, int D, bool words) {
+// compact: as many of these shares as the library's scratch memory has room for, two at least (less is refused: 8 heads of N = 1408
+// and 1472 at D = 256 have two of three, one head of N = 8192 has three of four; D = 128 has room for all).
+static int pair_split(int B, int H, int N, int D, bool words, bool compact) {
   const int nb = (N + 63) / 64;
   const int64_t row_blocks = (int64_t)B * H * nb;
-  return D == 256 ? pair_split_256(row_blocks, nb) : words ? pair_split_words(row_blocks, nb) : pair_split_128(row_blocks, nb);
+  int s = D == 256 ? pair_split_256(row_blocks, nb) : words ? pair_split_words(row_blocks, nb) : pair_split_128(row_blocks, nb);
+  if (compact)
+    while (s > 2 && pair_parts_bytes(B, H, N, D, s) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --s;
+  return s;
 }
 
 // Which launches fwd_short_kernel (D = 64) takes: pairs of wavefronts per workgroup (0: none) and shares of a row block's list.
@@ -1438,9 +1443,9 @@ bool launch_fwd_takes_mask(int B, int H, int N, int D) {
 }
 
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
-  if (D != 64) {     // (compact launches: block masks only; their parts at D = 128 are 32 MB at most)
-    const int block = pair_split(B, H, N, D, false);
-    return pair_parts_bytes(B, H, N, D, compact ? block : std::max(block, pair_split(B, H, N, D, true)));
+  if (D != 64) {     // (compact launches: block masks only)
+    const int block = pair_split(B, H, N, D, false, compact);
+    return pair_parts_bytes(B, H, N, D, compact ? block : std::max(block, pair_split(B, H, N, D, true, false)));
   }
   const int nb = (N + 63) / 64;
   if (const ShortPlan plan = short_plan((int64_t)B * H * nb, nb); plan.pairs > 0) return pair_parts_bytes(B, H, N, D, plan.split);
@@ -1556,7 +1561,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
   const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
   if (s.D != 64 || plan.pairs > 0) {
-    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr);
+    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr, s.compact);
     prm.place = place_of_eight(heads, prm.nb, prm.split);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;

@@ -71,6 +71,15 @@ def test_static_forward_matches_workspace_forward(dev):
     _both(dev, 1, 1, 1024, 256, torch.float16, 0.6, 14)
 
 
+@pytest.mark.parametrize("N", [1408, 1472])
+def test_static_forward_takes_the_shares_its_scratch_has_room_for(dev, N):
+    """8 heads at D = 256: three shares of a row block's list, which bsattn_fwd takes, are more than the scratch array holds."""
+    n = ctypes.c_size_t()
+    from fa2_custom_mask import _ext
+    assert _ext.lib().bsattn_fwd_workspace(1, 8, N, 256, ctypes.byref(n)) == 0 and n.value > (32 << 20)
+    _both(dev, 1, 8, N, 256, torch.float16, 0.6, 15)
+
+
 def test_static_forward_rejects_shapes_beyond_its_scratch(dev):
     from fa2_custom_mask import _ext
     lib = _ext.lib()
