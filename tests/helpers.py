@@ -44,3 +44,18 @@ def same_up_to_rounding(a, b, rel=2.0 ** -9, abs_=3e-4):
     a = a.detach().float().cpu().numpy() if isinstance(a, torch.Tensor) else np.asarray(a, dtype=np.float32)
     b = b.detach().float().cpu().numpy() if isinstance(b, torch.Tensor) else np.asarray(b, dtype=np.float32)
     return bool(np.all(np.abs(a - b) <= rel * np.abs(b) + abs_))
+
+
+def fwd_route_d64(B, H, N):
+    """Which of the forward's ways a launch at D = 64 goes: "pairs" (fwd_short_kernel), "workgroups" or "wavefronts" (ranges of
+    them), "rows" (a wavefront per row block).  Told by the size of the workspace, which has room for two parts per range, or for one
+    per workgroup for long row blocks."""
+    from fa2_custom_mask import _ext
+    if _ext.lib().bsattn_fwd_takes_mask(B, H, N, 64):
+        return "pairs"
+    heads, nb = B * H, -(-N // TILE)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    size = lambda parts: heads * parts * (64 * 64 + 128) * 4 + heads * nb * 8
+    n = _ext.fwd_workspace(B, H, nb * TILE, 64)
+    return {size(2 * (2 * cus // heads)): "workgroups", size(2 * (8 * cus // heads)): "wavefronts",
+            size(8 * cus // heads): "rows", 256: "rows"}[n]

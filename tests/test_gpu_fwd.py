@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import make_qkv, uniform_block_mask, causal_block_mask, errors, f32, same_up_to_rounding
+from helpers import make_qkv, uniform_block_mask, causal_block_mask, errors, f32, same_up_to_rounding, fwd_route_d64
 
 pytestmark = pytest.mark.gpu
 
@@ -97,12 +97,13 @@ def test_row_block_per_wavefront_several_workgroups_per_head(dev):
     run_case(dev, 2, 32, 2048, 64, torch.bfloat16, m2, 6, out_fp32=True)
 
 
-@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.bfloat16)])
-def test_short_and_long_row_blocks_mixed(dev, D, dtype):
-    """Runs of short row blocks inside a workgroup's range go one row block per wavefront, long
-    ones are shared by the wavefronts: block-causal masks (lengths 1..nb), alternating short / long /
-    empty row blocks, and a mask whose row blocks all hold one or two tiles."""
-    nb = 48
+@pytest.mark.parametrize("D,dtype,nb", [(64, torch.float16, 48), (128, torch.bfloat16, 48), (64, torch.float16, 130)])
+def test_short_and_long_row_blocks_mixed(dev, D, dtype, nb):
+    """Block-causal masks (lengths 1..nb), alternating short / long / empty row blocks, and a mask whose row blocks all hold one or
+    two tiles.  With 130 row blocks a workgroup has a range of the list: runs of short row blocks inside it go one row block per
+    wavefront, long ones are shared by the wavefronts; with 48 a row block is a workgroup's."""
+    if D == 64:
+        assert fwd_route_d64(1, 2, nb * 64) == ("pairs" if nb == 48 else "workgroups")
     run_case(dev, 1, 2, nb * 64, D, dtype, causal_block_mask(1, 1, nb, 0.6, 3), 41, out_fp32=True)
     g = torch.Generator().manual_seed(9)
     m = torch.zeros(1, 2, nb, nb, dtype=torch.bool)
@@ -115,10 +116,11 @@ def test_short_and_long_row_blocks_mixed(dev, D, dtype):
             m[0, 1, r, torch.randperm(nb, generator=g)[:30]] = True
         # kind 4: empty
     run_case(dev, 1, 2, nb * 64, D, dtype, m, 42, out_fp32=True)
-    m2 = torch.zeros(2, 3, nb, nb, dtype=torch.bool)
-    idx = torch.randint(0, nb, (2, 3, nb, 2), generator=g)
+    b2 = 2 if nb == 48 else 1
+    m2 = torch.zeros(b2, 3, nb, nb, dtype=torch.bool)
+    idx = torch.randint(0, nb, (b2, 3, nb, 2), generator=g)
     m2.scatter_(3, idx, True)
-    run_case(dev, 2, 3, nb * 64, D, dtype, m2, 43, out_fp32=True)
+    run_case(dev, b2, 3, nb * 64, D, dtype, m2, 43, out_fp32=True)
 
 
 def test_mask_none_is_dense_attention(dev):
@@ -163,9 +165,8 @@ def test_lists_cache_follows_the_mask(dev):
 
 
 def test_workspace_contents_do_not_matter(dev):
-    """Row blocks shared between workgroups are merged by whichever workgroup arrives last, counted
-    in the workspace: stale or random workspace contents, and repeated runs on the same workspace,
-    must give the same result."""
+    """Row blocks shared between workgroups leave their parts in the workspace, which a second launch sums: stale or random
+    workspace contents, and repeated runs on the same workspace, must give the same result."""
     import fa2_custom_mask as fm
     N, D = 4096, 64
     q, k, v = [x.to(dev) for x in make_qkv(1, 2, N, D, torch.float16, 77)]
@@ -191,6 +192,41 @@ def test_workspace_contents_do_not_matter(dev):
         fin = np.isfinite(lse_ref)
         assert np.array_equal(np.isfinite(lse.cpu().numpy()), fin)
         assert np.abs(lse.cpu().numpy()[fin] - lse_ref[fin]).max() <= 2e-3
+
+
+@pytest.mark.parametrize("H,N,route", [(1, 8256, "workgroups"), (3, 8256, "workgroups"), (12, 8192, "wavefronts"), (40, 5120, "rows")])
+def test_stale_counters_do_not_matter(dev, H, N, route):
+    """The same where row blocks are finished by whoever counts itself in last: the counters of an earlier call, of another launch or
+    of nobody in the workspace, then repeated runs on it."""
+    import fa2_custom_mask as fm
+    assert fwd_route_d64(1, H, N) == route
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, 64, torch.float16, 79)]
+    nb = N // 64
+    m = uniform_block_mask(1, 1, nb, 0.1, 80)
+    m[0, 0, 3, :] = True                                    # (row blocks much longer than the others)
+    m[0, 0, nb - 1, :] = True
+    m[0, 0, 5, :] = False
+    plan = fm.ForwardPlan(q, k, v, fm.block_mask_to_lists(m.to(dev)), 0.125)
+    g = torch.Generator(device="cpu").manual_seed(6)
+    for fill in ("ones", "random", None, "zeros", None):
+        if fill == "ones":
+            plan.ws.fill_(255)
+        elif fill == "zeros":
+            plan.ws.zero_()
+        elif fill == "random":
+            plan.ws.copy_(torch.randint(0, 256, plan.ws.shape, dtype=torch.uint8, generator=g))
+        plan.o.fill_(7.0)
+        plan.lse.fill_(7.0)
+        o, lse = plan.run()
+        torch.cuda.synchronize()
+        for h in sorted({0, H // 2, H - 1}):
+            keep = m[0, 0].to(dev).repeat_interleave(64, 0).repeat_interleave(64, 1)
+            s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~keep, float("-inf"))
+            ma, rl = errors(o[0, h], torch.softmax(s, -1).nan_to_num(0.0) @ v[0, h].float())
+            assert ma <= 2e-2 and rl <= RELL2, (fill, h, ma, rl)
+            ref = torch.logsumexp(s, -1)
+            fin = torch.isfinite(ref)
+            assert torch.equal(torch.isfinite(lse[0, h]), fin) and float((lse[0, h] - ref)[fin].abs().max()) <= 2e-3
 
 
 def test_dense_elementwise_mask_c2_small(dev):
@@ -357,7 +393,8 @@ def test_large_magnitudes(dev, dtype, out_fp32):
 
 
 @pytest.mark.parametrize("B,H,Bm,Hm,N,D,dtype", [(1, 1, 1, 1, 1024, 64, torch.float16), (2, 3, 1, 1, 512, 128, torch.bfloat16),
-                                                 (2, 2, 2, 2, 768, 64, torch.float16), (1, 2, 1, 2, 4096, 64, torch.float16)])
+                                                 (2, 2, 2, 2, 768, 64, torch.float16), (1, 2, 1, 2, 4096, 64, torch.float16),
+                                                 (1, 2, 1, 2, 8256, 64, torch.float16)])
 def test_lists_and_forward_from_one_call(dev, B, H, Bm, Hm, N, D, dtype):
     """bsattn_fwd_block_mask (the reference's whole forward call, fa2_custom_mask.py:43-94: lists of the block mask,
     then the kernel): O and LSE against the oracle, the lists it leaves against the oracle's, bit for bit, and the
@@ -397,9 +434,10 @@ def test_lists_and_forward_from_one_call(dev, B, H, Bm, Hm, N, D, dtype):
     assert ma <= tol_abs and rl <= tol_rel
     fin = np.isfinite(lse_ref)
     assert np.abs(lse.cpu().numpy()[fin] - lse_ref[fin]).max() <= 2e-3 and bool(torch.isinf(lse[0, 0, 64:128]).all())
-    # the Python operator takes the same route for a mask it has not seen
+    # the Python operator takes the same route for a mask it has not seen, or one without lists
     utils.lists_cache.clear()
     o2 = fm.flash_attention_custom_mask(qd, kd, vd, md, sc)
+    assert (utils.lists_cache.seen(md, N) is utils.UNMADE) == (lib.bsattn_fwd_takes_mask(B, H, N, D) == 1) == (N != 8256)
     cached = utils.lists_cache.get(md, N, False)
     assert cached is not None and np.array_equal(cached.row_ptr.cpu().numpy(), rp_ref)
     ma, rl = errors(o2, o_ref)

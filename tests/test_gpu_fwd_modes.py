@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import make_qkv, uniform_block_mask, errors, f32, same_up_to_rounding
+from helpers import make_qkv, uniform_block_mask, errors, f32, same_up_to_rounding, fwd_route_d64
 
 pytestmark = pytest.mark.gpu
 
@@ -23,12 +23,14 @@ def block_mask(nb, keep, seed):
 
 
 # wavefronts of the GPU: 2048.  2048 row blocks: ranges of wavefronts, each a whole number of row blocks on average;
-# 2080 and 2400: ranges that cut row blocks; 3200: whole row blocks; 8 ragged row blocks of 4 heads: ranges of workgroups
-@pytest.mark.parametrize("B,H,N", [(2, 16, 4096), (1, 40, 3300), (1, 24, 6337), (4, 40, 1250), (1, 4, 449)])
+# 2080 and 2400: ranges that cut row blocks; 3200: whole row blocks; 8 ragged row blocks of 4 heads: pairs of wavefronts; 130 of 3
+# heads: ranges of workgroups
+@pytest.mark.parametrize("B,H,N", [(2, 16, 4096), (1, 40, 3300), (1, 24, 6337), (4, 40, 1250), (1, 4, 449), (1, 3, 8300)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("elementwise", [False, True])
 def test_modes(dev, B, H, N, dtype, elementwise):
     import fa2_custom_mask as fm
+    assert fwd_route_d64(B, H, N) == {4096: "wavefronts", 3300: "wavefronts", 6337: "wavefronts", 1250: "rows", 449: "pairs", 8300: "workgroups"}[N]
     nb = -(-N // 64)
     q, k, v = make_qkv(B, H, N, 64, dtype, 500 + N)
     block = block_mask(nb, 0.3, 501 + N)
@@ -186,9 +188,9 @@ def test_long_row_blocks(dev, H, N, dtype, elementwise):
 
 
 # Heads that are not a multiple of 8 share the XCDs unevenly (place.h); every head has a mask of its own, so that one taken
-# for another shows.  D = 64: 24 row blocks (ranges of workgroups), 1690 (ranges of wavefronts), 3375 (row blocks, heads in
-# groups), 3250 (row blocks, all heads at once).
-@pytest.mark.parametrize("H,N,D", [(3, 449, 64), (13, 8300, 64), (27, 8000, 64), (25, 8320, 64), (3, 1000, 128), (11, 3200, 128), (5, 700, 256)])
+# for another shows.  D = 64: 24 row blocks (pairs of wavefronts), 390 (ranges of workgroups), 1690 (ranges of wavefronts), 3375
+# (row blocks, heads in groups), 3250 (row blocks, all heads at once).
+@pytest.mark.parametrize("H,N,D", [(3, 449, 64), (3, 8300, 64), (13, 8300, 64), (27, 8000, 64), (25, 8320, 64), (3, 1000, 128), (11, 3200, 128), (5, 700, 256)])
 def test_uneven_heads(dev, H, N, D):
     import fa2_custom_mask as fm
     nb = -(-N // 64)

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import make_qkv, uniform_block_mask, causal_block_mask, same_up_to_rounding
+from helpers import make_qkv, uniform_block_mask, causal_block_mask, same_up_to_rounding, fwd_route_d64
 
 pytestmark = pytest.mark.gpu
 
@@ -47,8 +47,24 @@ def replay_and_compare(dev, B, H, N, D, dtype, mask, seed, replays=4):
 
 
 def test_replay_d64_rows_shared_between_workgroups(dev):
-    """One head, 64 row blocks on 512 workgroups: every row block is finished from published parts."""
+    """One head, 64 row blocks: four shares of a row block's list, whose parts a second launch sums."""
     replay_and_compare(dev, 1, 1, 4096, 64, torch.float16, uniform_block_mask(1, 1, 64, 0.6, 3001), 3002)
+
+
+# one head, 129 row blocks on 512 workgroups: every row block is finished from published parts; 3 heads (ranges that are not the
+# same number on every XCD); ranges of wavefronts; row blocks, the long ones cut
+@pytest.mark.parametrize("H,N,dtype,route", [(1, 8256, torch.float16, "workgroups"), (3, 8256, torch.bfloat16, "workgroups"),
+                                             (12, 8192, torch.float16, "wavefronts"), (40, 5120, torch.bfloat16, "rows")])
+def test_replay_d64_parts_counted_in(dev, H, N, dtype, route):
+    """Row blocks that the workgroup counted in last finishes: a replay repeats the launch's mark, and the counters start from zero
+    in every one."""
+    assert fwd_route_d64(1, H, N) == route
+    nb = N // 64
+    m = uniform_block_mask(1, 1, nb, 0.1, 3011)
+    m[0, 0, 5, :] = True                                     # (row blocks much longer than the others)
+    m[0, 0, nb - 2, :] = True
+    m[0, 0, 7, :] = False
+    replay_and_compare(dev, 1, H, N, 64, dtype, m, 3012, replays=3)
 
 
 def test_replay_d128_bf16_many_heads(dev):
@@ -102,15 +118,17 @@ def test_replay_mask_to_lists(dev):
         assert np.array_equal(lists.col_idx[:T].cpu().numpy(), n_ref)
 
 
-@pytest.mark.parametrize("elementwise", [False, True])
-def test_lists_made_under_capture_are_the_graphs(dev, elementwise):
-    """A mask that is first seen while a graph is being captured: its lists are made by the replays, also of what is written
-    to the mask between them, and no eager call takes them for its own."""
+@pytest.mark.parametrize("elementwise,N", [(False, 640), (True, 640), (False, 8256)])
+def test_lists_made_under_capture_are_the_graphs(dev, elementwise, N):
+    """A mask that is first seen while a graph is being captured: its lists (a block mask has some for N = 8256 only, with the other
+    length the forward reads the mask itself) are made by the replays, also of what is written to the mask between them, and no
+    eager call takes them for its own."""
     import fa2_custom_mask as fm
+    from fa2_custom_mask import _ext
     from fa2_custom_mask.utils import lists_cache, grid_cache
-    N = 640
+    assert _ext.lib().bsattn_fwd_takes_mask(1, 2, N, 64) == (N == 640)
     q, k, v = [x.to(dev) for x in make_qkv(1, 2, N, 64, torch.float16, 81)]
-    masks = [uniform_block_mask(1, 1, 10, 0.4, 82 + i).to(dev) for i in range(4)]
+    masks = [uniform_block_mask(1, 1, N // 64, 0.4, 82 + i).to(dev) for i in range(4)]
     if elementwise:
         masks = [m.repeat_interleave(64, 2).repeat_interleave(64, 3).tril().contiguous() for m in masks]
     call = lambda mask: fm.flash_attention_custom_mask(q, k, v, mask, 0.125)

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import make_qkv, uniform_block_mask, errors, f32
+from helpers import make_qkv, uniform_block_mask, errors, f32, fwd_route_d64
 
 pytestmark = pytest.mark.gpu
 
@@ -27,14 +27,22 @@ CASES = [
     # B, H, N, D, keep (1.0: dense), dtype
     (1, 1, 17536, 64, 1.0, torch.float16),      # every row block is shared by about two workgroups
     (1, 1, 17536, 64, 0.1, torch.float16),
-    (1, 2, 4096, 64, 0.5, torch.bfloat16),
-    (1, 1, 8192, 128, 0.5, torch.float16),
-    (1, 1, 2048, 256, 1.0, torch.float16),      # row lists shared by the kernel for head dimension 256
+    (1, 2, 4096, 64, 0.5, torch.bfloat16),      # two shares of a row block's list, summed by a second launch
+    (1, 1, 8192, 128, 0.5, torch.float16),      # the same at D = 128
+    (1, 1, 2048, 256, 1.0, torch.float16),      # ... and at D = 256
+    (1, 2, 8256, 64, 0.5, torch.bfloat16),      # ranges of workgroups, two heads
+    (1, 3, 8256, 64, 0.5, torch.float16),       # ... a number of heads that does not divide 8
+    (1, 11, 8320, 64, 0.2, torch.float16),
+    (1, 12, 8192, 64, 0.2, torch.bfloat16),     # ranges of wavefronts
+    (1, 40, 5120, 64, 0.2, torch.float16),      # a wavefront per row block
 ]
+ROUTES = ["workgroups", "workgroups", "pairs", None, None, "workgroups", "workgroups", "workgroups", "wavefronts", "rows"]
 
 
 def _plan(dev, B, H, N, D, keep, dtype, stream=None, seed=5):
     import fa2_custom_mask as fm
+    if D == 64:
+        assert fwd_route_d64(B, H, N) == ROUTES[CASES.index((B, H, N, D, keep, dtype))]
     q, k, v = [x.to(dev) for x in make_qkv(B, H, N, D, dtype, seed)]
     nb = N // 64
     mask = torch.ones(1, 1, nb, nb, dtype=torch.bool) if keep >= 1.0 else uniform_block_mask(1, 1, nb, keep, seed)
@@ -71,10 +79,10 @@ def _masked_stream(n_cus):
     return hip, handle
 
 
-@pytest.mark.parametrize("case", CASES[:1] + CASES[3:4])
+@pytest.mark.parametrize("case", CASES[:1] + CASES[3:4] + CASES[6:7])
 def test_few_resident_workgroups_give_the_same_bits(dev, deterministic, case):
-    """At most 16 (D = 64) or 8 (D = 128) of the launch's workgroups run at a time: the holders of a
-    row block's parts rarely overlap in time, and the last of them still finds every part."""
+    """Few of the launch's workgroups run at a time (16 at D = 64, 32 pairs at D = 128): the holders of a row block's parts rarely
+    overlap in time, and the last of them still finds every part."""
     B, H, N, D, keep, dtype = case
     plan, mask = _plan(dev, *case)
     o_all, lse_all = [t.clone() for t in plan.run()]

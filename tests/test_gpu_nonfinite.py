@@ -58,8 +58,8 @@ def test_row_blocks_of_wavefront_pairs(dev, D, H, N, elementwise, dtype, what):
     check(dev, H, N, D, dtype, elementwise, what)
 
 
-# D = 64: ranges of workgroups (row blocks inside a range, and shared by several), ranges of wavefronts, a wavefront per
-# row block, long row blocks cut; D = 128: ranges of workgroups
+# D = 64: pairs of wavefronts (one share, four), ranges of wavefronts, a wavefront per row block, long row blocks cut; D = 128:
+# shared lists of block masks
 @pytest.mark.parametrize("what", ["key", "query", "inf"])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("D,H,N,elementwise", [(64, 2, 704, False), (64, 1, 4096, False), (64, 2, 1000, True), (64, 66, 2000, False),

@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from oracle import bsattn_oracle as orc
-from helpers import make_qkv, uniform_block_mask, errors, f32, same_up_to_rounding
+from helpers import make_qkv, uniform_block_mask, errors, f32, same_up_to_rounding, fwd_route_d64
 
 pytestmark = pytest.mark.gpu
 
@@ -62,7 +62,9 @@ def _both(dev, B, H, N, D, dtype, keep, seed):
 
 def test_static_forward_matches_workspace_forward(dev):
     # first call: one long head, whose row blocks are shared between workgroups (parts and flags in the
-    # scratch array are used); second call, smaller, right after it on the same array
+    # scratch array are used); then smaller ones, right after it on the same array
+    assert fwd_route_d64(1, 1, 8256) == "workgroups"
+    _both(dev, 1, 1, 8256, 64, torch.float16, 0.7, 10)
     _both(dev, 1, 1, 2048, 64, torch.float16, 0.7, 11)
     _both(dev, 1, 2, 512, 64, torch.float16, 0.5, 12)
     _both(dev, 1, 1, 1024, 128, torch.bfloat16, 0.6, 13)
