@@ -151,8 +151,7 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
     grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     if not grad and (seen is None or seen is UNMADE):
         # launches whose workgroups have a row block each take its columns from a block mask, new or not
-        block = None if seen is None else lists_cache.copy_of(mask, N)
-        if block is not None:
+        if seen is not None and (block := lists_cache.copy_of(mask, N)) is not None:
             made = _host.forward_mask(q, k, v, block, sm_scale, out_fp32, return_lse, False)
             if made is not None:
                 return made[0]

@@ -180,8 +180,6 @@ class _Captured:
         self._held = {}        # id of mask -> (weakref to mask, [objects])
 
     def hold(self, mask, *objects):
-        if not torch.cuda.is_current_stream_capturing():
-            return
         key = id(mask)
         entry = self._held.get(key)
         if entry is None or entry[0]() is not mask:
@@ -194,6 +192,7 @@ class _Captured:
 
 
 captured = _Captured()
+_capturing = torch.cuda.is_current_stream_capturing
 
 
 class _ListsCache:
@@ -217,61 +216,59 @@ class _ListsCache:
         except RuntimeError:
             return None
 
-    def seen(self, mask, N):
-        """Is there an entry for the row lists of the mask as it is: its lists, UNMADE, or None."""
-        entry = self._entries.get((id(mask), N, False))
+    def _entry(self, mask, key):
+        entry = self._entries.get(key)
         if entry is None or entry[0]() is not mask or self._version(mask) != entry[1]:
             return None
-        return entry[2]
+        return entry
 
-    @staticmethod
-    def _wait(mask, stream):
-        # an entry's lists (or copy of the mask) were filled by kernels on `stream` (a raw handle): work on another stream waits
+    def seen(self, mask, N):
+        """Is there an entry for the row lists of the mask as it is: its lists, UNMADE, or None."""
+        entry = self._entry(mask, (id(mask), N, False))
+        return None if entry is None else entry[2]
+
+    def _use(self, mask, key, entry):
+        """The lists of an entry (or the copy of the mask, where they are UNMADE) for a call on the current stream."""
+        try:
+            self._entries.move_to_end(key)
+        except KeyError:           # (another thread has dropped it)
+            pass
+        _, _, lists, stream, block = entry
+        current = _ext.raw_stream(mask.device)
+        if current and _capturing():                 # (the default stream cannot be captured)
+            captured.hold(mask, block if lists is UNMADE else lists)
+        # they were filled by kernels on `stream` (a raw handle): work on another stream waits
         # for what that stream has been given so far (no event is recorded when the lists are made: a mask
         # that changes with every call would pay for it every time)
-        if _ext.raw_stream(mask.device) == stream:
-            return False
-        torch.cuda.current_stream(mask.device).wait_stream(
-            torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
-        return True
+        if current != stream:
+            torch.cuda.current_stream(mask.device).wait_stream(
+                torch.cuda.ExternalStream(stream, device=mask.device) if stream else torch.cuda.default_stream(mask.device))
+            if lists is UNMADE and not _capturing():
+                block.record_stream(torch.cuda.current_stream(mask.device))
+        return block if lists is UNMADE else lists
 
     def get(self, mask, N, transpose):
         key = (id(mask), N, transpose)
-        entry = self._entries.get(key)
+        entry = self._entry(mask, key)
         if entry is None:
             return None
-        ref, version, lists, stream, block = entry
-        if ref() is not mask or self._version(mask) != version:
-            return None
-        captured.hold(mask, block if lists is UNMADE else lists)
-        if lists is UNMADE:
-            lists = block_mask_to_lists(self._copy(mask, stream, block), transpose=transpose)
+        lists = self._use(mask, key, entry)
+        if entry[2] is UNMADE:
+            lists = block_mask_to_lists(lists, transpose=transpose)
             self.put(mask, N, transpose, lists)
-            return lists
-        self._entries[key] = self._entries.pop(key, entry)
-        self._wait(mask, stream)
         return lists
-
-    def _copy(self, mask, stream, block):
-        if self._wait(mask, stream) and not torch.cuda.is_current_stream_capturing():
-            block.record_stream(torch.cuda.current_stream(mask.device))
-        return block
 
     def copy_of(self, mask, N):
         """Of a mask whose row lists are UNMADE: the copy of it that they will be made from, else None.  Forwards that need no lists
         take the copy, not the mask: a graph that captures one keeps seeing the mask as it was, as it would with lists."""
         key = (id(mask), N, False)
-        entry = self._entries.get(key)
-        if entry is None or entry[2] is not UNMADE or entry[0]() is not mask or self._version(mask) != entry[1]:
-            return None
-        self._entries[key] = self._entries.pop(key, entry)
-        captured.hold(mask, entry[4])
-        return self._copy(mask, entry[3], entry[4])
+        entry = self._entry(mask, key)
+        return self._use(mask, key, entry) if entry is not None and entry[2] is UNMADE else None
 
     def keeps(self, mask):
         """Would `put` keep anything for this mask?  (Lists made while a graph is being captured are filled by its replays only, in
         memory that is the graph's.)"""
-        return self._version(mask) is not None and not torch.cuda.is_current_stream_capturing()
+        return self._version(mask) is not None and not _capturing()
 
     def put(self, mask, N, transpose, lists, copy=None):
         if not self.keeps(mask):
@@ -314,13 +311,14 @@ class _GridCache:
                 current = torch.cuda.current_stream(mask.device)
                 if current != stream:
                     current.wait_event(ready)
-                captured.hold(mask, *grid)
+                if _capturing():
+                    captured.hold(mask, *grid)
                 return grid
         return None
 
     def put(self, mask, N, grid):
         version = _ListsCache._version(mask)
-        if version is None or torch.cuda.is_current_stream_capturing():
+        if version is None or _capturing():
             return
         stream = torch.cuda.current_stream(mask.device)
         ready = torch.cuda.Event()
