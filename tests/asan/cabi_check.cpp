@@ -35,6 +35,38 @@ int main() {
   EXPECT(fwd(buf + 2, P, 1, 1, 64, 64, 0, 0, ok, ok, P, big), BSATTN_ERR_STRIDE);
   EXPECT(fwd(P, P, 1, 1, 64, 64, 0, 0, ok, ok, nullptr, big), BSATTN_ERR_WORKSPACE);
   EXPECT(fwd(P, P, 1, 1, 64, 64, 0, 0, ok, ok, P, 16), BSATTN_ERR_WORKSPACE);
+  // the forward straight from a block mask, and with a copy of it
+  auto fwd_mask = [&](const void* q, const void* mask, const int64_t* ms, void* copy, int Bm, int B, int N, int D, int dt, int odt,
+                      const int64_t* qs, void* ws, size_t wsb) {
+    const int rc = bsattn_fwd_mask_copy_tokens(q, P, P, P, nullptr, (const uint8_t*)mask, ms, (uint8_t*)copy, Bm, 1, B, 1, N, D, dt,
+                                               odt, 0.125f, qs, ok, ok, ok, ws, wsb, nullptr);
+    EXPECT(bsattn_fwd_mask_tokens(q, P, P, P, nullptr, (const uint8_t*)mask, ms, Bm, 1, B, 1, N, D, dt, odt, 0.125f, qs, ok, ok, ok,
+                                  ws, wsb, nullptr), rc);
+    return rc;
+  };
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 64, 64), 1);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 100, 64), 1);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 64, 256), 1);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 17536, 64), 0);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 64 * 513, 128), 0);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 64, 96), 0);
+  EXPECT(bsattn_fwd_takes_mask(0, 1, 64, 64), 0);
+  EXPECT(bsattn_fwd_takes_mask(1, 1, 0, 64), 0);
+  EXPECT(fwd_mask(P, nullptr, ok, P, 1, 1, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_NULL);
+  EXPECT(fwd_mask(P, P, nullptr, P, 1, 1, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_NULL);
+  EXPECT(fwd_mask(nullptr, P, ok, nullptr, 1, 1, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_NULL);
+  EXPECT(fwd_mask(P, P, ok, nullptr, 1, 0, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_SHAPE);
+  EXPECT(fwd_mask(P, P, ok, P, 3, 2, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_SHAPE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 5, 0, ok, P, big), BSATTN_ERR_DTYPE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 0, 1, ok, P, big), BSATTN_ERR_DTYPE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 96, 0, 0, ok, P, big), BSATTN_ERR_HEAD_DIM);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 0, 0, inner2, P, big), BSATTN_ERR_STRIDE);
+  EXPECT(fwd_mask(buf + 2, P, ok, P, 1, 1, 64, 64, 0, 0, ok, P, big), BSATTN_ERR_STRIDE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 17536, 64, 0, 0, ok, P, big), BSATTN_ERR_RANGE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64 * 513, 128, 0, 0, ok, P, big), BSATTN_ERR_RANGE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 0, 0, ok, nullptr, big), BSATTN_ERR_WORKSPACE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 0, 0, ok, P, 16), BSATTN_ERR_WORKSPACE);
+  EXPECT(fwd_mask(P, P, ok, P, 1, 1, 64, 64, 0, 0, ok, buf + 8, big), BSATTN_ERR_STRIDE);
   EXPECT(bsattn_fwd_workspace(1, 1, 100, 64, &n), BSATTN_ERR_SHAPE);
   EXPECT(bsattn_fwd_workspace(1, 1, 128, 64, nullptr), BSATTN_ERR_NULL);
   EXPECT(bsattn_fwd_workspace(1, 1, 17536, 64, &n), BSATTN_OK);
