@@ -860,7 +860,7 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const BwdParams prm, int
 //            14 heads N = 1792              60 /  -  /  68                   105 /  -  /  92            121 /  -  / 135   (one share there)
 // (Elementwise masks, 8 heads N = 4000, a training step: window of 1000 135 / 156 / 140, of 2000 212 / 218 / 226,
 // token-causal 316 / 291 / 287: one share from 1.33 lists per compute unit on.)
-// (D = 64: what bwd_short_kernel does not take; the workspace has room for these shares all the same.)
+// (D = 64: what bwd_short_kernel does not take, D = 128: what two groups do not; the workspace has room for these shares all the same.)
 struct BwdShares { int split, whole; };
 static BwdShares bwd_shares(int B, int H, int N, int D, bool elementwise) {
   const int64_t lists = (int64_t)B * H * ((N + 63) / 64), cus = compute_units();

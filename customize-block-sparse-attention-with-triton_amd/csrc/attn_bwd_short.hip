@@ -410,7 +410,8 @@ __global__ __launch_bounds__(128 * S, 2) void bwd_short_kernel(const BwdParams p
 
 // dQ alone at D = 128, for launches with few lists (attn_bwd.hip, bwd_pairs_128): S pairs of wavefronts per row block where dq_kernel
 // has one or several workgroups of one.  Bound by the chain of a step, S and dP, exponentials, dQ: at two wavefronts per SIMD one's
-// products hide half of the other's chain.  One share per list: no parts, no sums.  (D = 256 with two pairs, a lone wavefront per SIMD
+// products hide half of the other's chain, and each has 256 registers: ten of the 24 variants keep 12 to 36 bytes per lane in scratch memory
+// (most: bf16 with P in fp16, 4 pairs).  One share per list: no parts, no sums.  (D = 256 with two pairs, a lone wavefront per SIMD
 // like dq_kernel's, took longer than dq_kernel's shares at every size: 2 heads N = 4096 dense, backward 183 -> 281 us.)
 template <int D, int S, bool EW> struct DqPairsCfg {
   static constexpr int DQ_STAGE = 2 * 32 * 2 * D + (EW ? 512 : 0), SUM_BYTES = 64 * (D + 4) * 4;

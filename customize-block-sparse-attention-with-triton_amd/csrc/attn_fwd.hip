@@ -1326,23 +1326,34 @@ static int long_row_groups(int B, int H, int nb, bool compact) {
   return compact && parts_bytes(B, H, nb, (int)W, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
-// D = 256: workgroups per row block, of fwd_pair_kernel and of fwd_wide_kernel alike (both have two on a compute unit).  A share costs the launch that sums the parts and their traffic (64 KB of
-// fp32 per row block and share, as much as a tile's operands), so only launches that leave the GPU's 512 pairs short share,
-// and short lists where few of them are in the launch.  us, N(0,1) bf16, fwd_pair_kernel, 1 / 2 / 3 / 4 / 6 / 8 shares:
-//    1 head  N = 512    keep 0.3   16 /  15 /  13 /  14 /  11 /  12    dense   23 /  18 /  16 /  14 /  15 /  13
-//    5 heads N = 832               21 /  22 /  21 /  22 /  24 /  26            35 /  29 /  27 /  29 /  29 /  32
-//   12 heads N = 832               29 /  30 /  29 /  36 /  35 /  37            36 /  37 /  34 /  45 /  45 /  53
-//   24 heads N = 1344              40 /  59 /  72 /  82 / 109 / 133            60 /  88 / 102 / 114 / 141 / 173
-//    4 heads N = 2048              41 /  34 /  32 /  30 /  42 /  44            78 /  54 /  47 /  42 /  57 /  57
-//    7 heads N = 2048              40 /  38 /  46 /  47 /  58 /  68            78 /  58 /  75 /  70 /  83 /  94
-//   14 heads N = 2048              46 /  64 /  73 /  84 / 105 / 130            82 / 108 / 118 / 132 / 154 / 173
-//    2 heads N = 4096              66 /  45 /  40 /  38 /  50 /  53           149 /  88 /  72 /  62 /  78 /  77
-//    4 heads N = 4096              80 /  60 /  66 /  65 /  74 /  88           149 /  97 / 131 / 110 / 120 / 138
-//   10 heads N = 4096             119 / 120 / 125 / 137 / 171 / 216           303 / 266 / 258 / 265 / 308 / 352
-//    3 heads N = 6016              89 /  95 /  81 /  90 /  98 / 107           217 / 242 / 176 / 196 / 195 / 195
-//    1 head  N = 8192             123 /  73 /  59 /  53 /  67 /  67           291 / 160 / 120 /  99 / 131 / 114
-//    5 heads N = 8192             211 / 191 / 188 / 201 / 231 / 271           595 / 489 / 456 / 452 / 505 / 533
-//    1 head  N = 12032            159 /  99 / 119 / 102 / 109 / 105           425 / 236 / 310 / 247 / 254 / 209
+// D = 256: workgroups per row block, of fwd_wide_kernel and of fwd_pair_kernel (elementwise masks) alike: both have two on a compute
+// unit.  A share costs the launch that sums the parts and their traffic (64 KB of fp32 per row block and share, as much as a
+// tile's operands), so only launches that leave the GPU's 512 workgroups short share, and short lists where few of them are in the
+// launch.  us of a call among others (the host needs about 12), N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares, * the rule's.  Block masks:
+//    1 head  N = 512    keep 0.3   13 /  14*/  14 /  14 /  13 /  14    dense   18 /  17*/  16 /  15 /  16 /  16
+//    5 heads N = 832               17 /  20*/  21 /  26 /  25 /  27            25 /  26*/  25 /  30 /  30 /  34
+//   12 heads N = 832               16*/  28 /  27 /  34 /  35 /  38            26*/  35 /  32 /  41 /  46 /  55
+//   24 heads N = 1344              34*/  57 /  70 /  84 / 107 / 126            58*/  83 /  94 / 109 / 137 / 172
+//    4 heads N = 2048              31 /  29 /  31 /  31*/  42 /  45            52 /  42 /  42 /  40*/  50 /  57
+//    7 heads N = 2048              29 /  35*/  43 /  47 /  60 /  70            53 /  54*/  64 /  67 /  82 /  93
+//   14 heads N = 2048              38*/  59 /  71 /  83 / 108 / 132            75*/ 100 / 111 / 118 / 146 / 169
+//    2 heads N = 4096              47 /  36 /  38 /  38*/  48 /  52            97 /  60 /  61 /  57*/  67 /  72
+//    4 heads N = 4096              50 /  51*/  62 /  66 /  76 /  93            98 /  92*/ 104 / 104 / 117 / 132
+//   10 heads N = 4096              89*/ 109 / 120 / 135 / 175 / 226           231*/ 218 / 234 / 243 / 284 / 332
+//    3 heads N = 6016              71 /  78 /  75*/  84 /  97 / 110           169 / 186 / 156*/ 167 / 171 / 179
+//    1 head  N = 8192              75 /  51 /  50 /  49*/  60 /  65           185 / 105 /  99 /  91*/ 103 / 106
+//    5 heads N = 8192             162 / 168*/ 177 / 192 / 230 / 278           447 / 396*/ 411 / 416 / 456 / 502
+//    1 head  N = 12032            109 /  81 /  99 /  93*/ 100 / 103           268 / 194 / 237 / 197*/ 210 / 199
+//   16 heads N = 3072              76*/ 105 / 127 / 152 / 208 / 261           179*/ 203 / 223 / 246 / 300 / 351
+// Elementwise masks, token window of N / 4 and token-causal:
+//    2 heads N = 1024              18 /  17 /  16 /  17*/  15 /  16            42 /  28 /  24 /  20*/  19 /  19
+//    4 heads N = 2048              28 /  28 /  28 /  29*/  37 /  42            79 /  49 /  43 /  39*/  46 /  49
+//    8 heads N = 2048              29 /  33*/  45 /  46 /  60 /  75            79 /  57*/  56 /  62 /  69 /  78
+//    2 heads N = 4096              46 /  34 /  33 /  33*/  45 /  50           152 /  86 /  67 /  56*/  65 /  65
+//    8 heads N = 4000              71 /  95*/ 106 / 118 / 143 / 174           205 / 133*/ 169 / 157 / 183 / 210
+//    1 head  N = 8192              83 /  52 /  46 /  42*/  59 /  59           299 / 159 / 116 /  93*/ 103 /  99
+// (Set on fwd_pair_kernel, which had the block masks then: fwd_wide_kernel gains less from shares, up to 7 us at 5 heads of N = 832 and 7 of
+// N = 2048 would be saved without.)
 static int pair_split_256(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   if (rows > 8 * nb || rows >= 1024) return 1;

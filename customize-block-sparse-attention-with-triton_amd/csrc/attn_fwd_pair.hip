@@ -425,7 +425,8 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
   if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + row] = row_lse(M, L);
 }
 
-// (shared lists: at most four workgroups per compute unit, so the values fit 32 bits)
+// (one thread per 4 results of a launch that shares lists, which has fewer than 4 row blocks per compute unit (pair_split_256; half of
+// that at other head dimensions): 64 D / 4 threads each, 4 096 at most, so the values fit 32 bits)
 template <bool BF16, int S = 2>
 static void launch_sum_parts_t(const FwdParams& prm, int D, hipStream_t st) {
   if constexpr (S < 8) {

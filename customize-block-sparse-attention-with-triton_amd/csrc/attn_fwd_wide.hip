@@ -12,7 +12,8 @@
 // 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  Ragged: 16 heads
 // N = 4000 causal keep 0.5 bf16 168 -> 95 (fwd_pair_kernel spilled), 10 heads N = 4090 keep 0.3 142 -> 93, fp16 N = 4065 dense
 // block-causal 214 -> 170.  The 256 registers
-// leave no room for mask words (20 to 140 spilled): elementwise masks stay on fwd_pair_kernel.
+// leave no room for mask words (20 to 140 spilled): elementwise masks stay on fwd_pair_kernel.  Three variants keep a few values in scratch
+// memory as it is: fp16 with strided rows 8 bytes per lane (ragged 20), ragged bf16 with P in fp16 and contiguous rows 8.
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196 of the reference).
 #include "common.h"
