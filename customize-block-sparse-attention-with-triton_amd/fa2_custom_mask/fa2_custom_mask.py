@@ -158,10 +158,11 @@ def _attend(q, k, v, mask, sm_scale, out_fp32, return_lse):
         else:
             _check_mask(mask)
             if is_block_form(mask, N):
-                made = _host.forward_mask(q, k, v, mask, sm_scale, out_fp32, return_lse, lists_cache.keeps(mask))
+                kept = lists_cache.keeps(mask)
+                made = _host.forward_mask(q, k, v, mask, sm_scale, out_fp32, return_lse, kept is not None)
                 if made is not None:
-                    if made[1] is not None:
-                        lists_cache.put(mask, N, False, UNMADE, made[1])
+                    if kept is not None:
+                        lists_cache.put(mask, N, False, UNMADE, made[1], kept)
                     return made[0]
     lists = lists_cache.get(mask, N, False)
     if grad:

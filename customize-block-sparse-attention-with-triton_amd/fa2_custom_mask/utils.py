@@ -266,14 +266,20 @@ class _ListsCache:
         return self._use(mask, key, entry) if entry is not None and entry[2] is UNMADE else None
 
     def keeps(self, mask):
-        """Would `put` keep anything for this mask?  (Lists made while a graph is being captured are filled by its replays only, in
-        memory that is the graph's.)"""
-        return self._version(mask) is not None and not _capturing()
-
-    def put(self, mask, N, transpose, lists, copy=None):
-        if not self.keeps(mask):
-            return
+        """(version of the mask, current stream) if `put` would keep something for this mask, else None.  (Lists made while a graph is
+        being captured are filled by its replays only, in memory that is the graph's.)"""
         version = self._version(mask)
+        if version is None:
+            return None
+        stream = _ext.raw_stream(mask.device)
+        return None if stream and _capturing() else (version, stream)       # (the default stream cannot be captured)
+
+    def put(self, mask, N, transpose, lists, copy=None, kept=None):
+        """kept: what `keeps` said in front of the call that made the lists, or None to ask it now."""
+        kept = kept or self.keeps(mask)
+        if kept is None:
+            return
+        version, stream = kept
         key = (id(mask), N, transpose)
         self._entries.pop(key, None)
         if len(self._entries) >= self.capacity:
@@ -281,7 +287,7 @@ class _ListsCache:
                 del self._entries[dead]
             while len(self._entries) >= self.capacity:
                 self._entries.popitem(last=False)
-        self._entries[key] = (weakref.ref(mask), version, lists, _ext.raw_stream(mask.device), copy)
+        self._entries[key] = (weakref.ref(mask), version, lists, stream, copy)
 
     def clear(self):
         self._entries.clear()
