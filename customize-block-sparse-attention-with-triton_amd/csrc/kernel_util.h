@@ -18,11 +18,10 @@ typedef unsigned int uintx2 __attribute__((ext_vector_type(2)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
 
-__device__ __forceinline__ float max3f(float a, float b, float c) {
-  float r;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-  return r;
-}
+// Left to the compiler, not written as an instruction: scores come straight from the matrix cores, the hardware does not wait for
+// their results (up to 18 states), and the compiler puts the wait only in front of instructions it knows.  With v_max3_f32 in
+// inline assembly fwd_wide_kernel's bf16 variants read unfinished scores, and two runs differed where P is rounded.
+__device__ __forceinline__ float max3f(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 __device__ __forceinline__ float xhalf_max(float x) {
   // max of lane l and lane l^32 (the two halves of a wavefront hold the same query)

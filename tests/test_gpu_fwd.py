@@ -445,3 +445,24 @@ def test_lists_and_forward_from_one_call(dev, B, H, Bm, Hm, N, D, dtype):
     o3, lse3 = fm.flash_attention_custom_mask_lse(qd, kd, vd, md, sc)            # second call: cached lists
     assert same_up_to_rounding(o3, o2, rel=2.0 ** -9 if dtype == torch.float16 else 2.0 ** -6, abs_=3e-4 if dtype == torch.float16 else 2e-3)
     assert np.abs(lse3.cpu().numpy()[fin] - lse_ref[fin]).max() <= 2e-3
+
+
+# kernels whose workgroups have a row block each: nothing depends on who comes first.  D = 64 pairs (without and with shares), 128
+# (one share, two), 256 (a wide launch, shares, elementwise masks); ragged lengths
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("D,H,N,elementwise", [(64, 3, 1000, False), (64, 1, 4096, False), (64, 3, 1000, True), (128, 2, 4096, False),
+                                               (128, 16, 2048, False), (128, 2, 1000, True), (256, 16, 2048, False), (256, 3, 3100, False),
+                                               (256, 2, 1000, True)])
+def test_runs_with_the_same_bits(dev, D, H, N, elementwise, dtype, out_fp32):
+    import fa2_custom_mask as fm
+    g = torch.Generator().manual_seed(N + D + H)
+    q, k, v = (torch.randn(1, H, N, D, generator=g).to(dtype).to(dev) for _ in range(3))
+    nb = -(-N // 64)
+    if elementwise:
+        mask = torch.ones(N, N, dtype=torch.bool).tril()[None, None].to(dev)
+    else:
+        mask = ((torch.rand(1, 1, nb, nb, generator=g) < 0.4) | torch.eye(nb, dtype=torch.bool)).to(dev)
+    first = fm.flash_attention_custom_mask_lse(q, k, v, mask, D ** -0.5, out_fp32=out_fp32)
+    for _ in range(4):
+        again = fm.flash_attention_custom_mask_lse(q, k, v, mask, D ** -0.5, out_fp32=out_fp32)
+        assert torch.equal(first[0], again[0]) and torch.equal(first[1], again[1])
