@@ -453,8 +453,7 @@ __device__ __forceinline__ void part_tile_load_async(const unsigned short* tile,
     const int j = wv * PER_WAVE + jj;
     const int c = j * 64 + lane, row = c / CPR, ch = c % CPR;
     const unsigned off = 2u * (unsigned)(row * (int)stride + ((ch ^ u_swz<D>(row)) * 8));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(lds_addr + j * 1024), "v"(off), "s"(tile) : "memory", "m0");
+    tile_load_async_one(tile, off, lds_addr + j * 1024);
   }
 }
 

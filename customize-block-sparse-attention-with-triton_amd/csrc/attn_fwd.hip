@@ -269,8 +269,7 @@ void fwd_kernel(const FwdRangeParams prm) {
       const unsigned long long* src = prm.tile_bits + (int64_t)t * 64;
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
-                     :: "s"(lds_bits_addr + j * 256), "v"(4u * (unsigned)lane + 256u * j), "s"(src) : "memory", "m0");
+        words_load_async(src, 4u * (unsigned)lane + 256u * j, lds_bits_addr + j * 256);
     }
   };
   auto v_copy_all = [&](int cb) {

@@ -153,8 +153,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
     }
     if constexpr (EW) {
       const unsigned long long* src = prm.tile_bits + (int64_t)t * 64;
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
-                   :: "s"(lds_bits_addr + w * 256), "v"(4u * (unsigned)lane + 256u * w), "s"(src) : "memory", "m0");
+      words_load_async(src, 4u * (unsigned)lane + 256u * w, lds_bits_addr + w * 256);
     }
   };
   auto v_copy = [&](int cb) {

@@ -114,8 +114,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
     }
     if constexpr (EW) {
       const unsigned long long* src = prm.tile_bits + (int64_t)t * 64;
-      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2"
-                   :: "s"(va + C::TILE_BYTES + w * 256), "v"(4u * (unsigned)lane + 256u * w), "s"(src) : "memory", "m0");
+      words_load_async(src, 4u * (unsigned)lane + 256u * w, va + C::TILE_BYTES + w * 256);
     }
   };
   int kaddr[2][KS];

@@ -74,8 +74,7 @@ __device__ __forceinline__ void half_tile_load_async(const unsigned short* tile,
     const int j = wv * PER_WAVE + jj;
     const int c = j * 64 + lane, row = c / CPR, ch = c % CPR;
     const unsigned off = 2u * (unsigned)(row * (int)stride + ((ch ^ u_swz<D>(row)) * 8));
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(lds_addr + j * 1024), "v"(off), "s"(tile) : "memory", "m0");
+    tile_load_async_one(tile, off, lds_addr + j * 1024);
   }
 }
 
@@ -104,8 +103,7 @@ __device__ __forceinline__ unsigned long long tail_word(int valid, int g) {
 
 // asynchronous copy of 64 consecutive floats (one per lane)
 __device__ __forceinline__ void stat_load_async(const float* src, int lane, unsigned lds_addr) {
-  const unsigned off = 4u * (unsigned)lane;
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dword %1, %2" :: "s"(lds_addr), "v"(off), "s"(src) : "memory", "m0");
+  words_load_async(src, 4u * (unsigned)lane, lds_addr);
 }
 
 // operand fragment (32 rows x 16 columns slice s) of a swizzled LDS tile: row r0 + ln, chunk 2s + g

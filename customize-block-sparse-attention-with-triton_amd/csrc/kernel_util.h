@@ -95,26 +95,23 @@ template <int D> __device__ __forceinline__ int v_swz(int row) { return D == 64 
 typedef unsigned char __attribute__((address_space(3)))* lds_ptr_t;
 typedef const int32_t __attribute__((address_space(4)))* cint_ptr_t;
 
-// Asynchronous global -> LDS copy of one 64 x D tile: D/8 instructions, each moving 16 bytes
-// per lane; the data of lane l lands at lds + j*1024 + l*16.  `off` holds the per-lane
-// source byte offsets from `tile` (a wave-uniform base).  The copies are issued from
-// inline assembly so that the compiler's own wait-count insertion does not serialise
-// them; completion is awaited explicitly with wait_vm<N>() (vector memory operations
-// retire in order, so "at most N outstanding" means everything older than the N youngest
-// has landed).
-template <int D>
-__device__ __forceinline__ void tile_load_async(const unsigned short* tile, const unsigned (&off)[D / 8],
-                                                unsigned lds_addr) {
-#pragma unroll
-  for (int j = 0; j < D / 8; ++j)
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :: "s"(lds_addr + j * 1024), "v"(off[j]), "s"(tile) : "memory", "m0");
+// Asynchronous global -> LDS copies, 16 bytes (4 bytes) per lane: the data of lane l lands at lds_addr + l*16 (l*4); `off` holds
+// the per-lane source byte offsets from `src` (a wave-uniform base).  The copies are issued from inline assembly so that the
+// compiler's own wait-count insertion does not serialise them; completion is awaited explicitly with wait_vm<N>() (vector
+// memory operations retire in order, so "at most N outstanding" means everything older than the N youngest has landed).
+// The compiler does not know what is inside, so the statement brings the waits the hardware does not make: one state between
+// writing m0 and the copy that uses it, five between a vector instruction that writes a scalar register (a spilled base comes back
+// by v_readlane) and a vector memory access that reads it.  Copying the base to a register of the statement is both: the
+// instruction in between, and a scalar instruction as the writer, which is waited for.
+__device__ __forceinline__ void tile_load_async_one(const unsigned short* src, unsigned off, unsigned lds_addr) {
+  const unsigned short* base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(base) : "s"(lds_addr), "v"(off), "s"(src) : "memory", "m0");
 }
-
-
-// one instruction of tile_load_async: 64 x 16 bytes to lds_addr (+ lane*16)
-__device__ __forceinline__ void tile_load_async_one(const unsigned short* tile, unsigned off, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds_addr), "v"(off), "s"(tile) : "memory", "m0");
+__device__ __forceinline__ void words_load_async(const void* src, unsigned off, unsigned lds_addr) {
+  const void* base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dword %2, %0"
+               : "=&s"(base) : "s"(lds_addr), "v"(off), "s"(src) : "memory", "m0");
 }
 
 // Four consecutive instructions of a tile copy whose rows follow each other without gaps: the
@@ -122,9 +119,10 @@ __device__ __forceinline__ void tile_load_async_one(const unsigned short* tile, 
 // four share one scalar base and one m0.
 __device__ __forceinline__ void tile_load_async_four(const unsigned short* src, unsigned o0, unsigned o1, unsigned o2,
                                                      unsigned o3, unsigned lds_addr) {
-  asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %5\n\tglobal_load_lds_dwordx4 %2, %5 offset:1024\n\t"
-               "global_load_lds_dwordx4 %3, %5 offset:2048\n\tglobal_load_lds_dwordx4 %4, %5 offset:3072"
-               :: "s"(lds_addr), "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(src) : "memory", "m0");
+  const unsigned short* base;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %6\n\tglobal_load_lds_dwordx4 %2, %0\n\tglobal_load_lds_dwordx4 %3, %0 offset:1024\n\t"
+               "global_load_lds_dwordx4 %4, %0 offset:2048\n\tglobal_load_lds_dwordx4 %5, %0 offset:3072"
+               : "=&s"(base) : "s"(lds_addr), "v"(o0), "v"(o1), "v"(o2), "v"(o3), "s"(src) : "memory", "m0");
 }
 
 template <int N> __device__ __forceinline__ void wait_vm() {

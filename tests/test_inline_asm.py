@@ -25,3 +25,16 @@ def test_no_vector_arithmetic():
     found = statements()
     assert len(found) >= 5
     assert not [(f, x) for f, s in found for x in s if x.startswith("v_")]
+
+
+def test_copies_into_lds():
+    """m0 is written at least one instruction in front of the copy that uses it, and the base address is in a register that a
+    scalar instruction of the same statement wrote (after a vector instruction, a spilled value's way back, five states are needed)."""
+    copies = [(f, s) for f, s in statements() if any(x.startswith("global_load_lds") for x in s)]
+    assert copies
+    for f, s in copies:
+        first = next(i for i, x in enumerate(s) if x.startswith("global_load_lds"))
+        m0 = [i for i, x in enumerate(s) if re.match(r"s_mov_b32 m0,", x)]
+        assert m0 and m0[-1] + 1 < first, (f, s)
+        written = {x.split()[1].rstrip(",") for x in s[:first] if x.startswith("s_mov_b64")}
+        assert all(x.split(",")[1].split()[0] in written for x in s[first:]), (f, s)
