@@ -661,6 +661,8 @@ void fwd_kernel(const FwdRangeParams prm) {
     const int lane_p = fresh_lane(lane), ln = lane_p & 31, g = lane_p >> 5;
     unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + row;
     unsigned long long seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    static_assert(DB == 2, "four accumulators");
+    matrix_wait(oacc[0][0], oacc[0][1], oacc[1][0], oacc[1][1]);
 #pragma unroll
     for (int quad = 0; quad < D / 4; ++quad) {
       const int idx = 4 * quad;

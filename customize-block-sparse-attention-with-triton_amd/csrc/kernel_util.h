@@ -212,10 +212,15 @@ __device__ __forceinline__ float coherent_load(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // The same accesses 16 bytes wide (p 16-byte aligned), written out, since an atomic type of that size does not
-// exist: `sc1` is what the compiler puts on the 4-byte ones above.
+// exist: `sc1` is what the compiler puts on the 4-byte ones above.  (Behind a store of more than 8 bytes its data must not be
+// overwritten for two states, which the compiler does not know of this one.)
 __device__ __forceinline__ void coherent_store4(float* p, float a, float b, float c, float d) {
   const floatx4 v = {a, b, c, d};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" :: "v"(p), "v"(v) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" :: "v"(p), "v"(v) : "memory");
+}
+// In front of such stores of accumulators, once: the matrix cores have finished them (18 states at most).
+__device__ __forceinline__ void matrix_wait(floatx16& a, floatx16& b, floatx16& c, floatx16& d) {
+  asm volatile("s_nop 15\n\ts_nop 1" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
 // Four such loads, 1 KB apart, and the wait for them (and for every earlier vector memory access of the wavefront)
 // in one statement: the compiler does not count loads it did not issue, so the values must not leave the statement

@@ -38,3 +38,12 @@ def test_copies_into_lds():
         assert m0 and m0[-1] + 1 < first, (f, s)
         written = {x.split()[1].rstrip(",") for x in s[:first] if x.startswith("s_mov_b64")}
         assert all(x.split(",")[1].split()[0] in written for x in s[first:]), (f, s)
+
+
+def test_wide_stores():
+    """The data of a store of more than 8 bytes may be overwritten two states later: the statement ends with them."""
+    stores = [(f, s) for f, s in statements() if any(re.match(r"global_store_dwordx[34]", x) for x in s)]
+    assert stores
+    for f, s in stores:
+        m = re.match(r"s_nop (\d+)$", s[-1])
+        assert m and int(m.group(1)) >= 1, (f, s)
