@@ -12,7 +12,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "fa2_custom_mask", "libbsattn.so")
 HOST = os.path.join(HERE, "fa2_custom_mask", "_host.so")
-SOURCES = ["api.hip", "mask_index.hip", "attn_fwd.hip", "attn_fwd_pair.hip", "attn_fwd_short.hip", "attn_fwd_wide.hip", "attn_bwd.hip", "attn_bwd_short.hip", "reorder.hip"]
+SOURCES = ["api.hip", "mask_index.hip", "attn_fwd.hip", "attn_fwd_pair.hip", "attn_fwd_short.hip", "attn_fwd_quad.hip", "attn_fwd_wide.hip", "attn_bwd.hip", "attn_bwd_short.hip", "reorder.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-I" + INCLUDE, "-I" + CSRC,
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",   # no packed fp32 VALU ops
          "-Wno-unused-command-line-argument", "-Wno-unknown-warning-option"]

@@ -1363,47 +1363,62 @@ static int pair_split_256(int64_t row_blocks, int nb) {
   return s < cap ? s : cap > 1 ? cap : 1;
 }
 
-// The same at D = 128 with block masks.  A share costs the launch that sums the parts (3 us) and their traffic, so short
-// lists are shared only where few of them are in the launch.  us, N(0,1), 1 / 2 / 3 / 4 / 6 shares, and fwd_kernel (ranges of
-// the lists, 512 registers a wavefront), which had these launches up to 512 row blocks before, with bf16 and with fp16:
-//   1 head  N = 832    keep 0.3  12 /  12 /  11 /  10 /  10    20   28     dense  20 /  16 /  14 /  13 /  12    21   30
-//   5 heads N = 832              13 /  14 /  14 /  16 /  16    21   29            20 /  18 /  17 /  19 /  20    22   31
-//  11 heads N = 1344             17 /  23 /  24 /  26 /  30    25   34            30 /  31 /  31 /  31 /  37    40   60
-//   1 head  N = 2048             23 /  17 /  15 /  14 /  16    22   31            42 /  27 /  22 /  19 /  18    32   47
-//   4 heads N = 2048             24 /  22 /  23 /  24 /  25    23   32            43 /  32 /  31 /  31 /  32    29   40
-//   2 heads N = 4096             36 /  27 /  27 /  26 /  26    27   41            81 /  51 /  44 /  39 /  37    37   59
-//   4 heads N = 4096             37 /  33 /  32 /  33 /  40    43   67            82 /  58 /  54 /  55 /  67    52   91
-//   6 heads N = 4096             46 /  41 /  44 /  45 /  52    50   80            88 /  74 /  91 /  85 /  90    89  165
-//   1 head  N = 8192             67 /  42 /  35 /  32 /  32    41   67           157 /  88 /  69 /  58 /  54    58   98
-//   3 heads N = 8192             75 /  58 /  68 /  63 /  70    71  124           168 / 128 / 159 / 143 / 146   143  257
-//   2 heads N = 12032            92 /  71 /  83 /  78 /  83    84  154           240 / 176 / 223 / 195 / 197   192  338
-//   8 heads N = 3072             31 /  34 /  39                                   67 /  64 /  73                  (1, 2, 3 shares)
-//   9 heads N = 2048             24 /  27 /  27                                   47 /  44 /  41    keep 0.1  15 / 25 / 24
-//   7 heads N = 4096             47 /  43 /  48                                   95 /  87 / 100    keep 0.1  24 / 32 / 34
-// From 480 row blocks on one: 8 heads N = 4000, keep 0.25, 44 / 49.
+// The same at D = 128, for what fwd_quad_kernel leaves of the launches that do not fill the GPU: long lists, of one or two heads.  us,
+// N(0,1) bf16, 1 / 2 / 3 / 4 / 6 shares; keep 0.3, dense:
+//    2 heads N = 12032 (376 row blocks)   92 /  71 /  83 /  78 /  83    240 / 176 / 223 / 195 / 197
 static int pair_split_128(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
-  if (nb < 56 && rows > 6 * nb) return 1;
-  const int s = rows >= 480 ? 1 : rows >= 320 ? 2 : rows >= 208 ? 3 : 4;
-  // a share of a dense list keeps 8 tiles, 4 in a launch of few lists, 12 in one of many short ones
-  const int cap = rows <= 64 && nb >= 12 ? nb / 4 : rows > 96 && nb < 48 ? nb / 12 : nb / 8;
-  return s < cap ? s : cap > 1 ? cap : 1;
+  if (nb < 150) return 1;
+  return rows >= 480 ? 1 : rows >= 320 ? 2 : rows >= 208 ? 3 : 4;
 }
 
-// The same at D = 128 with elementwise masks: about four workgroups per compute unit over the launch; at most 4 shares of a
-// row unless it is long (a share of a dense row then has 16 tiles), at least two tiles in one.  us, N(0,1) bf16, 1 / 2 / 3 /
-// 4 / 6 / 8 shares:
-//   8 heads N = 4000, token window of 1000   46 /  47 /  55 /  61 /  72 /  89
-//   8 heads N = 4000, token-causal          147 /  99 /  82 /  90 /  95 / 103
-//   4 heads N = 4096, token window of 1228   32 /  32 /  36 /  36 /  46 /  50
-//   1 head N = 8192, token-causal           160 /  93 /  73 /  67 /  57 /  57
-//   1 head N = 17000, keep 0.5              233 / 152 / 119 / 138 / 126 / 131
-//   2 heads N = 1000, token-causal           40 /  27 /  27 /  24 /  24 /  27
-static int pair_split_words(int64_t row_blocks, int nb) {
-  int64_t s = 4 * (int64_t)compute_units() / row_blocks;
-  const int few = nb / 2 < 4 ? nb / 2 : 4, cap = nb / 16 > few ? nb / 16 : few;
-  if (s > cap) s = cap;
-  return (int)(s > 8 ? 8 : s < 1 ? 1 : s);
+// Which launches fwd_quad_kernel (D = 128) takes: groups of four wavefronts per workgroup (0: none) and shares of a list, at most
+// (quad_shares.h).  With two groups a row block has a compute unit to itself, with one two share it.  us, fwd_pair_kernel with its shares
+// and the launch that summed them / 2 groups, whole lists / 2 groups, up to 2 shares / up to 4 / 1 group, whole / up to 2; N(0,1) bf16;
+// keep 0.1, 0.3, 1, block-causal:
+//    1 head  N = 2048 (32 row blocks)  12/13/13/13          15/16/16/16          20/25/21/19          19/25/20/18
+//    1 head  N = 4096 (64)             16/15/16/16          20/22/19/18          32/43/30/24          30/43/29/23
+//    7 heads N = 1000 (112)            11/10                17/12                28/17                28/16
+//    2 heads N = 4096 (128)            22/15/16             26/22/20             40/43/32             35/43/30
+//   11 heads N = 1344 (231)            10/10                17/13                30/20                30/19
+//    3 heads N = 4096 (192)            24/16/17             28/23/24             46/44/44             38/43/41
+//    2 heads N = 6016 (188)            25/18/19             33/31/32             57/60/61             48/59/45
+//    4 heads N = 4096 (256)            25/16/20             31/23/27             55/45/50             49/43/43
+//    1 head  N = 16064 (251)           40/32/35             67/61/62            163/160/163          143/147/124
+//    1 head  N = 12032 (188)           30/25/27             45/47/49             97/113/115           79/110/70       (not there)
+//    8 heads N = 3072 (384)            18/21/25/ - /17/18   33/34/44/ - /28/29   68/67/67/ - /59/59   65/35/51/ - /44/45
+//    3 heads N = 8192 (384)            37/36/42/ - /32/38   65/62/68/ - /56/60  139/158/143/ - /143/143  107/79/92/ - /103/84
+//    9 heads N = 4096 (576)            28/36/38/ - /29/30   46/57/66/ - /51/52  109/131/127/ - /124/111   94/93/88/ - /75/78     (nor there)
+//   24 heads N = 1280 (480)            14/18/28/ - / - /17  20/25/34/ - / - /22  33/37/47/ - / - /32    32/32/38/ - / - /39    (nor there)
+//    2 heads N = 12032 (376)           40/42/52/ - /36/38   79/88/87/ - /85/86  191/226/196/ - /202/202  145/113/119/ - /147/108   (nor there)
+// Elementwise masks (words), token window of 0.1 N, 0.25 N, 0.45 N, token-causal:
+//    2 heads N = 2000 (64)             15/11/ - /11         17/13/ - /13         20/17/ - /16         23/26/ - /17
+//    3 heads N = 4000 (189)            23/13/13             26/18/18             31/27/27             44/47/39
+//    8 heads N = 4000 (504)            30/24/28/ - /19/19   39/34/37/ - /27/27   52/50/51/ - /41/41   79/55/60/ - /69/59
+//    1 head  N = 17000 (266)           40/45/45/ - /37/37   68/65/66/ - /72/72  100/90/90/ - /122/121   191/176/134/ - /256/174
+//   10 heads N = 4000 (630)            25/36/36/ - /31/30   41/48/56/ - /41/45   66/63/72/ - /56/60  121/97/94/ - /80/81     (not there)
+//   16 heads N = 8000 (2000)           76/115/131/ - /88/88  145/184/202/ - /150/152  217/261/276/ - /217/219  274/345/362/ - /292/294   (nor there)
+struct QuadPlan { int groups, split; };
+static QuadPlan quad_plan(int64_t row_blocks, int nb, bool words) {
+  const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
+  if (rows > 512) return {0, 1};
+  if (words) {
+    const int groups = rows <= 256 || nb >= 200 ? 2 : 1;
+    return {groups, nb < SHARE_MIN_BLOCKS ? 1 : rows <= 64 ? 4 : rows <= 128 || nb >= 28 ? 2 : 1};
+  }
+  if (rows > 256) {
+    if (nb < 28 || nb >= 150) return {0, 1};
+    return {1, nb >= 80 ? 2 : 1};
+  }
+  if (rows > 150 && rows <= 230 && nb >= 150) return {0, 1};
+  if (rows <= 128) return {2, rows <= 64 && nb >= 20 ? 4 : nb >= 24 ? 2 : 1};
+  return {2, nb >= (rows <= 160 ? 40 : 80) ? 2 : 1};
+}
+static_assert(SHARE_MIN_BLOCKS <= 20, "heads of launches that share lists have as many row blocks");
+
+// the parts of shared lists and a counter per list
+static size_t quad_parts_bytes(int B, int H, int nb, int split) {
+  return 256 + (split > 1 ? (size_t)B * H * nb * (split * 64 * (size_t)(128 + 2) * sizeof(float) + sizeof(unsigned long long)) : 0);
 }
 
 static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
@@ -1412,10 +1427,10 @@ static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
 
 // compact: as many of these shares as the library's scratch memory has room for, two at least (less is refused: 8 heads of N = 1408
 // and 1472 at D = 256 have two of three, one head of N = 8192 has three of four; D = 128 has room for all).
-static int pair_split(int B, int H, int N, int D, bool words, bool compact) {
+static int pair_split(int B, int H, int N, int D, bool compact) {
   const int nb = (N + 63) / 64;
   const int64_t row_blocks = (int64_t)B * H * nb;
-  int s = D == 256 ? pair_split_256(row_blocks, nb) : words ? pair_split_words(row_blocks, nb) : pair_split_128(row_blocks, nb);
+  int s = D == 256 ? pair_split_256(row_blocks, nb) : pair_split_128(row_blocks, nb);
   if (compact)
     while (s > 2 && pair_parts_bytes(B, H, N, D, s) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --s;
   return s;
@@ -1447,6 +1462,14 @@ static ShortPlan short_plan(int64_t row_blocks, int nb) {
   return {takes ? 2 : 0, 1};
 }
 
+// compact: as many shares as the library's scratch memory has room for (4 heads of N = 8192 have one of two).
+static QuadPlan quad_plan(int B, int H, int nb, bool words, bool compact) {
+  QuadPlan plan = quad_plan((int64_t)B * H * nb, nb, words);
+  if (compact)
+    while (plan.split > 1 && quad_parts_bytes(B, H, nb, plan.split) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --plan.split;
+  return plan;
+}
+
 // Launches whose workgroups have a row block each need no lists of a block mask: they take its columns from the mask (3 heads
 // N = 891, D = 128, a mask per head and call, 21.3 -> 16.2 us; dense mask of N = 6400, D = 64, reduced in the call, 27.1 -> 22.9).
 bool launch_fwd_takes_mask(int B, int H, int N, int D) {
@@ -1455,9 +1478,14 @@ bool launch_fwd_takes_mask(int B, int H, int N, int D) {
 }
 
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
-  if (D != 64) {     // (compact launches: block masks only)
-    const int block = pair_split(B, H, N, D, false, compact);
-    return pair_parts_bytes(B, H, N, D, compact ? block : std::max(block, pair_split(B, H, N, D, true, false)));
+  if (D == 256) return pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
+  if (D == 128) {
+    const int nb = (N + 63) / 64;
+    auto bytes = [&](bool words) {
+      const QuadPlan plan = quad_plan(B, H, nb, words, compact);
+      return plan.groups > 0 ? quad_parts_bytes(B, H, nb, plan.split) : pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
+    };
+    return compact ? bytes(false) : std::max(bytes(false), bytes(true));       // (compact launches: block masks only)
   }
   const int nb = (N + 63) / 64;
   if (const ShortPlan plan = short_plan((int64_t)B * H * nb, nb); plan.pairs > 0) return pair_parts_bytes(B, H, N, D, plan.split);
@@ -1471,6 +1499,7 @@ size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_b
 
 void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
 void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st);   // attn_fwd_short.hip
+void launch_fwd_quad(const FwdParams& prm, int groups, int dt, bool elementwise, hipStream_t st);   // attn_fwd_quad.hip
 template <int D, int DT, int MODE, bool EW, int LAYOUT, bool SPREAD>
 static void launch_fwd_s(const FwdRangeParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
@@ -1572,8 +1601,24 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
   const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
   const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
+  const QuadPlan quads = s.D == 128 ? quad_plan(s.B, s.H, prm.nb, tile_bits != nullptr, s.compact) : QuadPlan{0, 1};
+  if (quads.groups > 0) {
+    const int slots = compute_units() * (quads.groups == 1 ? 2 : 1), rows = heads * prm.nb, left = rows % slots;
+    const size_t parts = (size_t)rows * quads.split * 64;
+    prm.split = quads.split;
+    prm.place = place_of_eight(heads, prm.nb, prm.split);
+    prm.load = (int)((int64_t)rows * 4096 / slots);
+    prm.tail_from = rows / slots * slots;
+    prm.tail_shares = left > 0 ? slots / left : 1;
+    prm.part_o = (float*)ws + 64;
+    prm.part_ml = prm.part_o + parts * 128;
+    prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
+    prm.epoch = next_epoch();
+    launch_fwd_quad(prm, quads.groups, dt, tile_bits != nullptr, st);
+    return launch_status();
+  }
   if (s.D != 64 || plan.pairs > 0) {
-    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, tile_bits != nullptr, s.compact);
+    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, s.compact);
     prm.place = place_of_eight(heads, prm.nb, prm.split);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;

@@ -4,6 +4,7 @@
 #include "common.h"
 #include "kernel_util.h"
 #include "place.h"
+#include "quad_shares.h"
 
 namespace bsattn {
 
@@ -24,6 +25,7 @@ struct FwdParams {
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair kernel: workgroups per row block (1: results written directly)
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
+  int tail_from, tail_shares, load;      // quad kernel: see quad_shares
   int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
@@ -116,6 +118,18 @@ __device__ __forceinline__ int columns_of_row(const FwdParams& prm, int b, int h
   }
   __builtin_amdgcn_wave_barrier();
   return n;
+}
+
+// The kept tiles of SHARE_SAMPLE rows of the block mask, from row m on.
+__device__ __forceinline__ int length_of_rows(const FwdParams& prm, int b, int h, int m, int lane) {
+  const unsigned char* row = prm.mask + (prm.Bm > 1 ? b : 0) * prm.ms[0] + (prm.Hm > 1 ? h : 0) * prm.ms[1] + m * prm.ms[2];
+  int n = 0;
+  for (int c = lane; c < prm.nb; c += 64)
+#pragma unroll
+    for (int i = 0; i < SHARE_SAMPLE; ++i) n += row[i * prm.ms[2] + (int64_t)c * prm.ms[3]] != 0;
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
+  return __builtin_amdgcn_readfirstlane(n);
 }
 
 __device__ __forceinline__ void* out_base(const FwdParams& prm, int b, int h) {
