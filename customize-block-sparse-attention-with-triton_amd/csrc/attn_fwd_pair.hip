@@ -33,9 +33,10 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   constexpr bool BF16 = DT != 0;
   constexpr bool PB = DT == 2;                   // P rounded to bf16, second product in bf16 (V as it is)
   constexpr bool FOLD = !BF16;
-  // V read before the softmax (see the loop): not where the compiler would then spill V's 64 registers in every tile (bf16
-  // elementwise; 8 heads of N = 4000, token window of 1000: 84.7 us with the spills)
-  constexpr bool EARLY_V = PORTIONS <= PAIR_EARLY_V && !(EW && BF16 && (TAIL || !PB));
+  // V read before the softmax (see the loop).  (Elementwise masks too, since a query without mass is looked after by sum_limit and not
+  // by every lane in every tile, which spilled V's registers with bf16: 32 heads N = 4000 token window of 1000 92 -> 86 us, token-causal
+  // 210 -> 199, 16 heads N = 4000 token-causal 135 -> 125.)
+  constexpr bool EARLY_V = PORTIONS <= PAIR_EARLY_V;
   constexpr int HALF = CPR / 2;                  // copy instructions per wavefront and tile
   constexpr int KOPS = HALF + (EW ? 1 : 0), VOPS = HALF;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -214,11 +215,11 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) { oacc[db][0][i] = 0.f; oacc[db][1][i] = 0.f; }
-  // (EW: a query that has no mass yet is recentred in every tile; one that does not exist never will have any)
+  // (while a query has no mass every tile is recentred (sum_limit); one that does not exist never would have any)
   float m_i = 0.f, l_i = EW && TAIL && !exists ? 1e-30f : 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
-  float limit = FOLD || EW ? SUM_LIMIT : 0.f;
+  float limit = FOLD ? SUM_LIMIT : 0.f;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
   __syncthreads();                                  // both halves of K(t0) and V(t0) and the column list are in LDS
 
@@ -310,12 +311,12 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
     auto numerators = [&]() {
       float lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
       // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD ? fresh && !(lnew >= 0.25f) : EW && fresh;
-      if (__any(first || (EW && l_i == 0.f) || !(lnew - l_i < limit))) {
-        recentre<DB, FOLD, EW>(s0, s1, oacc, 0, qk_scale, m_i, l_i, mfrag, fresh, g);
+      const bool first = FOLD && fresh && !(lnew >= 0.25f);
+      if (__any(first || !(lnew - l_i < limit))) {
+        recentre<DB, FOLD, false>(s0, s1, oacc, 0, qk_scale, m_i, l_i, mfrag, fresh, g);
         any_m = 1;
         lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
-        limit = sum_limit<EW>(lnew);
+        limit = sum_limit<false>(lnew);
       }
       l_i = lnew;
       fresh = false;
