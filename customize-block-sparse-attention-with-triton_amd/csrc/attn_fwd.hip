@@ -43,7 +43,7 @@ namespace bsattn {
 // A workgroup is four wavefronts, one per SIMD.  A wavefront needs 256 registers and two workgroups share a compute unit
 // (while one merges or waits for its first tiles the other computes).
 // (At D = 128 a wavefront that owns 64 queries needs all 512 registers of its SIMD and spills beside them: every launch was
-// slower here than with the pairs of attn_fwd_pair.hip, see pair_split_128.)
+// slower here than with the pairs of attn_fwd_pair.hip.)
 template <int D> struct FwdCfg {
   static constexpr int NW = 4;
   static constexpr int WG_PER_CU = 2;
@@ -1327,34 +1327,25 @@ static int long_row_groups(int B, int H, int nb, bool compact) {
   return compact && parts_bytes(B, H, nb, (int)W, ROWS_MODE) > (size_t)BSATTN_STATIC_SCRATCH_BYTES ? 0 : (int)W;
 }
 
-// D = 256: workgroups per row block, of fwd_wide_kernel and of fwd_pair_kernel (elementwise masks) alike: both have two on a compute
-// unit.  A share costs the launch that sums the parts and their traffic (64 KB of fp32 per row block and share, as much as a
-// tile's operands), so only launches that leave the GPU's 512 workgroups short share, and short lists where few of them are in the
-// launch.  us of a call among others (the host needs about 12), N(0,1) bf16, 1 / 2 / 3 / 4 / 6 / 8 shares, * the rule's.  Block masks:
-//    1 head  N = 512    keep 0.3   13 /  14*/  14 /  14 /  13 /  14    dense   18 /  17*/  16 /  15 /  16 /  16
-//    5 heads N = 832               17 /  20*/  21 /  26 /  25 /  27            25 /  26*/  25 /  30 /  30 /  34
-//   12 heads N = 832               16*/  28 /  27 /  34 /  35 /  38            26*/  35 /  32 /  41 /  46 /  55
-//   24 heads N = 1344              34*/  57 /  70 /  84 / 107 / 126            58*/  83 /  94 / 109 / 137 / 172
-//    4 heads N = 2048              31 /  29 /  31 /  31*/  42 /  45            52 /  42 /  42 /  40*/  50 /  57
-//    7 heads N = 2048              29 /  35*/  43 /  47 /  60 /  70            53 /  54*/  64 /  67 /  82 /  93
-//   14 heads N = 2048              38*/  59 /  71 /  83 / 108 / 132            75*/ 100 / 111 / 118 / 146 / 169
-//    2 heads N = 4096              47 /  36 /  38 /  38*/  48 /  52            97 /  60 /  61 /  57*/  67 /  72
-//    4 heads N = 4096              50 /  51*/  62 /  66 /  76 /  93            98 /  92*/ 104 / 104 / 117 / 132
-//   10 heads N = 4096              89*/ 109 / 120 / 135 / 175 / 226           231*/ 218 / 234 / 243 / 284 / 332
-//    3 heads N = 6016              71 /  78 /  75*/  84 /  97 / 110           169 / 186 / 156*/ 167 / 171 / 179
-//    1 head  N = 8192              75 /  51 /  50 /  49*/  60 /  65           185 / 105 /  99 /  91*/ 103 / 106
-//    5 heads N = 8192             162 / 168*/ 177 / 192 / 230 / 278           447 / 396*/ 411 / 416 / 456 / 502
-//    1 head  N = 12032            109 /  81 /  99 /  93*/ 100 / 103           268 / 194 / 237 / 197*/ 210 / 199
-//   16 heads N = 3072              76*/ 105 / 127 / 152 / 208 / 261           179*/ 203 / 223 / 246 / 300 / 351
-// Elementwise masks, token window of N / 4 and token-causal:
-//    2 heads N = 1024              18 /  17 /  16 /  17*/  15 /  16            42 /  28 /  24 /  20*/  19 /  19
-//    4 heads N = 2048              28 /  28 /  28 /  29*/  37 /  42            79 /  49 /  43 /  39*/  46 /  49
-//    8 heads N = 2048              29 /  33*/  45 /  46 /  60 /  75            79 /  57*/  56 /  62 /  69 /  78
-//    2 heads N = 4096              46 /  34 /  33 /  33*/  45 /  50           152 /  86 /  67 /  56*/  65 /  65
-//    8 heads N = 4000              71 /  95*/ 106 / 118 / 143 / 174           205 / 133*/ 169 / 157 / 183 / 210
-//    1 head  N = 8192              83 /  52 /  46 /  42*/  59 /  59           299 / 159 / 116 /  93*/ 103 /  99
-// (Set on fwd_pair_kernel, which had the block masks then: fwd_wide_kernel gains less from shares, up to 7 us at 5 heads of N = 832 and 7 of
-// N = 2048 would be saved without.)
+// D = 256: shares of a row block's list, at most (quad_shares.h says how many of them a list has).  fwd_wide_kernel has two workgroups on a
+// compute unit, so launches that leave the GPU's 512 short share, and those in little more than a round, whose last lists would run alone.
+// us, N(0,1) bf16, a fixed number of shares for all lists and a launch that summed their fp32 parts / the lists that their length
+// calls for, summed in the launch; keep 0.1, 0.3, 1, block-causal:
+//    1 head  N = 1024 (16 row blocks)   14 / 12     16 / 16     19 / 21     18 / 20
+//    2 heads N = 1344 (42)              17 / 12     20 / 18     25 / 23     23 / 22
+//    1 head  N = 4096 (64)              22 / 20     26 / 25     38 / 39     37 / 37
+//    4 heads N = 2048 (128)             26 / 21     30 / 23     39 / 36     36 / 32
+//    2 heads N = 4096 (128)             29 / 23     36 / 31     56 / 52     49 / 44
+//    7 heads N = 2048 (224)             29 / 18     35 / 28     53 / 46     48 / 40
+//    2 heads N = 6461 (202)             47 / 33     67 / 60    128 / 108    87 / 83
+//    3 heads N = 6016 (282)             50 / 34     74 / 64    150 / 158    98 / 87
+//    8 heads N = 4096 (512)             56 / 32     79 / 56    165 / 141   101 / 97
+//    5 heads N = 8192 (640)             94 / 67    162 / 153   396 / 394   223 / 215
+// Elementwise masks (on fwd_pair_kernel before), token window of 0.1 N, 0.25 N, 0.45 N, token-causal:
+//    2 heads N = 1024 (32)              14 / 11     17 / 14     19 / 18     20 / 20
+//    8 heads N = 2048 (256)             27 / 17     32 / 22     39 / 30     57 / 40
+//    8 heads N = 4000 (504)             70 / 29     95 / 44    127 / 65    134 / 94
+//    1 head  N = 8192 (128)             32 / 28     41 / 36     56 / 46     93 / 70
 static int pair_split_256(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   if (rows > 8 * nb || rows >= 1024) return 1;
@@ -1380,6 +1371,7 @@ static int pair_split_128(int64_t row_blocks, int nb) {
 //    1 head  N = 4096 (64)             16/15/16/16          20/22/19/18          32/43/30/24          30/43/29/23
 //    7 heads N = 1000 (112)            11/10                17/12                28/17                28/16
 //    2 heads N = 4096 (128)            22/15/16             26/22/20             40/43/32             35/43/30
+//    5 heads N = 256 (20)               - / -                                    9/10 (keep 0.9)                       (not there)
 //   11 heads N = 1344 (231)            10/10                17/13                30/20                30/19
 //    3 heads N = 4096 (192)            24/16/17             28/23/24             46/44/44             38/43/41
 //    2 heads N = 6016 (188)            25/18/19             33/31/32             57/60/61             48/59/45
@@ -1410,15 +1402,15 @@ static QuadPlan quad_plan(int64_t row_blocks, int nb, bool words) {
     if (nb < 28 || nb >= 150) return {0, 1};
     return {1, nb >= 80 ? 2 : 1};
   }
-  if (rows > 150 && rows <= 230 && nb >= 150) return {0, 1};
-  if (rows <= 128) return {2, rows <= 64 && nb >= 20 ? 4 : nb >= 24 ? 2 : 1};
+  if (nb < 6 || (rows > 150 && rows <= 230 && nb >= 150)) return {0, 1};
+  if (rows <= 128) return {2, rows <= 64 && nb >= SHARE_MIN_BLOCKS ? 4 : nb >= 24 ? 2 : 1};
   return {2, nb >= (rows <= 160 ? 40 : 80) ? 2 : 1};
 }
-static_assert(SHARE_MIN_BLOCKS <= 20, "heads of launches that share lists have as many row blocks");
+static_assert(SHARE_MIN_BLOCKS <= 24, "heads of launches that share lists have as many row blocks");
 
 // the parts of shared lists and a counter per list
-static size_t quad_parts_bytes(int B, int H, int nb, int split) {
-  return 256 + (split > 1 ? (size_t)B * H * nb * (split * 64 * (size_t)(128 + 2) * sizeof(float) + sizeof(unsigned long long)) : 0);
+static size_t quad_parts_bytes(int B, int H, int nb, int D, int split) {
+  return 256 + (split > 1 ? (size_t)B * H * nb * (split * 64 * (size_t)(D + 2) * sizeof(float) + sizeof(unsigned long long)) : 0);
 }
 
 static size_t pair_parts_bytes(int B, int H, int N, int D, int split) {
@@ -1466,8 +1458,29 @@ static ShortPlan short_plan(int64_t row_blocks, int nb) {
 static QuadPlan quad_plan(int B, int H, int nb, bool words, bool compact) {
   QuadPlan plan = quad_plan((int64_t)B * H * nb, nb, words);
   if (compact)
-    while (plan.split > 1 && quad_parts_bytes(B, H, nb, plan.split) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --plan.split;
+    while (plan.split > 1 && quad_parts_bytes(B, H, nb, 128, plan.split) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --plan.split;
   return plan;
+}
+
+// D = 256: the same by fwd_wide_kernel, at most this many shares of a list ...
+static int wide_split(int B, int H, int N, bool compact) {
+  const int nb = (N + 63) / 64;
+  int s = nb < SHARE_MIN_BLOCKS ? 1 : pair_split(B, H, N, 256, compact);
+  if (compact)
+    while (s > 1 && quad_parts_bytes(B, H, nb, 256, s) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --s;
+  return s;
+}
+
+// Tiles of a share, at least, of a launch that shares lists: a hand-off takes 2.5 us, three or four tiles' time where a workgroup is
+// alone on its compute unit, and evens out nothing where the GPU is full.  us, at least 4 / 6 / 8 (16, 24):
+//    D = 256   2 heads N = 1024, token-causal (32 row blocks)  20 / 21 / 26         1 head  N = 2048, keep 0.3 (32)  21 / 21 / 26
+//              2 heads N = 4096, keep 0.1 (128)                24 / 22 / 26         3 heads N = 4096, token-causal (192)  - / - / 50 (51, 69)
+//              8 heads N = 2048, token window of 512 (256)     25 / 21 / 22         5 heads N = 8192, keep 0.1 (640)  75 / 74 / 72 ( - , 66)
+//    D = 128   3 heads N = 1280, dense (60)                    26 / 17 / 17         2 heads N = 1024, token-causal (32)  14 / 14 / 16
+static int share_least(int64_t row_blocks, int D) {
+  const int64_t rows = row_blocks * 256 / compute_units();
+  if (D == 128) return rows <= 64 ? 6 : 8;
+  return rows <= 64 ? 4 : rows <= 256 ? 6 : 24;
 }
 
 // Launches whose workgroups have a row block each need no lists of a block mask: they take its columns from the mask (3 heads
@@ -1478,12 +1491,15 @@ bool launch_fwd_takes_mask(int B, int H, int N, int D) {
 }
 
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
-  if (D == 256) return pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
+  if (D == 256) {      // (compact: what a launch that sums parts of all lists would take, for which fewer shapes have room)
+    const size_t parts = pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
+    return compact ? parts : std::max(parts, quad_parts_bytes(B, H, (N + 63) / 64, D, wide_split(B, H, N, false)));
+  }
   if (D == 128) {
     const int nb = (N + 63) / 64;
     auto bytes = [&](bool words) {
       const QuadPlan plan = quad_plan(B, H, nb, words, compact);
-      return plan.groups > 0 ? quad_parts_bytes(B, H, nb, plan.split) : pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
+      return plan.groups > 0 ? quad_parts_bytes(B, H, nb, 128, plan.split) : pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
     };
     return compact ? bytes(false) : std::max(bytes(false), bytes(true));       // (compact launches: block masks only)
   }
@@ -1497,9 +1513,10 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
 // one size for bsattn_fwd and bsattn_fwd_elementwise
 size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_bytes(B, H, N, D); }
 
-void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
+void launch_fwd_pair(const FwdParams& prm, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
 void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st);   // attn_fwd_short.hip
 void launch_fwd_quad(const FwdParams& prm, int groups, int dt, bool elementwise, hipStream_t st);   // attn_fwd_quad.hip
+void launch_fwd_wide(const FwdParams& prm, int dt, bool elementwise, hipStream_t st);   // attn_fwd_wide.hip
 template <int D, int DT, int MODE, bool EW, int LAYOUT, bool SPREAD>
 static void launch_fwd_s(const FwdRangeParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
@@ -1601,7 +1618,8 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
   const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
   const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
-  const QuadPlan quads = s.D == 128 ? quad_plan(s.B, s.H, prm.nb, tile_bits != nullptr, s.compact) : QuadPlan{0, 1};
+  const QuadPlan quads = s.D == 128 ? quad_plan(s.B, s.H, prm.nb, tile_bits != nullptr, s.compact)
+                       : s.D == 256 ? QuadPlan{1, wide_split(s.B, s.H, s.N, s.compact)} : QuadPlan{0, 1};
   if (quads.groups > 0) {
     const int slots = compute_units() * (quads.groups == 1 ? 2 : 1), rows = heads * prm.nb, left = rows % slots;
     const size_t parts = (size_t)rows * quads.split * 64;
@@ -1610,11 +1628,13 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     prm.load = (int)((int64_t)rows * 4096 / slots);
     prm.tail_from = rows / slots * slots;
     prm.tail_shares = left > 0 ? slots / left : 1;
+    prm.share_least = share_least(rows, s.D);
     prm.part_o = (float*)ws + 64;
-    prm.part_ml = prm.part_o + parts * 128;
+    prm.part_ml = prm.part_o + parts * s.D;
     prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
     prm.epoch = next_epoch();
-    launch_fwd_quad(prm, quads.groups, dt, tile_bits != nullptr, st);
+    if (s.D == 128) launch_fwd_quad(prm, quads.groups, dt, tile_bits != nullptr, st);
+    else launch_fwd_wide(prm, dt, tile_bits != nullptr, st);
     return launch_status();
   }
   if (s.D != 64 || plan.pairs > 0) {
@@ -1624,7 +1644,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
     prm.part_len = (int*)(prm.part_ml + (size_t)prm.split * heads * s.N * 2);
     if (s.D == 64) launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
-    else launch_fwd_pair(prm, s.D, dt, tile_bits != nullptr, st);
+    else launch_fwd_pair(prm, dt, tile_bits != nullptr, st);
     return launch_status();
   }
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.compact);

@@ -1,4 +1,4 @@
-// Block-sparse FlashAttention-2 forward, head dimension 128, and 256 with elementwise masks (one wavefront per SIMD there, K and V fragments taken from LDS in two portions).
+// Block-sparse FlashAttention-2 forward, head dimension 128, launches that fill the GPU.
 //
 // At D = 128 a wavefront that owns 64 queries would need all 512 registers of its SIMD and be bound by instruction issue.
 // Here a row block belongs to a pair of wavefronts, 32 queries each (256 registers: two
@@ -18,16 +18,15 @@
 
 namespace bsattn {
 
-constexpr int PAIR_EARLY_V = 1;   // largest number of fragment portions (head dimension / 128) for which V is read early
+constexpr int PAIR_D = 128;
 constexpr int PAIR_COLS_CAP = 1024;                               // column indices of the row block kept in LDS
-template <int D> constexpr int pair_lds_bytes() { return 2 * 64 * 2 * D + 512 + PAIR_COLS_CAP * 4; }   // K tile, V tile, mask words, columns
+constexpr int PAIR_LDS_BYTES = 2 * 64 * 2 * PAIR_D + 512 + PAIR_COLS_CAP * 4;     // K tile, V tile, mask words, columns
 
-// CONTIG: the rows of K and of V follow each other without gaps (row stride = D).
 // TAIL: N is not a multiple of 64 (as in attn_fwd.hip: the copy of the last tile repeats its last key, the scores beyond
 // it are -inf, the queries beyond N are not written).
-template <int D, int DT, bool EW, bool CONTIG, bool TAIL>
-__global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const FwdParams prm) {
-  constexpr int KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, TILE_BYTES = 64 * ROWB;
+template <int DT, bool EW, bool TAIL>
+__global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
+  constexpr int D = PAIR_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, TILE_BYTES = 64 * ROWB;
   constexpr int PORTIONS = D / 128;              // K and V fragments are read in this many portions
   constexpr int KSP = KS / PORTIONS, DBP = DB / PORTIONS;
   constexpr bool BF16 = DT != 0;
@@ -36,7 +35,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   // V read before the softmax (see the loop).  (Elementwise masks too, since a query without mass is looked after by sum_limit and not
   // by every lane in every tile, which spilled V's registers with bf16: 32 heads N = 4000 token window of 1000 92 -> 86 us, token-causal
   // 210 -> 199, 16 heads N = 4000 token-causal 135 -> 125.)
-  constexpr bool EARLY_V = PORTIONS <= PAIR_EARLY_V;
+  constexpr bool CONTIG = false, EARLY_V = true;
   constexpr int HALF = CPR / 2;                  // copy instructions per wavefront and tile
   constexpr int KOPS = HALF + (EW ? 1 : 0), VOPS = HALF;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -370,7 +369,7 @@ __global__ __launch_bounds__(128, D == 128 ? 2 : 1) void fwd_pair_kernel(const F
   }
   const float inv = row_inverse<EW>(lsum);
   // the wavefront's 32 rows of O leave through its half of the (now idle) LDS
-  static_assert(2 * rows_out_bytes(D, true) <= pair_lds_bytes<D>(), "room for the result rows of both wavefronts");
+  static_assert(2 * rows_out_bytes(D, true) <= PAIR_LDS_BYTES, "room for the result rows of both wavefronts");
   __syncthreads();           // the other wavefront has left its last tile
   rows_out<BF16, D>(lds + w * rows_out_bytes(D, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2], prm.os[2], prm.out_f32,
                     lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return oacc[db][0][i] * inv; });
@@ -388,7 +387,7 @@ template <bool BF16, int S>
 __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm, int D, unsigned quads) {
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i >= quads) return;
-  const int qshift = D == 256 ? 6 : D == 128 ? 5 : 4;        // log2 of the threads per query row
+  const int qshift = D == 128 ? 5 : 4;                       // log2 of the threads per query row
   const unsigned rowg = i >> qshift;                         // row over all heads
   const int col = (int)(i & ((1u << qshift) - 1)) * 4;
   const int bh = (int)(rowg / (unsigned)prm.N), row = (int)(rowg - (unsigned)bh * prm.N);
@@ -425,11 +424,11 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
   if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + row] = row_lse(M, L);
 }
 
-// (one thread per 4 results of a launch that shares lists, which has fewer than 4 row blocks per compute unit (pair_split_256; half of
-// that at other head dimensions): 64 D / 4 threads each, 4 096 at most, so the values fit 32 bits)
+// (one thread per 4 results of a launch that shares lists, which has fewer than 2 row blocks per compute unit: 64 D / 4 threads each,
+// 2 048 at most, so the values fit 32 bits.  D: 64 or 128.)
 template <bool BF16, int S = 2>
 static void launch_sum_parts_t(const FwdParams& prm, int D, hipStream_t st) {
-  if constexpr (S < 8) {
+  if constexpr (S < 4) {
     if (prm.split != S) { launch_sum_parts_t<BF16, S + 1>(prm, D, st); return; }
   }
   const unsigned quads = (unsigned)((int64_t)prm.B * prm.H * prm.N * D / 4);
@@ -441,49 +440,35 @@ void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st) {
   else launch_sum_parts_t<false>(prm, D, st);
 }
 
-template <int D, int DT, bool EW, bool CONTIG, bool TAIL>
+template <int DT, bool EW, bool TAIL>
 static void launch_pair_c(const FwdParams& prm, int grid, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_pair_kernel<D, DT, EW, CONTIG, TAIL>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, pair_lds_bytes<D>());
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_pair_kernel<DT, EW, TAIL>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, PAIR_LDS_BYTES);
   });
-  hipLaunchKernelGGL((fwd_pair_kernel<D, DT, EW, CONTIG, TAIL>), dim3(grid), dim3(128), pair_lds_bytes<D>(), st, prm);
+  hipLaunchKernelGGL((fwd_pair_kernel<DT, EW, TAIL>), dim3(grid), dim3(128), PAIR_LDS_BYTES, st, prm);
 }
 
-template <int D, int DT, bool EW>
+template <int DT, bool EW>
 static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   const int grid = prm.place.per_share * prm.split;
-  // (the variant with immediate copy offsets: 5 % faster at D = 256, 3 % slower on dense masks at D = 128)
-  if (prm.N % 64 != 0) launch_pair_c<D, DT, EW, false, true>(prm, grid, st);
-  else if (D == 256 && prm.ks[2] == D && prm.vs[2] == D) launch_pair_c<D, DT, EW, D == 256, false>(prm, grid, st);
-  else launch_pair_c<D, DT, EW, false, false>(prm, grid, st);
-  if (prm.split > 1) launch_sum_parts(prm, D, DT != 0, st);
+  if (prm.N % 64 != 0) launch_pair_c<DT, EW, true>(prm, grid, st);
+  else launch_pair_c<DT, EW, false>(prm, grid, st);
+  if (prm.split > 1) launch_sum_parts(prm, PAIR_D, DT != 0, st);
 }
 
-template <int D>
-static void launch_pair_d(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
-  if constexpr (D == 128) {
-    if (!elementwise) {
-      if (dt == 0) launch_pair_t<D, 0, false>(prm, st);
-      else if (dt == 1) launch_pair_t<D, 1, false>(prm, st);
-      else launch_pair_t<D, 2, false>(prm, st);
-    }
-  }
-  if (elementwise) {
-    if (dt == 0) launch_pair_t<D, 0, true>(prm, st);
-    else if (dt == 1) launch_pair_t<D, 1, true>(prm, st);
-    else launch_pair_t<D, 2, true>(prm, st);
-  }
+template <bool EW>
+static void launch_pair_e(const FwdParams& prm, int dt, hipStream_t st) {
+  if (dt == 0) launch_pair_t<0, EW>(prm, st);
+  else if (dt == 1) launch_pair_t<1, EW>(prm, st);
+  else launch_pair_t<2, EW>(prm, st);
 }
 
-void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st);   // attn_fwd_wide.hip
-
-// D: 128 or 256 (block masks: attn_fwd_wide.hip, whose registers do not hold mask words beside the rest).  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
-void launch_fwd_pair(const FwdParams& prm, int D, int dt, bool elementwise, hipStream_t st) {
-  if (D == 128) launch_pair_d<128>(prm, dt, elementwise, st);
-  else if (!elementwise) launch_fwd_wide(prm, dt, st);
-  else launch_pair_d<256>(prm, dt, elementwise, st);
+// dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+void launch_fwd_pair(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
+  if (elementwise) launch_pair_e<true>(prm, dt, st);
+  else launch_pair_e<false>(prm, dt, st);
 }
 
 }  // namespace bsattn

@@ -78,15 +78,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdParams pr
   int shares = 1;
   if (prm.split > 1) {                            // this workgroup's share of the row block's list
     const int len = t1 - t0;
-    if (len >= 2 * SHARE_MIN) {
-      const bool last_round = (int)blockIdx.x - chunk * prm.place.per_share >= prm.tail_from;
-      int mid = 0, end = 0;
-      if (!last_round || prm.tail_shares < prm.split) {
-        if (listed) { mid = rp[nb / 2 + SHARE_SAMPLE / 2] - rp[nb / 2 - SHARE_SAMPLE / 2]; end = rp[nb] - rp[nb - SHARE_SAMPLE]; }
-        else { mid = length_of_rows(prm, b, h, nb / 2 - SHARE_SAMPLE / 2, lane); end = length_of_rows(prm, b, h, nb - SHARE_SAMPLE, lane); }
-      }
-      shares = quad_shares(len, mid, end, last_round ? prm.tail_shares : 1, prm.load, prm.split);
-    }
+    shares = shares_of_list(prm, rp, b, h, len, (int)blockIdx.x - chunk * prm.place.per_share, listed, lane);
     if (chunk >= shares) return;
     t1 = t0 + (int)((int64_t)len * (chunk + 1) / shares);
     t0 = t0 + (int)((int64_t)len * chunk / shares);
@@ -346,16 +338,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdParams pr
   }
   wait_vm<0>();
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long old = seen;
-    for (;;) {     // (ends: the counter only changes when another share is counted, at most `shares` times)
-      const unsigned long long want = (old >> 16) == prm.epoch ? old + 1 : ((prm.epoch << 16) | 1ull);
-      if (__hip_atomic_compare_exchange_strong(arrivals, &old, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-        lcols[0] = (int)(want & 0xffffull);
-        break;
-      }
-    }
-  }
+  if (threadIdx.x == 0) lcols[0] = count_in(arrivals, prm.epoch, seen);
   __syncthreads();
   if (__builtin_amdgcn_readfirstlane(*(volatile int*)lcols) != shares) return;
   floatx4 acc[QT];

@@ -1,19 +1,22 @@
 // Block-sparse FlashAttention-2 forward, head dimension 256.
 //
-// A workgroup of four wavefronts has one row block, or one of `split` contiguous shares of its list: wavefront (kh, w) takes keys
+// A workgroup of four wavefronts has one row block, or a share of its list (quad_shares.h): wavefront (kh, w) takes keys
 // 32 kh .. of every tile for queries 32 w .. .  O of 32 queries is 128 registers and Q 64; with the scores of 32 keys in place of
 // 64 the rest fits a quarter of a SIMD's registers, so two wavefronts share a SIMD and one's products run beside the other's
 // softmax.  A K and a V tile (64 KB) are shared by the four, two workgroups per compute unit; the next K tile is asked for as soon
-// as all hold their K fragments, the next V tile as soon as all hold their V fragments (four barriers per tile).  The two key halves
-// keep a reference exponent and a sum each and meet in LDS at the end, half of the columns each way.
+// as all hold their K fragments, the next V tile as soon as all hold their V fragments.  Two barriers per tile: in front of the one that
+// frees the K buffer every wavefront waits for its part of V, in front of the one that frees V for its part of the next K.  (Four, with
+// waits of their own: 10 heads N = 4090 keep 0.3 95 -> 92 us, 2 heads N = 20800 dense 978 -> 947, 16 heads N = 8192 keep 0.3 378 -> 369.)  The two
+// key halves keep a reference exponent and a sum each and meet in LDS at the end, half of the columns each way.  Shares of a list
+// (quad_shares.h) meet in the workspace, in the same launch.
 //
 // Before, fwd_pair_kernel: a wavefront with the scores of all 64 keys, up to 512 registers, alone on its SIMD, so that scores, softmax
 // and second product came one after the other.  us: 16 heads N = 4096 block-causal keep 0.5 bf16 108 -> 96, results in fp32
 // 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  Ragged: 16 heads
 // N = 4000 causal keep 0.5 bf16 168 -> 95 (fwd_pair_kernel spilled), 10 heads N = 4090 keep 0.3 142 -> 93, fp16 N = 4065 dense
-// block-causal 214 -> 170.  The 256 registers
-// leave no room for mask words (20 to 140 spilled): elementwise masks stay on fwd_pair_kernel.  Three variants keep a few values in scratch
-// memory as it is: fp16 with strided rows 8 bytes per lane (ragged 20), ragged bf16 with P in fp16 and contiguous rows 8.
+// block-causal 214 -> 170.  Elementwise masks: 16 heads N = 4000 token window of 1000 127 -> 81, token-causal 215 -> 143, fp16 N = 4096 101 -> 86
+// and 180 -> 156.  A few variants keep values in scratch memory: fp16 with strided rows 20 to 36 bytes per lane, fp16 elementwise with
+// contiguous rows 8 or 12, bf16 with P in either type, whole tiles and contiguous rows 12 (outside the walk).
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196 of the reference).
 #include "common.h"
@@ -25,7 +28,8 @@ namespace bsattn {
 constexpr int WIDE_D = 256, WIDE_COLS_CAP = 1024;                               // column indices of the row block kept in LDS
 constexpr int WIDE_TILE_BYTES = 64 * 2 * WIDE_D;
 constexpr int WIDE_COLS_OFF = 2 * WIDE_TILE_BYTES;
-constexpr int WIDE_LDS_BYTES = WIDE_COLS_OFF + WIDE_COLS_CAP * 4;               // K tile, V tile, columns
+constexpr int WIDE_BITS_OFF = WIDE_COLS_OFF + WIDE_COLS_CAP * 4;
+constexpr int WIDE_LDS_BYTES = WIDE_BITS_OFF + 512;                             // K tile, V tile, columns, mask words
 static_assert(MASK_MAX_BLOCKS <= WIDE_COLS_CAP, "all columns from the mask are in LDS");
 static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the result rows of all wavefronts");
 
@@ -33,7 +37,8 @@ static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the res
 // CONTIG: the rows of K and of V follow each other without gaps (row stride = 256).
 // TAIL: N is not a multiple of 64: the copy of the last tile repeats its last key, the scores beyond it are -inf (a half without
 // any key leaves the tile out), the queries beyond N are not written.
-template <int DT, bool CONTIG, bool TAIL>
+// EW: elementwise masks (bit 30 of a staged column says "partly set", the tile's 64 row words travel with K).
+template <int DT, bool CONTIG, bool TAIL, bool EW>
 __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   constexpr int D = WIDE_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
   constexpr int COPIES = CPR / 4;                // copy instructions per wavefront and tile
@@ -60,16 +65,17 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
     for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const uintx4*>(qp + 16 * s + 8 * g);
   }
   int* lcols = reinterpret_cast<int*>(lds + WIDE_COLS_OFF);
-  const bool listed = prm.mask == nullptr;
+  const bool listed = EW || prm.mask == nullptr;
   int t0, t1;
   if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
   else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols, chunk == 0 && wave == 0); }
+  int shares = 1;
   if (prm.split > 1) {                           // this workgroup's share of the row block's list
     const int len = t1 - t0;
-    if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
-    t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
-    t0 = t0 + (int)((int64_t)len * chunk / prm.split);
-    if (t0 == t1) return;                        // (pair_sum_parts_kernel knows which shares are empty)
+    shares = shares_of_list(prm, rp, b, h, len, (int)blockIdx.x - chunk * prm.place.per_share, listed, lane);
+    if (chunk >= shares) return;
+    t1 = t0 + (int)((int64_t)len * (chunk + 1) / shares);
+    t0 = t0 + (int)((int64_t)len * chunk / shares);
   }
   void* obase = out_base(prm, b, h);
   if (t0 == t1) {                                // no kept tile: O = 0, lse = -inf
@@ -92,7 +98,14 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
 
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
   const int first_t = listed ? t0 : 0;           // entry t of the list is lcols[t - first_t] once it is staged
-  auto col_of = [&](int t) { return t - first_t < WIDE_COLS_CAP ? lcols[t - first_t] : cols[t]; };
+  typedef const unsigned char __attribute__((address_space(4)))* cbyte_ptr_t;
+  constexpr int COL_MASK = 0x3fffffff;
+  auto flagged_col = [&](int t) {
+    int x = cols[t];
+    if constexpr (EW) x |= (int)((cbyte_ptr_t)(uintptr_t)prm.tile_partial)[t] << 30;
+    return x;
+  };
+  auto col_of = [&](int t) { return t - first_t < WIDE_COLS_CAP ? lcols[t - first_t] : flagged_col(t); };
 
   // asynchronous tile copies: instruction j covers tile rows 2j, 2j + 1; this wavefront issues [8 wave, 8 wave + 8) of a tile.
   // The swizzles repeat every 16 rows for K (8 instructions) and every 4 rows for V (2): instruction j reads chunk
@@ -127,7 +140,10 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       tile_load_async_one(tile, 2u * (unsigned)(src * (int)rs + (((lane_t % CPR) ^ swz(row)) * 8)), lds_addr + j * 1024);
     }
   };
-  auto k_copy = [&](int cb) {
+  auto k_copy = [&](int cb, int t) {
+    if constexpr (EW) {
+      if (wave < 2) words_load_async(prm.tile_bits + (int64_t)t * 64, 4u * (unsigned)lane + 256u * wave, lds_k_addr + WIDE_BITS_OFF + wave * 256);
+    }
     if (TAIL && cb == tail_cb) {
       tail_copy(kg + (int64_t)cb * 64 * prm.ks[2], prm.ks[2], lds_k_addr, [](int row) { return k_swz<D>(row); });
       return;
@@ -155,11 +171,16 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   const uintx4 ones_frag = {g == 0 ? 0x3c003c00u : 0u, 0u, 0u, 0u};
 
   // first tile's copies (its column from one scalar load), then the column list into LDS
-  int cb = listed ? cols[t0] : __builtin_amdgcn_readfirstlane(lcols[t0]);
-  k_copy(cb);
-  v_copy(cb);
-  if (listed)
-    for (int i = threadIdx.x; i < t1 - t0 && i < WIDE_COLS_CAP; i += 256) lcols[i] = prm.col_idx[t0 + i];
+  int cx = listed ? flagged_col(t0) : __builtin_amdgcn_readfirstlane(lcols[t0]);
+  k_copy(cx & COL_MASK, t0);
+  v_copy(cx & COL_MASK);
+  if (listed) {
+    for (int i = threadIdx.x; i < t1 - t0 && i < WIDE_COLS_CAP; i += 256) {
+      int x = prm.col_idx[t0 + i];
+      if constexpr (EW) x |= (int)prm.tile_partial[t0 + i] << 30;
+      lcols[i] = x;
+    }
+  }
   __builtin_amdgcn_s_waitcnt(0x0F70);               // vmcnt(0), visible to the compiler: Q and the first tiles
   if constexpr (FOLD) {
 #pragma unroll
@@ -175,7 +196,8 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
   for (int db = 0; db < DB; ++db)
 #pragma unroll
     for (int i = 0; i < 16; ++i) oacc[db][0][i] = 0.f;
-  float m_i = 0.f, l_i = 0.f;
+  // (while a query has no mass every tile is recentred (sum_limit); one that does not exist never would have any)
+  float m_i = 0.f, l_i = EW && TAIL && qrow >= prm.N ? 1e-30f : 0.f;
   uintx4 mfrag = {0u, 0u, 0u, 0u};
   bool fresh = true;
   float limit = FOLD ? SUM_LIMIT : 0.f;
@@ -184,12 +206,13 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
 
   for (int t = t0; t < t1; ++t) {
     const bool has1 = t + 1 < t1;
-    const int cbn = has1 ? __builtin_amdgcn_readfirstlane(col_of(t + 1)) : 0;
+    const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(t + 1)) : 0;
     asm volatile("" : "+v"(kbase), "+v"(vbase), "+v"(kx), "+v"(vx));    // (or the turned addresses are computed before the loop and held)
     // ---- S^T = K Q^T (- m when FOLD), K fragments in portions of four ----
     floatx16 sc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+    unsigned mw = 0u;
     uintx4 kfr[2][4];
     auto read_k = [&](int pt) {
 #pragma unroll
@@ -203,9 +226,13 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
     for (int pt = 0; pt < 4; ++pt) {
       if (pt < 3) read_k(pt + 1);
       if (pt == 3) {
+        if constexpr (EW) {
+          if ((cx >> 30) != 0) mw = reinterpret_cast<const unsigned*>(lds + WIDE_BITS_OFF)[2 * (32 * w + ln) + kh] >> (4 * g);
+        }
+        wait_vm<0>();                               // this wavefront's part of V(t) has landed
         lds_wait();
-        __syncthreads();                            // all wavefronts hold their K fragments: the K buffer is free
-        if (has1) k_copy(cbn);
+        __syncthreads();                            // ... and the others'; all hold their K fragments: the K buffer is free
+        if (has1) k_copy(cxn & COL_MASK, t + 1);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) sc = mfma_qk<BF16>(kfr[pt & 1][i], qf[4 * pt + i], sc);
@@ -214,14 +241,20 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       if (any_m) sc = mfma_qk<BF16>(ones_frag, mfrag, sc);
     }
     uintx4 pf[2];
-    const int keys = TAIL && cb == tail_cb ? valid - 32 * kh : 32;      // of this half
-    if (TAIL && keys < 32) {
+    const int keys = TAIL && !EW && cx == tail_cb ? valid - 32 * kh : 32;      // of this half
+    if constexpr (EW) {
+      if ((cx >> 30) != 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sc[i] = (mw & (1u << (8 * (i / 4) + (i % 4)))) ? sc[i] : -INFINITY;
+      }
+    }
+    if (TAIL && !EW && keys < 32) {
       int first_key = 4 * g;
       asm volatile("" : "+v"(first_key));
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[i] = 8 * (i / 4) + (i % 4) + first_key < keys ? sc[i] : -INFINITY;
     }
-    if (TAIL && keys <= 0) {
+    if (TAIL && !EW && keys <= 0) {
       pf[0] = pf[1] = uintx4{0u, 0u, 0u, 0u};
     } else {
       float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
@@ -236,8 +269,6 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
       l_i = lnew;
       fresh = false;
     }
-    if (has1) wait_vm<COPIES>(); else wait_vm<0>();   // this wavefront's part of V(t) has landed (K(t+1) may be in flight)
-    if (t > t0) __syncthreads();                    // ... and the others' (the first tile was waited for above)
     // ---- O^T += V^T P^T, V^T fragments in portions of two column blocks ----
     uintx4 vfr[2][2][2];
     auto read_v = [&](int pt) {
@@ -262,9 +293,10 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
     for (int pt = 0; pt < 4; ++pt) {
       if (pt < 3) read_v(pt + 1);
       if (pt == 3) {
+        wait_vm<0>();                               // this wavefront's part of K(t+1) has landed
         lds_wait();
-        __syncthreads();                            // all wavefronts hold their V fragments: the V buffer is free
-        if (has1) v_copy(cbn);
+        __syncthreads();                            // ... and the others'; all hold their V fragments: the V buffer is free
+        if (has1) v_copy(cxn & COL_MASK);
       }
 #pragma unroll
       for (int ts = 0; ts < 2; ++ts)
@@ -275,11 +307,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
           oacc[2 * pt + d][0] = mfma_qk<PB>(a, pf[ts], oacc[2 * pt + d][0]);
         }
     }
-    if (has1) {
-      wait_vm<COPIES>();                              // this wavefront's part of K(t+1) has landed (V(t+1) may be in flight)
-      __syncthreads();                              // ... and the others'
-    }
-    if constexpr (TAIL) cb = cbn;
+    if constexpr (TAIL || EW) cx = cxn;
   }
 
   // ---- the key halves meet: each hands over the columns the other finishes ----
@@ -303,12 +331,17 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) res[db][i] = kh == 0 ? oacc[db][0][i] : oacc[DB / 2 + db][0][i];
   }
+  unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + m;
+  unsigned long long seen = 0ull;      // (the read travels beside the merge)
+  if (shares > 1 && threadIdx.x == 0) seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   const int other = (64 * (1 - kh) + 32 * w + ln) * 2;
-  const float m_oth = ml[other], l_oth = ml[other + 1], M = fmaxf(m_own, m_oth);
+  const float m_oth = ml[other], l_oth = ml[other + 1];
+  float M = fmaxf(m_own, m_oth);
   const float wo = m_own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_own - M);
   const float wt = m_oth == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_oth - M);
-  const float L = wo * lsum + wt * l_oth;
+  // (both halves round it the same way: a share's sum is the same whether it comes from the workspace or from registers)
+  float L = (kh == 0 ? wo : wt) * (kh == 0 ? lsum : l_oth) + (kh == 0 ? wt : wo) * (kh == 0 ? l_oth : lsum);
 #pragma unroll
   for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
@@ -317,54 +350,94 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) res[db][4 * i4 + e] = wo * res[db][4 * i4 + e] + wt * x[e];
     }
-  if (prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
-    if (TAIL && qrow >= prm.N) return;
-    float* part = prm.part_o + ((int64_t)chunk * BH + bh) * prm.N * D;
+  if (shares > 1) {
+    // the shares of a list meet in the workspace, as the parts of a row block do in attn_fwd.hip: each is published with device-scope
+    // stores and counted in once these are acknowledged, the last one in adds all of them up in their order
+    const int64_t first_slot = ((int64_t)bh * nb + m) * prm.split;
+    auto slot_of = [&](int p) { return prm.part_o + (first_slot + p) * (64 * D) + wave * (64 * 64) + lane * 4; };      // [wavefront][quad][lane][4]
+    auto ml_of = [&](int p) { return prm.part_ml + (first_slot + p) * 128 + 2 * (32 * w + ln); };
 #pragma unroll
     for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4)
-        store_out4<BF16>(part, qrow * D + 128 * kh + 32 * db + 8 * i4 + 4 * g, true, res[db][4 * i4], res[db][4 * i4 + 1],
-                         res[db][4 * i4 + 2], res[db][4 * i4 + 3]);
-    if (g == 0 && kh == 0) {
-      float* pml = prm.part_ml + (((int64_t)chunk * BH + bh) * prm.N + qrow) * 2;
-      pml[0] = M; pml[1] = L;
+        coherent_store4(slot_of(chunk) + (4 * db + i4) * 256, res[db][4 * i4], res[db][4 * i4 + 1], res[db][4 * i4 + 2], res[db][4 * i4 + 3]);
+    if (kh == 0 && g == 0) { coherent_store(ml_of(chunk), M); coherent_store(ml_of(chunk) + 1, L); }
+    wait_vm<0>();
+    __syncthreads();
+    if (threadIdx.x == 0) lcols[0] = count_in(arrivals, prm.epoch, seen);
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(*(volatile int*)lcols) != shares) return;
+    floatx16 acc[DB / 2];
+#pragma unroll
+    for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
+    float Ms = -INFINITY, Ls = 0.f;
+    for (int p = 0; p < shares; ++p) {
+      floatx4 x[DB / 2][4];
+      float mp = M, lp = L;
+      if (p == chunk) {
+#pragma unroll
+        for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+          for (int i4 = 0; i4 < 4; ++i4) x[db][i4] = {res[db][4 * i4], res[db][4 * i4 + 1], res[db][4 * i4 + 2], res[db][4 * i4 + 3]};
+      } else {
+        mp = coherent_load(ml_of(p));
+        lp = coherent_load(ml_of(p) + 1);
+#pragma unroll
+        for (int db = 0; db < DB / 2; ++db) coherent_load4x4(slot_of(p) + db * 1024, x[db][0], x[db][1], x[db][2], x[db][3]);
+      }
+      const float mn = fmaxf(Ms, mp);              // a side without mass has maximum -inf and weight 0
+      const float ws = Ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Ms - mn), wp = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mn);
+      Ls = Ls * ws + lp * wp;
+      Ms = mn;
+#pragma unroll
+      for (int db = 0; db < DB / 2; ++db)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[db][i] = acc[db][i] * ws + wp * x[db][i / 4][i % 4];
     }
-    return;
+    // back to zero, so that a replay of this launch (same mark) starts from a clean counter
+    if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    M = Ms; L = Ls;
+#pragma unroll
+    for (int db = 0; db < DB / 2; ++db) res[db] = acc[db];
   }
-  const float inv = row_inverse<false>(L);
+  const float inv = row_inverse<EW>(L);
   __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
   rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
                         prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });
   if (prm.lse != nullptr && kh == 0 && g == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(M, L);
 }
 
-template <int DT, bool CONTIG, bool TAIL>
+template <int DT, bool CONTIG, bool TAIL, bool EW>
 static void launch_wide_c(const FwdParams& prm, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL, EW>), hipFuncAttributeMaxDynamicSharedMemorySize,
                               WIDE_LDS_BYTES);
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG, TAIL>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
+  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG, TAIL, EW>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
 }
 
-template <int DT>
+template <int DT, bool EW>
 static void launch_wide_t(const FwdParams& prm, hipStream_t st) {
   const bool contig = prm.ks[2] == WIDE_D && prm.vs[2] == WIDE_D;
-  if (prm.N % 64 != 0) { if (contig) launch_wide_c<DT, true, true>(prm, st); else launch_wide_c<DT, false, true>(prm, st); }
-  else { if (contig) launch_wide_c<DT, true, false>(prm, st); else launch_wide_c<DT, false, false>(prm, st); }
+  if (prm.N % 64 != 0) { if (contig) launch_wide_c<DT, true, true, EW>(prm, st); else launch_wide_c<DT, false, true, EW>(prm, st); }
+  else { if (contig) launch_wide_c<DT, true, false, EW>(prm, st); else launch_wide_c<DT, false, false, EW>(prm, st); }
 }
 
-void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st);   // attn_fwd_pair.hip
+// dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
+template <bool EW>
+static void launch_wide_e(const FwdParams& prm, int dt, hipStream_t st) {
+  if (dt == 0) launch_wide_t<0, EW>(prm, st);
+  else if (dt == 1) launch_wide_t<1, EW>(prm, st);
+  else launch_wide_t<2, EW>(prm, st);
+}
 
-// Block masks.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
-void launch_fwd_wide(const FwdParams& prm, int dt, hipStream_t st) {
-  if (dt == 0) launch_wide_t<0>(prm, st);
-  else if (dt == 1) launch_wide_t<1>(prm, st);
-  else launch_wide_t<2>(prm, st);
-  if (prm.split > 1) launch_sum_parts(prm, WIDE_D, dt != 0, st);
+void launch_fwd_wide(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
+  if (elementwise) launch_wide_e<true>(prm, dt, st);
+  else launch_wide_e<false>(prm, dt, st);
 }
 
 }  // namespace bsattn

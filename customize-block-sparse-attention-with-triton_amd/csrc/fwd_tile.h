@@ -25,7 +25,7 @@ struct FwdParams {
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair kernel: workgroups per row block (1: results written directly)
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
-  int tail_from, tail_shares, load;      // quad kernel: see quad_shares
+  int tail_from, tail_shares, load, share_least;      // quad and wide kernel: see quad_shares
   int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
@@ -130,6 +130,29 @@ __device__ __forceinline__ int length_of_rows(const FwdParams& prm, int b, int h
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
   return __builtin_amdgcn_readfirstlane(n);
+}
+
+// Shares of the list of len tiles of the row block of workgroup `linear` (of the workgroups that come first on their lists).
+__device__ __forceinline__ int shares_of_list(const FwdParams& prm, cint_ptr_t rp, int b, int h, int len, int linear, bool listed, int lane) {
+  if (len < 2 * prm.share_least) return 1;
+  const bool last_round = linear >= prm.tail_from;
+  int mid = 0, end = 0;
+  if (!last_round || prm.tail_shares < prm.split) {
+    const int nb = prm.nb;
+    if (listed) { mid = rp[nb / 2 + SHARE_SAMPLE / 2] - rp[nb / 2 - SHARE_SAMPLE / 2]; end = rp[nb] - rp[nb - SHARE_SAMPLE]; }
+    else { mid = length_of_rows(prm, b, h, nb / 2 - SHARE_SAMPLE / 2, lane); end = length_of_rows(prm, b, h, nb - SHARE_SAMPLE, lane); }
+  }
+  return quad_shares(len, mid, end, last_round ? prm.tail_shares : 1, prm.load, prm.split, prm.share_least);
+}
+
+// Counts a share of a list in, by one thread, when all accesses of its workgroup to its part have been acknowledged; returns how many
+// are in.  The counter holds (launch mark << 16 | shares counted); stale contents carry another mark.  seen: a first guess of it.
+__device__ __forceinline__ int count_in(unsigned long long* arrivals, unsigned long long epoch, unsigned long long seen) {
+  for (;;) {     // (ends: the counter only changes when another share is counted, at most as often as the list has shares)
+    const unsigned long long want = (seen >> 16) == epoch ? seen + 1 : ((epoch << 16) | 1ull);
+    if (__hip_atomic_compare_exchange_strong(arrivals, &seen, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return (int)(want & 0xffffull);
+  }
 }
 
 __device__ __forceinline__ void* out_base(const FwdParams& prm, int b, int h) {
