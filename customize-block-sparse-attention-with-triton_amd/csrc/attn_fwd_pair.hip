@@ -8,7 +8,9 @@
 // whose parts a second launch sums (pair_split).  Heads are taken in groups
 // of 8, head i of a group on XCD i (place.h), so that the
 // row blocks resident on an XCD share one head's K and V in its L2; long row blocks of
-// block-causal masks come first.
+// block-causal masks come first.  Two barriers per tile: in front of the one that frees the K buffer both wavefronts wait for their
+// halves of V, in front of the one that frees V for those of the next K.  (Four, with waits of their own: 16 heads N = 8192 dense 641 -> 541 us,
+// keep 0.3 193 -> 187, 28 heads N = 2048 dense 72 -> 70, 16 heads N = 4000 token-causal 125 -> 122; block-causal masks the same.)
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196
 // of the reference), with a single block of 32 queries per wavefront.
@@ -27,17 +29,13 @@ constexpr int PAIR_LDS_BYTES = 2 * 64 * 2 * PAIR_D + 512 + PAIR_COLS_CAP * 4;   
 template <int DT, bool EW, bool TAIL>
 __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
   constexpr int D = PAIR_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, TILE_BYTES = 64 * ROWB;
-  constexpr int PORTIONS = D / 128;              // K and V fragments are read in this many portions
-  constexpr int KSP = KS / PORTIONS, DBP = DB / PORTIONS;
   constexpr bool BF16 = DT != 0;
   constexpr bool PB = DT == 2;                   // P rounded to bf16, second product in bf16 (V as it is)
   constexpr bool FOLD = !BF16;
   // V read before the softmax (see the loop).  (Elementwise masks too, since a query without mass is looked after by sum_limit and not
   // by every lane in every tile, which spilled V's registers with bf16: 32 heads N = 4000 token window of 1000 92 -> 86 us, token-causal
   // 210 -> 199, 16 heads N = 4000 token-causal 135 -> 125.)
-  constexpr bool CONTIG = false, EARLY_V = true;
   constexpr int HALF = CPR / 2;                  // copy instructions per wavefront and tile
-  constexpr int KOPS = HALF + (EW ? 1 : 0), VOPS = HALF;
   extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -124,7 +122,7 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
     for (int par = 0; par < VPER; ++par)
       voff[par] = 2u * (unsigned)(row0 * (int)prm.vs[2] + ((ch ^ v_swz<D>(par * RPI + row0)) * 8));
   }
-  const int64_t k_rs = CONTIG ? (int64_t)D : prm.ks[2], v_rs = CONTIG ? (int64_t)D : prm.vs[2];   // row strides
+  const int64_t k_rs = prm.ks[2], v_rs = prm.vs[2];   // row strides
   // (the lane index as a value the compiler cannot trace back, or the offsets are computed before the loop and held)
   auto tail_copy = [&](const unsigned short* tile, int64_t rs, unsigned lds_addr, auto&& swz) {
     int lane_t = lane;
@@ -139,11 +137,6 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
     const unsigned short* tile = kg + (int64_t)cb * 64 * k_rs;
     if (TAIL && cb == tail_cb) {
       tail_copy(tile, k_rs, lds_k_addr, [](int row) { return k_swz<D>(row); });
-    } else if constexpr (CONTIG) {     // (instruction j reads at byte 1024 j of the tile and writes at byte 1024 j of the buffer)
-#pragma unroll
-      for (int jb = 0; jb < HALF; jb += 4)
-        tile_load_async_four(tile + (w * HALF + jb) * RPI * D, koff[jb % KPER], koff[(jb + 1) % KPER], koff[(jb + 2) % KPER],
-                             koff[(jb + 3) % KPER], lds_k_addr + (w * HALF + jb) * 1024);
     } else {
 #pragma unroll
       for (int jj = 0; jj < HALF; ++jj) {
@@ -160,11 +153,6 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
     const unsigned short* tile = vg + (int64_t)cb * 64 * v_rs;
     if (TAIL && cb == tail_cb) {
       tail_copy(tile, v_rs, lds_v_addr, [](int row) { return v_swz<D>(row); });
-    } else if constexpr (CONTIG) {
-#pragma unroll
-      for (int jb = 0; jb < HALF; jb += 4)
-        tile_load_async_four(tile + (w * HALF + jb) * RPI * D, voff[jb % VPER], voff[(jb + 1) % VPER], voff[(jb + 2) % VPER],
-                             voff[(jb + 3) % VPER], lds_v_addr + (w * HALF + jb) * 1024);
     } else {
 #pragma unroll
       for (int jj = 0; jj < HALF; ++jj) {
@@ -231,26 +219,26 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) { s0[i] = 0.f; s1[i] = 0.f; }
     unsigned long long mw = 0ull;
-#pragma unroll
-    for (int pt = 0; pt < PORTIONS; ++pt) {
-      uintx4 kfr[2][KSP];
+    {
+      uintx4 kfr[2][KS];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int s = 0; s < KSP; ++s) kfr[kb][s] = *reinterpret_cast<const uintx4*>(lds_k + kaddr[kb][pt * KSP + s]);
-      if (pt == PORTIONS - 1) {
+        for (int s = 0; s < KS; ++s) kfr[kb][s] = *reinterpret_cast<const uintx4*>(lds_k + kaddr[kb][s]);
+      {
         if constexpr (EW) { if (partial) mw = lds_bits[32 * w + ln] >> (4 * g); }
         else if constexpr (TAIL) {
           if (partial) { mw = ((1ull << valid) - 1ull) >> (4 * g); asm volatile("" : "+v"(mw)); }
         }
+        wait_vm<0>();                               // this wavefront's half of V(t) has landed
         lds_wait();
-        __syncthreads();                            // both wavefronts hold their K fragments: the K buffer is free
+        __syncthreads();                            // ... and the other half; both hold their K fragments: the K buffer is free
         if (has1) k_copy(cxn & COL_MASK, t + 1);
       }
 #pragma unroll
-      for (int s = 0; s < KSP; ++s) {
-        s0 = mfma_qk<BF16>(kfr[0][s], qf[0][pt * KSP + s], s0);
-        s1 = mfma_qk<BF16>(kfr[1][s], qf[0][pt * KSP + s], s1);
+      for (int s = 0; s < KS; ++s) {
+        s0 = mfma_qk<BF16>(kfr[0][s], qf[0][s], s0);
+        s1 = mfma_qk<BF16>(kfr[1][s], qf[0][s], s1);
       }
     }
     if constexpr (FOLD) {
@@ -272,19 +260,15 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
     }
     uintx4 pf[4][2];
     // ---- V^T fragments ----
-    auto v_landed = [&]() {
-      if (has1) wait_vm<KOPS>(); else wait_vm<0>();   // this wavefront's half of V(t) has landed (K(t+1) may be in flight)
-      if (t > t0) __syncthreads();                    // ... and the other half (the first tile was waited for above)
-    };
-    auto read_v = [&](int pt, uintx4 (&vfr)[4][DBP]) {
+    auto read_v = [&](uintx4 (&vfr)[4][DB]) {
 #pragma unroll
       for (int ts = 0; ts < 4; ++ts)
 #pragma unroll
-        for (int db = 0; db < DBP; ++db) {
+        for (int db = 0; db < DB; ++db) {
           uintx4 a;
 #pragma unroll
           for (int jh = 0; jh < 2; ++jh) {
-            const int key = 16 * ts + 8 * jh + vkey0, col = 32 * (pt * DBP + db) + vcol0;
+            const int key = 16 * ts + 8 * jh + vkey0, col = 32 * db + vcol0;
             const int addr = key * ROWB + (((col >> 3) ^ v_swz<D>(key)) * 16) + (col & 7) * 2;
             const short4v rr = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (short4v __attribute__((address_space(3)))*)(lds_v + addr));
@@ -296,16 +280,17 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
         }
     };
     auto v_free = [&]() {
+      wait_vm<0>();                               // this wavefront's half of K(t+1) has landed
       lds_wait();
-      __syncthreads();                            // both wavefronts hold their V fragments: the V buffer is free
+      __syncthreads();                            // ... and the other half; both hold their V fragments: the V buffer is free
       if (has1) v_copy(cxn & COL_MASK);
     };
-    auto second = [&](int pt, uintx4 (&vfr)[4][DBP]) {
+    auto second = [&](uintx4 (&vfr)[4][DB]) {
 #pragma unroll
       for (int ts = 0; ts < 4; ++ts)
 #pragma unroll
-        for (int db = 0; db < DBP; ++db)
-          oacc[pt * DBP + db][0] = mfma_qk<PB>(vfr[ts][db], pf[ts][0], oacc[pt * DBP + db][0]);
+        for (int db = 0; db < DB; ++db)
+          oacc[db][0] = mfma_qk<PB>(vfr[ts][db], pf[ts][0], oacc[db][0]);
     };
     auto numerators = [&]() {
       float lnew = softmax_tile<FOLD, PB>(s0, s1, qk_scale, m_i, l_i, pf, 0);
@@ -320,32 +305,14 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
       l_i = lnew;
       fresh = false;
     };
-    if constexpr (EARLY_V) {
+    {
       // The V fragments are read before the softmax (they take the registers of the K fragments), so
       // that the next V tile is requested that much earlier: its latency was exposed otherwise.
-      uintx4 vfr[PORTIONS][4][DBP];
-      v_landed();
-#pragma unroll
-      for (int pt = 0; pt < PORTIONS; ++pt) read_v(pt, vfr[pt]);
+      uintx4 vfr[4][DB];
+      read_v(vfr);
       v_free();
       numerators();
-#pragma unroll
-      for (int pt = 0; pt < PORTIONS; ++pt) second(pt, vfr[pt]);
-    } else {
-      numerators();
-      v_landed();
-      // ---- O^T += V^T P^T, the V^T fragments taken in PORTIONS portions ----
-#pragma unroll
-      for (int pt = 0; pt < PORTIONS; ++pt) {
-        uintx4 vfr[4][DBP];
-        read_v(pt, vfr);
-        if (pt == PORTIONS - 1) v_free();
-        second(pt, vfr);
-      }
-    }
-    if (has1) {
-      wait_vm<VOPS>();                              // this wavefront's half of K(t+1) has landed (V(t+1) may be in flight)
-      __syncthreads();                              // ... and the other half
+      second(vfr);
     }
     cx = cxn;
   }
