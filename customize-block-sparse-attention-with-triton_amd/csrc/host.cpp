@@ -9,6 +9,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 #include <dlfcn.h>
+#include <algorithm>
+#include <climits>
 #include <list>
 #include <mutex>
 #include "bsattn.h"
@@ -35,6 +37,8 @@ struct Library {
   decltype(&::bsattn_fwd_mask_copy_tokens) fwd_mask = nullptr;
   decltype(&::bsattn_bwd_workspace) bwd_workspace = nullptr;
   decltype(&::bsattn_bwd_tokens) bwd = nullptr;
+  decltype(&::bsattn_reorder_inplace_workspace) reorder_workspace = nullptr;
+  decltype(&::bsattn_reorder_inplace) reorder = nullptr;
 } lib;
 
 void bind(const std::string& path) {
@@ -56,6 +60,8 @@ void bind(const std::string& path) {
   get(lib.fwd_mask, "bsattn_fwd_mask_copy_tokens");
   get(lib.bwd_workspace, "bsattn_bwd_workspace");
   get(lib.bwd, "bsattn_bwd_tokens");
+  get(lib.reorder_workspace, "bsattn_reorder_inplace_workspace");
+  get(lib.reorder, "bsattn_reorder_inplace");
 }
 
 void check(int rc, const char* what) {
@@ -455,6 +461,75 @@ py::tuple forward_backward(const Tensor& q_, const Tensor& k_, const Tensor& v_,
   return py::make_tuple(unpadded(o, D), lse, unpadded(dq, D), unpadded(dk, D), unpadded(dv, D));
 }
 
+// ---- token reorder in place ----
+// Dimensions (stride, size) around stretches of `need` elements of which no two share an element.
+bool nested(std::vector<std::pair<int64_t, int64_t>> dims, int64_t need) {
+  std::sort(dims.begin(), dims.end());
+  for (const auto& [stride, size] : dims)
+    if (size > 1) {
+      if (stride < need) return false;
+      need += stride * (size - 1);
+    }
+  return true;
+}
+
+// The image tokens (behind n_text others) of every tensor moved where they are, head by head, by the permutation numbers [heads].
+// Returns the library's code, or none where it does not take the call: numbers that are not a tensor it can read, layouts, tensors
+// that autograd watches, sizes that do not fit (functional.py moves those out of place, or says what is wrong).  (In Python the views,
+// checks and marshalling took 15 us a call, two calls a layer: 23 heads of 2 807 tokens 33 us a pass, 19 here; 5 heads of 906 33 and 10.)
+std::optional<int> reorder_inplace(const std::vector<Tensor>& tensors, const Tensor& numbers, bool inverse, int64_t F, int64_t H, int64_t W,
+                                   int64_t n_text) {
+  constexpr size_t MOST = 4;
+  if (tensors.empty() || tensors.size() > MOST) return std::nullopt;
+  const Tensor& x = tensors[0];
+  if (!x.is_cuda() || x.dim() != 4 || F < 1 || H < 1 || W < 1 || F > INT_MAX || H > INT_MAX || W > INT_MAX) return std::nullopt;
+  const int64_t BS = x.size(0), NH = x.size(1), T = x.size(2) - n_text, D = x.size(3), e = x.element_size();
+  if (n_text < 0 || T < 1 || T > INT_MAX || F * H > T || F * H * W != T || BS < 1 || NH < 1 || D < 1) return std::nullopt;
+  if (!numbers.is_cuda() || numbers.device() != x.device() || (numbers.scalar_type() != at::kLong && numbers.scalar_type() != at::kInt) ||
+      numbers.dim() != 1 || numbers.size(0) != NH || !numbers.is_contiguous()) return std::nullopt;
+  const bool grad = at::GradMode::is_enabled();
+  std::vector<std::pair<int64_t, int64_t>> dims[MOST];
+  void* ptrs[MOST];
+  int64_t strides[3 * MOST];
+  for (size_t i = 0; i < tensors.size(); ++i) {
+    const Tensor& t = tensors[i];
+    if (!t.is_cuda() || t.device() != x.device() || t.sizes() != x.sizes() || t.scalar_type() != x.scalar_type() || (grad && t.requires_grad()) ||
+        t.stride(3) != 1) return std::nullopt;
+    ptrs[i] = (char*)t.data_ptr() + n_text * t.stride(2) * e;
+    if (((uintptr_t)ptrs[i] & 15) != 0) return std::nullopt;
+    for (int d = 0; d < 3; ++d) {
+      if (((t.stride(d) * e) & 15) != 0) return std::nullopt;
+      strides[3 * i + d] = t.stride(d);
+      dims[i].emplace_back(t.stride(d), d == 2 ? T : t.size(d));
+    }
+    if (!nested(dims[i], D)) return std::nullopt;
+    // no row shares memory with another tensor's (those cut from one storage: the q, k, v of a packed projection)
+    for (size_t j = 0; j < i; ++j) {
+      if (tensors[j].storage().data() != t.storage().data()) continue;
+      const int64_t apart = std::abs(t.storage_offset() - tensors[j].storage_offset());
+      auto both = dims[i];
+      both.emplace_back(apart, 2);
+      if (t.strides() != tensors[j].strides() || apart == 0 || !nested(both, D)) return std::nullopt;
+    }
+  }
+  const int n = (int)tensors.size();
+  size_t bytes = 0;
+  c10::DeviceGuard guard(x.device());
+  if (BS > INT_MAX || NH > INT_MAX || D > INT_MAX || lib.reorder_workspace(n, (int)BS, (int)NH, (int)F, (int)H, (int)W, (int)D, (int)e, &bytes) != 0) return std::nullopt;
+  const hipStream_t stream = stream_of(x);
+  Tensor ws;
+  {
+    const WorkspaceLock lock;
+    ws = workspace_locked(bytes, x.device(), stream, Use::reorder);
+  }
+  const int rc = lib.reorder(ptrs, strides, n, (int)BS, (int)NH, (int)F, (int)H, (int)W, (int)D, (int)e, numbers.const_data_ptr(),
+                             (int)numbers.element_size(), inverse ? 1 : 0, ws.data_ptr(), bytes, stream);
+  if (rc == 0)
+    for (const Tensor& t : tensors)
+      if (!t.is_inference()) t.unsafeGetTensorImpl()->bump_version();
+  return rc;
+}
+
 std::optional<Tensor> defined_or_none(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 }  // namespace
@@ -468,6 +543,7 @@ PYBIND11_MODULE(_host, m) {
     // (a view: the kept tensor itself never has a Python object, so it can be dropped without the GIL)
     return workspace_locked(bytes, like.device(), stream_of(like), Use::reorder).view({-1});
   });
+  m.def("reorder_inplace", &reorder_inplace);
   m.def("block_mask_to_lists", &block_mask_to_lists);
   m.def("forward", &forward);
   m.def("forward_block_mask", &forward_block_mask);

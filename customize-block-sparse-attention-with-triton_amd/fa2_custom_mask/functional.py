@@ -68,6 +68,11 @@ def _check_numbers(idx):
 def _reorder_image_tokens(tensors, idx, inverse, F, H, W, n_text_tokens):
     """Reorders (inverse: brings back) the image tokens of every tensor where they are, head by head, by the
     permutation numbers idx [heads]."""
+    if isinstance(idx, torch.Tensor) and idx.is_cuda and all(type(t) is torch.Tensor for t in tensors):
+        rc = _host.reorder_inplace(tensors, idx, inverse, F, H, W, n_text_tokens)
+        if rc is not None:
+            _ext.check(rc, "bsattn_reorder_inplace")
+            return
     _check_numbers(idx)
     x = tensors[0]
     image = [t[:, :, n_text_tokens:, :] for t in tensors]                     # functional.py:31-33, 81

@@ -126,3 +126,51 @@ def test_number_outside_the_table(dev, bad, number_type):
     assert torch.equal(xd.cpu(), x)                          # nothing was enqueued
     fm.permute_qkv_triton(xd, xd.clone(), xd.clone(), good, 0, **size)
     assert torch.equal(xd.cpu(), moved.cpu())
+
+
+FORMS = ["plain", "text of an odd width", "packed", "overlapping", "expanded heads", "requires grad", "other dtype", "numbers on the host", "strided numbers"]
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_native_call_takes_what_python_takes(dev, form):
+    """The native path and the general one agree on which layouts are moved in place, and on the result."""
+    import fa2_custom_mask as fm
+    from fa2_custom_mask import functional
+    from fa2_custom_mask.utils import _host
+    F, H, W, NH = 3, 5, 7, 4
+    D, text = (12, 1) if form == "text of an odd width" else (64, 2)
+    T = text + F * H * W
+    g = torch.Generator().manual_seed(17)
+    make = lambda *shape: torch.randn(*shape, generator=g).half().to(dev)
+    tensors = [make(1, NH, T, D) for _ in range(3)]
+    numbers = torch.tensor([3, 1, 5, 2], device=dev)
+    if form == "packed":
+        tensors = list(make(1, T, 3, NH, D).permute(2, 0, 3, 1, 4).unbind(0))
+    elif form == "overlapping":
+        base = make(1, NH, T + 1, D)
+        tensors = [base[:, :, :T], base[:, :, 1:], tensors[2]]
+    elif form == "expanded heads":
+        tensors[1] = make(1, 1, T, D).expand(1, NH, T, D)
+    elif form == "requires grad":
+        tensors[2].requires_grad_(True)
+    elif form == "other dtype":
+        tensors[1] = tensors[1].float()
+    elif form == "numbers on the host":
+        numbers = numbers.cpu()
+    elif form == "strided numbers":
+        numbers = torch.stack([numbers, numbers], 1)[:, 0]
+    with torch.no_grad():
+        want = [t.clone() for t in tensors]
+    image = [t[:, :, text:] for t in tensors]
+    size = dict(F=F, H=H, W=W, n_text_tokens=text)
+    takes = functional._inplace_workspace(tensors, image, F, H, W) is not None and numbers.is_cuda and numbers.is_contiguous()
+    assert takes == (form in ("plain", "packed"))
+    versions = [t._version for t in tensors]
+    rc = _host.reorder_inplace(tensors, numbers, False, F, H, W, text)
+    assert (rc is not None) == takes and (rc in (None, 0))
+    assert [t._version > v for t, v in zip(tensors, versions)] == [takes] * 3      # (views of one tensor count together)
+    if takes:
+        fm.permute_qkv_triton(*want, {"permute": [numbers.tolist()]}, 0, **size)      # (numbers the host holds: the general path)
+        assert all(torch.equal(a, b) for a, b in zip(tensors, want))
+    else:
+        assert all(torch.equal(a, b) for a, b in zip(tensors, want))                     # nothing was moved
