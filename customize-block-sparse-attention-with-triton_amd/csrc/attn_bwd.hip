@@ -183,8 +183,9 @@ __global__ __launch_bounds__(128, D == 256 ? 1 : 2) void dq_kernel(const BwdPara
           vt + C::TILE_BYTES + C::STAT_BYTES + (32 * wv + ln) * 8);
       if constexpr (KB == 1) mw >>= 32 * (u % STEPS);
       mw >>= 4 * g;
-      if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw);
-      else mask_scores(sacc[0], (unsigned)mw);
+      if constexpr (KB == 2) mask_partly(sacc[0], sacc[1], mw);
+      else if constexpr (D == 256) mask_scores(sacc[0], (unsigned)mw);
+      else mask_partly(sacc[0], (unsigned)mw);
     }
     if (tail_step) {
       const unsigned long long mw = tail_word(valid, g);
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(128, 2) void dkdv_kernel(const BwdParams prm) {
     if constexpr (EW) {
       unsigned long long mw = *reinterpret_cast<const unsigned long long*>(
           gt + C::TILE_BYTES + C::STAT_BYTES + (32 * wv + ln) * 8);
-      mask_scores(sacc, (unsigned)(mw >> (qoff + 4 * g)));
+      mask_partly(sacc, (unsigned)(mw >> (qoff + 4 * g)));
     }
     if (tail_step) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> qoff));
     // dO^T and Q^T fragments of the second products, read under the exponentials below
@@ -660,7 +661,8 @@ __global__ __launch_bounds__(256 * G, D == 128 ? 2 : 1) void dkdv4_kernel(const 
         dpacc = mfma_qk<BF16>(dlt_slice, ones_frag, dpacc);
       }
     }
-    if constexpr (EW) mask_scores(sacc, mw);
+    if constexpr (EW && D == 256) mask_scores(sacc, mw);
+    else if constexpr (EW) mask_partly(sacc, mw);
     if (tail_step) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> (32 * dh)));
     // (the fragments of the own block's second products are on their way while the vector ALU works)
     uintx4 fgt_own[2][DBW], fqt_own[2][DBW];

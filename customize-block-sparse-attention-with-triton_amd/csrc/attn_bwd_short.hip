@@ -167,8 +167,8 @@ __device__ __forceinline__ void short_dq(const BwdParams& prm, unsigned char* ld
       }
       if constexpr (EW) {
         const unsigned long long mw = *reinterpret_cast<const unsigned long long*>(kt + BITS_OFF + (32 * w + ln) * 8);
-        if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw >> (4 * g));
-        else mask_scores(sacc[0], (unsigned)(mw >> (32 * part + 4 * g)));
+        if constexpr (KB == 2) mask_partly(sacc[0], sacc[1], mw >> (4 * g));
+        else mask_scores(sacc[0], (unsigned)(mw >> (32 * part + 4 * g)));      // (D = 128: with the test 20 to 52 bytes per lane spilled)
       } else if (TAIL && cb == nb - 1) {
         const unsigned long long mw = tail_word(valid, g);
         if constexpr (KB == 2) mask_scores(sacc[0], sacc[1], mw);
@@ -322,7 +322,7 @@ __device__ __forceinline__ void short_dkdv(const BwdParams& prm, unsigned char* 
         if (g == 0) deltas[ln] = acc;
         __builtin_amdgcn_sched_barrier(0);
       }
-      if constexpr (EW) mask_scores(sacc, (unsigned)(*reinterpret_cast<const unsigned long long*>(qt + BITS_OFF + (32 * w + ln) * 8) >> (32 * half + 4 * g)));
+      if constexpr (EW) mask_partly(sacc, (unsigned)(*reinterpret_cast<const unsigned long long*>(qt + BITS_OFF + (32 * w + ln) * 8) >> (32 * half + 4 * g)));
       else if (TAIL && rb == nb - 1) mask_scores(sacc, (unsigned)(tail_word(valid, g) >> (32 * half)));
       uintx4 fgt[2][DB], fqt[2][DB];      // dO^T and Q^T fragments of the second products
 #pragma unroll
