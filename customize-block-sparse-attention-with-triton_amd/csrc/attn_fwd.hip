@@ -1515,8 +1515,8 @@ size_t fwd_workspace_bytes(int B, int H, int N, int D) { return coop_workspace_b
 
 void launch_fwd_pair(const FwdParams& prm, int dt, bool elementwise, hipStream_t st);   // attn_fwd_pair.hip
 void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st);   // attn_fwd_short.hip
-void launch_fwd_quad(const FwdParams& prm, int groups, int dt, bool elementwise, hipStream_t st);   // attn_fwd_quad.hip
-void launch_fwd_wide(const FwdParams& prm, int dt, bool elementwise, hipStream_t st);   // attn_fwd_wide.hip
+void launch_fwd_quad(const FwdShareParams& prm, int groups, int dt, bool elementwise, hipStream_t st);   // attn_fwd_quad.hip
+void launch_fwd_wide(const FwdShareParams& prm, int dt, bool elementwise, hipStream_t st);   // attn_fwd_wide.hip
 template <int D, int DT, int MODE, bool EW, int LAYOUT, bool SPREAD>
 static void launch_fwd_s(const FwdRangeParams& prm, int grid, hipStream_t st) {
   using C = FwdCfg<D>;
@@ -1623,18 +1623,20 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   if (quads.groups > 0) {
     const int slots = compute_units() * (quads.groups == 1 ? 2 : 1), rows = heads * prm.nb, left = rows % slots;
     const size_t parts = (size_t)rows * quads.split * 64;
-    prm.split = quads.split;
-    prm.place = place_of_eight(heads, prm.nb, prm.split);
-    prm.load = (int)((int64_t)rows * 4096 / slots);
-    prm.tail_from = rows / slots * slots;
-    prm.tail_shares = left > 0 ? slots / left : 1;
-    prm.share_least = share_least(rows, s.D);
-    prm.part_o = (float*)ws + 64;
-    prm.part_ml = prm.part_o + parts * s.D;
-    prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
-    prm.epoch = next_epoch();
-    if (s.D == 128) launch_fwd_quad(prm, quads.groups, dt, tile_bits != nullptr, st);
-    else launch_fwd_wide(prm, dt, tile_bits != nullptr, st);
+    FwdShareParams shared;
+    static_cast<FwdParams&>(shared) = prm;
+    shared.split = quads.split;
+    shared.place = place_of_eight(heads, prm.nb, shared.split);
+    shared.load = (int)((int64_t)rows * 4096 / slots);
+    shared.tail_from = rows / slots * slots;
+    shared.tail_shares = left > 0 ? slots / left : 1;
+    shared.share_least = share_least(rows, s.D);
+    shared.part_o = (float*)ws + 64;
+    shared.part_ml = shared.part_o + parts * s.D;
+    shared.flags = (unsigned long long*)(shared.part_ml + parts * 2);
+    shared.epoch = next_epoch();
+    if (s.D == 128) launch_fwd_quad(shared, quads.groups, dt, tile_bits != nullptr, st);
+    else launch_fwd_wide(shared, dt, tile_bits != nullptr, st);
     return launch_status();
   }
   if (s.D != 64 || plan.pairs > 0) {

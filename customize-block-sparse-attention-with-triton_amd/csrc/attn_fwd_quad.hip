@@ -43,7 +43,7 @@ template <int D, int S, bool EW> struct QuadCfg {
 // TAIL: N is not a multiple of 64 (as in attn_fwd.hip: the copy of the last tile repeats its last key, the scores beyond
 // it are -inf, the queries beyond N are not written; a half without any key leaves the tile out).
 template <int D, int S, int DT, bool EW, bool TAIL>
-__global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdParams prm) {
+__global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdShareParams prm) {
   using C = QuadCfg<D, S, EW>;
   constexpr int KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
   constexpr int COPIES = CPR / 4;                 // copy instructions per wavefront and tile
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdParams pr
 }
 
 template <int D, int S, int DT, bool EW, bool TAIL>
-static void launch_quad_t(const FwdParams& prm, hipStream_t st) {
+static void launch_quad_t(const FwdShareParams& prm, hipStream_t st) {
   constexpr int LDS = QuadCfg<D, S, EW>::LDS_BYTES;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
@@ -395,21 +395,21 @@ static void launch_quad_t(const FwdParams& prm, hipStream_t st) {
 }
 
 template <int D, int S, int DT>
-static void launch_quad_d(const FwdParams& prm, bool elementwise, hipStream_t st) {
+static void launch_quad_d(const FwdShareParams& prm, bool elementwise, hipStream_t st) {
   const bool tail = prm.N % 64 != 0;
   if (!elementwise) { if (tail) launch_quad_t<D, S, DT, false, true>(prm, st); else launch_quad_t<D, S, DT, false, false>(prm, st); }
   else { if (tail) launch_quad_t<D, S, DT, true, true>(prm, st); else launch_quad_t<D, S, DT, true, false>(prm, st); }
 }
 
 template <int D, int S>
-static void launch_quad_s(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
+static void launch_quad_s(const FwdShareParams& prm, int dt, bool elementwise, hipStream_t st) {
   if (dt == 0) launch_quad_d<D, S, 0>(prm, elementwise, st);
   else if (dt == 1) launch_quad_d<D, S, 1>(prm, elementwise, st);
   else launch_quad_d<D, S, 2>(prm, elementwise, st);
 }
 
 // D = 128.  groups: of four wavefronts per workgroup.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
-void launch_fwd_quad(const FwdParams& prm, int groups, int dt, bool elementwise, hipStream_t st) {
+void launch_fwd_quad(const FwdShareParams& prm, int groups, int dt, bool elementwise, hipStream_t st) {
   if (groups == 1) launch_quad_s<128, 1>(prm, dt, elementwise, st);
   else launch_quad_s<128, 2>(prm, dt, elementwise, st);
 }

@@ -39,7 +39,7 @@ static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the res
 // any key leaves the tile out), the queries beyond N are not written.
 // EW: elementwise masks (bit 30 of a staged column says "partly set", the tile's 64 row words travel with K).
 template <int DT, bool CONTIG, bool TAIL, bool EW>
-__global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
+__global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams prm) {
   constexpr int D = WIDE_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
   constexpr int COPIES = CPR / 4;                // copy instructions per wavefront and tile
   constexpr bool BF16 = DT != 0, PB = DT == 2, FOLD = !BF16;
@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdParams prm) {
 }
 
 template <int DT, bool CONTIG, bool TAIL, bool EW>
-static void launch_wide_c(const FwdParams& prm, hipStream_t st) {
+static void launch_wide_c(const FwdShareParams& prm, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL, EW>), hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -421,7 +421,7 @@ static void launch_wide_c(const FwdParams& prm, hipStream_t st) {
 }
 
 template <int DT, bool EW>
-static void launch_wide_t(const FwdParams& prm, hipStream_t st) {
+static void launch_wide_t(const FwdShareParams& prm, hipStream_t st) {
   const bool contig = prm.ks[2] == WIDE_D && prm.vs[2] == WIDE_D;
   if (prm.N % 64 != 0) { if (contig) launch_wide_c<DT, true, true, EW>(prm, st); else launch_wide_c<DT, false, true, EW>(prm, st); }
   else { if (contig) launch_wide_c<DT, true, false, EW>(prm, st); else launch_wide_c<DT, false, false, EW>(prm, st); }
@@ -429,13 +429,13 @@ static void launch_wide_t(const FwdParams& prm, hipStream_t st) {
 
 // dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
 template <bool EW>
-static void launch_wide_e(const FwdParams& prm, int dt, hipStream_t st) {
+static void launch_wide_e(const FwdShareParams& prm, int dt, hipStream_t st) {
   if (dt == 0) launch_wide_t<0, EW>(prm, st);
   else if (dt == 1) launch_wide_t<1, EW>(prm, st);
   else launch_wide_t<2, EW>(prm, st);
 }
 
-void launch_fwd_wide(const FwdParams& prm, int dt, bool elementwise, hipStream_t st) {
+void launch_fwd_wide(const FwdShareParams& prm, int dt, bool elementwise, hipStream_t st) {
   if (elementwise) launch_wide_e<true>(prm, dt, st);
   else launch_wide_e<false>(prm, dt, st);
 }

@@ -25,7 +25,6 @@ struct FwdParams {
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair kernel: workgroups per row block (1: results written directly)
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
-  int tail_from, tail_shares, load, share_least;      // quad and wide kernel: see quad_shares
   int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
@@ -37,6 +36,9 @@ struct FwdParams {
   PlaceOfEight place;              // kernels whose workgroups have a row block each
   Divisor per_batch;               // H
 };
+
+// fwd_quad_kernel's and fwd_wide_kernel's: what quad_shares asks for
+struct FwdShareParams : FwdParams { int tail_from, tail_shares, load, share_least; };
 
 // fwd_kernel's
 struct FwdRangeParams : FwdParams {
@@ -133,7 +135,7 @@ __device__ __forceinline__ int length_of_rows(const FwdParams& prm, int b, int h
 }
 
 // Shares of the list of len tiles of the row block of workgroup `linear` (of the workgroups that come first on their lists).
-__device__ __forceinline__ int shares_of_list(const FwdParams& prm, cint_ptr_t rp, int b, int h, int len, int linear, bool listed, int lane) {
+__device__ __forceinline__ int shares_of_list(const FwdShareParams& prm, cint_ptr_t rp, int b, int h, int len, int linear, bool listed, int lane) {
   if (len < 2 * prm.share_least) return 1;
   const bool last_round = linear >= prm.tail_from;
   int mid = 0, end = 0;
