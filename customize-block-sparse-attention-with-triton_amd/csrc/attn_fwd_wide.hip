@@ -15,8 +15,7 @@
 // 131 -> 117, dense block-causal fp16 189 -> 168 (831 TFLOP/s); 16 heads N = 8192 keep 0.3 472 -> 409 (806 TFLOP/s).  Ragged: 16 heads
 // N = 4000 causal keep 0.5 bf16 168 -> 95 (fwd_pair_kernel spilled), 10 heads N = 4090 keep 0.3 142 -> 93, fp16 N = 4065 dense
 // block-causal 214 -> 170.  Elementwise masks: 16 heads N = 4000 token window of 1000 127 -> 81, token-causal 215 -> 143, fp16 N = 4096 101 -> 86
-// and 180 -> 156.  A few variants keep values in scratch memory: fp16 with strided rows 20 to 36 bytes per lane, fp16 elementwise with
-// contiguous rows 8 or 12, bf16 with P in either type, whole tiles and contiguous rows 12 (outside the walk).
+// and 180 -> 156.  Two variants, fp16 elementwise with strided rows, keep 12 bytes per lane in scratch memory.
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196 of the reference).
 #include "common.h"
@@ -312,12 +311,16 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
 
   // ---- the key halves meet: each hands over the columns the other finishes ----
   // (after the last tile's barriers nobody reads a tile or a column any more: all of the LDS is free)
+  // (the lane index as a value the compiler cannot trace back: addresses would otherwise be made before the walk and held)
+  int lane_e = lane;
+  asm volatile("" : "+v"(lane_e));
+  const int ln_e = lane_e & 31, g_e = lane_e >> 5;
   const float lsum = l_i + __shfl_xor(l_i, 32);
   const float m_own = lsum != 0.f ? m_i : -INFINITY;       // (a sum that is not a number stays in)
   float* ml = reinterpret_cast<float*>(lds + WIDE_COLS_OFF);    // (m, l) per half and query
-  if (g == 0) { ml[(64 * kh + 32 * w + ln) * 2] = m_own; ml[(64 * kh + 32 * w + ln) * 2 + 1] = lsum; }
-  floatx4* give = reinterpret_cast<floatx4*>(lds) + (2 * (1 - kh) + w) * (DB / 2) * 4 * 64 + lane;
-  const floatx4* take = reinterpret_cast<const floatx4*>(lds) + (2 * kh + w) * (DB / 2) * 4 * 64 + lane;
+  if (g_e == 0) { ml[(64 * kh + 32 * w + ln_e) * 2] = m_own; ml[(64 * kh + 32 * w + ln_e) * 2 + 1] = lsum; }
+  floatx4* give = reinterpret_cast<floatx4*>(lds) + (2 * (1 - kh) + w) * (DB / 2) * 4 * 64 + lane_e;
+  const floatx4* take = reinterpret_cast<const floatx4*>(lds) + (2 * kh + w) * (DB / 2) * 4 * 64 + lane_e;
   floatx16 res[DB / 2];
 #pragma unroll
   for (int db = 0; db < DB / 2; ++db) {
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
   unsigned long long seen = 0ull;      // (the read travels beside the merge)
   if (shares > 1 && threadIdx.x == 0) seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
-  const int other = (64 * (1 - kh) + 32 * w + ln) * 2;
+  const int other = (64 * (1 - kh) + 32 * w + ln_e) * 2;
   const float m_oth = ml[other], l_oth = ml[other + 1];
   float M = fmaxf(m_own, m_oth);
   const float wo = m_own == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_own - M);
@@ -354,14 +357,14 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
     // the shares of a list meet in the workspace, as the parts of a row block do in attn_fwd.hip: each is published with device-scope
     // stores and counted in once these are acknowledged, the last one in adds all of them up in their order
     const int64_t first_slot = ((int64_t)bh * nb + m) * prm.split;
-    auto slot_of = [&](int p) { return prm.part_o + (first_slot + p) * (64 * D) + wave * (64 * 64) + lane * 4; };      // [wavefront][quad][lane][4]
-    auto ml_of = [&](int p) { return prm.part_ml + (first_slot + p) * 128 + 2 * (32 * w + ln); };
+    auto slot_of = [&](int p) { return prm.part_o + (first_slot + p) * (64 * D) + wave * (64 * 64) + lane_e * 4; };      // [wavefront][quad][lane][4]
+    auto ml_of = [&](int p) { return prm.part_ml + (first_slot + p) * 128 + 2 * (32 * w + ln_e); };
 #pragma unroll
     for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
       for (int i4 = 0; i4 < 4; ++i4)
         coherent_store4(slot_of(chunk) + (4 * db + i4) * 256, res[db][4 * i4], res[db][4 * i4 + 1], res[db][4 * i4 + 2], res[db][4 * i4 + 3]);
-    if (kh == 0 && g == 0) { coherent_store(ml_of(chunk), M); coherent_store(ml_of(chunk) + 1, L); }
+    if (kh == 0 && g_e == 0) { coherent_store(ml_of(chunk), M); coherent_store(ml_of(chunk) + 1, L); }
     wait_vm<0>();
     __syncthreads();
     if (threadIdx.x == 0) lcols[0] = count_in(arrivals, prm.epoch, seen);
@@ -405,8 +408,8 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
   const float inv = row_inverse<EW>(L);
   __syncthreads();           // all have taken what was handed over: the LDS is free for the result rows
   rows_out<BF16, D / 2>(lds + wave * rows_out_bytes(D / 2, true), obase, ((int64_t)m * 64 + 32 * w) * prm.os[2] + 128 * kh, prm.os[2],
-                        prm.out_f32, lane, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });
-  if (prm.lse != nullptr && kh == 0 && g == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(M, L);
+                        prm.out_f32, lane_e, TAIL ? prm.N - (m * 64 + 32 * w) : 32, [&](int db, int i) { return res[db][i] * inv; });
+  if (prm.lse != nullptr && kh == 0 && g_e == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(M, L);
 }
 
 template <int DT, bool CONTIG, bool TAIL, bool EW>
