@@ -73,8 +73,14 @@ def test_replay_d128_bf16_many_heads(dev):
 
 
 def test_replay_d256_lists_shared(dev):
-    """Head dimension 256 with few row blocks: forward and backward parts summed by second kernels."""
+    """Head dimension 256 with few row blocks: the forward's shares summed by the last one in, the backward's parts by a second kernel."""
     replay_and_compare(dev, 1, 2, 2048, 256, torch.float16, uniform_block_mask(1, 2, 32, 0.5, 3005), 3006, replays=3)
+
+
+@pytest.mark.parametrize("H,N", [(1, 2048), (3, 5120)])
+def test_replay_d128_lists_shared(dev, H, N):
+    """Head dimension 128 with few row blocks: up to four shares of every list, two of the long ones."""
+    replay_and_compare(dev, 1, H, N, 128, torch.bfloat16, causal_block_mask(1, 1, N // 64, 1.0, 3007), 3008, replays=3)
 
 
 def test_replay_elementwise_mask_ragged_length(dev):
