@@ -1354,13 +1354,24 @@ static int pair_split_256(int64_t row_blocks, int nb) {
   return s < cap ? s : cap > 1 ? cap : 1;
 }
 
-// The same at D = 128, for what fwd_quad_kernel leaves of the launches that do not fill the GPU: long lists, of one or two heads.  us,
-// N(0,1) bf16, 1 / 2 / 3 / 4 / 6 shares; keep 0.3, dense:
-//    2 heads N = 12032 (376 row blocks)   92 /  71 /  83 /  78 /  83    240 / 176 / 223 / 195 / 197
+// The same at D = 128 with block masks.  A share costs the launch that sums the parts (3 us) and their traffic, so short
+// lists are shared only where few of them are in the launch.  us, N(0,1), 1 / 2 / 3 / 4 / 6 shares; keep 0.3, dense:
+//    1 head  N = 832              12 /  12 /  11 /  10 /  10     20 /  16 /  14 /  13 /  12
+//    5 heads N = 832              13 /  14 /  14 /  16 /  16     20 /  18 /  17 /  19 /  20
+//   11 heads N = 1344             17 /  23 /  24 /  26 /  30     30 /  31 /  31 /  31 /  37
+//    1 head  N = 2048             23 /  17 /  15 /  14 /  16     42 /  27 /  22 /  19 /  18
+//    4 heads N = 2048             24 /  22 /  23 /  24 /  25     43 /  32 /  31 /  31 /  32
+//    2 heads N = 4096             36 /  27 /  27 /  26 /  26     81 /  51 /  44 /  39 /  37
+//    1 head  N = 8192             67 /  42 /  35 /  32 /  32    157 /  88 /  69 /  58 /  54
+//    3 heads N = 8192             75 /  58 /  68 /  63 /  70    168 / 128 / 159 / 143 / 146
+//    2 heads N = 12032            92 /  71 /  83 /  78 /  83    240 / 176 / 223 / 195 / 197
 static int pair_split_128(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
-  if (nb < 150) return 1;
-  return rows >= 480 ? 1 : rows >= 320 ? 2 : rows >= 208 ? 3 : 4;
+  if (nb < 56 && rows > 6 * nb) return 1;
+  const int s = rows >= 480 ? 1 : rows >= 320 ? 2 : rows >= 208 ? 3 : 4;
+  // a share of a dense list keeps 8 tiles, 4 in a launch of few lists, 12 in one of many short ones
+  const int cap = rows <= 64 && nb >= 12 ? nb / 4 : rows > 96 && nb < 48 ? nb / 12 : nb / 8;
+  return s < cap ? s : cap > 1 ? cap : 1;
 }
 
 // Which launches fwd_quad_kernel (D = 128) takes: groups of four wavefronts per workgroup (0: none) and shares of a list, at most
@@ -1481,6 +1492,20 @@ static int share_least(int64_t row_blocks, int D) {
   const int64_t rows = row_blocks * 256 / compute_units();
   if (D == 128) return rows <= 64 ? 6 : 8;
   return rows <= 64 ? 4 : rows <= 256 ? 6 : 24;
+}
+
+// How exact a launch's rows are at least, in hundredths of a tile (FwdShareParams::exact): as in a launch of pairs of wavefronts
+// (D = 256 with block masks: key halves) that cuts every list into the parts below, whatever its length.  A part's first tile gives the
+// reference, so that its largest numerator is exact: of what rounding the numerators of a tile costs a row (their squares), that is
+// 38 % with 64 keys of N(0,1) scores, 48 % with 32.  (fp16 with block masks keeps the reference at 0: nothing is exact there.)
+// fp32 results of bf16 against 64 bits, without this rule / with it / such a launch: D = 256 2 heads N = 4096 block-causal 1.84e-4 / 1.49e-4 / 1.70e-4,
+// 5 heads N = 3648 block-causal keep 0.3 1.78e-4 / 1.48e-4 / 1.71e-4; D = 128 8 heads N = 4000 token window of 1000 1.73e-4 / 1.51e-4 / 1.71e-4.
+static int exact_tiles(int64_t row_blocks, int nb, int D, bool words, bool fp16) {
+  if (!words) return fp16 ? 0 : D == 256 ? 48 * pair_split_256(row_blocks, nb) : 38 * pair_split_128(row_blocks, nb);
+  if (D == 256) return 38 * pair_split_256(row_blocks, nb);
+  // about four workgroups per compute unit, at most 4 parts of a row unless it is long
+  const int64_t few = nb / 2 < 4 ? nb / 2 : 4, cap = nb / 16 > few ? nb / 16 : few, s = 4 * (int64_t)compute_units() / row_blocks;
+  return 38 * (int)std::clamp<int64_t>(std::min(s, cap), 1, 8);
 }
 
 // Launches whose workgroups have a row block each need no lists of a block mask: they take its columns from the mask (3 heads
@@ -1631,6 +1656,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     shared.tail_from = rows / slots * slots;
     shared.tail_shares = left > 0 ? slots / left : 1;
     shared.share_least = share_least(rows, s.D);
+    shared.exact = exact_tiles(rows, prm.nb, s.D, tile_bits != nullptr, dt == 0);
     shared.part_o = (float*)ws + 64;
     shared.part_ml = shared.part_o + parts * s.D;
     shared.flags = (unsigned long long*)(shared.part_ml + parts * 2);

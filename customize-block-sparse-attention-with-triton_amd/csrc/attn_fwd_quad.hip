@@ -182,7 +182,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
   float limit = FOLD ? SUM_LIMIT : 0.f;
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
 
-  const int steps = (t1 - t0 + S - 1) / S;
+  const int steps = (t1 - t0 + S - 1) / S, two_parts = first_tiles<FOLD>(prm.exact, S * shares);
   for (int it = 0; it < steps; ++it) {
     wait_vm<0>();
     __syncthreads();                              // the step's tiles are complete; everybody has left the step before
@@ -245,12 +245,22 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
       uintx4 pf[2];
       float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
       // (FOLD: the first tile keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD && fresh && !(lnew >= 0.25f);
-      if (__any(first || !(lnew - l_i < limit))) {
-        recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
-        any_m = 1;
-        lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-        limit = sum_limit<false>(lnew);
+      const bool first = FOLD && fresh && !(lnew >= 0.25f), parts = it < two_parts;
+      if (__any(parts || first || !(lnew - l_i < limit))) {
+        if (!FOLD || __any(first || !(lnew - l_i < limit))) {
+          recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
+          any_m = 1;
+          lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+          limit = sum_limit<false>(lnew);
+        }
+        if (parts) {
+          uintx4 rest[2];
+          lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
+#pragma unroll
+          for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) oacc[db][0] = mfma_qk<PB>(vfr[ts][db], rest[ts], oacc[db][0]);
+        }
       }
       l_i = lnew;
       fresh = false;

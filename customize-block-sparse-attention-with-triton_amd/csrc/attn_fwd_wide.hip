@@ -203,6 +203,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
   int any_m = 0;     // (wave-uniform) some lane's reference exponent is not zero: the extra contraction slice is needed
   __syncthreads();                                  // all of K(t0), V(t0) and the column list are in LDS
 
+  const int two_parts_to = t0 + first_tiles<FOLD>(prm.exact, shares);
   for (int t = t0; t < t1; ++t) {
     const bool has1 = t + 1 < t1;
     const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(t + 1)) : 0;
@@ -253,22 +254,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
 #pragma unroll
       for (int i = 0; i < 16; ++i) sc[i] = 8 * (i / 4) + (i % 4) + first_key < keys ? sc[i] : -INFINITY;
     }
-    if (TAIL && !EW && keys <= 0) {
-      pf[0] = pf[1] = uintx4{0u, 0u, 0u, 0u};
-    } else {
-      float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-      // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD && fresh && !(lnew >= 0.25f);
-      if (__any(first || !(lnew - l_i < limit))) {
-        recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
-        any_m = 1;
-        lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-        limit = sum_limit<false>(lnew);
-      }
-      l_i = lnew;
-      fresh = false;
-    }
-    // ---- O^T += V^T P^T, V^T fragments in portions of two column blocks ----
+    // V^T fragments, in portions of two column blocks
     uintx4 vfr[2][2][2];
     auto read_v = [&](int pt) {
 #pragma unroll
@@ -287,6 +273,44 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
           vfr[pt & 1][d][ts] = a;
         }
     };
+    auto second = [&](int pt, const uintx4 (&p)[2]) {
+#pragma unroll
+      for (int ts = 0; ts < 2; ++ts)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+          uintx4 a = vfr[pt & 1][d][ts];
+          if constexpr (BF16 && !PB) a = bf16x8_to_f16x8(a);
+          oacc[2 * pt + d][0] = mfma_qk<PB>(a, p[ts], oacc[2 * pt + d][0]);
+        }
+    };
+    if (TAIL && !EW && keys <= 0) {
+      pf[0] = pf[1] = uintx4{0u, 0u, 0u, 0u};
+    } else {
+      float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+      // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
+      const bool first = FOLD && fresh && !(lnew >= 0.25f), parts = t < two_parts_to;
+      if (__any(parts || first || !(lnew - l_i < limit))) {
+        if (!FOLD || __any(first || !(lnew - l_i < limit))) {
+          recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
+          any_m = 1;
+          lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+          limit = sum_limit<false>(lnew);
+        }
+        if (parts) {
+          uintx4 rest[2];
+          lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
+#pragma unroll
+          for (int pt = 0; pt < 4; ++pt) {
+            read_v(pt);
+            second(pt, rest);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+      l_i = lnew;
+      fresh = false;
+    }
+    // ---- O^T += V^T P^T ----
     read_v(0);
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) {
@@ -297,14 +321,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
         __syncthreads();                            // ... and the others'; all hold their V fragments: the V buffer is free
         if (has1) v_copy(cxn & COL_MASK);
       }
-#pragma unroll
-      for (int ts = 0; ts < 2; ++ts)
-#pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          uintx4 a = vfr[pt & 1][d][ts];
-          if constexpr (BF16 && !PB) a = bf16x8_to_f16x8(a);
-          oacc[2 * pt + d][0] = mfma_qk<PB>(a, pf[ts], oacc[2 * pt + d][0]);
-        }
+      second(pt, pf);
     }
     if constexpr (TAIL || EW) cx = cxn;
   }

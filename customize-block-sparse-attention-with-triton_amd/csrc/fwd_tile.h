@@ -37,8 +37,11 @@ struct FwdParams {
   Divisor per_batch;               // H
 };
 
-// fwd_quad_kernel's and fwd_wide_kernel's: what quad_shares asks for
-struct FwdShareParams : FwdParams { int tail_from, tail_shares, load, share_least; };
+// fwd_quad_kernel's and fwd_wide_kernel's: what quad_shares asks for, and
+struct FwdShareParams : FwdParams {
+  int tail_from, tail_shares, load, share_least;
+  int exact;      // hundredths of a tile whose numerators have no rounding error, of a row, at least
+};
 
 // fwd_kernel's
 struct FwdRangeParams : FwdParams {
@@ -86,6 +89,43 @@ __device__ __forceinline__ float softmax_block(const floatx16& s, float qk_scale
       const unsigned int hp = pack2<PB>(p0, p1);
       l = add_packed2<PB>(hp, l);
       pf[ts][jj] = hp;
+    }
+  }
+  return l;
+}
+
+// The same in two parts of 16 bits, pf and rest, which the second product takes one after the other: numerators to 22 bits (PB: 16).  For the
+// first block of a list: what the rounding of P costs a row falls by that block's share of it, more than half for the short lists that weigh
+// most in a result's norm.  pf is cut and not rounded and rest is never 0 where the numerator is not, so that a value of V
+// that is not finite counts with one sign in both.
+template <bool FOLD, bool PB>
+__device__ __forceinline__ float softmax_block_parts(floatx16& s, float qk_scale, float m, float l, uintx4 (&pf)[2], uintx4 (&rest)[2]) {
+  constexpr float LEAST = 0x1p-24f;       // smallest fp16
+  if constexpr (FOLD) asm volatile("" : "+v"(s));      // (or the exponentials of softmax_block in front of it are kept for here, in 16 registers)
+  else asm volatile("" : "+v"(m));
+#pragma unroll
+  for (int ts = 0; ts < 2; ++ts) {
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) {
+      const int i = 8 * ts + 2 * jj;
+      const float p0 = __builtin_amdgcn_exp2f(FOLD ? s[i] : __builtin_fmaf(s[i], qk_scale, -m));
+      const float p1 = __builtin_amdgcn_exp2f(FOLD ? s[i + 1] : __builtin_fmaf(s[i + 1], qk_scale, -m));
+      unsigned int hp;
+      float h0, h1;
+      if constexpr (PB) {
+        const unsigned int b0 = __builtin_bit_cast(unsigned int, p0), b1 = __builtin_bit_cast(unsigned int, p1) & 0xffff0000u;
+        hp = b1 | (b0 >> 16);
+        h0 = __builtin_bit_cast(float, b0 & 0xffff0000u);
+        h1 = __builtin_bit_cast(float, b1);
+      } else {
+        hp = __builtin_bit_cast(unsigned int, __builtin_amdgcn_cvt_pkrtz(p0, p1));
+        const half2v h = __builtin_bit_cast(half2v, hp);
+        h0 = (float)h[0]; h1 = (float)h[1];
+      }
+      const unsigned int lp = pack2<PB>(__builtin_amdgcn_fmed3f(p0 - h0, LEAST, p0), __builtin_amdgcn_fmed3f(p1 - h1, LEAST, p1));
+      l = add_packed2<PB>(lp, add_packed2<PB>(hp, l));
+      pf[ts][jj] = hp;
+      rest[ts][jj] = lp;
     }
   }
   return l;
@@ -146,6 +186,11 @@ __device__ __forceinline__ int shares_of_list(const FwdShareParams& prm, cint_pt
   }
   return quad_shares(len, mid, end, last_round ? prm.tail_shares : 1, prm.load, prm.split, prm.share_least);
 }
+
+// Tiles at the front of a walk whose numerators are kept in two parts (softmax_block_parts), for a list that `walks` of them take on: without
+// any the largest numerator of a walk is exact, which counts 48 hundredths (FOLD: the reference stays at 0, and none is).
+template <bool FOLD>
+__device__ __forceinline__ int first_tiles(int exact, int walks) { return exact <= (FOLD ? 0 : 48) * walks ? 0 : exact <= 100 * walks ? 1 : 2; }
 
 // Counts a share of a list in, by one thread, when all accesses of its workgroup to its part have been acknowledged; returns how many
 // are in.  The counter holds (launch mark << 16 | shares counted); stale contents carry another mark.  seen: a first guess of it.

@@ -108,3 +108,31 @@ def test_scores_of_minus_infinity(dev, D, H, N, dtype, out_fp32, hidden):
         assert torch.equal(lse[0, h] == float("-inf"), none) and not bool(torch.isnan(lse[0, h]).any())
         assert float((o[0, h] - ref)[~none].abs().max()) <= MAXABS[dtype]
         assert float((lse[0, h] - ref_lse)[~none].abs().max()) <= (2e-3 if out_fp32 or dtype == torch.float16 else 2.0 ** -8)
+
+
+# A value of V that is not finite reaches the rows that keep its key, in its column, and no others: launches whose first tiles take
+# the numerators in two parts (D = 128: two groups of wavefronts, one; D = 256: whole lists, shared ones), and others.
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("dtype,out_fp32", [(torch.float16, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+@pytest.mark.parametrize("D,H,N", [(64, 2, 704), (128, 2, 1500), (128, 8, 2304), (128, 100, 700), (256, 2, 1000), (256, 1, 2048), (256, 100, 704)])
+def test_values_that_are_not_finite(dev, D, H, N, dtype, out_fp32, value):
+    import fa2_custom_mask as fm
+    q, k, v = [x.to(dev) for x in make_qkv(1, H, N, D, dtype, 970 + N + D)]
+    q = q * 0.25                                  # (no numerator of a kept key is rounded to 0)
+    nb = -(-N // 64)
+    tiles = torch.ones(nb, nb, dtype=torch.bool, device=dev).tril()
+    tiles[nb // 2, : nb // 2] = False             # a row block that keeps its own tile only
+    key = [3, N // 2, N - 2]
+    for i, x in enumerate(key):
+        v[0, 0, x, 5 + i] = value
+    o, _ = fm.flash_attention_custom_mask_lse(q, k, v, tiles[None, None], D ** -0.5, out_fp32=out_fp32)
+    keep = tiles.repeat_interleave(64, 0).repeat_interleave(64, 1)[:N, :N]
+    s = (q[0, 0].double() @ k[0, 0].double().T * D ** -0.5).masked_fill(~keep, float("-inf"))
+    ref = torch.softmax(s, -1) @ torch.nan_to_num(v[0, 0].double(), nan=0.0, posinf=0.0, neginf=0.0)
+    want = torch.zeros_like(ref, dtype=torch.bool)
+    for i, x in enumerate(key):
+        want[:, 5 + i] = keep[:, x]
+    got = o[0, 0].double()
+    assert bool(torch.isfinite(got)[~want].all()) and float((got - ref)[~want].abs().max()) <= MAXABS[dtype]
+    assert bool((torch.isnan(got[want]) if value != value else got[want] == value).all())
+    assert bool(torch.isfinite(o[:, 1:]).all())
