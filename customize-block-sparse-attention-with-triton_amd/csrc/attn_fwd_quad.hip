@@ -243,15 +243,21 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
         }
       }
       uintx4 pf[2];
-      float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-      // (FOLD: the first tile keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD && fresh && !(lnew >= 0.25f), parts = it < two_parts;
-      if (__any(parts || first || !(lnew - l_i < limit))) {
-        if (!FOLD || __any(first || !(lnew - l_i < limit))) {
+      float lnew = 0.f;
+      // A tile calls for a new reference: the first one (FOLD: it keeps 0 when its sums are of moderate size, else it is known beforehand and saves
+      // a softmax), and where numerators grow too large.  (With a softmax in front of every reference and of every tile in two parts, us:
+      // 1 head N = 1024 keep 0.1 11.4, so 11.0; 3 heads N = 3000 keep 0.1 15.5, 14.8; D = 256 1 head N = 1024 keep 0.1 14.5, 13.7.)
+      const bool parts = it < two_parts;
+      bool far = !FOLD && fresh;
+      if (!far) {
+        lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+        far = __any((FOLD && fresh && !(lnew >= 0.25f)) || !(lnew - l_i < limit));
+      }
+      if (far || parts) {
+        if (far) {
           recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
           any_m = 1;
-          lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-          limit = sum_limit<false>(lnew);
+          if (!parts) lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
         }
         if (parts) {
           uintx4 rest[2];
@@ -261,6 +267,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
 #pragma unroll
             for (int db = 0; db < DB; ++db) oacc[db][0] = mfma_qk<PB>(vfr[ts][db], rest[ts], oacc[db][0]);
         }
+        if (far) limit = sum_limit<false>(lnew);
       }
       l_i = lnew;
       fresh = false;
@@ -298,7 +305,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
   __syncthreads();
   void* obase = out_base(prm, b, h);
   constexpr int QPR = D / 4, QT = 64 * QPR / (256 * S);      // quads per row, per thread
-  static_assert(64 * QPR % (256 * S) == 0 && QT % 4 == 0, "whole rounds of four");
+  static_assert(64 * QPR % (256 * S) == 0 && (QT == 4 || QT == 8), "the loads of a part go out together");
   auto put = [&](int r, int col, const floatx4& acc, float M, float L) {
     const int64_t q = (int64_t)m * 64 + r;
     if (TAIL && q >= prm.N) return;
@@ -370,8 +377,8 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
         mp[it] = coherent_load(slot_ml + 2 * r);
         lp[it] = coherent_load(slot_ml + 2 * r + 1);
       }
-#pragma unroll
-      for (int it = 0; it < QT; it += 4) coherent_load4x4(slot + it * 256, x[it], x[it + 1], x[it + 2], x[it + 3]);
+      if constexpr (QT == 8) coherent_load4x8(slot, x);
+      else coherent_load4x4(slot, x[0], x[1], x[2], x[3]);
     }
 #pragma unroll
     for (int it = 0; it < QT; ++it) {

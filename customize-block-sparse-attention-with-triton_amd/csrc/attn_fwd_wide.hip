@@ -8,7 +8,8 @@
 // frees the K buffer every wavefront waits for its part of V, in front of the one that frees V for its part of the next K.  (Four, with
 // waits of their own: 10 heads N = 4090 keep 0.3 95 -> 92 us, 2 heads N = 20800 dense 978 -> 947, 16 heads N = 8192 keep 0.3 378 -> 369.)  The two
 // key halves keep a reference exponent and a sum each and meet in LDS at the end, half of the columns each way.  Shares of a list
-// (quad_shares.h) meet in the workspace, in the same launch.
+// (quad_shares.h) meet in the workspace, in the same launch; the last one in asks for all 16 KB per wavefront of a part at once (four
+// round trips per part: 1 head N = 1024 dense 22.0 -> 20.0 us, N = 1536 24.6 -> 23.2).
 //
 // Before, fwd_pair_kernel: a wavefront with the scores of all 64 keys, up to 512 registers, alone on its SIMD, so that scores, softmax
 // and second product came one after the other.  us: 16 heads N = 4096 block-causal keep 0.5 bf16 108 -> 96, results in fp32
@@ -286,15 +287,20 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
     if (TAIL && !EW && keys <= 0) {
       pf[0] = pf[1] = uintx4{0u, 0u, 0u, 0u};
     } else {
-      float lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-      // (FOLD: the first tile of a row block keeps the reference at 0 when its sums are of moderate size)
-      const bool first = FOLD && fresh && !(lnew >= 0.25f), parts = t < two_parts_to;
-      if (__any(parts || first || !(lnew - l_i < limit))) {
-        if (!FOLD || __any(first || !(lnew - l_i < limit))) {
+      float lnew = 0.f;
+      // (which tiles call for a new reference: attn_fwd_quad.hip; elementwise masks take the softmax first, or 8 to 20 bytes more spill in five variants)
+      const bool parts = t < two_parts_to;
+      bool far = !FOLD && !EW && fresh;
+      if (!far) {
+        lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+        far = __any((FOLD && fresh && !(lnew >= 0.25f)) || !(lnew - l_i < limit));
+      }
+      if (far || parts) {
+        if (far) {
           recentre_block<DB, FOLD>(sc, oacc, qk_scale, m_i, l_i, mfrag, fresh, g);
           any_m = 1;
-          lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
-          limit = sum_limit<false>(lnew);
+          if (EW || !parts) lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
+          if (EW) limit = sum_limit<false>(lnew);
         }
         if (parts) {
           uintx4 rest[2];
@@ -306,6 +312,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
             __builtin_amdgcn_sched_barrier(0);
           }
         }
+        if (!EW && far) limit = sum_limit<false>(lnew);
       }
       l_i = lnew;
       fresh = false;
@@ -394,18 +401,18 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
       for (int i = 0; i < 16; ++i) acc[db][i] = 0.f;
     float Ms = -INFINITY, Ls = 0.f;
     for (int p = 0; p < shares; ++p) {
-      floatx4 x[DB / 2][4];
+      floatx4 x[16];
+      static_assert(DB / 2 * 4 == 16, "quads of a part per lane");
       float mp = M, lp = L;
       if (p == chunk) {
 #pragma unroll
         for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
-          for (int i4 = 0; i4 < 4; ++i4) x[db][i4] = {res[db][4 * i4], res[db][4 * i4 + 1], res[db][4 * i4 + 2], res[db][4 * i4 + 3]};
+          for (int i4 = 0; i4 < 4; ++i4) x[4 * db + i4] = {res[db][4 * i4], res[db][4 * i4 + 1], res[db][4 * i4 + 2], res[db][4 * i4 + 3]};
       } else {
         mp = coherent_load(ml_of(p));
         lp = coherent_load(ml_of(p) + 1);
-#pragma unroll
-        for (int db = 0; db < DB / 2; ++db) coherent_load4x4(slot_of(p) + db * 1024, x[db][0], x[db][1], x[db][2], x[db][3]);
+        coherent_load4x16(slot_of(p), x);
       }
       const float mn = fmaxf(Ms, mp);              // a side without mass has maximum -inf and weight 0
       const float ws = Ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(Ms - mn), wp = mp == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mp - mn);
@@ -414,7 +421,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
 #pragma unroll
       for (int db = 0; db < DB / 2; ++db)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[db][i] = acc[db][i] * ws + wp * x[db][i / 4][i % 4];
+        for (int i = 0; i < 16; ++i) acc[db][i] = acc[db][i] * ws + wp * x[4 * db + i / 4][i % 4];
     }
     // back to zero, so that a replay of this launch (same mark) starts from a clean counter
     if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

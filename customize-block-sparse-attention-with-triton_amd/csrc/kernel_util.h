@@ -231,6 +231,30 @@ __device__ __forceinline__ void coherent_load4x4(const float* p, floatx4& a, flo
                "s_waitcnt vmcnt(0)"
                : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d) : "v"(p) : "memory");
 }
+// Eight and sixteen of them: a round trip to memory that other XCDs have written takes longer than all of the loads.
+__device__ __forceinline__ void coherent_load4x8(const float* p, floatx4 (&x)[8]) {
+  asm volatile("global_load_dwordx4 %0, %8, off offset:-4096 sc1\n\tglobal_load_dwordx4 %1, %8, off offset:-3072 sc1\n\t"
+               "global_load_dwordx4 %2, %8, off offset:-2048 sc1\n\tglobal_load_dwordx4 %3, %8, off offset:-1024 sc1\n\t"
+               "global_load_dwordx4 %4, %8, off sc1\n\tglobal_load_dwordx4 %5, %8, off offset:1024 sc1\n\t"
+               "global_load_dwordx4 %6, %8, off offset:2048 sc1\n\tglobal_load_dwordx4 %7, %8, off offset:3072 sc1\n\t"
+               "s_waitcnt vmcnt(0)"
+               : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7])
+               : "v"(p + 1024) : "memory");
+}
+__device__ __forceinline__ void coherent_load4x16(const float* p, floatx4 (&x)[16]) {
+  asm volatile("global_load_dwordx4 %0, %16, off offset:-4096 sc1\n\tglobal_load_dwordx4 %1, %16, off offset:-3072 sc1\n\t"
+               "global_load_dwordx4 %2, %16, off offset:-2048 sc1\n\tglobal_load_dwordx4 %3, %16, off offset:-1024 sc1\n\t"
+               "global_load_dwordx4 %4, %16, off sc1\n\tglobal_load_dwordx4 %5, %16, off offset:1024 sc1\n\t"
+               "global_load_dwordx4 %6, %16, off offset:2048 sc1\n\tglobal_load_dwordx4 %7, %16, off offset:3072 sc1\n\t"
+               "global_load_dwordx4 %8, %17, off offset:-4096 sc1\n\tglobal_load_dwordx4 %9, %17, off offset:-3072 sc1\n\t"
+               "global_load_dwordx4 %10, %17, off offset:-2048 sc1\n\tglobal_load_dwordx4 %11, %17, off offset:-1024 sc1\n\t"
+               "global_load_dwordx4 %12, %17, off sc1\n\tglobal_load_dwordx4 %13, %17, off offset:1024 sc1\n\t"
+               "global_load_dwordx4 %14, %17, off offset:2048 sc1\n\tglobal_load_dwordx4 %15, %17, off offset:3072 sc1\n\t"
+               "s_waitcnt vmcnt(0)"
+               : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3]), "=&v"(x[4]), "=&v"(x[5]), "=&v"(x[6]), "=&v"(x[7]),
+                 "=&v"(x[8]), "=&v"(x[9]), "=&v"(x[10]), "=&v"(x[11]), "=&v"(x[12]), "=&v"(x[13]), "=&v"(x[14]), "=&v"(x[15])
+               : "v"(p + 1024), "v"(p + 3072) : "memory");
+}
 
 // Swizzle for tiles that are read both ways (operand reads of 32 consecutive rows and
 // transpose reads of 4 consecutive rows x 64 bytes): a bijection of the row bits that
