@@ -1354,8 +1354,9 @@ static int pair_split_256(int64_t row_blocks, int nb) {
   return s < cap ? s : cap > 1 ? cap : 1;
 }
 
-// The same at D = 128 with block masks.  A share costs the launch that sums the parts (3 us) and their traffic, so short
-// lists are shared only where few of them are in the launch.  us, N(0,1), 1 / 2 / 3 / 4 / 6 shares; keep 0.3, dense:
+// The same at D = 128, by fwd_pair_kernel: for what quad_plan leaves of the launches that do not fill the GPU, and for exact_tiles.  A share
+// costs the launch that sums the parts (3 us) and their traffic, so short lists are shared only where few of them are in the launch.
+// us, N(0,1), 1 / 2 / 3 / 4 / 6 shares; keep 0.3, dense:
 //    1 head  N = 832              12 /  12 /  11 /  10 /  10     20 /  16 /  14 /  13 /  12
 //    5 heads N = 832              13 /  14 /  14 /  16 /  16     20 /  18 /  17 /  19 /  20
 //   11 heads N = 1344             17 /  23 /  24 /  26 /  30     30 /  31 /  31 /  31 /  37
@@ -1401,23 +1402,43 @@ static int pair_split_128(int64_t row_blocks, int nb) {
 //    1 head  N = 17000 (266)           40/45/45/ - /37/37   68/65/66/ - /72/72  100/90/90/ - /122/121   191/176/134/ - /256/174
 //   10 heads N = 4000 (630)            25/36/36/ - /31/30   41/48/56/ - /41/45   66/63/72/ - /56/60  121/97/94/ - /80/81     (not there)
 //   16 heads N = 8000 (2000)           76/115/131/ - /88/88  145/184/202/ - /150/152  217/261/276/ - /217/219  274/345/362/ - /292/294   (nor there)
-struct QuadPlan { int groups, split; };
+// Up to 32 row blocks fwd_pair_kernel in four shares is up to 2.4 us faster, and up to 7 % further from 64 bits with fp32 results of
+// bf16 (1 head N = 768 keep 0.1 1.63e-4 against 1.54e-4, N = 1536 dense 2.02e-4 and 1.91e-4); with its first tiles in two parts (softmax_block_parts)
+// it takes 1.9 to 4 us more.  Pairs / so / this kernel; keep 0.1, 0.3, 1, block-causal:
+//    1 head  N = 768  (12)     11/12/11   12/14/12   13/16/15   13/16/15         1 head  N = 1536 (24)     12/13/12   14/16/16   17/21/18   16/20/18
+//    1 head  N = 1024 (16)     10/11/11   12/14/14   14/17/17   14/16/16         2 heads N = 1024 (32)     11/12/11   13/15/14   15/18/17   14/17/16
+// Whole lists of two groups leave the compute units idle that have none.  Where three shares of every list fit one round of single groups,
+// up to 168 row blocks (tail_of), long lists take those (from there on two shares of one head's leave up to a third of the places empty,
+// which pairs fill, up to 230 row blocks); a little more than one round of two groups goes to single groups, whose lists
+// are cut in three to fill the GPU.  Pairs / two groups / this; keep 0.1, 0.3, 1, block-causal:
+//    1 head  N = 8320 (130)    26/25/26  37/43/35   74/ 87/ 66   61/ 52/59       2 heads N = 5120 (160)    25/17/20  33/33/30   55/61/50   46/39/42
+//    1 head  N = 9600 (150)    28/26/26  41/48/37   82/ 98/ 75   67/ 57/62       3 heads N = 3392 (159)    23/15/17  28/25/26   43/42/38   37/32/33    (two groups)
+//    1 head  N = 10880 (170)   29/ - /28 46/ - /55  93/ - /120   77/ - /66       (pairs)
+// Pairs / single groups, whole or by a list's own length / this:
+//    3 heads N = 5632 (264)    29/24/26  41/46/47   79/101/ 88   64/ 60/56       3 heads N = 6400 (300)    31/29/28  48/58/50   93/114/103  73/65/64
+//    4 heads N = 4352 (272)    26/20/20  36/35/36   66/ 80/ 75   54/ 59/50       4 heads N = 4800 (300)    29/23/23  41/43/44   75/ 86/ 84  59/64/50
+//    words: 1 head N = 20000 (313), two groups in place of the whole single ones    57/65/55  94/113/97  134/135/139  236/216/186
+//    words: 1 head N = 17920 (280)                                                  43/56/43  74/ 87/77  108/102/117  178/180/143
+// From 480 row blocks on a round of single groups is full (one head N = 32000 (500) 105/ - /92  263/ - /218  665/ - /586  636/ - /375).
+struct QuadPlan { int groups, split, most; };      // most: shares of a list by its own length; split: that, or what fills the GPU
 static QuadPlan quad_plan(int64_t row_blocks, int nb, bool words) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
-  if (rows > 512) return {0, 1};
+  auto plan = [](int groups, int most, int fill = 1) { return QuadPlan{groups, std::max(most, fill), most}; };
+  if (rows > 512) return plan(0, 1);
   if (words) {
-    const int groups = rows <= 256 || nb >= 200 ? 2 : 1;
-    return {groups, nb < SHARE_MIN_BLOCKS ? 1 : rows <= 64 ? 4 : rows <= 128 || nb >= 28 ? 2 : 1};
+    if (rows > 256 && (rows > 272 || nb < 200)) return plan(1, nb >= 28 ? 2 : 1, nb >= 64 && rows <= 336 ? 3 : 1);
+    return plan(2, nb < 16 ? 1 : rows <= 64 ? 4 : rows <= 128 || nb >= 28 ? 2 : 1);
   }
   if (rows > 256) {
-    if (nb < 28 || nb >= 150) return {0, 1};
-    return {1, nb >= 80 ? 2 : 1};
+    if (nb < 28 || (nb >= 150 && rows < 480)) return plan(0, 1);
+    return plan(1, nb >= 80 ? 2 : 1, nb >= 64 && rows <= 336 ? 3 : 1);
   }
-  if (nb < 6 || (rows > 150 && rows <= 230 && nb >= 150)) return {0, 1};
-  if (rows <= 128) return {2, rows <= 64 && nb >= SHARE_MIN_BLOCKS ? 4 : nb >= 24 ? 2 : 1};
-  return {2, nb >= (rows <= 160 ? 40 : 80) ? 2 : 1};
+  if (nb < 6 || (rows > 168 && rows <= 230 && nb >= 150)) return plan(0, 1);
+  if (rows > 128 && rows <= 168 && nb >= 64) return plan(1, 3);
+  if (rows <= 128) return plan(2, rows <= 64 && nb >= 16 ? 4 : nb >= 24 ? 2 : 1);
+  return plan(2, nb >= (rows <= 160 ? 40 : 56) ? 2 : 1);
 }
-static_assert(SHARE_MIN_BLOCKS <= 24, "heads of launches that share lists have as many row blocks");
+static_assert(SHARE_MIN_BLOCKS <= 16, "heads of launches that share lists have as many row blocks");
 
 // the parts of shared lists and a counter per list
 static size_t quad_parts_bytes(int B, int H, int nb, int D, int split) {
@@ -1470,6 +1491,7 @@ static QuadPlan quad_plan(int B, int H, int nb, bool words, bool compact) {
   QuadPlan plan = quad_plan((int64_t)B * H * nb, nb, words);
   if (compact)
     while (plan.split > 1 && quad_parts_bytes(B, H, nb, 128, plan.split) > (size_t)BSATTN_STATIC_SCRATCH_BYTES) --plan.split;
+  plan.most = std::min(plan.most, plan.split);
   return plan;
 }
 
@@ -1643,18 +1665,21 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   // V, fa2_fwd.py:189) and V is used as it is; an fp32 result keeps P in fp16
   const int dt = s.dtype != BSATTN_BF16 ? 0 : (prm.out_f32 ? 1 : 2), heads = s.B * s.H;
   const ShortPlan plan = s.D == 64 ? short_plan((int64_t)heads * prm.nb, prm.nb) : ShortPlan{0, 1};
-  const QuadPlan quads = s.D == 128 ? quad_plan(s.B, s.H, prm.nb, tile_bits != nullptr, s.compact)
-                       : s.D == 256 ? QuadPlan{1, wide_split(s.B, s.H, s.N, s.compact)} : QuadPlan{0, 1};
+  const int wide = s.D == 256 ? wide_split(s.B, s.H, s.N, s.compact) : 1;
+  const QuadPlan quads = s.D == 128 ? quad_plan(s.B, s.H, prm.nb, tile_bits != nullptr, s.compact) : QuadPlan{s.D == 256 ? 1 : 0, wide, wide};
   if (quads.groups > 0) {
-    const int slots = compute_units() * (quads.groups == 1 ? 2 : 1), rows = heads * prm.nb, left = rows % slots;
+    const int slots = compute_units() * (quads.groups == 1 ? 2 : 1), rows = heads * prm.nb;
     const size_t parts = (size_t)rows * quads.split * 64;
     FwdShareParams shared;
     static_cast<FwdParams&>(shared) = prm;
     shared.split = quads.split;
     shared.place = place_of_eight(heads, prm.nb, shared.split);
     shared.load = (int)((int64_t)rows * 4096 / slots);
-    shared.tail_from = rows / slots * slots;
-    shared.tail_shares = left > 0 ? slots / left : 1;
+    shared.most = quads.most;
+    const TailShares tail = tail_of(rows, slots, shared.split);
+    shared.tail_from = tail.from;
+    shared.tail_shares = tail.shares;
+    shared.tail_len = tail.len;
     shared.share_least = share_least(rows, s.D);
     shared.exact = exact_tiles(rows, prm.nb, s.D, tile_bits != nullptr, dt == 0);
     shared.part_o = (float*)ws + 64;

@@ -39,7 +39,7 @@ struct FwdParams {
 
 // fwd_quad_kernel's and fwd_wide_kernel's: what quad_shares asks for, and
 struct FwdShareParams : FwdParams {
-  int tail_from, tail_shares, load, share_least;
+  int tail_from, tail_shares, tail_len, load, most, share_least;
   int exact;      // hundredths of a tile whose numerators have no rounding error, of a row, at least
 };
 
@@ -177,14 +177,14 @@ __device__ __forceinline__ int length_of_rows(const FwdParams& prm, int b, int h
 // Shares of the list of len tiles of the row block of workgroup `linear` (of the workgroups that come first on their lists).
 __device__ __forceinline__ int shares_of_list(const FwdShareParams& prm, cint_ptr_t rp, int b, int h, int len, int linear, bool listed, int lane) {
   if (len < 2 * prm.share_least) return 1;
-  const bool last_round = linear >= prm.tail_from;
+  const int tail = linear >= prm.tail_from && len >= prm.tail_len ? prm.tail_shares : 1;
   int mid = 0, end = 0;
-  if (!last_round || prm.tail_shares < prm.split) {
+  if (tail < prm.most) {
     const int nb = prm.nb;
     if (listed) { mid = rp[nb / 2 + SHARE_SAMPLE / 2] - rp[nb / 2 - SHARE_SAMPLE / 2]; end = rp[nb] - rp[nb - SHARE_SAMPLE]; }
     else { mid = length_of_rows(prm, b, h, nb / 2 - SHARE_SAMPLE / 2, lane); end = length_of_rows(prm, b, h, nb - SHARE_SAMPLE, lane); }
   }
-  return quad_shares(len, mid, end, last_round ? prm.tail_shares : 1, prm.load, prm.split, prm.share_least);
+  return quad_shares(len, mid, end, tail, prm.load, prm.most, prm.share_least);
 }
 
 // Tiles at the front of a walk whose numerators are kept in two parts (softmax_block_parts), for a list that `walks` of them take on: without
