@@ -1509,11 +1509,13 @@ static int wide_split(int B, int H, int N, bool compact) {
 //    D = 256   2 heads N = 1024, token-causal (32 row blocks)  20 / 21 / 26         1 head  N = 2048, keep 0.3 (32)  21 / 21 / 26
 //              2 heads N = 4096, keep 0.1 (128)                24 / 22 / 26         3 heads N = 4096, token-causal (192)  - / - / 50 (51, 69)
 //              8 heads N = 2048, token window of 512 (256)     25 / 21 / 22         5 heads N = 8192, keep 0.1 (640)  75 / 74 / 72 ( - , 66)
+//    D = 256, at least 3 / 4 (whole 18, 24, 24, 19, 20, 24, 25): 1 head N = 768, keep 0.3 (12) 17 / 18, dense 19 / 19,
+//              block-causal 18 / 20; 1 head N = 1024, keep 0.3 (16) 18 / 19, dense 20 / 20; 4 heads N = 768, block-causal (48) 19 / 20, dense 21 / 20
 //    D = 128   3 heads N = 1280, dense (60)                    26 / 17 / 17         2 heads N = 1024, token-causal (32)  14 / 14 / 16
 static int share_least(int64_t row_blocks, int D) {
   const int64_t rows = row_blocks * 256 / compute_units();
   if (D == 128) return rows <= 64 ? 6 : 8;
-  return rows <= 64 ? 4 : rows <= 256 ? 6 : 24;
+  return rows <= 64 ? 3 : rows <= 256 ? 6 : 24;
 }
 
 // How exact a launch's rows are at least, in hundredths of a tile (FwdShareParams::exact): as in a launch of pairs of wavefronts

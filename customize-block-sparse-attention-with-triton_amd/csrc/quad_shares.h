@@ -6,7 +6,7 @@
 namespace bsattn {
 
 constexpr int SHARE_SAMPLE = 4;       // lists looked at in the middle and at the end of a head
-constexpr int SHARE_MIN_BLOCKS = 16;  // row blocks of a head whose lists may be cut, at least
+constexpr int SHARE_MIN_BLOCKS = 8;   // row blocks of a head whose lists may be cut, at least
 
 // len: tiles of the list; mid, end: of SHARE_SAMPLE lists in the middle of the head and of its last ones; tail: shares that a list of
 // the last, incomplete round of workgroups is cut into (tail_of; 1: it is in front of it); load: row blocks per resident workgroup, times

@@ -18,7 +18,7 @@ SIZES = [(1, 1), (1, 65), (2, 447), (7, 1000),       # two groups, whole lists
          (1, 8300),                                  # block masks: one group, three shares; words: two groups
          (4, 4096),                                  # two groups, one row block per compute unit
          (8, 2304), (4, 5121), (3, 5504)]            # one group; ... two shares; ... three of the longest lists, which fill the GPU
-WIDE_SIZES = [(2, 1500, False),                      # D = 256: up to four shares
+WIDE_SIZES = [(1, 450, True), (1, 512, False), (1, 700, True), (2, 1500, False),       # lists cut from six tiles on, at D = 256
               (3, 5504, True),                       # more than a workgroup per compute unit: three shares of the longest
               (8, 4000, True), (10, 4161, False)]    # nearly two; more than a round, whose last lists are cut
 
