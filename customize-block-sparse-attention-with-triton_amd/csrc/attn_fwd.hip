@@ -1424,7 +1424,7 @@ struct QuadPlan { int groups, split, most; };      // most: shares of a list by 
 static QuadPlan quad_plan(int64_t row_blocks, int nb, bool words) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   auto plan = [](int groups, int most, int fill = 1) { return QuadPlan{groups, std::max(most, fill), most}; };
-  if (rows > 512) return plan(0, 1);
+  if (rows > 512 || nb > QUAD_MAX_BLOCKS) return plan(0, 1);
   if (words) {
     if (rows > 256 && (rows > 272 || nb < 200)) return plan(1, nb >= 28 ? 2 : 1, nb >= 64 && rows <= 336 ? 3 : 1);
     return plan(2, nb < 16 ? 1 : rows <= 64 ? 4 : rows <= 128 || nb >= 28 ? 2 : 1);
@@ -1541,8 +1541,7 @@ bool launch_fwd_takes_mask(int B, int H, int N, int D) {
 
 size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
   if (D == 256) {      // (compact: what a launch that sums parts of all lists would take, for which fewer shapes have room)
-    const size_t parts = pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, compact));
-    return compact ? parts : std::max(parts, quad_parts_bytes(B, H, (N + 63) / 64, D, wide_split(B, H, N, false)));
+    return compact ? pair_parts_bytes(B, H, N, D, pair_split(B, H, N, D, true)) : quad_parts_bytes(B, H, (N + 63) / 64, D, wide_split(B, H, N, false));
   }
   if (D == 128) {
     const int nb = (N + 63) / 64;
@@ -1693,7 +1692,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     return launch_status();
   }
   if (s.D != 64 || plan.pairs > 0) {
-    prm.split = s.D == 64 ? plan.split : pair_split(s.B, s.H, s.N, s.D, s.compact);
+    prm.split = s.D == 64 ? plan.split : tile_bits != nullptr ? 1 : pair_split(s.B, s.H, s.N, s.D, s.compact);
     prm.place = place_of_eight(heads, prm.nb, prm.split);
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;

@@ -65,7 +65,7 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
   int t0, t1;
   if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
   else { t0 = 0; t1 = columns_of_row<MASK_MAX_BLOCKS>(prm, b, h, m, lane, lcols, chunk == 0 && w == 0); }
-  if (prm.split > 1) {                           // this workgroup's share of the row block's list
+  if (!EW && prm.split > 1) {                    // this workgroup's share of the row block's list (elementwise masks: launches that fill the GPU)
     const int len = t1 - t0;
     if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
     t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
 
   // ---- normalise and write ----
   const float lsum = l_i + __shfl_xor(l_i, 32);
-  if (prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
+  if (!EW && prm.split > 1) {   // unnormalised fp32 part with its reference exponent and row sum
     if (!exists) return;
     float* part = prm.part_o + ((int64_t)chunk * BH + bh) * prm.N * D;
 #pragma unroll
@@ -423,7 +423,7 @@ static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   const int grid = prm.place.per_share * prm.split;
   if (prm.N % 64 != 0) launch_pair_c<DT, EW, true>(prm, grid, st);
   else launch_pair_c<DT, EW, false>(prm, grid, st);
-  if (prm.split > 1) launch_sum_parts(prm, PAIR_D, DT != 0, st);
+  if (!EW && prm.split > 1) launch_sum_parts(prm, PAIR_D, DT != 0, st);
 }
 
 template <bool EW>

@@ -33,7 +33,7 @@ template <int D, int S, bool EW> struct QuadCfg {
   static constexpr int PART_BYTES = 64 * PITCH * 4;
   static constexpr int GROUP_BYTES = 2 * (STAGE_BYTES > PART_BYTES ? STAGE_BYTES : PART_BYTES);     // two stages, then two results
   static constexpr int COLS_OFF = S * GROUP_BYTES;
-  static constexpr int COLS_CAP = 1024;                                         // column indices of the list kept in LDS
+  static constexpr int COLS_CAP = QUAD_MAX_BLOCKS;                              // column indices of the list kept in LDS
   static constexpr int ML_OFF = COLS_OFF + COLS_CAP * 4;                        // (m, l) per key half, group and query
   static constexpr int LDS_BYTES = ML_OFF + 2 * S * 64 * 2 * 4;
   static_assert(MASK_MAX_BLOCKS <= COLS_CAP, "all columns from the mask are in LDS");
@@ -54,7 +54,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = wave >> 2, quarter = wave & 3, kh = quarter >> 1, w = wave & 1;
   const int ln = lane & 31, g = lane >> 5;
-  const int nb = prm.nb, BH = prm.B * prm.H;
+  const int nb = prm.nb;
   int chunk;
   const Place p = prm.place.of(blockIdx.x, chunk);
   const int bh = p.head, m = nb - 1 - p.item;
@@ -88,15 +88,8 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
   const unsigned short* vg = (const unsigned short*)prm.v + b * prm.vs[0] + h * prm.vs[1];
   const float qk_scale = prm.qk_scale;
   const cint_ptr_t cols = (cint_ptr_t)(uintptr_t)prm.col_idx;
-  typedef const unsigned char __attribute__((address_space(4)))* cbyte_ptr_t;
   constexpr int COL_MASK = 0x3fffffff;            // (EW: bit 30 of a staged column says "partly set")
-  auto flagged_col = [&](int t) {
-    int x = cols[t];
-    if constexpr (EW) x |= (int)((cbyte_ptr_t)(uintptr_t)prm.tile_partial)[t] << 30;
-    return x;
-  };
   const int first_t = listed ? t0 : 0;            // entry t of the list is lcols[t - first_t] once it is staged
-  auto col_of = [&](int t) { return t - first_t < C::COLS_CAP ? lcols[t - first_t] : flagged_col(t); };
   unsigned char* mine = lds + c * C::GROUP_BYTES;
   const unsigned mine_addr = (unsigned)(uintptr_t)(lds_ptr_t)lds + c * C::GROUP_BYTES;
 
@@ -154,7 +147,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
     issue(cx, t, 0);
   }
   if (listed) {
-    for (int i = threadIdx.x; i < t1 - t0 && i < C::COLS_CAP; i += 256 * S) {
+    for (int i = threadIdx.x; i < t1 - t0; i += 256 * S) {
       int x = prm.col_idx[t0 + i];
       if constexpr (EW) x |= (int)prm.tile_partial[t0 + i] << 30;
       lcols[i] = x;
@@ -190,7 +183,7 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
     const int tn = t + S;
     int cxn = 0;
     if (tn < t1) {
-      cxn = __builtin_amdgcn_readfirstlane(col_of(tn));
+      cxn = __builtin_amdgcn_readfirstlane(lcols[tn - first_t]);
       issue(cxn & COL_MASK, tn, (it + 1) & 1);
     }
     const int keys = TAIL && !EW && cx == tail_cb ? valid - 32 * kh : 32;      // of this half

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kh = wave >> 1, w = wave & 1;
   const int ln = lane & 31, g = lane >> 5;
-  const int nb = prm.nb, BH = prm.B * prm.H;
+  const int nb = prm.nb;
   int chunk;
   const Place p = prm.place.of(blockIdx.x, chunk);
   const int bh = p.head, m = nb - 1 - p.item;

@@ -37,6 +37,8 @@ struct FwdParams {
   Divisor per_batch;               // H
 };
 
+constexpr int QUAD_MAX_BLOCKS = 1024;      // row blocks of a head that fwd_quad_kernel takes, at most
+
 // fwd_quad_kernel's and fwd_wide_kernel's: what quad_shares asks for, and
 struct FwdShareParams : FwdParams {
   int tail_from, tail_shares, tail_len, load, most, share_least;

@@ -215,9 +215,9 @@ int bsattn_fwd_block_mask(const void* q, const void* k, const void* v, void* o, 
  * graph capture, tight serving loops, harnesses that forbid allocation.  Same arguments, results and
  * kernels as bsattn_fwd, with the workspace replaced by a device array of
  * BSATTN_STATIC_SCRATCH_BYTES that is part of the library (every GPU the library runs on holds its
- * own copy until the process ends).  Shapes whose parts and flags (the memory
- * bsattn_fwd's kernels use out of its workspace) exceed that size are
- * rejected with BSATTN_ERR_STATIC_LIMIT before any device work.  All calls on one GPU share the
+ * own copy until the process ends).  Shapes whose parts and flags exceed that size are
+ * rejected with BSATTN_ERR_STATIC_LIMIT before any device work; at D = 256 these are taken to be two parts at least of
+ * every row block's list in launches of few row blocks, also where the kernels would do with fewer.  All calls on one GPU share the
  * array: two calls that overlap in time on the same GPU (different streams or threads) race and
  * must be serialised by the caller; calls on one stream are ordered and safe.  Nothing has to be
  * cleared between calls (stale contents are told apart by a per-launch number).  The first call on
