@@ -93,8 +93,8 @@ def test_very_long_sequence_n262144(dev):
 
 
 def test_head_dim_256_row_lists_shared_by_workgroups(dev):
-    """D = 256, one head, 128 row blocks: every row list is split over 8 workgroups whose fp32 parts a
-    second kernel sums.  Rows with fewer tiles than parts (empty parts), a full row and an empty row."""
+    """D = 256, one head, 128 row blocks: lists are split over up to 4 workgroups by their
+    length, whose fp32 parts the last one in sums.  Rows with fewer tiles than parts, a full row and an empty row."""
     nb = 128
     mask = uniform_block_mask(1, 1, nb, 0.04, 1241)
     mask[0, 0, 5, :] = True

@@ -80,9 +80,8 @@ def test_nothing_beyond_the_last_token_is_touched(dev, D, N, contiguous_rows):
         assert ma <= 2e-2 and (rl <= 1e-3 or ma <= 1e-5), (name, ma, rl)     # (a zero gradient has no relative error)
 
 
-# D = 128, elementwise masks and ragged lengths: row lists shared by 2 (504 row blocks), 4 (short rows), 1 (two tiles a
-# row) and 5 (81 long rows) workgroups, shares without tiles among them; 512 row blocks: by 2 with an elementwise mask
-# only.  Backward: lists of 13 and 16 tiles shared at D = 64 and 256.
+# D = 128, elementwise masks and ragged lengths: single groups of wavefronts (504 and 512 row blocks), two groups (32, 6 and 81), whose lists are
+# shared by up to 4 workgroups.  Backward: lists of 13 and 16 tiles shared at D = 64 and 256.
 @pytest.mark.parametrize("H,N,D", [(8, 4000, 128), (8, 4090, 128), (2, 1000, 128), (3, 100, 128), (1, 5184, 128), (8, 777, 64),
                                    (2, 1000, 64), (8, 777, 256), (2, 1000, 256), (12, 1400, 256)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
@@ -214,7 +213,7 @@ def test_uneven_heads(dev, H, N, D):
             assert errors(got[sl], ref)[1] <= 1e-3, h
 
 
-# D = 128, block masks: 3 shares of 13 tiles, 2 of 24 (with a ragged length too), 4 and 3 of long lists, 1 with more row blocks
+# D = 128, block masks: two groups of wavefronts, up to four and two shares, single groups
 @pytest.mark.parametrize("H,N", [(1, 832), (6, 1536), (6, 1500), (2, 4096), (4, 4096), (5, 4096), (7, 2048)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_shares_of_block_mask_lists(dev, H, N, dtype):

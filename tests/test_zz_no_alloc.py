@@ -69,7 +69,7 @@ def test_static_forward_matches_workspace_forward(dev):
     _both(dev, 1, 2, 512, 64, torch.float16, 0.5, 12)
     _both(dev, 1, 1, 1024, 128, torch.bfloat16, 0.6, 13)
     # D = 256 with few row blocks: the row lists are shared between workgroups and the scratch array holds
-    # their fp32 parts, which a second kernel sums (2 MB here)
+    # their fp32 parts, which the last one in sums (4 MB here)
     _both(dev, 1, 1, 1024, 256, torch.float16, 0.6, 14)
 
 
