@@ -1331,21 +1331,23 @@ static int long_row_groups(int B, int H, int nb, bool compact) {
 // compute unit, so launches that leave the GPU's 512 short share, and those in little more than a round, whose last lists would run alone.
 // us, N(0,1) bf16, a fixed number of shares for all lists and a launch that summed their fp32 parts / the lists that their length
 // calls for, summed in the launch; keep 0.1, 0.3, 1, block-causal:
-//    1 head  N = 1024 (16 row blocks)   14 / 12     16 / 16     19 / 21     18 / 20
-//    2 heads N = 1344 (42)              17 / 12     20 / 18     25 / 23     23 / 22
-//    1 head  N = 4096 (64)              22 / 20     26 / 25     38 / 39     37 / 37
-//    4 heads N = 2048 (128)             26 / 21     30 / 23     39 / 36     36 / 32
-//    2 heads N = 4096 (128)             29 / 23     36 / 31     56 / 52     49 / 44
-//    7 heads N = 2048 (224)             29 / 18     35 / 28     53 / 46     48 / 40
-//    2 heads N = 6461 (202)             47 / 33     67 / 60    128 / 108    87 / 83
-//    3 heads N = 6016 (282)             50 / 34     74 / 64    150 / 158    98 / 87
-//    8 heads N = 4096 (512)             56 / 32     79 / 56    165 / 141   101 / 97
-//    5 heads N = 8192 (640)             94 / 67    162 / 153   396 / 394   223 / 215
+//    1 head  N = 768 (12 row blocks)      15 /  14     16 /  17     18 /  19     18 /  18
+//    1 head  N = 1024 (16)                14 /  14     17 /  17     19 /  20     19 /  20
+//    2 heads N = 1344 (42)                18 /  16     22 /  19     27 /  23     24 /  22
+//    1 head  N = 4096 (64)                23 /  20     29 /  27     42 /  41     39 /  37
+//    4 heads N = 2048 (128)               28 /  21     32 /  26     42 /  38     38 /  33
+//    2 heads N = 4096 (128)               30 /  26     38 /  33     60 /  55     52 /  47
+//    7 heads N = 2048 (224)               31 /  22     39 /  31     57 /  52     50 /  44
+//    2 heads N = 6461 (202)               50 /  36     72 /  61    132 / 122     90 /  90
+//    3 heads N = 6016 (282)               52 /  37     76 /  76    159 / 151    101 /  93
+//    8 heads N = 4096 (512)               59 /  34     87 /  67    180 / 154    110 / 102
+//    5 heads N = 8192 (640)              104 /  75    176 / 163    386 / 366    239 / 214
 // Elementwise masks (on fwd_pair_kernel before), token window of 0.1 N, 0.25 N, 0.45 N, token-causal:
-//    2 heads N = 1024 (32)              14 / 11     17 / 14     19 / 18     20 / 20
-//    8 heads N = 2048 (256)             27 / 17     32 / 22     39 / 30     57 / 40
-//    8 heads N = 4000 (504)             70 / 29     95 / 44    127 / 65    134 / 94
-//    1 head  N = 8192 (128)             32 / 28     41 / 36     56 / 46     93 / 70
+//    1 head  N = 768 (12)                 12 /  14     14 /  14     16 /  17     18 /  17
+//    2 heads N = 1024 (32)                14 /  13     18 /  16     20 /  18     20 /  19
+//    8 heads N = 2048 (256)               30 /  20     35 /  25     42 /  33     60 /  45
+//    8 heads N = 4000 (504)               75 /  34    100 /  53    131 /  76    138 / 101
+//    1 head  N = 8192 (128)               34 /  27     43 /  37     60 /  51     96 /  75
 static int pair_split_256(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   if (rows > 8 * nb || rows >= 1024) return 1;
@@ -1378,7 +1380,7 @@ static int pair_split_128(int64_t row_blocks, int nb) {
 // Which launches fwd_quad_kernel (D = 128) takes: groups of four wavefronts per workgroup (0: none) and shares of a list, at most
 // (quad_shares.h).  With two groups a row block has a compute unit to itself, with one two share it.  us, fwd_pair_kernel with its shares
 // and the launch that summed them / 2 groups, whole lists / 2 groups, up to 2 shares / up to 4 / 1 group, whole / up to 2; N(0,1) bf16;
-// keep 0.1, 0.3, 1, block-causal:
+// keep 0.1, 0.3, 1, block-causal (this kernel without tiles in two parts, which take 0.5 us each, up to two: exact_tiles):
 //    1 head  N = 2048 (32 row blocks)  12/13/13/13          15/16/16/16          20/25/21/19          19/25/20/18
 //    1 head  N = 4096 (64)             16/15/16/16          20/22/19/18          32/43/30/24          30/43/29/23
 //    7 heads N = 1000 (112)            11/10                17/12                28/17                28/16

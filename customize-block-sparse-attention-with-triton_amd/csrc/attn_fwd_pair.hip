@@ -10,7 +10,7 @@
 // row blocks resident on an XCD share one head's K and V in its L2; long row blocks of
 // block-causal masks come first.  Two barriers per tile: in front of the one that frees the K buffer both wavefronts wait for their
 // halves of V, in front of the one that frees V for those of the next K.  (Four, with waits of their own: 16 heads N = 8192 dense 641 -> 541 us,
-// keep 0.3 193 -> 187, 28 heads N = 2048 dense 72 -> 70, 16 heads N = 4000 token-causal 125 -> 122; block-causal masks the same.)
+// on another card 648 -> 572, keep 0.3 193 -> 187, 28 heads N = 2048 dense 72 -> 70, 16 heads N = 4000 token-causal 125 -> 122; block-causal masks the same.)
 //
 // Tile arithmetic, softmax and layouts are those of attn_fwd.hip (fa2_custom_mask/fa2_fwd.py:146-196
 // of the reference), with a single block of 32 queries per wavefront.
