@@ -1418,7 +1418,9 @@ static int pair_split_128(int64_t row_blocks, int nb) {
 //    1 head  N = 10880 (170)   29/ - /28 46/ - /55  93/ - /120   77/ - /66       (pairs)
 // Pairs / single groups, whole or by a list's own length / this:
 //    3 heads N = 5632 (264)    29/24/26  41/46/47   79/101/ 88   64/ 60/56       3 heads N = 6400 (300)    31/29/28  48/58/50   93/114/103  73/65/64
-//    4 heads N = 4352 (272)    26/20/20  36/35/36   66/ 80/ 75   54/ 59/50       4 heads N = 4800 (300)    29/23/23  41/43/44   75/ 86/ 84  59/64/50
+//    4 heads N = 4352 (272)    26/20/20  36/35/36   66/ 80/ 75   54/ 59/50       4 heads N = 4800 (300)    29/23/23  41/43/44   75/ 86/ 84  59/64/50    (whole)
+// (Room for a share that a list never gets costs the launch the workgroups that find so, 1 to 2 us at a full round: 2 x 2 heads N = 3825
+// keep 0.63 (240) whole 34.5, with room for two shares 38.9; 3 heads N = 4096 (192) keep 0.3 27.5 and 29.)
 //    words: 1 head N = 20000 (313), two groups in place of the whole single ones    57/65/55  94/113/97  134/135/139  236/216/186
 //    words: 1 head N = 17920 (280)                                                  43/56/43  74/ 87/77  108/102/117  178/180/143
 // From 480 row blocks on a round of single groups is full (one head N = 32000 (500) 105/ - /92  263/ - /218  665/ - /586  636/ - /375).
@@ -1427,18 +1429,19 @@ static QuadPlan quad_plan(int64_t row_blocks, int nb, bool words) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   auto plan = [](int groups, int most, int fill = 1) { return QuadPlan{groups, std::max(most, fill), most}; };
   if (rows > 512 || nb > QUAD_MAX_BLOCKS) return plan(0, 1);
+  const int fill = nb >= 3 * FILL_GAIN && rows <= 336 ? 3 : 1;      // (more than 256 row blocks: thirds of lists, tail_of)
   if (words) {
-    if (rows > 256 && (rows > 272 || nb < 200)) return plan(1, nb >= 28 ? 2 : 1, nb >= 64 && rows <= 336 ? 3 : 1);
+    if (rows > 256 && (rows > 272 || nb < 200)) return plan(1, nb >= 28 ? 2 : 1, fill);
     return plan(2, nb < 16 ? 1 : rows <= 64 ? 4 : rows <= 128 || nb >= 28 ? 2 : 1);
   }
   if (rows > 256) {
     if (nb < 28 || (nb >= 150 && rows < 480)) return plan(0, 1);
-    return plan(1, nb >= 80 ? 2 : 1, nb >= 64 && rows <= 336 ? 3 : 1);
+    return plan(1, nb >= 80 ? 2 : 1, fill);
   }
   if (nb < 6 || (rows > 168 && rows <= 230 && nb >= 150)) return plan(0, 1);
   if (rows > 128 && rows <= 168 && nb >= 64) return plan(1, 3);
   if (rows <= 128) return plan(2, rows <= 64 && nb >= 16 ? 4 : nb >= 24 ? 2 : 1);
-  return plan(2, nb >= (rows <= 160 ? 40 : 56) ? 2 : 1);
+  return plan(2, nb >= (rows <= 160 ? 40 : 80) ? 2 : 1);
 }
 static_assert(SHARE_MIN_BLOCKS <= 16, "heads of launches that share lists have as many row blocks");
 

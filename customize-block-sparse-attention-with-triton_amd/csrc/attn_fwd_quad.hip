@@ -42,7 +42,9 @@ template <int D, int S, bool EW> struct QuadCfg {
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
 // TAIL: N is not a multiple of 64 (as in attn_fwd.hip: the copy of the last tile repeats its last key, the scores beyond
 // it are -inf, the queries beyond N are not written; a half without any key leaves the tile out).
-template <int D, int S, int DT, bool EW, bool TAIL>
+// PARTS: some first tiles keep their numerators in two parts (first_tiles; launches that have none run without the code for it: 7 heads
+// N = 3000 dense 63 -> 59 us, D = 256 10 heads N = 4090 dense 225 -> 220).
+template <int D, int S, int DT, bool EW, bool TAIL, bool PARTS>
 __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdShareParams prm) {
   using C = QuadCfg<D, S, EW>;
   constexpr int KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
@@ -237,11 +239,11 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
       }
       uintx4 pf[2];
       float lnew = 0.f;
-      // A tile calls for a new reference: the first one (FOLD: it keeps 0 when its sums are of moderate size, else it is known beforehand and saves
-      // a softmax), and where numerators grow too large.  (With a softmax in front of every reference and of every tile in two parts, us:
-      // 1 head N = 1024 keep 0.1 11.4, so 11.0; 3 heads N = 3000 keep 0.1 15.5, 14.8; D = 256 1 head N = 1024 keep 0.1 14.5, 13.7.)
-      const bool parts = it < two_parts;
-      bool far = !FOLD && fresh;
+      // A tile calls for a new reference: the first one (FOLD: it keeps 0 when its sums are of moderate size), and where numerators grow too
+      // large.  PARTS: a first one that is known to (all but FOLD) saves a softmax, and another if it is in two parts (us, with them: 1 head N = 1024
+      // keep 0.1 11.4, so 11.0; 3 heads N = 3000 keep 0.1 15.5, 14.8; D = 256 1 head N = 1024 keep 0.1 14.5, 13.7; the test for it costs long lists 1 %).
+      const bool parts = PARTS && it < two_parts;
+      bool far = PARTS && !FOLD && fresh;
       if (!far) {
         lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
         far = __any((FOLD && fresh && !(lnew >= 0.25f)) || !(lnew - l_i < limit));
@@ -252,13 +254,15 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
           any_m = 1;
           if (!parts) lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
         }
-        if (parts) {
-          uintx4 rest[2];
-          lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
+        if constexpr (PARTS) {
+          if (parts) {
+            uintx4 rest[2];
+            lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
 #pragma unroll
-          for (int ts = 0; ts < 2; ++ts)
+            for (int ts = 0; ts < 2; ++ts)
 #pragma unroll
-            for (int db = 0; db < DB; ++db) oacc[db][0] = mfma_qk<PB>(vfr[ts][db], rest[ts], oacc[db][0]);
+              for (int db = 0; db < DB; ++db) oacc[db][0] = mfma_qk<PB>(vfr[ts][db], rest[ts], oacc[db][0]);
+          }
         }
         if (far) limit = sum_limit<false>(lnew);
       }
@@ -393,15 +397,22 @@ __global__ __launch_bounds__(256 * S, 2) void fwd_quad_kernel(const FwdSharePara
   if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int D, int S, int DT, bool EW, bool TAIL>
-static void launch_quad_t(const FwdShareParams& prm, hipStream_t st) {
+template <int D, int S, int DT, bool EW, bool TAIL, bool PARTS>
+static void launch_quad_p(const FwdShareParams& prm, hipStream_t st) {
   constexpr int LDS = QuadCfg<D, S, EW>::LDS_BYTES;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_quad_kernel<D, S, DT, EW, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_quad_kernel<D, S, DT, EW, TAIL, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((fwd_quad_kernel<D, S, DT, EW, TAIL>), dim3(grid), dim3(256 * S), LDS, st, prm);
+  hipLaunchKernelGGL((fwd_quad_kernel<D, S, DT, EW, TAIL, PARTS>), dim3(grid), dim3(256 * S), LDS, st, prm);
+}
+
+template <int D, int S, int DT, bool EW, bool TAIL>
+static void launch_quad_t(const FwdShareParams& prm, hipStream_t st) {
+  if constexpr (DT == 0) launch_quad_p<D, S, DT, EW, TAIL, EW>(prm, st);       // (fp16: none with block masks, one at least with elementwise ones)
+  else if (first_tiles<false>(prm.exact, S) > 0) launch_quad_p<D, S, DT, EW, TAIL, true>(prm, st);
+  else launch_quad_p<D, S, DT, EW, TAIL, false>(prm, st);
 }
 
 template <int D, int S, int DT>

@@ -37,8 +37,9 @@ static_assert(4 * rows_out_bytes(128, true) <= WIDE_LDS_BYTES, "room for the res
 // CONTIG: the rows of K and of V follow each other without gaps (row stride = 256).
 // TAIL: N is not a multiple of 64: the copy of the last tile repeats its last key, the scores beyond it are -inf (a half without
 // any key leaves the tile out), the queries beyond N are not written.
+// PARTS: some first tiles keep their numerators in two parts (attn_fwd_quad.hip).
 // EW: elementwise masks (bit 30 of a staged column says "partly set", the tile's 64 row words travel with K).
-template <int DT, bool CONTIG, bool TAIL, bool EW>
+template <int DT, bool CONTIG, bool TAIL, bool EW, bool PARTS>
 __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams prm) {
   constexpr int D = WIDE_D, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, RPI = 64 / CPR;
   constexpr int COPIES = CPR / 4;                // copy instructions per wavefront and tile
@@ -289,8 +290,8 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
     } else {
       float lnew = 0.f;
       // (which tiles call for a new reference: attn_fwd_quad.hip; elementwise masks take the softmax first, or 8 to 20 bytes more spill in five variants)
-      const bool parts = t < two_parts_to;
-      bool far = !FOLD && !EW && fresh;
+      const bool parts = PARTS && t < two_parts_to;
+      bool far = PARTS && !FOLD && !EW && fresh;
       if (!far) {
         lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
         far = __any((FOLD && fresh && !(lnew >= 0.25f)) || !(lnew - l_i < limit));
@@ -302,14 +303,16 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
           if (EW || !parts) lnew = softmax_block<FOLD, PB>(sc, qk_scale, m_i, l_i, pf);
           if (EW) limit = sum_limit<false>(lnew);
         }
-        if (parts) {
-          uintx4 rest[2];
-          lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
+        if constexpr (PARTS) {
+          if (parts) {
+            uintx4 rest[2];
+            lnew = softmax_block_parts<FOLD, PB>(sc, qk_scale, m_i, l_i, pf, rest);
 #pragma unroll
-          for (int pt = 0; pt < 4; ++pt) {
-            read_v(pt);
-            second(pt, rest);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int pt = 0; pt < 4; ++pt) {
+              read_v(pt);
+              second(pt, rest);
+              __builtin_amdgcn_sched_barrier(0);
+            }
           }
         }
         if (!EW && far) limit = sum_limit<false>(lnew);
@@ -436,15 +439,22 @@ __global__ __launch_bounds__(256, 2) void fwd_wide_kernel(const FwdShareParams p
   if (prm.lse != nullptr && kh == 0 && g_e == 0 && (!TAIL || qrow < prm.N)) prm.lse[(int64_t)bh * prm.N + qrow] = row_lse(M, L);
 }
 
-template <int DT, bool CONTIG, bool TAIL, bool EW>
-static void launch_wide_c(const FwdShareParams& prm, hipStream_t st) {
+template <int DT, bool CONTIG, bool TAIL, bool EW, bool PARTS>
+static void launch_wide_p(const FwdShareParams& prm, hipStream_t st) {
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL, EW>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_wide_kernel<DT, CONTIG, TAIL, EW, PARTS>), hipFuncAttributeMaxDynamicSharedMemorySize,
                               WIDE_LDS_BYTES);
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG, TAIL, EW>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
+  hipLaunchKernelGGL((fwd_wide_kernel<DT, CONTIG, TAIL, EW, PARTS>), dim3(grid), dim3(256), WIDE_LDS_BYTES, st, prm);
+}
+
+template <int DT, bool CONTIG, bool TAIL, bool EW>
+static void launch_wide_c(const FwdShareParams& prm, hipStream_t st) {
+  if constexpr (DT == 0) launch_wide_p<DT, CONTIG, TAIL, EW, EW>(prm, st);      // (fp16: as in attn_fwd_quad.hip)
+  else if (first_tiles<false>(prm.exact, 1) > 0) launch_wide_p<DT, CONTIG, TAIL, EW, true>(prm, st);
+  else launch_wide_p<DT, CONTIG, TAIL, EW, false>(prm, st);
 }
 
 template <int DT, bool EW>

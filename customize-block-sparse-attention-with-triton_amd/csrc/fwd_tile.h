@@ -192,7 +192,7 @@ __device__ __forceinline__ int shares_of_list(const FwdShareParams& prm, cint_pt
 // Tiles at the front of a walk whose numerators are kept in two parts (softmax_block_parts), for a list that `walks` of them take on: without
 // any the largest numerator of a walk is exact, which counts 48 hundredths (FOLD: the reference stays at 0, and none is).
 template <bool FOLD>
-__device__ __forceinline__ int first_tiles(int exact, int walks) { return exact <= (FOLD ? 0 : 48) * walks ? 0 : exact <= 100 * walks ? 1 : 2; }
+constexpr int first_tiles(int exact, int walks) { return exact <= (FOLD ? 0 : 48) * walks ? 0 : exact <= 100 * walks ? 1 : 2; }
 
 // Counts a share of a list in, by one thread, when all accesses of its workgroup to its part have been acknowledged; returns how many
 // are in.  The counter holds (launch mark << 16 | shares counted); stale contents carry another mark.  seen: a first guess of it.
