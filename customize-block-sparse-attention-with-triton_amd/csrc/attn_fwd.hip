@@ -818,12 +818,19 @@ void fwd_kernel(const FwdRangeParams prm) {
     }
   } else if constexpr (MODE == WAVE) {
     // ================= one wavefront, one range =================
+    // The range's last row block is walked first, then the others from the range's beginning: what is kept of the last row block begins
+    // in an early column, and the rest of the first one goes on about where that has ended (row blocks of equal length: a range is one of
+    // them and a bit).  So all wavefronts of an XCD walk the columns from the first to the last at the same time, whatever row block their range
+    // begins in, and the tiles at work at once fit its L2, which K and V of a long head do not.  In list order / so, us:
+    //   8 heads N = 17536 dense 718 / 695, N = 24000 dense 1381 / 1287, keep 0.1 161 / 154; 5 heads N = 32000 keep 0.5 915 / 745, keep 0.1 209 / 171;
+    //   6 heads N = 17536 keep 0.1 80 / 74; 9 heads N = 20032 keep 0.5 555 / 531; within the L2: 10 heads N = 12000 dense 456 / 427, 16 heads
+    //   N = 12032 dense 663 / 655, N = 8192 keep 0.1 54 / 51, causal keep 0.2 91 / 93 and 54 / 54, 24 heads N = 4096 keep 0.1 29.6 / 29.7.
     // first row block of the range: largest r with rp[r] <= g0 < rp[r+1]
     // A range boundary within `snap` tiles of an end of the row block it falls in moves to that end
     // (the nearer one): sharing a row block costs a merge, a published part and a pull, several
     // tiles' worth each, and row blocks of up to 2 `snap` tiles are never shared.  Every workgroup
     // applies the same rule with the same distance to both of its boundaries, so the ranges still tile the list.
-    int r, g0, g1;
+    int r, g0, g1, start, r_first = 0, r_last = 0;      // start: the first tile walked
     {
       // the row blocks in which the two ends of the range lie (positions behind a row block's tiles count as
       // its end), then the tiles themselves
@@ -841,26 +848,38 @@ void fwd_kernel(const FwdRangeParams prm) {
         g1 = hs.lo + hs.T;
       }
       if (g0 >= g1) return;
+      start = g0;
+      if (x1 < hs.X && s1 > g0 && s1 < g1) { start = s1; r_last = c1 - 1; }
     }
     // two slots per workgroup: a range can end inside one row block (that part goes to slot 1: it holds the row
     // block's first tiles) after having begun inside another (slot 0)
     auto wg_slot = [&](int p, bool head) { return prm.ws + (((int64_t)bh * prm.W + p) * 2 + (head ? 1 : 0)) * partial_floats(D); };
-    int cx = flagged_col(g0);                                  // current tile: column block | flag
-    k_copy_all(cx & COL_MASK, g0);
+    int cx = flagged_col(start);                               // current tile: column block | flag
+    k_copy_all(cx & COL_MASK, start);
     v_copy_all(cx & COL_MASK);
     stage_cols(g0, g1);
     auto col_of = [&](int t) { return t - g0 < COLS_CAP ? lcols[t - g0] : flagged_col(t); };
-    int t = g0;
-    while (t < g1) {
+    int t = start, end = g1;
+    bool wrapped = start == g0;
+    if (!wrapped) { r_first = r; r = r_last; }
+    for (;;) {
+      if (t >= end) {
+        if (wrapped) break;
+        wrapped = true;
+        t = g0;
+        end = start;
+        r = r_first;
+      }
       const int row_s = rp[r], row_e = rp[r + 1];
       if (row_e <= t) { ++r; continue; }          // row block without kept tiles in the range
-      const int seg_b = row_e < g1 ? row_e : g1;
+      const int seg_b = row_e < end ? row_e : end;
       reset_acc();
       load_q(r);
       for (int j = t; j < seg_b; ++j) {           // (the next tile is prefetched across the end of the row block)
-        const bool has1 = j + 1 < g1;
-        const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(j + 1)) : 0;
-        tile(has1, cxn & COL_MASK, j + 1, has1, is_partial(cx), [] {});
+        const bool has1 = j + 1 < end || !wrapped;
+        const int nxt = j + 1 < end ? j + 1 : g0;
+        const int cxn = has1 ? __builtin_amdgcn_readfirstlane(col_of(nxt)) : 0;
+        tile(has1, cxn & COL_MASK, nxt, has1, is_partial(cx), [] {});
         cx = cxn;
       }
       if (t == row_s && seg_b == row_e) {
@@ -1252,21 +1271,26 @@ int compute_units() {
 }
 
 // How a launch is split at D = 64, by its row blocks against the wavefronts that are resident at once (8 per compute unit).
-// From half as many more on a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us; 24 heads of
-// N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there).  From three
-// quarters as many on a wavefront takes a range of the list, with fewer the ranges of whole workgroups are the faster
-// ones: they share a row block's merge.  bf16, us, ranges of workgroups / of wavefronts, keep 0.1, 0.3, 1 and block-causal:
-//   12 heads N = 8192 (0.75)   53 /  47    92 /  90   247 / 250   137 / 138      8 heads N = 8192 (0.5)   36 / 41   65 / 72   167 / 162    98 / 105
-//    9 heads N = 12000 (0.83)  71 /  65   139 / 138   398 / 404   211 / 208      6 heads N = 12000 (0.55) 53 / 52   96 / 98   265 / 270   153 / 153
-//   24 heads N = 4096 (0.75)   33 /  31    61 /  55   137 / 135    86 /  77     17 heads N = 4096 (0.53)  30 / 28   47 / 45    99 / 101    66 /  67
-//   48 heads N = 2048 (0.75)   26 /  24    40 /  38    85 /  79    54 /  58     56 heads N = 2048 (0.88)  28 / 25   41 / 42    94 /  86    61 /  60
-//    5 heads N = 24064 (0.92) 115 / 116   273 / 288   889 / 902   435 / 445    (above 300 row blocks per head: from one per wavefront on)
+// With many a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us), with about as many a range of the list, with few
+// the ranges of whole workgroups are the faster ones: they share a row block's merge.
+// bf16, us, ranges of workgroups / of wavefronts, dense, block-causal, keep 0.5, 0.2, 0.1, 0.05:
+//   20 heads N = 4096 (0.62)  122 / 117    78 /  72    70 /  70    46 /  41    31 /  29    26 / 24
+//    3 heads N = 32000 (0.73) 994 / 904   491 / 473   505 / 470   219 / 208   124 / 117    77 / 72      6 heads N = 20032 (0.92) 738 / 711  383 / 375  387 / 374  173 / 163   98 /  92  64 / 58
+//   11 heads N = 8192 (0.69)  238 / 233   131 / 132   131 / 129    71 /  67    45 /  45    32 / 31      5 heads N = 17536 (0.67) 481 / 466  245 / 248  249 / 249  113 / 110   74 /  70  54 / 48    (not there)
+//   13 heads N = 6400 (0.63)  178 / 174   101 / 101   102 / 101    61 /  59    36 /  38    30 / 29      9 heads N = 8192 (0.56)  197 / 195  110 / 110  109 / 109   57 /  60   44 /  39  30 / 28    (nor there)
+//    4 heads N = 20032 (0.61) 483 / 482   256 / 256   258 / 257   116 / 118    72 /  74    50 / 49      3 heads N = 20032 (0.46) 388 / 375  197 / 201  201 / 200   91 /  94   63 /  61  41 / 43    (nor there)
+// whole row blocks / ranges of wavefronts:
+//   24 heads N = 8192 (1.50)  481 / 490   266 / 263   284 / 265   128 / 119    75 /  71    49 / 47     12 heads N = 17536 (1.61) 1231 / 1094  593 / 564  649 / 568  272 / 249  149 / 134  86 / 83
+//   14 heads N = 17536 (1.87) 1286 / 1258 681 / 657   685 / 655   292 / 283   168 / 163    99 / 104    16 heads N = 16640 (2.03) 1464 / 1278  665 / 676  755 / 675  317 / 290  175 / 166  104 / 100
+//   26 heads N = 8192 (1.62)  587 / 535   292 / 283   317 / 290   137 / 130    79 /  79    56 / 52     28 heads N = 8192 (1.75)  597 / 569   312 / 304   329 / 306   147 / 141    85 /  81    54 / 61    (not there)
+//   52 heads N = 4096 (1.62)  293 / 282   164 / 156   166 / 154    74 /  76    50 /  52    38 / 38     40 heads N = 6400 (1.95)  487 / 497   311 / 275   273 / 266   127 / 125    79 /  79    50 / 58    (nor there)
+//   18 heads N = 17536 (2.41) 1029 / 867  852 / 841   372 / 380   205 / 227   114 / 135                34 heads N = 8192 (2.12)  743 / 690   354 / 370   395 / 367   177 / 165    99 / 104   65 / 75    (nor there)
+// (compact: WAVE has four times as many ranges, hence parts, and there is no room for them.)
 static int wave_slots() { return FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * compute_units(); }    // wavefronts resident at once, D = 64
 static int fwd_mode(int B, int H, int nb, bool compact) {
-  const int64_t rows = (int64_t)B * H * nb, slots = wave_slots();
-  if (2 * rows >= 3 * slots) return ROWS_MODE;
-  if (compact) return COOP;                                             // (WAVE has four times as many ranges, hence parts)
-  return rows >= slots || (nb >= 32 && nb <= 300 && 20 * rows >= (nb >= 48 ? 15 : 16) * slots) ? WAVE : COOP;
+  const int64_t per_slot = 100ll * B * H * nb, slots = wave_slots();                 // (row blocks, in hundredths)
+  if (per_slot >= (compact || nb < 96 ? 150 : nb < 250 ? 174 : 216) * slots) return ROWS_MODE;
+  return !compact && per_slot >= (nb < 32 ? 100 : nb < 96 ? 60 : 70) * slots ? WAVE : COOP;
 }
 
 // ROWS_MODE: the workgroups per head for long row blocks, and the slots for their parts: as many as are resident at once,

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from helpers import fwd_route_d64
 from oracle import bsattn_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -125,3 +126,41 @@ def test_forward_against_naive(dev, seed):
         assert float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
     bar = 3e-3 if (dtype == torch.bfloat16 and not out_fp32) else 1e-3
     assert rel_l2(o, o_ref) <= bar
+
+
+# About as many row blocks as wavefronts: ranges of single wavefronts, whose last row block is walked before the first one.  Sizes
+# at both ends of that regime (0.6 to 1.5 row blocks per wavefront below 96 row blocks, 0.7 to 1.74 below 250, to 2.16 above) and inside it,
+# ranges that lie in one row block, end with one, and span several; bounds as above.
+@pytest.mark.parametrize("B,H,N,dtype,out_fp32,seed", [
+    (1, 20, 4096, torch.float16, False, 0), (1, 24, 4096, torch.bfloat16, True, 1), (1, 24, 4033, torch.bfloat16, False, 2),
+    (1, 16, 8160, torch.float16, True, 3), (2, 23, 4096, torch.float16, False, 4), (2, 8, 8192, torch.bfloat16, True, 5),
+    (1, 27, 8192, torch.float16, False, 6), (1, 16, 16100, torch.bfloat16, False, 7), (1, 47, 4064, torch.float16, True, 8)])
+def test_ranges_of_wavefronts(dev, B, H, N, dtype, out_fp32, seed):
+    import fa2_custom_mask as fm
+    rs = np.random.RandomState(100 + seed)
+    g = torch.Generator(device=dev).manual_seed(seed)
+    nb = (N + 63) // 64
+    assert fwd_route_d64(B, H, N) == "wavefronts"
+    q, k, v = [torch.randn(B, H, N, 64, generator=g, device=dev).to(dtype) for _ in range(3)]
+    bar = 3e-3 if (dtype == torch.bfloat16 and not out_fp32) else 1e-3
+    for step in range(3):
+        kind, keep, mask = make_mask(rs, H if step == 1 else 1, nb)
+        md = mask.to(dev)
+        print(dict(kind=kind, keep=keep, tiles=int(mask.sum())), flush=True)
+        o_ref, lse_ref = naive_forward(q, k, v, md, 0.125)
+        o, lse = fm.flash_attention_custom_mask_lse(q, k, v, md, 0.125, out_fp32=out_fp32)
+        none = torch.isinf(lse_ref)
+        assert torch.equal(torch.isinf(lse), none) and bool((o[none] == 0).all()) and bool(torch.isfinite(o).all())
+        if (~none).any():
+            assert float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
+        assert rel_l2(o, o_ref) <= bar
+        again, _ = fm.flash_attention_custom_mask_lse(q, k, v, md, 0.125, out_fp32=out_fp32)
+        assert torch.equal(o, again)                       # (a range's order is fixed)
+    if N <= 4096 and B == 1:                               # elementwise: a window of tokens
+        i = torch.arange(N, device=dev)
+        d = i[:, None] - i[None, :]
+        tokens = ((d >= 0) & (d < N // 3))[None, None]
+        o = fm.flash_attention_custom_mask(q, k, v, tokens, 0.125)
+        for h in (0, H - 1):
+            s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~tokens[0, 0], float("-inf"))
+            assert rel_l2(o[0, h], torch.softmax(s, -1) @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
