@@ -1015,8 +1015,9 @@ int launch_bwd(const void* q, const void* k, const void* v, const void* o, const
   const BwdPairs pairs = s.D == 128 ? bwd_pairs_128((int64_t)s.B * s.H * prm.nb, prm.nb, shares.split) : BwdPairs{0, 1};
   prm.split = plan.pairs > 0 ? plan.split : pairs.groups > 1 ? 1 : shares.split;
   prm.whole = plan.pairs > 0 || pairs.groups > 1 ? -1 : shares.whole;
-  prm.place = place_of_eight(s.B * s.H, prm.nb, plan.pairs > 0 ? 2 * prm.split : prm.split);
-  prm.place_dq = place_of_eight(s.B * s.H, prm.nb, 1);
+  const Groups group = groups_of_heads(s.B * s.H, s.N, s.D);
+  prm.place = place_of_eight(s.B * s.H, prm.nb, plan.pairs > 0 ? 2 * prm.split : prm.split, group);
+  prm.place_dq = place_of_eight(s.B * s.H, prm.nb, 1, group);
   prm.first_sum = pairs.dq_pairs > 0 ? 1 : 0;
   prm.per_batch = divisor((unsigned)s.H, (uint64_t)s.B * s.H);
   {

@@ -1703,7 +1703,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     FwdShareParams shared;
     static_cast<FwdParams&>(shared) = prm;
     shared.split = quads.split;
-    shared.place = place_of_eight(heads, prm.nb, shared.split);
+    shared.place = place_of_eight(heads, prm.nb, shared.split, groups_of_heads(heads, s.N, s.D));
     shared.load = (int)((int64_t)rows * 4096 / slots);
     shared.most = quads.most;
     const TailShares tail = tail_of(rows, slots, shared.split);
@@ -1722,7 +1722,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   }
   if (s.D != 64 || plan.pairs > 0) {
     prm.split = s.D == 64 ? plan.split : tile_bits != nullptr ? 1 : pair_split(s.B, s.H, s.N, s.D, s.compact);
-    prm.place = place_of_eight(heads, prm.nb, prm.split);
+    prm.place = place_of_eight(heads, prm.nb, prm.split, groups_of_heads(heads, s.N, s.D));
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
     prm.part_len = (int*)(prm.part_ml + (size_t)prm.split * heads * s.N * 2);

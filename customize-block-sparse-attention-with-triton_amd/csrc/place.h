@@ -52,23 +52,58 @@ constexpr Place place(int L, int heads, int group, int items) {
   return {first + p.head, p.item};
 }
 
-// The same for groups of 8 heads in a launch of `split` shares of all items (the share is the slowest index, so that a head stays
-// on its XCDs).
+// A launch of `split` shares of all items (the share is the slowest index, so that a head stays on its XCDs): heads in groups of `group` (a
+// multiple of 8), as above; then a last group of 8 `whole` heads and the `rest` in eighths, all of them at once: an XCD has `whole` heads and
+// `rest` units, and takes eight items of each of the former and one of each of the latter in turn.
+struct Groups { int group, whole, rest; };
 struct PlaceOfEight {
-  int heads, items, split, per_share;      // workgroups of a share
-  Divisor per_group, left;                 // 8 items; heads % 8
+  int split, per_share;                    // per_share: workgroups of a share
+  int first, first_ids, group, items;      // heads in groups of `group`, their linear ids
+  int whole, rest;
+  Divisor per_group, in_group;             // group items; group
+  Divisor per_rank, in_rank;               // 8 whole + rest; whole
   constexpr Place of(int L, int& share) const {
     for (share = 0; share + 1 < split && L >= per_share; ++share) L -= per_share;
-    const int grp = heads < XCDS ? 0 : (int)per_group.of((unsigned)L), whole = heads / XCDS;
-    if (__builtin_expect(grp < whole, 1)) { const int l = L - grp * XCDS * items; return {XCDS * grp + l % XCDS, l / XCDS}; }
-    const int rest = heads % XCDS, l = L - whole * XCDS * items, x = l % XCDS, i = l / XCDS;
-    const int rank = (int)left.of((unsigned)i), unit = rest * x + (i - rank * rest);
-    return {whole * XCDS + unit / XCDS, rank * XCDS + unit % XCDS};
+    if (__builtin_expect(L < first_ids, 1)) {
+      const int grp = (int)per_group.of((unsigned)L), l = L - grp * group * items, item = (int)in_group.of((unsigned)l);
+      return {group * grp + l - item * group, item};
+    }
+    L -= first_ids;
+    const int x = L % XCDS, i = L / XCDS, rank = (int)per_rank.of((unsigned)i), k = i - rank * (XCDS * whole + rest);
+    if (k < XCDS * whole) {
+      const int j = (int)in_rank.of((unsigned)k);
+      return {first + XCDS * (k - j * whole) + x, rank * XCDS + j};
+    }
+    const int unit = rest * x + k - XCDS * whole;
+    return {first + XCDS * whole + unit / XCDS, rank * XCDS + unit % XCDS};
   }
 };
-constexpr PlaceOfEight place_of_eight(int heads, int items, int split) {
-  const int n = placed(heads, XCDS, items);
-  return {heads, items, split, n, divisor((unsigned)(XCDS * items), (uint64_t)n), divisor(heads % XCDS ? (unsigned)(heads % XCDS) : 1u, (uint64_t)n)};
+constexpr PlaceOfEight place_of_eight(int heads, int items, int split, Groups g) {
+  const int first = heads - XCDS * g.whole - g.rest, ids = first * items, per_rank = XCDS * g.whole + g.rest;
+  const int n = ids + XCDS * per_rank * ((items + XCDS - 1) / XCDS);
+  auto by = [&](int d) { return divisor(d > 0 ? (unsigned)d : 1u, (uint64_t)n); };
+  return {split, n, first, ids, g.group, items, g.whole, g.rest, by(g.group * items), by(g.group), by(per_rank), by(g.whole)};
+}
+constexpr PlaceOfEight place_of_eight(int heads, int items, int split) { return place_of_eight(heads, items, split, Groups{XCDS, 0, heads % XCDS}); }
+
+// The groups for kernels whose workgroups walk a list each: as many heads per XCD at once as its L2 (4 MB) holds the K and V (or Q and dO) of,
+// at most 8.  With one head per XCD a causal mask's last heads start their longest lists when the short ones of the heads before have
+// ended, and these are all that is left in the end; with more than the L2 holds the sparse uniform masks get slower.
+// us, bf16, a forward / its training step, 8 heads at a time and so; block-causal, causal keep 0.25, keep 0.2, dense:
+//   D = 64    16 heads N = 4096    55 / 263 ->  54 / 232    27 / 103 ->  24 /  93    32 / 112 ->  31 / 110    91 /  362 ->  91 /  361
+//             10 heads N = 4096    45 / 162 ->  36 / 138    21 /  72 ->  17 /  72    25 /  81 ->  24 /  79    70 /  262 ->  70 /  262
+//   D = 128   32 heads N = 4096   180 / 712 -> 152 / 647    62 / 268 ->  58 / 263    76 / 321 ->  77 / 323   305 / 1222 -> 306 / 1225
+//             64 heads N = 2048   102 / 412 ->  82 / 353    41 / 166 ->  37 / 152    47 / 200 ->  48 / 197   151 /  656 -> 151 /  657
+//             24 heads N = 2048    56 / 190 ->  47 / 163    26 /  88 ->  21 /  81    28 / 104 ->  24 /  98    63 /  259 ->  64 /  260
+//   D = 256   16 heads N = 2048    63 / 261 ->  56 / 248    30 / 122 ->  26 / 118    33 / 148 ->  29 / 141    77 /  360 ->  77 /  358
+// More than the L2 holds, 32 heads at once in place of 8:
+//   D = 128   32 heads N = 8192 (4 MB)   forward 560 -> 546   177 -> 177   251 -> 329      D = 256   32 heads N = 4096 (4 MB)   292 -> 288   107 -> 119   142 -> 192
+constexpr Groups groups_of_heads(int heads, int64_t N, int D) {
+  const int64_t fit = (4ll << 20) / (4 * N * D);
+  const int per_xcd = heads / XCDS, rest = heads % XCDS, most = fit < 1 ? 1 : fit > 8 ? 8 : (int)fit;
+  int n = per_xcd < most ? per_xcd : most;       // (like groups)
+  while (n > 1 && per_xcd % n != 0) --n;
+  return {XCDS * (n > 1 ? n : 1), rest > 0 ? n : 0, rest};
 }
 
 // ---- W ranges per head, all resident at once ----

@@ -35,6 +35,34 @@ int main() {
           if (n > heads / XCDS + 2) return bad("heads of an XCD", heads, group, items);
         }
       }
+  // (the groups that the L2 holds: every item once, an XCD on as few heads as at once, the items of a group in ascending order)
+  for (int heads = 1; heads <= 100; ++heads)
+    for (int D : {64, 128, 256})
+      for (int items : {1, 3, 8, 9, 16, 47, 64, 128, 274}) {
+        const Groups g = groups_of_heads(heads, 64 * items, D);
+        const PlaceOfEight e = place_of_eight(heads, items, 2, g);
+        if (g.group % XCDS != 0 || g.rest != heads % XCDS || (heads - XCDS * g.whole - g.rest) % g.group != 0) return bad("groups", heads, items, D);
+        for (int share = 0; share < 2; ++share) {
+          std::vector<int> seen(heads * items);
+          std::vector<std::vector<int>> last(XCDS, std::vector<int>(heads, -1));
+          for (int L = 0; L < e.per_share; ++L) {
+            int got = -1;
+            const Place p = e.of(L + share * e.per_share, got);
+            if (got != share) return bad("share", heads, items, D);
+            if (p.item >= items) continue;
+            if (p.head < 0 || p.head >= heads || p.item < 0 || seen[p.head * items + p.item]++) return bad("of a group", heads, items, D);
+            if (last[L % XCDS][p.head] >= p.item) return bad("order", heads, items, D);
+            last[L % XCDS][p.head] = p.item;
+          }
+          for (int n : seen) if (n != 1) return bad("not of a group", heads, items, D);
+          if (e.per_share % XCDS != 0) return bad("ids", heads, items, D);
+          for (auto& x : last) {
+            int n = 0;
+            for (int i : x) n += i >= 0;
+            if (n > heads / XCDS + 2) return bad("heads on an XCD", heads, items, D);
+          }
+        }
+      }
   for (unsigned d : {1u, 2u, 3u, 5u, 6u, 7u, 8u, 24u, 513u, 2192u, 65535u, 1u << 20})
     for (uint64_t most : {10ull, 1000ull, 65535ull, 1ull << 20, 1ull << 31}) {
       const Divisor v = divisor(d, most);
