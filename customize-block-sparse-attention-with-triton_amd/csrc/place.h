@@ -96,12 +96,18 @@ constexpr PlaceOfEight place_of_eight(int heads, int items, int split) { return 
 //             64 heads N = 2048   102 / 412 ->  82 / 353    41 / 166 ->  37 / 152    47 / 200 ->  48 / 197   151 /  656 -> 151 /  657
 //             24 heads N = 2048    56 / 190 ->  47 / 163    26 /  88 ->  21 /  81    28 / 104 ->  24 /  98    63 /  259 ->  64 /  260
 //   D = 256   16 heads N = 2048    63 / 261 ->  56 / 248    30 / 122 ->  26 / 118    33 / 148 ->  29 / 141    77 /  360 ->  77 /  358
-// More than the L2 holds, 32 heads at once in place of 8:
-//   D = 128   32 heads N = 8192 (4 MB)   forward 560 -> 546   177 -> 177   251 -> 329      D = 256   32 heads N = 4096 (4 MB)   292 -> 288   107 -> 119   142 -> 192
+// Half as much again where these are all heads (block-causal, causal keep 0.5, keep 0.25, 0.1):
+//   D = 128   16 heads N = 6016 (3 MB)   176 / 737 -> 160 / 692    98 / 414 ->  90 / 387   103 / 425 -> 102 / 419    53 / 208 -> 52 / 209
+//   D = 256   16 heads N = 3000          94 / 455 ->  88 / 452     57 / 275 ->  54 / 262    62 / 293 ->  61 / 276    39 / 171 -> 38 / 169
+// With twice as much the causal launches gain and the sparse uniform ones lose:
+//   D = 128   32 heads N = 8192 (4 MB)   560 / 2454 -> 557 / 2419  177 / 762 -> 167 / 741  251 / 1091 -> 267 / 1140 150 / 644 -> 154 / 651   (keep 0.25, causal and not)
+//   D = 256   16 heads N = 4096          150 / 717 -> 150 / 705    88 / 424 ->  84 / 404    96 / 461 ->  97 / 452    58 / 274 -> 61 / 277
+// (A choice by the lists, in the kernels, costs the backward's registers: 8 heads N = 4096 D = 128 dense 334 -> 345.)
 constexpr Groups groups_of_heads(int heads, int64_t N, int D) {
-  const int64_t fit = (4ll << 20) / (4 * N * D);
+  const int64_t bytes = 4 * N * D, fit = (4ll << 20) / bytes;
   const int per_xcd = heads / XCDS, rest = heads % XCDS, most = fit < 1 ? 1 : fit > 8 ? 8 : (int)fit;
   int n = per_xcd < most ? per_xcd : most;       // (like groups)
+  if (rest == 0 && per_xcd <= 8 && 10 * per_xcd * bytes <= (64ll << 20)) n = per_xcd;
   while (n > 1 && per_xcd % n != 0) --n;
   return {XCDS * (n > 1 ? n : 1), rest > 0 ? n : 0, rest};
 }
