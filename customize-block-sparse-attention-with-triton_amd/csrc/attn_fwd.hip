@@ -1494,8 +1494,6 @@ static int pair_split(int B, int H, int N, int D, bool compact) {
 // 2 pairs / 4 pairs / 4 pairs and 2 shares; keep 0.1, 0.3, 1, block-causal (fp16 the first five, bf16 the others):
 //    5 heads N = 512 (40 row blocks)   11 /  8 /  8 / 10     11 /  8 /  8 / 10     12 /  8 /  8 / 10     11 /  8 /  8 / 10
 //    8 heads N = 2048 (256)            13 /  9 /  9 / 19     16 / 12 / 11 / 21     20 / 19 / 17 / 27     19 / 18 / 16 / 22
-//    1 head  N = 4096 (64; 4 shares 12, 12, 15, 15)  13 / 10 / 10 / 12   16 / 15 / 13 / 13   22 / 30 / 25 / 19   23 / 29 / 24 / 18
-//    1 head  N = 6400 (100)            17 / 12 / 11 / 13     21 / 20 / 18 / 17     27 / 43 / 36 / 26     24 / 43 / 35 / 24
 //    2 heads N = 8192 (256)            17 / 15 / 14 / 21     27 / 26 / 23 / 30     53 / 55 / 44 / 57     38 / 54 / 44 / 35
 //   16 heads N = 3072 (768)            22 / 18 / 21          32 / 28 / 32          59 / 56 / 60          42 / 34 / 40
 //   32 heads N = 3072 (1536)           30 / 27 / 40          52 / 47 / 61         101 /103 /126          65 / 62 / 81
@@ -1505,12 +1503,27 @@ static int pair_split(int B, int H, int N, int D, bool compact) {
 //    3 heads N = 6400 (300)            20 / 15 / 17          29 / 29 / 30          50 / 65 / 73          37 / 48 / 37   (nor there)
 //    5 heads N = 6400 (500)            26 / 16 / 20          41 / 30 / 34          73 / 71 / 75          46 / 51 / 45
 //    1 head  N = 10048 (157)           19 / 16 / 13 / 20     26 / 30 / 25 / 30     44 / 72 / 55 / 64     32 / 71 / 53 / 35   (nor there)
+// Shares of a list, that meet in the launch (kernel time and launch among others, fp16), of at least 8 tiles: none / 2 / 3 / 4 (and 4 of at
+// least one tile); keep 0.1, 0.3, dense, block-causal:
+//    1 head  N = 1024 (16)              5.7/ 5.9/ 5.8/ 5.7 ( 8.3)    7.0/ 7.1/ 7.1/ 7.1 ( 9.1)    9.5/10.0/10.0/10.1 ( 9.8)    9.3/ 9.4/ 9.5/ 9.6 ( 9.6)    (not there)
+//    1 head  N = 1536 (24)              6.4/ 6.5/ 6.5/ 6.5 ( 8.9)    8.6/ 8.6/ 8.6/ 8.6 ( 9.3)   11.9/11.3/10.5/10.6 (10.5)   11.7/10.8/10.6/10.9 (10.2)
+//    1 head  N = 4096 (64)              8.0/ 8.2/ 8.2/ 8.2 ( 9.8)   12.9/11.8/11.2/11.2 (11.0)   24.0/17.7/15.4/14.6 (14.8)   23.6/17.1/14.4/13.2 (13.2)
+//    1 head  N = 5120 (80)              9.0/ 9.1/ 9.1/ 9.1 (13.4)   14.8/12.9/11.5/16.7 (16.6)   28.8/20.3/17.4/24.7 (24.7)   28.4/19.4/16.4/17.4 (17.3)
+//    5 heads N = 1536 (120)             6.5/ 6.7/ 6.7/ 6.7 (14.7)    9.0/ 9.0/ 9.0/ 9.0 (14.4)   12.0/12.0/17.0/16.9 (16.7)   11.9/11.2/11.3/11.3 (15.2)   (nor there)
+//    4 heads N = 2048 (128)             7.1/ 7.3/ 7.3/ 7.3 (14.4)   10.6/10.5/10.6/10.6 (15.0)   14.7/13.6/18.6/18.3 (18.1)   14.5/12.5/15.7/16.9 (16.0)
+//    1 head  N = 8192 (128)            11.2/10.9/10.9/10.9 (15.4)   21.4/16.8/22.0/20.8 (21.0)   44.0/29.6/39.1/34.4 (34.3)   42.9/27.2/27.2/27.9 (28.5)
+//    3 heads N = 5120 (240)             9.2/10.1/11.4/12.7 (23.5)   17.4/22.3/27.5/31.4 (29.4)   31.0/38.3/43.3/46.9 (47.2)   29.3/25.9/30.2/32.4 (32.6)   (nor there)
+// (With bf16 from 56 row blocks on also the shortest lists are shared: a share's first tiles have exact largest numerators, without which its
+// rows are further from 64 bits.)
 struct ShortPlan { int pairs, split; };
 static ShortPlan short_plan(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
   if (nb > SHORT_MAX_BLOCKS) return {0, 1};
   // long lists: as many shares as fill the GPU
-  if (rows <= 256) return {4, nb < 56 || rows > 128 ? 1 : rows > 64 ? 2 : 4};
+  if (rows <= 256) {
+    const int split = rows > 128 ? 1 : rows > 85 ? 2 : rows > 64 ? 3 : 4;       // (workgroups of 4 pairs are alone on their compute unit)
+    return {4, nb < (split == 4 ? 20 : 28) ? 1 : split};
+  }
   const bool takes = nb <= 48 ? rows <= 1792 : nb <= 64 ? rows <= 1024 : rows >= 400 && rows <= 512;
   return {takes ? 2 : 0, 1};
 }
@@ -1581,7 +1594,7 @@ size_t coop_workspace_bytes(int B, int H, int N, int D, bool compact) {
     return compact ? bytes(false) : std::max(bytes(false), bytes(true));       // (compact launches: block masks only)
   }
   const int nb = (N + 63) / 64;
-  if (const ShortPlan plan = short_plan((int64_t)B * H * nb, nb); plan.pairs > 0) return pair_parts_bytes(B, H, N, D, plan.split);
+  if (const ShortPlan plan = short_plan((int64_t)B * H * nb, nb); plan.pairs > 0) return quad_parts_bytes(B, H, nb, 64, plan.split);
   const int mode = fwd_mode(B, H, nb, compact);
   const int W = groups_per_head(B, H, nb, mode, compact);
   return W == 0 ? 256 : parts_bytes(B, H, nb, W, mode);      // (0: nothing is shared)
@@ -1726,7 +1739,14 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
     prm.part_o = (float*)ws + 64;
     prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
     prm.part_len = (int*)(prm.part_ml + (size_t)prm.split * heads * s.N * 2);
-    if (s.D == 64) launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
+    if (s.D == 64) {
+      const size_t parts = (size_t)heads * prm.nb * prm.split * 64;
+      prm.part_ml = prm.part_o + parts * 64;
+      prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
+      prm.epoch = next_epoch();
+      prm.share_tiles = dt != 0 && prm.nb >= 56 ? 1 : 8;      // (short_plan)
+      launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
+    }
     else launch_fwd_pair(prm, dt, tile_bits != nullptr, st);
     return launch_status();
   }

@@ -352,12 +352,13 @@ __global__ __launch_bounds__(128, 2) void fwd_pair_kernel(const FwdParams prm) {
 // waited for another's and rows were found by 64-bit divisions: 2 heads of N = 4096, D = 256, 8 shares 21.8 -> 14.9 us (71 MB:
 // 4.8 TB/s); 8 heads of N = 4000, D = 128, 2 shares, the whole training step 136.9 -> 132.3.
 template <bool BF16, int S>
-__global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm, int D, unsigned quads) {
+__global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm, unsigned quads) {
+  constexpr int D = PAIR_D, QSHIFT = 5;                      // log2 of the threads per query row
+  static_assert(D == 4 << QSHIFT, "four values per thread");
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
   if (i >= quads) return;
-  const int qshift = D == 128 ? 5 : 4;                       // log2 of the threads per query row
-  const unsigned rowg = i >> qshift;                         // row over all heads
-  const int col = (int)(i & ((1u << qshift) - 1)) * 4;
+  const unsigned rowg = i >> QSHIFT;                         // row over all heads
+  const int col = (int)(i & ((1u << QSHIFT) - 1)) * 4;
   const int bh = (int)(rowg / (unsigned)prm.N), row = (int)(rowg - (unsigned)bh * prm.N);
   const int b = bh / prm.H, h = bh % prm.H, BH = prm.B * prm.H;
   const int len = prm.part_len[bh * prm.nb + row / 64];
@@ -393,19 +394,14 @@ __global__ __launch_bounds__(256) void pair_sum_parts_kernel(const FwdParams prm
 }
 
 // (one thread per 4 results of a launch that shares lists, which has fewer than 2 row blocks per compute unit: 64 D / 4 threads each,
-// 2 048 at most, so the values fit 32 bits.  D: 64 or 128.)
+// 2 048 at most, so the values fit 32 bits.)
 template <bool BF16, int S = 2>
-static void launch_sum_parts_t(const FwdParams& prm, int D, hipStream_t st) {
+static void launch_sum_parts_t(const FwdParams& prm, hipStream_t st) {
   if constexpr (S < 4) {
-    if (prm.split != S) { launch_sum_parts_t<BF16, S + 1>(prm, D, st); return; }
+    if (prm.split != S) { launch_sum_parts_t<BF16, S + 1>(prm, st); return; }
   }
-  const unsigned quads = (unsigned)((int64_t)prm.B * prm.H * prm.N * D / 4);
-  hipLaunchKernelGGL((pair_sum_parts_kernel<BF16, S>), dim3((quads + 255) / 256), dim3(256), 0, st, prm, D, quads);
-}
-
-void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st) {
-  if (bf16) launch_sum_parts_t<true>(prm, D, st);
-  else launch_sum_parts_t<false>(prm, D, st);
+  const unsigned quads = (unsigned)((int64_t)prm.B * prm.H * prm.N * PAIR_D / 4);
+  hipLaunchKernelGGL((pair_sum_parts_kernel<BF16, S>), dim3((quads + 255) / 256), dim3(256), 0, st, prm, quads);
 }
 
 template <int DT, bool EW, bool TAIL>
@@ -423,7 +419,7 @@ static void launch_pair_t(const FwdParams& prm, hipStream_t st) {
   const int grid = prm.place.per_share * prm.split;
   if (prm.N % 64 != 0) launch_pair_c<DT, EW, true>(prm, grid, st);
   else launch_pair_c<DT, EW, false>(prm, grid, st);
-  if (!EW && prm.split > 1) launch_sum_parts(prm, PAIR_D, DT != 0, st);
+  if (!EW && prm.split > 1) launch_sum_parts_t<DT != 0>(prm, st);
 }
 
 template <bool EW>

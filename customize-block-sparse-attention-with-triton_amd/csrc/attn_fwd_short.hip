@@ -19,6 +19,19 @@
 
 namespace bsattn {
 
+constexpr int SHARING_PAIRS = 4, SHARING_MOST = 4;      // pairs of the workgroups that share lists; shares of a list, at most
+
+// Two quads of each of four parts, 8 KB apart, and the wait for them in one statement (kernel_util.h, coherent_load4x4).
+__device__ __forceinline__ void coherent_load_pairs(const float* a, const float* b, const float* c, const float* d, floatx4 (&x)[4][2]) {
+  asm volatile("global_load_dwordx4 %0, %8, off sc1\n\tglobal_load_dwordx4 %1, %9, off sc1\n\t"
+               "global_load_dwordx4 %2, %10, off sc1\n\tglobal_load_dwordx4 %3, %11, off sc1\n\t"
+               "global_load_dwordx4 %4, %12, off sc1\n\tglobal_load_dwordx4 %5, %13, off sc1\n\t"
+               "global_load_dwordx4 %6, %14, off sc1\n\tglobal_load_dwordx4 %7, %15, off sc1\n\t"
+               "s_waitcnt vmcnt(0)"
+               : "=&v"(x[0][0]), "=&v"(x[0][1]), "=&v"(x[1][0]), "=&v"(x[1][1]), "=&v"(x[2][0]), "=&v"(x[2][1]), "=&v"(x[3][0]), "=&v"(x[3][1])
+               : "v"(a), "v"(a + 2048), "v"(b), "v"(b + 2048), "v"(c), "v"(c + 2048), "v"(d), "v"(d + 2048) : "memory");
+}
+
 // S: pairs of wavefronts per workgroup.  Lists of at most SHORT_MAX_BLOCKS tiles.
 template <int S, bool EW> struct ShortCfg {
   static constexpr int TILE_BYTES = 64 * 128;
@@ -35,7 +48,8 @@ template <int S, bool EW> struct ShortCfg {
 // DT: 0 fp16; 1 bf16 with P rounded to fp16 (V fragments converted); 2 bf16 with P rounded to bf16.
 // TAIL: N is not a multiple of 64 (as in attn_fwd.hip: the copy of the last tile repeats its last key, the scores beyond
 // it are -inf, the queries beyond N are not written).
-template <int S, int DT, bool EW, bool TAIL>
+// SHARED: lists are shared by workgroups (a variant of its own: the code, even where it is jumped over, costs a launch of one short head 0.3 us).
+template <int S, int DT, bool EW, bool TAIL, bool SHARED>
 __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams prm) {
   using C = ShortCfg<S, EW>;
   constexpr int D = 64, KS = D / 16, DB = D / 32, CPR = D / 8, ROWB = 2 * D, HALF = CPR / 2, RPI = 64 / CPR;
@@ -44,7 +58,7 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = wave >> 1, w = wave & 1;
   const int ln = lane & 31, g = lane >> 5;
-  const int nb = prm.nb, BH = prm.B * prm.H;
+  const int nb = prm.nb;
   int chunk;
   const Place p = prm.place.of(blockIdx.x, chunk);
   const int bh = p.head, m = nb - 1 - p.item;
@@ -65,12 +79,13 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   int t0, t1;
   if (listed) { t0 = rp[m]; t1 = rp[m + 1]; }
   else { t0 = 0; t1 = columns_of_row<SHORT_MAX_BLOCKS>(prm, b, h, m, lane, lcols, chunk == 0 && wave == 0); }
-  if (prm.split > 1) {                            // this workgroup's share of the row block's list
+  int shares = 1;
+  if constexpr (SHARED) {                         // this workgroup's share of the row block's list
     const int len = t1 - t0;
-    if (chunk == 0 && threadIdx.x == 0) prm.part_len[bh * nb + m] = len;
-    t1 = t0 + (int)((int64_t)len * (chunk + 1) / prm.split);
-    t0 = t0 + (int)((int64_t)len * chunk / prm.split);
-    if (t0 == t1) return;                         // (pair_sum_parts_kernel knows which shares are empty)
+    shares = len >= prm.split * prm.share_tiles ? prm.split : len < 2 * prm.share_tiles ? 1 : len / prm.share_tiles;
+    if (chunk >= shares) return;
+    t1 = t0 + (int)((int64_t)len * (chunk + 1) / shares);
+    t0 = t0 + (int)((int64_t)len * chunk / shares);
   }
   const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64, tail_cb = TAIL ? nb - 1 : -1;
   const unsigned short* kg = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1];
@@ -257,6 +272,9 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   // ---- merge the pairs: every wavefront's 32 rows into its pair's stages, then 4 consecutive columns of a row per thread ----
   const float lsum = l_i + __shfl_xor(l_i, 32);
   float* ml = reinterpret_cast<float*>(lds + C::ML_OFF);
+  unsigned long long* arrivals = prm.flags + (int64_t)bh * nb + m;
+  unsigned long long seen = 0ull;      // (the read travels beside the merge)
+  if (SHARED && shares > 1 && threadIdx.x == 0) seen = __hip_atomic_load(arrivals, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();           // everybody has left the last step
   {
     float* own = reinterpret_cast<float*>(mine) + (32 * w + ln) * C::PITCH + 4 * g;
@@ -274,13 +292,12 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   }
   __syncthreads();
   void* obase = out_base(prm, b, h);
-#pragma unroll
-  for (int i = threadIdx.x; i < 64 * 16; i += 128 * S) {
+  auto merge = [&](int i, float& M, float& L) {      // quad i: row i / 16, columns 4 (i % 16) .. + 3
     const int r = i >> 4, col = (i & 15) * 4;
-    const int64_t q = (int64_t)m * 64 + r;
-    if (TAIL && q >= prm.N) break;
-    float mp[S], lp[S], M = -INFINITY, L = 0.f;
+    float mp[S], lp[S];
     floatx4 acc = {0.f, 0.f, 0.f, 0.f}, part[S];
+    M = -INFINITY;
+    L = 0.f;
 #pragma unroll
     for (int cc = 0; cc < S; ++cc) {
       mp[cc] = ml[(cc * 64 + r) * 2];
@@ -296,27 +313,93 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] += wgt * part[cc][e];
     }
-    if (prm.split > 1) {     // unnormalised fp32 part with its reference exponent and row sum
-      const int64_t at = ((int64_t)chunk * BH + bh) * prm.N + q;
-      *reinterpret_cast<floatx4*>(prm.part_o + at * D + col) = acc;
-      if (col == 0) { prm.part_ml[at * 2] = M; prm.part_ml[at * 2 + 1] = L; }
-    } else {
-      const float inv = EW || steps == 0 ? row_inverse<true>(L) : row_inverse<false>(L);     // (no kept tile or no key: O = 0)
-      store_out4<BF16>(obase, q * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
-      if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + q] = row_lse(M, L);
+    return acc;
+  };
+  auto put = [&](int i, const floatx4& acc, float M, float L) {
+    const int col = (i & 15) * 4;
+    const int64_t q = (int64_t)m * 64 + (i >> 4);
+    if (TAIL && q >= prm.N) return;
+    const float inv = EW || steps == 0 ? row_inverse<true>(L) : row_inverse<false>(L);     // (no kept tile or no key: O = 0)
+    store_out4<BF16>(obase, q * prm.os[2] + col, prm.out_f32, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+    if (col == 0 && prm.lse != nullptr) prm.lse[(int64_t)bh * prm.N + q] = row_lse(M, L);
+  };
+  if constexpr (SHARED) {
+    if (shares > 1) {
+      // The shares of a list meet in the workspace, as the parts of a row block do in attn_fwd.hip: each is published with device-scope
+      // stores and counted in once these are acknowledged, the last one in asks for all of them at once and adds them up in their order.
+      // (A launch that summed the parts took 1 to 2 us more: 1 head N = 6400 keep 0.3 18.6 -> 16.7 us, N = 4096 bf16 keep 0.1 12.7 -> 11.1, dense
+      // 17.2 -> 16.4, 2 heads N = 4000 causal keep 0.25 14.0 -> 12.1, N = 8192 token window of 2048 17.3 -> 15.0.)
+      constexpr int HALF_QUADS = 64 * 16 / 2;
+      static_assert(128 * S == HALF_QUADS && SHARING_MOST == 4, "two quads per thread, four shares at most");
+      const int i = threadIdx.x, r = i >> 4;
+      const int64_t first = ((int64_t)bh * nb + m) * prm.split;
+      auto slot = [&](int p) { return prm.part_o + (first + p) * (64 * D) + 4 * i; };
+      auto ml_of = [&](int p) { return prm.part_ml + (first + p) * 128 + 2 * r; };
+      float M[2], L[2];
+      const floatx4 x0 = merge(i, M[0], L[0]), x1 = merge(i + HALF_QUADS, M[1], L[1]);
+      coherent_store4(slot(chunk), x0[0], x0[1], x0[2], x0[3]);
+      coherent_store4(slot(chunk) + 4 * HALF_QUADS, x1[0], x1[1], x1[2], x1[3]);
+      if ((i & 15) == 0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) { coherent_store(ml_of(chunk) + 64 * j, M[j]); coherent_store(ml_of(chunk) + 64 * j + 1, L[j]); }
+      }
+      wait_vm<0>();
+      __syncthreads();                                   // (and all have read the pairs' results)
+      if (threadIdx.x == 0) lcols[0] = count_in(arrivals, prm.epoch, seen);
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(*(volatile int*)lcols) != shares) return;
+      float mp[SHARING_MOST][2], lp[SHARING_MOST][2];
+      floatx4 part[SHARING_MOST][2];
+#pragma unroll
+      for (int p = 0; p < SHARING_MOST; ++p)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float* at = ml_of(p < shares ? p : 0) + 64 * j;
+          mp[p][j] = coherent_load(at);
+          lp[p][j] = p < shares ? coherent_load(at + 1) : 0.f;
+        }
+      coherent_load_pairs(slot(0), slot(1), slot(shares > 2 ? 2 : 0), slot(shares > 3 ? 3 : 0), part);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        float Ms = -INFINITY, Ls = 0.f;
+        floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+        // (a share without mass is one whose sum is zero: a sum that is not a number goes into the result like any other)
+#pragma unroll
+        for (int p = 0; p < SHARING_MOST; ++p) Ms = lp[p][j] != 0.f ? fmaxf(Ms, mp[p][j]) : Ms;
+#pragma unroll
+        for (int p = 0; p < SHARING_MOST; ++p) {
+          if (lp[p][j] == 0.f) continue;
+          const float wgt = __builtin_amdgcn_exp2f(mp[p][j] - Ms);
+          Ls += wgt * lp[p][j];
+          acc += wgt * part[p][j];
+        }
+        put(i + j * HALF_QUADS, acc, Ms, Ls);
+      }
+      // back to zero, so that a replay of this launch (same mark) starts from a clean counter
+      if (threadIdx.x == 0) __hip_atomic_store(arrivals, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
     }
+  }
+#pragma unroll
+  for (int i = threadIdx.x; i < 64 * 16; i += 128 * S) {
+    float M, L;
+    const floatx4 acc = merge(i, M, L);
+    put(i, acc, M, L);
   }
 }
 
-template <int S, int DT, bool EW, bool TAIL>
+template <int S, int DT, bool EW, bool TAIL, bool SHARED = false>
 static void launch_short_t(const FwdParams& prm, hipStream_t st) {
+  if constexpr (S == SHARING_PAIRS && !SHARED) {
+    if (prm.split > 1) { launch_short_t<S, DT, EW, TAIL, true>(prm, st); return; }
+  }
   constexpr int LDS = ShortCfg<S, EW>::LDS_BYTES;
   static std::atomic<unsigned long long> configured{0};   // raising the dynamic LDS limit is idempotent
   once_per_device(configured, [] {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_short_kernel<S, DT, EW, TAIL>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_short_kernel<S, DT, EW, TAIL, SHARED>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
   });
   const int grid = prm.place.per_share * prm.split;
-  hipLaunchKernelGGL((fwd_short_kernel<S, DT, EW, TAIL>), dim3(grid), dim3(128 * S), LDS, st, prm);
+  hipLaunchKernelGGL((fwd_short_kernel<S, DT, EW, TAIL, SHARED>), dim3(grid), dim3(128 * S), LDS, st, prm);
 }
 
 template <int S, int DT>
@@ -333,13 +416,10 @@ static void launch_short_s(const FwdParams& prm, int dt, bool elementwise, hipSt
   else launch_short_d<S, 2>(prm, elementwise, st);
 }
 
-void launch_sum_parts(const FwdParams& prm, int D, bool bf16, hipStream_t st);   // attn_fwd_pair.hip
-
 // pairs: 2 or 4 per workgroup.  dt: 0 fp16, 1 bf16 with P rounded to fp16 (V converted), 2 bf16 with P rounded to bf16.
 void launch_fwd_short(const FwdParams& prm, int pairs, int dt, bool elementwise, hipStream_t st) {
   if (pairs == 2) launch_short_s<2>(prm, dt, elementwise, st);
   else launch_short_s<4>(prm, dt, elementwise, st);
-  if (prm.split > 1) launch_sum_parts(prm, 64, dt != 0, st);
 }
 
 }  // namespace bsattn

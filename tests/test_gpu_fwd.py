@@ -165,7 +165,7 @@ def test_lists_cache_follows_the_mask(dev):
 
 
 def test_workspace_contents_do_not_matter(dev):
-    """Row blocks shared between workgroups leave their parts in the workspace, which a second launch sums: stale or random
+    """Row blocks shared between workgroups leave their parts in the workspace, which the last one in sums: stale or random
     workspace contents, and repeated runs on the same workspace, must give the same result."""
     import fa2_custom_mask as fm
     N, D = 4096, 64

@@ -47,7 +47,7 @@ def replay_and_compare(dev, B, H, N, D, dtype, mask, seed, replays=4):
 
 
 def test_replay_d64_rows_shared_between_workgroups(dev):
-    """One head, 64 row blocks: four shares of a row block's list, whose parts a second launch sums."""
+    """One head, 64 row blocks: up to four shares of a row block's list, whose parts the last one in sums."""
     replay_and_compare(dev, 1, 1, 4096, 64, torch.float16, uniform_block_mask(1, 1, 64, 0.6, 3001), 3002)
 
 

@@ -27,7 +27,7 @@ CASES = [
     # B, H, N, D, keep (1.0: dense), dtype
     (1, 1, 17536, 64, 1.0, torch.float16),      # every row block is shared by about two workgroups
     (1, 1, 17536, 64, 0.1, torch.float16),
-    (1, 2, 4096, 64, 0.5, torch.bfloat16),      # two shares of a row block's list, summed by a second launch
+    (1, 2, 4096, 64, 0.5, torch.bfloat16),      # shares of a row block's list, summed by the last one in
     (1, 1, 8192, 128, 0.5, torch.float16),      # shares of a list at D = 128, summed by the last one in
     (1, 1, 2048, 256, 1.0, torch.float16),      # ... and at D = 256
     (1, 2, 8256, 64, 0.5, torch.bfloat16),      # ranges of workgroups, two heads

@@ -164,3 +164,36 @@ def test_ranges_of_wavefronts(dev, B, H, N, dtype, out_fp32, seed):
         for h in (0, H - 1):
             s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~tokens[0, 0], float("-inf"))
             assert rel_l2(o[0, h], torch.softmax(s, -1) @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
+
+
+# Few row blocks at D = 64: shares of a list that meet in the launch, two, three or four at most, of at least 8 tiles (bf16 from 56 row
+# blocks on: of one).  Row block r keeps r tiles (modulo the row blocks), so that every length is there, none and all among them.
+@pytest.mark.parametrize("H,N,dtype,out_fp32", [(1, 1536, torch.float16, False), (1, 3600, torch.bfloat16, True), (1, 5120, torch.float16, True),
+                                               (1, 5100, torch.bfloat16, False), (2, 4096, torch.float16, False), (1, 8190, torch.bfloat16, True)])
+def test_shares_of_every_length(dev, H, N, dtype, out_fp32):
+    import fa2_custom_mask as fm
+    assert fwd_route_d64(1, H, N) == "pairs"
+    nb = (N + 63) // 64
+    g = torch.Generator(device=dev).manual_seed(N)
+    q, k, v = [torch.randn(1, H, N, 64, generator=g, device=dev).to(dtype) for _ in range(3)]
+    order = torch.rand(nb, nb, generator=g, device=dev).argsort(1).argsort(1)
+    mask = (order < ((torch.arange(nb, device=dev) * 7) % (nb + 1))[:, None])[None, None]
+    mask[0, 0, 3] = True
+    mask[0, 0, 4] = False
+    o_ref, lse_ref = naive_forward(q, k, v, mask, 0.125)
+    bar = 3e-3 if (dtype == torch.bfloat16 and not out_fp32) else 1e-3
+    none = torch.isinf(lse_ref)
+    first = None
+    for step in range(4):
+        o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, 0.125, out_fp32=out_fp32)
+        assert torch.equal(torch.isinf(lse), none) and bool((o[none] == 0).all())
+        assert rel_l2(o, o_ref) <= bar and float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
+        assert first is None or torch.equal(o, first)
+        first = o
+    tokens = mask.repeat_interleave(64, 2).repeat_interleave(64, 3)[..., :N, :N].clone()
+    tokens[0, 0, 1::2, ::3] = False                        # words: partly set tiles
+    o = fm.flash_attention_custom_mask(q, k, v, tokens, 0.125)
+    for h in (0, H - 1):
+        s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~tokens[0, 0], float("-inf"))
+        p = torch.nan_to_num(torch.softmax(s, -1), nan=0.0)
+        assert rel_l2(o[0, h], p @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
