@@ -133,6 +133,7 @@ void fwd_kernel(const FwdRangeParams prm) {
   HeadSplit hs;
   int snap = 0;
   int64_t x0 = 0, x1 = 0;
+  int r = 0, g0 = 0, g1 = 0;         // COOP: first row block and tiles of the range, g0 < g1 where they are known already
   if constexpr (!ROWS) {
     hs = head_split(rp, nb, prm.W, /*min_tiles=*/ONE ? 4 : NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
     // Long ranges (the regime of the weighted shares) are cut on the axis with gaps and boundaries move to a row
@@ -191,10 +192,36 @@ void fwd_kernel(const FwdRangeParams prm) {
         if (prm.lse != nullptr && threadIdx.x < 64 && (!TAIL || r0 * 64 + (int)threadIdx.x < prm.N)) prm.lse[(int64_t)bh * prm.N + (int64_t)r0 * 64 + threadIdx.x] = -INFINITY;
       }
     }
-    if (hs.T == 0 || wg >= hs.Peff) return;
-    // where the range begins and ends on the cutting axis
-    x0 = split_pos(hs, wg); x1 = split_pos(hs, wg + 1);
-    if (x0 >= x1) return;
+    if (hs.T == 0) return;
+    // Short lists of about the same length, with about as many row blocks as ranges: a workgroup takes a row block.  Nothing has to be searched
+    // for and nothing meets in the workspace, 3 to 8 us of a launch; the ranges balance the work of uneven lists (a causal mask's, told by its
+    // first half of rows) and of few row blocks, and long lists by what the first-comers on a compute unit are faster.  (Not with strided K or
+    // V, where the variant for a number of heads that does not divide 8 would spill registers.)
+    // Ranges / row blocks, fp16, us; tiles of a row block, 3, 8, 16, 32, 48, 64:
+    //   1 head  N = 32000 (500 of 512)   16.1 / 13.6   23.9 / 18.9   29.6 / 24.2   40.5 / 33.2   53.1 / 41.7   55.3 / 51.8    causal, 25: 34.0 / 38.2
+    //   2 heads N = 16064 (251 of 256)   14.7 / 13.7   21.5 / 17.6   28.6 / 22.2   40.1 / 31.4   44.2 / 41.7   52.3 / 50.9    causal, 26: 34.3 / 34.8
+    //   3 heads N = 10048 (157 of 170)   15.9 / 13.5   22.3 / 17.2   28.7 / 22.6   38.6 / 29.9   48.5 / 39.4   49.9 / 47.6    causal, 16: 26.5 / 25.6
+    //   2 heads N = 12032 (188 of 256)   14.8 / 13.1   19.6 / 17.9   20.9 / 20.6   28.1 / 29.2   36.6 / 35.9   45.0 / 44.8    causal, 19: 24.3 / 27.5
+    //   1 head  N = 24000 (375 of 512)   16.2 / 13.4   17.7 / 17.0   22.1 / 22.5   29.3 / 29.6   37.1 / 38.3   45.6 / 45.8    (from 5 tiles on not there)
+    //   1 head  N = 17536 (274 of 512)   14.5 / 12.2   15.4 / 16.3   19.2 / 22.1   25.6 / 29.4   30.1 / 37.6   36.7 / 44.5    (nor there)
+    // (the pointer as a value the compiler cannot trace back: looked up only where needed)
+    auto tiles_to_middle = [&]() {
+      cint_ptr_t p = rp;
+      asm volatile("" : "+s"(p));
+      return p[nb / 2] - hs.lo;
+    };
+    if (MODE == COOP && CONTIG && hs.T <= prm.own_row_tiles && 8 * tiles_to_middle() > 3 * hs.T) {
+      if (wg >= nb) return;
+      r = wg;
+      g0 = rp[wg];
+      g1 = rp[wg + 1];
+      if (g0 >= g1) return;
+    } else {
+      if (wg >= hs.Peff) return;
+      // where the range begins and ends on the cutting axis
+      x0 = split_pos(hs, wg); x1 = split_pos(hs, wg + 1);
+      if (x0 >= x1) return;
+    }
   }
 
   unsigned char* lds_k = lds + w * C::WAVE_LDS;
@@ -911,8 +938,7 @@ void fwd_kernel(const FwdRangeParams prm) {
     // (the nearer one): sharing a row block costs a merge, a published part and a pull, several
     // tiles' worth each, and row blocks of up to 2 `snap` tiles are never shared.  Every workgroup
     // applies the same rule with the same distance to both of its boundaries, so the ranges still tile the list.
-    int r, g0, g1;
-    {
+    if (g0 == g1) {
       // the row blocks in which the two ends of the range lie (positions behind a row block's tiles count as
       // its end), then the tiles themselves
       int c0, c1, s0, e0, s1, e1;
@@ -1761,6 +1787,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.place_quot = prm.place_fast / heads;
   prm.place_rest = prm.place_fast % heads;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
+  prm.own_row_tiles = mode != COOP || prm.nb > prm.W ? 0 : (20 * prm.nb >= 17 * prm.W ? 64 : 4) * prm.nb;
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();

@@ -197,3 +197,29 @@ def test_shares_of_every_length(dev, H, N, dtype, out_fp32):
         s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~tokens[0, 0], float("-inf"))
         p = torch.nan_to_num(torch.softmax(s, -1), nan=0.0)
         assert rel_l2(o[0, h], p @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
+
+
+# Ranges of workgroups, about as many as row blocks, and short lists of like length: a workgroup takes a row block (at most 64 tiles each on
+# average, at most 4 where there are more workgroups).  Both sides of the line, rows without tiles, uneven lists.
+@pytest.mark.parametrize("H,N,tiles,dtype", [(3, 10048, 20, torch.float16), (3, 10048, 63, torch.bfloat16), (3, 10048, 66, torch.float16),
+                                             (2, 16100, 5, torch.float16), (1, 12000, 4, torch.bfloat16), (1, 12000, 5, torch.float16),
+                                             (1, 28000, 12, torch.float16), (7, 4640, 30, torch.bfloat16)])
+@pytest.mark.parametrize("kind", ["even", "causal", "holes"])
+def test_row_blocks_of_workgroups(dev, H, N, tiles, dtype, kind):
+    import fa2_custom_mask as fm
+    assert fwd_route_d64(1, H, N) == "workgroups"
+    nb = (N + 63) // 64
+    g = torch.Generator(device=dev).manual_seed(tiles)
+    q, k, v = [torch.randn(1, H, N, 64, generator=g, device=dev).to(dtype) for _ in range(3)]
+    mask = torch.rand(1, H if kind == "holes" else 1, nb, nb, generator=g, device=dev) < tiles / nb
+    i = torch.arange(nb, device=dev)
+    if kind == "causal":
+        mask &= i[:, None] >= i[None, :]
+    if kind == "holes":
+        mask &= (i % 5 != 0)[:, None]
+        mask[0, 0] &= (i < 3)[:, None]                     # a head with three lists
+    o_ref, lse_ref = naive_forward(q, k, v, mask, 0.125)
+    o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, 0.125)
+    none = torch.isinf(lse_ref)
+    assert torch.equal(torch.isinf(lse), none) and bool((o[none] == 0).all())
+    assert rel_l2(o, o_ref) <= (3e-3 if dtype == torch.bfloat16 else 1e-3) and float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
