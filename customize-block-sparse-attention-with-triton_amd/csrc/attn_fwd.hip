@@ -133,6 +133,8 @@ void fwd_kernel(const FwdRangeParams prm) {
   HeadSplit hs;
   int snap = 0;
   int64_t x0 = 0, x1 = 0;
+  int own_first = 0, own_parts = 0;  // a workgroup takes a row block or a part of it: where its parts begin, how many they are
+  constexpr int PART_TILES = 8;
   int r = 0, g0 = 0, g1 = 0;         // COOP: first row block and tiles of the range, g0 < g1 where they are known already
   if constexpr (!ROWS) {
     hs = head_split(rp, nb, prm.W, /*min_tiles=*/ONE ? 4 : NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
@@ -156,6 +158,7 @@ void fwd_kernel(const FwdRangeParams prm) {
     // dense 31.2 -> 29.0 us, where 12 are best for N = 17536 dense, 102.1 against 104.0 us)
     const int long_gap = MODE == WAVE || (int64_t)hs.T >= (int64_t)EQUAL_SPLIT_BELOW * hs.Peff ? LONG_GAP : 2 * LONG_GAP;
     if (long_ranges) { hs.gap = long_gap; hs.X = (int64_t)hs.T + (int64_t)long_gap * nb; }
+    const int own_row = wg;          // (the first workgroups on their compute units are the first row blocks')
     // Which range this workgroup takes (launches with few heads and long ranges): the ranges of a head start at
     // all phases of a row, and workgroups that share an XCD, hence an L2, get ranges of like phase, so that they
     // walk the same column blocks at the same time (dense N = 17536, one head: 42 instead of 196 MB fetched from
@@ -193,29 +196,44 @@ void fwd_kernel(const FwdRangeParams prm) {
       }
     }
     if (hs.T == 0) return;
-    // Short lists of about the same length, with about as many row blocks as ranges: a workgroup takes a row block.  Nothing has to be searched
-    // for and nothing meets in the workspace, 3 to 8 us of a launch; the ranges balance the work of uneven lists (a causal mask's, told by its
-    // first half of rows) and of few row blocks, and long lists by what the first-comers on a compute unit are faster.  (Not with strided K or
-    // V, where the variant for a number of heads that does not divide 8 would spill registers.)
-    // Ranges / row blocks, fp16, us; tiles of a row block, 3, 8, 16, 32, 48, 64:
-    //   1 head  N = 32000 (500 of 512)   16.1 / 13.6   23.9 / 18.9   29.6 / 24.2   40.5 / 33.2   53.1 / 41.7   55.3 / 51.8    causal, 25: 34.0 / 38.2
-    //   2 heads N = 16064 (251 of 256)   14.7 / 13.7   21.5 / 17.6   28.6 / 22.2   40.1 / 31.4   44.2 / 41.7   52.3 / 50.9    causal, 26: 34.3 / 34.8
-    //   3 heads N = 10048 (157 of 170)   15.9 / 13.5   22.3 / 17.2   28.7 / 22.6   38.6 / 29.9   48.5 / 39.4   49.9 / 47.6    causal, 16: 26.5 / 25.6
-    //   2 heads N = 12032 (188 of 256)   14.8 / 13.1   19.6 / 17.9   20.9 / 20.6   28.1 / 29.2   36.6 / 35.9   45.0 / 44.8    causal, 19: 24.3 / 27.5
-    //   1 head  N = 24000 (375 of 512)   16.2 / 13.4   17.7 / 17.0   22.1 / 22.5   29.3 / 29.6   37.1 / 38.3   45.6 / 45.8    (from 5 tiles on not there)
-    //   1 head  N = 17536 (274 of 512)   14.5 / 12.2   15.4 / 16.3   19.2 / 22.1   25.6 / 29.4   30.1 / 37.6   36.7 / 44.5    (nor there)
+    // Short lists of about the same length: the first workgroups on their compute units take a row block each, the second ones the row
+    // blocks that are left, in as many parts of 8 tiles or more as there are workgroups for.  Nothing has to be searched for and little meets in the
+    // workspace, 3 to 8 us of a launch, and no compute unit has two whole row blocks beside others that have none (where ranges snap to row
+    // blocks).  The ranges balance the work of uneven lists (a causal mask's, told by its first half of rows) and long lists by what the first-comers
+    // on a compute unit are faster.  (Not with strided K or V, where the variant for a number of heads that does not divide 8 would spill
+    // registers.)  Ranges / so, fp16, us; tiles of a row block, about 3, 8, 16, 26, 32, 48, 64:
+    //   1 head  N = 10048 (157 row blocks, 256 first workgroups)  13.0/10.7   15.9/13.1   18.9/16.0   20.7/18.4   22.1/22.1   25.2/26.9   27.8/30.7
+    //   1 head  N = 16384 (256)                                   12.1/11.2   15.1/14.0   18.2/16.7   22.5/20.0   25.1/23.1   29.7/28.9   35.5/35.1
+    //   1 head  N = 17536 (274, parts; 8 masks each)              14.5/12.9   16.1/16.5   18.3/18.7   23.6/21.8   26.8/24.8   30.0/29.1   35.8/35.8
+    //   1 head  N = 20032 (313)                                   15.8/14.5   16.6/17.7   19.3/19.5   25.2/22.8   28.5/26.3   32.6/31.3   38.9/37.3
+    //   2 heads N = 9024 (141 of 128, parts)                      14.4/12.8   15.7/16.0   17.7/18.2   23.1/21.1   26.2/24.2   29.8/28.3   35.3/34.0
+    //   1 head  N = 24000 (375, parts)                            15.7/15.2   19.8/17.5   21.7/20.8   26.4/24.4   29.3/27.9   37.5/34.4   45.9/40.2
+    //   1 head  N = 27008 (422, whole)                                 -      20.7/18.0   25.6/22.7   30.5/27.2   35.9/30.7   39.6/40.5   47.9/53.2
+    //   1 head  N = 32000 (500, whole)                            16.0/13.9   23.8/19.1   29.3/24.9   35.4/29.1   41.3/35.0   54.4/43.1   56.0/53.1    (causal, 25: 34 / 38)
+    //   3 heads N = 10048 (157 of 85, whole)                      15.9/13.9   22.1/17.7   29.0/23.4   33.9/26.9   39.3/31.1   49.3/41.2   51.6/50.0
     // (the pointer as a value the compiler cannot trace back: looked up only where needed)
     auto tiles_to_middle = [&]() {
       cint_ptr_t p = rp;
       asm volatile("" : "+s"(p));
       return p[nb / 2] - hs.lo;
     };
-    if (MODE == COOP && CONTIG && hs.T <= prm.own_row_tiles && 8 * tiles_to_middle() > 3 * hs.T) {
-      if (wg >= nb) return;
-      r = wg;
-      g0 = rp[wg];
-      g1 = rp[wg + 1];
-      if (g0 >= g1) return;
+    if (MODE == COOP && CONTIG && hs.T <= prm.own_row_most && (hs.T >= prm.own_row_least || hs.T <= 4 * nb) && 8 * tiles_to_middle() > 3 * hs.T) {
+      const int firsts = prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0;
+      r = own_row;
+      int part = 0, most = 1;
+      if (own_row >= firsts && nb > firsts) {
+        most = (prm.W - firsts) / (nb - firsts);
+        r = firsts + (own_row - firsts) / most;
+        part = (own_row - firsts) % most;
+      }
+      if (r >= nb) return;
+      const int row_s = rp[r], len = rp[r + 1] - row_s, parts = len < 2 * PART_TILES ? 1 : len / PART_TILES < most ? len / PART_TILES : most;
+      if (part >= parts || len == 0) return;
+      g0 = row_s + len * part / parts;
+      g1 = row_s + len * (part + 1) / parts;
+      wg = own_row;
+      own_first = own_row - part;
+      own_parts = parts;
     } else {
       if (wg >= hs.Peff) return;
       // where the range begins and ends on the cutting axis
@@ -1157,10 +1175,16 @@ void fwd_kernel(const FwdRangeParams prm) {
           // The workgroups pf .. pl hold the parts of this row block: pf is the one before the first range
           // boundary that stays inside the row block (boundaries close to an end move there), pl the one
           // after the last.  Every holder computes the same two numbers.
-          const int64_t xrow = row_pos(hs, r, row_s);
-          int pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)), pf_ = split_of_pos(hs, xrow);
-          while (pl_ > pf_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pl_), r, row_s, row_e), row_s, row_e) >= row_e) --pl_;
-          while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
+          int pl_, pf_;
+          if (own_parts > 0) {
+            pf_ = own_first;
+            pl_ = own_first + own_parts - 1;
+          } else {
+            const int64_t xrow = row_pos(hs, r, row_s);
+            pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)); pf_ = split_of_pos(hs, xrow);
+            while (pl_ > pf_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pl_), r, row_s, row_e), row_s, row_e) >= row_e) --pl_;
+            while (pf_ < pl_ && snap_boundary(snap, tile_of_pos(hs, split_pos(hs, pf_ + 1), r, row_s, row_e), row_s, row_e) <= row_s) ++pf_;
+          }
           const int nparts = pl_ - pf_ + 1;
           // The part is counted in once every wavefront's stores have been acknowledged (vmcnt 0, then the
           // barrier).  Every access to a part, stores here and loads below, is itself an access at device
@@ -1787,7 +1811,12 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.place_quot = prm.place_fast / heads;
   prm.place_rest = prm.place_fast % heads;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
-  prm.own_row_tiles = mode != COOP || prm.nb > prm.W ? 0 : (20 * prm.nb >= 17 * prm.W ? 64 : 4) * prm.nb;
+  {      // (the line between row blocks of workgroups and ranges, by a head's tiles: see the table in the kernel)
+    const int nb = prm.nb, W = prm.W, firsts = prm.first_ids / heads;
+    const bool whole = nb <= firsts || 4 * nb >= 3 * W;       // no row block is left for parts, or no workgroups
+    prm.own_row_most = mode != COOP || nb > W ? 0 : (nb <= firsts ? 32 : !whole ? 56 : 20 * nb >= 17 * W ? 64 : 30) * nb;
+    prm.own_row_least = whole || 10 * nb >= 7 * W ? 0 : 17 * nb;
+  }
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();

@@ -199,11 +199,12 @@ def test_shares_of_every_length(dev, H, N, dtype, out_fp32):
         assert rel_l2(o[0, h], p @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
 
 
-# Ranges of workgroups, about as many as row blocks, and short lists of like length: a workgroup takes a row block (at most 64 tiles each on
-# average, at most 4 where there are more workgroups).  Both sides of the line, rows without tiles, uneven lists.
+# Ranges of workgroups and short lists of like length: a workgroup takes a row block, or a part of one of those that are left (three heads:
+# none, one and two: parts; the numbers of tiles lie on both sides of the lines).  Rows without tiles, uneven lists.
 @pytest.mark.parametrize("H,N,tiles,dtype", [(3, 10048, 20, torch.float16), (3, 10048, 63, torch.bfloat16), (3, 10048, 66, torch.float16),
-                                             (2, 16100, 5, torch.float16), (1, 12000, 4, torch.bfloat16), (1, 12000, 5, torch.float16),
-                                             (1, 28000, 12, torch.float16), (3, 9300, 30, torch.bfloat16)])
+                                             (2, 16100, 5, torch.float16), (1, 12000, 4, torch.bfloat16), (1, 12000, 30, torch.float16),
+                                             (2, 9024, 24, torch.float16), (2, 9000, 50, torch.bfloat16), (2, 11000, 16, torch.float16),
+                                             (1, 17536, 28, torch.float16), (1, 20000, 40, torch.bfloat16), (3, 9300, 30, torch.bfloat16)])
 @pytest.mark.parametrize("kind", ["even", "causal", "holes"])
 def test_row_blocks_of_workgroups(dev, H, N, tiles, dtype, kind):
     import fa2_custom_mask as fm
