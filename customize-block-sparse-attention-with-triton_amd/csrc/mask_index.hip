@@ -19,6 +19,11 @@ __device__ __forceinline__ unsigned bools16(const u32x4& d) {
 // dense [.,.,N,N] bool -> block [.,.,nb,nb] bool (tile kept iff any element set).
 // One wavefront owns 64 rows x 1024 columns (16 tiles): every lane ORs its 16-byte column
 // slice over the 64 rows, then a ballot folds 4 lanes into one tile flag.
+// Bound by HBM, or below about 5000 rows by the launch.  All 64 loads stand before the first OR: the compiler then
+// holds twelve in flight from the first row to the last, in 60 registers, where batches of 16 ended in a wait for the
+// whole batch: N = 7040 8.2 -> 7.4 us, N = 8192 9.3 -> 8.7, N = 10240 15.6 -> 15.1 (6.9 TB/s), 8 heads N = 8192
+// 78.3 -> 76.6, N = 17536 the same.  28 in flight (124 registers): -1 % from N = 17536 on, nothing below.  Spans shared by two
+// or four wavefronts, 32 or 16 rows each: N = 17536 -3 %, but N = 8192 +10 %.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void reduce_dense_kernel(const uint8_t* __restrict__ dense, int N,
                                                            int nb, int H, int64_t sb, int64_t sh,
@@ -34,8 +39,11 @@ __global__ __launch_bounds__(256) void reduce_dense_kernel(const uint8_t* __rest
   const uint8_t* p = dense + b * sb + h * sh + (int64_t)rb * 64 * sm + (in ? col : 0);
   typedef unsigned int uintx4 __attribute__((ext_vector_type(4)));
   uintx4 acc = {0u, 0u, 0u, 0u};
-#pragma unroll 16
-  for (int r = 0; r < 64; ++r) acc |= __builtin_nontemporal_load(reinterpret_cast<const uintx4*>(p + r * sm));
+  uintx4 d[64];
+#pragma unroll
+  for (int r = 0; r < 64; ++r) d[r] = __builtin_nontemporal_load(reinterpret_cast<const uintx4*>(p + r * sm));
+#pragma unroll
+  for (int r = 0; r < 64; ++r) acc |= d[r];
   const bool nz = in && ((acc[0] | acc[1] | acc[2] | acc[3]) != 0u);
   const unsigned long long bal = __ballot(nz);
   if (lane < 16) {
