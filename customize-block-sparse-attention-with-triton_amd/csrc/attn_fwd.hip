@@ -133,10 +133,19 @@ void fwd_kernel(const FwdRangeParams prm) {
   HeadSplit hs;
   int snap = 0;
   int64_t x0 = 0, x1 = 0;
-  int own_first = 0, own_parts = 0;  // a workgroup takes a row block or a part of it: where its parts begin, how many they are
-  constexpr int PART_TILES = 8;
+  int own_first = 0, own_parts_n = 0;  // a workgroup takes a row block or a part of it: where its parts begin, how many they are
   int r = 0, g0 = 0, g1 = 0;         // COOP: first row block and tiles of the range, g0 < g1 where they are known already
   if constexpr (!ROWS) {
+    // (where the head's lists begin, for the choice below: every wavefront asks for all of them now, beside the head's ends, and does
+    // not wait; as atomics, which the compiler does not move to their use)
+    constexpr int OWN_LOADS = OWN_ROWS_MOST / 64 + 1;
+    int begins[OWN_LOADS] = {};
+    if (MODE == COOP && CONTIG && prm.own.most > 0) {
+      const int32_t* p = prm.row_ptr + (int64_t)mh * nb;
+#pragma unroll
+      for (int j = 0; j < OWN_LOADS; ++j)
+        if (64 * j <= nb) begins[j] = __hip_atomic_load(p + (64 * j + lane < nb ? 64 * j + lane : nb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
     hs = head_split(rp, nb, prm.W, /*min_tiles=*/ONE ? 4 : NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
     // Long ranges (the regime of the weighted shares) are cut on the axis with gaps and boundaries move to a row
     // block's end only from very close; short ranges are cut on the plain tile axis and their boundaries move to
@@ -196,11 +205,16 @@ void fwd_kernel(const FwdRangeParams prm) {
       }
     }
     if (hs.T == 0) return;
-    // Short lists of about the same length: the first workgroups on their compute units take a row block each, the second ones the row
+    // Short lists of about the same length (own_rows.h): the first workgroups on their compute units take a row block each, the second ones the row
     // blocks that are left, in as many parts of 8 tiles or more as there are workgroups for.  Nothing has to be searched for and little meets in the
     // workspace, 3 to 8 us of a launch, and no compute unit has two whole row blocks beside others that have none (where ranges snap to row
-    // blocks).  The ranges balance the work of uneven lists (a causal mask's, told by its first half of rows) and long lists by what the first-comers
-    // on a compute unit are faster.  (Not with strided K or V, where the variant for a number of heads that does not divide 8 would spill
+    // blocks).  The ranges balance the work of uneven lists and long lists by what the first-comers on a compute unit are faster: a causal mask's,
+    // told by its first half of rows; heads with a list longer than the rest saves (lists of about 26 tiles and one of 42, 50, 74, 1 head N = 17536:
+    // 23.1 / 22.0, 22.9 / 24.7, 23.3 / 30.9; of 42, 58, 74 where every compute unit has two row blocks, 2 heads N = 16064: 34.2 / 28.0, 33.5 / 31.8, 33.7 / 36.3), as row
+    // blocks kept whole are (0-3 and column blocks 0-3, ranges / so / as it is: N = 17536 keep 0.1 34.6 / 90 / 35.0, N = 12032 31.4 / 62 / 31.7, N = 32000
+    // keep 0.05 41 / 161 / 42, 3 heads N = 10048 keep 0.1 33.6 / 57 / 34.0); and heads of which more than a quarter of the lists are much longer than the mean
+    // (every other one twice as long, N = 32000 keep 0.05 32.3 / 39.6 / 32.6).  Looking at all lists costs 0.1 to 0.5 us.  (Not with strided K or V, where the
+    // variant for a number of heads that does not divide 8 would spill
     // registers.)  Ranges / so, fp16, us; tiles of a row block, about 3, 8, 16, 26, 32, 48, 64:
     //   1 head  N = 10048 (157 row blocks, 256 first workgroups)  13.0/10.7   15.9/13.1   18.9/16.0   20.7/18.4   22.1/22.1   25.2/26.9   27.8/30.7
     //   1 head  N = 16384 (256)                                   12.1/11.2   15.1/14.0   18.2/16.7   22.5/20.0   25.1/23.1   29.7/28.9   35.5/35.1
@@ -211,29 +225,32 @@ void fwd_kernel(const FwdRangeParams prm) {
     //   1 head  N = 27008 (422, whole)                                 -      20.7/18.0   25.6/22.7   30.5/27.2   35.9/30.7   39.6/40.5   47.9/53.2
     //   1 head  N = 32000 (500, whole)                            16.0/13.9   23.8/19.1   29.3/24.9   35.4/29.1   41.3/35.0   54.4/43.1   56.0/53.1    (causal, 25: 34 / 38)
     //   3 heads N = 10048 (157 of 85, whole)                      15.9/13.9   22.1/17.7   29.0/23.4   33.9/26.9   39.3/31.1   49.3/41.2   51.6/50.0
-    // (the pointer as a value the compiler cannot trace back: looked up only where needed)
-    auto tiles_to_middle = [&]() {
-      cint_ptr_t p = rp;
-      asm volatile("" : "+s"(p));
-      return p[nb / 2] - hs.lo;
-    };
-    if (MODE == COOP && CONTIG && hs.T <= prm.own_row_most && (hs.T >= prm.own_row_least || hs.T <= 4 * nb) && 8 * tiles_to_middle() > 3 * hs.T) {
-      const int firsts = prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0;
-      r = own_row;
-      int part = 0, most = 1;
-      if (own_row >= firsts && nb > firsts) {
-        most = (prm.W - firsts) / (nb - firsts);
-        r = firsts + (own_row - firsts) / most;
-        part = (own_row - firsts) % most;
+    auto of_like_length = [&]() {
+      const int longest = own_rows_longest(prm.own, hs.T), even = own_rows_even(prm.own, hs.T);
+      int most = 0, uneven = 0, middle = 0;
+#pragma unroll
+      for (int j = 0; j + 1 < OWN_LOADS; ++j) {
+        if (64 * j >= nb) break;
+        // (a list ends where the next lane's begins; behind the last one all begin at the head's end)
+        const int next = __builtin_amdgcn_update_dpp(__builtin_amdgcn_readfirstlane(begins[j + 1]), begins[j], /*wave_shl:1*/ 0x130, 0xf, 0xf, false);
+        const int end = 64 * j + lane < nb ? next : begins[j], len = end - begins[j];
+        most = len > most ? len : most;
+        uneven += __builtin_popcountll(__ballot(len > even));
+        if (nb / 128 == j) middle = __builtin_amdgcn_readlane(begins[j], nb / 2 % 64) - hs.lo;
       }
+      return own_rows_by_middle(hs.T, middle) && !__any(most > longest) && 4 * uneven <= nb;
+    };
+    if (MODE == COOP && CONTIG && own_rows_by_tiles(prm.own, hs.T, nb) && of_like_length()) {
+      const OwnItem it = own_item(own_row, nb, prm.W, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0);
+      r = it.row;
       if (r >= nb) return;
-      const int row_s = rp[r], len = rp[r + 1] - row_s, parts = len < 2 * PART_TILES ? 1 : len / PART_TILES < most ? len / PART_TILES : most;
-      if (part >= parts || len == 0) return;
-      g0 = row_s + len * part / parts;
-      g1 = row_s + len * (part + 1) / parts;
+      const int row_s = rp[r], len = rp[r + 1] - row_s, parts = own_parts(len, it.most);
+      if (it.part >= parts || len == 0) return;
+      g0 = row_s + len * it.part / parts;
+      g1 = row_s + len * (it.part + 1) / parts;
       wg = own_row;
-      own_first = own_row - part;
-      own_parts = parts;
+      own_first = own_row - it.part;
+      own_parts_n = parts;
     } else {
       if (wg >= hs.Peff) return;
       // where the range begins and ends on the cutting axis
@@ -1181,9 +1198,9 @@ void fwd_kernel(const FwdRangeParams prm) {
           // boundary that stays inside the row block (boundaries close to an end move there), pl the one
           // after the last.  Every holder computes the same two numbers.
           int pl_, pf_;
-          if (own_parts > 0) {
+          if (own_parts_n > 0) {
             pf_ = own_first;
-            pl_ = own_first + own_parts - 1;
+            pl_ = own_first + own_parts_n - 1;
           } else {
             const int64_t xrow = row_pos(hs, r, row_s);
             pl_ = split_of_pos(hs, xrow + (row_e - 1 - row_s)); pf_ = split_of_pos(hs, xrow);
@@ -1816,12 +1833,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   prm.place_quot = prm.place_fast / heads;
   prm.place_rest = prm.place_fast % heads;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
-  {      // (the line between row blocks of workgroups and ranges, by a head's tiles: see the table in the kernel)
-    const int nb = prm.nb, W = prm.W, firsts = prm.first_ids / heads;
-    const bool whole = nb <= firsts || 4 * nb >= 3 * W;       // no row block is left for parts, or no workgroups
-    prm.own_row_most = mode != COOP || nb > W ? 0 : (nb <= firsts ? 32 : !whole ? 56 : 20 * nb >= 17 * W ? 64 : 30) * nb;
-    prm.own_row_least = whole || 10 * nb >= 7 * W ? 0 : 17 * nb;
-  }
+  prm.own = mode == COOP ? own_lines(prm.nb, prm.W, prm.first_ids / heads) : OwnLines{};
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();
   prm.deterministic = get_deterministic();

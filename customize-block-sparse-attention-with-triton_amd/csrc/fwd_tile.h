@@ -3,6 +3,7 @@
 #pragma once
 #include "common.h"
 #include "kernel_util.h"
+#include "own_rows.h"
 #include "place.h"
 #include "quad_shares.h"
 
@@ -52,7 +53,7 @@ struct FwdRangeParams : FwdParams {
   // are cut into exactly perm_n ranges, the first perm_fast of them with the larger weight (perm_n = 0: none; see
   // range_permutation)
   int perm_n, perm_fast, perm_min_tiles;
-  int own_row_most, own_row_least;   // fwd_kernel, ranges of workgroups: tiles of heads that may be taken a row block per workgroup
+  OwnLines own;                    // fwd_kernel, ranges of workgroups: heads that go a row block to a workgroup
   unsigned short perm[512];        // (RANGE_PERM_MAX of range_perm.h)
   unsigned short perm_causal[512]; // the same for heads whose mask is the dense block-causal one
 };

@@ -200,12 +200,13 @@ def test_shares_of_every_length(dev, H, N, dtype, out_fp32):
 
 
 # Ranges of workgroups and short lists of like length: a workgroup takes a row block, or a part of one of those that are left (three heads:
-# none, one and two: parts; the numbers of tiles lie on both sides of the lines).  Rows without tiles, uneven lists.
+# none, one and two: parts; the numbers of tiles lie on both sides of the lines).  Rows without tiles; uneven lists, which stay on the ranges:
+# growing ones, some of all tiles, long and short ones in turn (which heads are taken: own_rows_check.cpp).
 @pytest.mark.parametrize("H,N,tiles,dtype", [(3, 10048, 20, torch.float16), (3, 10048, 63, torch.bfloat16), (3, 10048, 66, torch.float16),
                                              (2, 16100, 5, torch.float16), (1, 12000, 4, torch.bfloat16), (1, 12000, 30, torch.float16),
                                              (2, 9024, 24, torch.float16), (2, 9000, 50, torch.bfloat16), (2, 11000, 16, torch.float16),
                                              (1, 17536, 28, torch.float16), (1, 20000, 40, torch.bfloat16), (3, 9300, 30, torch.bfloat16)])
-@pytest.mark.parametrize("kind", ["even", "causal", "holes"])
+@pytest.mark.parametrize("kind", ["even", "causal", "holes", "whole", "turns"])
 def test_row_blocks_of_workgroups(dev, H, N, tiles, dtype, kind):
     import fa2_custom_mask as fm
     assert fwd_route_d64(1, H, N) == "workgroups"
@@ -219,8 +220,33 @@ def test_row_blocks_of_workgroups(dev, H, N, tiles, dtype, kind):
     if kind == "holes":
         mask &= (i % 5 != 0)[:, None]
         mask[0, 0] &= (i < 3)[:, None]                     # a head with three lists
+    if kind == "whole":
+        mask[..., [1, nb // 2, nb - 1], :] = True
+        mask[..., 0] = True
+    if kind == "turns":
+        mask[..., ::2, nb // 16:] = False
     o_ref, lse_ref = naive_forward(q, k, v, mask, 0.125)
     o, lse = fm.flash_attention_custom_mask_lse(q, k, v, mask, 0.125)
     none = torch.isinf(lse_ref)
     assert torch.equal(torch.isinf(lse), none) and bool((o[none] == 0).all())
     assert rel_l2(o, o_ref) <= (3e-3 if dtype == torch.bfloat16 else 1e-3) and float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
+
+
+# The same for elementwise masks: a window of tokens, whose lists but the first ones are of like length, and one whose first tokens and
+# last keep all others.
+@pytest.mark.parametrize("kind", ["window", "window and whole rows"])
+@pytest.mark.parametrize("H,N,tokens,dtype", [(1, 12000, 1000, torch.float16), (3, 9300, 1500, torch.bfloat16), (2, 9024, 1400, torch.float16)])
+def test_row_blocks_of_workgroups_elementwise(dev, H, N, tokens, dtype, kind):
+    import fa2_custom_mask as fm
+    assert fwd_route_d64(1, H, N) == "workgroups"
+    g = torch.Generator(device=dev).manual_seed(tokens)
+    q, k, v = [torch.randn(1, H, N, 64, generator=g, device=dev).to(dtype) for _ in range(3)]
+    i = torch.arange(N, device=dev)
+    mask = (i[:, None] - i[None, :]).abs() < tokens
+    if kind != "window":
+        mask[:70] = True
+        mask[-1] = True
+    o = fm.flash_attention_custom_mask(q, k, v, mask[None, None], 0.125)
+    for h in (0, H - 1):
+        s = (q[0, h].float() @ k[0, h].float().T * 0.125).masked_fill(~mask, float("-inf"))
+        assert rel_l2(o[0, h], torch.softmax(s, -1) @ v[0, h].float()) <= (3e-3 if dtype == torch.bfloat16 else 1e-3)
