@@ -1343,26 +1343,33 @@ int compute_units() {
 }
 
 // How a launch is split at D = 64, by its row blocks against the wavefronts that are resident at once (8 per compute unit).
-// With many a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us), with about as many a range of the list, with few
-// the ranges of whole workgroups are the faster ones: they share a row block's merge.
-// bf16, us, ranges of workgroups / of wavefronts, dense, block-causal, keep 0.5, 0.2, 0.1, 0.05:
-//   20 heads N = 4096 (0.62)  122 / 117    78 /  72    70 /  70    46 /  41    31 /  29    26 / 24
-//    3 heads N = 32000 (0.73) 994 / 904   491 / 473   505 / 470   219 / 208   124 / 117    77 / 72      6 heads N = 20032 (0.92) 738 / 711  383 / 375  387 / 374  173 / 163   98 /  92  64 / 58
-//   11 heads N = 8192 (0.69)  238 / 233   131 / 132   131 / 129    71 /  67    45 /  45    32 / 31      5 heads N = 17536 (0.67) 481 / 466  245 / 248  249 / 249  113 / 110   74 /  70  54 / 48    (not there)
-//   13 heads N = 6400 (0.63)  178 / 174   101 / 101   102 / 101    61 /  59    36 /  38    30 / 29      9 heads N = 8192 (0.56)  197 / 195  110 / 110  109 / 109   57 /  60   44 /  39  30 / 28    (nor there)
-//    4 heads N = 20032 (0.61) 483 / 482   256 / 256   258 / 257   116 / 118    72 /  74    50 / 49      3 heads N = 20032 (0.46) 388 / 375  197 / 201  201 / 200   91 /  94   63 /  61  41 / 43    (nor there)
+// From half as many more on a wavefront takes a row block (48 heads of N = 17776, keep 0.3: 2127 -> 1298 us; 24 heads of
+// N = 8192 dense 493 -> 425, causal 16 heads of N = 8192, one row block per wavefront, 172 -> 231: not there).  From three
+// quarters as many on a wavefront takes a range of the list, with fewer the ranges of whole workgroups are the faster
+// ones: they share a row block's merge.  bf16, us, ranges of workgroups / of wavefronts, keep 0.1, 0.3, 1 and block-causal:
+//   12 heads N = 8192 (0.75)   53 /  47    92 /  90   247 / 250   137 / 138      8 heads N = 8192 (0.5)   36 / 41   65 / 72   167 / 162    98 / 105
+//    9 heads N = 12000 (0.83)  71 /  65   139 / 138   398 / 404   211 / 208      6 heads N = 12000 (0.55) 53 / 52   96 / 98   265 / 270   153 / 153
+//   24 heads N = 4096 (0.75)   33 /  31    61 /  55   137 / 135    86 /  77     17 heads N = 4096 (0.53)  30 / 28   47 / 45    99 / 101    66 /  67
+//   48 heads N = 2048 (0.75)   26 /  24    40 /  38    85 /  79    54 /  58     56 heads N = 2048 (0.88)  28 / 25   41 / 42    94 /  86    61 /  60
+//    5 heads N = 24064 (0.92) 115 / 116   273 / 288   889 / 902   435 / 445    (above 300 row blocks per head: from one per wavefront on)
+// With the ranges walked from their last row block on more sizes gain by them, but not with every mask and not in bf16, whose rows have
+// fewer first tiles with an exact largest numerator in ranges of wavefronts (20 heads N = 4096 keep 0.5, 6 heads N = 20032 keep 0.15: 2.024e-4 -> 2.036e-4
+// and 2.031e-4 -> 2.045e-4 from 64 bits).  fp16, ranges of workgroups / of wavefronts, keep 0.03, 0.1, 0.3, dense, windows of 0.1 and 0.3, row and column
+// blocks 0-3 whole in keep 0.05, 0.02 and a diagonal with two whole row blocks:
+//   20 heads N = 4096 (0.62)   22 / 22    30 / 29    50 / 54   119 / 116    27 / 25    48 / 48    38 / 43    28 / 36
+//   14 heads N = 6656 (0.71)   29 / 23    38 / 38    77 / 71   185 / 185    33 / 39    73 / 67    42 / 50    32 / 43
+//    6 heads N = 20032 (0.92)  50 / 42    96 / 86   228 / 211  701 / 649    91 / 83   210 / 197   79 / 82    57 / 66
+//    3 heads N = 32000 (0.73)  51 / 52   111 / 108  296 / 264  935 / 825   105 / 103  262 / 247   85 / 104   55 / 91
 // whole row blocks / ranges of wavefronts:
-//   24 heads N = 8192 (1.50)  481 / 490   266 / 263   284 / 265   128 / 119    75 /  71    49 / 47     12 heads N = 17536 (1.61) 1231 / 1094  593 / 564  649 / 568  272 / 249  149 / 134  86 / 83
-//   14 heads N = 17536 (1.87) 1286 / 1258 681 / 657   685 / 655   292 / 283   168 / 163    99 / 104    16 heads N = 16640 (2.03) 1464 / 1278  665 / 676  755 / 675  317 / 290  175 / 166  104 / 100
-//   26 heads N = 8192 (1.62)  587 / 535   292 / 283   317 / 290   137 / 130    79 /  79    56 / 52     28 heads N = 8192 (1.75)  597 / 569   312 / 304   329 / 306   147 / 141    85 /  81    54 / 61    (not there)
-//   52 heads N = 4096 (1.62)  293 / 282   164 / 156   166 / 154    74 /  76    50 /  52    38 / 38     40 heads N = 6400 (1.95)  487 / 497   311 / 275   273 / 266   127 / 125    79 /  79    50 / 58    (nor there)
-//   18 heads N = 17536 (2.41) 1029 / 867  852 / 841   372 / 380   205 / 227   114 / 135                34 heads N = 8192 (2.12)  743 / 690   354 / 370   395 / 367   177 / 165    99 / 104   65 / 75    (nor there)
-// (compact: WAVE has four times as many ranges, hence parts, and there is no room for them.)
+//   24 heads N = 8192 (1.50)   38 / 38    72 / 70   167 / 153  436 / 446    62 / 76   140 / 151   84 / 75    77 / 56
+//   14 heads N = 17536 (1.87)  70 / 75   157 / 151  392 / 382 1155 / 1151  132 / 164  353 / 374  138 / 122  113 / 89
+//   16 heads N = 16640 (2.03)  68 / 70   156 / 151  439 / 386 1322 / 1178  144 / 180  366 / 388  132 / 129  112 / 88
 static int wave_slots() { return FwdCfg<64>::NW * FwdCfg<64>::WG_PER_CU * compute_units(); }    // wavefronts resident at once, D = 64
 static int fwd_mode(int B, int H, int nb, bool compact) {
-  const int64_t per_slot = 100ll * B * H * nb, slots = wave_slots();                 // (row blocks, in hundredths)
-  if (per_slot >= (compact || nb < 96 ? 150 : nb < 250 ? 174 : 216) * slots) return ROWS_MODE;
-  return !compact && per_slot >= (nb < 32 ? 100 : nb < 96 ? 60 : 70) * slots ? WAVE : COOP;
+  const int64_t rows = (int64_t)B * H * nb, slots = wave_slots();
+  if (2 * rows >= 3 * slots) return ROWS_MODE;
+  if (compact) return COOP;                                             // (WAVE has four times as many ranges, hence parts)
+  return rows >= slots || (nb >= 32 && nb <= 300 && 20 * rows >= (nb >= 48 ? 15 : 16) * slots) ? WAVE : COOP;
 }
 
 // ROWS_MODE: the workgroups per head for long row blocks, and the slots for their parts: as many as are resident at once,
