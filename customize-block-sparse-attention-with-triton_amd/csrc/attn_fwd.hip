@@ -107,13 +107,10 @@ void fwd_kernel(const FwdRangeParams prm) {
     // few heads in its L2 (rows_group); in a group the last row blocks of all heads, the long ones of block-causal masks,
     // first.  Behind the first `first_ids` of them, which fill the GPU, W workgroups per head for the long row blocks
     // (wg >= nb; see below).
-    const int extras = placed(BH, prm.group, prm.W), id = blockIdx.x;
-    const bool extra = id >= prm.first_ids && id < prm.first_ids + extras;
-    const int L = id < prm.first_ids ? id : extra ? id - prm.first_ids : id - extras, per = extra ? prm.W : nb;
-    const Place p = place(L, BH, prm.group, per);
-    if (p.item >= per) return;                   // padding of the last group
+    const Place p = place_rows(blockIdx.x, BH, prm.group, nb, prm.W, prm.first_ids);
+    if (p.item < 0) return;                      // padding of the last group
     bh = p.head;
-    wg = per - 1 - p.item + (extra ? nb : 0);
+    wg = p.item;
   } else if constexpr (SPREAD) {
     const Place p = place_range(blockIdx.x, BH, prm.W, prm.place_fast, prm.place_quot, prm.place_rest);
     bh = p.head;
@@ -1831,15 +1828,15 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   }
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.compact);
   prm.W = groups_per_head(s.B, s.H, prm.nb, mode, s.compact);
-  // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are.  (Not WAVE: single
-  // wavefronts that arrive while another kernel ends do not fill the SIMDs in order, and two with the larger share on one
-  // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
-  // after a pause 677 against 707.)
-  prm.first_ids = mode == COOP ? compute_units() : (mode == ROWS_MODE ? wave_slots() / 8 * 8 : 0);
   prm.place_fast = mode == COOP ? std::min(compute_units(), prm.W * heads) : 0;
   prm.place_quot = prm.place_fast / heads;
   prm.place_rest = prm.place_fast % heads;
   prm.group = mode == ROWS_MODE ? rows_group(s.B, s.H, prm.nb) : 0;
+  // with two workgroups per compute unit the first-comers are faster: tell the kernel which they are.  (Not WAVE: single
+  // wavefronts that arrive while another kernel ends do not fill the SIMDs in order, and two with the larger share on one
+  // SIMD cost more than the shares gain: 8 heads of N = 17536 dense after a kernel on its inputs 858-933 us against 732-816,
+  // after a pause 677 against 707.)
+  prm.first_ids = mode == COOP ? compute_units() : mode == ROWS_MODE ? first_ids_of_rows(wave_slots() / 8 * 8, heads, prm.group, prm.nb) : 0;
   prm.own = mode == COOP ? own_lines(prm.nb, prm.W, prm.first_ids / heads) : OwnLines{};
   prm.flags = (unsigned long long*)((char*)ws + slots_bytes(s.B, s.H, prm.W, mode));
   prm.epoch = next_epoch();

@@ -52,6 +52,21 @@ constexpr Place place(int L, int heads, int group, int items) {
   return {first + p.head, p.item};
 }
 
+// A launch of whole row blocks, nb of each head and W workgroups per head for parts of long ones, which come behind the first `first_ids` ids.
+// Item: a row block, the last ones first; nb + i: workgroup W - 1 - i of those for parts; -1: none (an id that only fills a group up).
+// (No more than the row blocks' ids are first ones: an id behind them would be a row block of a head that is not there.)
+constexpr int first_ids_of_rows(int resident, int heads, int group, int nb) {
+  const int ids = placed(heads, group, nb);
+  return resident < ids ? resident : ids;
+}
+constexpr Place place_rows(int id, int heads, int group, int nb, int W, int first_ids) {
+  const int extras = placed(heads, group, W);
+  const bool extra = id >= first_ids && id < first_ids + extras;
+  const int L = id < first_ids ? id : extra ? id - first_ids : id - extras, per = extra ? W : nb;
+  const Place p = place(L, heads, group, per);
+  return {p.head, p.item >= per ? -1 : per - 1 - p.item + (extra ? nb : 0)};
+}
+
 // A launch of `split` shares of all items (the share is the slowest index, so that a head stays on its XCDs): heads in groups of `group` (a
 // multiple of 8), as above; then a last group of 8 `whole` heads and the `rest` in eighths, all of them at once: an XCD has `whole` heads and
 // `rest` units, and takes eight items of each of the former and one of each of the latter in turn.
