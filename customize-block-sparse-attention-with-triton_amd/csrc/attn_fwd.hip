@@ -1820,7 +1820,7 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
       prm.part_ml = prm.part_o + parts * 64;
       prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
       prm.epoch = next_epoch();
-      prm.share_tiles = dt != 0 && prm.nb >= 56 ? 1 : 8;      // (short_plan)
+      prm.share_shift = dt != 0 && prm.nb >= 56 ? 0 : 3;      // (short_plan)
       launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
     }
     else launch_fwd_pair(prm, dt, tile_bits != nullptr, st);

@@ -82,10 +82,10 @@ __global__ __launch_bounds__(128 * S, 2) void fwd_short_kernel(const FwdParams p
   int shares = 1;
   if constexpr (SHARED) {                         // this workgroup's share of the row block's list
     const int len = t1 - t0;
-    shares = len >= prm.split * prm.share_tiles ? prm.split : len < 2 * prm.share_tiles ? 1 : len / prm.share_tiles;
+    shares = short_shares(len, prm.split, prm.share_shift);
     if (chunk >= shares) return;
-    t1 = t0 + (int)((int64_t)len * (chunk + 1) / shares);
-    t0 = t0 + (int)((int64_t)len * chunk / shares);
+    t1 = t0 + short_share_begins(len, chunk + 1, shares);
+    t0 = t0 + short_share_begins(len, chunk, shares);
   }
   const int valid = TAIL ? prm.N - (nb - 1) * 64 : 64, tail_cb = TAIL ? nb - 1 : -1;
   const unsigned short* kg = (const unsigned short*)prm.k + b * prm.ks[0] + h * prm.ks[1];

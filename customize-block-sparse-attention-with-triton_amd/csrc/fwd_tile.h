@@ -25,7 +25,7 @@ struct FwdParams {
   unsigned long long epoch;        // distinguishes this launch's counters from stale contents
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair and short kernel: workgroups per row block (1: results written directly)
-  int share_tiles;                 // short kernel, split > 1: tiles of a share, at least
+  int share_shift;                 // short kernel, split > 1: a share has at least 2^share_shift tiles
   float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
   int* part_len;                   // ... and the length of every row block's list [B*H][nb]
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)

@@ -1,9 +1,21 @@
-// Into how many shares the list of a row block is cut (fwd_quad_kernel, fwd_wide_kernel), by its own length.  Plain C++ (constexpr functions are
+// Into how many shares the list of a row block is cut (fwd_short_kernel; fwd_quad_kernel, fwd_wide_kernel), by its own length.  Plain C++ (constexpr functions are
 // usable on the device too).
 #pragma once
 #include "place.h"
 
 namespace bsattn {
+
+// fwd_short_kernel: shares of a list of len tiles, `split` at most (2 to 4), of at least 2^shift tiles each, and where share c begins (c = shares: the
+// list's end).  Without divisions, which stand in front of a workgroup's first access: launches of short lists take 0.1 to 0.3 us less without them
+// (1 head N = 3400 keep 0.1 10.25 -> 9.95, a window of 0.1 8.60 -> 8.39, N = 2048 keep 0.1 8.94 -> 8.82; where lists are never shared 9.93, 8.25, 8.80).
+constexpr int short_shares(int len, int split, int shift) {
+  const int n = len >> shift;
+  return n < 2 ? 1 : n < split ? n : split;
+}
+constexpr int short_share_begins(int len, int c, int shares) {      // len * c / shares, below 2^16
+  const int n = len * c;
+  return shares == 1 ? n : shares == 2 ? n / 2 : shares == 3 ? (int)((unsigned)n * 43691u >> 17) : n / 4;
+}
 
 constexpr int SHARE_SAMPLE = 4;       // lists looked at in the middle and at the end of a head
 constexpr int SHARE_MIN_BLOCKS = 8;   // row blocks of a head whose lists may be cut, at least
