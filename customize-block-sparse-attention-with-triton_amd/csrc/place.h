@@ -101,9 +101,9 @@ constexpr PlaceOfEight place_of_eight(int heads, int items, int split, Groups g)
 }
 constexpr PlaceOfEight place_of_eight(int heads, int items, int split) { return place_of_eight(heads, items, split, Groups{XCDS, 0, heads % XCDS}); }
 
-// The groups for kernels whose workgroups walk a list each: as many heads per XCD at once as its L2 (4 MB) holds the K and V (or Q and dO) of,
-// at most 8.  With one head per XCD a causal mask's last heads start their longest lists when the short ones of the heads before have
-// ended, and these are all that is left in the end; with more than the L2 holds the sparse uniform masks get slower.
+// The groups for kernels whose workgroups walk a list each: as many heads per XCD at once as its L2 (4 MB) holds the K and V (or Q and dO) of and
+// as divide the heads of an XCD, at most 8.  With one head per XCD a causal mask's last heads start their longest lists when the short ones of the
+// heads before have ended, and these are all that is left in the end; with more than the L2 holds the sparse uniform masks get slower.
 // us, bf16, a forward / its training step, 8 heads at a time and so; block-causal, causal keep 0.25, keep 0.2, dense:
 //   D = 64    16 heads N = 4096    55 / 263 ->  54 / 232    27 / 103 ->  24 /  93    32 / 112 ->  31 / 110    91 /  362 ->  91 /  361
 //             10 heads N = 4096    45 / 162 ->  36 / 138    21 /  72 ->  17 /  72    25 /  81 ->  24 /  79    70 /  262 ->  70 /  262
@@ -111,20 +111,31 @@ constexpr PlaceOfEight place_of_eight(int heads, int items, int split) { return 
 //             64 heads N = 2048   102 / 412 ->  82 / 353    41 / 166 ->  37 / 152    47 / 200 ->  48 / 197   151 /  656 -> 151 /  657
 //             24 heads N = 2048    56 / 190 ->  47 / 163    26 /  88 ->  21 /  81    28 / 104 ->  24 /  98    63 /  259 ->  64 /  260
 //   D = 256   16 heads N = 2048    63 / 261 ->  56 / 248    30 / 122 ->  26 / 118    33 / 148 ->  29 / 141    77 /  360 ->  77 /  358
-// Half as much again where these are all heads (block-causal, causal keep 0.5, keep 0.25, 0.1):
+// 1.6 times as much where these are all heads (block-causal, causal keep 0.5, keep 0.25, 0.1):
 //   D = 128   16 heads N = 6016 (3 MB)   176 / 737 -> 160 / 692    98 / 414 ->  90 / 387   103 / 425 -> 102 / 419    53 / 208 -> 52 / 209
 //   D = 256   16 heads N = 3000          94 / 455 ->  88 / 452     57 / 275 ->  54 / 262    62 / 293 ->  61 / 276    39 / 171 -> 38 / 169
 // With twice as much the causal launches gain and the sparse uniform ones lose:
 //   D = 128   32 heads N = 8192 (4 MB)   560 / 2454 -> 557 / 2419  177 / 762 -> 167 / 741  251 / 1091 -> 267 / 1140 150 / 644 -> 154 / 651   (keep 0.25, causal and not)
 //   D = 256   16 heads N = 4096          150 / 717 -> 150 / 705    88 / 424 ->  84 / 404    96 / 461 ->  97 / 452    58 / 274 -> 61 / 277
+// Heads beyond a multiple of 8 go out with the last group, but three or more of them behind it where a head and they are more than 1.6 times
+// what the L2 holds, or 1.4 times where there is no other group, which these do not touch (D = 128 and 256; the backward of D = 64 loses nothing by
+// them).  Behind / with it, forward and step; keep 0.3, 0.1, block-causal, window of 0.3:
+//   D = 128   12 heads N = 8192 (8 MB)   161 /  668 -> 163 /  671    68 / 272 ->  71 / 283   244 / 1090 -> 229 / 1008   137 / 562 -> 140 / 555   (not there)
+//             15 heads N = 8000          181 /  785 -> 184 /  789    78 / 321 ->  82 / 342   267 / 1168 -> 264 / 1167   157 / 639 -> 158 / 642   (nor there)
+//   D = 256   14 heads N = 6000 (12 MB)  211 /  975 -> 222 /  994   105 / 455 -> 109 / 462   297 / 1438 -> 286 / 1358   171 / 767 -> 174 / 779   (nor there)
+//             12 heads N = 3000 (6 MB)    67 /  304 ->  66 /  304    35 / 151 ->  35 / 154    94 /  451 ->  89 /  409    54 / 225 ->  54 / 234   (nor there)
+//             20 heads N = 3000            88 /  400 ->   89 /  398     50 /  213 ->   49 /  209    146 /  704 ->  131 /  571     79 /  338 ->   78 /  339
+//             17 heads N = 5000 (10 MB)  183 /  875 -> 183 /  855    89 / 398 ->  91 / 398   314 / 1532 -> 251 / 1205   153 / 710 -> 151 / 688   (one head alone)
 // (A choice by the lists, in the kernels, costs the backward's registers: 8 heads N = 4096 D = 128 dense 334 -> 345.)
 constexpr Groups groups_of_heads(int heads, int64_t N, int D) {
   const int64_t bytes = 4 * N * D, fit = (4ll << 20) / bytes;
   const int per_xcd = heads / XCDS, rest = heads % XCDS, most = fit < 1 ? 1 : fit > 8 ? 8 : (int)fit;
+  auto fits = [&](int n, int tenths) { return 10 * n * bytes <= (int64_t)tenths * (4 << 20); };      // tenths of the L2
   int n = per_xcd < most ? per_xcd : most;       // (like groups)
-  if (rest == 0 && per_xcd <= 8 && 10 * per_xcd * bytes <= (64ll << 20)) n = per_xcd;
+  if (rest == 0 && per_xcd <= 8 && fits(per_xcd, 16)) n = per_xcd;
   while (n > 1 && per_xcd % n != 0) --n;
-  return {XCDS * (n > 1 ? n : 1), rest > 0 ? n : 0, rest};
+  const bool behind = rest >= 3 && D > 64 && !fits(2, per_xcd > 1 ? 16 : 14);      // (n is 1 then)
+  return {XCDS * (n > 1 ? n : 1), rest > 0 && !behind ? n : 0, rest};
 }
 
 // ---- W ranges per head, all resident at once ----

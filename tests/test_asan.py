@@ -11,4 +11,4 @@ def test_make_asan(tmp_path):
     out = subprocess.run(["make", "-C", os.path.join(ROOT, "tests", "asan"), "asan", "OUT=" + str(tmp_path)],
                          capture_output=True, text=True)
     assert out.returncode == 0, out.stdout[-3000:] + out.stderr[-3000:]
-    assert out.stdout.count("\nok") >= 9
+    assert out.stdout.count("\nok") >= 10
