@@ -1589,8 +1589,9 @@ static int pair_split(int B, int H, int N, int D, bool compact) {
 //    4 heads N = 2048 (128)             7.1/ 7.3/ 7.3/ 7.3 (14.4)   10.6/10.5/10.6/10.6 (15.0)   14.7/13.6/18.6/18.3 (18.1)   14.5/12.5/15.7/16.9 (16.0)
 //    1 head  N = 8192 (128)            11.2/10.9/10.9/10.9 (15.4)   21.4/16.8/22.0/20.8 (21.0)   44.0/29.6/39.1/34.4 (34.3)   42.9/27.2/27.2/27.9 (28.5)
 //    3 heads N = 5120 (240)             9.2/10.1/11.4/12.7 (23.5)   17.4/22.3/27.5/31.4 (29.4)   31.0/38.3/43.3/46.9 (47.2)   29.3/25.9/30.2/32.4 (32.6)   (nor there)
-// (With bf16 from 56 row blocks on also the shortest lists are shared: a share's first tiles have exact largest numerators, without which its
-// rows are further from 64 bits.)
+// (With bf16 from 56 row blocks on also the shortest lists are shared, as they were when a launch of its own summed four shares of every list there:
+// a share's first tiles have exact largest numerators, so that rows of fewer shares would be further from 64 bits than they were.  Lists of fewer
+// row blocks never were shared that way.)
 struct ShortPlan { int pairs, split; };
 static ShortPlan short_plan(int64_t row_blocks, int nb) {
   const int64_t cus = compute_units(), rows = row_blocks * 256 / cus;       // (as if there were 256 compute units)
@@ -1812,18 +1813,18 @@ int launch_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
   if (s.D != 64 || plan.pairs > 0) {
     prm.split = s.D == 64 ? plan.split : tile_bits != nullptr ? 1 : pair_split(s.B, s.H, s.N, s.D, s.compact);
     prm.place = place_of_eight(heads, prm.nb, prm.split, groups_of_heads(heads, s.N, s.D));
+    const size_t parts = s.D == 64 ? (size_t)heads * prm.nb * prm.split * 64 : (size_t)prm.split * heads * s.N;      // rows of them
     prm.part_o = (float*)ws + 64;
-    prm.part_ml = prm.part_o + (size_t)prm.split * heads * s.N * s.D;
-    prm.part_len = (int*)(prm.part_ml + (size_t)prm.split * heads * s.N * 2);
+    prm.part_ml = prm.part_o + parts * s.D;
     if (s.D == 64) {
-      const size_t parts = (size_t)heads * prm.nb * prm.split * 64;
-      prm.part_ml = prm.part_o + parts * 64;
       prm.flags = (unsigned long long*)(prm.part_ml + parts * 2);
       prm.epoch = next_epoch();
       prm.share_shift = dt != 0 && prm.nb >= 56 ? 0 : 3;      // (short_plan)
       launch_fwd_short(prm, plan.pairs, dt, tile_bits != nullptr, st);
+      return launch_status();
     }
-    else launch_fwd_pair(prm, dt, tile_bits != nullptr, st);
+    prm.part_len = (int*)(prm.part_ml + parts * 2);
+    launch_fwd_pair(prm, dt, tile_bits != nullptr, st);
     return launch_status();
   }
   const int mode = fwd_mode(s.B, s.H, prm.nb, s.compact);

@@ -26,8 +26,10 @@ struct FwdParams {
   int deterministic;               // tiles go to the wavefronts of a workgroup in a fixed pattern
   int split;                       // pair and short kernel: workgroups per row block (1: results written directly)
   int share_shift;                 // short kernel, split > 1: a share has at least 2^share_shift tiles
-  float* part_o; float* part_ml;   // split > 1: unnormalised fp32 O parts [split][B*H][N][D] and their (m, l) [split][B*H][N][2]
-  int* part_len;                   // ... and the length of every row block's list [B*H][nb]
+  // split > 1: unnormalised fp32 O parts and their (m, l).  Pair kernel: [split][B*H][N][D] and [split][B*H][N][2], and the length of every
+  // row block's list [B*H][nb]; short kernel: [B*H][nb][split][64][D] and [B*H][nb][split][64][2]
+  float* part_o; float* part_ml;
+  int* part_len;
   int B, H, N, nb, Bm, Hm, W;   // W: workgroups per head (ROWS: those for long row blocks)
   int first_ids;                // workgroups with a linear id below this are the first on their compute unit (ROWS: fill the GPU)
   int place_fast, place_quot, place_rest;   // SPREAD: place_range's arguments

@@ -129,18 +129,21 @@ def test_forward_against_naive(dev, seed):
 
 
 # About as many row blocks as wavefronts: ranges of single wavefronts, whose last row block is walked before the first one.  Sizes
-# at both ends of that regime (0.75 to 1.5 row blocks per wavefront, from 1 on below 32 and above 300 row blocks) and inside it,
+# at both ends of that regime (0.75 to 1.5 row blocks per wavefront, from 1 on below 32 and above 300 row blocks), inside it and just outside it,
 # ranges that lie in one row block, end with one, and span several; bounds as above.
 @pytest.mark.parametrize("B,H,N,dtype,out_fp32,seed", [
     (1, 25, 4096, torch.float16, False, 0), (1, 24, 4096, torch.bfloat16, True, 1), (1, 24, 4033, torch.bfloat16, False, 2),
     (1, 16, 8160, torch.float16, True, 3), (2, 23, 4096, torch.float16, False, 4), (2, 8, 8192, torch.bfloat16, True, 5),
-    (1, 23, 8192, torch.float16, False, 6), (1, 12, 16100, torch.bfloat16, False, 7), (1, 47, 4064, torch.float16, True, 8)])
+    (1, 23, 8192, torch.float16, False, 6), (1, 12, 16100, torch.bfloat16, False, 7), (1, 47, 4064, torch.float16, True, 8),
+    (1, 20, 4096, torch.float16, False, 0), (1, 27, 8192, torch.float16, False, 6), (1, 16, 16100, torch.bfloat16, False, 7)])
 def test_ranges_of_wavefronts(dev, B, H, N, dtype, out_fp32, seed):
     import fa2_custom_mask as fm
     rs = np.random.RandomState(100 + seed)
     g = torch.Generator(device=dev).manual_seed(seed)
     nb = (N + 63) // 64
-    assert fwd_route_d64(B, H, N) == "wavefronts"
+    per_wavefront = B * H * nb / (8 * torch.cuda.get_device_properties(0).multi_processor_count)
+    route = "workgroups" if per_wavefront < 0.75 else "wavefronts" if per_wavefront < 1.5 else "rows"
+    assert fwd_route_d64(B, H, N) == route
     q, k, v = [torch.randn(B, H, N, 64, generator=g, device=dev).to(dtype) for _ in range(3)]
     bar = 3e-3 if (dtype == torch.bfloat16 and not out_fp32) else 1e-3
     for step in range(3):
@@ -155,7 +158,7 @@ def test_ranges_of_wavefronts(dev, B, H, N, dtype, out_fp32, seed):
             assert float((lse[~none] - lse_ref[~none]).abs().max()) <= 2e-3
         assert rel_l2(o, o_ref) <= bar
         again, _ = fm.flash_attention_custom_mask_lse(q, k, v, md, 0.125, out_fp32=out_fp32)
-        assert torch.equal(o, again)                       # (a range's order is fixed)
+        assert route == "workgroups" or torch.equal(o, again)                       # (a wavefront's order is fixed)
     if N <= 4096 and B == 1:                               # elementwise: a window of tokens
         i = torch.arange(N, device=dev)
         d = i[:, None] - i[None, :]
