@@ -209,9 +209,10 @@ void fwd_kernel(const FwdRangeParams prm) {
     // told by its first half of rows; heads with a list longer than the rest saves (lists of about 26 tiles and one of 42, 50, 74, 1 head N = 17536:
     // 23.1 / 22.0, 22.9 / 24.7, 23.3 / 30.9; of 42, 58, 74 where every compute unit has two row blocks, 2 heads N = 16064: 34.2 / 28.0, 33.5 / 31.8, 33.7 / 36.3), as row
     // blocks kept whole are (0-3 and column blocks 0-3, ranges / so / as it is: N = 17536 keep 0.1 34.6 / 90 / 35.0, N = 12032 31.4 / 62 / 31.7, N = 32000
-    // keep 0.05 41 / 161 / 42, 3 heads N = 10048 keep 0.1 33.6 / 57 / 34.0); and heads of which more than a quarter of the lists are much longer than the mean
-    // (every other one twice as long, N = 32000 keep 0.05 32.3 / 39.6 / 32.6).  Looking at all lists costs 0.1 to 0.5 us.  (Not with strided K or V, where the
-    // variant for a number of heads that does not divide 8 would spill
+    // keep 0.05 41 / 161 / 42, 3 heads N = 10048 keep 0.1 33.6 / 57 / 34.0); and, where compute units have more than one row block, heads of which more than a
+    // quarter of the lists are much longer than the mean (every other row at keep 0.1, the others at 0.01: N = 30000 38.5 / 47.8 / 39.0; taken: 3 heads N = 10048
+    // 24.6 / 21.9 / 22.3, and with a row block per compute unit N = 10048 19.8 / 16.8 / 17.2).  Looking at all lists costs 0.1 to 0.5 us.  (Not with strided K or V,
+    // where the variant for a number of heads that does not divide 8 would spill
     // registers.)  Ranges / so, fp16, us; tiles of a row block, about 3, 8, 16, 26, 32, 48, 64:
     //   1 head  N = 10048 (157 row blocks, 256 first workgroups)  13.0/10.7   15.9/13.1   18.9/16.0   20.7/18.4   22.1/22.1   25.2/26.9   27.8/30.7
     //   1 head  N = 16384 (256)                                   12.1/11.2   15.1/14.0   18.2/16.7   22.5/20.0   25.1/23.1   29.7/28.9   35.5/35.1

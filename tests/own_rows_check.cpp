@@ -63,15 +63,15 @@ int main() {
     bool sound = true;
     const int longest = h.longest_piece(sound);
     if (!sound) { printf("%d heads of %d row blocks: not every row block once\n", l.heads, l.nb); return 1; }
-    if (longest > 16 + 1.5 * h.T / h.nb) { printf("%d heads of %d row blocks, mean %.1f: a workgroup walks %d tiles\n", l.heads, l.nb, (double)h.T / h.nb, longest); return 1; }
+    if (longest > 20 + 1.5 * h.T / h.nb) { printf("%d heads of %d row blocks, mean %.1f: a workgroup walks %d tiles\n", l.heads, l.nb, (double)h.T / h.nb, longest); return 1; }
   }
   if (heads < 1000) { printf("only %d heads taken\n", heads); return 1; }
-  // one or four row blocks kept whole in a sparse mask, a few lists of all row blocks and none beside them, long and short ones in turn: the ranges'
+  // one or four row blocks kept whole in a sparse mask, a few lists of all row blocks and none beside them, much longer and short ones in turn: the ranges'
   for (const auto& [l, keep] : std::vector<std::pair<Launch, double>>{{{1, 274}, 0.1}, {{1, 188}, 0.1}, {{1, 256}, 0.03}, {{2, 141}, 0.1}, {{1, 500}, 0.05}, {{3, 157}, 0.1}, {{2, 251}, 0.05}})
     for (int whole : {1, 4}) {
-      std::vector<int> len = random(l.nb, keep), one = len, few(l.nb, 0), every(l.nb, 1), turns(l.nb, 2);
+      std::vector<int> len = random(l.nb, keep), one = len, few(l.nb, 0), every(l.nb, 1), turns(l.nb, 2);      // (of 56 tiles: 29 on the average)
       for (int r = 0; r < whole; ++r) len[r] = one[l.nb / 2 + r] = few[r * 7] = every[l.nb / 3] = l.nb;
-      for (int r = 0; r < l.nb; r += 2) turns[r] = 30;
+      for (int r = 0; r < l.nb; r += 2) turns[r] = 56;
       for (const auto& x : {len, one, few, every, turns})
         if (Head(l, x).taken()) { printf("%d heads of %d row blocks, keep %.2f, %d whole: taken\n", l.heads, l.nb, keep, whole); return 1; }
     }
