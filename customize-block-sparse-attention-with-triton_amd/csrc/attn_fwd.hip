@@ -137,11 +137,11 @@ void fwd_kernel(const FwdRangeParams prm) {
     // not wait; as atomics, which the compiler does not move to their use)
     constexpr int OWN_LOADS = OWN_ROWS_MOST / 64 + 1;
     int begins[OWN_LOADS] = {};
-    if (MODE == COOP && CONTIG && prm.own.most > 0) {
+    if constexpr (MODE == COOP && CONTIG) {
       const int32_t* p = prm.row_ptr + (int64_t)mh * nb;
 #pragma unroll
       for (int j = 0; j < OWN_LOADS; ++j)
-        if (64 * j <= nb) begins[j] = __hip_atomic_load(p + (64 * j + lane < nb ? 64 * j + lane : nb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        begins[j] = __hip_atomic_load(p + (64 * j + lane < nb ? 64 * j + lane : nb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
     }
     hs = head_split(rp, nb, prm.W, /*min_tiles=*/ONE ? 4 : NW, prm.first_ids > bh ? (prm.first_ids - bh + BH - 1) / BH : 0, 0);
     // Long ranges (the regime of the weighted shares) are cut on the axis with gaps and boundaries move to a row
