@@ -107,10 +107,10 @@ void fwd_kernel(const FwdRangeParams prm) {
     // few heads in its L2 (rows_group); in a group the last row blocks of all heads, the long ones of block-causal masks,
     // first.  Behind the first `first_ids` of them, which fill the GPU, W workgroups per head for the long row blocks
     // (wg >= nb; see below).
-    const Place p = place_rows(blockIdx.x, BH, prm.group, nb, prm.W, prm.first_ids);
-    if (p.item < 0) return;                      // padding of the last group
-    bh = p.head;
-    wg = p.item;
+    const PlaceOfRows at = place_rows(blockIdx.x, BH, prm.group, nb, prm.W, prm.first_ids);
+    if (at.p.item >= at.per) return;             // padding of the last group
+    bh = at.p.head;
+    wg = at.per - 1 - at.p.item + (at.extra ? nb : 0);
   } else if constexpr (SPREAD) {
     const Place p = place_range(blockIdx.x, BH, prm.W, prm.place_fast, prm.place_quot, prm.place_rest);
     bh = p.head;

@@ -52,19 +52,19 @@ constexpr Place place(int L, int heads, int group, int items) {
   return {first + p.head, p.item};
 }
 
-// A launch of whole row blocks, nb of each head and W workgroups per head for parts of long ones, which come behind the first `first_ids` ids.
-// Item: a row block, the last ones first; nb + i: workgroup W - 1 - i of those for parts; -1: none (an id that only fills a group up).
+// A launch of whole row blocks, nb of each head and W workgroups per head for parts of long ones, which come behind the first `first_ids` ids: one of
+// the latter (extra) or not, and which of its kind's `per` items of a head; item >= per: an id that only fills a group up.
 // (No more than the row blocks' ids are first ones: an id behind them would be a row block of a head that is not there.)
 constexpr int first_ids_of_rows(int resident, int heads, int group, int nb) {
   const int ids = placed(heads, group, nb);
   return resident < ids ? resident : ids;
 }
-constexpr Place place_rows(int id, int heads, int group, int nb, int W, int first_ids) {
+struct PlaceOfRows { Place p; int per; bool extra; };
+constexpr PlaceOfRows place_rows(int id, int heads, int group, int nb, int W, int first_ids) {
   const int extras = placed(heads, group, W);
   const bool extra = id >= first_ids && id < first_ids + extras;
   const int L = id < first_ids ? id : extra ? id - first_ids : id - extras, per = extra ? W : nb;
-  const Place p = place(L, heads, group, per);
-  return {p.head, p.item >= per ? -1 : per - 1 - p.item + (extra ? nb : 0)};
+  return {place(L, heads, group, per), per, extra};
 }
 
 // A launch of `split` shares of all items (the share is the slowest index, so that a head stays on its XCDs): heads in groups of `group` (a

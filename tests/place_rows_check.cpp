@@ -15,10 +15,11 @@ int main() {
             std::vector<int> seen(heads * (nb + W));
             int taken = 0;
             for (int id = 0; id < ids; ++id) {
-              const Place p = place_rows(id, heads, group, nb, W, first);
-              if (p.item < 0) continue;
-              if (p.head < 0 || p.head >= heads || p.item >= nb + W || seen[p.head * (nb + W) + p.item]++ || (p.item >= nb && id < first)) {
-                std::printf("%d heads of %d row blocks, group %d, %d workgroups for parts, %d resident: id %d takes head %d item %d\n", heads, nb, group, W, resident, id, p.head, p.item);
+              const PlaceOfRows at = place_rows(id, heads, group, nb, W, first);
+              if (at.p.item >= at.per) continue;
+              const int item = at.p.item + (at.extra ? nb : 0);
+              if (at.p.head < 0 || at.p.head >= heads || at.per != (at.extra ? W : nb) || at.p.item < 0 || seen[at.p.head * (nb + W) + item]++ || (at.extra && id < first)) {
+                std::printf("%d heads of %d row blocks, group %d, %d workgroups for parts, %d resident: id %d takes head %d item %d\n", heads, nb, group, W, resident, id, at.p.head, item);
                 return 1;
               }
               ++taken;
